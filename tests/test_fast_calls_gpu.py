@@ -1,0 +1,108 @@
+"""The direct calls (csrc/host/fast_calls.cpp) against the registered ops: the same bits where they answer, and no answer
+where something sits between the call and the device implementation."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _w4(device, k, n, group, dtype, bias):
+    from vllm_amd.layers.linear import LinearBase
+    from vllm_amd.layers.quantization import get_quantization_config
+    g = torch.Generator(device=device).manual_seed(k + n)
+    config = get_quantization_config("gptq_marlin").from_config(dict(bits=4, group_size=group, desc_act=False, sym=True))
+    layer = LinearBase(k, n, bias=bias, quant_config=config, params_dtype=dtype, return_bias=False).to(device)
+    layer.qweight.data.copy_(torch.randint(-2 ** 31, 2 ** 31 - 1, layer.qweight.shape, dtype=torch.int32, device=device, generator=g))
+    layer.scales.data.copy_(torch.rand(layer.scales.shape, device=device, generator=g) * 0.01 + 1e-3)
+    layer.g_idx.data.copy_(torch.arange(k, device=device) // (group if group > 0 else k))
+    layer.process_weights_after_loading()
+    return layer
+
+
+def _registered(layer, x):
+    import vllm_amd._custom_ops as ops  # noqa: F401
+    from vllm_amd.scalar_type import scalar_types
+    kern, rows = layer.quant_method.kernel, x.reshape(-1, x.shape[-1])
+    size_k, size_n = kern.config.partition_weight_shape
+    out = torch.ops.vllm_amd.gptq_marlin_gemm(rows, None, layer.qweight, layer.bias, layer.scales, None, layer.qzeros, layer.g_idx,
+                                              layer.g_idx_sort_indices, kern.workspace, scalar_types.uint4b8.id, rows.shape[0],
+                                              size_n, size_k)
+    return out.reshape(x.shape[:-1] + (size_n,))
+
+
+@pytest.mark.parametrize("shape", [(1, 512), (65, 512), (2, 3, 512), (512,)])
+@pytest.mark.parametrize("group,dtype,bias", [(128, torch.bfloat16, False), (32, torch.float16, True), (-1, torch.bfloat16, True)])
+def test_w4_layer_equals_the_registered_op(device, shape, group, dtype, bias):
+    from vllm_amd import _custom_ops as ops
+    layer = _w4(device, 512, 192, group, dtype, bias)
+    x = torch.randn(shape, device=device).to(dtype)
+    got = layer(x)
+    assert got.shape == shape[:-1] + (192,) and got.is_contiguous()
+    assert torch.equal(got, _registered(layer, x))
+    strided = torch.randn(7, 1024, device=device).to(dtype)[:, :512]
+    assert torch.equal(layer(strided), _registered(layer, strided))
+    direct = ops._fast.w4_linear(x, layer.qweight, layer.bias, layer.scales, layer.qzeros, layer.g_idx, layer.g_idx_sort_indices,
+                                 layer.quant_method.kernel.workspace, layer.quant_method.quant_config.quant_type.id, 192, 512, True)
+    assert direct is not None, "a plain call went through the dispatcher"
+
+
+@pytest.mark.parametrize("shape", [(1, 256), (67, 256), (2, 5, 256)])
+@pytest.mark.parametrize("static", [False, True])
+@pytest.mark.parametrize("bias", [False, True])
+def test_fp8_layer_equals_its_two_steps(device, shape, static, bias):
+    from vllm_amd import _custom_ops as ops
+    w = (torch.randn(320, 256, device=device) * 0.05).to(torch.bfloat16)
+    wq, ws = ops.scaled_fp8_quant(w, use_per_token_if_dynamic=True)
+    b = torch.randn(320, device=device).to(torch.bfloat16) if bias else None
+    x = torch.randn(shape, device=device).to(torch.bfloat16)
+    scale = torch.full((1,), 0.01, device=device) if static else None
+    got = ops.fp8_linear(x, wq.t(), ws, scale, None, torch.bfloat16, b)
+    rows = x.reshape(-1, 256)
+    q = torch.empty(rows.shape, dtype=torch.float8_e4m3fn, device=device)
+    s = scale if static else torch.empty(rows.shape[0], 1, device=device)
+    if static:
+        torch.ops.vllm_amd.static_scaled_fp8_quant(q, rows, s)
+    else:
+        torch.ops.vllm_amd.dynamic_per_token_scaled_fp8_quant(q, rows, s, None)
+    ref = torch.empty(rows.shape[0], 320, dtype=torch.bfloat16, device=device)
+    torch.ops.vllm_amd.cutlass_scaled_mm(ref, q, wq.t(), s, ws, b)
+    assert got is not None and torch.equal(got, ref.reshape(shape[:-1] + (320,)))
+    q2, s2 = ops._fast.fp8_quant(rows, scale, None, not static, None)
+    assert torch.equal(q2.view(torch.uint8), q.view(torch.uint8)) and torch.equal(s2, s)
+    assert torch.equal(ops._fast.scaled_mm(q2, wq.t(), s2, ws, torch.bfloat16, b), ref)
+
+
+def test_no_answer_where_something_is_in_between(device):
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from vllm_amd import _custom_ops as ops, _tuning
+
+    class Seen(TorchDispatchMode):
+        calls = ()
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.calls += (str(func),)
+            return func(*args, **(kwargs or {}))
+
+    class Sub(torch.Tensor):
+        pass
+
+    x = torch.randn(4, 64, device=device).to(torch.bfloat16)
+    one = torch.ones(1, device=device)
+    plain = ops._fast.fp8_quant(x, one, None, False, None)
+    assert plain is not None
+    with Seen() as seen:
+        got = ops.scaled_fp8_quant(x, one)
+    assert any("static_scaled_fp8_quant" in c for c in seen.calls)
+    assert torch.equal(got[0].view(torch.uint8), plain[0].view(torch.uint8))
+    assert ops._fast.fp8_quant(x.as_subclass(Sub), one, None, False, None) is None
+    assert ops._fast.fp8_quant(x.cpu(), one, None, False, None) is None
+    assert ops._fast.fp8_quant(x.t(), one, None, False, None) is None
+    grad = x.float().requires_grad_()
+    assert ops._fast.fp8_quant(grad, one, None, False, None) is None
+    with torch.no_grad():
+        assert ops._fast.fp8_quant(grad, one, None, False, None) is not None
+    with torch.inference_mode():
+        assert ops._fast.fp8_quant(x, one, None, False, None) is not None
+    with _tuning.override(quant_wg_per_row=1):
+        assert ops._fast.fp8_quant(x, one, None, False, None) is None
+    assert ops._fast.fp8_quant(x, one, None, False, None) is not None

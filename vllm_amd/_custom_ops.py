@@ -716,6 +716,29 @@ _register("cutlass_scaled_mm", "(Tensor! out, Tensor a, Tensor b, Tensor a_scale
 _ops = getattr(torch.ops, _NS)
 
 
+# ============================================================================ direct calls
+
+# The public functions below first try ``vllm_amd._fast_calls`` (csrc/host/fast_calls.cpp): checks, allocation and launch in
+# one C call for plain device tensors with nothing between the call and the device implementation.  It answers None, having
+# done nothing, in every other case -- bad arguments, subclasses, modes, a profiler, autograd, tuning overrides -- and the
+# call goes through the registered op.  A graph compiler sees the registered ops only.
+class _NotBuilt:
+    def __getattr__(self, name):
+        raise RuntimeError("vllm_amd/_fast_calls.so is missing or does not load: the native code is not built (run "
+                           f"`python -m vllm_amd.build`).  {_fast_error}")
+
+
+try:
+    from . import _fast_calls as _fast
+    _fast.setup(_FP8_COUNTERS, _tuning.depth, tuple(t.id for t in (scalar_types.uint4, scalar_types.uint4b8,
+                                                                   scalar_types.uint8b128, scalar_types.float8_e4m3fn)))
+except ImportError as e:
+    _fast_error = str(e)
+    _fast = _NotBuilt()
+
+_tracing = torch.compiler.is_dynamo_compiling
+
+
 # ============================================================================ public wrappers (reference signatures)
 
 def gptq_marlin_repack(b_q_weight: torch.Tensor, perm: torch.Tensor, size_k: int, size_n: int, num_bits: int, *,
@@ -742,6 +765,11 @@ def gptq_marlin_gemm(a: torch.Tensor, c: torch.Tensor | None, b_q_weight: torch.
                      b_q_type: ScalarType, size_m: int, size_n: int, size_k: int, is_k_full: bool = True,
                      use_atomic_add: bool = False, use_fp32_reduce: bool = False,
                      is_zp_float: bool = False) -> torch.Tensor:
+    if global_scale is None and not is_zp_float and not _tracing():
+        out = _fast.w4_gemm(a, c, b_q_weight, b_bias, b_scales, b_zeros, g_idx, perm, workspace, b_q_type.id, size_m, size_n,
+                            size_k, is_k_full)
+        if out is not None:
+            return out
     return _ops.gptq_marlin_gemm(a, c, b_q_weight, b_bias, b_scales, global_scale, b_zeros, g_idx, perm, workspace,
                                  b_q_type.id, size_m, size_n, size_k, is_k_full, use_atomic_add, use_fp32_reduce,
                                  is_zp_float)
@@ -756,6 +784,10 @@ def rms_norm_dynamic_per_token_quant(input: torch.Tensor, weight: torch.Tensor, 
                                      residual: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
     """RMSNorm (+ in-place residual add) and dynamic per-token quantisation in one pass (reference:
     _custom_ops.py:394-410).  Returns (quantised [.., hidden], scales [tokens, 1])."""
+    if quant_dtype == FP8_DTYPE and not _tracing():
+        pair = _fast.rms_norm_dynamic_quant(input, weight, epsilon, scale_ub, residual)
+        if pair is not None:
+            return pair
     output = torch.empty_like(input, dtype=quant_dtype)
     scales = torch.empty((input.numel() // input.shape[-1], 1), device=input.device, dtype=torch.float32)
     _ops.rms_norm_dynamic_per_token_quant(output, input, weight, scales, epsilon, scale_ub, residual)
@@ -766,18 +798,21 @@ def rms_norm_static_fp8_quant(out: torch.Tensor, input: torch.Tensor, weight: to
                               epsilon: float) -> None:
     """``out = fp8(rms_norm(input) * weight / scale)``; the reference exposes it only as ``torch.ops._C`` op
     (csrc/torch_bindings.cpp:200-205)."""
-    _ops.rms_norm_static_fp8_quant(out, input, weight, scale, epsilon)
+    if _tracing() or _fast.rms_norm_static_quant(out, input, None, weight, scale, epsilon) is None:
+        _ops.rms_norm_static_fp8_quant(out, input, weight, scale, epsilon)
 
 
 def fused_add_rms_norm_static_fp8_quant(out: torch.Tensor, input: torch.Tensor, residual: torch.Tensor,
                                         weight: torch.Tensor, scale: torch.Tensor, epsilon: float) -> None:
     """``residual += input; out = fp8(rms_norm(residual) * weight / scale)`` (csrc/torch_bindings.cpp:208-213)."""
-    _ops.fused_add_rms_norm_static_fp8_quant(out, input, residual, weight, scale, epsilon)
+    if residual is None or _tracing() or _fast.rms_norm_static_quant(out, input, residual, weight, scale, epsilon) is None:
+        _ops.fused_add_rms_norm_static_fp8_quant(out, input, residual, weight, scale, epsilon)
 
 
 def silu_and_mul_quant(out: torch.Tensor, input: torch.Tensor, scale: torch.Tensor) -> None:
     """``out = fp8(silu(input[..., :d]) * input[..., d:] / scale)`` (csrc/torch_bindings.cpp:121-123)."""
-    _ops.silu_and_mul_quant(out, input, scale)
+    if _tracing() or _fast.silu_and_mul_quant(out, input, scale) is None:
+        _ops.silu_and_mul_quant(out, input, scale)
 
 
 def scaled_fp8_quant(input: torch.Tensor, scale: torch.Tensor | None = None, num_token_padding: int | None = None,
@@ -786,6 +821,10 @@ def scaled_fp8_quant(input: torch.Tensor, scale: torch.Tensor | None = None, num
     """Quantise ``input`` [tokens, hidden] to FP8 (e4m3fn); static if ``scale`` is given, else dynamic per tensor or,
     with ``use_per_token_if_dynamic``, per token.  Rows beyond ``input.shape[0]`` of a padded output are left
     uninitialised, as in the reference."""
+    if not num_token_padding and not _tracing():
+        pair = _fast.fp8_quant(input, scale, scale_ub if scale is None else None, use_per_token_if_dynamic, output)
+        if pair is not None:
+            return pair
     assert input.ndim == 2
     shape = tuple(input.shape)
     if num_token_padding:
@@ -811,6 +850,10 @@ def scaled_fp8_quant(input: torch.Tensor, scale: torch.Tensor | None = None, num
 def cutlass_scaled_mm(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor, scale_b: torch.Tensor,
                       out_dtype: torch.dtype, bias: torch.Tensor | None = None) -> torch.Tensor:
     """``(scale_a * a) @ (scale_b * b) + bias`` with fp8 ``a`` [M,K] row-major, ``b`` [K,N] column-major, fused."""
+    if not _tracing():
+        out = _fast.scaled_mm(a, b, scale_a, scale_b, out_dtype, bias)
+        if out is not None:
+            return out
     assert out_dtype is torch.bfloat16 or out_dtype is torch.float16
     assert bias is None or bias.numel() == b.shape[1] and bias.dtype == out_dtype
     target_shape = (*a.shape[:-1], b.shape[1])
@@ -818,3 +861,28 @@ def cutlass_scaled_mm(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor, s
     out = torch.empty((a.shape[0], b.shape[1]), dtype=out_dtype, device=a.device)
     _ops.cutlass_scaled_mm(out, a, b, scale_a, scale_b, bias)
     return out.view(*target_shape)
+
+
+# ============================================================================ whole linear layers
+
+def w4a16_linear(x: torch.Tensor, b_q_weight: torch.Tensor, b_bias: torch.Tensor | None, b_scales: torch.Tensor,
+                 b_zeros: torch.Tensor | None, g_idx: torch.Tensor | None, perm: torch.Tensor | None,
+                 workspace: torch.Tensor, b_q_type: ScalarType, size_n: int, size_k: int,
+                 is_k_full: bool = True) -> torch.Tensor:
+    """``gptq_marlin_gemm`` on activations of any rank: [..., K] -> [..., N]."""
+    if not _tracing():
+        out = _fast.w4_linear(x, b_q_weight, b_bias, b_scales, b_zeros, g_idx, perm, workspace, b_q_type.id, size_n, size_k,
+                              is_k_full)
+        if out is not None:
+            return out
+    rows = x.reshape(-1, x.shape[-1])
+    out = gptq_marlin_gemm(rows, None, b_q_weight, b_bias, b_scales, None, b_zeros, g_idx, perm, workspace, b_q_type,
+                           size_m=rows.shape[0], size_n=size_n, size_k=size_k, is_k_full=is_k_full, use_fp32_reduce=True)
+    return out.reshape(x.shape[:-1] + (size_n,))
+
+
+def fp8_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor, input_scale: torch.Tensor | None,
+               scale_ub: torch.Tensor | None, out_dtype: torch.dtype, bias: torch.Tensor | None) -> torch.Tensor | None:
+    """Quantise [..., K] activations (per token, or with the given per-tensor scale) and multiply: [..., N].  None where
+    the two steps have to be taken one by one."""
+    return None if _tracing() else _fast.fp8_linear(x, weight, weight_scale, input_scale, scale_ub, out_dtype, bias)

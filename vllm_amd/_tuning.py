@@ -13,6 +13,8 @@ import threading
 from ._lib import VaqTuning
 
 _state = threading.local()
+depth = [0]      # overrides in force on any thread: while there are some, every call takes the registered ops
+_depth_lock = threading.Lock()
 
 
 def current() -> VaqTuning | None:
@@ -38,8 +40,12 @@ def override(**fields):
         else:
             setattr(t, name, int(value))
     prev = current()
+    with _depth_lock:
+        depth[0] += 1
     _state.tuning = t
     try:
         yield t
     finally:
         _state.tuning = prev
+        with _depth_lock:
+            depth[0] -= 1

@@ -10,6 +10,7 @@ import torch
 
 from ..parameter import BasevLLMParameter, PerTensorScaleParameter, _ColumnvLLMParameter
 from .quantization.base_config import LinearMethodBase, QuantizationConfig
+from .quantization.utils.quant_utils import layer_tensor
 
 
 class UnquantizedLinearMethod(LinearMethodBase):
@@ -85,7 +86,7 @@ class LinearBase(torch.nn.Module):
         self.quant_method.process_weights_after_loading(self)
 
     def forward(self, x: torch.Tensor):
-        bias = self.bias if not self.skip_bias_add else None
+        bias = layer_tensor(self, "bias") if not self.skip_bias_add else None
         output = self.quant_method.apply(self, x, bias)
         if not self.return_bias:
             return output

@@ -170,8 +170,10 @@ class AWQMarlinLinearMethod(LinearMethodBase):
             layer.bias.data = marlin_permute_bias(layer.bias.data)
 
     def apply(self, layer: torch.nn.Module, x: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
-        return apply_awq_marlin_linear(input=x, weight=layer.qweight, weight_scale=layer.scales, weight_zp=layer.qzeros,
-                                       g_idx=layer.g_idx, g_idx_sort_indices=layer.g_idx_sort_indices,
-                                       workspace=layer.workspace, quant_type=self.quant_config.quant_type,
-                                       output_size_per_partition=layer.output_size_per_partition,
-                                       input_size_per_partition=layer.input_size_per_partition, bias=bias)
+        try:
+            p = layer._parameters
+            w, scales, zeros, g_idx, perm = p["qweight"], p["scales"], p["qzeros"], p["g_idx"], p["g_idx_sort_indices"]
+        except KeyError:
+            w, scales, zeros, g_idx, perm = (layer.qweight, layer.scales, layer.qzeros, layer.g_idx, layer.g_idx_sort_indices)
+        return apply_awq_marlin_linear(x, w, scales, zeros, g_idx, perm, layer.workspace, self.quant_config.quant_type,
+                                       layer.output_size_per_partition, layer.input_size_per_partition, bias)

@@ -14,6 +14,7 @@ from vllm_amd.parameter import ModelWeightParameter, PerTensorScaleParameter
 from .base_config import LinearMethodBase, QuantizationConfig, QuantizeMethodBase
 from .input_quant_fp8 import GroupShape
 from .utils.marlin_utils_fp8 import apply_fp8_marlin_linear, prepare_fp8_layer_for_marlin
+from .utils.quant_utils import layer_tensor
 from .utils.w8a8_utils import Fp8LinearOp
 
 ACTIVATION_SCHEMES = ["static", "dynamic"]
@@ -152,9 +153,9 @@ class Fp8LinearMethod(LinearMethodBase):
             return apply_fp8_marlin_linear(input=x, weight=layer.weight, weight_scale=layer.weight_scale,
                                            workspace=layer.workspace, size_n=layer.output_size_per_partition,
                                            size_k=layer.input_size_per_partition, bias=bias)
-        return self.fp8_linear.apply(input=x, weight=layer.weight, weight_scale=layer.weight_scale,
-                                     out_dtype=self.out_dtype if x.dtype not in (torch.float16, torch.bfloat16) else x.dtype,
-                                     input_scale=layer.input_scale, bias=bias)
+        return self.fp8_linear.apply(x, layer_tensor(layer, "weight"), layer_tensor(layer, "weight_scale"),
+                                     self.out_dtype if x.dtype not in (torch.float16, torch.bfloat16) else x.dtype,
+                                     layer_tensor(layer, "input_scale"), None, bias)
 
 
 class PTPCFp8Config(Fp8Config):
@@ -199,5 +200,5 @@ class PTPCFp8LinearMethod(Fp8LinearMethod):
         layer.input_scale = None
 
     def apply(self, layer: torch.nn.Module, x: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
-        return self.fp8_linear.apply(input=x, weight=layer.weight, weight_scale=layer.weight_scale, out_dtype=x.dtype,
-                                     input_scale=None, input_scale_ub=None, bias=bias)
+        return self.fp8_linear.apply(x, layer_tensor(layer, "weight"), layer_tensor(layer, "weight_scale"), x.dtype, None, None,
+                                     bias)

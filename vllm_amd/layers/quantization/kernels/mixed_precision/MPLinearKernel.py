@@ -63,5 +63,10 @@ class MPLinearKernel(ABC):
             replace_parameter(layer, name, torch.nn.Parameter(new_param.data, requires_grad=False))
 
     def _get_weight_params(self, layer: torch.nn.Module):
+        p = layer._parameters      # (torch.nn.Module's attribute lookup costs 0.3 us per parameter and call)
+        try:
+            return p[self.w_q_name], p[self.w_s_name], p[self.w_zp_name], p[self.w_gidx_name]
+        except KeyError:
+            pass
         return (getattr(layer, self.w_q_name), getattr(layer, self.w_s_name),
                 getattr(layer, self.w_zp_name or "", None), getattr(layer, self.w_gidx_name or "", None))

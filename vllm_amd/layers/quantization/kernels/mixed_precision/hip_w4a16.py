@@ -11,7 +11,7 @@ from ...utils.marlin_utils import (HIP_W4A16_SUPPORTED_GROUP_SIZES, HIP_W8A16_SU
                                    check_marlin_supports_shape, marlin_is_k_full, marlin_make_empty_g_idx,
                                    marlin_make_workspace_new, marlin_permute_bias, marlin_permute_scales,
                                    marlin_sort_g_idx, marlin_zero_points, query_marlin_supported_quant_types)
-from ...utils.quant_utils import unpack_cols
+from ...utils.quant_utils import layer_tensor, unpack_cols
 from .MPLinearKernel import MPLinearKernel, MPLinearLayerConfig
 
 
@@ -115,8 +115,6 @@ class HipW4A16LinearKernel(MPLinearKernel):
     def apply_weights(self, layer: torch.nn.Module, x: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
         c = self.config
         w_q, w_s, w_zp, w_gidx = self._get_weight_params(layer)
-        return apply_gptq_marlin_linear(input=x, weight=w_q, weight_scale=w_s, weight_zp=w_zp, g_idx=w_gidx,
-                                        g_idx_sort_indices=layer.g_idx_sort_indices, workspace=self.workspace,
-                                        wtype=c.weight_type, input_size_per_partition=c.partition_weight_shape[0],
-                                        output_size_per_partition=c.partition_weight_shape[1],
-                                        is_k_full=self.is_k_full, bias=bias)
+        size_k, size_n = c.partition_weight_shape
+        return apply_gptq_marlin_linear(x, w_q, w_s, w_zp, w_gidx, layer_tensor(layer, "g_idx_sort_indices"), self.workspace,
+                                        c.weight_type, size_n, size_k, self.is_k_full, bias)

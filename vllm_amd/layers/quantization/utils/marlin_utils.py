@@ -196,17 +196,9 @@ def apply_gptq_marlin_linear(input: torch.Tensor, weight: torch.Tensor, weight_s
                              workspace: torch.Tensor, wtype: ScalarType, output_size_per_partition: int,
                              input_size_per_partition: int, is_k_full: bool, bias: torch.Tensor | None = None,
                              use_fp32_reduce: bool = USE_FP32_REDUCE_DEFAULT) -> torch.Tensor:
-    """marlin_utils.py:435-482."""
-    reshaped_x = input.reshape(-1, input.shape[-1])
-    out_shape = input.shape[:-1] + (output_size_per_partition,)
-    use_atomic_add = should_use_atomic_add_reduce(m=reshaped_x.size(0), n=output_size_per_partition,
-                                                  k=reshaped_x.size(1), device=input.device, dtype=input.dtype)
-    output = ops.gptq_marlin_gemm(reshaped_x, None, weight, bias, weight_scale, None, weight_zp, g_idx,
-                                  g_idx_sort_indices, workspace, wtype, size_m=reshaped_x.shape[0],
-                                  size_n=output_size_per_partition, size_k=input_size_per_partition,
-                                  is_k_full=is_k_full, use_atomic_add=use_atomic_add, use_fp32_reduce=use_fp32_reduce,
-                                  is_zp_float=False)
-    return output.reshape(out_shape)
+    """marlin_utils.py:435-482.  (The GEMM has one reduction, in fp32: `use_fp32_reduce` selects nothing.)"""
+    return ops.w4a16_linear(input, weight, bias, weight_scale, weight_zp, g_idx, g_idx_sort_indices, workspace, wtype,
+                            output_size_per_partition, input_size_per_partition, is_k_full)
 
 
 def apply_awq_marlin_linear(input: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor,
@@ -215,15 +207,8 @@ def apply_awq_marlin_linear(input: torch.Tensor, weight: torch.Tensor, weight_sc
                             input_size_per_partition: int, bias: torch.Tensor | None = None,
                             use_fp32_reduce: bool = USE_FP32_REDUCE_DEFAULT) -> torch.Tensor:
     """marlin_utils.py:485-530."""
-    reshaped_x = input.reshape(-1, input.shape[-1])
-    out_shape = input.shape[:-1] + (output_size_per_partition,)
-    use_atomic_add = should_use_atomic_add_reduce(m=reshaped_x.size(0), n=output_size_per_partition,
-                                                  k=reshaped_x.size(1), device=input.device, dtype=input.dtype)
-    output = ops.gptq_marlin_gemm(reshaped_x, None, weight, bias, weight_scale, None, weight_zp, g_idx,
-                                  g_idx_sort_indices, workspace, quant_type, size_m=reshaped_x.shape[0],
-                                  size_n=output_size_per_partition, size_k=input_size_per_partition,
-                                  use_atomic_add=use_atomic_add, use_fp32_reduce=use_fp32_reduce, is_zp_float=False)
-    return output.reshape(out_shape)
+    return ops.w4a16_linear(input, weight, bias, weight_scale, weight_zp, g_idx, g_idx_sort_indices, workspace, quant_type,
+                            output_size_per_partition, input_size_per_partition)
 
 
 def check_marlin_supports_layer(layer: torch.nn.Module, group_size: int) -> bool:

@@ -51,3 +51,9 @@ def pack_rows(q_w: torch.Tensor, num_bits: int, size_k: int, size_n: int) -> tor
 
 def gptq_pack(q_w: torch.Tensor, num_bits: int, size_k: int, size_n: int) -> torch.Tensor:
     return pack_rows(q_w, num_bits, size_k, size_n)
+
+
+def layer_tensor(layer: torch.nn.Module, name: str):
+    """``getattr(layer, name)`` without torch.nn.Module's attribute lookup, which costs 0.3 us per parameter and call."""
+    parameters = layer._parameters
+    return parameters[name] if name in parameters else getattr(layer, name)

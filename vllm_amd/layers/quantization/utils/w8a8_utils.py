@@ -32,12 +32,19 @@ class Fp8LinearOp:
         self.output_padding = None      # padding is only useful to the torch._scaled_mm fallback, which does not exist here
         self.act_quant_static = act_quant_static
         self.act_quant_group_shape = act_quant_group_shape
+        self.act_quant_per_token = act_quant_group_shape == GroupShape.PER_TOKEN
         self.quant_fp8 = QuantFP8(static=act_quant_static, group_shape=act_quant_group_shape,
                                   num_token_padding=self.output_padding)
 
     def apply(self, input: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor,
               out_dtype: torch.dtype | None = None, input_scale: torch.Tensor | None = None,
               input_scale_ub: torch.Tensor | None = None, bias: torch.Tensor | None = None) -> torch.Tensor:
+        static = self.act_quant_static
+        if input.dtype != ops.FP8_DTYPE and (input_scale is not None) == static and \
+                (input_scale_ub is None if static else self.act_quant_per_token):
+            output = ops.fp8_linear(input, weight, weight_scale, input_scale, input_scale_ub, out_dtype or input.dtype, bias)
+            if output is not None:
+                return output
         input_2d = input.view(-1, input.shape[-1])
         output_shape = [*input.shape[:-1], weight.shape[1]]
         if out_dtype is None:
