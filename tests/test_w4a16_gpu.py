@@ -93,6 +93,32 @@ def test_repack_8bit_bit_exact_both_layouts(device, k, n, act_order):
     assert np.array_equal(native.cpu().numpy(), nl.native_pack8(q_sorted)), "native order differs from its spec"
 
 
+@pytest.mark.parametrize("k,n,bits", [(20480, 64, 4), (20608, 64, 4), (10240, 128, 8), (10368, 64, 8), (128, 320, 4), (384, 192, 8)])
+@pytest.mark.parametrize("act_order", [False, True])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_repack_native_strips_and_their_limits(device, k, n, bits, act_order, offset):
+    """The strip kernels at the largest K whose 16-column strip fits LDS and one tile beyond, at column counts that are no
+    multiple of a workgroup's, and on a tensor that is not 16-byte aligned (which takes the one-word-per-thread kernel)."""
+    import vllm_amd._custom_ops as ops
+    rng = np.random.default_rng(k + n + bits)
+    q = rng.integers(0, 1 << bits, size=(k, n), dtype=np.int32)
+    perm_np = rng.permutation(k).astype(np.int32) if act_order else np.arange(k, dtype=np.int32)
+    perm = to_dev(perm_np, device) if act_order else torch.empty(0, dtype=torch.int32, device=device)
+    packed = torch.from_numpy(np.ascontiguousarray(o.gptq_pack(q, bits)))
+    buf = torch.empty(packed.numel() + offset, dtype=torch.int32, device=device)
+    qw = buf[offset:].view(packed.shape).copy_(packed.to(device))
+    want = nl.native_pack(q[perm_np]) if bits == 4 else nl.native_pack8(q[perm_np])
+    assert np.array_equal(ops.gptq_marlin_repack(qw, perm, k, n, bits).cpu().numpy(), want)
+    if bits == 4 and not act_order:
+        packed = torch.from_numpy(np.ascontiguousarray(o.awq_pack(q, 4)))
+        buf = torch.empty(packed.numel() + offset, dtype=torch.int32, device=device)
+        qw = buf[offset:].view(packed.shape).copy_(packed.to(device))
+        assert np.array_equal(ops.awq_marlin_repack(qw, k, n, 4).cpu().numpy(), want)
+    if bits == 8:
+        got = ops.gptq_marlin_repack(qw, perm, k, n, 8, layout="native_bytes")
+        assert np.array_equal(got.cpu().numpy(), nl.native_pack8_bytes(q[perm_np]))
+
+
 # ------------------------------------------------------------------------------------------------ permute_cols
 
 @pytest.mark.parametrize("m,k", [(1, 128), (3, 1024), (7, 4096), (130, 14336), (5, 70000)])

@@ -749,6 +749,10 @@ def gptq_marlin_repack(b_q_weight: torch.Tensor, perm: torch.Tensor, size_k: int
     reproduces the reference's Marlin order bit-for-bit; ``layout="native_bytes"`` (``num_bits = 8`` only) keeps whole
     bytes in the native tiles, for FP8 weights (``b_q_type = float8_e4m3fn``).  Callers treat the result as opaque.
     """
+    if perm is not None and not _tracing():
+        out = _fast.repack(b_q_weight, perm, size_k, size_n, num_bits, _LAYOUTS[layout])
+        if out is not None:
+            return out
     return _ops.gptq_marlin_repack(b_q_weight, perm, size_k, size_n, num_bits, _LAYOUTS[layout])
 
 
@@ -756,6 +760,10 @@ def awq_marlin_repack(b_q_weight: torch.Tensor, size_k: int, size_n: int, num_bi
                       layout: str = "native") -> torch.Tensor:
     """AutoAWQ int32[K, N/8] -> repacked int32[K/16, 2N] (reference: _custom_ops.py:1145-1148).  Same two layouts as
     ``gptq_marlin_repack``: ``"marlin"`` is bit-exact with the reference, ``"native"`` is what the GEMM reads."""
+    if not _tracing():
+        out = _fast.repack(b_q_weight, None, size_k, size_n, num_bits, _LAYOUTS[layout])
+        if out is not None:
+            return out
     return _ops.awq_marlin_repack(b_q_weight, size_k, size_n, num_bits, _LAYOUTS[layout])
 
 

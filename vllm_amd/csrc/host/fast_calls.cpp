@@ -516,6 +516,32 @@ PyObject* py_silu_and_mul_quant(PyObject*, PyObject* const* v, Py_ssize_t nargs)
   END_HANDLE_TH_ERRORS
 }
 
+// repack(codes, perm or None, k, n, bits, layout) -> Tensor | None; perm None: an AWQ checkpoint's tensor
+PyObject* py_repack(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 6 || !plain_thread()) return decline();
+  Call call;
+  const TensorBase* w = call.tensor(v[0]);
+  const TensorBase* perm = call.optional(v[1]);
+  if (!call.current()) return decline();
+  const int64_t k = PyLong_AsLongLong(v[2]), n = PyLong_AsLongLong(v[3]), bits = PyLong_AsLongLong(v[4]), layout = PyLong_AsLongLong(v[5]);
+  if (PyErr_Occurred() || k <= 0 || n <= 0 || k % 16 != 0 || n % 64 != 0 || (bits != 4 && bits != 8) || (!perm && bits != 4)) return decline();
+  const int64_t pack = 32 / bits;
+  if (w->scalar_type() != at::kInt || !w->is_contiguous() || w->dim() != 2 || w->size(0) != (perm ? k / pack : k) ||
+      w->size(1) != (perm ? n : n / pack))
+    return decline();
+  if (perm && (perm->scalar_type() != at::kInt || !perm->is_contiguous() || (perm->numel() != 0 && perm->numel() != k))) return decline();
+  TensorBase out = empty({k / 16, n * 16 / pack}, at::kInt, call.device);
+  const int32_t* src = (const int32_t*)w->const_data_ptr();
+  int32_t* dst = (int32_t*)out.mutable_data_ptr();
+  const int rc = perm ? vaq_w4a16_repack(src, perm->numel() ? (const int32_t*)perm->const_data_ptr() : nullptr, dst, k, n, (int)bits,
+                                         (int)layout, stream_of(call.device))
+                      : vaq_w4a16_repack_awq(src, dst, k, n, (int)bits, (int)layout, stream_of(call.device));
+  if (rc != VAQ_OK) return raise_status(rc);
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
 // setup(fp8_counters: dict, tuning_depth: list, (u4, u4b8, u8b128, fe4m3): ids)
 PyObject* py_setup(PyObject*, PyObject* args) {
   PyObject *counters, *depth;
@@ -539,7 +565,7 @@ PyObject* py_setup(PyObject*, PyObject* args) {
 PyMethodDef g_methods[] = {
     {"setup", py_setup, METH_VARARGS, nullptr},
     FAST(w4_gemm), FAST(w4_linear), FAST(scaled_mm), FAST(fp8_linear), FAST(fp8_quant), FAST(rms_norm_dynamic_quant),
-    FAST(rms_norm_static_quant), FAST(silu_and_mul_quant), {nullptr, nullptr, 0, nullptr}};
+    FAST(rms_norm_static_quant), FAST(silu_and_mul_quant), FAST(repack), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_fast_calls", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -212,6 +212,172 @@ __global__ __launch_bounds__(256) void repack_marlin8_kernel(const uint32_t* __r
   }
 }
 
+// ----------------------------------------------------------------------------- native order, whole tiles
+// The three kernels below write every output tile as the 16-byte pieces its lanes own (a wavefront store is contiguous)
+// and read the checkpoint tensor in whole 64-byte pieces or more.  Bound: HBM.  What the one-word-per-thread kernels above
+// lose is the gather: 8 four-byte loads per output word with act_order or AWQ, from lines that other workgroups fetch again.
+// They stay for the MARLIN order, for pointers that are not 16-byte aligned, and for an act_order strip beyond LDS.
+
+// OUT 0: 4-bit codes; 1: 8-bit codes as two nibble planes; 2: 8-bit codes as bytes.
+template <int OUT>
+__device__ inline void put_code(v4u (&lo)[4], v4u (&hi)[4], int c, int j, int e, uint32_t word, int shift) {
+  constexpr int pos[8] = {0, 4, 1, 5, 2, 6, 3, 7};      // nibble position of element e
+  if constexpr (OUT == 0) {
+    lo[c][j] |= ((word >> shift) & 0xFu) << (4 * pos[e]);
+  } else if constexpr (OUT == 1) {
+    const uint32_t b = word >> shift;
+    lo[c][j] |= ((b >> 4) & 0xFu) << (4 * pos[e]);      // plane 0: high nibbles
+    hi[c][j] |= (b & 0xFu) << (4 * pos[e]);
+  } else {      // lane's 16 bytes of block h = j / 2: word 2 (j & 1) + e / 4, byte e % 4
+    const uint32_t b = ((word >> shift) & 0xFFu) << (8 * (e & 3));
+    if (j < 2) lo[c][2 * (j & 1) + (e >> 2)] |= b;
+    else hi[c][2 * (j & 1) + (e >> 2)] |= b;
+  }
+}
+
+template <int OUT>
+__device__ inline void store_tile(uint32_t* __restrict__ out, int64_t tile, int lane, const v4u& lo, const v4u& hi) {
+  v4u* o = reinterpret_cast<v4u*>(out);
+  if constexpr (OUT == 0) {
+    o[tile * 64 + lane] = lo;
+  } else {
+    o[tile * 128 + lane] = lo;
+    o[tile * 128 + 64 + lane] = hi;
+  }
+}
+
+// act_order: output row k takes input row perm[k], anywhere in K.  A workgroup holds one 16-column strip of the whole
+// checkpoint tensor in LDS (K / 8 rows of 64 bytes; 8-bit: K / 4) and gathers from there.  A thread builds the pieces of four
+// lanes (o, r = 4c + q for c = 0 .. 3), so that an index is looked up and turned into an address and a shift once for
+// four columns, which one 16-byte LDS read brings: the strip is kept column-transposed (position 4q + c holds column
+// 4c + q), and the four lanes q of one store are neighbours.  Strips that share a 128-byte line run on one XCD.
+// Measured, 4096 x 28672 (4 bits, 117 MB in and out): 129 -> 29 us = 4.1 TB/s; the random rows cost LDS bank conflicts, so that it
+// stays behind the 20 us of the kernel without a permutation.
+template <int OUT>
+__global__ __launch_bounds__(1024) void repack_native_perm_kernel(const uint32_t* __restrict__ qw, const int32_t* __restrict__ perm,
+                                                                  uint32_t* __restrict__ out, int size_k, int size_n, int strips_per_xcd) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t strip[];
+  const int nt = (int)(blockIdx.x & 7) * strips_per_xcd + (int)(blockIdx.x >> 3);
+  if (nt * 16 >= size_n) return;
+  constexpr int LOG_ROWS = OUT == 0 ? 3 : 2;      // codes per word, log2
+  const int rows = size_k >> LOG_ROWS;
+  for (int i = threadIdx.x; i < rows * 4; i += blockDim.x) {
+    const int row = i >> 2, c = i & 3;
+    const v4u w = *reinterpret_cast<const v4u*>(qw + (int64_t)row * size_n + nt * 16 + 4 * c);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) strip[row * 16 + 4 * q + c] = w[q];
+  }
+  __syncthreads();
+  const int k_tiles = size_k >> 7;
+  for (int i = threadIdx.x; i < k_tiles * 16; i += blockDim.x) {
+    const int q = i & 3, o = (i >> 2) & 3, kt = i >> 4;
+    v4u lo[4] = {}, hi[4] = {};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const v4i* p = reinterpret_cast<const v4i*>(perm + kt * 128 + j * 32 + o * 8);
+      const v4i p0 = p[0], p1 = p[1];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int src = e < 4 ? p0[e & 3] : p1[e & 3];
+        const v4u w = *reinterpret_cast<const v4u*>(strip + (src >> LOG_ROWS) * 16 + 4 * q);
+        const int shift = (src & ((1 << LOG_ROWS) - 1)) * (32 >> LOG_ROWS);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) put_code<OUT>(lo, hi, c, j, e, w[c], shift);
+      }
+    }
+    const int64_t tile = (int64_t)nt * k_tiles + kt;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) store_tile<OUT>(out, tile, 16 * o + 4 * c + q, lo[c], hi[c]);
+  }
+}
+
+// GPTQ order kept: a lane's 8 codes of one word are one input word (8-bit: two).  A wavefront makes one tile, the four of
+// a workgroup neighbouring tiles of one K step (256 contiguous bytes per input row).  4096 x 28672: 20.3 us = 5.8 TB/s.
+template <int OUT>
+__global__ __launch_bounds__(256) void repack_native_rows_kernel(const uint32_t* __restrict__ qw, uint32_t* __restrict__ out, int size_k,
+                                                                 int size_n) {
+  const int lane = threadIdx.x & 63, o = lane >> 4, r = lane & 15;
+  const int nt = blockIdx.x * 4 + (threadIdx.x >> 6), kt = blockIdx.y;
+  const uint32_t* src = qw + nt * 16 + r;
+  v4u lo[1][4] = {}, hi[1][4] = {};
+  v4u (&l)[4] = lo[0];
+  v4u (&h)[4] = hi[0];
+  uint32_t w[4][OUT == 0 ? 1 : 2];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int64_t octet = (int64_t)kt * 16 + j * 4 + o;
+    if constexpr (OUT == 0) {
+      w[j][0] = src[octet * size_n];
+    } else {
+      w[j][0] = src[octet * 2 * size_n];
+      w[j][1] = src[(octet * 2 + 1) * size_n];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      put_code<OUT>(l, h, 0, j, e, OUT == 0 ? w[j][0] : w[j][e >> 2], OUT == 0 ? 4 * e : 8 * (e & 3));
+  store_tile<OUT>(out, (int64_t)nt * (size_k >> 7) + kt, lane, l[0], h[0]);
+}
+
+// AWQ: input rows are K, a word holds 8 columns of one row.  A workgroup takes 128 rows x 256 columns (whole 128-byte lines;
+// 64 columns per workgroup: 45.9 us) through LDS; a lane's output word is 8 rows' nibbles of its column.  4096 x 28672:
+// 23.4 us = 5.0 TB/s.
+__global__ __launch_bounds__(256) void repack_native_awq_kernel(const uint32_t* __restrict__ qw, uint32_t* __restrict__ out, int size_k,
+                                                                int size_n) {
+  constexpr int PITCH = 33;      // words per row: the rows of one o and of the next start in different banks
+  __shared__ uint32_t tile_in[128 * PITCH];
+  const int kt = blockIdx.y, n_words = size_n >> 3, w0 = blockIdx.x * 32;
+  const int words = n_words - w0 < 32 ? n_words - w0 : 32;      // (a multiple of 8)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = i * 32 + (threadIdx.x >> 3), c = (threadIdx.x & 7) * 4;
+    if (c < words) {
+      const v4u w = *reinterpret_cast<const v4u*>(qw + ((int64_t)kt * 128 + row) * n_words + w0 + c);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) tile_in[row * PITCH + c + q] = w[q];
+    }
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, o = lane >> 4, r = lane & 15;
+  const int shift = (((r & 1) << 2) | ((r & 7) >> 1)) * 4;
+  for (int t = threadIdx.x >> 6; 2 * t < words; t += 4) {
+    v4u lo[4] = {}, hi[4] = {};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) put_code<0>(lo, hi, 0, j, e, tile_in[(j * 32 + o * 8 + e) * PITCH + t * 2 + (r >> 3)], shift);
+    store_tile<0>(out, (int64_t)(blockIdx.x * 16 + t) * (size_k >> 7) + kt, lane, lo[0], hi[0]);
+  }
+}
+
+// Whether the kernels above take a problem: 16-byte pointers, 32-bit indexes, and with act_order a strip that fits LDS.
+constexpr int64_t REPACK_LDS_MAX = 160 * 1024;
+static bool repack_tiles_ok(const void* qweight, const void* perm, const void* out, int64_t size_k, int64_t size_n, int num_bits) {
+  if (((uintptr_t)qweight % 16) || ((uintptr_t)out % 16) || ((uintptr_t)perm % 16)) return false;
+  if (size_k > (1 << 22) || size_n > (1 << 24)) return false;
+  return !perm || size_k * 2 * num_bits <= REPACK_LDS_MAX;
+}
+
+template <int OUT>
+static int launch_repack_tiles(const uint32_t* qw, const int32_t* perm, uint32_t* out, int64_t size_k, int64_t size_n, hipStream_t s) {
+  if (!perm) {
+    hipLaunchKernelGGL(repack_native_rows_kernel<OUT>, dim3((unsigned)(size_n / 64), (unsigned)(size_k / 128)), dim3(256), 0, s, qw, out,
+                       (int)size_k, (int)size_n);
+    return VAQ_OK;
+  }
+  const size_t lds = (size_t)size_k * (OUT == 0 ? 8 : 16);
+  static size_t reserved[VAQ_MAX_DEVICES];
+  const int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(&repack_native_perm_kernel<OUT>), lds, reserved, "w4a16_repack");
+  if (rc != VAQ_OK) return rc;
+  const int per_xcd = (int)((size_n / 16 + 7) / 8);
+  // one strip per compute unit where two do not fit: then as many wavefronts as it holds
+  const int threads = lds > REPACK_LDS_MAX / 2 ? 1024 : 512;
+  hipLaunchKernelGGL(repack_native_perm_kernel<OUT>, dim3(per_xcd * 8), dim3(threads), lds, s, qw, perm, out, (int)size_k, (int)size_n, per_xcd);
+  return VAQ_OK;
+}
+
 }  // namespace vaq
 
 static int repack_common(const int32_t* qweight, const int32_t* perm, int32_t* out, int64_t size_k, int64_t size_n,
@@ -239,7 +405,16 @@ static int repack_common(const int32_t* qweight, const int32_t* perm, int32_t* o
   const uint32_t* qw = (const uint32_t*)qweight;
   uint32_t* o = (uint32_t*)out;
   const dim3 grid((unsigned)blocks), block(threads);
-  if (num_bits == 8) {
+  if (layout != VAQ_LAYOUT_MARLIN && repack_tiles_ok(qweight, perm, out, size_k, size_n, num_bits)) {
+    int rc = VAQ_OK;
+    if (awq)
+      hipLaunchKernelGGL(repack_native_awq_kernel, dim3((unsigned)((size_n + 255) / 256), (unsigned)(size_k / 128)), dim3(256), 0, s, qw, o,
+                         (int)size_k, (int)size_n);
+    else if (num_bits == 4) rc = launch_repack_tiles<0>(qw, perm, o, size_k, size_n, s);
+    else if (layout == VAQ_LAYOUT_NATIVE) rc = launch_repack_tiles<1>(qw, perm, o, size_k, size_n, s);
+    else rc = launch_repack_tiles<2>(qw, perm, o, size_k, size_n, s);
+    if (rc != VAQ_OK) return rc;
+  } else if (num_bits == 8) {
     if (layout == VAQ_LAYOUT_NATIVE) hipLaunchKernelGGL(repack_native8_kernel, grid, block, 0, s, qw, perm, o, size_k, size_n);
     else if (layout == VAQ_LAYOUT_NATIVE_BYTES) hipLaunchKernelGGL(repack_native8_bytes_kernel, grid, block, 0, s, qw, perm, o, size_k, size_n);
     else hipLaunchKernelGGL(repack_marlin8_kernel, grid, block, 0, s, qw, perm, o, size_k, size_n);
