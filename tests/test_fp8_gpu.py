@@ -457,6 +457,25 @@ def test_scaled_mm_every_tile_shape_exact(device, cfg):
         assert bool((t == 0).all()), "arrival counters not restored to zero"
 
 
+@pytest.mark.parametrize("cfg", [1, 3, 13, 6, 9, 19])
+def test_scaled_mm_slices_requested_together_exact(device, cfg):
+    """The shapes that request two slices of K at a time: step counts around the ring depth, odd ones, parts of a split K that
+    start at odd steps, and several tile rows over small weights (each starts its K loop elsewhere and wraps around)."""
+    import vllm_amd._custom_ops as ops
+    from vllm_amd import _tuning
+    g = torch.Generator().manual_seed(cfg)
+    for m, n, steps, split in ((130, 256, 3, 1), (70, 192, 4, 1), (257, 320, 5, 1), (257, 320, 6, 1), (33, 80, 11, 2), (700, 512, 21, 1),
+                               (700, 512, 22, 1), (520, 272, 23, 3), (64, 640, 46, 5), (300, 384, 33, 8)):
+        k = 64 * steps
+        a = torch.randint(-2, 3, (m, k), generator=g).float()
+        w = torch.randint(-1, 2, (n, k), generator=g).float()
+        with _tuning.override(fp8_path=2, fp8_tile_cfg=cfg, fp8_split=split):
+            out = ops.cutlass_scaled_mm(a.to(torch.float8_e4m3fn).to(device), w.to(torch.float8_e4m3fn).to(device).t(),
+                                        torch.ones(m, 1, device=device), torch.ones(n, 1, device=device), torch.float16)
+        assert torch.equal(out.cpu().float(), a @ w.t()), (cfg, m, n, k)
+    assert all(bool((t == 0).all()) for t in ops._FP8_COUNTERS.values()), "arrival counters not restored to zero"
+
+
 @pytest.mark.parametrize("m,n,k", [(17 * 256, 4096, 2048), (21 * 256 - 5, 3328, 2048)])
 def test_scaled_mm_tiles_of_last_round_split_exact(device, m, n, k):
     """More 256 x 256 tiles than compute units with a last round of workgroups at most half full (17 x 16 tiles on 256

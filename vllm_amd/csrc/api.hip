@@ -18,6 +18,7 @@ static thread_local const VaqTuning* g_tuning = nullptr;
 static const VaqTuning g_no_tuning = {};
 
 const VaqTuning& tuning() { return g_tuning ? *g_tuning : g_no_tuning; }
+bool tuning_active() { return g_tuning != nullptr; }
 TuningScope::TuningScope(const VaqTuning* t) : prev_(g_tuning) { g_tuning = t; }
 TuningScope::~TuningScope() { g_tuning = prev_; }
 

@@ -17,6 +17,8 @@
 #include "vaq_common.h"
 #include "tile_handover.h"
 
+#include <math.h>
+
 #include <type_traits>
 
 namespace vaq {
@@ -414,6 +416,12 @@ __global__ __launch_bounds__(256) void fp8_mm_tile2_kernel(const Fp8MMParams p) 
 //  * LDS rows are 64 bytes; four rows form one 256-byte line of 16 chunks (chunk index (row & 3) * 4 + c) and the chunk
 //    index is XOR-ed with (row >> 2) & 3.  The LDS has 64 banks (256 bytes per cycle): 16 lanes reading 16 consecutive
 //    rows at the same k chunk touch 16 different 16-byte bank groups;
+//  * two slices of K are requested at a time (KS = 2, or PP = 2 where the ring has no room for whole pairs), for the reason at
+//    load_slices below, and by eight wavefronts even for a 128 x 128 tile: with four a compute unit has fewer requests under
+//    way.  128 x 128 tiles, cold: 4096 x 6144 at M = 333 23.3 -> 19.5 us, 5120 x 13824 at M = 250 29.3 -> 24.3 us (cached);
+//    256 x 128: 4096 x 4096 at M = 2048 40.7 -> 35.8 us; 256 x 256: 4096 x 4096 at M = 4096 59.0 -> 56.1 us (2.45 PFLOP/s),
+//    14336 x 4096 195.5 -> 183.1 us.  Not kept: four slices at a time in two stages, K slices dealt to two groups of
+//    wavefronts of the same tile (fewer fragment reads, same time), sixteen wavefronts, four-slice stages of 64 x 64 tiles;
 //  * WAVES_M x WAVES_N wavefronts; tiles are handed out in bands of 4 tile rows inside each XCD's contiguous range so
 //    that the tiles resident on one XCD share activation rows and weight columns in its L2.
 // Requires K % 64 == 0 (a partial last step would read the neighbouring row instead of zeros) and M*lda, N*ldb < 2^32.
@@ -460,7 +468,10 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   // K may be split over workgroups: this one covers the steps [s_lo, s_hi)
   const int all_steps = p.K / (64 * KS);
-  const int s_lo = (int)(((int64_t)all_steps * sl.split) / sl.nsplit), s_hi = (int)(((int64_t)all_steps * (sl.split + 1)) / sl.nsplit);
+  // (in pairs: parts start at even steps, so that the two slices of a request share their cache lines)
+  constexpr bool PAIR = PP == 2;
+  const auto part = [&](int i) { return i >= sl.nsplit ? all_steps : (int)(((int64_t)all_steps * i) / sl.nsplit) & (PAIR ? ~1 : ~0); };
+  const int s_lo = part(sl.split), s_hi = part(sl.split + 1);
   const int steps = s_hi - s_lo;
   // Few tile rows (M at most 4 tiles high) on a device that the tiles do not fill: the tiles of one column would read
   // the same weight rows at the same time, which leaves only (ring depth x 64 KS) bytes per weight row in flight --
@@ -471,29 +482,39 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
   // of two all of them ask the same few L2 channels for the same lines at the same time.  Tile column tn starts tn / tiles_n
   // of the way into K instead (4096 x 28672 at M = 72 .. 256, cold: 33.9 .. 45.4 -> 31.1 .. 43.6 us; no change on K = 3584 or
   // 5120; with 16 tile rows it costs 3-9 %: the tiles of one column then no longer read their weights together).
-  const int rot = p.rotate_k == 1 ? (tm * steps) / tiles_m : (p.rotate_k == 2 ? (tn * steps) / tiles_n : 0);
-  auto issue_loads = [&](int step_in, int stage) {
-    int step = step_in - s_lo + rot;
-    if (step >= steps) step -= steps;
-    step += s_lo;
+  int rot = p.rotate_k == 1 ? (tm * steps) / tiles_m : (p.rotate_k == 2 ? (tn * steps) / tiles_n : 0);
+  if (PAIR) rot = steps & 1 ? 0 : rot & ~1;      // a pair never wraps around
+  // Requests for the slices from K byte `koff` on, slice i into slot(i).  The loads of neighbouring slices follow each other
+  // row by row: a row's 64-byte pieces are halves of one 128-byte line, which crosses from the L2 once when both are asked
+  // for together and twice otherwise -- and that port bounds the kernel (operands out of the L2 into LDS without any
+  // arithmetic: 30 bytes per cycle and compute unit one slice at a time, 45 in whole lines).
+  auto load_slices = [&](auto count, uint32_t koff, auto slot) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      uint8_t* Ab = lds8 + (size_t)stage * STAGE + ks * SLICE;
-      uint8_t* Bb = Ab + A_ST;
-      const uint32_t koff = (uint32_t)(step * KS + ks) * 64u;
+    for (int i = 0; i < A_LD; ++i) {
+      const int r0 = (wave * A_LD + i) * 16;
 #pragma unroll
-      for (int i = 0; i < A_LD; ++i) {
-        const int r0 = (wave * A_LD + i) * 16;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(Ab + r0 * 64), 16, (int)voff_a,
-                                                 (int)((uint32_t)(m0 + r0) * (uint32_t)p.lda + koff), 0, 0);
-      }
-#pragma unroll
-      for (int i = 0; i < B_LD; ++i) {
-        const int r0 = (wave * B_LD + i) * 16;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(Bb + r0 * 64), 16, (int)voff_b,
-                                                 (int)((uint32_t)(n0 + r0) * (uint32_t)p.ldb + koff), 0, 0);
-      }
+      for (int c = 0; c < decltype(count)::value; ++c)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(slot(c) + r0 * 64), 16, (int)voff_a,
+                                                 (int)((uint32_t)(m0 + r0) * (uint32_t)p.lda + koff + 64u * c), 0, 0);
     }
+#pragma unroll
+    for (int i = 0; i < B_LD; ++i) {
+      const int r0 = (wave * B_LD + i) * 16;
+#pragma unroll
+      for (int c = 0; c < decltype(count)::value; ++c)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(slot(c) + A_ST + r0 * 64), 16, (int)voff_b,
+                                                 (int)((uint32_t)(n0 + r0) * (uint32_t)p.ldb + koff + 64u * c), 0, 0);
+    }
+  };
+  auto k_of = [&](int step) {      // first byte of K of a step, rotation applied
+    const int rel = step - s_lo + rot;
+    return (uint32_t)((s_lo + (rel >= steps ? rel - steps : rel)) * KS) * 64u;
+  };
+  auto issue_loads = [&](int step, int stage) {
+    load_slices(std::integral_constant<int, KS>{}, k_of(step), [&](int c) { return lds8 + (size_t)stage * STAGE + c * SLICE; });
+  };
+  auto issue_pair = [&](int step, int stage, int stage2) {      // steps `step` and `step` + 1, one slice each
+    load_slices(std::integral_constant<int, 2>{}, k_of(step), [&](int c) { return lds8 + (size_t)(c ? stage2 : stage) * STAGE; });
   };
 
   v16f acc[WMB][WNB];
@@ -548,7 +569,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
 
   // Invariant at the start of step s: the tile of step s complete in LDS, the tiles of steps s+1 .. s+NST-2 requested,
   // stage (s-1) % NST free.  The requests of step s+NST-1 go out first thing in step s.
-  if (PP != 0 && steps >= NST) {
+  if (PP != 0 && steps >= NST) {      // (a pair's prologue requests NST - 1 slices)
     // Alternating phases: the two wavefronts that share a SIMD run half a step apart, so that one reads its fragments
     // (and requests tiles) while the other one issues its MFMAs.  A step is [requests, fragment reads, wait] barrier
     // [MFMAs] barrier; the late half of the workgroup passes one extra barrier first and skips its last one, so every
@@ -586,19 +607,44 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
     const bool late = wave >= NW / 2;     // wavefronts w and w + 4 share a SIMD (the other pairing measured 10-25 % slower)
     v8i af[KS][WMB], bf[KS][WNB];
 #pragma unroll
-    for (int s0 = 0; s0 < NST - 1; ++s0) issue_loads(s_lo + s0, s0);
-    sync_step(WAIT_STEADY{});           // tile 0 landed
+    for (int s0 = 0; s0 < NST - 1; ++s0) {
+      if (!PAIR) issue_loads(s_lo + s0, s0);
+      else if (!(s0 & 1)) issue_pair(s_lo + s0, s0, s0 + 1);
+    }
+    sync_step(std::integral_constant<int, (NST - (PAIR ? 3 : 2)) * LPW>{});      // the first tile (pair) landed
     if (late) bare_barrier();
     int cur = 0, dst = NST - 1;
     int step = 0;
-    for (; step + NST - 1 < steps; ++step) {
-      issue_loads(s_lo + step + NST - 1, dst);
-      read_frags(cur, af, bf);
-      sync_step(WAIT_STEADY{});
-      mfmas(af, bf);
-      bare_barrier();
-      cur = cur + 1 == NST ? 0 : cur + 1;
-      dst = dst + 1 == NST ? 0 : dst + 1;
+    auto next = [](int stage) { return stage + 1 == NST ? 0 : stage + 1; };
+    if constexpr (PAIR) {
+      // Slices NST - 2 and NST - 1 ahead are requested together in every odd step, into the two stages that are free then;
+      // what has to be in LDS at the end of its read phase is everything but that pair, and after an even step nothing new.
+      static_assert(KS == 1 && (NST & 1), "one stage more than whole pairs");
+      for (; step + NST < steps; step += 2) {
+        read_frags(cur, af, bf);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        mfmas(af, bf);
+        bare_barrier();
+        cur = next(cur);
+        issue_pair(s_lo + step + NST - 1, dst, next(dst));
+        read_frags(cur, af, bf);
+        sync_step(std::integral_constant<int, (NST - 3) * LPW>{});
+        mfmas(af, bf);
+        bare_barrier();
+        cur = next(cur);
+        dst = next(next(dst));
+      }
+      if (step + NST - 1 < steps) issue_loads(s_lo + step + NST - 1, dst);      // an odd last slice: its stage is free already
+    } else {
+      for (; step + NST - 1 < steps; ++step) {
+        issue_loads(s_lo + step + NST - 1, dst);
+        read_frags(cur, af, bf);
+        sync_step(WAIT_STEADY{});
+        mfmas(af, bf);
+        bare_barrier();
+        cur = next(cur);
+        dst = next(dst);
+      }
     }
     for (; step < steps; ++step) {      // nothing left to request: drain
       read_frags(cur, af, bf);
@@ -1031,8 +1077,8 @@ static int launch_tile3(const Fp8MMParams& p, hipStream_t s) {
 }
 
 struct Fp8TilePlan {
-  int cfg, sk, bm, bn, nw;
-  int64_t tiles;
+  int cfg = -1, sk = 1, bm = 0, bn = 0, nw = 0;
+  int64_t tiles = 0;
   int64_t tail_first = 0;      // > 0: only the tiles from this position on are split (tile_handover.h)
   int64_t extra_tiles = 0;     // split K: the tiles of a tile row past M that runs beside the real ones (see m_tiles_extra in dispatch_tile)
   // scratch of the K split: partial tiles and arrival counters of the tiles that are split
@@ -1041,215 +1087,105 @@ struct Fp8TilePlan {
   int64_t counter_ints() const { return split_tiles() * nw; }
 };
 
-// Tile shape and K split of the multi-stage kernel.  K is split when the output tiles alone leave compute units idle,
-// at most 8 ways; the rules for large and small tiles are below, each measured with cold weights.
-static Fp8TilePlan plan_tile3(int M, int N, int K) {
-  const int cus = num_cus_current_device();
-  auto tiles = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  Fp8TilePlan pl;
-  pl.cfg = tuning().fp8_tile_cfg;
-  // the largest tile shape that fills 70 % of the compute units (measured on the Llama shapes, M = 256 .. 4096: a
-  // partly filled device of large tiles beats a full one of small tiles by 25-40 %); for 128 x 128 also when two
-  // parts of a long K get it there (14336 x 4096 at M = 512, cold, 73 -> 62 us)
-  // ... and for 256 x 256 when two parts of a very long K do (14336 x 4096 at M = 1536 / 2048, cold: 139 / 145 -> 116 / 130 us;
-  // 4096 x 4096 at M = 2048 in two parts: 45 -> 66 us)
-  // (256 x 256 from 55 % of the compute units on, 50 % in two parts of a long K: 4096 x 6144 at M = 1408 .. 1792 70 ->
-  // 49 .. 55 us, 4096 x 4096 at M = 2304 / 2560 70 -> 54 us, 14336 x 4096 at M = 1024 / 1280 89 / 132 -> 79 / 105 us;
-  // at 47-50 % on a short K the smaller tiles win, 4096 x 4096 at M = 2048 45 against 53 us)
-  const int parts128 = K / 64 >= 128 ? 2 : 1;
-  const int parts256 = K / 64 >= 160 ? 2 : 1;      // (11008 x 4096 at M = 2048 in two parts: 115 -> 98 us)
-  // 128 x 128 also from half a device's worth of tiles on a long K (14336 x 4096 at M = 160 / 224: 42 -> 35 us), and
-  // wherever the 64 x 128 tiles (one workgroup per compute unit) would need a second round and these do not
-  // (4096 x 6144 at M = 384: 39 -> 27 us; 4096 x 4096 at M = 640: 38.5 -> 28 us)
-  const bool take128 = tiles(128, 128) * parts128 * 10 >= cus * (parts128 == 2 ? 5 : 7) ||
-                       (tiles(64, 128) > cus && tiles(128, 128) <= cus);
-  // ... and when the K parts that 256 x 256 tiles get, counted only down to 40 steps, bring them to 60 % of the compute units
-  // and M fills 80 % of their rows (cold: 18944 x 3584 at M = 640 .. 1024, 42 / 56 tiles in 4 parts, 94 .. 101 -> 76 .. 84 us;
-  // 8192 x 8192 at M = 640 / 768, 96 tiles in 2 parts, 84 / 81 -> 62 / 70 us; 14336 x 4096 at M = 640 / 768 79 -> 64 / 71 us;
-  // parts of 32 steps lose 5 %, 8192 x 8192 at M = 512; rows filled to 75 % lose 15 %, 13824 x 5120 at M = 384)
-  auto long_k_256 = [&]() {
-    const int64_t t = tiles(256, 256);
-    if (t >= cus || t < 1) return false;
-    // the parts these tiles would get below, of those only parts of at least 40 steps
-    const int min_steps = t * 4 <= cus ? 32 : 64;
-    int sk = (int)((int64_t)cus / t);
-    if (sk > 8) sk = 8;
-    if (sk > K / 64 / min_steps) sk = K / 64 / min_steps;
-    if (sk < 1) sk = 1;
-    while (sk & (sk - 1)) --sk;
-    while (sk > 1 && K / 64 / sk < 40) sk /= 2;
-    // (rows filled to 80 %; to 70 % from three tile rows on, where the poorly filled row is a third of the tiles or less:
-    // 14336 x 4096 at M = 544 .. 608, cold, 74 .. 76 -> 61 .. 62 us)
-    const int64_t rows256 = (M + 255) / 256;
-    const bool filled = (int64_t)M * 5 >= rows256 * 256 * 4 || (rows256 >= 3 && (int64_t)M * 10 >= rows256 * 256 * 7);
-    return t * sk * 10 >= (int64_t)cus * 6 && filled;
-  };
-  const bool take256 = tiles(256, 256) * parts256 * 20 >= cus * (parts256 == 2 ? 10 : 11) || long_k_256();
-  // (not when M fills less than 70 % of the 256-row tiles and the 128 x 256 tiles fit the device in one round: 3584 x 18944
-  // at M = 288 / 320, 222 tiles, 47.4 -> 41.3 us; on 4096 x 28672, 336 tiles, the 256 x 256 tiles stay ahead, 53 against 75 us)
-  const bool rows_poorly_filled = (int64_t)M * 10 < (int64_t)((M + 255) / 256) * 256 * 7 && tiles(128, 256) <= cus &&
-                                  tiles(128, 256) * 10 >= cus * 7 && tuning().exp[9] != 1;
-  // (128 x 256 from 70 % of the compute units on.  Between 55 and 70 % they win on weights that are already cached -- 4096 x
-  // 6144 at M = 768, 144 tiles, 40.5 -> 36.1 us -- and lose on cold ones, 36.1 against 42.5 us for the 128 x 128 tiles: a
-  // layer's weights are cold when its turn comes, so the cold figure decides.)
-  if (pl.cfg <= 0)
-    pl.cfg = take256 && !rows_poorly_filled ? 1 : (tiles(128, 256) * 10 >= cus * 7 ? 7 : (take128 ? 3 : 4));
-  // One tile row of 129 .. 256 rows on a wide layer: 256 x 128 tiles (8 wavefronts of 64 x 64) from 55 % of the compute units
-  // up to one round -- as many tiles as 128 x 256 ones, but every weight row is read by one workgroup only (cold:
-  // 4096 x 28672 at M = 224 / 256 49.7 / 51.9 -> 45.0 / 47.0 us, 3584 x 18944 at M = 136 .. 256 37.5 .. 46.3 -> 31.2 .. 39.1 us,
-  // 8192 x 28672 at M = 256 97.9 -> 85.7 us; at 42-44 % of the units, 5120 x 13824 and 4096 x 14336, the 128 x 128 tiles
-  // stay ahead by 6-10 %)
-  if (tuning().fp8_tile_cfg <= 0 && M > 128 && M <= 256 && tiles(256, 128) <= cus && tiles(256, 128) * 20 >= (int64_t)cus * 11)
-    pl.cfg = 9;
-  // 256 x 384 tiles (wavefronts of 128 x 96) where the 256 x 256 tiles leave the last round of workgroups badly filled and
-  // these do not: 4096 x 6144 at M = 4096 is 384 tiles = 1.5 rounds, or 256 = one round (101.4 -> 92.3 us).  Per tile they
-  // are slower (4096 x 4096 at M = 4096: 62.8 against 72.7 us), so only for a gain of a fifth in the fill of the rounds.
-  if (tuning().fp8_tile_cfg <= 0 && pl.cfg == 1 && N % 384 == 0 && K / 64 < 160) {
-    auto fill = [&](int64_t t) { return (double)t / (double)(((t + cus - 1) / cus) * cus); };
-    if (tiles(256, 256) > cus && fill(tiles(256, 384)) >= 1.2 * fill(tiles(256, 256))) pl.cfg = 10;
-  }
-  // the smallest tile with two k-slices per step: 5-8 % faster on a short K (half the barriers), no gain on a long one
-  if (tuning().fp8_tile_cfg <= 0 && pl.cfg == 4 && K % 128 == 0 && K <= 8192) pl.cfg = 14;
-  // 64 x 64 tiles while they fit the device in one round, on a short K: twice the workgroups with loads in flight
-  // (cold weights: 4096 x 6144 at M = 128 21.8 -> 15.0 us, 4096 x 4096 at M = 192 19.8 -> 13.8 us; 14336 x 4096 at
-  // M = 128 30.0 -> 34.0 us, and slower as soon as the tiles need a second round)
-  if (tuning().fp8_tile_cfg <= 0 && pl.cfg == 14 && tiles(64, 64) <= cus) pl.cfg = 15;
-  // 128 x 64 tiles where the 64 x 64 ones need a second round: up to three tile rows, each weight row read by one workgroup
-  // per tile row as with the 64 x 64 tiles, when they leave compute units for one more row of workgroups past M (see
-  // m_tiles_extra in dispatch_tile), or are more workgroups than the 64 x 128 tiles while the last tile row holds at most
-  // 32 rows of M.  Cold: 4096 x 4096 at M = 264 .. 384 18.0 .. 18.6 -> 15.2 .. 15.5 us, 5120 x 5120 at M = 200 .. 288 22.5 .. 24.2
-  // -> 19.6 .. 20.3 us, 3584 x 4608 at M = 200 / 256 16.7 / 16.9 -> 13.9 / 14.0 us, 6656 x 6656 at M = 136 31.0 -> 24.4 us,
-  // 4096 x 6144 at M = 136 / 160 19.0 -> 15.4 / 16.3 us and at M = 176 / 192, 48 / 64 rows in the last tile row, 19.1 -> 20.0 us;
-  // with as many workgroups as the 64 x 128 tiles and no room for the row past M they lose 6 % (4096 x 6144 at M = 256).
-  if (tuning().fp8_tile_cfg <= 0 && pl.cfg == 14 && K <= 6656 && M <= 384 && tiles(128, 64) <= cus && tuning().exp[14] != 1) {
-    const int64_t t = tiles(128, 64), cols = (N + 63) / 64;
-    const int last_rows = M - (M - 1) / 128 * 128;
-    if (t + cols <= (int64_t)cus || (t > tiles(64, 128) && last_rows <= 32)) pl.cfg = 16;
-  }
-  if (pl.cfg >= 10 && K % 128 != 0) pl.cfg %= 10;      // two k-slices per step need K % 128 == 0
-  int sk = 1;
+// The tile shapes of the multi-stage kernel and what a launch of each costs, in us: a workgroup takes `base` plus, per 64-byte
+// step of K, `step` + `load` * (share of the device that runs beside it, up to `slots` workgroups per compute unit).  Fitted to
+// 1553 problems with M = 9 .. 8192, K = 1024 .. 16384, N = 1024 .. 28672 drawn over the logarithm, every shape and K split of
+// each timed on cold weights (some 20000 launches; 7.6 % rms).  The plan with the least predicted time is on average
+// 0.8 % slower than the fastest of all plans of a problem, where the rules by size that it replaces were 11 % slower at M = 33 .. 1024.
+// (4096 x 13824 at M = 384 49 -> 33 us, 8192 x 4096 at M = 180 25 -> 19 us, 14336 x 2048 at M = 384 39 -> 27 us.)
+struct Fp8TileShape {
+  int cfg, bm, bn, nw, slots;      // cfg: id for K % 128 == 0; the two-slice shapes have one with a slice per step, id - 10
+  double base, step, load;
+};
+constexpr Fp8TileShape FP8_TILE_SHAPES[] = {
+    {13, 128, 128, 8, 1, 2.24, 0.192, 0.121}, {14, 64, 128, 4, 1, 1.75, 0.172, 0.090}, {15, 64, 64, 4, 2, 0.86, 0.103, 0.043},
+    {16, 128, 64, 4, 1, 1.75, 0.152, 0.048},  {17, 128, 256, 8, 1, 4.81, 0.344, 0.160}, {19, 256, 128, 8, 1, 4.55, 0.311, 0.124},
+    {1, 256, 256, 8, 1, 10.46, 0.476, 0.218}, {10, 256, 384, 8, 1, 22.66, 0.580, 0.451}};
+constexpr double FP8_SHARED_UNIT = 0.107;      // us per step where two workgroups share a compute unit
+constexpr double FP8_WEIGHT_US_PER_MB = 0.204; // cold weights arrive no faster than this
+// hand-over of a K split: fixed, per part, per MB of partial tiles
+constexpr double FP8_HANDOVER_US = 2.56, FP8_HANDOVER_US_PER_PART = 0.725, FP8_HANDOVER_US_PER_MB = 0.184;
+
+static Fp8TilePlan make_plan_tile3(int M, int N, int K) {
+  const int64_t cus = num_cus_current_device();
   const int steps = K / 64;
-  Fp8TilePlan saved = pl;
-  for (int pass = 0; pass < 2; ++pass) {
-  sk = 1;
-  switch (pl.cfg) {
-    case 3: case 13: case 23: pl.bm = 128; pl.bn = 128; pl.nw = 4; break;
-    case 4: case 14: case 24: pl.bm = 64; pl.bn = 128; pl.nw = 4; break;
-    case 5: case 15: pl.bm = 64; pl.bn = 64; pl.nw = 4; break;
-    case 16: pl.bm = 128; pl.bn = 64; pl.nw = 4; break;
-    case 7: case 17: pl.bm = 128; pl.bn = 256; pl.nw = 8; break;
-    case 9: pl.bm = 256; pl.bn = 128; pl.nw = 8; break;
-    case 2: pl.bm = 256; pl.bn = 256; pl.nw = 4; break;
-    case 10: case 11: pl.bm = 256; pl.bn = 384; pl.nw = 8; break;
-    default: pl.bm = 256; pl.bn = 256; pl.nw = 8; break;
-  }
-  pl.tiles = tiles(pl.bm, pl.bn);
-  if (pl.tiles < cus && pl.bm * pl.bn >= 128 * 256) {
-    // large tiles, one workgroup per compute unit
-    const int min_steps = pl.tiles * 4 <= cus ? 32 : 64;        // shorter parts only when the tiles leave 3/4 of the device idle
-    sk = (int)((int64_t)cus / pl.tiles);
-    if (sk > 8) sk = 8;
-    if (sk > steps / min_steps) sk = steps / min_steps;
-    if (sk < 1) sk = 1;
-    while (sk & (sk - 1)) --sk;       // a power of two (3 splits measured slower than 2)
-  } else if (pl.tiles < cus) {
-    // Small tiles (two workgroups share a compute unit), measured with cold weights on the Llama shapes, M = 48 .. 512:
-    // tiles that leave 2/3 of the device idle are split until there is about one workgroup per compute unit (parts of
-    // at least 16 steps: 4096 x 4096 at M = 128, 4 parts of 16 steps 15.7 us, 2 of 32 18.4 us, 8 of 8 22.7 us); fuller
-    // devices stay unsplit (the rotated K loop of the unsplit kernel is worth more there: 4096 x 6144 at M = 192,
-    // 20.8 against 31.0 us in 2 parts; 96 tiles in 2 parts: -3 % on 4096 x 6144, +6 % on 4096 x 4096) unless K is very
-    // long, where a part is halved while the halves stay 50 steps long and the workgroups fit the device at once
-    // (14336 x 4096 at M = 256: 62.6 / 45.8 / 44.3 us in 1 / 2 / 4 parts).
-    if (pl.tiles * 3 <= (int64_t)cus) {
-      sk = (int)((int64_t)cus / pl.tiles);
-      if (sk > 8) sk = 8;
-      // (parts of at least 16 steps; 32 between 1/4 and 1/3 of the device: 5120 x 5120 at M = 64, 80 tiles in two parts
-      // of 40 steps, 22.8 -> 18.2 us; 2560 x 2560 at M = 128 in two parts of 20, 11.5 -> 12.3 us)
-      const int min_part = pl.tiles * 4 <= (int64_t)cus ? 16 : 32;
-      if (sk > steps / min_part) sk = steps / min_part;
-      if (sk < 1) sk = 1;
-      while (sk & (sk - 1)) --sk;
-      // (two tile rows and more of a short K stay whole: their tile rows start at different K steps, which parts of 16
-      // steps and a hand-over do not beat -- 2048 x 2048 at M = 72 .. 128, 64 tiles: 9.7 .. 10.6 us in two parts, 7.5 .. 8.6 us
-      // whole, 3072 x 1024 at M = 128 11.8 against 11.0 us; from 56 steps on the parts are ahead, 3584 x 2048 at M = 128: 11.9
-      // against 12.8 us, 4096 x 2048: 12.4 against 13.1 us)
-      if (M > pl.bm && steps < 56) sk = 1;
+  const VaqTuning& tn = tuning();
+  Fp8TilePlan best;
+  double best_us = -1;
+  // `part_tiles` tiles in `sk` parts beside `whole_rounds` rounds of whole ones
+  auto consider = [&](const Fp8TileShape& t, int64_t tiles, int sk, int64_t tail_first) {
+    const int64_t split_tiles = tail_first > 0 ? tiles - tail_first : tiles, cap = cus * t.slots;
+    const int64_t rounds = tail_first > 0 ? tail_first / cus : tiles * sk / cap;
+    const double rest = (double)(tail_first > 0 ? split_tiles * sk : tiles * sk % cap) / (double)cus;
+    const double part = (double)steps / sk, whole = tail_first > 0 ? (double)steps : part;
+    double us = (double)rounds * (t.base + whole * (t.step + t.load * t.slots + (t.slots > 1 ? FP8_SHARED_UNIT : 0)));
+    if (rest > 0) us += t.base + part * (t.step + t.load * rest + (rest > 1 ? FP8_SHARED_UNIT : 0));
+    const double mem = FP8_WEIGHT_US_PER_MB * 1e-6 * (double)N * K;
+    us = sqrt(sqrt(us * us * us * us + mem * mem * mem * mem)) + 2.0;
+    if (sk > 1)
+      us += FP8_HANDOVER_US + FP8_HANDOVER_US_PER_PART * sk + FP8_HANDOVER_US_PER_MB * 4e-6 * (double)(split_tiles * t.bm * t.bn) * sk;
+    // (a handful of left-over tiles: the estimate is 7 % high there, 2048 x 4096 at M = 4352 58.7 against 54.9 us)
+    if (tail_first > 0 && split_tiles * 8 <= cus) us *= 0.9;
+    if (best_us >= 0 && us >= best_us) return;
+    if ((uint64_t)sk * (uint64_t)split_tiles * t.bm * t.bn * 4 >= (1ull << 32) && sk > 1) return;      // 32-bit buffer offsets
+    best_us = us;
+    best.bm = t.bm; best.bn = t.bn; best.nw = t.nw;
+    best.tiles = tiles;
+    best.sk = sk;
+    best.tail_first = tail_first;
+    best.cfg = tn.fp8_tile_cfg > 0 ? tn.fp8_tile_cfg : (t.cfg > 10 && K % 128 != 0 ? t.cfg - 10 : t.cfg);
+  };
+  for (const Fp8TileShape& t : FP8_TILE_SHAPES) {
+    if (tn.fp8_tile_cfg > 0 ? tn.fp8_tile_cfg != t.cfg && tn.fp8_tile_cfg != t.cfg - 10 : t.cfg == 10 && N % 384 != 0) continue;
+    const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    const int64_t rest = tiles % cus;
+    if (tn.fp8_split > 0) {
+      consider(t, tiles, tn.fp8_split <= steps ? tn.fp8_split : steps, 0);
+      continue;
     }
-    while (sk < 8 && steps / sk >= 100 && pl.tiles * sk * 2 <= 2 * (int64_t)cus) sk *= 2;
-    // between one and 1.75 workgroups per compute unit some units run two of them and set the pace: the parts that give
-    // one per unit instead, unless they get longer than 128 steps (13824 x 5120 at M = 65 .. 256, 80 tiles: 320 workgroups
-    // 41 .. 57 us, 240 workgroups 33 .. 42 us; 6656 x 6656 at M = 65, 208 tiles of 64 x 64: 20.8 -> 17.7 us unsplit;
-    // 17920 x 6656 at M = 512, 208 tiles: 97 us in two parts of 140 steps, 105 us unsplit)
-    const int64_t wgs = pl.tiles * sk;
-    if (sk > 1 && wgs > cus && wgs * 4 < (int64_t)cus * 7) {
-      const int fit = (int)((int64_t)cus / pl.tiles);
-      // (an unsplit K, which also saves the hand-over, from 60 % of the units on -- 6656 x 6656 at M = 136 / 192, 156 tiles:
-      // 41 / 45 -> 33 us, 7680 x 7680 47 / 51 -> 40 us; fewer parts from 90 % on -- 14336 x 4096
-      // at M = 384, 96 tiles: 4 parts 52.0 us, 2 parts 54.8 us)
-      const int64_t filled = (int64_t)fit * pl.tiles;
-      if (fit >= 1 && steps / fit <= 128 && (fit == 1 ? filled * 5 >= (int64_t)cus * 3 : filled * 10 >= (int64_t)cus * 9)) sk = fit;
-    }
-    // Up to three tile rows of K <= 6656 with compute units left for one more row of workgroups stay whole: that row
-    // then runs past M beside them (see m_tiles_extra in dispatch_tile), which parts and their hand-over do not beat:
-    // 5120 x 5120 at M = 40 .. 128 14.2 .. 18.4 -> 13.2 us, 6656 x 6656 at M = 40 / 64 17.7 / 20.7 -> 16.0 / 16.7 us, 4096 x 2048 at
-    // M = 192 12.6 -> 10.6 us; on K = 7168 and 8192 the parts stay ahead, 8192 x 3584 at M = 64 15.7 against 17.8 us.
-    {
-      const int64_t rows = (M + pl.bm - 1) / pl.bm;
-      if (K <= 6656 && rows <= 3 && pl.tiles + pl.tiles / rows <= (int64_t)cus && tuning().exp[13] != 1) sk = 1;
-    }
+    // K in up to 8 parts of at least 8 steps, on up to 2.3 rounds of workgroups
+    for (int sk : {1, 2, 3, 4, 6, 8})
+      if (sk == 1 || (steps / sk >= 8 && tiles * sk * 10 <= cus * 23)) consider(t, tiles, sk, 0);
+    // 256 x 256 tiles that end in a round of workgroups at most half full: the tiles of that round in parts of at least 16
+    // steps that fill it, the others whole
+    if (t.cfg == 1 && tiles > cus && rest > 0 && tn.exp[10] != 1)
+      for (int sk : {2, 3, 4})
+        if (rest * sk <= cus && steps / sk >= 16) consider(t, tiles, sk, tiles - rest);
   }
-  // 64 x 128 tiles of a long K whose parts still run 64 steps and more: 128 x 128 tiles instead -- half the tiles, so twice
-  // the parts of half the length on the same number of workgroups (cold, M = 80 .. 128: 18944 x 3584 33.8 -> 31.7 us,
-  // 9216 x 4608 30.7 -> 25.9 us, 17920 x 6656 52.6 -> 42.2 us, 24576 x 6144 71.7 -> 61.1 us; M = 136 .. 256: 12288 x 3072
-  // 41 -> 32 us; with parts of 56 steps and less they lose 1-9 %: 14336 x 4096, 11008 x 4096, 10240 x 2560)
-  // -- where those are fewer tiles (M beyond one 64-row block) and come to at least 80 % of the workgroups, or of the compute
-  // units if the 64 x 128 tiles exceed them (13824 x 5120, 20480 x 5120: 240 against 160 workgroups, +3 .. +9 %)
-  if (pass == 0 && tuning().fp8_tile_cfg <= 0 && tuning().fp8_split <= 0 && pl.cfg == 4 && steps / sk >= 64 &&
-      tiles(128, 128) < pl.tiles) {
-    saved = pl;
-    saved.sk = sk;
-    pl.cfg = 3;
-    continue;
+  if (best_us < 0) {      // an unknown id was forced: the caller's other kernels take the problem
+    best = Fp8TilePlan{};
+    best.cfg = -1;
+    best.sk = 1;
+    return best;
   }
-  if (pass == 1) {
-    const int64_t w4 = saved.tiles * saved.sk < cus ? saved.tiles * saved.sk : cus;
-    if (pl.tiles * sk * 10 < w4 * 8) {      // too few workgroups: back to the 64 x 128 plan
-      pl = saved;
-      sk = saved.sk;
-    }
-  }
-  break;
-  }
-  // 256 x 256 tiles (one workgroup per compute unit) whose count ends in a round of workgroups that is at most half full:
-  // the tiles of that round are split over K so that their parts fill it, the others stay whole.  Parts of at least 16
-  // steps.  (The gain is less than the rounds saved: a half-empty round runs faster per workgroup than a full one -- the
-  // device is power-limited -- and the parts' hand-over costs 10-15 us.)
-  pl.tail_first = 0;
-  if (sk == 1 && pl.bm == 256 && pl.bn == 256 && pl.nw == 8 && pl.tiles > cus && tuning().exp[10] != 1 && tuning().fp8_split <= 0) {
-    const int64_t rest = pl.tiles % cus;
-    if (rest > 0 && rest * 2 <= cus && steps >= 32 && (steps >= 128 || rest * 8 <= cus || tuning().exp[10] == 2)) {
-      int parts = (int)(cus / rest);
-      if (parts > 4) parts = 4;
-      if (parts > steps / 16) parts = steps / 16;
-      if (parts >= 2) {
-        sk = parts;
-        pl.tail_first = pl.tiles - rest;
-      }
-    }
-  }
-  if (tuning().fp8_split > 0) sk = tuning().fp8_split <= steps ? tuning().fp8_split : steps;
-  while (sk > 1 && (uint64_t)sk * (uint64_t)(pl.tiles - pl.tail_first) * pl.bm * pl.bn * 4 >= (1ull << 32)) --sk;   // 32-bit buffer offsets
-  pl.sk = sk;
-  if (sk == 1) pl.tail_first = 0;
+  if (best.cfg > 10 && K % 128 != 0) best.cfg -= 10;
   // A split K with compute units left for the parts of one more tile row: that row runs past M beside the real ones, as
   // with an unsplit K (see m_tiles_extra in dispatch_tile); its workgroups take no part in the hand-over, but tile
   // positions -- and with them the places in the scratch -- count it.  Cold: 7168 x 2048 at M = 40 / 64 / 192 12.1 / 13.6 /
   // 18.0 -> 10.3 / 10.4 / 12.8 us, 8192 x 1024 at M = 40 .. 192 12.4 .. 13.2 -> 10.7 .. 11.0 us.
-  if (sk > 1 && pl.tail_first == 0 && tuning().exp[13] != 1) {
-    const int64_t rows = (M + pl.bm - 1) / pl.bm, cols = pl.tiles / rows;
-    if (rows <= 3 && (pl.tiles + cols) * sk <= (int64_t)cus) pl.extra_tiles = cols;
+  if (best.sk > 1 && best.tail_first == 0 && tn.exp[13] != 1) {
+    const int64_t rows = (M + best.bm - 1) / best.bm, cols = best.tiles / rows;
+    if (rows <= 3 && (best.tiles + cols) * best.sk <= cus) best.extra_tiles = cols;
   }
-  return pl;
+  return best;
+}
+
+// The plan of a problem, kept for the next call on it (weighing 50 plans takes 2 us of host time): one small table per
+// thread, replaced on collision; calls with overrides neither read nor fill it.
+static Fp8TilePlan plan_tile3(int M, int N, int K) {
+  struct Entry {
+    int m = -1, n = 0, k = 0, cus = 0;
+    Fp8TilePlan plan;
+  };
+  static thread_local Entry table[64];
+  if (tuning_active()) return make_plan_tile3(M, N, K);
+  const int cus = num_cus_current_device();
+  Entry& e = table[((uint32_t)M * 2654435761u ^ (uint32_t)N * 2246822519u ^ (uint32_t)K * 3266489917u) >> 26];
+  if (e.m != M || e.n != N || e.k != K || e.cus != cus) {
+    e.plan = make_plan_tile3(M, N, K);
+    e.m = M; e.n = N; e.k = K; e.cus = cus;
+  }
+  return e.plan;
 }
 
 template <bool BF16_OUT>
@@ -1266,7 +1202,7 @@ static int dispatch_tile(const Fp8MMParams& p_in, int64_t c_tmp_bytes, int64_t c
     if (pl.sk == 1) pl.tail_first = 0;
     p.SK = pl.sk;
     p.tail_first = (int)pl.tail_first;
-    {
+    if (pl.cfg > 0) {
       const int64_t tiles_m = (p.M + pl.bm - 1) / pl.bm;
       const int64_t cus = num_cus_current_device();
       // (with K split over workgroups the rotation gains nothing on cold weights and costs 20-30 % on cached ones.)
@@ -1303,24 +1239,21 @@ static int dispatch_tile(const Fp8MMParams& p_in, int64_t c_tmp_bytes, int64_t c
       }
     }
     switch (pl.cfg) {
-      case 1: return launch_tile3<BF16_OUT, 256, 256, 2, 4, 5, 1, 1>(p, s);   // alternating phases (see the kernel)
-      case 8: return launch_tile3<BF16_OUT, 256, 256, 2, 4, 5>(p, s);
-      case 2: return launch_tile3<BF16_OUT, 256, 256, 2, 2, 5>(p, s);
+      case 1: return launch_tile3<BF16_OUT, 256, 256, 2, 4, 5, 1, 2>(p, s);    // alternating phases, slices requested in pairs (see the kernel)
       case 10: return launch_tile3<BF16_OUT, 256, 384, 2, 4, 4, 1, 1>(p, s);   // 8 wavefronts of 128 x 96, alternating phases
-      case 11: return launch_tile3<BF16_OUT, 256, 384, 2, 4, 4>(p, s);
-      case 3: return launch_tile3<BF16_OUT, 128, 128, 2, 2, 5>(p, s);
-      case 4: return launch_tile3<BF16_OUT, 64, 128, 2, 2, 5>(p, s);
-      case 6: return launch_tile3<BF16_OUT, 256, 256, 2, 4, 3>(p, s);
-      case 7: return launch_tile3<BF16_OUT, 128, 256, 2, 4, 5>(p, s);
       // two k-slices per step (K % 128 == 0)
-      case 13: return launch_tile3<BF16_OUT, 128, 128, 2, 2, 4, 2>(p, s);
-      case 23: return launch_tile3<BF16_OUT, 128, 128, 2, 2, 2, 2>(p, s);
+      case 13: return launch_tile3<BF16_OUT, 128, 128, 2, 4, 4, 2>(p, s);
       case 14: return launch_tile3<BF16_OUT, 64, 128, 2, 2, 5, 2>(p, s);
-      case 24: return launch_tile3<BF16_OUT, 64, 128, 2, 2, 3, 2>(p, s);
       case 15: return launch_tile3<BF16_OUT, 64, 64, 2, 2, 5, 2>(p, s);
-      case 5: return launch_tile3<BF16_OUT, 64, 64, 2, 2, 5>(p, s);
       case 16: return launch_tile3<BF16_OUT, 128, 64, 2, 2, 5, 2>(p, s);
       case 17: return launch_tile3<BF16_OUT, 128, 256, 2, 4, 3, 2>(p, s);
+      case 19: return launch_tile3<BF16_OUT, 256, 128, 4, 2, 3, 2>(p, s);
+      // one
+      case 3: return launch_tile3<BF16_OUT, 128, 128, 2, 4, 5>(p, s);
+      case 4: return launch_tile3<BF16_OUT, 64, 128, 2, 2, 5>(p, s);
+      case 5: return launch_tile3<BF16_OUT, 64, 64, 2, 2, 5>(p, s);
+      case 6: return launch_tile3<BF16_OUT, 128, 64, 2, 2, 5>(p, s);
+      case 7: return launch_tile3<BF16_OUT, 128, 256, 2, 4, 5>(p, s);
       case 9: return launch_tile3<BF16_OUT, 256, 128, 4, 2, 5>(p, s);
       default: break;
     }
@@ -1364,23 +1297,11 @@ static bool stream_offsets_fit(const Fp8MMParams& p) {
 // a wavefront's K slab live in registers: at most 8 wavefronts along K, 14 steps each for one m-block, 8 for two).
 static int stream_steps_per_wave(int64_t M, int64_t N, int64_t K) {
   const int64_t steps = (K + 127) / 128;
-  // three and four m-blocks: K = 1664 .. 4096 (4 steps per wavefront keep the registers, and the workgroup must have a
-  // wavefront per m-block for the reduction).  Measured against the tile kernel with K split, cold weights, M = 48 / 64:
-  // 4096 x 4096 21.0 / 21.4 -> 11.6 / 13.4 us, 4096 x 6144 22.7 / 22.9 -> 14.6 / 16.5 us, 4096 x 28672 36.3 / 37.3 ->
-  // 35.9 / 38.7 us: four m-blocks only up to two rounds of workgroups.
-  if (M > 32) {
-    const bool fits = steps <= 8 * 4 && steps >= 13;
-    // ... unless the 64 x 64 tiles with one more tile row past M fit the device (see m_tiles_extra in dispatch_tile) and the
-    // weights are large enough: that plan takes the same time for 33 as for 64 rows, this kernel's time grows with the
-    // m-blocks.  Cold, M = 40 / 64: 4096 x 6144 12.1 / 15.0 -> 11.3 / 11.4 us, 4096 x 8192 13.2 / 16.1 -> 12.0 / 12.2 us, 4096 x 4096
-    // 9.8 / 12.7 against 10.8 / 10.8 us (the tiles from 49 rows on), 3072 x 3072 7.6 / 9.6 against 9.1 / 9.1 us, 2048 x 2048
-    // 5.5 / 7.0 against 7.4 / 7.4 us (this kernel).
-    const int64_t cols = (N + 63) / 64;
-    if (tuning().exp[13] != 1 && tuning().fp8_tile_cfg <= 0 && K % 128 == 0 && 2 * cols <= (int64_t)num_cus_current_device() &&
-        (K * N >= ((int64_t)20 << 20) || (M > 48 && K * N >= ((int64_t)8 << 20))))
-      return 0;
-    return (fits && (M <= 48 || (M <= 64 && N / 16 <= 2 * num_cus_current_device()))) ? 4 : 0;
-  }
+  // three m-blocks: K = 1664 .. 4096 (4 steps per wavefront keep the registers, and the workgroup must have a wavefront per
+  // m-block for the reduction) of a narrow layer.  Cold against the tile kernel at M = 35 .. 47: 3712 x 3712 8.6 against 10.2 us,
+  // 2048 x 2304 5.9 against 6.6, 2816 x 3840 7.2 against 8.0 us; level at N = 4500, behind on wider layers (2304 x 14144 11.7
+  // against 10.4 us) and with a fourth m-block (3072 x 2304 at M = 59 9.3 against 8.3 us).
+  if (M > 32) return M <= 48 && N <= 4096 && steps <= 8 * 4 && steps >= 13 ? 4 : 0;
   if (steps <= 8 * 4) return 4;
   if (steps <= 8 * 8) return 8;
   if (steps <= 8 * 14 && M <= 16) return 14;
@@ -1389,11 +1310,13 @@ static int stream_steps_per_wave(int64_t M, int64_t N, int64_t K) {
 
 // The stream kernel over two halves of K (two workgroups per n-tile range, partial tiles handed over through the caller's
 // scratch): K steps per wavefront, 0 if this route does not take the problem.  It covers what the registers of one
-// workgroup cannot at two m-blocks: 16 < M <= 32 up to K = 16384 (cold weights, against the tile kernel with K split:
-// 14336 x 4096 at M = 24 / 32 34.7 / 35.1 -> 21.6 / 22.5 us, 16384 x 4096 at M = 32 37.1 -> 27.4 us).  For M <= 16 beyond
-// K = 14336 (14 steps per wavefront and half) the tile kernel stays ahead: 28672 x 8192 72 against 85 us.
+// workgroup cannot at two m-blocks: 16 < M <= 32 up to K = 16384, on layers whose workgroups fit the device at once (cold
+// against the tile kernel with K split: 9728 x 1152 at M = 17 11.0 against 11.9 us, 10112 x 1920 at M = 27 12.4 against 13.5 us; on
+// wider ones the tiles are ahead, 12544 x 2560 at M = 17 15.2 against 19.6 us, 8320 x 9920 at M = 22 23.0 against 32.2 us).
 static int stream_split_steps_per_wave(int64_t M, int64_t N, int64_t K) {
-  if (tuning().fp8_stream_split < 0 || M <= 16 || M > 32 || stream_steps_per_wave(M, N, K) != 0) return 0;
+  if (tuning().fp8_stream_split < 0 || M <= 16 || M > 32 || stream_steps_per_wave(M, N, K) != 0 ||
+      N / 8 > num_cus_current_device())
+    return 0;
   const int64_t half = ((K + 127) / 128 + 1) / 2;
   return half <= 8 * 8 ? 8 : 0;
 }
@@ -1506,10 +1429,8 @@ static bool dispatch_stream(const Fp8MMParams& p, hipStream_t s) {
   } else if (MB == 2) {
     if (ks == 4) launch_stream<BF16_OUT, 4, 2>(p, wk, gx, s);
     else launch_stream<BF16_OUT, 8, 2>(p, wk, gx, s);
-  } else if (MB == 3) {
-    launch_stream<BF16_OUT, 4, 3>(p, wk, gx, s);
   } else {
-    launch_stream<BF16_OUT, 4, 4>(p, wk, gx, s);
+    launch_stream<BF16_OUT, 4, 3>(p, wk, gx, s);
   }
   return true;
 }

@@ -45,6 +45,7 @@ int num_cus_current_device();   // cached per device, api.hip
 // the caller's struct; the host code below it reads `tuning()`, which is all zeros (= automatic) outside a scope.  The
 // pointer lives in a thread-local for the duration of that one call: nothing persists between calls or crosses threads.
 const VaqTuning& tuning();
+bool tuning_active();      // inside a scope with a struct
 class TuningScope {
  public:
   explicit TuningScope(const VaqTuning* t);
