@@ -236,6 +236,23 @@ def test_prefill_every_tile_shape(device, asym, dtype):
         assert bool((layer.workspace == 0).all()), "workspace counters not restored to zero"
 
 
+@pytest.mark.parametrize("group_size,bits", [(128, 4), (-1, 4), (64, 4), (32, 4), (128, 8), (32, 8)])
+@pytest.mark.parametrize("tile", [12, 14, 15, 16])
+def test_prefill_eight_wavefront_tiles_every_format(device, tile, group_size, bits):
+    """The tile shapes below 256 x 256 forced on every weight format: ragged M and N, K of one group and more, K in parts."""
+    from vllm_amd import _tuning
+    for k, n, m, splits in ((128, 64, 65, (1,)), (640, 320, 257, (1, 2)), (1024, 448, 130, (1, 3))):
+        case = o.make_w4a16_case(k, n, group_size, asym=bits == 4, seed=k + n + m, num_bits=bits)
+        layer = W4A16Layer(case, device)
+        a = _acts(m, k, device, seed=m)
+        ref = o.gemm_ref(a.cpu(), o.case_w_ref(case))
+        for split in splits:
+            with _tuning.override(prefill_tile=tile + 1, prefill_split=split, exp=[0, 0, 1]):
+                out = layer(a)
+            check_gemm_close(out, ref, f"tile {tile} split {split} g={group_size} bits={bits} k={k} n={n} m={m}")
+        assert bool((layer.workspace == 0).all()), "workspace counters not restored to zero"
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("asym", [False, True])
 def test_prefill_register_dequant_tile(device, dtype, asym):

@@ -16,8 +16,7 @@
 // k0 + 32*q .. k0 + 32*q + 31 of its row.
 #include "vaq_common.h"
 #include "tile_handover.h"
-
-#include <math.h>
+#include "tile_plan.h"
 
 #include <type_traits>
 
@@ -1076,89 +1075,46 @@ static int launch_tile3(const Fp8MMParams& p, hipStream_t s) {
   return VAQ_OK;
 }
 
-struct Fp8TilePlan {
-  int cfg = -1, sk = 1, bm = 0, bn = 0, nw = 0;
-  int64_t tiles = 0;
-  int64_t tail_first = 0;      // > 0: only the tiles from this position on are split (tile_handover.h)
-  int64_t extra_tiles = 0;     // split K: the tiles of a tile row past M that runs beside the real ones (see m_tiles_extra in dispatch_tile)
-  // scratch of the K split: partial tiles and arrival counters of the tiles that are split
-  int64_t split_tiles() const { return sk > 1 ? tiles + extra_tiles - tail_first : 0; }
-  int64_t tmp_bytes() const { return (int64_t)sk * split_tiles() * bm * bn * 4; }
-  int64_t counter_ints() const { return split_tiles() * nw; }
-};
+// The tile shapes of the multi-stage kernel (ids for K % 128 == 0; the two-slice shapes have one with a slice per step, id - 10).
+// Fitted to 1553 problems with M = 9 .. 8192, K = 1024 .. 16384, N = 1024 .. 28672 drawn over the logarithm, every shape and K
+// split of each timed on cold weights (some 20000 launches; 7.6 % rms).  The plan with the least predicted time is on average
+// 0.8 % slower than the fastest of all plans of a problem, where rules by size were 11 % slower at M = 33 .. 1024
+// (4096 x 13824 at M = 384 49 -> 33 us, 8192 x 4096 at M = 180 25 -> 19 us, 14336 x 2048 at M = 384 39 -> 27 us).
+constexpr TileShape FP8_TILE_SHAPES[] = {
+    {13, 128, 128, 8, 1, 2.24, 0.192, 0.121, 0, 0}, {14, 64, 128, 4, 1, 1.75, 0.172, 0.090, 0, 0},
+    {15, 64, 64, 4, 2, 0.86, 0.103, 0.043, 0.107, 0}, {16, 128, 64, 4, 1, 1.75, 0.152, 0.048, 0, 0},
+    {17, 128, 256, 8, 1, 4.81, 0.344, 0.160, 0, 0}, {19, 256, 128, 8, 1, 4.55, 0.311, 0.124, 0, 0},
+    {1, 256, 256, 8, 1, 10.46, 0.476, 0.218, 0, 0}, {10, 256, 384, 8, 1, 22.66, 0.580, 0.451, 0, 0}};
+constexpr TileCosts FP8_TILE_COSTS = {0.204, 2.56, 0.725, 0.184};
 
-// The tile shapes of the multi-stage kernel and what a launch of each costs, in us: a workgroup takes `base` plus, per 64-byte
-// step of K, `step` + `load` * (share of the device that runs beside it, up to `slots` workgroups per compute unit).  Fitted to
-// 1553 problems with M = 9 .. 8192, K = 1024 .. 16384, N = 1024 .. 28672 drawn over the logarithm, every shape and K split of
-// each timed on cold weights (some 20000 launches; 7.6 % rms).  The plan with the least predicted time is on average
-// 0.8 % slower than the fastest of all plans of a problem, where the rules by size that it replaces were 11 % slower at M = 33 .. 1024.
-// (4096 x 13824 at M = 384 49 -> 33 us, 8192 x 4096 at M = 180 25 -> 19 us, 14336 x 2048 at M = 384 39 -> 27 us.)
-struct Fp8TileShape {
-  int cfg, bm, bn, nw, slots;      // cfg: id for K % 128 == 0; the two-slice shapes have one with a slice per step, id - 10
-  double base, step, load;
-};
-constexpr Fp8TileShape FP8_TILE_SHAPES[] = {
-    {13, 128, 128, 8, 1, 2.24, 0.192, 0.121}, {14, 64, 128, 4, 1, 1.75, 0.172, 0.090}, {15, 64, 64, 4, 2, 0.86, 0.103, 0.043},
-    {16, 128, 64, 4, 1, 1.75, 0.152, 0.048},  {17, 128, 256, 8, 1, 4.81, 0.344, 0.160}, {19, 256, 128, 8, 1, 4.55, 0.311, 0.124},
-    {1, 256, 256, 8, 1, 10.46, 0.476, 0.218}, {10, 256, 384, 8, 1, 22.66, 0.580, 0.451}};
-constexpr double FP8_SHARED_UNIT = 0.107;      // us per step where two workgroups share a compute unit
-constexpr double FP8_WEIGHT_US_PER_MB = 0.204; // cold weights arrive no faster than this
-// hand-over of a K split: fixed, per part, per MB of partial tiles
-constexpr double FP8_HANDOVER_US = 2.56, FP8_HANDOVER_US_PER_PART = 0.725, FP8_HANDOVER_US_PER_MB = 0.184;
-
-static Fp8TilePlan make_plan_tile3(int M, int N, int K) {
+static TilePlan make_plan_tile3(int M, int N, int K) {
   const int64_t cus = num_cus_current_device();
   const int steps = K / 64;
   const VaqTuning& tn = tuning();
-  Fp8TilePlan best;
-  double best_us = -1;
-  // `part_tiles` tiles in `sk` parts beside `whole_rounds` rounds of whole ones
-  auto consider = [&](const Fp8TileShape& t, int64_t tiles, int sk, int64_t tail_first) {
-    const int64_t split_tiles = tail_first > 0 ? tiles - tail_first : tiles, cap = cus * t.slots;
-    const int64_t rounds = tail_first > 0 ? tail_first / cus : tiles * sk / cap;
-    const double rest = (double)(tail_first > 0 ? split_tiles * sk : tiles * sk % cap) / (double)cus;
-    const double part = (double)steps / sk, whole = tail_first > 0 ? (double)steps : part;
-    double us = (double)rounds * (t.base + whole * (t.step + t.load * t.slots + (t.slots > 1 ? FP8_SHARED_UNIT : 0)));
-    if (rest > 0) us += t.base + part * (t.step + t.load * rest + (rest > 1 ? FP8_SHARED_UNIT : 0));
-    const double mem = FP8_WEIGHT_US_PER_MB * 1e-6 * (double)N * K;
-    us = sqrt(sqrt(us * us * us * us + mem * mem * mem * mem)) + 2.0;
-    if (sk > 1)
-      us += FP8_HANDOVER_US + FP8_HANDOVER_US_PER_PART * sk + FP8_HANDOVER_US_PER_MB * 4e-6 * (double)(split_tiles * t.bm * t.bn) * sk;
-    // (a handful of left-over tiles: the estimate is 7 % high there, 2048 x 4096 at M = 4352 58.7 against 54.9 us)
-    if (tail_first > 0 && split_tiles * 8 <= cus) us *= 0.9;
-    if (best_us >= 0 && us >= best_us) return;
-    if ((uint64_t)sk * (uint64_t)split_tiles * t.bm * t.bn * 4 >= (1ull << 32) && sk > 1) return;      // 32-bit buffer offsets
-    best_us = us;
-    best.bm = t.bm; best.bn = t.bn; best.nw = t.nw;
-    best.tiles = tiles;
-    best.sk = sk;
-    best.tail_first = tail_first;
-    best.cfg = tn.fp8_tile_cfg > 0 ? tn.fp8_tile_cfg : (t.cfg > 10 && K % 128 != 0 ? t.cfg - 10 : t.cfg);
-  };
-  for (const Fp8TileShape& t : FP8_TILE_SHAPES) {
-    if (tn.fp8_tile_cfg > 0 ? tn.fp8_tile_cfg != t.cfg && tn.fp8_tile_cfg != t.cfg - 10 : t.cfg == 10 && N % 384 != 0) continue;
+  TilePlan best;
+  for (const TileShape& t : FP8_TILE_SHAPES) {
+    if (tn.fp8_tile_cfg > 0 ? tn.fp8_tile_cfg != t.id && tn.fp8_tile_cfg != t.id - 10 : t.id == 10 && N % 384 != 0) continue;
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
     const int64_t rest = tiles % cus;
+    auto consider = [&](int sk, int64_t tail_first) {
+      consider_tile_plan(best, t, FP8_TILE_COSTS, M, N, (double)N * K, tiles, sk, tail_first, steps, cus, 1ll << 32);   // (32-bit offsets)
+    };
     if (tn.fp8_split > 0) {
-      consider(t, tiles, tn.fp8_split <= steps ? tn.fp8_split : steps, 0);
+      consider(tn.fp8_split <= steps ? tn.fp8_split : steps, 0);
       continue;
     }
     // K in up to 8 parts of at least 8 steps, on up to 2.3 rounds of workgroups
     for (int sk : {1, 2, 3, 4, 6, 8})
-      if (sk == 1 || (steps / sk >= 8 && tiles * sk * 10 <= cus * 23)) consider(t, tiles, sk, 0);
+      if (sk == 1 || (steps / sk >= 8 && tiles * sk * 10 <= cus * 23)) consider(sk, 0);
     // 256 x 256 tiles that end in a round of workgroups at most half full: the tiles of that round in parts of at least 16
     // steps that fill it, the others whole
-    if (t.cfg == 1 && tiles > cus && rest > 0 && tn.exp[10] != 1)
+    if (t.id == 1 && tiles > cus && rest > 0 && tn.exp[10] != 1)
       for (int sk : {2, 3, 4})
-        if (rest * sk <= cus && steps / sk >= 16) consider(t, tiles, sk, tiles - rest);
+        if (rest * sk <= cus && steps / sk >= 16) consider(sk, tiles - rest);
   }
-  if (best_us < 0) {      // an unknown id was forced: the caller's other kernels take the problem
-    best = Fp8TilePlan{};
-    best.cfg = -1;
-    best.sk = 1;
-    return best;
-  }
-  if (best.cfg > 10 && K % 128 != 0) best.cfg -= 10;
+  if (best.id < 0) return best;      // an unknown shape was forced: the other kernels take the problem
+  if (tn.fp8_tile_cfg > 0) best.id = tn.fp8_tile_cfg;
+  if (best.id > 10 && K % 128 != 0) best.id -= 10;
   // A split K with compute units left for the parts of one more tile row: that row runs past M beside the real ones, as
   // with an unsplit K (see m_tiles_extra in dispatch_tile); its workgroups take no part in the hand-over, but tile
   // positions -- and with them the places in the scratch -- count it.  Cold: 7168 x 2048 at M = 40 / 64 / 192 12.1 / 13.6 /
@@ -1170,22 +1126,10 @@ static Fp8TilePlan make_plan_tile3(int M, int N, int K) {
   return best;
 }
 
-// The plan of a problem, kept for the next call on it (weighing 50 plans takes 2 us of host time): one small table per
-// thread, replaced on collision; calls with overrides neither read nor fill it.
-static Fp8TilePlan plan_tile3(int M, int N, int K) {
-  struct Entry {
-    int m = -1, n = 0, k = 0, cus = 0;
-    Fp8TilePlan plan;
-  };
-  static thread_local Entry table[64];
+static TilePlan plan_tile3(int M, int N, int K) {
+  static thread_local TilePlanTable table;
   if (tuning_active()) return make_plan_tile3(M, N, K);
-  const int cus = num_cus_current_device();
-  Entry& e = table[((uint32_t)M * 2654435761u ^ (uint32_t)N * 2246822519u ^ (uint32_t)K * 3266489917u) >> 26];
-  if (e.m != M || e.n != N || e.k != K || e.cus != cus) {
-    e.plan = make_plan_tile3(M, N, K);
-    e.m = M; e.n = N; e.k = K; e.cus = cus;
-  }
-  return e.plan;
+  return table.get(M, N, K, num_cus_current_device(), [&] { return make_plan_tile3(M, N, K); });
 }
 
 template <bool BF16_OUT>
@@ -1194,7 +1138,7 @@ static int dispatch_tile(const Fp8MMParams& p_in, int64_t c_tmp_bytes, int64_t c
   const bool direct_ok = tuning().fp8_tile_impl == 0 && p.K % 64 == 0 && (uint64_t)p.M * (uint64_t)p.lda < (1ull << 32) &&
                          (uint64_t)p.N * (uint64_t)p.ldb < (1ull << 32);
   if (direct_ok && tuning().fp8_tile_impl == 0 && tuning().fp8_tile_cfg >= 0) {
-    Fp8TilePlan pl = plan_tile3(p.M, p.N, p.K);
+    TilePlan pl = plan_tile3(p.M, p.N, p.K);
     // without (enough) scratch from the caller the unsplit kernel still gives the result
     if (pl.sk > 1 && (p.c_tmp == nullptr || p.counters == nullptr || counter_ints < pl.counter_ints() ||
                       c_tmp_bytes < pl.tmp_bytes()))
@@ -1202,7 +1146,7 @@ static int dispatch_tile(const Fp8MMParams& p_in, int64_t c_tmp_bytes, int64_t c
     if (pl.sk == 1) pl.tail_first = 0;
     p.SK = pl.sk;
     p.tail_first = (int)pl.tail_first;
-    if (pl.cfg > 0) {
+    if (pl.id > 0) {
       const int64_t tiles_m = (p.M + pl.bm - 1) / pl.bm;
       const int64_t cus = num_cus_current_device();
       // (with K split over workgroups the rotation gains nothing on cold weights and costs 20-30 % on cached ones.)
@@ -1238,7 +1182,7 @@ static int dispatch_tile(const Fp8MMParams& p_in, int64_t c_tmp_bytes, int64_t c
         p.rotate_k = 0;
       }
     }
-    switch (pl.cfg) {
+    switch (pl.id) {
       case 1: return launch_tile3<BF16_OUT, 256, 256, 2, 4, 5, 1, 2>(p, s);    // alternating phases, slices requested in pairs (see the kernel)
       case 10: return launch_tile3<BF16_OUT, 256, 384, 2, 4, 4, 1, 1>(p, s);   // 8 wavefronts of 128 x 96, alternating phases
       // two k-slices per step (K % 128 == 0)
@@ -1461,7 +1405,7 @@ extern "C" int vaq_fp8_scaled_mm_workspace_tuned(int64_t size_m, int64_t size_n,
     return VAQ_OK;
   }
   if (size_k % 64 != 0 || tuning().fp8_tile_impl != 0 || tuning().fp8_tile_cfg < 0) return VAQ_OK;
-  const Fp8TilePlan pl = plan_tile3((int)size_m, (int)size_n, (int)size_k);
+  const TilePlan pl = plan_tile3((int)size_m, (int)size_n, (int)size_k);
   *c_tmp_bytes = (size_t)pl.tmp_bytes();
   *counter_ints = (size_t)pl.counter_ints();
   return VAQ_OK;

@@ -243,6 +243,9 @@ static bool row_split_config(int M, int N, int K, int sub, int wt, bool has_perm
   if (c.sk != 1) return false;
   *out = c;
   if (tuning().exp[2] == 2) return true;
+  // (beyond four m-blocks not on a short K, where the tiles are ahead: 1280 x 4288 at M = 118 9.4 against 12.4 us, 1152 x 4928 at
+  // M = 185 10.8 against 15.1 us; at K = 2048 this kernel is, 2048 x 2048 at M = 128 6.3 us)
+  if (M > DECODE2_MAX_M && K < 2048) return false;
   const long cus = num_cus_current_device();
   if (M <= DECODE2_MAX_M) {
     // Against two to four m-blocks in one workgroup: one round of full workgroups.  Measured: 4096 x 4096 at M = 32 / 64:
