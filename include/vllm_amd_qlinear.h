@@ -233,6 +233,18 @@ int vaq_fp8_scaled_mm_ws(const uint8_t* a, int64_t lda, const uint8_t* b, int64_
                          int64_t size_m, int64_t size_n, int64_t size_k, float* c_tmp, int64_t c_tmp_bytes,
                          int32_t* counters, int64_t counter_ints, void* stream);
 
+/*
+ * Quantisation and GEMM of a few rows in one launch, with the bits of vaq_fp8_quant_per_token (x_scale NULL, no upper bound
+ * on the scales) or vaq_fp8_quant_static followed by vaq_fp8_scaled_mm.
+ *   x  F16/BF16 [M, K], 16-byte aligned, row stride a multiple of 8;  x_scale  fp32 scalar (device) or NULL;
+ *   b, sb, bias, out as above, out and bias of the type of x
+ * Takes the sizes for which vaq_fp8_quant_scaled_mm_takes is 1: those it is faster for than the two calls.
+ */
+int vaq_fp8_quant_scaled_mm_takes(int64_t size_m, int64_t size_n, int64_t size_k, int per_token);
+int vaq_fp8_quant_scaled_mm(const void* x, int64_t ldx, const float* x_scale, const uint8_t* b, int64_t ldb, const float* sb,
+                            int64_t sb_count, const void* bias, void* out, int64_t ldc, int dtype, int64_t size_m,
+                            int64_t size_n, int64_t size_k, void* stream);
+
 #pragma GCC visibility pop
 
 #ifdef __cplusplus

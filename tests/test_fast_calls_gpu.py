@@ -72,6 +72,33 @@ def test_fp8_layer_equals_its_two_steps(device, shape, static, bias):
     assert torch.equal(ops._fast.scaled_mm(q2, wq.t(), s2, ws, torch.bfloat16, b), ref)
 
 
+@pytest.mark.parametrize("k,n", [(16, 16), (144, 320), (1040, 256), (2064, 4128), (4096, 528), (4112, 64), (8176, 80), (8192, 48), (16384, 32)])
+@pytest.mark.parametrize("static", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_fp8_rows_quantised_by_the_gemm(device, k, n, static, dtype):
+    """One launch for the quantisation and the product of a few rows: the bits of the two launches, special values too."""
+    from vllm_amd import _custom_ops as ops, _lib
+    lib, taken = _lib.load(), 0
+    g = torch.Generator(device=device).manual_seed(k + n)
+    wq, ws = ops.scaled_fp8_quant(torch.randn(n, k, device=device, generator=g).to(dtype), use_per_token_if_dynamic=True)
+    for m in range(1, 10):
+        x = torch.randn(m, k + 16, device=device, generator=g).to(dtype)[:, :k]
+        if m >= 3:
+            x[1] = 0
+        if m >= 6:
+            x[0, 3], x[2, 7], x[4, k - 1], x[5] = float("inf"), float("nan"), -float("inf"), x[5] * 1e-6
+        if m >= 8:
+            x[6], x[7] = float("nan"), -0.0
+        scale = torch.full((1,), 0.011, device=device) if static else None
+        bias = torch.randn(n, device=device, generator=g).to(dtype) if m % 2 else None
+        taken += lib.vaq_fp8_quant_scaled_mm_takes(m, n, k, not static)
+        got = ops.fp8_linear(x, wq.t(), ws if m % 3 else ws[:1].contiguous(), scale, None, dtype, bias)
+        q, s = ops.scaled_fp8_quant(x.contiguous(), scale, use_per_token_if_dynamic=True)
+        ref = ops.cutlass_scaled_mm(q, wq.t(), s, ws if m % 3 else ws[:1].contiguous(), dtype, bias)
+        assert torch.equal(got.view(torch.int16), ref.view(torch.int16)), m
+    assert taken >= (4 if k > 4096 else 8)
+
+
 def test_no_answer_where_something_is_in_between(device):
     from torch.utils._python_dispatch import TorchDispatchMode
     from vllm_amd import _custom_ops as ops, _tuning

@@ -52,6 +52,9 @@ _SIGNATURES = {
     "vaq_fp8_scaled_mm_ws": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p,
                                      c_void_p, c_int64, c_int, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p,
                                      c_int64, c_void_p]),
+    "vaq_fp8_quant_scaled_mm_takes": (c_int, [c_int64, c_int64, c_int64, c_int]),
+    "vaq_fp8_quant_scaled_mm": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p,
+                                        c_int64, c_int, c_int64, c_int64, c_int64, c_void_p]),
 }
 class VaqTuning(ctypes.Structure):
     """``VaqTuning`` of the header: kernel-variant overrides for ONE call (tests, benchmarks); all zero = automatic."""

@@ -41,11 +41,9 @@ typedef struct VaqTuning {
                         /*   activation fill, [1] = ring variant + 1, [2] rows over workgroups (1 off, 2 forced) of   */
                         /*   the LDS-staged decode kernel, [3] = 1 sixteen staged rows for M = 5 .. 8, [5] = 1 two K   */
                         /*   slabs never merged into one; [4] FP8 streaming through LDS (1 / 2 / 3 = 8 / 4 / 16 steps   */
-                        /*   per wavefront, 9 = off); [8] = 1 W4A16 tile kernel: no 128 x 128 tiles for long K parts;   */
-                        /*   [9] = 1 W4A16 tile kernel: 256-row tiles also when M fills them poorly; [10] = 1 both tile     */
-                        /*   kernels: never split only the tiles of a half-empty last round; [11] = 1 W4A16 tile kernel:  */
-                        /*   no 128 x 256 tiles; [12] = 1 FP8 tile kernel: every tile starts at the first K step;       */
-                        /*   [13] = 1 FP8 tile kernel: no tile row past M; [14] unused;  */
+                        /*   per wavefront, 9 = off); [10] = 1 both tile kernels: never split only the tiles of a half-empty last round; */
+                        /*   [12] = 1 FP8 tile kernel: every tile starts at the first K step; [13] = 1 FP8 tile kernel: no tile  */
+                        /*   row past M; [6], [8], [9], [11], [14] unused;                                              */
                         /*   [7] = 1 LDS-staged decode kernel: n-tiles in launch order, not grouped by XCD             */
 } VaqTuning;
 
