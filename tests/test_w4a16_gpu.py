@@ -582,6 +582,26 @@ def test_rows_over_workgroups_beyond_four_m_blocks(device, k, n, m, dtype):
         assert torch.equal(layer(hot.to(device)).cpu(), w_ref[rows]), "one-hot rows must return the dequantised weights exactly"
 
 
+@pytest.mark.parametrize("bits,group_size,asym", [(4, 64, False), (4, 64, True), (4, 32, True), (8, -1, False), (8, 128, False), (8, 64, False), (8, 32, False)])
+@pytest.mark.parametrize("k,n,m,gs", [(128, 64, 17, 2), (1024, 448, 33, 4), (1920, 576, 47, 8), (2048, 1024, 256, 16), (3968, 320, 100, 16)])
+def test_rows_over_workgroups_other_formats(device, bits, group_size, asym, k, n, m, gs):
+    """Workgroups of 16 rows each with groups of 64 / 32 rows and 8-bit codes: one weight tile to a whole K per workgroup, ragged
+    last slices and m-blocks, every stream length, against the fp64 oracle; one-hot rows bit for bit."""
+    from vllm_amd import _tuning
+    case = o.make_w4a16_case(k, n, group_size, asym=asym, seed=k + n + m, num_bits=bits)
+    layer = W4A16Layer(case, device)
+    w_ref = o.case_w_ref(case)
+    a = _acts(m, k, device, seed=m)
+    hot = torch.zeros(m, k, dtype=a.dtype)
+    rows = [(37 * i + 5) % k for i in range(m)]
+    for i, r in enumerate(rows):
+        hot[i, r] = 1
+    for forced in (dict(), dict(decode2_gs=gs)):
+        with _tuning.override(exp=[0, 0, 2], **forced):
+            check_gemm_close(layer(a), o.gemm_ref(a.cpu(), w_ref), f"{bits=} {group_size=} k={k} n={n} m={m} {forced}")
+            assert torch.equal(layer(hot.to(device)).cpu(), w_ref[rows])
+
+
 @pytest.mark.parametrize("k,n", [(4096, 4096), (4096, 6144), (1024, 1472), (2048, 1984), (4096, 3008), (2048, 2048), (14336, 4096)])
 def test_decode_n_tiles_grouped_by_xcd_same_bits(device, k, n):
     """On narrow layers the decode kernel hands the workgroups of one XCD neighbouring n-tiles (a permutation of which

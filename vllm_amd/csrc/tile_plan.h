@@ -65,14 +65,15 @@ inline void consider_tile_plan(TilePlan& best, const TileShape& t, const TileCos
 
 // A small table of finished plans, one per thread, replaced on collision: weighing the plans of a problem takes 2 us of host
 // time.  (Calls with tuning overrides neither read nor fill it.)
-struct TilePlanTable {
+template <class Plan>
+struct PlanTable {
   struct Entry {
     int m = -1, n = 0, k = 0, key = 0;
-    TilePlan plan;
+    Plan plan;
   };
   Entry entry[64];
   template <class Make>
-  const TilePlan& get(int m, int n, int k, int key, Make make) {
+  const Plan& get(int m, int n, int k, int key, Make make) {
     Entry& e = entry[((uint32_t)m * 2654435761u ^ (uint32_t)n * 2246822519u ^ (uint32_t)k * 3266489917u ^ (uint32_t)key * 668265263u) >> 26];
     if (e.m != m || e.n != n || e.k != k || e.key != key) {
       e.plan = make();
@@ -81,5 +82,6 @@ struct TilePlanTable {
     return e.plan;
   }
 };
+using TilePlanTable = PlanTable<TilePlan>;
 
 }  // namespace vaq

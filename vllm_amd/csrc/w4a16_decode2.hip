@@ -1,5 +1,6 @@
 // Host side of the LDS-staged decode kernel (w4a16_decode2_kernel.h): configuration choice, workspace sizes, launch
 // of the instances for quantisation groups of 128 rows and channelwise scales.
+#include "tile_plan.h"
 #include "w4a16_decode2_kernel.h"
 
 namespace vaq {
@@ -23,10 +24,40 @@ static int round_gs(int x, int sub, bool w8) {
   return 16;
 }
 
+// Workgroups of `waves` wavefronts and `lds_wg` bytes of LDS that share a compute unit (at least one).
+static inline long wg_slots(int waves, size_t lds_wg) {
+  const long by_waves = D2_WAVES / waves, by_lds = (long)((size_t)(160 * 1024) / lds_wg);
+  const long slots = by_waves < by_lds ? by_waves : by_lds;
+  return slots < 1 ? 1 : slots;
+}
+
+// n-tiles per workgroup (at most 16 / wks).  A compute unit holds 16 of these wavefronts and as many workgroups as its LDS
+// allows (`lds_wg` bytes each).  First the fewest rounds of workgroups per compute unit, then the fewest wavefronts on the
+// busiest compute unit (i.e. spread over the device), then the smaller workgroup.
+static int pick_wn(int NT, int sk, int wks, size_t lds_wg, long* rounds_out) {
+  const int cus = num_cus_current_device();
+  int best_wn = 1;
+  long best_rounds = -1, best_waves = -1;
+  for (int wn = 1; wn <= D2_WAVES / wks; ++wn) {
+    const long slots = wg_slots(wks * wn, lds_wg);
+    const long wgs = (long)((NT + wn - 1) / wn) * sk;
+    const long per_cu = (wgs + cus - 1) / cus;
+    const long rounds = (per_cu + slots - 1) / slots;
+    const long waves = (per_cu < slots ? per_cu : slots) * wn * wks;
+    if (best_rounds < 0 || rounds < best_rounds || (rounds == best_rounds && waves < best_waves)) {
+      best_rounds = rounds;
+      best_waves = waves;
+      best_wn = wn;
+    }
+  }
+  if (rounds_out) *rounds_out = best_rounds;
+  return best_wn;
+}
+
 // Groups per slab are limited by LDS (128 KiB of activations, 256 bytes per group and staged row): 512 / rows.
 // G, gslab, gs and slab_max below count weight tiles: one per 128 rows of K, two (nibble planes) for 8-bit codes.
 // `nt_mult`: copies of every n-tile's stream that run side by side (rows split over workgroups, see the kernel).
-static Decode2Config pick_decode2_config(int M, int N, int K, int sub, bool w8, int nt_mult = 1, bool allow8 = true) {
+static Decode2Config pick_by_rule(int M, int N, int K, int sub, bool w8, int nt_mult = 1, bool allow8 = true) {
   const int TPG = w8 ? 2 : 1;
   const int G = K / 128 * TPG, NT = N / 16 * nt_mult;
   const int MB = (M + 15) / 16;
@@ -55,38 +86,13 @@ static Decode2Config pick_decode2_config(int M, int N, int K, int sub, bool w8, 
   // Two m-blocks of a long K on a layer of at most one n-tile per compute unit: slabs of one 14-tile stream per
   // wavefront with the four-slot ring (14336 x 4096 at M = 17 / 32: 13.8 / 14.7 -> 12.9 / 13.2 us; 11008 x 4096 14.1 -> 12.4 us;
   // 16-tile streams, two slices of 7 or 8, and the same on 8192 x 8192 or a 28672-wide layer are slower).
-  // n-tiles per workgroup (at most 16 / wks).  A compute unit holds 16 of these wavefronts and as many workgroups as
-  // its LDS allows.  First the fewest rounds of workgroups per compute unit, then the fewest wavefronts on the busiest
-  // compute unit (i.e. spread over the device), then the smaller workgroup.
-  auto pick_wn = [&](int wks_, int gs_, int sk_, long* rounds_out) {
-    int best_wn = 1;
-    long best_rounds = -1, best_waves = -1;
-    const size_t lds_wg = decode2_lds_bytes(wks_, gs_ / TPG, c.mr, MB);
-    for (int wn = 1; wn <= D2_WAVES / wks_; ++wn) {
-      long slots = D2_WAVES / (wks_ * wn);
-      const long lds_slots = (long)((size_t)(160 * 1024) / lds_wg);
-      if (slots > lds_slots) slots = lds_slots;
-      if (slots < 1) slots = 1;
-      const long wgs = (long)((NT + wn - 1) / wn) * sk_;
-      const long per_cu = (wgs + cus - 1) / cus;
-      const long rounds = (per_cu + slots - 1) / slots;
-      const long waves = (per_cu < slots ? per_cu : slots) * wn * wks_;
-      if (best_rounds < 0 || rounds < best_rounds || (rounds == best_rounds && waves < best_waves)) {
-        best_rounds = rounds;
-        best_waves = waves;
-        best_wn = wn;
-      }
-    }
-    if (rounds_out) *rounds_out = best_rounds;
-    return best_wn;
-  };
   bool long_k_two_blocks = MB == 2 && NT <= cus && G >= 80 && sub == 1 && !w8 && nt_mult == 1;
   if (long_k_two_blocks) {
     // ... and only as one round of workgroups of 7 to 10 wavefronts that fill 85 % of the device (measured slower with
     // 4, 11 and 15 wavefronts: 14336 x 2048 10.3 -> 12.2 us, 16384 x 4096 14.2 -> 15.5 us, 24576 x 4096 18.9 -> 20.3 us)
     const int sk_b = (G + 13) / 14;
     long rounds_b = 0;
-    const int wn_b = pick_wn(1, 14, sk_b, &rounds_b);
+    const int wn_b = pick_wn(NT, sk_b, 1, decode2_lds_bytes(1, 14, c.mr, MB), &rounds_b);
     const long wgs_b = (long)((NT + wn_b - 1) / wn_b) * sk_b;
     long_k_two_blocks = rounds_b == 1 && wn_b >= 7 && wn_b <= 10 && wgs_b * 100 >= (long)cus * 85;
   }
@@ -161,17 +167,14 @@ static Decode2Config pick_decode2_config(int M, int N, int K, int sub, bool w8, 
   c.gs = gs;
   c.wks = wks;
   const size_t lds_wg = decode2_lds_bytes(wks, gs / TPG, c.mr, MB);
-  const int best_wn = pick_wn(wks, gs, c.sk, nullptr);
+  const int best_wn = pick_wn(NT, c.sk, wks, lds_wg, nullptr);
   c.wn = tn.decode2_wn > 0 ? tn.decode2_wn : best_wn;
   if (c.wn * wks > D2_WAVES) c.wn = D2_WAVES / wks;
   // ring variant of long streams (instances exist for 4-bit codes in groups of 128 rows / channelwise, up to two
   // m-blocks): by the wavefronts that share a compute unit
   c.rc = 0;
   if (sub == 1 && !w8 && MB <= 2 && gs >= 7) {
-    long slots = D2_WAVES / (wks * c.wn);
-    const long lds_slots = (long)((size_t)(160 * 1024) / lds_wg);
-    if (slots > lds_slots) slots = lds_slots;
-    if (slots < 1) slots = 1;
+    const long slots = wg_slots(wks * c.wn, lds_wg);
     const long per_cu = ((long)((NT + c.wn - 1) / c.wn) * c.sk + cus - 1) / cus;
     const long waves_cu = (per_cu < slots ? per_cu : slots) * wks * c.wn;
     if (long_k_two_blocks && wks == 1 && gs == 14) c.rc = 1;
@@ -185,9 +188,158 @@ static Decode2Config pick_decode2_config(int M, int N, int K, int sub, bool w8, 
   // against 7.5 us; 5120 x 27648, 32 + 8, 23.2 against 20.8 us; 17920 x 6656, 4 x 32 + 12, 20.0 against 16.9 us)
   if (c.mr == 8 && c.sk > 1 && tn.decode2_gs <= 0 && tn.decode2_wks <= 0) {
     const int slab = c.wks * c.gs, last = G - (c.sk - 1) * slab;
-    if (last * 10 < slab * 6) return pick_decode2_config(M, N, K, sub, w8, nt_mult, false);
+    if (last * 10 < slab * 6) return pick_by_rule(M, N, K, sub, w8, nt_mult, false);
   }
   return c;
+}
+
+// ----------------------------------------------------------------------------- plans by predicted time
+// What a launch costs, in us: per round of workgroups on a compute unit `round`, the activation fill (`fill_kb` per KB staged on it), the
+// stream of weight tiles -- per tile the latency `tile_latency` over the tiles in flight, or the arithmetic of all wavefronts
+// that share the unit, `tile_work` each -- and the reduction over the K slices (`reduce` per doubling); beside that the weights
+// from memory (`mem_mb` per MB, and `again` times that for every further copy of the stream, which L2 serves); `base` per launch;
+// a K split over workgroups costs `handover` + `part` per part + `part_mb` per MB of partial results.
+// [.]: one staged row, 4 or 8, 16.  `sub_work`: groups of 128, 64, 32 rows.
+// Fitted to the cold times of 1.3e5 launches: 3700 random layers (K 1024 .. 14336, N 1024 .. 28672, 1 .. 256 rows), each with up to
+// 60 splits.  The cheapest plan by these figures takes 1.03-1.05 of the fastest one's time (geometric mean).
+struct Decode2Cost {
+  double base, round, fill_kb, mem_mb, again, reduce, handover, part, part_mb;
+  double tile_latency[3], tile_work[3], sub_work[3];
+};
+constexpr Decode2Cost D2_COST_W8 = {2.52, 0, 0.0089, 0.187, 0, 0.148, 0.87, 0.21, 0.32,
+                                    {0.96, 1.04, 0.89}, {0.0284, 0.0301, 0.0341}, {1, 1.24, 1.87}};
+constexpr Decode2Cost D2_COST_SUB = {2.41, 0, 0.0089, 0.228, 0, 0.051, 0.87, 0.21, 0,
+                                     {1.11, 1.29, 1.36}, {0.0412, 0.0422, 0.0478}, {1, 1.03, 1.54}};
+// two m-blocks (groups of 128 rows / channelwise: three and four)
+constexpr Decode2Cost D2_COST_W8_MB2 = {1.08, 0.32, 0.0034, 0.201, 0, 0.57, 0.98, 0.22, 0.31,
+                                        {1.80, 1.80, 1.80}, {0.0586, 0.0586, 0.0586}, {1, 1.20, 1.69}};
+constexpr Decode2Cost D2_COST_SUB_MB2 = {1.04, 0.68, 0.0113, 0.190, 0, 0.23, 1.13, 0.18, 0.16,
+                                         {1.84, 1.84, 1.84}, {0.0643, 0.0643, 0.0643}, {1, 1.25, 1.56}};
+constexpr Decode2Cost D2_COST_MB34 = {1.47, 0.89, 0.0124, 0.229, 0, 0.204, 1.15, 0.18, 0.14,
+                                      {1.97, 1.97, 1.97}, {0.0886, 0.0886, 0.0886}, {1, 1, 1}};
+// the rows split over workgroups (never with a split K)
+constexpr Decode2Cost D2_COST_ROWS_W8 = {2.48, 0, 0.0067, 0.250, 0.653, 0.281, 0, 0, 0,
+                                         {0.86, 0.86, 0.86}, {0.0336, 0.0336, 0.0336}, {1, 1.21, 1.81}};
+constexpr Decode2Cost D2_COST_ROWS_SUB = {2.45, 0, 0.0098, 0.298, 0.518, 0.055, 0, 0, 0,
+                                          {1.36, 1.36, 1.36}, {0.0476, 0.0476, 0.0476}, {1, 0.98, 1.48}};
+constexpr Decode2Cost D2_COST_ROWS = {2.23, 0, 0.0104, 0.233, 0.779, 0.105, 0, 0, 0,
+                                      {1.02, 1.02, 1.02}, {0.037, 0.037, 0.037}, {1, 1, 1}};
+
+static const Decode2Cost& workgroup_cost(int M, int sub, bool w8) {
+  if (w8) return M > 16 ? D2_COST_W8_MB2 : D2_COST_W8;
+  if (sub > 1) return M > 16 ? D2_COST_SUB_MB2 : D2_COST_SUB;
+  return D2_COST_MB34;
+}
+
+static double decode2_us(const Decode2Cost& t, const Decode2Config& c, int M, int N, int K, int sub, bool w8, int MB, int copies) {
+  const int cus = num_cus_current_device(), TPG = w8 ? 2 : 1;
+  const int ri = c.mr == 1 ? 0 : c.mr <= 8 ? 1 : 2;
+  const long slots = wg_slots(c.wks * c.wn, decode2_lds_bytes(c.wks, c.gs / TPG, c.mr, MB));
+  const long wgs = (long)((N / 16 + c.wn - 1) / c.wn) * c.sk * copies, per_cu = (wgs + cus - 1) / cus;
+  const double rounds = (double)((per_cu + slots - 1) / slots), side = (double)(per_cu < slots ? per_cu : slots);
+  const bool whole = c.mr <= 4 && c.gs <= (sub > 1 ? 4 : 8);      // short streams with few rows are requested whole
+  const double flight = whole || c.gs < 3 ? c.gs : 3;
+  auto p4 = [](double x) { return x * x * x * x; };
+  const double tile = sqrt(sqrt(p4(t.tile_latency[ri] / flight) +
+                                p4(side * c.wks * c.wn * t.tile_work[ri] * t.sub_work[sub == 4 ? 2 : sub - 1])));
+  const double fill = t.fill_kb * side * (c.wks * c.gs / TPG) * (c.mr * MB * 256 / 1024.0);
+  const double core = rounds * (t.round + fill + c.gs * tile + t.reduce * log2((double)c.wks));
+  const double mem = t.mem_mb * 0.5e-6 * (double)K * N * TPG * (1 + t.again * (copies - 1));
+  double us = t.base + cbrt(core * core * core + mem * mem * mem);
+  if (c.sk > 1) us += t.handover + c.sk * (t.part + t.part_mb * 4e-6 * (double)M * N);
+  return us;
+}
+
+struct Decode2Plan {
+  Decode2Config c{};
+  double us = -1;      // predicted; negative: no plan
+};
+
+// The cheapest plan of one workgroup for all rows (rows == false) or of workgroups of 16 rows each.
+static Decode2Plan cheapest_decode2(const Decode2Cost& t, int M, int N, int K, int sub, bool w8, bool rows) {
+  const int TPG = w8 ? 2 : 1, G = K / 128 * TPG, NT = N / 16;
+  const int copies = rows ? (M + 15) / 16 : 1, MB = rows ? 1 : (M + 15) / 16;
+  const VaqTuning& tn = tuning();
+  Decode2Plan best;
+  Decode2Config c{};
+  c.mr = rows ? 16 : M == 1 ? 1 : M <= 4 ? 4 : 16;
+  const int slab_max = 512 / (c.mr * MB) * TPG;
+  for (int gs : {1, 2, 4, 7, 8, 14, 16}) {
+    if (gs != round_gs(gs, sub, w8)) continue;
+    if (tn.decode2_gs > 0 && gs != tn.decode2_gs) continue;
+    for (int wks = 1; wks <= 16; wks *= 2) {
+      if (tn.decode2_wks > 0 && wks != tn.decode2_wks) continue;
+      // (four sub-grouped tiles of two m-blocks, unrolled whole, do not fit the registers: twice the time of eight)
+      if (MB == 2 && sub == 4 && gs == 4 && !w8 && tn.decode2_gs <= 0) continue;
+      if (wks * gs > slab_max || (wks > 1 && gs > 2 && wks * gs >= 2 * G)) continue;
+      c.gs = gs;
+      c.wks = wks;
+      c.sk = (G + wks * gs - 1) / (wks * gs);
+      if (rows && c.sk != 1) continue;
+      if (c.sk > 8 && tn.decode2_gs <= 0) continue;
+      if (c.sk > 1 && K <= 2048 && tn.decode2_gs <= 0) continue;       // (fits one slab whatever the format: no hand-over)
+      if (c.sk > 1 && (size_t)c.sk * NT * MB * 1024 > VAQ_STATIC_SCRATCH_DATA_BYTES) continue;      // (the library-owned scratch)
+      const int fixed = tn.decode2_wn > 0 ? min(tn.decode2_wn, D2_WAVES / wks)
+                                          : rows ? 0 : pick_wn(NT, c.sk, wks, decode2_lds_bytes(wks, gs / TPG, c.mr, MB), nullptr);
+      for (int wn = fixed > 0 ? fixed : 1; wn <= (fixed > 0 ? fixed : D2_WAVES / wks); ++wn) {
+        if (fixed <= 0 && wks * wn < 4) continue;
+        c.wn = wn;
+        const double us = decode2_us(t, c, M, N, K, sub, w8, MB, copies);
+        if (best.us >= 0 && us >= best.us) continue;
+        best.us = us;
+        best.c = c;
+      }
+    }
+  }
+  if (rows && best.us >= 0 && sub == 1 && !w8 && best.c.gs >= 7) {      // the ring, as in pick_by_rule
+    const int cus = num_cus_current_device();
+    const long slots = wg_slots(best.c.wks * best.c.wn, decode2_lds_bytes(best.c.wks, best.c.gs, 16, 1));
+    const long per_cu = ((long)((NT + best.c.wn - 1) / best.c.wn) * copies + cus - 1) / cus;
+    if (best.c.gs >= 8 || (per_cu < slots ? per_cu : slots) * best.c.wks * best.c.wn <= 8) best.c.rc = 2;
+    if (tn.exp[1] > 0) best.c.rc = tn.exp[1] - 1;
+  }
+  return best;
+}
+
+// One workgroup for all rows (up to two m-blocks; 4-bit codes in groups of 128 rows / channelwise: up to four).  The rule for the
+// latter, whose choices are within 2-4 % of the predicted ones up to two m-blocks.  For the other formats, which the rule was not
+// made for, the cheapest plan, with 8-bit codes where it is predicted 5 % ahead (M = 1 .. 4 over random layers, mean: 8-bit codes 1.13 -> 1.04 of the
+// fastest plan's time, groups of 64 / 32 rows 1.13 -> 1.04).
+static Decode2Plan plan_workgroup(int M, int N, int K, int sub, bool w8) {
+  Decode2Plan p;
+  p.c = pick_by_rule(M, N, K, sub, w8);
+  p.us = decode2_us(workgroup_cost(M, sub, w8), p.c, M, N, K, sub, w8, (M + 15) / 16, 1);
+  if (sub > 1 || w8) {
+    const Decode2Plan q = cheapest_decode2(workgroup_cost(M, sub, w8), M, N, K, sub, w8, false);
+    if (q.us >= 0 && q.us < (w8 ? 0.95 : 1.0) * p.us) return q;
+  }
+  return p;
+}
+
+// Rows split over workgroups, one m-block each (see the kernel): needs no split of K.
+static Decode2Plan plan_rows(int M, int N, int K, int sub, bool w8) {
+  if (sub == 1 && !w8 && M <= 32) {      // by the rule, see w4a16_decode2_choose
+    Decode2Plan p;
+    p.c = pick_by_rule(16, N, K, sub, w8, (M + 15) / 16);
+    p.us = decode2_us(D2_COST_ROWS, p.c, M, N, K, sub, w8, 1, (M + 15) / 16);
+    if (p.c.sk == 1) return p;
+  }
+  return cheapest_decode2(w8 ? D2_COST_ROWS_W8 : sub > 1 ? D2_COST_ROWS_SUB : D2_COST_ROWS, M, N, K, sub, w8, true);
+}
+
+// Finished plans, one table per thread (see PlanTable); calls with this kernel's switches set neither read nor fill it.
+template <class Make>
+static Decode2Plan cached_plan(bool rows, int M, int N, int K, int sub, bool w8, Make make) {
+  static thread_local PlanTable<Decode2Plan> table;
+  const VaqTuning& tn = tuning();
+  if (tn.decode2_gs > 0 || tn.decode2_wks > 0 || tn.decode2_wn > 0 || tn.exp[1] > 0 || tn.exp[3] > 0 || tn.exp[5] > 0) return make();
+  return table.get(M, N, K, ((num_cus_current_device() * 8 + sub) * 2 + (w8 ? 1 : 0)) * 2 + (rows ? 1 : 0), make);
+}
+static Decode2Plan workgroup_plan(int M, int N, int K, int sub, bool w8) {
+  return cached_plan(false, M, N, K, sub, w8, [&] { return plan_workgroup(M, N, K, sub, w8); });
+}
+static Decode2Plan rows_plan(int M, int N, int K, int sub, bool w8) {
+  return cached_plan(true, M, N, K, sub, w8, [&] { return plan_rows(M, N, K, sub, w8); });
 }
 
 template <bool BF16, int MB, bool HAS_ZP, int MR, int GS>
@@ -232,67 +384,38 @@ static int dispatch_mr2(const Decode2Params& p, const Decode2Config& c, bool bf1
   }
 }
 
-// Rows split over workgroups (one m-block each, see the kernel) instead of several m-blocks per workgroup: 4-bit codes
-// in groups of 128 rows / channelwise, no act_order, and only where a single m-block needs no split of K.  On success
-// `out` is the configuration of the one-m-block kernel that every workgroup runs.
-// (development switch exp[2]: 1 forces it off, 2 on wherever it is built)
-static bool row_split_config(int M, int N, int K, int sub, int wt, bool has_perm, Decode2Config* out) {
-  if (M <= 16 || sub != 1 || wt != 0 || has_perm || tuning().exp[2] == 1) return false;
-  const int MB = (M + 15) / 16, NT = N / 16;
-  Decode2Config c = pick_decode2_config(16, N, K, sub, false, MB);
-  if (c.sk != 1) return false;
-  *out = c;
-  if (tuning().exp[2] == 2) return true;
-  // (beyond four m-blocks not on a short K, where the tiles are ahead: 1280 x 4288 at M = 118 9.4 against 12.4 us, 1152 x 4928 at
-  // M = 185 10.8 against 15.1 us; at K = 2048 this kernel is, 2048 x 2048 at M = 128 6.3 us)
-  if (M > DECODE2_MAX_M && K < 2048) return false;
-  const long cus = num_cus_current_device();
-  if (M <= DECODE2_MAX_M) {
-    // Against two to four m-blocks in one workgroup: one round of full workgroups.  Measured: 4096 x 4096 at M = 32 / 64:
-    // 8.5 / 10.5 -> 6.6 / 9.2 us, 4096 x 6144: 8.8 / 11.4 -> 8.7 / 10.6 us; with three m-blocks the grids of those layers spill
-    // into a second round (15 us) or leave ten wavefronts per workgroup (9.9 -> 11.7 us).  A 28672-wide layer would need
-    // streams of 32 tiles (measured 20.4 -> 21.7 us).
-    // (Two m-blocks also as eight wavefronts of 8-tile streams with the three-slot ring: 4096 x 4096 at M = 32 6.3 us.)
-    const long wgs = (long)((NT + c.wn - 1) / c.wn) * MB;
-    return wgs <= cus && c.wks * c.wn >= (M <= 32 ? 8 : 12);
+// Which kernel takes more than 16 rows: workgroups of all rows (`wg_ok`: built for this case), of 16 rows each, or the tile
+// kernel (`tile_ok`, predicted to take `tile_us`).  No act_order and no FP8 weights among the workgroups of 16 rows.
+// 17 .. 32 rows of 4-bit codes in groups of 128 rows / channelwise: 16 rows each where one m-block needs no split of K and one
+// round of workgroups of at least eight wavefronts takes them all; 4096 x 4096 at M = 32 8.5 -> 6.3 us; a 28672-wide layer would
+// need streams of 32 tiles (20.4 -> 21.7 us).  Everything else by predicted time.
+// (development switch exp[2]: 1 never 16 rows each, 2 wherever it is built)
+int w4a16_decode2_choose(int M, int N, int K, int sub, int wt, bool has_perm, bool wg_ok, bool tile_ok, double tile_us) {
+  const bool w8 = wt != 0, rows_ok = M > 16 && M <= DECODE2_MAX_M_ROWS && wt != 2 && !has_perm && tuning().exp[2] != 1;
+  if (!rows_ok && !tile_ok) return D2_WORKGROUP;
+  Decode2Plan r;
+  if (rows_ok) r = rows_plan(M, N, K, sub, w8);
+  if (r.us >= 0 && tuning().exp[2] == 2) return D2_ROWS;
+  if (wg_ok && M <= 32 && sub == 1 && !w8) {
+    const long wgs = r.us >= 0 ? (long)((N / 16 + r.c.wn - 1) / r.c.wn) * ((M + 15) / 16) : 0;
+    return r.us >= 0 && wgs <= num_cus_current_device() && r.c.wks * r.c.wn >= 8 ? D2_ROWS : D2_WORKGROUP;
   }
-  // Five to sixteen m-blocks, against the tile kernel (whose K step is a latency chain of half a microsecond at these
-  // sizes): the fewest n-tiles per workgroup whose grid -- counted exactly -- is one round of workgroups with at least 12
-  // wavefronts on a compute unit.  Cold: 4096 x 4096 at M = 128 16.2 -> 13.4 us, 4096 x 6144 at M = 80 18.8 -> 13.5 us,
-  // 4096 x 2048 at M = 128 / 256 14.8 / 16.0 -> 8.8 / 13.2 us, 2048 x 2048 at M = 128 / 256 11.5 / 12.5 -> 6.3 / 8.3 us; grids
-  // of a second round lose (4096 x 4096 at M = 96 with 258 workgroups: 16.1 -> 22.3 us), ten wavefronts too (M = 80: 20.2 us).
-  // (An odd number of n-tiles gives way to the next even one where that grid passes too: seven n-tiles -- 14 wavefronts and
-  // a ragged last workgroup -- measured 15-20 % behind eight, 4096 x 4096 at M = 96 15.6 against 13.3 us, 4096 x 2048 at
-  // M = 192 / 208 15.4 / 15.7 against 13.1 us, and five behind six, 2048 x 2048 at M = 144 9.0 against 7.6 us.)
-  const long lds_slots = (long)((size_t)(160 * 1024) / decode2_lds_bytes(c.wks, c.gs, c.mr, 1));
-  auto passes = [&](int wn) {
-    if (wn * c.wks > D2_WAVES) return false;
-    long slots = D2_WAVES / (c.wks * wn);
-    if (slots > lds_slots) slots = lds_slots;
-    if (slots < 1) slots = 1;
-    const long wgs = (long)((NT + wn - 1) / wn) * MB;
-    const long per_cu = (wgs + cus - 1) / cus;
-    return per_cu <= slots && per_cu * c.wks * wn >= 12;
-  };
-  for (int wn = 1; wn * c.wks <= D2_WAVES; ++wn) {
-    if (tuning().decode2_wn > 0 && wn != tuning().decode2_wn) continue;
-    if (!passes(wn)) continue;
-    if (tuning().decode2_wn <= 0 && wn >= 3 && (wn & 1) && passes(wn + 1)) continue;
-    out->wn = wn;
-    return true;
+  int best = D2_TILE;
+  double us = tile_ok ? tile_us + (has_perm ? 4.0 : 0.0) : -1;      // (act_order: a launch that permutes the columns first)
+  if (wg_ok) {
+    const double t = workgroup_plan(M, N, K, sub, w8).us;
+    if (us < 0 || t < us) { us = t; best = D2_WORKGROUP; }
   }
-  return false;
-}
-
-bool w4a16_decode2_takes_rows(int M, int N, int K, int sub, int wt, bool has_perm) {
-  Decode2Config c;
-  return M > DECODE2_MAX_M && M <= DECODE2_MAX_M_ROWS && row_split_config(M, N, K, sub, wt, has_perm, &c);
+  if (r.us >= 0 && (us < 0 || r.us < us)) best = D2_ROWS;
+  return best;
 }
 
 int decode2_launch_msp(const Decode2Params& p, int gs, int rc, bool bf16, bool zp, hipStream_t s);      // w4a16_decode2_msp.hip
+int decode2_launch_msp_sub(const Decode2Params& p, int sub, int gs, bool bf16, bool zp, hipStream_t s);     // w4a16_decode2_msp_sub.hip
+int decode2_launch_msp_w8(const Decode2Params& p, int sub, int gs, bool bf16, hipStream_t s);               // w4a16_decode2_msp_w8.hip
 
 int w4a16_decode2_workspace(int M, int N, int K, int sub, bool w8, size_t* c_tmp_bytes, size_t* counter_ints) {
-  const Decode2Config c = pick_decode2_config(M, N, K, sub, w8);
+  const Decode2Config c = workgroup_plan(M, N, K, sub, w8).c;
   const int MB = (M + 15) / 16;
   const int NT = N / 16;
   *c_tmp_bytes = c.sk > 1 ? (size_t)c.sk * NT * MB * 64 * sizeof(v4f) : 0;
@@ -303,7 +426,7 @@ int w4a16_decode2_workspace(int M, int N, int K, int sub, bool w8, size_t* c_tmp
 int w4a16_decode2_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
                          const int32_t* perm, const void* bias, void* c, float* c_tmp, int64_t c_tmp_bytes,
                          int32_t* counters, int64_t counter_ints, int M, int N, int K, int sub, bool channelwise,
-                         int wt, int dtype, hipStream_t s) {
+                         int wt, int dtype, bool rows, hipStream_t s) {
   const bool w8 = wt != 0;      // 8-bit weights of either kind (1: nibble planes, 2: FP8 bytes): two blocks per 128 rows
   Decode2Params p;
   p.a = (const uint16_t*)a;
@@ -324,12 +447,10 @@ int w4a16_decode2_launch(const void* a, int64_t lda, const int32_t* b, const voi
   p.z_stride = channelwise ? 0 : N / 8;
   p.k_mask = 0x000f000fu;
   p.k_ex = dtype == VAQ_BF16 ? 0x43004300u : 0x64006400u;
-  Decode2Config cfg;
-  const bool row_split = row_split_config(M, N, K, sub, wt, perm != nullptr, &cfg);
-  if (!row_split) {
-    VAQ_CHECK_ARG(M <= DECODE2_MAX_M, "w4a16_gemm(decode): %d rows without the split of the rows over workgroups", M);
-    cfg = pick_decode2_config(M, N, K, sub, w8);
-  }
+  VAQ_CHECK_ARG(rows || M <= DECODE2_MAX_M, "w4a16_gemm(decode): %d rows without the split of the rows over workgroups", M);
+  const Decode2Plan plan = rows ? rows_plan(M, N, K, sub, w8) : workgroup_plan(M, N, K, sub, w8);
+  VAQ_CHECK_SUPPORTED(plan.us >= 0, "w4a16_gemm(decode): K = %d does not fit one workgroup of 16 rows", K);
+  const Decode2Config cfg = plan.c;
   p.SK = cfg.sk;
   p.WKS = cfg.wks;
   p.WN = cfg.wn;
@@ -350,7 +471,9 @@ int w4a16_decode2_launch(const void* a, int64_t lda, const int32_t* b, const voi
   }
   const bool bf16 = dtype == VAQ_BF16, zp = zeros != nullptr;
   int rc;
-  if (row_split) rc = decode2_launch_msp(p, cfg.gs, cfg.rc, bf16, zp, s);
+  if (rows && w8) rc = decode2_launch_msp_w8(p, sub, cfg.gs, bf16, s);
+  else if (rows && sub > 1) rc = decode2_launch_msp_sub(p, sub, cfg.gs, bf16, zp, s);
+  else if (rows) rc = decode2_launch_msp(p, cfg.gs, cfg.rc, bf16, zp, s);
   else if (wt == 2) rc = decode2_launch_f8(p, cfg.gs, MB, cfg.mr, bf16, s);
   else if (w8 && sub > 1) rc = decode2_launch_w8sub(p, sub, cfg.gs, MB, cfg.mr, bf16, s);
   else if (w8) rc = decode2_launch_w8(p, cfg.gs, MB, cfg.mr, bf16, s);

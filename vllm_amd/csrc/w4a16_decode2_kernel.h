@@ -72,6 +72,7 @@ static inline uint32_t d2_sat32(uint64_t bytes) { return bytes > 0xffffffffull ?
 constexpr int D2_WAVES = 16;
 constexpr int DECODE2_MAX_M = 64;           // rows of one workgroup: up to four m-blocks of 16
 constexpr int DECODE2_MAX_M_ROWS = 256;     // rows when every m-block has workgroups of its own (see MSP)
+enum { D2_TILE, D2_WORKGROUP, D2_ROWS };    // see w4a16_decode2_choose
 
 template <bool BF16, int GS, int MB, bool HAS_ZP, int MR, int SUBG, int WT = 0, int RC = 0, bool MSP = false>
 __global__ __launch_bounds__(D2_WAVES * 64) void w4a16_decode2_kernel(const Decode2Params p) {
@@ -102,6 +103,8 @@ __global__ __launch_bounds__(D2_WAVES * 64) void w4a16_decode2_kernel(const Deco
   //    share a compute unit and overlap each other (about 28 KiB in flight per unit; deeper rings measured 2-6 % slower
   //    on 4096 x 28672).  (Four slots with 16 staged rows: the activation fill takes 2 us during which nothing else is
   //    requested, and four tiles in flight fill that gap.)
+  //    Groups of 64 / 32 rows: each slot holds two or four rows of scales and zero points, and deep rings spill: up front at
+  //    most four tiles, else two slots.
   //  * Long streams, RC = 1 / 2: four / three slots, each refilled only after its tile's arithmetic has been issued: no
   //    register copies, and the wait in front of a tile leaves the other R - 1 tiles in flight.  For launches with at
   //    most 8 wavefronts per compute unit, which are latency-bound with two slots (14336 x 4096 at M = 1: 9.2 -> 8.0 us
@@ -114,11 +117,11 @@ __global__ __launch_bounds__(D2_WAVES * 64) void w4a16_decode2_kernel(const Deco
   constexpr bool SPRE = MB >= 2 && WT == 0 && SUBG == 1;
   constexpr int LPT = 1 + SUBG * (HAS_ZP ? 2 : 1);              // vector-memory instructions per tile request
   constexpr int R_SHORT = (GS < 63 / LPT ? GS : 63 / LPT) & (WT != 0 ? ~1 : ~0);      // (8-bit weights: whole block pairs)
-  constexpr bool SHORT = MR <= 4 && GS <= 8 && GS >= 2;
+  constexpr bool SHORT = MR <= 4 && GS <= (SUBG > 1 ? 4 : 8) && GS >= 2;
   constexpr bool LATE = RC != 0 && !SHORT;
   constexpr int R_LATE = RC == 1 ? 4 : (RC == 2 ? 3 : 2);
   static_assert(!(WT != 0 && RC != 0), "8-bit weights take the block of a tile from the slot parity: even rings only");
-  constexpr int R = SHORT ? R_SHORT : (LATE ? (GS < R_LATE ? GS : R_LATE) : ((MR >= 8 && MB == 1 && GS >= 7) ? 4 : (GS < 2 ? GS : 2)));
+  constexpr int R = SHORT ? R_SHORT : (LATE ? (GS < R_LATE ? GS : R_LATE) : ((MR >= 8 && MB == 1 && GS >= 7 && SUBG == 1) ? 4 : (GS < 2 ? GS : 2)));
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
   const int lane = threadIdx.x;

@@ -11,11 +11,13 @@ int w4a16_decode_launch(const void* a, int64_t lda, const int32_t* b, const void
                         int32_t* counters, int64_t counter_ints, int M, int N, int K, bool channelwise, int dtype,
                         hipStream_t s);
 int w4a16_decode2_workspace(int M, int N, int K, int sub, bool w8, size_t* c_tmp_bytes, size_t* counter_ints);
-bool w4a16_decode2_takes_rows(int M, int N, int K, int sub, int wt, bool has_perm);
+int w4a16_decode2_choose(int M, int N, int K, int sub, int wt, bool has_perm, bool wg_ok, bool tile_ok, double tile_us);
+double w4a16_prefill_us(int M, int N, int K, bool reg_ok);
+enum { D2_TILE, D2_WORKGROUP, D2_ROWS };
 int w4a16_decode2_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
                          const int32_t* perm, const void* bias, void* c, float* c_tmp, int64_t c_tmp_bytes,
                          int32_t* counters, int64_t counter_ints, int M, int N, int K, int sub, bool channelwise,
-                         int wt, int dtype, hipStream_t s);      // wt: 0 4-bit codes, 1 8-bit codes, 2 FP8 e4m3 bytes
+                         int wt, int dtype, bool rows, hipStream_t s);      // wt: 0 4-bit codes, 1 8-bit codes, 2 FP8 e4m3 bytes
 int w4a16_prefill_workspace(int M, int N, int K, size_t* c_tmp_bytes, size_t* counter_ints);
 int w4a16_prefill_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
                          const void* bias, void* c, float* c_tmp, int64_t c_tmp_bytes, int32_t* counters,
@@ -85,18 +87,21 @@ extern "C" int vaq_w4a16_gemm_workspace_tuned(int64_t size_m, int64_t size_n, in
       rc = w4a16_decode_workspace((int)size_m, (int)size_n, (int)size_k, &t2, &n2);
       if (rc != VAQ_OK) return rc;
       take();
-      rc = w4a16_decode2_workspace((int)size_m, (int)size_n, (int)size_k, 2, false, &t2, &n2);   // groups below 128 rows
-      if (rc != VAQ_OK) return rc;
-      take();
-      rc = w4a16_decode2_workspace((int)size_m, (int)size_n, (int)size_k, 1, true, &t2, &n2);    // 8-bit codes
-      if (rc != VAQ_OK) return rc;
-      take();
-    } else {
-      // those cases take the prefill kernel above 32 rows
+      for (int sub : {1, 2, 4}) {                              // groups below 128 rows, 8-bit codes
+        for (bool w8 : {false, true}) {
+          if (sub == 1 && !w8) continue;
+          rc = w4a16_decode2_workspace((int)size_m, (int)size_n, (int)size_k, sub, w8, &t2, &n2);
+          if (rc != VAQ_OK) return rc;
+          take();
+        }
+      }
+    }
+    if (size_m > 16) {
+      // those cases take the tile kernel where it is ahead, above 32 rows always or the rows split over workgroups
       rc = w4a16_prefill_workspace((int)size_m, (int)size_n, (int)size_k, &t2, &n2);
       if (rc != VAQ_OK) return rc;
       take();
-      if (has_perm) *a_tmp_bytes = (size_t)size_m * (size_t)size_k * 2;
+      if (has_perm && size_m > DECODE_MAX_M_2BLK) *a_tmp_bytes = (size_t)size_m * (size_t)size_k * 2;
     }
     *c_tmp_bytes = t;
     *counter_ints = n;
@@ -155,22 +160,29 @@ extern "C" int vaq_w4a16_gemm_tuned(const void* a, int64_t lda, const int32_t* b
   const bool two_blocks_only = sub > 1 || w8 || decode_impl_for(size_m, size_n, lda, sub, w8) != 0;
   // (measured: four m-blocks beat the tile kernel by 1.5-2x on the narrow layers and lose 3 % on a 28672-wide one)
   const int64_t dec_max = two_blocks_only ? DECODE_MAX_M_2BLK : (size_n > 8192 ? 48 : DECODE_MAX_M);
-  bool decode = size_m <= dec_max;
-  if (force_path == 1) {
-    VAQ_CHECK_ARG(size_m <= dec_max, "w4a16_gemm: decode path forced with size_m = %lld > %lld", (long long)size_m,
-                  (long long)dec_max);
-    decode = true;
-  } else if (force_path == 2) {
+  bool decode = size_m <= dec_max, rows = false;
+  VAQ_CHECK_ARG(force_path != 1 || decode, "w4a16_gemm: decode path forced with size_m = %lld > %lld", (long long)size_m,
+                (long long)dec_max);
+  if (force_path == 2) {
     decode = false;
-  } else if (!decode && !two_blocks_only && size_m <= 256 && size_n < (1 << 24) && size_k < (1 << 24) &&
-             w4a16_decode2_takes_rows((int)size_m, (int)size_n, (int)size_k, sub, wt, perm != nullptr)) {
-    // more rows than one workgroup of the decode kernel takes, on a layer narrow enough that workgroups of 16 rows each
-    // make one round: ahead of the tile kernel there (see row_split_config in w4a16_decode2.hip); needs no scratch
-    decode = true;
+  } else if (size_m > 16 && size_m <= 256 && size_n < (1 << 24) && size_k < (1 << 24) &&
+             decode_impl_for(size_m, size_n, lda, sub, w8) == 0) {
+    // 17 .. 256 rows: the decode kernel's workgroups of all rows or of 16 rows each, or the tile kernel (where it is given the
+    // scratch that its plan asks for; up to 32 rows that need not be so, and act_order stays with the decode kernel)
+    bool tile_ok = force_path == 0;
+    if (tile_ok && size_m <= DECODE_MAX_M_2BLK) {
+      size_t t = 0, n = 0;
+      w4a16_prefill_workspace((int)size_m, (int)size_n, (int)size_k, &t, &n);
+      tile_ok = perm == nullptr && c_tmp_bytes >= (int64_t)t && counter_ints >= (int64_t)n;
+    }
+    const int kind = w4a16_decode2_choose((int)size_m, (int)size_n, (int)size_k, sub, wt, perm != nullptr, decode, tile_ok || !decode,
+                                          w4a16_prefill_us((int)size_m, (int)size_n, (int)size_k, !w8 && sub == 1));
+    decode = kind != D2_TILE;
+    rows = kind == D2_ROWS;
   }
   if (decode && decode_impl_for(size_m, size_n, lda, sub, w8) == 0)
     return w4a16_decode2_launch(a, lda, b, scales, zeros, perm, bias, c, c_tmp, c_tmp_bytes, counters, counter_ints, (int)size_m,
-                                (int)size_n, (int)size_k, sub, channelwise, wt, dtype, s);
+                                (int)size_n, (int)size_k, sub, channelwise, wt, dtype, rows, s);
   if (decode) {
     VAQ_CHECK_SUPPORTED(sub == 1 && !w8, "w4a16_gemm: group_size = %d / 8-bit weights with an A of 2 GiB or more are not built",
                         group_size);

@@ -106,6 +106,9 @@ static TilePlan plan_prefill(int M, int N, int K, bool direct_ok, bool reg_ok) {
   return table.get(M, N, K, num_cus_current_device() * 2 + (reg_ok ? 1 : 0), [&] { return make_plan_prefill(M, N, K, reg_ok); });
 }
 
+// Predicted time of the tile kernel (negative: not known, register-staged tiles).
+double w4a16_prefill_us(int M, int N, int K, bool reg_ok) { return plan_prefill(M, N, K, true, reg_ok).us; }
+
 int w4a16_prefill_workspace(int M, int N, int K, size_t* c_tmp_bytes, size_t* counter_ints) {
   // enough for either choice of shapes: the weight format is not known here
   const TilePlan a = plan_prefill(M, N, K, true, false), b = plan_prefill(M, N, K, true, true);
