@@ -238,7 +238,9 @@ int vaq_fp8_scaled_mm_ws(const uint8_t* a, int64_t lda, const uint8_t* b, int64_
  * on the scales) or vaq_fp8_quant_static followed by vaq_fp8_scaled_mm.
  *   x  F16/BF16 [M, K], 16-byte aligned, row stride a multiple of 8;  x_scale  fp32 scalar (device) or NULL;
  *   b, sb, bias, out as above, out and bias of the type of x
- * Takes the sizes for which vaq_fp8_quant_scaled_mm_takes is 1: those it is faster for than the two calls.
+ * Takes the sizes for which vaq_fp8_quant_scaled_mm_takes is 1: those it is faster for than the two calls.  Any other size,
+ * and row strides with which b does not end below 2 GiB or x not below 2^30 elements, return VAQ_ERR_UNSUPPORTED and launch
+ * nothing: the two calls take them.
  */
 int vaq_fp8_quant_scaled_mm_takes(int64_t size_m, int64_t size_n, int64_t size_k, int per_token);
 int vaq_fp8_quant_scaled_mm(const void* x, int64_t ldx, const float* x_scale, const uint8_t* b, int64_t ldb, const float* sb,

@@ -133,3 +133,33 @@ def test_no_answer_where_something_is_in_between(device):
     with _tuning.override(quant_wg_per_row=1):
         assert ops._fast.fp8_quant(x, one, None, False, None) is None
     assert ops._fast.fp8_quant(x, one, None, False, None) is not None
+
+
+def _fp8_codes(n, k, device, seed):
+    """Finite e4m3 codes, made in place (the weights below are 2 GiB)."""
+    g = torch.Generator(device=device).manual_seed(seed)
+    q = torch.empty(n, k, dtype=torch.uint8, device=device)
+    q.random_(0, 0x60, generator=g)
+    return q.view(torch.float8_e4m3fn)
+
+
+@pytest.mark.parametrize("m", [1, 4, 9])
+@pytest.mark.parametrize("static", [False, True])
+def test_fp8_layer_with_weights_that_end_past_2_gib(device, m, static):
+    """Contiguous and strided: few rows leave the kernel that quantises and multiplies, whose offsets are 32-bit."""
+    from vllm_amd import _custom_ops as ops
+    scale = torch.full((1,), 0.01, device=device) if static else None
+    n, k = 270336, 8192
+    big = _fp8_codes(n, k, device, 1)
+    strided = torch.as_strided(big.view(-1), (32, 1024), (2 ** 26 + 2 ** 22, 1))      # the last row ends beyond 2 GiB
+    assert 31 * strided.stride(0) + 1024 > 2 ** 31
+    for w in (big, strided):
+        x = torch.randn(m, w.shape[1], device=device).to(torch.bfloat16)
+        ws = torch.rand(w.shape[0], 1, device=device) * 1e-2 + 1e-3
+        got = ops.fp8_linear(x, w.t(), ws, scale, None, torch.bfloat16, None)
+        assert got is not None and got.shape == (m, w.shape[0])
+        q, s = ops.scaled_fp8_quant(x, scale, use_per_token_if_dynamic=True)
+        cols = torch.cat([torch.arange(min(16, w.shape[0])), torch.arange(w.shape[0] - 16, w.shape[0])]).to(device)
+        ref = (q.float() @ w[cols].float().t()) * s.reshape(-1, 1) * ws[cols].t()
+        # one rounding to bf16 (2^-9) beside fp32 sums of products of like sign at most
+        assert torch.allclose(got[:, cols].float(), ref, rtol=2 ** -8, atol=float(ref.abs().mean()) * 2e-3)

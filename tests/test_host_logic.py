@@ -463,3 +463,17 @@ def test_workspace_from_the_helper_covers_every_batch_size():
             assert lib.vaq_w4a16_gemm_workspace(m, n, k, 0, 0, ctypes.byref(t), ctypes.byref(a), ctypes.byref(c)) == _lib.VAQ_OK
             assert c.value <= marlin_workspace_ints(n), (n, k, m, c.value)
             assert c.value <= marlin_workspace_ints(None), (n, k, m, c.value)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 262144, 8192), (4, 152064, 14336), (2, 131072, 16384), (8, 524288, 4096)])
+@pytest.mark.parametrize("per_token", [0, 1])
+def test_fp8_single_launch_leaves_weights_of_2_gib_to_the_two_calls(m, n, k, per_token):
+    """The kernel that quantises and multiplies in one launch addresses the weights with 32-bit offsets.  What it says to
+    take it has to take: a larger weight belongs to the quantisation kernel and the GEMM (which the caller turns to on 0)."""
+    from vllm_amd import _lib
+    lib = _lib.load()
+    assert lib.vaq_fp8_quant_scaled_mm_takes(m, n, k, per_token) == 0
+    assert lib.vaq_fp8_quant_scaled_mm_takes(m, (2 ** 31 - 1) // k // 16 * 16, k, per_token) == int(k <= 4096 or m <= 4)
+    # a row stride that puts the end of a small weight there: refused as a size of the two calls', not as an error
+    rc = lib.vaq_fp8_quant_scaled_mm(None, k, None, None, 2 ** 31, None, 1, None, None, 32, _lib.VAQ_BF16, 1, 32, k, None)
+    assert rc == _lib.VAQ_ERR_UNSUPPORTED and b"two kernels" in lib.vaq_last_error()

@@ -50,7 +50,8 @@ static int dispatch_rows(const Fp8MMParams& p, int wk, int gx, hipStream_t s) {
 //  * per token, M > 4 up to K = 4096 only (K = 4100 .. 8000: 1-15 % slower than two launches); no M > 4 with 16 steps, whose
 //    registers are full.
 static int quant_mm_steps(int64_t M, int64_t N, int64_t K, bool per_token) {
-  if (M < 1 || M > 8 || K % 16 != 0 || N % 16 != 0) return 0;
+  // (the kernel addresses the weights with 32-bit offsets: they end below 2 GiB whatever the row stride)
+  if (M < 1 || M > 8 || K % 16 != 0 || N % 16 != 0 || N >= (1ll << 31) || K >= (1ll << 31) || N * K >= (1ll << 31)) return 0;
   const int64_t steps = (K + 127) / 128, NT = N / 16, cus = num_cus_current_device();
   if (steps <= 16) return 4;
   if (steps <= 32) return M == 1 || (M <= 4 && NT >= 4 * cus && steps <= 24) ? 8 : 4;

@@ -360,8 +360,8 @@ PyObject* py_scaled_mm(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
 }
 
 // fp8_linear(x, weight, weight_scale, input_scale or None, scale_ub or None, out_dtype, bias) -> Tensor [..., n] | None
-// Activations quantised per token (input_scale None) or with a static per-tensor scale, then the GEMM: two launches, and
-// the quantised activations and their scales are one allocation that nobody else sees.
+// Activations quantised per token (input_scale None) or with a static per-tensor scale, then the GEMM: one launch for a few
+// rows, else two, and the quantised activations and their scales are one allocation that nobody else sees.
 PyObject* py_fp8_linear(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   if (nargs != 7 || !plain_thread() || !THPDtype_Check(v[5])) return decline();
@@ -380,16 +380,16 @@ PyObject* py_fp8_linear(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
   const int64_t k = b->size(0), n = b->size(1);
   int64_t m = 0, ldx = 0;
   if (!as_rows(*x, k, &m, &ldx) || m <= 0) return decline();
-  // a few rows: one launch that quantises what it multiplies
-  if (!ub && x->scalar_type() == out_type && ldx >= k && ldx % 8 == 0 && (m == 1 || ldx < (1 << 24)) && k < (1 << 24) && ((uintptr_t)x->const_data_ptr() % 16) == 0 &&
-      vaq_fp8_quant_scaled_mm_takes(m, n, k, in_scale == nullptr)) {
+  // a few rows: one launch that quantises what it multiplies, unless the strides are beyond it
+  const bool x_ok = x->scalar_type() == out_type && ldx >= k && ldx % 8 == 0 && aligned16(x->const_data_ptr());
+  if (!ub && x_ok && vaq_fp8_quant_scaled_mm_takes(m, n, k, in_scale == nullptr)) {
     TensorBase out = empty({m, n}, out_type, call.device);
     const int rc = vaq_fp8_quant_scaled_mm(x->const_data_ptr(), ldx, in_scale ? (const float*)in_scale->const_data_ptr() : nullptr,
                                            (const uint8_t*)b->const_data_ptr(), b->stride(1), (const float*)sb->const_data_ptr(),
                                            sb->numel(), bias ? bias->const_data_ptr() : nullptr, out.mutable_data_ptr(), n, in_tag, m,
                                            n, k, stream_of(call.device));
-    if (rc != VAQ_OK) return raise_status(rc);
-    return wrap_rows(*x, std::move(out), n);
+    if (rc == VAQ_OK) return wrap_rows(*x, std::move(out), n);
+    if (rc != VAQ_ERR_UNSUPPORTED) return raise_status(rc);
   }
   Fp8Scratch scratch;
   const int r = fp8_scratch(call, m, n, k, scratch);
