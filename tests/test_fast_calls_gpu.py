@@ -163,3 +163,70 @@ def test_fp8_layer_with_weights_that_end_past_2_gib(device, m, static):
         ref = (q.float() @ w[cols].float().t()) * s.reshape(-1, 1) * ws[cols].t()
         # one rounding to bf16 (2^-9) beside fp32 sums of products of like sign at most
         assert torch.allclose(got[:, cols].float(), ref, rtol=2 ** -8, atol=float(ref.abs().mean()) * 2e-3)
+
+
+def test_other_threads_run_while_a_call_allocates(device):
+    """The interpreter's lock is given up around allocation and launch.  Nothing else gives it up here: the interpreter itself
+    would only after 1000 s."""
+    import sys
+    import threading
+    from vllm_amd import _custom_ops as ops
+    x = torch.randn(8192, 4096, device=device, dtype=torch.bfloat16)
+    one = torch.ones(1, device=device)
+    assert ops._fast.fp8_quant(x, one, None, False, None) is not None
+    torch.cuda.empty_cache()      # (every output below is an allocation of its own from the driver)
+    go, ran = threading.Event(), []
+    other = threading.Thread(target=lambda: (go.wait(), ran.append(True)))
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1000)
+    try:
+        other.start()
+        go.set()
+        kept = [ops._fast.fp8_quant(x, one, None, False, None) for _ in range(32)]
+        seen = bool(ran)
+    finally:
+        sys.setswitchinterval(interval)
+        other.join()
+    assert seen, "32 calls, and the other thread had no turn"
+    assert all(torch.equal(q.view(torch.uint8), kept[0][0].view(torch.uint8)) for q, _ in kept)
+
+
+def test_layers_called_from_two_threads(device):
+    """Two threads on streams of their own, a W4A16 layer each and one FP8 layer between them, over sizes of every path
+    (single launch, stream and tile kernels, split K with its counters per stream): the results of one thread alone."""
+    import threading
+    from vllm_amd import _custom_ops as ops
+    from vllm_amd.layers.quantization.input_quant_fp8 import GroupShape
+    from vllm_amd.layers.quantization.utils.w8a8_utils import Fp8LinearOp
+    fp8 = Fp8LinearOp(act_quant_static=False, act_quant_group_shape=GroupShape.PER_TOKEN)
+    layers = [_w4(device, 1024, 512, 128, torch.bfloat16, False), _w4(device, 2048, 256, 32, torch.bfloat16, True)]
+    wq, ws = ops.scaled_fp8_quant((torch.randn(512, 8192, device=device) * 0.05).to(torch.bfloat16), use_per_token_if_dynamic=True)
+    sizes = (1, 5, 16, 33, 100, 300)
+
+    def step(layer, x4, x8):
+        return layer(x4), fp8.apply(x8, wq.t(), ws, torch.bfloat16)
+
+    inputs = [[(torch.randn(m, l.input_size, device=device).to(torch.bfloat16), torch.randn(m, 8192, device=device).to(torch.bfloat16))
+               for m in sizes] for l in layers]
+    expect = [[step(l, *i) for i in per] for l, per in zip(layers, inputs)]
+    torch.cuda.synchronize()
+    errors, start = [], threading.Barrier(2)
+
+    def work(t):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                start.wait(30)
+                got = [[step(layers[t], *i) for i in inputs[t]] for _ in range(60)]
+                torch.cuda.current_stream().synchronize()
+                for round_ in got:
+                    for (a, b), (ra, rb) in zip(round_, expect[t]):
+                        assert torch.equal(a, ra) and torch.equal(b, rb)
+        except BaseException as e:      # noqa: BLE001 (reported by the test below)
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors

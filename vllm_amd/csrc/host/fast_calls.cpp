@@ -59,6 +59,21 @@ bool plain_type(PyObject* o) {
   return THPVariable_CheckExact(o) || _PyType_Lookup(Py_TYPE(o), g_function_name) == g_no_function;
 }
 
+// Allocation and launch run without the interpreter's lock: either can wait -- a launch for a place in a full hardware
+// queue, an allocation for work that has to end before cached blocks can be given back -- and meanwhile the program's
+// other threads go on, among them one that the device itself is waiting for (a host callback written in Python).
+// Everything that touches a Python object comes before or after; an exception takes the lock back on its way out.
+class NoGil {
+ public:
+  NoGil() : state_(PyEval_SaveThread()) {}
+  ~NoGil() { PyEval_RestoreThread(state_); }
+  NoGil(const NoGil&) = delete;
+  NoGil& operator=(const NoGil&) = delete;
+
+ private:
+  PyThreadState* state_;
+};
+
 // A call in progress: which device it runs on, and whether everything seen so far was plain.
 struct Call {
   bool ok = true;
@@ -169,17 +184,21 @@ int w4_gemm(const Call& call, const W4Call& q, int64_t lda, TensorBase& out) {
     if (rc != VAQ_OK) return 0;
     z.m = m; z.n = n; z.k = k; z.flags = flags;
   }
-  if (q.c) out = *q.c;
-  else out = empty({m, n}, dtype, call.device);
-  TensorBase c_tmp, a_tmp;
-  if (z.c_tmp) c_tmp = empty({(int64_t)(z.c_tmp / 4)}, at::kFloat, call.device);
-  if (z.extra) a_tmp = empty({(int64_t)(z.extra / 2)}, dtype, call.device);
-  const int rc = vaq_w4a16_gemm(
-      q.a->const_data_ptr(), lda, (const int32_t*)q.w->const_data_ptr(), q.scales->const_data_ptr(),
-      zp ? (const int32_t*)q.zeros->const_data_ptr() : nullptr, act_order ? (const int32_t*)q.perm->const_data_ptr() : nullptr,
-      q.bias ? q.bias->const_data_ptr() : nullptr, out.mutable_data_ptr(), z.c_tmp ? (float*)c_tmp.mutable_data_ptr() : nullptr,
-      (int64_t)z.c_tmp, z.extra ? a_tmp.mutable_data_ptr() : nullptr, (int32_t*)q.workspace->mutable_data_ptr(),
-      q.workspace->numel(), m, n, k, (int)group_size, dtype_tag(dtype), wtype, 0, stream_of(call.device));
+  int rc;
+  {
+    NoGil nogil;
+    if (q.c) out = *q.c;
+    else out = empty({m, n}, dtype, call.device);
+    TensorBase c_tmp, a_tmp;
+    if (z.c_tmp) c_tmp = empty({(int64_t)(z.c_tmp / 4)}, at::kFloat, call.device);
+    if (z.extra) a_tmp = empty({(int64_t)(z.extra / 2)}, dtype, call.device);
+    rc = vaq_w4a16_gemm(
+        q.a->const_data_ptr(), lda, (const int32_t*)q.w->const_data_ptr(), q.scales->const_data_ptr(),
+        zp ? (const int32_t*)q.zeros->const_data_ptr() : nullptr, act_order ? (const int32_t*)q.perm->const_data_ptr() : nullptr,
+        q.bias ? q.bias->const_data_ptr() : nullptr, out.mutable_data_ptr(), z.c_tmp ? (float*)c_tmp.mutable_data_ptr() : nullptr,
+        (int64_t)z.c_tmp, z.extra ? a_tmp.mutable_data_ptr() : nullptr, (int32_t*)q.workspace->mutable_data_ptr(),
+        q.workspace->numel(), m, n, k, (int)group_size, dtype_tag(dtype), wtype, 0, stream_of(call.device));
+  }
   if (rc != VAQ_OK) {
     raise_status(rc);
     return -1;
@@ -289,12 +308,10 @@ bool fp8_weight_ok(const TensorBase& b, const TensorBase& sb, const TensorBase* 
   return !bias || (bias->dim() == 1 && bias->numel() == n && bias->is_contiguous() && bias->scalar_type() == out_type);
 }
 
-// The scratch of one GEMM, found before anything is launched.  1 ready, 0 not this way, -1 an exception is set.
+// What one GEMM needs for its K split, found before anything is launched.  1 ready, 0 not this way, -1 an exception is set.
 struct Fp8Scratch {
-  TensorBase c_tmp;
   size_t c_tmp_bytes = 0;
-  int32_t* counters = nullptr;
-  int64_t counter_ints = 0;
+  TensorBase counters;      // (a reference of its own: the table of counters may change while the lock is given up)
   void* stream = nullptr;
 };
 int fp8_scratch(const Call& call, int64_t m, int64_t n, int64_t k, Fp8Scratch& s) {
@@ -316,20 +333,22 @@ int fp8_scratch(const Call& call, int64_t m, int64_t n, int64_t k, Fp8Scratch& s
   if (!t || !THPVariable_Check(t)) return PyErr_Occurred() ? -1 : 0;
   const TensorBase& c = THPVariable_Unpack(t);
   if (c.numel() < (int64_t)z.extra) return 0;
-  s.counters = (int32_t*)c.mutable_data_ptr();
-  s.counter_ints = c.numel();
-  s.c_tmp = empty({(int64_t)(z.c_tmp / 4)}, at::kFloat, call.device);
+  s.counters = c;
   return 1;
 }
 
+// (without the lock)
 int fp8_mm(const Fp8Scratch& s, const void* a, int64_t lda, int64_t m, const float* sa, int64_t sa_count, const TensorBase& b,
            const TensorBase& sb, const TensorBase* bias, const TensorBase& out) {
   const int64_t k = b.size(0), n = b.size(1);
+  TensorBase c_tmp;
+  if (s.c_tmp_bytes) c_tmp = empty({(int64_t)(s.c_tmp_bytes / 4)}, at::kFloat, out.device().index());
   return vaq_fp8_scaled_mm_ws((const uint8_t*)a, lda, (const uint8_t*)b.const_data_ptr(), b.stride(1), sa, sa_count,
                               (const float*)sb.const_data_ptr(), sb.numel(), bias ? bias->const_data_ptr() : nullptr,
                               out.mutable_data_ptr(), n, dtype_tag(out.scalar_type()), m, n, k,
-                              s.c_tmp_bytes ? (float*)s.c_tmp.mutable_data_ptr() : nullptr, (int64_t)s.c_tmp_bytes, s.counters,
-                              s.counter_ints, s.stream);
+                              s.c_tmp_bytes ? (float*)c_tmp.mutable_data_ptr() : nullptr, (int64_t)s.c_tmp_bytes,
+                              s.c_tmp_bytes ? (int32_t*)s.counters.mutable_data_ptr() : nullptr,
+                              s.c_tmp_bytes ? s.counters.numel() : 0, s.stream);
 }
 
 // scaled_mm(a, b, scale_a, scale_b, out_dtype, bias) -> Tensor [..., n] | None
@@ -352,8 +371,13 @@ PyObject* py_scaled_mm(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
   const int r = fp8_scratch(call, m, b->size(1), b->size(0), scratch);
   if (r < 0) return nullptr;
   if (r == 0) return decline();
-  TensorBase out = empty({m, b->size(1)}, out_type, call.device);
-  const int rc = fp8_mm(scratch, a->const_data_ptr(), lda, m, (const float*)sa->const_data_ptr(), sa->numel(), *b, *sb, bias, out);
+  TensorBase out;
+  int rc;
+  {
+    NoGil nogil;
+    out = empty({m, b->size(1)}, out_type, call.device);
+    rc = fp8_mm(scratch, a->const_data_ptr(), lda, m, (const float*)sa->const_data_ptr(), sa->numel(), *b, *sb, bias, out);
+  }
   if (rc != VAQ_OK) return raise_status(rc);
   return wrap_rows(*a, std::move(out), b->size(1));
   END_HANDLE_TH_ERRORS
@@ -380,14 +404,19 @@ PyObject* py_fp8_linear(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
   const int64_t k = b->size(0), n = b->size(1);
   int64_t m = 0, ldx = 0;
   if (!as_rows(*x, k, &m, &ldx) || m <= 0) return decline();
+  TensorBase out;
+  int rc;
   // a few rows: one launch that quantises what it multiplies, unless the strides are beyond it
   const bool x_ok = x->scalar_type() == out_type && ldx >= k && ldx % 8 == 0 && aligned16(x->const_data_ptr());
   if (!ub && x_ok && vaq_fp8_quant_scaled_mm_takes(m, n, k, in_scale == nullptr)) {
-    TensorBase out = empty({m, n}, out_type, call.device);
-    const int rc = vaq_fp8_quant_scaled_mm(x->const_data_ptr(), ldx, in_scale ? (const float*)in_scale->const_data_ptr() : nullptr,
-                                           (const uint8_t*)b->const_data_ptr(), b->stride(1), (const float*)sb->const_data_ptr(),
-                                           sb->numel(), bias ? bias->const_data_ptr() : nullptr, out.mutable_data_ptr(), n, in_tag, m,
-                                           n, k, stream_of(call.device));
+    {
+      NoGil nogil;
+      out = empty({m, n}, out_type, call.device);
+      rc = vaq_fp8_quant_scaled_mm(x->const_data_ptr(), ldx, in_scale ? (const float*)in_scale->const_data_ptr() : nullptr,
+                                   (const uint8_t*)b->const_data_ptr(), b->stride(1), (const float*)sb->const_data_ptr(),
+                                   sb->numel(), bias ? bias->const_data_ptr() : nullptr, out.mutable_data_ptr(), n, in_tag, m,
+                                   n, k, stream_of(call.device));
+    }
     if (rc == VAQ_OK) return wrap_rows(*x, std::move(out), n);
     if (rc != VAQ_ERR_UNSUPPORTED) return raise_status(rc);
   }
@@ -395,15 +424,18 @@ PyObject* py_fp8_linear(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
   const int r = fp8_scratch(call, m, n, k, scratch);
   if (r < 0) return nullptr;
   if (r == 0) return decline();
-  const int64_t codes = m * k;      // (a multiple of 16: the scales behind them are aligned)
-  TensorBase q = empty({codes + (in_scale ? 0 : 4 * m)}, at::kByte, call.device);
-  uint8_t* qp = (uint8_t*)q.mutable_data_ptr();
-  const float* sa = in_scale ? (const float*)in_scale->const_data_ptr() : (const float*)(qp + codes);
-  TensorBase out = empty({m, n}, out_type, call.device);
-  int rc = in_scale ? vaq_fp8_quant_static(x->const_data_ptr(), in_tag, ldx, qp, k, sa, m, k, scratch.stream)
-                    : vaq_fp8_quant_per_token(x->const_data_ptr(), in_tag, ldx, qp, k, (float*)(qp + codes),
-                                              ub ? (const float*)ub->const_data_ptr() : nullptr, m, k, scratch.stream);
-  if (rc == VAQ_OK) rc = fp8_mm(scratch, qp, k, m, sa, in_scale ? 1 : m, *b, *sb, bias, out);
+  {
+    NoGil nogil;
+    const int64_t codes = m * k;      // (a multiple of 16: the scales behind them are aligned)
+    TensorBase q = empty({codes + (in_scale ? 0 : 4 * m)}, at::kByte, call.device);
+    uint8_t* qp = (uint8_t*)q.mutable_data_ptr();
+    const float* sa = in_scale ? (const float*)in_scale->const_data_ptr() : (const float*)(qp + codes);
+    out = empty({m, n}, out_type, call.device);
+    rc = in_scale ? vaq_fp8_quant_static(x->const_data_ptr(), in_tag, ldx, qp, k, sa, m, k, scratch.stream)
+                  : vaq_fp8_quant_per_token(x->const_data_ptr(), in_tag, ldx, qp, k, (float*)(qp + codes),
+                                            ub ? (const float*)ub->const_data_ptr() : nullptr, m, k, scratch.stream);
+    if (rc == VAQ_OK) rc = fp8_mm(scratch, qp, k, m, sa, in_scale ? 1 : m, *b, *sb, bias, out);
+  }
   if (rc != VAQ_OK) return raise_status(rc);
   return wrap_rows(*x, std::move(out), n);
   END_HANDLE_TH_ERRORS
@@ -429,17 +461,20 @@ PyObject* py_fp8_quant(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
                 given->stride(1) != 1))
     return decline();
   if ((scale && !one_float(*scale)) || (ub && !one_float(*ub))) return decline();
-  TensorBase out = given ? *given : empty({m, k}, at::kFloat8_e4m3fn, call.device);
-  void* stream = stream_of(call.device);
-  TensorBase scales;
+  TensorBase out, scales;
   int rc;
-  if (scale) {
-    rc = vaq_fp8_quant_static(x->const_data_ptr(), in_tag, x->stride(0), (uint8_t*)out.mutable_data_ptr(), out.stride(0),
-                              (const float*)scale->const_data_ptr(), m, k, stream);
-  } else {
-    scales = empty({m, 1}, at::kFloat, call.device);
-    rc = vaq_fp8_quant_per_token(x->const_data_ptr(), in_tag, x->stride(0), (uint8_t*)out.mutable_data_ptr(), out.stride(0),
-                                 (float*)scales.mutable_data_ptr(), ub ? (const float*)ub->const_data_ptr() : nullptr, m, k, stream);
+  {
+    NoGil nogil;
+    out = given ? *given : empty({m, k}, at::kFloat8_e4m3fn, call.device);
+    void* stream = stream_of(call.device);
+    if (scale) {
+      rc = vaq_fp8_quant_static(x->const_data_ptr(), in_tag, x->stride(0), (uint8_t*)out.mutable_data_ptr(), out.stride(0),
+                                (const float*)scale->const_data_ptr(), m, k, stream);
+    } else {
+      scales = empty({m, 1}, at::kFloat, call.device);
+      rc = vaq_fp8_quant_per_token(x->const_data_ptr(), in_tag, x->stride(0), (uint8_t*)out.mutable_data_ptr(), out.stride(0),
+                                   (float*)scales.mutable_data_ptr(), ub ? (const float*)ub->const_data_ptr() : nullptr, m, k, stream);
+    }
   }
   if (rc != VAQ_OK) return raise_status(rc);
   return Py_BuildValue("(NN)", given ? Py_NewRef(v[4]) : THPVariable_Wrap(std::move(out)),
@@ -470,12 +505,17 @@ PyObject* py_rms_norm_dynamic_quant(PyObject*, PyObject* const* v, Py_ssize_t na
   if (PyErr_Occurred() || !norm_ok(*x, *weight, residual, &tokens, &stride) || (ub && !one_float(*ub))) return decline();
   // (the output takes the memory format of the input: the rows of a strided one are left to the registered op)
   if (!x->is_contiguous()) return decline();
-  TensorBase out = empty(x->sizes(), at::kFloat8_e4m3fn, call.device);
-  TensorBase scales = empty({tokens, 1}, at::kFloat, call.device);
-  const int rc = vaq_rms_norm_dynamic_per_token_fp8_quant(
-      (uint8_t*)out.mutable_data_ptr(), (float*)scales.mutable_data_ptr(), x->const_data_ptr(), stride, weight->const_data_ptr(),
-      ub ? (const float*)ub->const_data_ptr() : nullptr, (float)eps, residual ? residual->mutable_data_ptr() : nullptr,
-      dtype_tag(x->scalar_type()), tokens, x->size(-1), stream_of(call.device));
+  TensorBase out, scales;
+  int rc;
+  {
+    NoGil nogil;
+    out = empty(x->sizes(), at::kFloat8_e4m3fn, call.device);
+    scales = empty({tokens, 1}, at::kFloat, call.device);
+    rc = vaq_rms_norm_dynamic_per_token_fp8_quant(
+        (uint8_t*)out.mutable_data_ptr(), (float*)scales.mutable_data_ptr(), x->const_data_ptr(), stride, weight->const_data_ptr(),
+        ub ? (const float*)ub->const_data_ptr() : nullptr, (float)eps, residual ? residual->mutable_data_ptr() : nullptr,
+        dtype_tag(x->scalar_type()), tokens, x->size(-1), stream_of(call.device));
+  }
   if (rc != VAQ_OK) return raise_status(rc);
   return Py_BuildValue("(NN)", THPVariable_Wrap(std::move(out)), THPVariable_Wrap(std::move(scales)));
   END_HANDLE_TH_ERRORS
@@ -497,10 +537,14 @@ PyObject* py_rms_norm_static_quant(PyObject*, PyObject* const* v, Py_ssize_t nar
   if (PyErr_Occurred() || !norm_ok(*x, *weight, residual, &tokens, &stride) || !one_float(*scale) ||
       out->scalar_type() != at::kFloat8_e4m3fn || !out->is_contiguous() || out->numel() != x->numel())
     return decline();
-  const int rc = vaq_rms_norm_static_fp8_quant((uint8_t*)out->mutable_data_ptr(), x->const_data_ptr(), stride, weight->const_data_ptr(),
-                                               (const float*)scale->const_data_ptr(), (float)eps,
-                                               residual ? residual->mutable_data_ptr() : nullptr, dtype_tag(x->scalar_type()),
-                                               tokens, x->size(-1), stream_of(call.device));
+  int rc;
+  {
+    NoGil nogil;
+    rc = vaq_rms_norm_static_fp8_quant((uint8_t*)out->mutable_data_ptr(), x->const_data_ptr(), stride, weight->const_data_ptr(),
+                                       (const float*)scale->const_data_ptr(), (float)eps,
+                                       residual ? residual->mutable_data_ptr() : nullptr, dtype_tag(x->scalar_type()),
+                                       tokens, x->size(-1), stream_of(call.device));
+  }
   if (rc != VAQ_OK) return raise_status(rc);
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -520,8 +564,12 @@ PyObject* py_silu_and_mul_quant(PyObject*, PyObject* const* v, Py_ssize_t nargs)
     return decline();
   const int64_t d = x->size(-1) / 2, tokens = x->numel() / (2 * d);
   if (tokens <= 0 || out->numel() != tokens * d) return decline();
-  const int rc = vaq_silu_and_mul_fp8_quant((uint8_t*)out->mutable_data_ptr(), x->const_data_ptr(), (const float*)scale->const_data_ptr(),
-                                            dtype_tag(x->scalar_type()), tokens, d, stream_of(call.device));
+  int rc;
+  {
+    NoGil nogil;
+    rc = vaq_silu_and_mul_fp8_quant((uint8_t*)out->mutable_data_ptr(), x->const_data_ptr(), (const float*)scale->const_data_ptr(),
+                                    dtype_tag(x->scalar_type()), tokens, d, stream_of(call.device));
+  }
   if (rc != VAQ_OK) return raise_status(rc);
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -542,12 +590,17 @@ PyObject* py_repack(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
       w->size(1) != (perm ? n : n / pack))
     return decline();
   if (perm && (perm->scalar_type() != at::kInt || !perm->is_contiguous() || (perm->numel() != 0 && perm->numel() != k))) return decline();
-  TensorBase out = empty({k / 16, n * 16 / pack}, at::kInt, call.device);
-  const int32_t* src = (const int32_t*)w->const_data_ptr();
-  int32_t* dst = (int32_t*)out.mutable_data_ptr();
-  const int rc = perm ? vaq_w4a16_repack(src, perm->numel() ? (const int32_t*)perm->const_data_ptr() : nullptr, dst, k, n, (int)bits,
-                                         (int)layout, stream_of(call.device))
-                      : vaq_w4a16_repack_awq(src, dst, k, n, (int)bits, (int)layout, stream_of(call.device));
+  TensorBase out;
+  int rc;
+  {
+    NoGil nogil;
+    out = empty({k / 16, n * 16 / pack}, at::kInt, call.device);
+    const int32_t* src = (const int32_t*)w->const_data_ptr();
+    int32_t* dst = (int32_t*)out.mutable_data_ptr();
+    rc = perm ? vaq_w4a16_repack(src, perm->numel() ? (const int32_t*)perm->const_data_ptr() : nullptr, dst, k, n, (int)bits,
+                                 (int)layout, stream_of(call.device))
+              : vaq_w4a16_repack_awq(src, dst, k, n, (int)bits, (int)layout, stream_of(call.device));
+  }
   if (rc != VAQ_OK) return raise_status(rc);
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
