@@ -477,3 +477,49 @@ def test_fp8_single_launch_leaves_weights_of_2_gib_to_the_two_calls(m, n, k, per
     # a row stride that puts the end of a small weight there: refused as a size of the two calls', not as an error
     rc = lib.vaq_fp8_quant_scaled_mm(None, k, None, None, 2 ** 31, None, 1, None, None, 32, _lib.VAQ_BF16, 1, 32, k, None)
     assert rc == _lib.VAQ_ERR_UNSUPPORTED and b"two kernels" in lib.vaq_last_error()
+
+
+@pytest.mark.parametrize("hook", ["pre", "post", "backward", "all modules", "forward", "subclass"])
+def test_fp8_layer_calls_its_quantisation_module_where_something_hangs_on_it(hook, monkeypatch):
+    """The direct call of an FP8 layer skips the ``QuantFP8`` module: only while calling it would run its forward and nothing
+    else."""
+    import torch.nn.modules.module as module
+    from vllm_amd import _custom_ops as ops
+    from vllm_amd.layers.quantization.input_quant_fp8 import GroupShape, QuantFP8
+    from vllm_amd.layers.quantization.utils.w8a8_utils import Fp8LinearOp
+    x, w, s = torch.zeros(2, 32), torch.zeros(32, 16), torch.ones(1)
+    seen = []
+    monkeypatch.setattr(ops, "fp8_linear", lambda *a: seen.append("direct") or torch.zeros(2, 16))
+    monkeypatch.setattr(ops, "scaled_fp8_quant", lambda t, *a, **k: (t, s))
+    monkeypatch.setattr(ops, "cutlass_scaled_mm", lambda a, b, **k: torch.zeros(a.shape[0], b.shape[1]))
+    op = Fp8LinearOp(act_quant_static=False, act_quant_group_shape=GroupShape.PER_TOKEN)
+    op.apply(x, w, s)
+    assert seen == ["direct"]
+    seen.clear()
+    quant, note, handle = op.quant_fp8, lambda *a: seen.append(hook), None
+    if hook == "pre":
+        handle = quant.register_forward_pre_hook(note)
+    elif hook == "post":
+        handle = quant.register_forward_hook(note)
+    elif hook == "backward":
+        handle = quant.register_full_backward_pre_hook(lambda *a: None)
+    elif hook == "all modules":
+        handle = module.register_module_forward_hook(note)
+    elif hook == "forward":
+        quant.forward = lambda *a: seen.append(hook) or (x, s)
+    else:
+        class Other(QuantFP8):
+            def forward(self, *a):
+                seen.append(hook)
+                return super().forward(*a)
+        op.quant_fp8 = Other(static=False, group_shape=GroupShape.PER_TOKEN)
+    try:
+        assert op.apply(x, w, s).shape == (2, 16)
+        assert seen == ([] if hook == "backward" else [hook])
+    finally:
+        if handle is not None:
+            handle.remove()
+    if handle is not None:
+        seen.clear()
+        op.apply(x, w, s)
+        assert seen == ["direct"]

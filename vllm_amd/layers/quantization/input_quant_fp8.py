@@ -6,6 +6,7 @@ from __future__ import annotations
 from typing import NamedTuple
 
 import torch
+import torch.nn.modules.module as _module
 
 from vllm_amd import _custom_ops as ops
 
@@ -43,6 +44,14 @@ class QuantFP8(torch.nn.Module):
                                     and scale_ub.numel() == 1)
         return ops.scaled_fp8_quant(x, scale, num_token_padding=self.num_token_padding, scale_ub=scale_ub,
                                     use_per_token_if_dynamic=self.use_per_token_if_dynamic)
+
+    def runs_forward_only(self) -> bool:
+        """Whether a call of this module is a call of ``forward`` above: no hooks, of its own or of all modules, no other
+        ``forward``.  (A layer's direct call does what ``forward`` does without calling it.)"""
+        return not (self._forward_pre_hooks or self._forward_hooks or self._backward_pre_hooks or self._backward_hooks
+                    or _module._global_forward_pre_hooks or _module._global_forward_hooks
+                    or _module._global_backward_pre_hooks or _module._global_backward_hooks
+                    or self._compiled_call_impl is not None or "forward" in self.__dict__)
 
     forward_cuda = forward
     forward_hip = forward

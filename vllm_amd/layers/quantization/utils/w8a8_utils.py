@@ -39,9 +39,10 @@ class Fp8LinearOp:
     def apply(self, input: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor,
               out_dtype: torch.dtype | None = None, input_scale: torch.Tensor | None = None,
               input_scale_ub: torch.Tensor | None = None, bias: torch.Tensor | None = None) -> torch.Tensor:
-        static = self.act_quant_static
+        static, quant = self.act_quant_static, self.quant_fp8
         if input.dtype != ops.FP8_DTYPE and (input_scale is not None) == static and \
-                (input_scale_ub is None if static else self.act_quant_per_token):
+                (input_scale_ub is None if static else self.act_quant_per_token) and \
+                not torch.compiler.is_dynamo_compiling() and type(quant) is QuantFP8 and quant.runs_forward_only():
             output = ops.fp8_linear(input, weight, weight_scale, input_scale, input_scale_ub, out_dtype or input.dtype, bias)
             if output is not None:
                 return output
