@@ -230,3 +230,16 @@ def test_layers_called_from_two_threads(device):
     for t in threads:
         t.join()
     assert not errors, errors
+
+
+def test_an_override_on_one_thread_leaves_the_others_their_direct_calls(device):
+    import threading
+    from vllm_amd import _custom_ops as ops, _tuning
+    x, one = torch.randn(4, 64, device=device).to(torch.bfloat16), torch.ones(1, device=device)
+    answers = []
+    with _tuning.override(quant_wg_per_row=1):
+        t = threading.Thread(target=lambda: answers.append(ops._fast.fp8_quant(x, one, None, False, None)))
+        t.start()
+        t.join()
+        assert ops._fast.fp8_quant(x, one, None, False, None) is None
+    assert answers[0] is not None

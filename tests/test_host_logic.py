@@ -523,3 +523,33 @@ def test_fp8_layer_calls_its_quantisation_module_where_something_hangs_on_it(hoo
         seen.clear()
         op.apply(x, w, s)
         assert seen == ["direct"]
+
+
+def test_tuning_override_leaves_the_direct_calls_of_other_threads_alone():
+    import threading
+    from vllm_amd import _custom_ops, _tuning  # noqa: F401
+    from vllm_amd import _fast_calls
+
+    def state():      # (reads by setting: the same value goes back)
+        was = _fast_calls.tuned(False)
+        _fast_calls.tuned(was)
+        return was
+
+    def on_another_thread():
+        got = []
+        t = threading.Thread(target=lambda: got.append((state(), _tuning.current())))
+        t.start()
+        t.join()
+        return got[0]
+
+    assert state() is False
+    with _tuning.override(fp8_split=2):
+        assert state() is True and on_another_thread() == (False, None)
+        with _tuning.override(fp8_split=3):
+            assert state() is True
+        assert state() is True and _tuning.current().fp8_split == 2
+    assert state() is False
+    with pytest.raises(TypeError):
+        with _tuning.override(no_such_field=1):
+            pass
+    assert state() is False and _tuning.current() is None

@@ -730,8 +730,8 @@ class _NotBuilt:
 
 try:
     from . import _fast_calls as _fast
-    _fast.setup(_FP8_COUNTERS, _tuning.depth, tuple(t.id for t in (scalar_types.uint4, scalar_types.uint4b8,
-                                                                   scalar_types.uint8b128, scalar_types.float8_e4m3fn)))
+    _fast.setup(_FP8_COUNTERS, tuple(t.id for t in (scalar_types.uint4, scalar_types.uint4b8, scalar_types.uint8b128,
+                                                    scalar_types.float8_e4m3fn)))
 except ImportError as e:
     _fast_error = str(e)
     _fast = _NotBuilt()

@@ -10,11 +10,16 @@ import contextlib
 import ctypes
 import threading
 
+import torch  # noqa: F401 (_fast_calls links against its libraries)
+
 from ._lib import VaqTuning
 
+try:
+    from . import _fast_calls
+except ImportError:      # (not built: the ops say so when they are called)
+    _fast_calls = None
+
 _state = threading.local()
-depth = [0]      # overrides in force on any thread: while there are some, every call takes the registered ops
-_depth_lock = threading.Lock()
 
 
 def current() -> VaqTuning | None:
@@ -25,6 +30,13 @@ def current() -> VaqTuning | None:
 def current_ref():
     t = current()
     return None if t is None else ctypes.byref(t)
+
+
+def _set(tuning: VaqTuning | None) -> None:
+    """On this thread; while there is one, the direct calls leave this thread's calls to the registered ops."""
+    _state.tuning = tuning
+    if _fast_calls is not None:
+        _fast_calls.tuned(tuning is not None)
 
 
 @contextlib.contextmanager
@@ -40,12 +52,8 @@ def override(**fields):
         else:
             setattr(t, name, int(value))
     prev = current()
-    with _depth_lock:
-        depth[0] += 1
-    _state.tuning = t
+    _set(t)
     try:
         yield t
     finally:
-        _state.tuning = prev
-        with _depth_lock:
-            depth[0] -= 1
+        _set(prev)

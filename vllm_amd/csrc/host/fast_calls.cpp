@@ -34,7 +34,7 @@ using at::ScalarType;
 using at::TensorBase;
 
 PyObject* g_fp8_counters = nullptr;      // the dict (device index, stream) -> zeroed int32 counters of _custom_ops
-PyObject* g_tuning_depth = nullptr;      // list of one int: tuning overrides in force in this process
+thread_local bool t_tuned = false;       // a tuning override is in force on this thread (vllm_amd/_tuning.py)
 PyObject* g_no_function = nullptr;       // torch._C._disabled_torch_function_impl
 PyObject* g_function_name = nullptr;     // "__torch_function__"
 
@@ -51,7 +51,7 @@ bool plain_keys(const TensorBase& t) {
 bool plain_thread() {
   return (c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty() &&
          !c10::impl::TorchDispatchModeTLS::any_modes_set() && !at::impl::torch_function_mode_enabled() &&
-         !at::hasCallbacks() && PyLong_AsLong(PyList_GET_ITEM(g_tuning_depth, 0)) == 0;
+         !at::hasCallbacks() && !t_tuned;
 }
 
 // Whether operators on `o` run as they are: a Tensor, a Parameter, or a subclass with torch's own disabled __torch_function__.
@@ -606,13 +606,21 @@ PyObject* py_repack(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// setup(fp8_counters: dict, tuning_depth: list, (u4, u4b8, u8b128, fe4m3): ids)
+// tuned(on) -> what it was: whether this thread's calls are left to the registered ops, which pass the override on
+PyObject* py_tuned(PyObject*, PyObject* on) {
+  const int value = PyObject_IsTrue(on);
+  if (value < 0) return nullptr;
+  const bool was = t_tuned;
+  t_tuned = value != 0;
+  return PyBool_FromLong(was);
+}
+
+// setup(fp8_counters: dict, (u4, u4b8, u8b128, fe4m3): ids)
 PyObject* py_setup(PyObject*, PyObject* args) {
-  PyObject *counters, *depth;
+  PyObject* counters;
   long long u4, u4b8, u8b128, fe4m3;
-  if (!PyArg_ParseTuple(args, "O!O!(LLLL)", &PyDict_Type, &counters, &PyList_Type, &depth, &u4, &u4b8, &u8b128, &fe4m3)) return nullptr;
+  if (!PyArg_ParseTuple(args, "O!(LLLL)", &PyDict_Type, &counters, &u4, &u4b8, &u8b128, &fe4m3)) return nullptr;
   Py_XSETREF(g_fp8_counters, Py_NewRef(counters));
-  Py_XSETREF(g_tuning_depth, Py_NewRef(depth));
   if (!g_no_function) {
     PyObject* torch_c = PyImport_ImportModule("torch._C");
     if (!torch_c) return nullptr;
@@ -628,6 +636,7 @@ PyObject* py_setup(PyObject*, PyObject* args) {
 #define FAST(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr}
 PyMethodDef g_methods[] = {
     {"setup", py_setup, METH_VARARGS, nullptr},
+    {"tuned", py_tuned, METH_O, nullptr},
     FAST(w4_gemm), FAST(w4_linear), FAST(scaled_mm), FAST(fp8_linear), FAST(fp8_quant), FAST(rms_norm_dynamic_quant),
     FAST(rms_norm_static_quant), FAST(silu_and_mul_quant), FAST(repack), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_fast_calls", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
