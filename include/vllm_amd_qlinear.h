@@ -129,7 +129,8 @@ int vaq_w4a16_gemm(const void* a, int64_t lda, const int32_t* b, const void* sca
  * file-scope device array of VAQ_STATIC_SCRATCH_COUNTER_INTS ints + VAQ_STATIC_SCRATCH_DATA_BYTES bytes per GPU, which
  * a GPU holds from the library's first use on it until the process ends.  The call allocates and frees nothing.
  * A problem whose scratch (vaq_w4a16_gemm_workspace, without the optional use of c_tmp described above, which this
- * entry point never makes) exceeds that returns VAQ_ERR_INVALID_ARG and launches nothing.
+ * entry point never makes, and with the tile kernel's K split no larger than the permuted activations leave room for)
+ * exceeds that returns VAQ_ERR_INVALID_ARG and launches nothing.
  * Every call on a GPU uses that GPU's one array: calls that may overlap in time on one GPU (different streams or
  * threads) race on it and must be serialised by the caller.  The first call on a GPU looks the array's address up
  * (hipGetSymbolAddress); make it outside any graph capture.

@@ -553,3 +553,26 @@ def test_tuning_override_leaves_the_direct_calls_of_other_threads_alone():
         with _tuning.override(no_such_field=1):
             pass
     assert state() is False and _tuning.current() is None
+
+
+def test_library_owned_scratch_takes_every_act_order_problem_whose_activations_fit():
+    """The K split of a problem on the library's own 16 MiB has to leave room for act_order's permuted activations: every
+    problem whose activations fit is taken, with a smaller split or none.  (Null operands: nothing is ever launched.)"""
+    import random
+    from vllm_amd import _lib
+    lib = _lib.load()
+    rng = random.Random(1)
+    problems = [(2969, 384, 1920), (500, 1984, 3456), (952, 1216, 2816), (73, 5248, 5888), (192, 7168, 2944), (319, 5248, 5120)]
+    problems += [(int(33 * (8000 / 33) ** rng.random()), 64 * int(2 * 200 ** rng.random()), 128 * int(2 * 110 ** rng.random()))
+                 for _ in range(4000)]
+    for m, n, k in problems:
+        if 2 * m * k > _lib_scratch_bytes() - 1024 or m <= 64:
+            continue
+        lib.vaq_w4a16_gemm_static(None, k, None, None, None, 4096, None, None, m, n, k, 128, _lib.VAQ_BF16, _lib.VAQ_WTYPE_U4B8, None)
+        assert b"library-owned" not in lib.vaq_last_error(), (m, n, k, lib.vaq_last_error())
+
+
+def _lib_scratch_bytes():
+    text = open(os.path.join(ROOT, "include", "vllm_amd_qlinear.h")).read()
+    mib = re.search(r"VAQ_STATIC_SCRATCH_DATA_BYTES \((\d+)u << 20\)", text)
+    return int(mib.group(1)) << 20

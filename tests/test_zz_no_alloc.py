@@ -68,3 +68,18 @@ def test_w4a16_gemm_static_rejects_oversized_scratch(device):
     rc = lib.vaq_w4a16_gemm_static(None, 4096, None, None, None, None, None, None, 40, 128256, 4096, 128, _lib.VAQ_BF16,
                                    _lib.VAQ_WTYPE_U4B8, None)
     assert rc == _lib.VAQ_ERR_INVALID_ARG and b"library-owned scratch" in lib.vaq_last_error()
+
+
+@pytest.mark.parametrize("m,n,k", [(192, 7168, 2944), (500, 1984, 3456), (952, 1216, 2816)])
+def test_w4a16_gemm_static_act_order_beside_a_k_split(device, m, n, k):
+    """Problems whose preferred K split leaves no room for the permuted activations: a smaller split gives the same numbers
+    up to the order of the fp32 sums."""
+    from vllm_amd import _lib
+    lib = _lib.load()
+    case = o.make_w4a16_case(k, n, 128, asym=False, act_order=True, seed=m)
+    layer = W4A16Layer(case, device)
+    a = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(torch.bfloat16).to(device)
+    out, ref, sizes = _run_both(lib, _lib, layer, a, m, n, k, True)
+    assert sizes[0] + sizes[1] > 16 << 20, "the preferred split fits: this no longer tests anything"
+    check_gemm_close(out, ref.cpu(), "library-owned scratch against the caller's")
+    check_gemm_close(out, o.gemm_ref(a.cpu(), o.case_w_ref(case)), "library-owned scratch against the oracle")

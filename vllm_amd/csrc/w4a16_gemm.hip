@@ -252,6 +252,10 @@ extern "C" int vaq_w4a16_gemm_static(const void* a, int64_t lda, const int32_t* 
   // tens of MB of partial tiles at thousands of rows, and whole tiles give the same result.
   VaqTuning whole_tiles = {};
   whole_tiles.exp[10] = 1;
+  // What act_order's permuted activations leave of the scratch is what the K split may use for its partial tiles: a plan
+  // that asked for more would have the call refused, where a smaller split, or none, gives the same result.
+  const size_t perm_bytes = perm != nullptr && size_m > DECODE_MAX_M_2BLK && size_k > 0 ? (size_t)size_m * (size_t)size_k * 2 : 0;
+  whole_tiles.exp[14] = perm_bytes + 1024 < STATIC_DATA_BYTES ? (int)((STATIC_DATA_BYTES - perm_bytes) / 1024) : 1;
   int rc = vaq_w4a16_gemm_workspace_tuned(size_m, size_n, size_k, perm != nullptr, 0, &c_tmp_bytes, &a_tmp_bytes, &counter_ints,
                                           &whole_tiles);
   if (rc != VAQ_OK) return rc;

@@ -58,8 +58,8 @@ static TilePlan make_plan_prefill(int M, int N, int K, bool reg_ok) {
   const VaqTuning& tn = tuning();
   const int forced = tn.prefill_tile - 1;
   TilePlan best;
-  // partial tiles are addressed with 32-bit offsets; the entry point on library-owned scratch (exp[10] = 1) holds 16 MiB
-  const int64_t most = tn.exp[10] == 1 ? (int64_t)VAQ_STATIC_SCRATCH_DATA_BYTES : (1ll << 32);
+  // partial tiles are addressed with 32-bit offsets; the entry point on library-owned scratch says what room it has for them
+  const int64_t most = tn.exp[14] > 0 ? (int64_t)tn.exp[14] * 1024 : (1ll << 32);
   for (const TileShape& t : W4_TILE_SHAPES) {
     const bool is256 = t.id == 20;
     if (forced >= 0 ? forced != t.id && !(is256 && (forced == 10 || forced == 11 || forced == 30)) : t.id == 13 && !reg_ok) continue;
