@@ -576,3 +576,31 @@ def _lib_scratch_bytes():
     text = open(os.path.join(ROOT, "include", "vllm_amd_qlinear.h")).read()
     mib = re.search(r"VAQ_STATIC_SCRATCH_DATA_BYTES \((\d+)u << 20\)", text)
     return int(mib.group(1)) << 20
+
+
+def test_price_formula_of_the_fit_is_the_one_of_the_library():
+    """profiles/plan_prices/fit.py restates `decode2_us`: its price of every plan that the library chooses is the library's."""
+    import ctypes
+    import importlib.util
+    import random
+    from vllm_amd import _lib
+    spec = importlib.util.spec_from_file_location("plan_price_fit", os.path.join(ROOT, "profiles", "plan_prices", "fit.py"))
+    fit = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(fit)
+    lib, plan, rng = _lib.load(), (ctypes.c_double * 6)(), random.Random(3)
+    rows, want = [], []
+    for _ in range(300):
+        m, k, n = int(256 ** rng.random()), 128 * int(110 ** rng.random()), 64 * int(2 * 1000 ** rng.random())
+        sub, w8 = rng.choice([1, 2, 4]), rng.choice([0, 1])
+        kind = int(m > 16 and rng.random() < 0.5 or m > 32)
+        if sub == 1 and not w8 and m <= 32:
+            continue      # (by rule, not by price)
+        assert lib.vaq_w4a16_decode_plan(m, n, k, sub, w8, 2 if kind else 0, plan) == _lib.VAQ_OK
+        if plan[5] >= 0:
+            rows.append([k, n, m, sub, w8, kind, plan[0], plan[1], plan[2], 1.0])
+            want.append(plan[5])
+    d = fit.Decode()
+    d.load_rows(np.array(rows))
+    assert len(want) > 150 and np.allclose(d.prices(), want, rtol=1e-9)
+    assert lib.vaq_w4a16_decode_plan(300, 64, 128, 1, 0, 2, plan) == _lib.VAQ_ERR_INVALID_ARG
+    assert lib.vaq_w4a16_decode_plan(40, 64, 100, 1, 0, 2, plan) == _lib.VAQ_ERR_INVALID_ARG

@@ -707,3 +707,16 @@ def test_gemm_reference_grid_weights_quantized_from_float(device, quant_type, ac
         # the reference's own pass criterion, against its own 16-bit matmul
         ref16 = o.gemm_ref_like_reference(a.float(), case["w_ref"].float())
         assert o.rel_err_mean(out.cpu().float(), ref16) < 0.04
+
+
+@pytest.mark.parametrize("bits,group_size", [(4, 128), (4, 64), (4, 32), (8, 128), (8, 64), (8, 32)])
+@pytest.mark.parametrize("k,n", [(256, 33024), (640, 16448), (17408, 128)])
+def test_gemm_very_wide_and_very_long_layers(device, bits, group_size, k, n):
+    """The automatic plan where a layer is many rounds of workgroups of a short K, or one strip of a long one."""
+    case = o.make_w4a16_case(k, n, group_size, asym=False, seed=k + n, num_bits=bits)
+    layer = W4A16Layer(case, device)
+    w_ref = o.case_w_ref(case)
+    for m in (1, 3, 9, 16, 17, 30, 40, 64, 70, 200):
+        a = _acts(m, k, device, seed=m)
+        check_gemm_close(layer(a), o.gemm_ref(a.cpu(), w_ref), f"{bits=} {group_size=} k={k} n={n} m={m}")
+    assert bool((layer.workspace == 0).all()), "workspace counters not restored to zero"

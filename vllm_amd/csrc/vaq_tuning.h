@@ -66,6 +66,13 @@ int vaq_fp8_quant_per_token_tuned(const void* in, int in_dtype, int64_t in_row_s
                                   int64_t out_row_stride, float* scales, const float* scale_ub, int64_t rows,
                                   int64_t hidden, void* stream, const VaqTuning* tuning);
 
+/*
+ * The plan of the W4A16 decode kernel for a problem, without launching anything: plan[0 .. 5] = weight tiles per wavefront, K
+ * slices and n-tiles per workgroup, parts of K, staged rows, predicted us (negative: no plan).  `sub` = groups per 128
+ * rows, `w8` = 8-bit codes, `kind` = 0 workgroups of all rows, 1 the same by the rule instead of the price, 2 of 16 rows.
+ */
+int vaq_w4a16_decode_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub, int w8, int kind, double* plan);
+
 #pragma GCC visibility pop
 #ifdef __cplusplus
 }

@@ -194,36 +194,42 @@ static Decode2Config pick_by_rule(int M, int N, int K, int sub, bool w8, int nt_
 }
 
 // ----------------------------------------------------------------------------- plans by predicted time
-// What a launch costs, in us: per round of workgroups on a compute unit `round`, the activation fill (`fill_kb` per KB staged on it), the
-// stream of weight tiles -- per tile the latency `tile_latency` over the tiles in flight, or the arithmetic of all wavefronts
-// that share the unit, `tile_work` each -- and the reduction over the K slices (`reduce` per doubling); beside that the weights
-// from memory (`mem_mb` per MB, and `again` times that for every further copy of the stream, which L2 serves); `base` per launch;
-// a K split over workgroups costs `handover` + `part` per part + `part_mb` per MB of partial results.
-// [.]: one staged row, 4 or 8, 16.  `sub_work`: groups of 128, 64, 32 rows.
-// Fitted to the cold times of 1.3e5 launches: 3700 random layers (K 1024 .. 14336, N 1024 .. 28672, 1 .. 256 rows), each with up to
-// 60 splits.  The cheapest plan by these figures takes 1.03-1.05 of the fastest one's time (geometric mean).
+// What a launch costs, in us: per round of workgroups on a compute unit `round` over the workgroups that share it, the activation
+// fill (`fill_kb` per KB staged on it), the stream of weight tiles -- per tile `chain` and the latency `tile_latency` over the
+// tiles in flight, or the arithmetic of all wavefronts that share the unit, `tile_work` each -- and the reduction over the K
+// slices (`reduce` per doubling); a started round beyond the first counts by `last` beyond its share; workgroups of two
+// wavefronts, more than four to a unit, take `pair` times as long; beside that the weights from memory (`mem_mb` per MB, and
+// `again` times that for every further copy of the stream, which L2 serves); `base` per launch; a K split over workgroups costs
+// `handover` + `part` per part + `part_mb` per MB of partial results.  [.]: one staged row, 4 or 8, 16.  `sub_work`: groups of
+// 128, 64, 32 rows.
+// Fitted to the cold times of 1.5e5 launches: 6400 problems of random layers, half of them with K 1024 .. 14336 and N 1024 ..
+// 28672, half with K 256 .. 28672 and N 256 .. 152064, 1 .. 256 rows, each with up to 60 splits (profiles/plan_prices).  The cheapest
+// plan by these figures takes 1.02 of the fastest one's time (geometric mean; 99 of 100 less than 1.23), N > 28672 1.03, K or N
+// below 1024 1.014.  Constants of the formula without `chain`, `last` and `pair`, fitted to the first half only, were at 1.047, 1.067
+// and 1.060 over these problems.
 struct Decode2Cost {
   double base, round, fill_kb, mem_mb, again, reduce, handover, part, part_mb;
   double tile_latency[3], tile_work[3], sub_work[3];
+  double chain, last, pair;
 };
-constexpr Decode2Cost D2_COST_W8 = {2.52, 0, 0.0089, 0.187, 0, 0.148, 0.87, 0.21, 0.32,
-                                    {0.96, 1.04, 0.89}, {0.0284, 0.0301, 0.0341}, {1, 1.24, 1.87}};
-constexpr Decode2Cost D2_COST_SUB = {2.41, 0, 0.0089, 0.228, 0, 0.051, 0.87, 0.21, 0,
-                                     {1.11, 1.29, 1.36}, {0.0412, 0.0422, 0.0478}, {1, 1.03, 1.54}};
+constexpr Decode2Cost D2_COST_W8 = {1.09, 1.63, 0.0154, 0.0469, 0, 0.00669, 1.12, 0.275, 0.409,
+                                    {0.9, 0.875, 0.665}, {0.0215, 0.022, 0.0209}, {1.15, 1.35, 1.95}, 0.116, 0.108, 1.29};
+constexpr Decode2Cost D2_COST_SUB = {1.18, 1.3, 0.0144, 0.0468, 0, 0.0041, 1.16, 0.301, 0,
+                                     {0.796, 0.909, 0.834}, {0.0278, 0.0271, 0.028}, {1, 1.11, 1.55}, 0.127, 0.143, 1.35};
 // two m-blocks (groups of 128 rows / channelwise: three and four)
-constexpr Decode2Cost D2_COST_W8_MB2 = {1.08, 0.32, 0.0034, 0.201, 0, 0.57, 0.98, 0.22, 0.31,
-                                        {1.80, 1.80, 1.80}, {0.0586, 0.0586, 0.0586}, {1, 1.20, 1.69}};
-constexpr Decode2Cost D2_COST_SUB_MB2 = {1.04, 0.68, 0.0113, 0.190, 0, 0.23, 1.13, 0.18, 0.16,
-                                         {1.84, 1.84, 1.84}, {0.0643, 0.0643, 0.0643}, {1, 1.25, 1.56}};
-constexpr Decode2Cost D2_COST_MB34 = {1.47, 0.89, 0.0124, 0.229, 0, 0.204, 1.15, 0.18, 0.14,
-                                      {1.97, 1.97, 1.97}, {0.0886, 0.0886, 0.0886}, {1, 1, 1}};
+constexpr Decode2Cost D2_COST_W8_MB2 = {0.149, 0.0523, 0.000908, 0.0746, 0, 0.848, 0.588, 0.231, 0.597,
+                                        {1.8, 1.8, 1.59}, {0.0586, 0.0586, 0.0342}, {1.41, 1.65, 2.41}, 0.142, 0.428, 1.06};
+constexpr Decode2Cost D2_COST_SUB_MB2 = {0.772, 0.979, 0.0147, 0.071, 0, 0.218, 0.395, 0.3, 0.46,
+                                         {1.84, 1.84, 1.63}, {0.0643, 0.0643, 0.0498}, {1, 1.08, 1.46}, 0.0313, 0.379, 0.968};
+constexpr Decode2Cost D2_COST_MB34 = {1.97, 1.26, 0.0179, 0.158, 0, 0.0465, 0.224, 0.328, 0.782,
+                                      {1.97, 1.97, 0.468}, {0.0886, 0.0886, 0.00497}, {1.72, 1, 1}, 0.107, 0.395, 1.2};
 // the rows split over workgroups (never with a split K)
-constexpr Decode2Cost D2_COST_ROWS_W8 = {2.48, 0, 0.0067, 0.250, 0.653, 0.281, 0, 0, 0,
-                                         {0.86, 0.86, 0.86}, {0.0336, 0.0336, 0.0336}, {1, 1.21, 1.81}};
-constexpr Decode2Cost D2_COST_ROWS_SUB = {2.45, 0, 0.0098, 0.298, 0.518, 0.055, 0, 0, 0,
-                                          {1.36, 1.36, 1.36}, {0.0476, 0.0476, 0.0476}, {1, 0.98, 1.48}};
-constexpr Decode2Cost D2_COST_ROWS = {2.23, 0, 0.0104, 0.233, 0.779, 0.105, 0, 0, 0,
-                                      {1.02, 1.02, 1.02}, {0.037, 0.037, 0.037}, {1, 1, 1}};
+constexpr Decode2Cost D2_COST_ROWS_W8 = {1.51, 1.63, 0.00925, 0.341, 0.124, 0.0156, 0, 0, 0,
+                                         {0.86, 0.86, 0.389}, {0.0336, 0.0336, 0.0171}, {1.33, 1.57, 2.22}, 0.126, 0.138, 1.2};
+constexpr Decode2Cost D2_COST_ROWS_SUB = {1.54, 1.24, 0.0103, 0.229, 0.267, 0.00948, 0, 0, 0,
+                                          {1.36, 1.36, 0.0918}, {0.0476, 0.0476, 0.0195}, {1, 1.49, 2.01}, 0.151, 0.153, 1.2};
+constexpr Decode2Cost D2_COST_ROWS = {1.4, 1.16, 0.0093, 0.0946, 0.368, 0.0106, 0, 0, 0,
+                                      {1.02, 1.02, 0.392}, {0.037, 0.037, 0.0181}, {1.74, 1, 1}, 0.107, 0.237, 1.2};
 
 static const Decode2Cost& workgroup_cost(int M, int sub, bool w8) {
   if (w8) return M > 16 ? D2_COST_W8_MB2 : D2_COST_W8;
@@ -236,14 +242,17 @@ static double decode2_us(const Decode2Cost& t, const Decode2Config& c, int M, in
   const int ri = c.mr == 1 ? 0 : c.mr <= 8 ? 1 : 2;
   const long slots = wg_slots(c.wks * c.wn, decode2_lds_bytes(c.wks, c.gs / TPG, c.mr, MB));
   const long wgs = (long)((N / 16 + c.wn - 1) / c.wn) * c.sk * copies, per_cu = (wgs + cus - 1) / cus;
-  const double rounds = (double)((per_cu + slots - 1) / slots), side = (double)(per_cu < slots ? per_cu : slots);
+  const double side = (double)(per_cu < slots ? per_cu : slots), even = (double)per_cu / (double)slots;
+  const double rounds = per_cu > slots ? even + t.last * ((double)((per_cu + slots - 1) / slots) - even) : 1;
   const bool whole = c.mr <= 4 && c.gs <= (sub > 1 ? 4 : 8);      // short streams with few rows are requested whole
   const double flight = whole || c.gs < 3 ? c.gs : 3;
   auto p4 = [](double x) { return x * x * x * x; };
   const double tile = sqrt(sqrt(p4(t.tile_latency[ri] / flight) +
-                                p4(side * c.wks * c.wn * t.tile_work[ri] * t.sub_work[sub == 4 ? 2 : sub - 1])));
+                                p4(side * c.wks * c.wn * t.tile_work[ri] * t.sub_work[sub == 4 ? 2 : sub - 1]))) +
+                      t.chain * t.sub_work[sub == 4 ? 2 : sub - 1];
   const double fill = t.fill_kb * side * (c.wks * c.gs / TPG) * (c.mr * MB * 256 / 1024.0);
-  const double core = rounds * (t.round + fill + c.gs * tile + t.reduce * log2((double)c.wks));
+  const double slow = c.wks * c.wn == 2 && per_cu > 4 ? t.pair : 1;
+  const double core = slow * rounds * (t.round / (double)slots + fill + c.gs * tile + t.reduce * log2((double)c.wks));
   const double mem = t.mem_mb * 0.5e-6 * (double)K * N * TPG * (1 + t.again * (copies - 1));
   double us = t.base + cbrt(core * core * core + mem * mem * mem);
   if (c.sk > 1) us += t.handover + c.sk * (t.part + t.part_mb * 4e-6 * (double)M * N);
@@ -303,15 +312,17 @@ static Decode2Plan cheapest_decode2(const Decode2Cost& t, int M, int N, int K, i
 
 // One workgroup for all rows (up to two m-blocks; 4-bit codes in groups of 128 rows / channelwise: up to four).  The rule for the
 // latter, whose choices are within 2-4 % of the predicted ones up to two m-blocks.  For the other formats, which the rule was not
-// made for, the cheapest plan, with 8-bit codes where it is predicted 5 % ahead (M = 1 .. 4 over random layers, mean: 8-bit codes 1.13 -> 1.04 of the
-// fastest plan's time, groups of 64 / 32 rows 1.13 -> 1.04).
+// made for, the cheapest plan where it is predicted 5 % (4-bit codes in groups of 64 / 32 rows, up to 16 rows: 8 %) ahead of the
+// rule's: nearer than that the price is more often wrong than right (over 3863 problems the mean gain over the rule is 4.7-10.4 %
+// either way, the share that is 5 % slower than by the rule falls from 3-8 % to 1-3 %).
 static Decode2Plan plan_workgroup(int M, int N, int K, int sub, bool w8) {
   Decode2Plan p;
   p.c = pick_by_rule(M, N, K, sub, w8);
   p.us = decode2_us(workgroup_cost(M, sub, w8), p.c, M, N, K, sub, w8, (M + 15) / 16, 1);
   if (sub > 1 || w8) {
     const Decode2Plan q = cheapest_decode2(workgroup_cost(M, sub, w8), M, N, K, sub, w8, false);
-    if (q.us >= 0 && q.us < (w8 ? 0.95 : 1.0) * p.us) return q;
+    const double ahead = w8 || M > 16 ? 0.95 : 0.92;
+    if (q.us >= 0 && q.us < ahead * p.us) return q;
   }
   return p;
 }
@@ -401,7 +412,10 @@ int w4a16_decode2_choose(int M, int N, int K, int sub, int wt, bool has_perm, bo
     return r.us >= 0 && wgs <= num_cus_current_device() && r.c.wks * r.c.wn >= 8 ? D2_ROWS : D2_WORKGROUP;
   }
   int best = D2_TILE;
-  double us = tile_ok ? tile_us + (has_perm ? 4.0 : 0.0) : -1;      // (act_order: a launch that permutes the columns first)
+  // (The tile kernel's price is that of 4-bit codes and 2-5 % low at these sizes, 9-13 % with 8-bit codes; the prices of these
+  // workgroups are 3-9 % low.  With these factors the kind chosen is within 0.2 - 0.6 % of the fastest one's time in the mean,
+  // 1.3 % for groups of 64 / 32 rows at 17 .. 32 rows; 6600 problems.  act_order: a launch that permutes the columns first.)
+  double us = tile_ok ? tile_us * (!w8 ? 1.04 : M <= 64 ? 1.06 : 1.0) + (has_perm ? 4.0 : 0.0) : -1;
   if (wg_ok) {
     const double t = workgroup_plan(M, N, K, sub, w8).us;
     if (us < 0 || t < us) { us = t; best = D2_WORKGROUP; }
@@ -413,6 +427,28 @@ int w4a16_decode2_choose(int M, int N, int K, int sub, int wt, bool has_perm, bo
 int decode2_launch_msp(const Decode2Params& p, int gs, int rc, bool bf16, bool zp, hipStream_t s);      // w4a16_decode2_msp.hip
 int decode2_launch_msp_sub(const Decode2Params& p, int sub, int gs, bool bf16, bool zp, hipStream_t s);     // w4a16_decode2_msp_sub.hip
 int decode2_launch_msp_w8(const Decode2Params& p, int sub, int gs, bool bf16, hipStream_t s);               // w4a16_decode2_msp_w8.hip
+
+}  // namespace vaq
+
+extern "C" int vaq_w4a16_decode_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub, int w8, int kind, double* plan) {
+  using namespace vaq;
+  VAQ_CHECK_ARG(size_m > 0 && size_m <= DECODE2_MAX_M_ROWS && size_n > 0 && size_n % 64 == 0 && size_k > 0 && size_k % 128 == 0 &&
+                    size_n < (1 << 24) && size_k < (1 << 24) && (sub == 1 || sub == 2 || sub == 4) && plan != nullptr &&
+                    (kind == 2 || size_m <= DECODE2_MAX_M), "w4a16_decode_plan: bad arguments");
+  const int M = (int)size_m, N = (int)size_n, K = (int)size_k;
+  Decode2Plan p;
+  if (kind == 2) p = rows_plan(M, N, K, sub, w8 != 0);
+  else if (kind == 0) p = workgroup_plan(M, N, K, sub, w8 != 0);
+  else {
+    p.c = pick_by_rule(M, N, K, sub, w8 != 0);
+    p.us = decode2_us(workgroup_cost(M, sub, w8 != 0), p.c, M, N, K, sub, w8 != 0, (M + 15) / 16, 1);
+  }
+  const double out[6] = {(double)p.c.gs, (double)p.c.wks, (double)p.c.wn, (double)p.c.sk, (double)p.c.mr, p.us};
+  for (int i = 0; i < 6; ++i) plan[i] = out[i];
+  return VAQ_OK;
+}
+
+namespace vaq {
 
 int w4a16_decode2_workspace(int M, int N, int K, int sub, bool w8, size_t* c_tmp_bytes, size_t* counter_ints) {
   const Decode2Config c = workgroup_plan(M, N, K, sub, w8).c;
