@@ -690,3 +690,14 @@ def test_scaled_mm_split_k_first_call_under_graph_capture(device):
         torch.cuda.synchronize()
         assert torch.equal(out, eager) and torch.equal(out.cpu().float(), a @ w.t())
         assert torch.equal(ops.cutlass_scaled_mm(*args), eager)      # eager work between the replays
+
+
+@pytest.mark.parametrize("m,n,k", [(384, 65616, 256), (130, 33024, 384), (1040, 192, 640), (40, 48, 20480), (200, 144, 17024)])
+def test_scaled_mm_very_wide_and_very_long_layers_exact(device, m, n, k):
+    import vllm_amd._custom_ops as ops
+    g = torch.Generator().manual_seed(m)
+    a = torch.randint(-1, 2, (m, k), generator=g).float()
+    w = torch.randint(-1, 2, (n, k), generator=g).float()
+    out = ops.cutlass_scaled_mm(a.to(torch.float8_e4m3fn).to(device), w.to(torch.float8_e4m3fn).to(device).t(),
+                                torch.ones(m, 1, device=device), torch.ones(n, 1, device=device), torch.float16)
+    assert torch.equal(out, (a.to(device) @ w.to(device).t()).half())

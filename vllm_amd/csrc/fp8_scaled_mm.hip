@@ -896,16 +896,18 @@ static int launch_tile3(const Fp8MMParams& p, hipStream_t s) {
 }
 
 // The tile shapes of the multi-stage kernel (ids for K % 128 == 0; the two-slice shapes have one with a slice per step, id - 10).
-// Fitted to 1553 problems with M = 9 .. 8192, K = 1024 .. 16384, N = 1024 .. 28672 drawn over the logarithm, every shape and K
-// split of each timed on cold weights (some 20000 launches; 7.6 % rms).  The plan with the least predicted time is on average
-// 0.8 % slower than the fastest of all plans of a problem, where rules by size were 11 % slower at M = 33 .. 1024
-// (4096 x 13824 at M = 384 49 -> 33 us, 8192 x 4096 at M = 180 25 -> 19 us, 14336 x 2048 at M = 384 39 -> 27 us).
+// Fitted to 2064 problems with M = 9 .. 8192, half of them with K = 1024 .. 14336 and N = 1024 .. 28672, half with K = 256 .. 28672 and
+// N = 256 .. 152064, drawn over the logarithm, every shape and K split of each timed on cold weights (30154 launches,
+// profiles/plan_prices).  The plan with the least predicted time is on average 0.5 % slower than the fastest of all plans of a
+// problem (99 of 100 less than 11 %), where rules by size were 11 % slower at M = 33 .. 1024 (4096 x 13824 at M = 384 49 -> 33 us,
+// 8192 x 4096 at M = 180 25 -> 19 us, 14336 x 2048 at M = 384 39 -> 27 us).  Constants fitted to the first half's sizes alone lost 4.3 % at
+// N > 28672 and 3.5 % at K or N below 1024 (5120 x 152064 at M = 384 400 -> 326 us, 896 x 4864 at M = 2048 24.2 -> 18.8 us with these).
 constexpr TileShape FP8_TILE_SHAPES[] = {
-    {13, 128, 128, 8, 1, 2.24, 0.192, 0.121, 0, 0}, {14, 64, 128, 4, 1, 1.75, 0.172, 0.090, 0, 0},
-    {15, 64, 64, 4, 2, 0.86, 0.103, 0.043, 0.107, 0}, {16, 128, 64, 4, 1, 1.75, 0.152, 0.048, 0, 0},
-    {17, 128, 256, 8, 1, 4.81, 0.344, 0.160, 0, 0}, {19, 256, 128, 8, 1, 4.55, 0.311, 0.124, 0, 0},
-    {1, 256, 256, 8, 1, 10.46, 0.476, 0.218, 0, 0}, {10, 256, 384, 8, 1, 22.66, 0.580, 0.451, 0, 0}};
-constexpr TileCosts FP8_TILE_COSTS = {0.204, 2.56, 0.725, 0.184};
+    {13, 128, 128, 8, 1, 3.48, 0.205, 0.0739, 0, 0}, {14, 64, 128, 4, 1, 3.05, 0.161, 0.118, 0, 0},
+    {15, 64, 64, 4, 2, 1.63, 0.103, 0.0209, 0.173, 0}, {16, 128, 64, 4, 1, 2.69, 0.158, 0.0327, 0, 0},
+    {17, 128, 256, 8, 1, 5.22, 0.354, 0.17, 0, 0}, {19, 256, 128, 8, 1, 4.93, 0.32, 0.107, 0, 0},
+    {1, 256, 256, 8, 1, 7.24, 0.524, 0.118, 0, 0}, {10, 256, 384, 8, 1, 18.4, 0.594, 0.38, 0, 0}};
+constexpr TileCosts FP8_TILE_COSTS = {0.149, 1.14, 0.56, 0.254};
 
 static TilePlan make_plan_tile3(int M, int N, int K) {
   const int64_t cus = num_cus_current_device();
@@ -928,9 +930,10 @@ static TilePlan make_plan_tile3(int M, int N, int K) {
       if (sk == 1 || (steps / sk >= 8 && tiles * sk * 10 <= cus * 23)) consider(sk, 0);
     // 256 x 256 tiles that end in a round of workgroups at most half full: the tiles of that round in parts of at least 16
     // steps that fill it, the others whole
+    if (t.id == 1 && tiles > cus && rest > 0 && tn.exp[6] > 1) best = TilePlan();      // (development switch: this plan alone)
     if (t.id == 1 && tiles > cus && rest > 0 && tn.exp[10] != 1)
       for (int sk : {2, 3, 4})
-        if (rest * sk <= cus && steps / sk >= 16) consider(sk, tiles - rest);
+        if (rest * sk <= cus && (tn.exp[6] > 1 ? sk == tn.exp[6] && steps / sk >= 4 : steps / sk >= 16)) consider(sk, tiles - rest);
   }
   if (best.id < 0) return best;      // an unknown shape was forced: the other kernels take the problem
   if (tn.fp8_tile_cfg > 0) best.id = tn.fp8_tile_cfg;

@@ -43,8 +43,6 @@ inline double tile_plan_us(const TileShape& t, const TileCosts& c, int64_t M, in
   const double mem = c.weight_mb * 1e-6 * weight_bytes;
   us = sqrt(sqrt(us * us * us * us + mem * mem * mem * mem)) + 2.0 + t.out * 2e-6 * (double)M * (double)N;
   if (sk > 1) us += c.handover + c.part * sk + c.handover_mb * 4e-6 * (double)(split_tiles * t.bm * t.bn) * sk;
-  // (a handful of left-over tiles: the estimate is 7 % high there; FP8, 2048 x 4096 at M = 4352 58.7 against 54.9 us)
-  if (tail_first > 0 && split_tiles * 8 <= cus) us *= 0.9;
   return us;
 }
 

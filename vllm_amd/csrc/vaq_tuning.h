@@ -43,7 +43,8 @@ typedef struct VaqTuning {
                         /*   slabs never merged into one; [4] FP8 streaming through LDS (1 / 2 / 3 = 8 / 4 / 16 steps   */
                         /*   per wavefront, 9 = off); [10] = 1 both tile kernels: never split only the tiles of a half-empty last round; */
                         /*   [12] = 1 FP8 tile kernel: every tile starts at the first K step; [13] = 1 FP8 tile kernel: no tile  */
-                        /*   row past M; [14] > 0 W4A16 tile kernel: KiB that the partial tiles of a K split may take; [6], [8], [9], [11] unused;           */
+                        /*   row past M; [14] > 0 W4A16 tile kernel: KiB that the partial tiles of a K split may take; [6] > 1 both tile     */
+                        /*   kernels, 256 x 256 tiles: the tiles of the last round in this many parts of K; [8], [9], [11] unused;       */
                         /*   [7] = 1 LDS-staged decode kernel: n-tiles in launch order, not grouped by XCD             */
 } VaqTuning;
 

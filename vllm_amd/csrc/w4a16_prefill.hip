@@ -78,9 +78,10 @@ static TilePlan make_plan_prefill(int M, int N, int K, bool reg_ok) {
       if (sk == 1 || (G / sk >= 3 && tiles * sk * 10 <= cus * 24)) consider(sk, 0);
     // 256 x 256 tiles that end in a round of workgroups at most half full: the tiles of that round in parts of at least 8 groups
     // that fill it, the others whole (4096 x 6144 at M = 4096: 384 tiles = 256 whole + 128 in two parts each, 205 -> 189 us)
+    if (is256 && tiles > cus && rest > 0 && tn.exp[6] > 1) best = TilePlan();      // (development switch: this plan alone)
     if (is256 && tiles > cus && rest > 0 && tn.exp[10] != 1)
       for (int sk : {2, 3, 4})
-        if (rest * sk <= cus && G / sk >= 8) consider(sk, tiles - rest);
+        if (rest * sk <= cus && (tn.exp[6] > 1 ? sk == tn.exp[6] && G / sk >= 3 : G / sk >= 8)) consider(sk, tiles - rest);
   }
   if (forced >= 0 && best.id >= 0) {
     best.id = forced;
