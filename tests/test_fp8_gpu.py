@@ -692,6 +692,24 @@ def test_scaled_mm_split_k_first_call_under_graph_capture(device):
         assert torch.equal(ops.cutlass_scaled_mm(*args), eager)      # eager work between the replays
 
 
+@pytest.mark.parametrize("k", [1552, 1664, 2560, 2576, 3072, 3088, 3584, 4096])
+@pytest.mark.parametrize("m", [33, 48, 49, 56, 57, 64])
+def test_scaled_mm_stream_kernel_three_and_four_m_blocks_exact(device, k, m):
+    """33 .. 64 rows on both sides of every line of the rule that gives them to the weight-streaming kernel, and forced there."""
+    import vllm_amd._custom_ops as ops
+    from vllm_amd import _tuning
+    g = torch.Generator().manual_seed(k + m)
+    for n in (16, 528, 4096, 4112, 8208):
+        a = torch.randint(-2, 3, (m, k), generator=g).float()
+        w = torch.randint(-1, 2, (n, k), generator=g).float()
+        args = (a.to(torch.float8_e4m3fn).to(device), w.to(torch.float8_e4m3fn).to(device).t(), torch.ones(m, 1, device=device),
+                torch.ones(n, 1, device=device), torch.float16)
+        ref = (a.to(device) @ w.to(device).t()).half()
+        assert torch.equal(ops.cutlass_scaled_mm(*args), ref), n
+        with _tuning.override(fp8_path=1):
+            assert torch.equal(ops.cutlass_scaled_mm(*args), ref), n
+
+
 @pytest.mark.parametrize("m,n,k", [(384, 65616, 256), (130, 33024, 384), (1040, 192, 640), (40, 48, 20480), (200, 144, 17024)])
 def test_scaled_mm_very_wide_and_very_long_layers_exact(device, m, n, k):
     import vllm_amd._custom_ops as ops

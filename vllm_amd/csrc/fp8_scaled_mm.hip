@@ -1064,11 +1064,18 @@ static bool stream_offsets_fit(const Fp8MMParams& p) {
 // a wavefront's K slab live in registers: at most 8 wavefronts along K, 14 steps each for one m-block, 8 for two).
 static int stream_steps_per_wave(int64_t M, int64_t N, int64_t K) {
   const int64_t steps = (K + 127) / 128;
-  // three m-blocks: K = 1664 .. 4096 (4 steps per wavefront keep the registers, and the workgroup must have a wavefront per
-  // m-block for the reduction) of a narrow layer.  Cold against the tile kernel at M = 35 .. 47: 3712 x 3712 8.6 against 10.2 us,
-  // 2048 x 2304 5.9 against 6.6, 2816 x 3840 7.2 against 8.0 us; level at N = 4500, behind on wider layers (2304 x 14144 11.7
-  // against 10.4 us) and with a fourth m-block (3072 x 2304 at M = 59 9.3 against 8.3 us).
-  if (M > 32) return M <= 48 && N <= 4096 && steps <= 8 * 4 && steps >= 13 ? 4 : 0;
+  // three and four m-blocks: K = 1664 .. 4096 (4 steps per wavefront keep the registers, and the workgroup must have a
+  // wavefront per m-block for the reduction).  The time of the tile kernel over this one's, geometric means over 3093 random
+  // problems, cold:                 K 1665-2560   2561-3072   3073-3584   3585-4096
+  //   M 33 .. 48, N <= 4096          1.29 - 1.51   1.16 - 1.42  1.03 - 1.27  0.95 - 1.12
+  //   M 33 .. 48, N 4097 .. 8192     1.02 - 1.16   1.03 - 1.13  1.04 - 1.11  0.91 - 1.04
+  //   M 49 .. 64, N <= 4096          1.08 - 1.34   0.96 - 1.28  0.87 - 1.19  0.82 - 0.93
+  // and 0.79 .. 1.05 on wider layers.  (2048 x 960 at M = 49 7.1 -> 6.0 us, 1664 x 4992 at M = 34 6.9 -> 6.4 us)
+  if (M > 32) {
+    if (M > 64 || steps < 13 || steps > 8 * 4) return 0;
+    if (tuning().fp8_path == 1) return 4;
+    return M <= 48 ? (N <= (steps <= 28 ? 8192 : 4096) ? 4 : 0) : (N <= 4096 && steps <= (M <= 56 ? 24 : 20) ? 4 : 0);
+  }
   if (steps <= 8 * 4) return 4;
   if (steps <= 8 * 8) return 8;
   if (steps <= 8 * 14 && M <= 16) return 14;
@@ -1123,10 +1130,11 @@ static bool launch_stream2(const Fp8MMParams& p_in, int wk, int gx, hipStream_t 
 
 // Steps per wavefront of the stream kernel with the weights through LDS, 0 where the kernel above stays.  From 13500 problems
 // drawn over M = 1 .. 32, K = 1024 .. 16384, N = 1024 .. 28672 with cold weights, every choice timed:
-//  * up to 16 rows: 4 steps up to K = 1536 (2-7 % ahead of 8), 8 up to K = 3072, 16 beyond.  Fewer wavefronts with longer
-//    streams: against 8 steps 2-5 % at K = 3100 .. 4096, 6-8 % at K = 4100 .. 8192 (M = 1 / 4 / 16, us, against the kernel above:
+//  * up to 16 rows: 4 steps up to K = 1536 (2-7 % ahead of 8), 8 up to K = 3584, 16 beyond.  Fewer wavefronts with longer
+//    streams: against 8 steps -10 .. -14 % at K = 2500 .. 3072, -1 .. -6 % to 3584, level to 3840, +1.5 % to 4096 (9356 problems),
+//    6-8 % at K = 4100 .. 8192 (M = 1 / 4 / 16, us, against the kernel above:
 //    4096 x 6144 8.6 / 9.0 / 10.3 -> 6.6 / 6.7 / 7.2, 4096 x 28672 25.8 / 26.1 / 27.8 -> 19.4 / 19.6 / 20.6, 14336 x 4096 13.8 /
-//    14.8 / 18.0 -> 12.0 / 12.4 / 15.3); below K = 3072 one or two wavefronts are too few, 16 steps 5-20 % behind 8;
+//    14.8 / 18.0 -> 12.0 / 12.4 / 15.3);
 //  * two m-blocks: 4 steps up to K = 1536 (4 % ahead), 8 to K = 8192 (3-7 % ahead of 4; against the kernel above, M = 24 / 32:
 //    5120 x 5120 13.9 / 14.7 -> 10.9 / 11.8 us, 8192 x 8192 20.9 / 22.3 -> 19.4 / 20.7 us); 16 do not fit the registers.
 // (development switch exp[4]: 1 / 2 / 3 force 8 / 4 / 16 steps, 9 switches the kernel off)
@@ -1136,7 +1144,7 @@ static int stream2_steps_per_wave(const Fp8MMParams& p) {
   const int steps = (p.K + 127) / 128, MB = (p.M + 15) / 16;
   int ks = 0;
   if (sw >= 1 && sw <= 3) ks = sw == 1 ? 8 : (sw == 2 ? 4 : 16);
-  else if (MB == 1) ks = steps <= 12 ? 4 : (steps <= 24 ? 8 : (steps <= 128 ? 16 : 0));
+  else if (MB == 1) ks = steps <= 12 ? 4 : (steps <= 28 ? 8 : (steps <= 128 ? 16 : 0));
   else ks = steps <= 12 ? 4 : (steps <= 64 ? 8 : 0);
   if (ks == 0 || (steps + ks - 1) / ks > 8 || (MB == 2 && ks == 16)) return 0;
   return ks;
@@ -1196,8 +1204,10 @@ static bool dispatch_stream(const Fp8MMParams& p, hipStream_t s) {
   } else if (MB == 2) {
     if (ks == 4) launch_stream<BF16_OUT, 4, 2>(p, wk, gx, s);
     else launch_stream<BF16_OUT, 8, 2>(p, wk, gx, s);
-  } else {
+  } else if (MB == 3) {
     launch_stream<BF16_OUT, 4, 3>(p, wk, gx, s);
+  } else {
+    launch_stream<BF16_OUT, 4, 4>(p, wk, gx, s);
   }
   return true;
 }
