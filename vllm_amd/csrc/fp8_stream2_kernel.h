@@ -76,14 +76,14 @@ static __device__ inline uint32_t wave_maxima(uint32_t (&v)[MQ]) {
 }
 
 // ----------------------------------------------------------------------------- stream kernel, weights through LDS
-// The stream kernel above fetches the weights in the MFMA operand layout: every load instruction takes 64-byte pieces
-// of 16 rows, half a cache line each.  Measured on bare reads of a 4096 x 28672 byte matrix with cold lines, that
+// fp8_mm_stream_kernel (fp8_scaled_mm.hip) fetches the weights in the MFMA operand layout: every load instruction takes
+// 64-byte pieces of 16 rows, half a cache line each.  Measured on bare reads of a 4096 x 28672 byte matrix with cold lines, that
 // pattern reaches 4.2-5.3 TB/s where instructions that read whole lines reach 5.3-5.9 TB/s.  Here every load
 // instruction is a direct-to-LDS load of 4 rows x 256 contiguous bytes into a ring that belongs to the wavefront alone
 // (no barrier: the wavefront waits on its own load counter), and the operands are read back from LDS, 16-byte chunks
 // XOR-swizzled by the row so that the 16 rows of an operand read hit 16 different bank groups.
 //  * blockDim = (64, WK).  Wavefront w owns K steps [w*KS, (w+1)*KS) of 128 bytes; its activations live in registers;
-//    the workgroup walks a contiguous range of 16-row n-tiles; per n-tile the wavefronts reduce through LDS as above.
+//    the workgroup walks a contiguous range of 16-row n-tiles; per n-tile the wavefronts reduce through LDS as there.
 //  * A stage is two steps (16 rows x 256 bytes = 4 KiB, four load instructions); the ring holds NSR stages, and the
 //    stage NSR ahead -- of this n-tile or the next -- is requested as soon as a stage's operands have been read.
 //  * MQ > 0: the activations come as the 16-bit numbers they are before their quantisation (type BF16_OUT, at most MQ rows),

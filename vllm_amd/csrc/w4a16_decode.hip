@@ -21,7 +21,7 @@
 //  * The WK wavefronts of a workgroup cover WK*TG groups of the same n-tile and reduce through LDS (one barrier per
 //    n-tile, double-buffered).  If K needs more than one workgroup (SK > 1) the partial tiles go to `c_tmp` and the
 //    last workgroup to arrive at a per-tile counter sums them in a fixed order (deterministic) and resets the counter.
-#include "vaq_common.h"
+#include "w4a16_kernels.h"
 
 namespace vaq {
 

@@ -2,6 +2,7 @@
 // of the instances for quantisation groups of 128 rows and channelwise scales.
 #include "tile_plan.h"
 #include "w4a16_decode2_kernel.h"
+#include "w4a16_kernels.h"
 
 namespace vaq {
 

@@ -72,7 +72,6 @@ static inline uint32_t d2_sat32(uint64_t bytes) { return bytes > 0xffffffffull ?
 constexpr int D2_WAVES = 16;
 constexpr int DECODE2_MAX_M = 64;           // rows of one workgroup: up to four m-blocks of 16
 constexpr int DECODE2_MAX_M_ROWS = 256;     // rows when every m-block has workgroups of its own (see MSP)
-enum { D2_TILE, D2_WORKGROUP, D2_ROWS };    // see w4a16_decode2_choose
 
 template <bool BF16, int GS, int MB, bool HAS_ZP, int MR, int SUBG, int WT = 0, int RC = 0, bool MSP = false>
 __global__ __launch_bounds__(D2_WAVES * 64) void w4a16_decode2_kernel(const Decode2Params p) {

@@ -1,28 +1,9 @@
 // C-ABI entry of the W4A16 GEMM: argument validation and the decode / prefill dispatch.
-#include "vaq_common.h"
+#include "w4a16_kernels.h"
 
 #include <mutex>
 
 namespace vaq {
-// `sub` = quantisation groups per 128-row weight tile (1, 2, 4); `channelwise` = one scale row for all of K (sub == 1)
-int w4a16_decode_workspace(int M, int N, int K, size_t* c_tmp_bytes, size_t* counter_ints);
-int w4a16_decode_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
-                        const int32_t* perm, const void* bias, void* c, float* c_tmp, int64_t c_tmp_bytes,
-                        int32_t* counters, int64_t counter_ints, int M, int N, int K, bool channelwise, int dtype,
-                        hipStream_t s);
-int w4a16_decode2_workspace(int M, int N, int K, int sub, bool w8, size_t* c_tmp_bytes, size_t* counter_ints);
-int w4a16_decode2_choose(int M, int N, int K, int sub, int wt, bool has_perm, bool wg_ok, bool tile_ok, double tile_us);
-double w4a16_prefill_us(int M, int N, int K, bool reg_ok);
-enum { D2_TILE, D2_WORKGROUP, D2_ROWS };
-int w4a16_decode2_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
-                         const int32_t* perm, const void* bias, void* c, float* c_tmp, int64_t c_tmp_bytes,
-                         int32_t* counters, int64_t counter_ints, int M, int N, int K, int sub, bool channelwise,
-                         int wt, int dtype, bool rows, hipStream_t s);      // wt: 0 4-bit codes, 1 8-bit codes, 2 FP8 e4m3 bytes
-int w4a16_prefill_workspace(int M, int N, int K, size_t* c_tmp_bytes, size_t* counter_ints);
-int w4a16_prefill_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
-                         const void* bias, void* c, float* c_tmp, int64_t c_tmp_bytes, int32_t* counters,
-                         int64_t counter_ints, int M, int N, int K, int sub, bool channelwise, int wt, int dtype,
-                         hipStream_t s);
 
 constexpr int64_t DECODE_MAX_M = 64;          // up to four m-blocks of 16 rows on the LDS-staged kernel
 constexpr int64_t DECODE_MAX_M_2BLK = 32;     // the register-resident kernel, groups below 128 rows and 8-bit codes: two

@@ -1,0 +1,27 @@
+// The kernels behind the W4A16 GEMM, as its entry point (w4a16_gemm.hip) sees them.
+#pragma once
+#include "vaq_common.h"
+
+namespace vaq {
+// `sub` = quantisation groups per 128-row weight tile (1, 2, 4); `channelwise` = one scale row for all of K (sub == 1)
+int w4a16_decode_workspace(int M, int N, int K, size_t* c_tmp_bytes, size_t* counter_ints);
+int w4a16_decode_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
+                        const int32_t* perm, const void* bias, void* c, float* c_tmp, int64_t c_tmp_bytes,
+                        int32_t* counters, int64_t counter_ints, int M, int N, int K, bool channelwise, int dtype,
+                        hipStream_t s);
+int w4a16_decode2_workspace(int M, int N, int K, int sub, bool w8, size_t* c_tmp_bytes, size_t* counter_ints);
+// Which kernel takes more than 16 rows: the tile kernel, the decode kernel's workgroups of all rows, or of 16 rows each.
+enum { D2_TILE, D2_WORKGROUP, D2_ROWS };
+int w4a16_decode2_choose(int M, int N, int K, int sub, int wt, bool has_perm, bool wg_ok, bool tile_ok, double tile_us);
+double w4a16_prefill_us(int M, int N, int K, bool reg_ok);
+int w4a16_decode2_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
+                         const int32_t* perm, const void* bias, void* c, float* c_tmp, int64_t c_tmp_bytes,
+                         int32_t* counters, int64_t counter_ints, int M, int N, int K, int sub, bool channelwise,
+                         int wt, int dtype, bool rows, hipStream_t s);      // wt: 0 4-bit codes, 1 8-bit codes, 2 FP8 e4m3 bytes
+int w4a16_prefill_workspace(int M, int N, int K, size_t* c_tmp_bytes, size_t* counter_ints);
+int w4a16_prefill_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
+                         const void* bias, void* c, float* c_tmp, int64_t c_tmp_bytes, int32_t* counters,
+                         int64_t counter_ints, int M, int N, int K, int sub, bool channelwise, int wt, int dtype,
+                         hipStream_t s);
+
+}  // namespace vaq

@@ -1,6 +1,7 @@
 // Host side of the prefill kernels (w4a16_prefill_kernel.h): tile and K-split choice, workspace sizes, launch of the
 // instances for quantisation groups of 128 rows and channelwise scales.
 #include "tile_plan.h"
+#include "w4a16_kernels.h"
 #include "w4a16_prefill_kernel.h"
 
 namespace vaq {

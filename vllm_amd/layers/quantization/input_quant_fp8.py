@@ -6,7 +6,8 @@ from __future__ import annotations
 from typing import NamedTuple
 
 import torch
-import torch.nn.modules.module as _module
+from torch.nn.modules.module import (_global_backward_hooks, _global_backward_pre_hooks, _global_forward_hooks,
+                                     _global_forward_pre_hooks)      # the dictionaries themselves: filled in place
 
 from vllm_amd import _custom_ops as ops
 
@@ -48,10 +49,10 @@ class QuantFP8(torch.nn.Module):
     def runs_forward_only(self) -> bool:
         """Whether a call of this module is a call of ``forward`` above: no hooks, of its own or of all modules, no other
         ``forward``.  (A layer's direct call does what ``forward`` does without calling it.)"""
-        return not (self._forward_pre_hooks or self._forward_hooks or self._backward_pre_hooks or self._backward_hooks
-                    or _module._global_forward_pre_hooks or _module._global_forward_hooks
-                    or _module._global_backward_pre_hooks or _module._global_backward_hooks
-                    or self._compiled_call_impl is not None or "forward" in self.__dict__)
+        own = self.__dict__
+        return not (own["_forward_pre_hooks"] or own["_forward_hooks"] or own["_backward_pre_hooks"] or own["_backward_hooks"]
+                    or _global_forward_pre_hooks or _global_forward_hooks or _global_backward_pre_hooks
+                    or _global_backward_hooks or "forward" in own or "_compiled_call_impl" in own)
 
     forward_cuda = forward
     forward_hip = forward
