@@ -791,6 +791,26 @@ def mfma_pass(dev):
         ", ".join(f"{k}x{n}: {2.0 * m * n * k:.0f}" for (k, n) in LLAMA_SHAPES))
 
 
+def case_pass(dev, passes=20):
+    """For kernel traces and counters: eager passes of every listed case of perf/cases.py, in order, each case announced by a
+    cumsum (a kernel that nothing else here launches); no timing."""
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("perf_cases", os.path.join(ROOT, "perf", "cases.py"))
+    cases = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(cases)
+    mark = torch.ones(256, device=dev)
+    for case in cases.listed():
+        state = cases.prepare(case, 1)
+        torch.cuda.synchronize()
+        torch.cumsum(mark, 0)
+        for _ in range(passes):
+            cases.run(state)
+        torch.cuda.synchronize()
+        log(f"[case pass] {case['name']}")
+        del state
+        torch.cuda.empty_cache()
+
+
 def counter_pass(dev):
     """Workload for a hardware-counter run: a plain 256 MiB device-to-device copy (the calibration kernel: it reads and
     writes exactly 262144 KiB) followed by one eager pass over the 12 headline GEMMs, three times; the last repetition's
@@ -919,6 +939,8 @@ def main():
                     help="run the weight access pattern probe (bench-only library) and print its table; no product timing")
     ap.add_argument("--mix-probe", action="store_true",
                     help="run the matrix-core instruction-mix probe (bench-only library) and print its table; no product timing")
+    ap.add_argument("--case-pass", action="store_true",
+                    help="for `rocprofv3`: 20 eager passes of every listed case of perf/cases.py, a cumsum ahead of each case, no timing")
     ap.add_argument("--counter-pass", action="store_true",
                     help="for `rocprofv3 --pmc`: three eager passes of [256 MiB device copy, the 12 headline GEMMs], no timing")
     args = ap.parse_args()
@@ -939,6 +961,9 @@ def main():
         return
     if args.mix_probe:
         print(json.dumps(mix_probe(dev), indent=1))
+        return
+    if args.case_pass:
+        case_pass(dev)
         return
     if args.counter_pass:
         counter_pass(dev)
