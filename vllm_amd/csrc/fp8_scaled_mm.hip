@@ -3,13 +3,14 @@
 // a is [M,K] row-major, b is [K,N] column-major (= weight [N,K] row-major with row pitch ldb), so both operands are
 // k-contiguous and go to the matrix cores without any data re-arrangement.
 //
-// Two kernels:
-//  * tile kernel (any M): one workgroup of 4 wavefronts (2 x 2) per BM x BN output tile, K walked in steps of 128
-//    bytes through double-buffered, padded LDS (pitch 144 B), v_mfma_f32_32x32x64_f8f6f4 (the full-rate gfx950 FP8
-//    instruction, 32 bytes per lane per operand);
-//  * stream kernel (M <= 32; M <= 64 on narrow layers with K <= 4096): weight-streaming GEMV-like kernel, weights are the A operand of
-//    v_mfma_f32_16x16x128_f8f6f4 straight from global memory, activations stay in registers, the wavefronts of a
-//    workgroup split K and reduce through LDS.
+// The kernels:
+//  * tile kernel (any M; fp8_mm_tile3_kernel): one workgroup of 4 or 8 wavefronts per BM x BN output tile, both operands by
+//    direct-to-LDS loads through a ring of stages, v_mfma_f32_32x32x64_f8f6f4 (the full-rate gfx950 FP8 instruction, 32
+//    bytes per lane per operand).  fp8_mm_tile_kernel, K in steps of 128 bytes through double-buffered, padded LDS
+//    (pitch 144 B), takes what the multi-stage kernel cannot address;
+//  * stream kernels (M <= 32; M <= 64 on narrow layers with K <= 4096): weight-streaming GEMV-like, weights are the A operand
+//    of v_mfma_f32_16x16x128_f8f6f4, activations stay in registers, the wavefronts of a workgroup split K and reduce
+//    through LDS; fp8_mm_stream2_kernel (fp8_stream2_kernel.h) brings the weights in through LDS as whole cache lines.
 //
 // The per-lane byte -> k assignment inside an MFMA operand is the same function for A and B, so any consistent choice
 // of which 32 bytes a lane supplies yields the exact dot product; both kernels give lane (row, q) the bytes
@@ -898,8 +899,8 @@ static int launch_tile3(const Fp8MMParams& p, hipStream_t s) {
 // The tile shapes of the multi-stage kernel (ids for K % 128 == 0; the two-slice shapes have one with a slice per step, id - 10).
 // Fitted to 2064 problems with M = 9 .. 8192, half of them with K = 1024 .. 14336 and N = 1024 .. 28672, half with K = 256 .. 28672 and
 // N = 256 .. 152064, drawn over the logarithm, every shape and K split of each timed on cold weights (30154 launches,
-// profiles/plan_prices).  The plan with the least predicted time is on average 0.5 % slower than the fastest of all plans of a
-// problem (99 of 100 less than 11 %), where rules by size were 11 % slower at M = 33 .. 1024 (4096 x 13824 at M = 384 49 -> 33 us,
+// profiles/plan_prices).  The plan with the least predicted time is on average 0.7 % slower than the fastest of all plans of a
+// problem (99 of 100 less than 13 %), where rules by size were 11 % slower at M = 33 .. 1024 (4096 x 13824 at M = 384 49 -> 33 us,
 // 8192 x 4096 at M = 180 25 -> 19 us, 14336 x 2048 at M = 384 39 -> 27 us).  Constants fitted to the first half's sizes alone lost 4.3 % at
 // N > 28672 and 3.5 % at K or N below 1024 (5120 x 152064 at M = 384 400 -> 326 us, 896 x 4864 at M = 2048 24.2 -> 18.8 us with these).
 constexpr TileShape FP8_TILE_SHAPES[] = {
@@ -907,7 +908,11 @@ constexpr TileShape FP8_TILE_SHAPES[] = {
     {15, 64, 64, 4, 2, 1.63, 0.103, 0.0209, 0.173, 0}, {16, 128, 64, 4, 1, 2.69, 0.158, 0.0327, 0, 0},
     {17, 128, 256, 8, 1, 5.22, 0.354, 0.17, 0, 0}, {19, 256, 128, 8, 1, 4.93, 0.32, 0.107, 0, 0},
     {1, 256, 256, 8, 1, 7.24, 0.524, 0.118, 0, 0}, {10, 256, 384, 8, 1, 18.4, 0.594, 0.38, 0, 0}};
-constexpr TileCosts FP8_TILE_COSTS = {0.149, 1.14, 0.56, 0.254};
+// The hand-over is priced 1 us above its fit (1.14): a call under graph capture fills counters of its own ahead of a split K, 2.3 us
+// a replay.  Mean over the problems, plans chosen with 1.14 / 2.14 / 3.44 against the fastest: 0.5 / 0.7 / 1.2 % slower without
+// that fill, 0.7 / 0.5 / 0.4 % with it (9 .. 256 rows 0.6 / 0.9 / 1.7 and 1.0 / 0.5 / 0.4 %); 4096 x 6144 at M = 40 .. 64 stays
+// whole: 11.3 .. 12.0 -> 11.1 us; as the operator's call replayed from a graph 14.4 -> 11.9 us at M = 64, 4096 x 4096 13.0 -> 10.8.
+constexpr TileCosts FP8_TILE_COSTS = {0.149, 2.14, 0.56, 0.254};
 
 static TilePlan make_plan_tile3(int M, int N, int K) {
   const int64_t cus = num_cus_current_device();
