@@ -34,10 +34,12 @@ static int dispatch_tile(const PrefillParams& p, int tile, hipStream_t s) {
 }
 
 // Fitted to 815 problems with M = 65 .. 6000, K = 1024 .. 14336, N = 1024 .. 28672 drawn over the logarithm (4-bit codes with zero
-// points, bf16), every shape and K split of each timed on cold weights: 5.4 % rms.  The cheapest plan is on average 1.2 % slower
-// than the fastest one, where rules by size were 10 % slower (5 % of it the eight-wavefront shapes 12, 14 and 16 that came
-// with it: 4096 x 4096 at M = 1024 50.7 -> 45.6 us, at M = 2048 77 -> 71 us, 4096 x 6144 at M = 333 34.6 -> 32.8 us, 4096 x 28672 at
-// M = 100 48.7 -> 43.1 us).
+// points, bf16), every shape and K split of each timed on cold weights.  Over the same 815 problems the plans that rules by size
+// had chosen were in the mean 10 % slower than the fastest one (5 % of it the eight-wavefront shapes 12, 14 and 16 that came with
+// the prices: 4096 x 4096 at M = 1024 50.7 -> 45.6 us, at M = 2048 77 -> 71 us, 4096 x 6144 at M = 333 34.6 -> 32.8 us, 4096 x 28672
+// at M = 100 48.7 -> 43.1 us; nothing where the rules had the 256 x 256 tiles right, M = 4096).  Checked over 1468 problems with M = 9 ..
+// 8192, K = 256 .. 28672, N = 256 .. 152064 (18770 launches, profiles/plan_prices): the cheapest plan is in the mean 1.1 % slower than
+// the fastest (N > 28672 0.9 %, K or N below 1024 0.7 %, 65 .. 128 rows 2.5 %), 99 of 100 less than 14 %.
 constexpr TileShape W4_TILE_SHAPES[] = {
     {12, 128, 128, 8, 2, 0.39, 0.578, 0.092, 0.352, 0.226}, {14, 64, 128, 8, 2, 0, 0.426, 0.041, 0.230, 0.330},
     {15, 128, 64, 4, 2, 0, 0.456, 0.025, 0.176, 0.392},     {16, 256, 128, 8, 1, 2.57, 0.764, 0.194, 0, 0.122},
