@@ -72,7 +72,7 @@ class Tiles:
     def price(self, p_shape, p_costs):
         bm, bn, _, slots = self.shape[self.which].T
         base, step, load, shared, out = p_shape[self.which].T
-        weight_mb, handover, part_cost, handover_mb = p_costs[:4]
+        weight_mb, handover, part_cost, handover_mb, sum_mb = p_costs[:5]
         tiles = np.ceil(self.m / bm) * np.ceil(self.n / bn)
         steps = self.k // 64
         tail = self.tail > 0
@@ -86,7 +86,7 @@ class Tiles:
         us = us + (rest > 0) * (base + part * (step + load * rest + np.where(rest > 1, shared, 0)))
         mem = weight_mb * 1e-6 * self.bytes * self.k * self.n
         us = (us ** 4 + mem ** 4) ** 0.25 + 2.0 + out * 2e-6 * self.m * self.n
-        us = us + (self.sk > 1) * (handover + part_cost * self.sk + handover_mb * 4e-6 * split * bm * bn * self.sk)
+        us = us + (self.sk > 1) * (handover + self.sk * (part_cost + 4e-6 * bm * bn * (handover_mb * split + sum_mb)))
         return us
 
     def prices(self, p=None):
@@ -199,7 +199,7 @@ def tile_prices(k, n, m, any_shape):
         t.which = np.full(len(k), i)
         bm, bn = t.shape[i][:2]
         tiles = np.ceil(m / bm) * np.ceil(n / bn)
-        for sk, tail in [(s, 0) for s in (1, 2, 3, 4, 6, 8)] + [(s, 1) for s in (2, 3, 4)]:
+        for sk, tail in [(s, 0) for s in range(1, 9)] + [(s, 1) for s in (2, 3, 4)]:
             t.sk, t.tail = np.full(len(k), sk), np.full(len(k), tail)
             ok = t.allowed() & ((ident != 13) | any_shape)
             if tail:

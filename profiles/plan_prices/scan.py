@@ -146,7 +146,7 @@ def tile_plans(kind, k, n, m):
         # (shapes that leave most of every tile empty, or of the device, are never the fastest)
         if bm > 64 and bm >= 2 * m:
             continue
-        for sk in (1, 2, 3, 4, 6, 8):
+        for sk in range(1, 9):
             if sk == 1 or (steps // sk >= (6 if kind == "fp8_tile" else 3) and tiles * sk <= CUS * 3 and ident != 30):
                 yield ident, sk, 0
         if ident in (1, 20) and tiles > CUS and rest:

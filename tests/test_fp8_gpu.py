@@ -476,6 +476,19 @@ def test_scaled_mm_slices_requested_together_exact(device, cfg):
     assert all(bool((t == 0).all()) for t in ops._FP8_COUNTERS.values()), "arrival counters not restored to zero"
 
 
+@pytest.mark.parametrize("k", range(4096, 24576, 2048))
+def test_scaled_mm_automatic_parts_exact(device, k):
+    """Plans of up to eight parts of K as the automatic choice makes them (five and seven among them), ragged rows."""
+    import vllm_amd._custom_ops as ops
+    g = torch.Generator().manual_seed(k)
+    for m, n in ((128, 1536), (117, 1168)):
+        a, w = torch.randint(-2, 3, (m, k), generator=g).float(), torch.randint(-1, 2, (n, k), generator=g).float()
+        out = ops.cutlass_scaled_mm(a.to(torch.float8_e4m3fn).to(device), w.to(torch.float8_e4m3fn).to(device).t(),
+                                    torch.ones(m, 1, device=device), torch.ones(n, 1, device=device), torch.float16)
+        assert torch.equal(out.cpu().float(), a @ w.t()), (m, n, k)
+    assert all(bool((t == 0).all()) for t in ops._FP8_COUNTERS.values()), "arrival counters not restored to zero"
+
+
 @pytest.mark.parametrize("m,n,k", [(17 * 256, 4096, 2048), (21 * 256 - 5, 3328, 2048)])
 def test_scaled_mm_tiles_of_last_round_split_exact(device, m, n, k):
     """More 256 x 256 tiles than compute units with a last round of workgroups at most half full (17 x 16 tiles on 256

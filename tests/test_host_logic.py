@@ -606,10 +606,25 @@ def test_price_formula_of_the_fit_is_the_one_of_the_library():
     assert lib.vaq_w4a16_decode_plan(40, 64, 100, 1, 0, 2, plan) == _lib.VAQ_ERR_INVALID_ARG
 
 
+def test_tile_plans_weigh_every_number_of_parts():
+    """K in five and seven parts too: 48 tiles of 256 x 256 make one round of the device in five parts and no other number."""
+    import ctypes
+    from vllm_amd import _lib
+    tmp, a_tmp, cnt = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_size_t()
+    for m, n, k in ((512, 6144, 24576), (768, 4096, 28672)):
+        assert _lib.load().vaq_w4a16_gemm_workspace(m, n, k, 0, 0, ctypes.byref(tmp), ctypes.byref(a_tmp), ctypes.byref(cnt)) == _lib.VAQ_OK
+        assert tmp.value == 5 * m * n * 4
+    parts = set()
+    for k in range(4096, 24576, 512):
+        assert _lib.load().vaq_fp8_scaled_mm_workspace(128, 1536, k, ctypes.byref(tmp), ctypes.byref(cnt)) == _lib.VAQ_OK
+        parts.add(tmp.value / (128 * 1536 * 4))
+    assert parts & {5, 7}
+
+
 def test_fp8_tile_plans_hold_for_calls_replayed_from_a_graph():
     """A captured call fills arrival counters of its own ahead of a split K (2.3 us a replay).  Over the recorded timings the
-    plans chosen are within 0.8 % of the fastest without that fill and within 0.6 % with it (mean of the logarithms; 33 .. 64
-    rows 0.7 %), and the two layers that lost most by a split keep K whole."""
+    plans chosen are 0.78 % above the fastest without that fill and 0.54 % with it (mean of the logarithms; 33 .. 64 rows 1.05 and
+    0.71 %; with the hand-over at its fit 0.56 and 0.79 %, 0.71 and 1.32 %), and the two layers that lost most by a split keep K whole."""
     import ctypes
     import importlib.util
     from vllm_amd import _lib
@@ -618,7 +633,7 @@ def test_fp8_tile_plans_hold_for_calls_replayed_from_a_graph():
     spec.loader.exec_module(fit)
     t = fit.Tiles("fp8_tile")
     t.load([os.path.join(ROOT, "profiles", "plan_prices", "fp8_tile.csv.gz")])
-    for fill, most, most_few_rows in ((0.0, 1.008, 1.009), (2.3, 1.006, 1.007)):
+    for fill, most, most_few_rows in ((0.0, 1.009, 1.012), (2.3, 1.006, 1.008)):
         loss = fit.report(t.prices(), t.us + fill * (t.sk > 1), t.key, t.allowed(), {})
         few = np.zeros(len(loss), bool)
         few[t.key[(t.m >= 33) & (t.m <= 64)]] = True

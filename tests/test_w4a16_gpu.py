@@ -236,6 +236,21 @@ def test_prefill_every_tile_shape(device, asym, dtype):
         assert bool((layer.workspace == 0).all()), "workspace counters not restored to zero"
 
 
+@pytest.mark.parametrize("tile", [12, 13, 14, 15, 16, 20])
+def test_prefill_five_and_seven_parts(device, tile):
+    """K in five and seven parts of unequal length (19 and 23 groups), ragged M and N."""
+    from vllm_amd import _tuning
+    for k, n, m, split in ((19 * 128, 192, 150, 5), (23 * 128, 320, 270, 7), (5 * 128, 64, 65, 5)):
+        case = o.make_w4a16_case(k, n, 128, asym=True, seed=k + n + m)
+        layer = W4A16Layer(case, device)
+        a = _acts(m, k, device, seed=m)
+        ref = o.gemm_ref(a.cpu(), o.case_w_ref(case))
+        with _tuning.override(prefill_tile=tile + 1, prefill_split=split, exp=[0, 0, 1]):
+            out = layer(a)
+        check_gemm_close(out, ref, f"tile {tile} split {split} k={k} n={n} m={m}")
+        assert bool((layer.workspace == 0).all()), "workspace counters not restored to zero"
+
+
 @pytest.mark.parametrize("group_size,bits", [(128, 4), (-1, 4), (64, 4), (32, 4), (128, 8), (32, 8)])
 @pytest.mark.parametrize("tile", [12, 14, 15, 16])
 def test_prefill_eight_wavefront_tiles_every_format(device, tile, group_size, bits):

@@ -899,8 +899,8 @@ static int launch_tile3(const Fp8MMParams& p, hipStream_t s) {
 // The tile shapes of the multi-stage kernel (ids for K % 128 == 0; the two-slice shapes have one with a slice per step, id - 10).
 // Fitted to 2064 problems with M = 9 .. 8192, half of them with K = 1024 .. 14336 and N = 1024 .. 28672, half with K = 256 .. 28672 and
 // N = 256 .. 152064, drawn over the logarithm, every shape and K split of each timed on cold weights (30154 launches,
-// profiles/plan_prices).  The plan with the least predicted time is on average 0.7 % slower than the fastest of all plans of a
-// problem (99 of 100 less than 13 %), where rules by size were 11 % slower at M = 33 .. 1024 (4096 x 13824 at M = 384 49 -> 33 us,
+// the first half of those in profiles/plan_prices).  Over all 5493 problems there (91351 launches) the plan with the least predicted
+// time is on average 0.8 % slower than the fastest (99 of 100 less than 15 %), where rules by size were 11 % slower at M = 33 .. 1024 (4096 x 13824 at M = 384 49 -> 33 us,
 // 8192 x 4096 at M = 180 25 -> 19 us, 14336 x 2048 at M = 384 39 -> 27 us).  Constants fitted to the first half's sizes alone lost 4.3 % at
 // N > 28672 and 3.5 % at K or N below 1024 (5120 x 152064 at M = 384 400 -> 326 us, 896 x 4864 at M = 2048 24.2 -> 18.8 us with these).
 constexpr TileShape FP8_TILE_SHAPES[] = {
@@ -912,7 +912,8 @@ constexpr TileShape FP8_TILE_SHAPES[] = {
 // a replay.  Mean over the problems, plans chosen with 1.14 / 2.14 / 3.44 against the fastest: 0.5 / 0.7 / 1.2 % slower without
 // that fill, 0.7 / 0.5 / 0.4 % with it (9 .. 256 rows 0.6 / 0.9 / 1.7 and 1.0 / 0.5 / 0.4 %); 4096 x 6144 at M = 40 .. 64 stays
 // whole: 11.3 .. 12.0 -> 11.1 us; as the operator's call replayed from a graph 14.4 -> 11.9 us at M = 64, 4096 x 4096 13.0 -> 10.8.
-constexpr TileCosts FP8_TILE_COSTS = {0.149, 2.14, 0.56, 0.254};
+// (The last constant, by hand: 1.0 against none, 1.3 against 0.9 % in the mean over the problems whose plan has an odd number of parts.)
+constexpr TileCosts FP8_TILE_COSTS = {0.149, 2.14, 0.56, 0.254, 1.0};
 
 static TilePlan make_plan_tile3(int M, int N, int K) {
   const int64_t cus = num_cus_current_device();
@@ -930,8 +931,9 @@ static TilePlan make_plan_tile3(int M, int N, int K) {
       consider(tn.fp8_split <= steps ? tn.fp8_split : steps, 0);
       continue;
     }
-    // K in up to 8 parts of at least 8 steps, on up to 2.3 rounds of workgroups
-    for (int sk : {1, 2, 3, 4, 6, 8})
+    // K in up to 8 parts of at least 8 steps, on up to 2.3 rounds of workgroups.  (All of 1 .. 8: without 5 and 7 4 % of the
+    // problems had another plan, in the mean 1.3 % slower; 11776 x 576 at M = 1180 27.5 -> 22.5 us)
+    for (int sk = 1; sk <= 8; ++sk)
       if (sk == 1 || (steps / sk >= 8 && tiles * sk * 10 <= cus * 23)) consider(sk, 0);
     // 256 x 256 tiles that end in a round of workgroups at most half full: the tiles of that round in parts of at least 16
     // steps that fill it, the others whole

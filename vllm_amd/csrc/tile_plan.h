@@ -13,9 +13,10 @@ struct TileShape {
   int id, bm, bn, nw, slots;
   double base, step, load, shared, out;
 };
-// Per MB of weights that come from memory; fixed, per part and per MB of partial tiles of a K split.
+// Per MB of weights that come from memory; of a K split: fixed, per part, per MB of all partial tiles (written and read by the
+// device) and per MB of one tile's (read by the workgroup that sums them).
 struct TileCosts {
-  double weight_mb, handover, part, handover_mb;
+  double weight_mb, handover, part, handover_mb, sum_mb;
 };
 
 struct TilePlan {
@@ -42,7 +43,7 @@ inline double tile_plan_us(const TileShape& t, const TileCosts& c, int64_t M, in
   if (rest > 0) us += t.base + part * (t.step + t.load * rest + (rest > 1 ? t.shared : 0));
   const double mem = c.weight_mb * 1e-6 * weight_bytes;
   us = sqrt(sqrt(us * us * us * us + mem * mem * mem * mem)) + 2.0 + t.out * 2e-6 * (double)M * (double)N;
-  if (sk > 1) us += c.handover + c.part * sk + c.handover_mb * 4e-6 * (double)(split_tiles * t.bm * t.bn) * sk;
+  if (sk > 1) us += c.handover + sk * (c.part + 4e-6 * (double)(t.bm * t.bn) * (c.handover_mb * (double)split_tiles + c.sum_mb));
   return us;
 }
 

@@ -37,14 +37,14 @@ static int dispatch_tile(const PrefillParams& p, int tile, hipStream_t s) {
 // points, bf16), every shape and K split of each timed on cold weights.  Over the same 815 problems the plans that rules by size
 // had chosen were in the mean 10 % slower than the fastest one (5 % of it the eight-wavefront shapes 12, 14 and 16 that came with
 // the prices: 4096 x 4096 at M = 1024 50.7 -> 45.6 us, at M = 2048 77 -> 71 us, 4096 x 6144 at M = 333 34.6 -> 32.8 us, 4096 x 28672
-// at M = 100 48.7 -> 43.1 us; nothing where the rules had the 256 x 256 tiles right, M = 4096).  Checked over 1468 problems with M = 9 ..
-// 8192, K = 256 .. 28672, N = 256 .. 152064 (18770 launches, profiles/plan_prices): the cheapest plan is in the mean 1.1 % slower than
-// the fastest (N > 28672 0.9 %, K or N below 1024 0.7 %, 65 .. 128 rows 2.5 %), 99 of 100 less than 14 %.
+// at M = 100 48.7 -> 43.1 us; nothing where the rules had the 256 x 256 tiles right, M = 4096).  Checked over 3276 problems with M = 17 ..
+// 8192, K = 256 .. 28672, N = 256 .. 152064 (47137 launches, profiles/plan_prices): the cheapest plan is in the mean 1.1 % slower than
+// the fastest (N > 28672 0.8 %, K or N below 1024 0.8 %, 17 .. 128 rows 1.4 - 2.0 %), 99 of 100 less than 15 %.
 constexpr TileShape W4_TILE_SHAPES[] = {
     {12, 128, 128, 8, 2, 0.39, 0.578, 0.092, 0.352, 0.226}, {14, 64, 128, 8, 2, 0, 0.426, 0.041, 0.230, 0.330},
     {15, 128, 64, 4, 2, 0, 0.456, 0.025, 0.176, 0.392},     {16, 256, 128, 8, 1, 2.57, 0.764, 0.194, 0, 0.122},
     {13, 128, 256, 8, 1, 2.93, 0.869, 0.186, 0, 0.061},     {20, 256, 256, 8, 1, 6.10, 1.200, 0.422, 0, 0.024}};
-constexpr TileCosts W4_TILE_COSTS = {0.277, 1.42, 0.796, 0.162};
+constexpr TileCosts W4_TILE_COSTS = {0.277, 1.42, 0.796, 0.162, 0.0};
 
 // Without direct-to-LDS loads (an A of 4 GiB and more): the largest register-staged tile that fills the device.
 static int pick_register_staged(int M, int N) {
@@ -76,8 +76,10 @@ static TilePlan make_plan_prefill(int M, int N, int K, bool reg_ok) {
       consider_tile_plan(best, t, W4_TILE_COSTS, M, N, 0.5 * N * K, tiles, sk, 0, 2.0 * G, cus, 1ll << 32);
       continue;
     }
-    // K in up to 8 parts of at least 3 groups, on up to 2.4 rounds of workgroups
-    for (int sk : {1, 2, 3, 4, 6, 8})
+    // K in up to 8 parts of at least 3 groups, on up to 2.4 rounds of workgroups.  (All of 1 .. 8: without 5 and 7 12 % of the
+    // problems had another plan, in the mean 3.2 % slower; 48 tiles fill one round in five parts only, 24576 x 6144 at M = 512
+    // 154 -> 146 us, 11648 x 1984 at M = 277 27.6 -> 21.4 us)
+    for (int sk = 1; sk <= 8; ++sk)
       if (sk == 1 || (G / sk >= 3 && tiles * sk * 10 <= cus * 24)) consider(sk, 0);
     // 256 x 256 tiles that end in a round of workgroups at most half full: the tiles of that round in parts of at least 8 groups
     // that fill it, the others whole (4096 x 6144 at M = 4096: 384 tiles = 256 whole + 128 in two parts each, 205 -> 189 us)
