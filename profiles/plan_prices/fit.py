@@ -248,7 +248,7 @@ class Decode:
 
     def price(self, t, at):
         base, round_, fill_kb, mem_mb, again, reduce_, handover, part, part_mb = t[:9]
-        latency, work, sub_work, chain, last, pair = t[9:12], t[12:15], t[15:18], t[18], t[19], t[20]
+        latency, work, sub_work, chain, last, pair, spread = t[9:12], t[12:15], t[15:18], t[18], t[19], t[20], t[21]
         k, n, m, gs, wks, wn, sk, mr, mb, copies, tpg = (a[at] for a in (self.k, self.n, self.m, self.gs, self.wks, self.wn, self.sk,
                                                                        self.mr, self.mb, self.copies, self.tpg))
         sub = self.sub[at]
@@ -266,6 +266,8 @@ class Decode:
         core = slow * rounds * (round_ / slots + fill + gs * tile + reduce_ * np.log2(wks))
         mem = mem_mb * 0.5e-6 * k * n * tpg * (1 + again * (copies - 1))
         us = base + (core ** 3 + mem ** 3) ** (1 / 3)
+        xcds = 8 // np.gcd(-(-(n // 16) // wn), 8)
+        us = us + spread * (np.minimum(copies, xcds) - 1) / 7.0
         return us + (sk > 1) * (handover + sk * (part + part_mb * 4e-6 * m * n))
 
     def prices(self, p=None):
@@ -319,11 +321,11 @@ def main():
             def prices(p, at=at, where=where):
                 out = t.tile_us[at]
                 for j, w in enumerate(where):
-                    out[w] = t.price(p[21 * j:21 * j + 21], at[w])
+                    out[w] = t.price(p[22 * j:22 * j + 22], at[w])
                 return out
             p = fit(prices, np.concatenate([t.p[x] for x in names]), t.us[at], np.unique(t.key[at], return_inverse=True)[1], 0.15)
             for j, name in enumerate(names):
-                t.p[name] = p[21 * j:21 * j + 21]
+                t.p[name] = p[22 * j:22 * j + 22]
                 print(name, ", ".join(f"{v:.3g}" for v in t.p[name]))
     elif refit:
         at = t.allowed()

@@ -214,8 +214,8 @@ def scan_decode(lib, rng, until, out):
             if us is not None:
                 print(k, n, m, 128 // group, int(bits == 8), 2, 0, 0, 0, f"{us:.2f}", sep=",", file=out)
             for split, gs, wks, nt in decode_plans(k, n, m, group, bits):
-                wns = sorted({w for w in (1, 2, 3, 4, 6, 7, 8, 12, 16) if 4 <= w * wks <= 16}) if split else [0]
-                for wn in rng.sample(wns, min(3, len(wns))):
+                wns = [w for w in range(1, 17) if 4 <= w * wks <= 16] if split else [0]
+                for wn in rng.sample(wns, min(4, len(wns))):
                     fields = dict(decode_impl=1, decode2_gs=gs, decode2_wks=wks, decode2_wn=wn)
                     us = layer.time(lib, m, path=0 if split else 1, exp={2: 2 if split else 1}, **fields)
                     if us is not None:

@@ -642,3 +642,15 @@ def test_fp8_tile_plans_hold_for_calls_replayed_from_a_graph():
     for m, n, k in ((64, 4096, 4096), (48, 6144, 4096), (64, 6144, 4096)):
         assert _lib.load().vaq_fp8_scaled_mm_workspace(m, n, k, ctypes.byref(tmp), ctypes.byref(cnt)) == _lib.VAQ_OK
         assert tmp.value == 0 and cnt.value == 0
+
+
+def test_rows_over_workgroups_keep_copies_of_a_stream_on_one_xcd():
+    """Workgroups of 16 rows: the copies of an n-tile range lie a grid row apart, on one XCD where 8 divides the row's length, on all
+    eight where it is odd.  On layers of few megabytes no plan of many copies has an odd row."""
+    import ctypes
+    from vllm_amd import _lib
+    lib, plan = _lib.load(), (ctypes.c_double * 6)()
+    for m, n, k in ((201, 704, 768), (102, 1280, 896), (136, 2048, 1024), (85, 3584, 1024), (165, 2048, 1280), (162, 3072, 384), (98, 8192, 1792),
+                    (98, 5632, 512)):
+        assert lib.vaq_w4a16_decode_plan(m, n, k, 1, 0, 2, plan) == _lib.VAQ_OK and plan[5] > 0
+        assert -(-n // 16 // int(plan[2])) % 2 == 0, (m, n, k, list(plan))

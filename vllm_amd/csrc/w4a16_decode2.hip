@@ -202,35 +202,40 @@ static Decode2Config pick_by_rule(int M, int N, int K, int sub, bool w8, int nt_
 // wavefronts, more than four to a unit, take `pair` times as long; beside that the weights from memory (`mem_mb` per MB, and
 // `again` times that for every further copy of the stream, which L2 serves); `base` per launch; a K split over workgroups costs
 // `handover` + `part` per part + `part_mb` per MB of partial results.  [.]: one staged row, 4 or 8, 16.  `sub_work`: groups of
-// 128, 64, 32 rows.
+// 128, 64, 32 rows.  `spread`: rows over workgroups, the copies of an n-tile range are a grid row (gx workgroups) apart and meet on
+// one XCD only if 8 divides gx; with gx odd they are on all eight, each of which brings the stream into its L2 (14-20 % of a launch
+// below 4 MB of weights, 6-10 % to 16 MB: 1 .. 1.5 us whatever the size).  768 x 704 at M = 201 5.6 -> 4.2 us (one n-tile to a
+// workgroup, gx = 44, instead of three, gx = 15), 1792 x 8192 at M = 98 14.4 -> 12.3 us; over 6808 problems whose plan it changes
+// 3.3 % in the mean.
 // Fitted to the cold times of 1.5e5 launches: 6400 problems of random layers, half of them with K 1024 .. 14336 and N 1024 ..
-// 28672, half with K 256 .. 28672 and N 256 .. 152064, 1 .. 256 rows, each with up to 60 splits (profiles/plan_prices).  The cheapest
-// plan by these figures takes 1.02 of the fastest one's time (geometric mean; 99 of 100 less than 1.23), N > 28672 1.03, K or N
-// below 1024 1.014.  Constants of the formula without `chain`, `last` and `pair`, fitted to the first half only, were at 1.047, 1.067
+// 28672, half with K 256 .. 28672 and N 256 .. 152064, 1 .. 256 rows, each with up to 60 splits (the first part of those in
+// profiles/plan_prices; rows over workgroups with 8-bit codes and `spread` to all of them).  The cheapest plan by these figures takes
+// 1.016 of the fastest one's time (geometric mean over 16672 problems; 99 of 100 less than 1.21), N > 28672 1.026, K or N below 1024
+// 1.013.  Constants of the formula without `chain`, `last` and `pair`, fitted to the first half only, were at 1.047, 1.067
 // and 1.060 over these problems.
 struct Decode2Cost {
   double base, round, fill_kb, mem_mb, again, reduce, handover, part, part_mb;
   double tile_latency[3], tile_work[3], sub_work[3];
-  double chain, last, pair;
+  double chain, last, pair, spread;
 };
 constexpr Decode2Cost D2_COST_W8 = {1.09, 1.63, 0.0154, 0.0469, 0, 0.00669, 1.12, 0.275, 0.409,
-                                    {0.9, 0.875, 0.665}, {0.0215, 0.022, 0.0209}, {1.15, 1.35, 1.95}, 0.116, 0.108, 1.29};
+                                    {0.9, 0.875, 0.665}, {0.0215, 0.022, 0.0209}, {1.15, 1.35, 1.95}, 0.116, 0.108, 1.29, 0};
 constexpr Decode2Cost D2_COST_SUB = {1.18, 1.3, 0.0144, 0.0468, 0, 0.0041, 1.16, 0.301, 0,
-                                     {0.796, 0.909, 0.834}, {0.0278, 0.0271, 0.028}, {1, 1.11, 1.55}, 0.127, 0.143, 1.35};
+                                     {0.796, 0.909, 0.834}, {0.0278, 0.0271, 0.028}, {1, 1.11, 1.55}, 0.127, 0.143, 1.35, 0};
 // two m-blocks (groups of 128 rows / channelwise: three and four)
 constexpr Decode2Cost D2_COST_W8_MB2 = {0.149, 0.0523, 0.000908, 0.0746, 0, 0.848, 0.588, 0.231, 0.597,
-                                        {1.8, 1.8, 1.59}, {0.0586, 0.0586, 0.0342}, {1.41, 1.65, 2.41}, 0.142, 0.428, 1.06};
+                                        {1.8, 1.8, 1.59}, {0.0586, 0.0586, 0.0342}, {1.41, 1.65, 2.41}, 0.142, 0.428, 1.06, 0};
 constexpr Decode2Cost D2_COST_SUB_MB2 = {0.772, 0.979, 0.0147, 0.071, 0, 0.218, 0.395, 0.3, 0.46,
-                                         {1.84, 1.84, 1.63}, {0.0643, 0.0643, 0.0498}, {1, 1.08, 1.46}, 0.0313, 0.379, 0.968};
+                                         {1.84, 1.84, 1.63}, {0.0643, 0.0643, 0.0498}, {1, 1.08, 1.46}, 0.0313, 0.379, 0.968, 0};
 constexpr Decode2Cost D2_COST_MB34 = {1.97, 1.26, 0.0179, 0.158, 0, 0.0465, 0.224, 0.328, 0.782,
-                                      {1.97, 1.97, 0.468}, {0.0886, 0.0886, 0.00497}, {1.72, 1, 1}, 0.107, 0.395, 1.2};
+                                      {1.97, 1.97, 0.468}, {0.0886, 0.0886, 0.00497}, {1.72, 1, 1}, 0.107, 0.395, 1.2, 0};
 // the rows split over workgroups (never with a split K)
-constexpr Decode2Cost D2_COST_ROWS_W8 = {1.51, 1.63, 0.00925, 0.341, 0.124, 0.0156, 0, 0, 0,
-                                         {0.86, 0.86, 0.389}, {0.0336, 0.0336, 0.0171}, {1.33, 1.57, 2.22}, 0.126, 0.138, 1.2};
+constexpr Decode2Cost D2_COST_ROWS_W8 = {1.15, 1.41, 0.013, 0.409, 0.0868, 0.0134, 0, 0, 0,
+                                         {0.86, 0.86, 0.411}, {0.0336, 0.0336, 0.0173}, {1.27, 1.51, 2.19}, 0.113, 0.146, 1.2, 2.57};
 constexpr Decode2Cost D2_COST_ROWS_SUB = {1.54, 1.24, 0.0103, 0.229, 0.267, 0.00948, 0, 0, 0,
-                                          {1.36, 1.36, 0.0918}, {0.0476, 0.0476, 0.0195}, {1, 1.49, 2.01}, 0.151, 0.153, 1.2};
+                                          {1.36, 1.36, 0.0918}, {0.0476, 0.0476, 0.0195}, {1, 1.49, 2.01}, 0.151, 0.153, 1.2, 1.5};
 constexpr Decode2Cost D2_COST_ROWS = {1.4, 1.16, 0.0093, 0.0946, 0.368, 0.0106, 0, 0, 0,
-                                      {1.02, 1.02, 0.392}, {0.037, 0.037, 0.0181}, {1.74, 1, 1}, 0.107, 0.237, 1.2};
+                                      {1.02, 1.02, 0.392}, {0.037, 0.037, 0.0181}, {1.74, 1, 1}, 0.107, 0.237, 1.2, 1.5};
 
 static const Decode2Cost& workgroup_cost(int M, int sub, bool w8) {
   if (w8) return M > 16 ? D2_COST_W8_MB2 : D2_COST_W8;
@@ -257,6 +262,10 @@ static double decode2_us(const Decode2Cost& t, const Decode2Config& c, int M, in
   const double mem = t.mem_mb * 0.5e-6 * (double)K * N * TPG * (1 + t.again * (copies - 1));
   double us = t.base + cbrt(core * core * core + mem * mem * mem);
   if (c.sk > 1) us += t.handover + c.sk * (t.part + t.part_mb * 4e-6 * (double)M * N);
+  if (copies > 1) {
+    const long gx = (N / 16 + c.wn - 1) / c.wn, xcds = gx % 8 == 0 ? 1 : gx % 4 == 0 ? 2 : gx % 2 == 0 ? 4 : 8;
+    us += t.spread * (double)((copies < xcds ? copies : xcds) - 1) / 7.0;
+  }
   return us;
 }
 
