@@ -1,7 +1,7 @@
 """Fits the price formulas of the tile kernels and of the W4A16 decode kernel to the timings of scan.py, and says how good
 the plans are that they choose.
 
-    python profiles/plan_prices/fit.py fp8_tile|w4_tile|w4_decode TIMINGS.csv[.gz] [...] [--fit]
+    python profiles/plan_prices/fit.py fp8_tile|w4_tile|w8_tile|w4_decode TIMINGS.csv[.gz] [...] [--fit]
 
 Without --fit: the constants of the sources, read from them.  The formulas are those of `tile_plan_us` in
 vllm_amd/csrc/tile_plan.h and `decode2_us` in vllm_amd/csrc/w4a16_decode2.hip.
@@ -40,13 +40,13 @@ class Tiles:
         self.kind = kind
         fp8 = kind == "fp8_tile"
         file = "fp8_scaled_mm.hip" if fp8 else "w4a16_prefill.hip"
-        prefix = "FP8" if fp8 else "W4"
+        prefix = kind.split("_")[0].upper()
         rows = np.array(source_table(file, f"{prefix}_TILE_SHAPES")).reshape(-1, 10)
         self.ids = rows[:, 0].astype(int)
         self.shape = rows[:, 1:5]                        # bm, bn, nw, slots
         self.p_shape = rows[:, 5:]                       # base, step, load, shared, out
         self.p_costs = np.array(source_table(file, f"{prefix}_TILE_COSTS"))
-        self.bytes = 1.0 if fp8 else 0.5
+        self.bytes = 0.5 if kind in ("w4_tile", "lds_tile") else 1.0
 
     def pack(self):
         return np.concatenate([self.p_shape.ravel(), self.p_costs])
@@ -191,8 +191,9 @@ def pick_wn(nt, sk, wks, lds):
 
 
 def tile_prices(k, n, m, any_shape):
-    """What the W4A16 tile kernel's cheapest plan is priced at; `any_shape`: the 128 x 256 tiles are built for the format."""
-    t = Tiles("w4_tile")
+    """What the cheapest plan of the W4A16 tile kernel with weights through LDS is priced at, which the decode kernels are weighed
+    against; `any_shape`: the 128 x 256 tiles are built for the format."""
+    t = Tiles("lds_tile")
     best = np.full(len(k), np.inf)
     t.k, t.n, t.m = k, n, m
     for i, ident in enumerate(t.ids):

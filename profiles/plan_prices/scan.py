@@ -1,14 +1,15 @@
 """Times every plan of random problems, for the price formulas that choose among them (fit.py).
 
-    python profiles/plan_prices/scan.py fp8_tile|w4_tile|w4_decode SECONDS SEED OUT.csv
+    python profiles/plan_prices/scan.py fp8_tile|w4_tile|w8_tile|w4_decode SECONDS SEED OUT.csv
 
 Runs on the GPU; the *.csv.gz beside it are what it wrote on an MI355X.  A problem is a layer (K, N) and a number of rows; a plan is forced through the `_tuned` entry points
 (vllm_amd/csrc/vaq_tuning.h).  Weights are cold: a graph of launches walks over copies of the layer (640 MB of them, at most
 400).  One line per plan, with the time of a launch in us:
 
-    fp8_tile, w4_tile:  k, n, m, tile id, parts of K, 1 if only the tiles of the last round are in parts, us
+    fp8_tile, w4_tile, w8_tile (8-bit codes):  k, n, m, tile id, parts of K, 1 if only the tiles of the last round are in parts, us
     w4_decode:          k, n, m, groups of 128 rows (1, 2, 4), 8-bit codes, kind, gs, wks, wn (0: by the planner), us
-                        kind 0 workgroups of all rows, 1 of 16 rows, 2 the tile kernel by its own plan (gs, wks, wn 0)
+                        kind 0 workgroups of all rows, 1 of 16 rows, 2 the tile kernel by its own plan (gs, wks, wn 0; recorded
+                        with the shapes up to 20 only, at whose price the decode kernels are weighed)
 """
 from __future__ import annotations
 
@@ -133,7 +134,11 @@ def shape(rng, step_n, most):
 
 
 TILES = {"fp8_tile": {13: (128, 128), 14: (64, 128), 15: (64, 64), 16: (128, 64), 17: (128, 256), 19: (256, 128), 1: (256, 256), 10: (256, 384)},
-         "w4_tile": {12: (128, 128), 14: (64, 128), 15: (128, 64), 16: (256, 128), 13: (128, 256), 20: (256, 256), 30: (256, 256)}}
+         "w4_tile": {12: (128, 128), 14: (64, 128), 15: (128, 64), 16: (256, 128), 13: (128, 256), 20: (256, 256), 30: (256, 256),
+                     41: (32, 128), 51: (32, 64), 42: (64, 128), 52: (64, 64), 43: (96, 128), 44: (128, 128), 46: (128, 256), 66: (128, 256),
+                     48: (256, 256)},
+         "w8_tile": {12: (128, 128), 14: (64, 128), 15: (128, 64), 16: (256, 128), 20: (256, 256), 41: (32, 128), 51: (32, 64), 42: (64, 128),
+                     52: (64, 64), 43: (96, 128), 44: (128, 128), 46: (128, 256)}}
 
 
 def tile_plans(kind, k, n, m):
@@ -149,7 +154,7 @@ def tile_plans(kind, k, n, m):
         for sk in range(1, 9):
             if sk == 1 or (steps // sk >= (6 if kind == "fp8_tile" else 3) and tiles * sk <= CUS * 3 and ident != 30):
                 yield ident, sk, 0
-        if ident in (1, 20) and tiles > CUS and rest:
+        if ident in (1, 20, 48) and tiles > CUS and rest:
             for sk in (2, 3, 4):
                 if rest * sk <= CUS and steps // sk >= (12 if kind == "fp8_tile" else 6):
                     yield ident, sk, 1
@@ -162,7 +167,7 @@ def scan_tiles(lib, kind, rng, until, out):
         rows = [m for m in (log(rng, 9 if fp8 else 17, 8192, 1) for _ in range(3)) if 2.0 * m * n * k < 2e12 and m * n < 6e8]
         if not rows:
             continue
-        layer = Layer(fp8, k, n, max(rows))
+        layer = Layer(fp8, k, n, max(rows), 8 if kind == "w8_tile" else 4)
         if not layer.fits():
             continue
         for m in rows:

@@ -124,4 +124,41 @@ __device__ inline bool handover_finish(float* c_tmp, int32_t* counters, v16f (&a
   return true;
 }
 
+// The same for a wavefront that holds NP 16-byte pieces of the tile's sum per lane (KiB-sized units, one counter per wavefront).
+template <int NP, int NW>
+__device__ inline bool handover_pieces(float* c_tmp, int32_t* counters, v4f (&part)[NP], const TileSlot& sl, int wave, int lane) {
+  constexpr int SC1 = 16;
+  const int nsplit = sl.nsplit;
+  const uint32_t unit = (uint32_t)((sl.unit * NW + wave) * NP) * 1024u;          // bytes
+  const uint32_t split_stride = (uint32_t)sl.units * (uint32_t)(NW * NP) * 1024u;
+  const __amdgpu_buffer_rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc(c_tmp, 0, (int)(split_stride * (uint32_t)nsplit), 0x00020000);
+#pragma unroll
+  for (int c = 0; c < NP; ++c)
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, part[c]), rt, lane * 16, (int)(sl.split * split_stride + unit + c * 1024), SC1);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // the part is acknowledged before the counter moves
+  int32_t* ctr = counters + (int64_t)sl.unit * NW + wave;
+  int old = 0;
+  if (lane == 0) old = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  old = __builtin_amdgcn_readfirstlane(old);
+  if (old != nsplit - 1) return false;
+#pragma unroll
+  for (int c = 0; c < NP; ++c) part[c] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < nsplit; s0 += 2) {
+    const int s1 = s0 + 1 < nsplit ? s0 + 1 : s0;
+    v4u r0[NP], r1[NP];
+#pragma unroll
+    for (int c = 0; c < NP; ++c) r0[c] = __builtin_amdgcn_raw_buffer_load_b128(rt, lane * 16, (int)(s0 * split_stride + unit + c * 1024), SC1);
+#pragma unroll
+    for (int c = 0; c < NP; ++c) r1[c] = __builtin_amdgcn_raw_buffer_load_b128(rt, lane * 16, (int)(s1 * split_stride + unit + c * 1024), SC1);
+#pragma unroll
+    for (int c = 0; c < NP; ++c) part[c] += __builtin_bit_cast(v4f, r0[c]);
+    if (s0 + 1 < nsplit) {
+#pragma unroll
+      for (int c = 0; c < NP; ++c) part[c] += __builtin_bit_cast(v4f, r1[c]);
+    }
+  }
+  if (lane == 0) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
 }  // namespace vaq

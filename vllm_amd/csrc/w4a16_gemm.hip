@@ -157,7 +157,7 @@ extern "C" int vaq_w4a16_gemm_tuned(const void* a, int64_t lda, const int32_t* b
       tile_ok = perm == nullptr && c_tmp_bytes >= (int64_t)t && counter_ints >= (int64_t)n;
     }
     const int kind = w4a16_decode2_choose((int)size_m, (int)size_n, (int)size_k, sub, wt, perm != nullptr, decode, tile_ok || !decode,
-                                          w4a16_prefill_us((int)size_m, (int)size_n, (int)size_k, !w8 && sub == 1));
+                                          w4a16_staged_us((int)size_m, (int)size_n, (int)size_k, !w8 && sub == 1));
     decode = kind != D2_TILE;
     rows = kind == D2_ROWS;
   }

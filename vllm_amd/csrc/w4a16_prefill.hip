@@ -4,6 +4,8 @@
 #include "w4a16_kernels.h"
 #include "w4a16_prefill_kernel.h"
 
+#include <iterator>
+
 namespace vaq {
 
 // ----------------------------------------------------------------------------- host side
@@ -11,6 +13,10 @@ namespace vaq {
 // tile ids: 0..2 = register-staged kernel (256x256, 128x128, 64x128); 10.. = direct-to-LDS kernel (BM x BN);
 // 30 = 256 x 256 with the weights dequantised in registers (w4a16_prefill3_kernel.h)
 int prefill_launch_reg(const PrefillParams& p, bool bf16, bool zp, hipStream_t s);      // w4a16_prefill3.hip
+// w4a16_strip*.hip
+int prefill_launch_strip(const PrefillParams& p, int tile, bool bf16, bool zp, hipStream_t s);
+int prefill_launch_strip_sub(const PrefillParams& p, int sub, int tile, bool bf16, bool zp, hipStream_t s);
+int prefill_launch_strip_w8(const PrefillParams& p, int sub, int tile, bool bf16, hipStream_t s);
 
 template <bool BF16, bool HAS_ZP>
 static int dispatch_tile(const PrefillParams& p, int tile, hipStream_t s) {
@@ -33,18 +39,50 @@ static int dispatch_tile(const PrefillParams& p, int tile, hipStream_t s) {
   return VAQ_ERR_UNSUPPORTED;
 }
 
-// Fitted to 815 problems with M = 65 .. 6000, K = 1024 .. 14336, N = 1024 .. 28672 drawn over the logarithm (4-bit codes with zero
-// points, bf16), every shape and K split of each timed on cold weights.  Over the same 815 problems the plans that rules by size
-// had chosen were in the mean 10 % slower than the fastest one (5 % of it the eight-wavefront shapes 12, 14 and 16 that came with
-// the prices: 4096 x 4096 at M = 1024 50.7 -> 45.6 us, at M = 2048 77 -> 71 us, 4096 x 6144 at M = 333 34.6 -> 32.8 us, 4096 x 28672
-// at M = 100 48.7 -> 43.1 us; nothing where the rules had the 256 x 256 tiles right, M = 4096).  Checked over 3276 problems with M = 17 ..
-// 8192, K = 256 .. 28672, N = 256 .. 152064 (47137 launches, profiles/plan_prices): the cheapest plan is in the mean 1.1 % slower than
-// the fastest (N > 28672 0.8 %, K or N below 1024 0.8 %, 17 .. 128 rows 1.4 - 2.0 %), 99 of 100 less than 15 %.
+// What the tile shapes cost, by weight format (tile_plan.h).
+// 4-bit codes: fitted to 2712 problems with M = 17 .. 8192, half of them with K = 1024 .. 14336 and N = 1024 .. 28672, half with K =
+// 256 .. 28672 and N = 256 .. 152064, drawn over the logarithm, every shape and K split of each timed on cold weights (104302
+// launches, profiles/plan_prices; bf16, zero points).  The cheapest plan is in the mean 0.7 % slower than the fastest, 99 of 100 less
+// than 10 %; groups of 64 / 32 rows take the same constants (568 problems of 32-row groups: 0.7 %).  The fastest plan of the shapes
+// 12 .. 20 (weights through LDS) takes this much more than that of the shapes from 41 on (strips): 41 / 29 / 26 / 22 / 17 / 11 / 8 / 3 %
+// at M up to 32 / 64 / 128 / 256 / 512 / 1024 / 2048 / 8192; at M > 512 it is ahead in 10-25 % of the problems, by a few percent.
 constexpr TileShape W4_TILE_SHAPES[] = {
+    {12, 128, 128, 8, 2, 0.536, 0.606, 0.0793, 0.375, 0.153}, {14, 64, 128, 8, 2, 0, 0.535, 0.0271, 0.177, 0.252},
+    {15, 128, 64, 4, 2, 0, 0.553, 0.0166, 0.0944, 0.337},     {16, 256, 128, 8, 1, 1.88, 0.781, 0.176, 0, 0.0912},
+    {13, 128, 256, 8, 1, 2.36, 0.829, 0.193, 0, 0.0731},      {20, 256, 256, 8, 1, 3.75, 1.23, 0.279, 0, 0.0186},
+    {41, 32, 128, 8, 2, 1.99, 0.202, 0.0375, 0.163, 0.118},   {51, 32, 64, 8, 2, 1.43, 0.104, 0.0134, 0.148, 0.399},
+    {42, 64, 128, 8, 2, 2.44, 0.233, 0.0366, 0.25, 0.116},    {52, 64, 64, 8, 1, 2.68, 0.138, 0.0327, 0, 0.0886},
+    {43, 96, 128, 8, 1, 3.1, 0.266, 0.085, 0, 0.169},         {44, 128, 128, 8, 1, 3.63, 0.328, 0.114, 0, 0.126},
+    {46, 128, 256, 8, 1, 3.64, 0.495, 0.324, 0, 0.0655},      {66, 128, 256, 8, 1, 6.38, 0.566, 0.164, 0, 0.119},
+    {48, 256, 256, 8, 1, 8.35, 0.917, 0.387, 0, 0.0423}};
+constexpr TileCosts W4_TILE_COSTS = {0.163, 0.628, 0.63, 0.253, 0.0};
+// 8-bit codes, whose dequantisation takes longer: 993 such problems, 27863 launches, in the mean 0.8 % (2.4 % with the constants above).
+constexpr TileShape W8_TILE_SHAPES[] = {
+    {12, 128, 128, 8, 2, 0.783, 0.635, 0.0684, 0.441, 0.0986}, {14, 64, 128, 8, 2, 0.0101, 0.595, 0.0269, 0.17, 0.261},
+    {15, 128, 64, 4, 2, 0.0105, 0.608, 0.0138, 0.106, 0.362},  {16, 256, 128, 8, 1, 1.74, 0.879, 0.156, 0, 0.0659},
+    {20, 256, 256, 8, 1, 4.63, 1.25, 0.226, 0, 0.0177},
+    {41, 32, 128, 8, 2, 3.13, 0.244, 0.0253, 0.251, 0.104},    {51, 32, 64, 8, 1, 1.55, 0.164, 0.0131, 0, 0.676},
+    {42, 64, 128, 8, 1, 2.76, 0.323, 0.0451, 0, 0.104},        {52, 64, 64, 8, 1, 2.7, 0.187, 0.0172, 0, 0.0905},
+    {43, 96, 128, 8, 1, 3.07, 0.371, 0.0552, 0, 0.297},        {44, 128, 128, 8, 1, 3.6, 0.421, 0.0724, 0, 0.247},
+    {46, 128, 256, 8, 1, 5.19, 0.669, 0.163, 0, 0.0913}};
+constexpr TileCosts W8_TILE_COSTS = {0.176, 0.376, 0.706, 0.291, 0.0};
+// The shapes with weights through LDS by themselves, fitted to 815 problems of 4-bit codes: what FP8 weights are built for (but 13),
+// and the price that up to 256 rows are weighed against the decode kernels at (w4a16_staged_us).
+constexpr TileShape LDS_TILE_SHAPES[] = {
     {12, 128, 128, 8, 2, 0.39, 0.578, 0.092, 0.352, 0.226}, {14, 64, 128, 8, 2, 0, 0.426, 0.041, 0.230, 0.330},
     {15, 128, 64, 4, 2, 0, 0.456, 0.025, 0.176, 0.392},     {16, 256, 128, 8, 1, 2.57, 0.764, 0.194, 0, 0.122},
     {13, 128, 256, 8, 1, 2.93, 0.869, 0.186, 0, 0.061},     {20, 256, 256, 8, 1, 6.10, 1.200, 0.422, 0, 0.024}};
-constexpr TileCosts W4_TILE_COSTS = {0.277, 1.42, 0.796, 0.162, 0.0};
+constexpr TileCosts LDS_TILE_COSTS = {0.277, 1.42, 0.796, 0.162, 0.0};
+struct TilePrices {
+  const TileShape *begin, *end;
+  const TileCosts& costs;
+  double weight_bytes;      // per element, as the fit counted them
+};
+static TilePrices tile_prices(TileFormat format) {
+  if (format == TILES_8BIT) return {std::begin(W8_TILE_SHAPES), std::end(W8_TILE_SHAPES), W8_TILE_COSTS, 1.0};
+  if (format == TILES_FP8 || format == TILES_PLAIN_STAGED) return {std::begin(LDS_TILE_SHAPES), std::end(LDS_TILE_SHAPES), LDS_TILE_COSTS, 0.5};
+  return {std::begin(W4_TILE_SHAPES), std::end(W4_TILE_SHAPES), W4_TILE_COSTS, 0.5};
+}
 
 // Without direct-to-LDS loads (an A of 4 GiB and more): the largest register-staged tile that fills the device.
 static int pick_register_staged(int M, int N) {
@@ -53,27 +91,30 @@ static int pick_register_staged(int M, int N) {
   return tiles(256, 256) >= cus ? 0 : (tiles(128, 128) >= cus ? 1 : 2);
 }
 
-// Tile shape and K split for a problem.  `reg_ok`: 4-bit codes in groups of 128 rows or channelwise -- what the shapes 13 and 30
-// are built for.
-static TilePlan make_plan_prefill(int M, int N, int K, bool reg_ok) {
+// Tile shape and K split for a problem (the shapes 13, 30, 48 and 66 are built for TILES_PLAIN).
+static TilePlan make_plan_prefill(int M, int N, int K, TileFormat format) {
   const int64_t cus = num_cus_current_device();
   const int G = K / 128;
   const VaqTuning& tn = tuning();
   const int forced = tn.prefill_tile - 1;
+  const bool plain = format == TILES_PLAIN || format == TILES_PLAIN_STAGED;
+  const TilePrices prices = tile_prices(format);
+  const double weight_bytes = prices.weight_bytes * N * K;
   TilePlan best;
   // partial tiles are addressed with 32-bit offsets; the entry point on library-owned scratch says what room it has for them
   const int64_t most = tn.exp[14] > 0 ? (int64_t)tn.exp[14] * 1024 : (1ll << 32);
-  for (const TileShape& t : W4_TILE_SHAPES) {
-    const bool is256 = t.id == 20;
-    if (forced >= 0 ? forced != t.id && !(is256 && (forced == 10 || forced == 11 || forced == 30)) : t.id == 13 && !reg_ok) continue;
+  for (const TileShape* shape = prices.begin; shape != prices.end; ++shape) {
+    const TileShape& t = *shape;
+    const bool is256 = t.id == 20 || t.id == 48;
+    if (forced >= 0 ? forced != t.id && !(t.id == 20 && (forced == 10 || forced == 11 || forced == 30)) : (t.id == 13 || t.id == 48 || t.id == 66) && !plain) continue;
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
     const int64_t rest = tiles % cus;
     auto consider = [&](int sk, int64_t tail_first) {
-      consider_tile_plan(best, t, W4_TILE_COSTS, M, N, 0.5 * N * K, tiles, sk, tail_first, 2.0 * G, cus, sk > 1 ? most : 1);
+      consider_tile_plan(best, t, prices.costs, M, N, weight_bytes, tiles, sk, tail_first, 2.0 * G, cus, sk > 1 ? most : 1);
     };
     if (tn.prefill_split > 0) {
       const int sk = tn.prefill_split <= G ? tn.prefill_split : G;
-      consider_tile_plan(best, t, W4_TILE_COSTS, M, N, 0.5 * N * K, tiles, sk, 0, 2.0 * G, cus, 1ll << 32);
+      consider_tile_plan(best, t, prices.costs, M, N, weight_bytes, tiles, sk, 0, 2.0 * G, cus, 1ll << 32);
       continue;
     }
     // K in up to 8 parts of at least 3 groups, on up to 2.4 rounds of workgroups.  (All of 1 .. 8: without 5 and 7 12 % of the
@@ -91,7 +132,7 @@ static TilePlan make_plan_prefill(int M, int N, int K, bool reg_ok) {
   if (forced >= 0 && best.id >= 0) {
     best.id = forced;
     if (forced == 11 || forced == 30) best.nw = 4;
-  } else if (best.id == 20 && best.sk == 1 && reg_ok && K >= 4096 && best.tiles * 5 >= cus * 4) {
+  } else if (best.id == 20 && best.sk == 1 && plain && K >= 4096 && best.tiles * 5 >= cus * 4) {
     // Whole 256 x 256 tiles on most of the device and a long K: dequantised in registers (four wavefronts of 256 x 64), 2 % ahead
     // of the eight wavefronts with alternating phases; on a short K, with fewer tiles or with a split K 1-7 % behind.
     best.id = 30;
@@ -100,7 +141,7 @@ static TilePlan make_plan_prefill(int M, int N, int K, bool reg_ok) {
   return best;
 }
 
-static TilePlan plan_prefill(int M, int N, int K, bool direct_ok, bool reg_ok) {
+static TilePlan plan_prefill(int M, int N, int K, bool direct_ok, TileFormat format) {
   const int forced = tuning().prefill_tile - 1;
   if (!direct_ok || (forced >= 0 && forced < 10)) {
     TilePlan pl;
@@ -108,18 +149,24 @@ static TilePlan plan_prefill(int M, int N, int K, bool direct_ok, bool reg_ok) {
     return pl;
   }
   static thread_local TilePlanTable table;
-  if (tuning_active()) return make_plan_prefill(M, N, K, reg_ok);
-  return table.get(M, N, K, num_cus_current_device() * 2 + (reg_ok ? 1 : 0), [&] { return make_plan_prefill(M, N, K, reg_ok); });
+  if (tuning_active()) return make_plan_prefill(M, N, K, format);
+  return table.get(M, N, K, num_cus_current_device() * 8 + format, [&] { return make_plan_prefill(M, N, K, format); });
 }
 
-// Predicted time of the tile kernel (negative: not known, register-staged tiles).
-double w4a16_prefill_us(int M, int N, int K, bool reg_ok) { return plan_prefill(M, N, K, true, reg_ok).us; }
+// Predicted time of the tile kernel whose weights pass through LDS (negative: not known, register-staged tiles): what the decode
+// kernels are weighed against.  The strips are faster than that, but both tile kernels round the scaled weights to 16 bits and the
+// decode kernels keep their scales in fp32: problems go from these to the strips only where they went to a tile kernel before there
+// were strips.
+double w4a16_staged_us(int M, int N, int K, bool plain) { return plan_prefill(M, N, K, true, plain ? TILES_PLAIN_STAGED : TILES_FP8).us; }
 
 int w4a16_prefill_workspace(int M, int N, int K, size_t* c_tmp_bytes, size_t* counter_ints) {
-  // enough for either choice of shapes: the weight format is not known here
-  const TilePlan a = plan_prefill(M, N, K, true, false), b = plan_prefill(M, N, K, true, true);
-  *c_tmp_bytes = (size_t)(a.tmp_bytes() > b.tmp_bytes() ? a.tmp_bytes() : b.tmp_bytes());
-  *counter_ints = (size_t)(a.counter_ints() > b.counter_ints() ? a.counter_ints() : b.counter_ints());
+  // enough for every weight format: it is not known here
+  *c_tmp_bytes = *counter_ints = 0;
+  for (TileFormat format : {TILES_PLAIN, TILES_SUB, TILES_8BIT, TILES_FP8}) {
+    const TilePlan pl = plan_prefill(M, N, K, true, format);
+    if ((size_t)pl.tmp_bytes() > *c_tmp_bytes) *c_tmp_bytes = (size_t)pl.tmp_bytes();
+    if ((size_t)pl.counter_ints() > *counter_ints) *counter_ints = (size_t)pl.counter_ints();
+  }
   return VAQ_OK;
 }
 
@@ -148,7 +195,7 @@ int w4a16_prefill_launch(const void* a, int64_t lda, const int32_t* b, const voi
     set_error("w4a16_gemm(prefill): 8-bit weights with an A of 4 GiB or more are not built");
     return VAQ_ERR_UNSUPPORTED;
   }
-  TilePlan pl = plan_prefill(M, N, K, direct_ok, !w8 && sub == 1);
+  TilePlan pl = plan_prefill(M, N, K, direct_ok, tile_format(sub, wt));
   // A caller that passes no scratch at all gets the unsplit kernel (same result, no K split); scratch that is there but
   // too small is the caller's mistake and is reported, not worked around.
   if (pl.sk > 1 && c_tmp == nullptr && counters == nullptr) pl.sk = 1;
@@ -170,7 +217,11 @@ int w4a16_prefill_launch(const void* a, int64_t lda, const int32_t* b, const voi
   int rc;
   // the alternating-phase and the register-dequantising variants exist for 4-bit codes in groups of 128 rows / channelwise
   const int tile_other = (pl.id == 20 || pl.id == 30) ? 10 : pl.id;
-  if (wt == 2) rc = prefill_launch_f8(p, tile_other, bf16, s);
+  if (pl.id > 40) {
+    if (w8) rc = prefill_launch_strip_w8(p, sub, pl.id, bf16, s);
+    else if (sub > 1) rc = prefill_launch_strip_sub(p, sub, pl.id, bf16, zp, s);
+    else rc = prefill_launch_strip(p, pl.id, bf16, zp, s);
+  } else if (wt == 2) rc = prefill_launch_f8(p, tile_other, bf16, s);
   else if (w8) rc = prefill_launch_w8(p, sub, tile_other, bf16, s);
   else if (sub > 1) rc = prefill_launch_sub(p, sub, tile_other, bf16, zp, s);
   else if (bf16) rc = zp ? dispatch_tile<true, true>(p, pl.id, s) : dispatch_tile<true, false>(p, pl.id, s);
