@@ -20,7 +20,6 @@ constexpr float FP8_MAX = 448.0f;
 // (measured: 512 threads with 4 vectors each against 256 x 8: 2.95 -> 2.68 us at 16 rows of 4096, 3.65 -> 3.3 us at 256
 // rows, 41.5 -> 39.5 us at 4096 rows of 14336, unchanged at 4096 x 4096; 1024 x 2 and 128 x 16 are slower)
 constexpr int QT = 512;         // threads per workgroup of the row-per-workgroup kernel (its TPB: QT or QT / 2)
-constexpr int QV = 4;           // cached 8-element vectors per thread
 constexpr int QTW = 256;        // threads per workgroup of the row-per-wavefront kernel (four rows)
 
 template <typename T>
@@ -40,49 +39,34 @@ __device__ inline float clamp448(float x) { return fmaxf(-FP8_MAX, fminf(x, FP8_
 __device__ inline uint32_t cvt2(float a, float b) { return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false) & 0xffffu; }
 __device__ inline uint8_t cvt1(float a) { return (uint8_t)(__builtin_amdgcn_cvt_pk_fp8_f32(a, a, 0, false) & 0xff); }
 
-// 8 consecutive elements of a row as floats
+// 8 consecutive elements of a row: requested by load(), as floats after unpack().  Apart, because a conversion behind each load
+// under its own condition waits for that load before the next is requested: four latencies for a row of 14336 instead of one.
 template <typename T>
 struct Vec8 {
   float f[8];
+  v4u raw[sizeof(T) / 2];
   __device__ inline void load(const T* p) {
-    if constexpr (sizeof(T) == 2) {
-      const v4u r = *reinterpret_cast<const v4u*>(p);
-      const uint32_t w[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        T lo, hi;
-        lo.v = (uint16_t)(w[i] & 0xffffu);
-        hi.v = (uint16_t)(w[i] >> 16);
-        f[2 * i] = load_as_float<T>(&lo);
-        f[2 * i + 1] = load_as_float<T>(&hi);
+    for (int i = 0; i < (int)sizeof(T) / 2; ++i) raw[i] = reinterpret_cast<const v4u*>(p)[i];
+  }
+  __device__ inline void unpack() {
+    const uint32_t* w = reinterpret_cast<const uint32_t*>(raw);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if constexpr (sizeof(T) == 2) {
+        const T h{(uint16_t)(w[i / 2] >> (16 * (i & 1)))};
+        f[i] = load_as_float<T>(&h);
+      } else {
+        f[i] = __builtin_bit_cast(float, w[i]);
       }
-    } else {
-      const v4f a = *reinterpret_cast<const v4f*>(p);
-      const v4f b = *reinterpret_cast<const v4f*>(p + 4);
-      f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w;
-      f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
     }
   }
 };
 
-template <int TPB>
-__device__ inline float block_max(float v, float* smem) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (lane == 0) smem[wave] = v;
-  __syncthreads();
-  float r = smem[0];
-#pragma unroll
-  for (int i = 1; i < TPB / 64; ++i) r = fmaxf(r, smem[i]);
-  __syncthreads();
-  return r;
-}
-
 // MODE 0: dynamic per token (divide by row scale, scale written per row)
 // MODE 1: per tensor with a given scale (multiply by reciprocal) -- static, and pass 2 of dynamic per tensor
 // MODE 2: absmax only: atomic max of rowmax/448 into *scale (pass 1 of dynamic per tensor)
-template <typename T, int MODE, int TPB>
+template <typename T, int MODE, int TPB, int QV>
 __global__ __launch_bounds__(TPB) void fp8_quant_kernel(const T* __restrict__ in, int64_t in_stride,
                                                         uint8_t* __restrict__ out, int64_t out_stride,
                                                         float* __restrict__ scales, const float* __restrict__ scale_ub,
@@ -96,7 +80,16 @@ __global__ __launch_bounds__(TPB) void fp8_quant_kernel(const T* __restrict__ in
   const bool vec_ok = (hidden % 8 == 0) && (((uintptr_t)x % 16) == 0) && (((uintptr_t)y % 8) == 0) &&
                       (hidden <= TPB * QV * 8);
   Vec8<T> cache[QV];
+  const float given = MODE == 1 ? *scales : 0.f;
   const int nvec = hidden / 8;
+
+  if (vec_ok) {
+#pragma unroll
+    for (int i = 0; i < QV; ++i) {
+      const int v = tid + i * TPB;
+      if (v < nvec) cache[i].load(x + (int64_t)v * 8);
+    }
+  }
 
   float scale_or_inv;
   if constexpr (MODE != 1) {
@@ -104,9 +97,8 @@ __global__ __launch_bounds__(TPB) void fp8_quant_kernel(const T* __restrict__ in
     if (vec_ok) {
 #pragma unroll
       for (int i = 0; i < QV; ++i) {
-        const int v = tid + i * TPB;
-        if (v < nvec) {
-          cache[i].load(x + (int64_t)v * 8);
+        if (tid + i * TPB < nvec) {
+          cache[i].unpack();
 #pragma unroll
           for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(cache[i].f[e]));
         }
@@ -126,14 +118,7 @@ __global__ __launch_bounds__(TPB) void fp8_quant_kernel(const T* __restrict__ in
       scale_or_inv = s;
     }
   } else {
-    scale_or_inv = 1.0f / (*scales);
-    if (vec_ok) {
-#pragma unroll
-      for (int i = 0; i < QV; ++i) {
-        const int v = tid + i * TPB;
-        if (v < nvec) cache[i].load(x + (int64_t)v * 8);
-      }
-    }
+    scale_or_inv = 1.0f / given;
   }
 
   // MODE 0 on 16-bit inputs whose quotients cannot leave the normal range (no upper bound that could shrink the scale
@@ -167,7 +152,10 @@ __global__ __launch_bounds__(TPB) void fp8_quant_kernel(const T* __restrict__ in
 #pragma unroll
       for (int i = 0; i < QV; ++i) {
         const int v = tid + i * TPB;
-        if (v < nvec) *reinterpret_cast<v2u*>(y + (int64_t)v * 8) = pack8(cache[i].f, conv);
+        if (v < nvec) {
+          if constexpr (MODE == 1) cache[i].unpack();
+          *reinterpret_cast<v2u*>(y + (int64_t)v * 8) = pack8(cache[i].f, conv);
+        }
       }
     }
   } else {
@@ -201,12 +189,12 @@ __global__ __launch_bounds__(QTW) void fp8_quant_row_per_wave_kernel(const T* __
   for (int i = 0; i < NV; ++i) {
     const int v = lane + i * 64;
     if (v < nvec) {
+      cache[i].unpack();
 #pragma unroll
       for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(cache[i].f[e]));
     }
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+  amax = wave_max(amax);
   float s = scale_ub ? fminf(amax, *scale_ub) : amax;
   s = fmaxf(s / FP8_MAX, 1.0f / (FP8_MAX * 512.0f));
   if (lane == 0) scales[row] = s;
@@ -258,25 +246,21 @@ static void launch_row_per_wave(const void* in, int64_t in_stride, uint8_t* out,
                        scales, ub, (int)hidden, rows);
 }
 
-// Many rows of at most 5120 elements run on workgroups of 256 threads: twice the workgroups per compute unit, each a
-// dependent chain of load, reduction and store of its own, and half the wavefronts in every barrier (4096 rows of 3072 /
-// 4096 / 5120: 10.5 / 12.4 / 14.2 -> 8.3 / 11.0 / 13.4 us, 8192 x 4096 20.9 -> 17.8 us; rows of 8192: 18.6 against 19.3 us
-// with 512 threads; a few hundred rows of 4096: 3.0 against 3.2 us).
-template <int MODE, int TPB>
+template <int MODE, int TPB, int QV>
 static int launch_quant_tpb(const void* in, int in_dtype, int64_t in_stride, uint8_t* out, int64_t out_stride,
                             float* scales, const float* ub, int64_t rows, int64_t hidden, hipStream_t s) {
   const dim3 grid((unsigned)rows), block(TPB);
   switch (in_dtype) {
     case VAQ_BF16:
-      hipLaunchKernelGGL((fp8_quant_kernel<bf16_t, MODE, TPB>), grid, block, 0, s, (const bf16_t*)in, in_stride, out,
+      hipLaunchKernelGGL((fp8_quant_kernel<bf16_t, MODE, TPB, QV>), grid, block, 0, s, (const bf16_t*)in, in_stride, out,
                          out_stride, scales, ub, (int)hidden);
       break;
     case VAQ_F16:
-      hipLaunchKernelGGL((fp8_quant_kernel<f16_t, MODE, TPB>), grid, block, 0, s, (const f16_t*)in, in_stride, out,
+      hipLaunchKernelGGL((fp8_quant_kernel<f16_t, MODE, TPB, QV>), grid, block, 0, s, (const f16_t*)in, in_stride, out,
                          out_stride, scales, ub, (int)hidden);
       break;
     case VAQ_F32:
-      hipLaunchKernelGGL((fp8_quant_kernel<float, MODE, TPB>), grid, block, 0, s, (const float*)in, in_stride, out,
+      hipLaunchKernelGGL((fp8_quant_kernel<float, MODE, TPB, QV>), grid, block, 0, s, (const float*)in, in_stride, out,
                          out_stride, scales, ub, (int)hidden);
       break;
     default:
@@ -286,12 +270,28 @@ static int launch_quant_tpb(const void* in, int in_dtype, int64_t in_stride, uin
   return VAQ_OK;
 }
 
+// Threads to a row and vectors of 8 elements to a thread.  One vector where 256 or 512 threads hold the row: the code is a third of
+// that for four, and a launch of few rows is mostly latency (768 rows of 1024 / 2048 / 4096 per token: 3.3 / 3.5 / 3.9 -> 2.6 / 2.9 /
+// 3.5 us, 16 rows of 4096 2.7 -> 2.4).  Many rows of up to 5120 elements run on 256 threads: twice the workgroups per compute unit,
+// each a dependent chain of load, reduction and store of its own, and half the wavefronts in every barrier (4096 rows of 4096 / 5120:
+// 10.7 / 12.6 us, 512 threads 12.4 / 14.2; 8192 wide 512 threads are ahead, 18.6 against 19.3).  Rows above 16384 take eight vectors
+// to a thread instead of reading memory twice by single elements (one row of 20480 13.2 -> 3.4 us, 4096 of them 121 -> 39).
 template <int MODE>
 static int launch_quant(const void* in, int in_dtype, int64_t in_stride, uint8_t* out, int64_t out_stride,
                         float* scales, const float* ub, int64_t rows, int64_t hidden, hipStream_t s) {
-  if (rows >= 1024 && hidden <= 5120)
-    return launch_quant_tpb<MODE, QT / 2>(in, in_dtype, in_stride, out, out_stride, scales, ub, rows, hidden, s);
-  return launch_quant_tpb<MODE, QT>(in, in_dtype, in_stride, out, out_stride, scales, ub, rows, hidden, s);
+  auto launch = [&](auto tpb, auto qv) {
+    return launch_quant_tpb<MODE, decltype(tpb)::value, decltype(qv)::value>(in, in_dtype, in_stride, out, out_stride, scales, ub,
+                                                                             rows, hidden, s);
+  };
+  const std::integral_constant<int, QT / 2> half;
+  const std::integral_constant<int, QT> full;
+  const std::integral_constant<int, 1> one;
+  const std::integral_constant<int, 4> four;
+  const std::integral_constant<int, 8> eight;
+  if (hidden <= QT / 2 * 8) return launch(half, one);
+  if (rows >= 1024 && hidden <= 5120) return launch(half, four);
+  if (hidden <= QT * 8) return launch(full, one);
+  return hidden <= QT * 4 * 8 ? launch(full, four) : launch(full, eight);
 }
 
 static int check_quant(const char* who, const void* in, int64_t in_stride, const uint8_t* out, int64_t out_stride,

@@ -56,34 +56,6 @@ __device__ inline float nq_mul_round16(float a, float b) {
   }
 }
 
-template <int TPB>
-__device__ inline float nq_block_sum(float v, float* smem) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (lane == 0) smem[wave] = v;
-  __syncthreads();
-  float r = smem[0];
-#pragma unroll
-  for (int i = 1; i < TPB / 64; ++i) r += smem[i];
-  __syncthreads();
-  return r;
-}
-
-template <int TPB>
-__device__ inline float nq_block_max(float v, float* smem) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (lane == 0) smem[wave] = v;
-  __syncthreads();
-  float r = smem[0];
-#pragma unroll
-  for (int i = 1; i < TPB / 64; ++i) r = fmaxf(r, smem[i]);
-  __syncthreads();
-  return r;
-}
-
 __device__ inline void nq_unpack8(v4u r, float* f, bool bf16) {
   const uint32_t w[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
@@ -172,8 +144,7 @@ __global__ __launch_bounds__(NQ_W) void rms_norm_fp8_row_per_wave_kernel(uint8_t
       for (int e = 0; e < 8; ++e) ss += x[v][e] * x[v][e];
     }
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
+  ss = wave_sum(ss);
   const float rms = rsqrtf(ss / (float)hidden + eps);
   float amax = 0.f;
 #pragma unroll
@@ -190,8 +161,7 @@ __global__ __launch_bounds__(NQ_W) void rms_norm_fp8_row_per_wave_kernel(uint8_t
     }
   }
   if constexpr (DYN) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    amax = wave_max(amax);
     if (scale_ub) amax = fminf(amax, *scale_ub);
     const float s = fmaxf(amax / NQ_FP8_MAX, 1.0f / (NQ_FP8_MAX * 512.0f));
     if (lane == 0) scales[tok] = s;
@@ -218,6 +188,12 @@ __global__ __launch_bounds__(NQ_W) void rms_norm_fp8_row_per_wave_kernel(uint8_t
   }
 }
 
+// Whether a thread requests all its chunks before it waits for the first (a wait inside each chunk's condition costs a latency per
+// chunk: few rows of 14336 without residual 4.4 -> 4.0 us, 4096 of them 39.1 -> 31.4 with a static scale) or takes them one after
+// another: with a residual and four chunks and more the chip's loads then come in a burst, ahead of all stores (4096 rows of 14336
+// with residual 65.4 us, all requested first 69.2).
+constexpr bool nq_ahead(bool has_res, int nv) { return !has_res || nv <= 2; }
+
 template <bool BF16, bool HAS_RES, int NV, int TPB>
 __global__ __launch_bounds__(TPB) void rms_norm_per_token_fp8_kernel(uint8_t* __restrict__ out, float* __restrict__ scales,
                                                                       const uint16_t* __restrict__ input,
@@ -226,7 +202,7 @@ __global__ __launch_bounds__(TPB) void rms_norm_per_token_fp8_kernel(uint8_t* __
                                                                       uint16_t* __restrict__ residual, int hidden,
                                                                       int64_t in_stride) {
   using T = F16Traits<BF16>;
-  __shared__ float smem[TPB / 64];
+  __shared__ float smem[2 * TPB / 64];
   const int64_t tok = blockIdx.x;
   const uint16_t* row = input + tok * in_stride;
   uint16_t* res = HAS_RES ? residual + tok * (int64_t)hidden : nullptr;
@@ -239,17 +215,30 @@ __global__ __launch_bounds__(TPB) void rms_norm_per_token_fp8_kernel(uint8_t* __
 
   if (cached) {
     float x[NV][8];
-    v4u wv[NV];          // the weight chunks, requested together with the row: no dependent load after the reduction
+    v4u xv[NV], rv[NV], wv[NV];      // row, residual and weight
+    constexpr bool AHEAD = nq_ahead(HAS_RES, NV);
     float ss = 0.f;
+    auto request = [&](int v) {
+      const int c = threadIdx.x + v * TPB;
+      if (c < chunks) {
+        xv[v] = *reinterpret_cast<const v4u*>(row + c * 8);
+        if constexpr (HAS_RES) rv[v] = *reinterpret_cast<const v4u*>(res + c * 8);
+        wv[v] = *reinterpret_cast<const v4u*>(weight + c * 8);
+      }
+    };
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) request(v);
+    }
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       const int c = threadIdx.x + v * TPB;
+      if constexpr (!AHEAD) request(v);
       if (c < chunks) {
-        wv[v] = *reinterpret_cast<const v4u*>(weight + c * 8);
-        nq_unpack8(*reinterpret_cast<const v4u*>(row + c * 8), x[v], BF16);
+        nq_unpack8(xv[v], x[v], BF16);
         if constexpr (HAS_RES) {
           float r[8];
-          nq_unpack8(*reinterpret_cast<const v4u*>(res + c * 8), r, BF16);
+          nq_unpack8(rv[v], r, BF16);
           v4u back;
           uint32_t* bw = reinterpret_cast<uint32_t*>(&back);
 #pragma unroll
@@ -263,7 +252,7 @@ __global__ __launch_bounds__(TPB) void rms_norm_per_token_fp8_kernel(uint8_t* __
         for (int e = 0; e < 8; ++e) ss += x[v][e] * x[v][e];
       }
     }
-    ss = nq_block_sum<TPB>(ss, smem);
+    ss = block_sum<TPB>(ss, smem);
     const float rms = rsqrtf(ss / (float)hidden + eps);
     float amax = 0.f;
 #pragma unroll
@@ -279,7 +268,7 @@ __global__ __launch_bounds__(TPB) void rms_norm_per_token_fp8_kernel(uint8_t* __
         }
       }
     }
-    amax = nq_block_max<TPB>(amax, smem);
+    amax = block_max<TPB>(amax, smem + TPB / 64);
     if (scale_ub) amax = fminf(amax, *scale_ub);
     const float s = fmaxf(amax / NQ_FP8_MAX, min_scale);
     if (threadIdx.x == 0) scales[tok] = s;
@@ -310,7 +299,7 @@ __global__ __launch_bounds__(TPB) void rms_norm_per_token_fp8_kernel(uint8_t* __
     }
     ss += x * x;
   }
-  ss = nq_block_sum<TPB>(ss, smem);
+  ss = block_sum<TPB>(ss, smem);
   const float rms = rsqrtf(ss / (float)hidden + eps);
   float amax = 0.f;
   for (int i = threadIdx.x; i < hidden; i += TPB) {
@@ -319,7 +308,7 @@ __global__ __launch_bounds__(TPB) void rms_norm_per_token_fp8_kernel(uint8_t* __
     const float y = nq_mul_round16<BF16>(nq_mul_round16<BF16>(x, rms), nq_to_float<BF16>(weight[i]));
     amax = fmaxf(amax, fabsf(y));
   }
-  amax = nq_block_max<TPB>(amax, smem);
+  amax = block_max<TPB>(amax, smem + TPB / 64);
   if (scale_ub) amax = fminf(amax, *scale_ub);
   const float s = fmaxf(amax / NQ_FP8_MAX, min_scale);
   if (threadIdx.x == 0) scales[tok] = s;
@@ -352,21 +341,35 @@ __global__ __launch_bounds__(TPB) void rms_norm_static_fp8_kernel(uint8_t* __res
   const bool cached = (hidden % 8 == 0) && chunks <= TPB * NV && (in_stride % 8 == 0) &&
                       ((reinterpret_cast<uintptr_t>(input) | reinterpret_cast<uintptr_t>(weight) |
                         reinterpret_cast<uintptr_t>(out) | (HAS_RES ? reinterpret_cast<uintptr_t>(residual) : 0)) % 16 == 0);
-  const float inv = 1.0f / *scale;
+
+  const float given = *scale;
 
   if (cached) {
     float x[NV][8];
-    v4u wv[NV];          // the weight chunks, requested together with the row
+    v4u xv[NV], rv[NV], wv[NV];      // row, residual and weight
+    constexpr bool AHEAD = nq_ahead(HAS_RES, NV);
     float ss = 0.f;
+    auto request = [&](int v) {
+      const int c = threadIdx.x + v * TPB;
+      if (c < chunks) {
+        xv[v] = *reinterpret_cast<const v4u*>(row + c * 8);
+        if constexpr (HAS_RES) rv[v] = *reinterpret_cast<const v4u*>(res + c * 8);
+        wv[v] = *reinterpret_cast<const v4u*>(weight + c * 8);
+      }
+    };
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) request(v);
+    }
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       const int c = threadIdx.x + v * TPB;
+      if constexpr (!AHEAD) request(v);
       if (c < chunks) {
-        wv[v] = *reinterpret_cast<const v4u*>(weight + c * 8);
-        nq_unpack8(*reinterpret_cast<const v4u*>(row + c * 8), x[v], BF16);
+        nq_unpack8(xv[v], x[v], BF16);
         if constexpr (HAS_RES) {
           float r[8];
-          nq_unpack8(*reinterpret_cast<const v4u*>(res + c * 8), r, BF16);
+          nq_unpack8(rv[v], r, BF16);
           v4u back;
           uint32_t* bw = reinterpret_cast<uint32_t*>(&back);
           uint16_t z[8];
@@ -383,7 +386,8 @@ __global__ __launch_bounds__(TPB) void rms_norm_static_fp8_kernel(uint8_t* __res
         for (int e = 0; e < 8; ++e) ss += x[v][e] * x[v][e];
       }
     }
-    ss = nq_block_sum<TPB>(ss, smem);
+    ss = block_sum<TPB>(ss, smem);
+    const float inv = 1.0f / given;
     const float rms = rsqrtf(ss / (float)hidden + eps);
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
@@ -422,7 +426,8 @@ __global__ __launch_bounds__(TPB) void rms_norm_static_fp8_kernel(uint8_t* __res
     }
     ss += x * x;
   }
-  ss = nq_block_sum<TPB>(ss, smem);  // its barrier also orders this workgroup's own writes to `res` before the re-reads
+  ss = block_sum<TPB>(ss, smem);      // (every thread re-reads what it has written to `res` itself)
+  const float inv = 1.0f / given;
   const float rms = rsqrtf(ss / (float)hidden + eps);
   for (int i = threadIdx.x; i < hidden; i += TPB) {
     const float x = nq_to_float<BF16>(HAS_RES ? res[i] : row[i]);
@@ -504,12 +509,15 @@ static bool nq_row_per_wave(const void* out, const void* in, const void* w, cons
   return can && (hidden <= 1024 ? tokens >= 1024 : tokens >= 2048);
 }
 
-// Rows of at most 4096 elements run on workgroups of 256 threads (two chunks of 8 elements per thread): twice the
-// workgroups per compute unit, each a dependent chain of load, reduction(s) and store of its own, and half the
-// wavefronts in every barrier.  4096 tokens of 4096: dynamic per-token 16.2 -> 13.6 us, with residual and a static scale
-// 20.0 -> 19.2 us, static scale 13.5 -> 13.5 us; longer rows are better off with 512 threads (8192: 22.0 against 24.0 us
-// static; 14336 with residual 65.7 against 70.5 us).
-static bool nq_half_workgroup(int64_t hidden) { return hidden <= (NQ_T / 2) * 8 * 2; }
+// Rows on workgroups of 256 threads (at most two chunks of 8 elements per thread) instead of 512: where many of them share a compute
+// unit, each is a dependent chain of load, reduction(s) and store of its own, with half the wavefronts in every barrier (4096 tokens
+// of 4096, dynamic 14.5 us against 16.2 with 512; 768 of 2048 3.5 against 3.9), and where one chunk per thread holds the row they
+// lose nothing.  Few rows of 4096 are a single chain, shorter with one chunk per thread (16 tokens with residual 3.01 against 3.10
+// us, static 2.50 against 2.73); at 512 tokens and more the first counts.  Longer rows are better off with 512 threads (4096 tokens
+// of 8192, static: 22.0 against 24.0 us; 14336 with residual 65.7 against 70.5).
+static bool nq_half_workgroup(int64_t tokens, int64_t hidden) {
+  return hidden <= (NQ_T / 2) * 8 || (tokens >= 512 && hidden <= (NQ_T / 2) * 8 * 2);
+}
 
 // run-time (dtype, residual, chunks per thread) -> compile-time template arguments
 template <typename F>
@@ -557,7 +565,7 @@ extern "C" int vaq_rms_norm_dynamic_per_token_fp8_quant(uint8_t* out, float* sca
     return VAQ_OK;
   }
   const int nv = hidden <= NQ_T * 8 * 2 ? 2 : (hidden <= NQ_T * 8 * 4 ? 4 : NQ_V_MAX);
-  const bool half_wg = nq_half_workgroup(hidden);
+  const bool half_wg = nq_half_workgroup(tokens, hidden);
   auto launch = [&](auto bf, auto rs, auto nvc) {
     if (half_wg)
       hipLaunchKernelGGL((rms_norm_per_token_fp8_kernel<decltype(bf)::value, decltype(rs)::value, 2, NQ_T / 2>), grid,
@@ -599,7 +607,7 @@ extern "C" int vaq_rms_norm_static_fp8_quant(uint8_t* out, const void* input, in
     return VAQ_OK;
   }
   const int nv = hidden <= NQ_T * 8 * 2 ? 2 : (hidden <= NQ_T * 8 * 4 ? 4 : NQ_V_MAX);
-  const bool half_wg = nq_half_workgroup(hidden);
+  const bool half_wg = nq_half_workgroup(tokens, hidden);
   auto launch = [&](auto bf, auto rs, auto nvc) {
     if (half_wg)
       hipLaunchKernelGGL((rms_norm_static_fp8_kernel<decltype(bf)::value, decltype(rs)::value, 2, NQ_T / 2>), grid, dim3(NQ_T / 2),

@@ -165,4 +165,48 @@ __device__ inline v4u dequant_biased(uint32_t w) {
   return r;
 }
 
+// op over the 64 lanes of a wavefront (all active), the result in every lane: halves, rows of 16 and rotations inside a row, all in
+// registers.  The pairs of a butterfly with distances 32, 16, 8, 4, 2, 1, so that a sum is the one that __shfl_xor gives; that goes
+// through LDS, six dependent round trips of 0.05 us.
+template <typename Op>
+__device__ inline float wave_reduce(float v, Op op) {
+  auto f = [](auto u) { return __builtin_bit_cast(float, u); };
+  auto u = [](float x) { return __builtin_bit_cast(uint32_t, x); };
+  const auto a = __builtin_amdgcn_permlane32_swap(u(v), u(v), false, false);
+  v = op(f((uint32_t)a[0]), f((uint32_t)a[1]));
+  const auto b = __builtin_amdgcn_permlane16_swap(u(v), u(v), false, false);
+  v = op(f((uint32_t)b[0]), f((uint32_t)b[1]));
+  v = op(v, f(__builtin_amdgcn_mov_dpp((int)u(v), 0x128, 0xf, 0xf, true)));      // row_ror:8
+  v = op(v, f(__builtin_amdgcn_mov_dpp((int)u(v), 0x124, 0xf, 0xf, true)));      // row_ror:4
+  v = op(v, f(__builtin_amdgcn_mov_dpp((int)u(v), 0x122, 0xf, 0xf, true)));      // row_ror:2
+  return op(v, f(__builtin_amdgcn_mov_dpp((int)u(v), 0x121, 0xf, 0xf, true)));   // row_ror:1
+}
+__device__ inline float wave_max(float v) {
+  return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
+}
+__device__ inline float wave_sum(float v) {
+  return wave_reduce(v, [](float a, float b) { return a + b; });
+}
+
+// The wavefronts' values of a workgroup of TPB threads through `smem` (TPB / 64 floats of this reduction's own: nothing protects
+// them against a second use), combined in their order.  The barrier waits for LDS only: a __syncthreads() also waits until the
+// stores before it are acknowledged, and those of a norm's residual take a microsecond.
+template <int TPB, typename Op>
+__device__ inline float block_combine(float v, float* smem, Op op) {
+  if ((threadIdx.x & 63) == 0) smem[threadIdx.x >> 6] = v;
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  float r = smem[0];
+#pragma unroll
+  for (int i = 1; i < TPB / 64; ++i) r = op(r, smem[i]);
+  return r;
+}
+template <int TPB>
+__device__ inline float block_max(float v, float* smem) {
+  return block_combine<TPB>(wave_max(v), smem, [](float a, float b) { return fmaxf(a, b); });
+}
+template <int TPB>
+__device__ inline float block_sum(float v, float* smem) {
+  return block_combine<TPB>(wave_sum(v), smem, [](float a, float b) { return a + b; });
+}
+
 }  // namespace vaq
