@@ -119,6 +119,25 @@ def test_repack_native_strips_and_their_limits(device, k, n, bits, act_order, of
         assert np.array_equal(got.cpu().numpy(), nl.native_pack8_bytes(q[perm_np]))
 
 
+@pytest.mark.parametrize("k,n,bits", [
+    (128, 64, 4), (6272, 1024, 4), (6144, 2048, 4), (6272, 2112, 4), (128, 4160, 8), (3200, 192, 8),      # 8-column strips, then 16 columns
+    (20608, 2112, 4), (40960, 64, 4), (41088, 64, 4), (10368, 2112, 8), (20480, 64, 8), (20608, 64, 8)])  # the two limits in K
+def test_repack_act_order_half_strips(device, k, n, bits):
+    """act_order strips of 8 and of 16 columns on both sides of each line of the choice between them (few strips; K beyond the
+    LDS of a whole strip, and of half of one), with rounds of pieces that do not fill the workgroup: words equal the layout's."""
+    import vllm_amd._custom_ops as ops
+    rng = np.random.default_rng(k + n + bits)
+    q = rng.integers(0, 1 << bits, size=(k, n), dtype=np.int32)
+    perm_np = rng.permutation(k).astype(np.int32)
+    perm = to_dev(perm_np, device)
+    qw = torch.from_numpy(np.ascontiguousarray(o.gptq_pack(q, bits))).to(device)
+    want = nl.native_pack(q[perm_np]) if bits == 4 else nl.native_pack8(q[perm_np])
+    assert np.array_equal(ops.gptq_marlin_repack(qw, perm, k, n, bits).cpu().numpy(), want)
+    if bits == 8:
+        got = ops.gptq_marlin_repack(qw, perm, k, n, 8, layout="native_bytes")
+        assert np.array_equal(got.cpu().numpy(), nl.native_pack8_bytes(q[perm_np]))
+
+
 # ------------------------------------------------------------------------------------------------ permute_cols
 
 @pytest.mark.parametrize("m,k", [(1, 128), (3, 1024), (7, 4096), (130, 14336), (5, 70000)])

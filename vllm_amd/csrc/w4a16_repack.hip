@@ -220,18 +220,18 @@ __global__ __launch_bounds__(256) void repack_marlin8_kernel(const uint32_t* __r
 
 // OUT 0: 4-bit codes; 1: 8-bit codes as two nibble planes; 2: 8-bit codes as bytes.
 template <int OUT>
-__device__ inline void put_code(v4u (&lo)[4], v4u (&hi)[4], int c, int j, int e, uint32_t word, int shift) {
+__device__ inline void put_code(v4u& lo, v4u& hi, int j, int e, uint32_t word, int shift) {
   constexpr int pos[8] = {0, 4, 1, 5, 2, 6, 3, 7};      // nibble position of element e
   if constexpr (OUT == 0) {
-    lo[c][j] |= ((word >> shift) & 0xFu) << (4 * pos[e]);
+    lo[j] |= ((word >> shift) & 0xFu) << (4 * pos[e]);
   } else if constexpr (OUT == 1) {
     const uint32_t b = word >> shift;
-    lo[c][j] |= ((b >> 4) & 0xFu) << (4 * pos[e]);      // plane 0: high nibbles
-    hi[c][j] |= (b & 0xFu) << (4 * pos[e]);
+    lo[j] |= ((b >> 4) & 0xFu) << (4 * pos[e]);      // plane 0: high nibbles
+    hi[j] |= (b & 0xFu) << (4 * pos[e]);
   } else {      // lane's 16 bytes of block h = j / 2: word 2 (j & 1) + e / 4, byte e % 4
     const uint32_t b = ((word >> shift) & 0xFFu) << (8 * (e & 3));
-    if (j < 2) lo[c][2 * (j & 1) + (e >> 2)] |= b;
-    else hi[c][2 * (j & 1) + (e >> 2)] |= b;
+    if (j < 2) lo[2 * (j & 1) + (e >> 2)] |= b;
+    else hi[2 * (j & 1) + (e >> 2)] |= b;
   }
 }
 
@@ -246,48 +246,59 @@ __device__ inline void store_tile(uint32_t* __restrict__ out, int64_t tile, int 
   }
 }
 
-// act_order: output row k takes input row perm[k], anywhere in K.  A workgroup holds one 16-column strip of the whole
-// checkpoint tensor in LDS (K / 8 rows of 64 bytes; 8-bit: K / 4) and gathers from there.  A thread builds the pieces of four
-// lanes (o, r = 4c + q for c = 0 .. 3), so that an index is looked up and turned into an address and a shift once for
-// four columns, which one 16-byte LDS read brings: the strip is kept column-transposed (position 4q + c holds column
-// 4c + q), and the four lanes q of one store are neighbours.  Strips that share a 128-byte line run on one XCD.
-// Measured, 4096 x 28672 (4 bits, 117 MB in and out): 129 -> 29 us = 4.1 TB/s; the random rows cost LDS bank conflicts, so that it
-// stays behind the 20 us of the kernel without a permutation.
-template <int OUT>
-__global__ __launch_bounds__(1024) void repack_native_perm_kernel(const uint32_t* __restrict__ qw, const int32_t* __restrict__ perm,
-                                                                  uint32_t* __restrict__ out, int size_k, int size_n, int strips_per_xcd) {
+constexpr int64_t REPACK_LDS_MAX = 160 * 1024;
+// act_order: output row k takes input row perm[k], anywhere in K.  A workgroup holds one strip of 4 C columns of the whole
+// checkpoint tensor in LDS (K / 8 rows of 16 C bytes; 8-bit: K / 4) and gathers from there.  A thread builds the pieces of C
+// lanes (o, r = 4c + q for c = 0 .. C - 1), so that an index is looked up and turned into an address and a shift once for
+// C columns, which one LDS read brings: the strip is kept column-transposed (position C q + c holds column
+// 4c + q), and the four lanes q of one store are neighbours.  Strips that share a 128-byte line run on one XCD.  A thread's
+// first 32 indexes are requested ahead of the barrier: their round trip is over when the strip has arrived.
+// Measured, us, indexes behind the barrier -> this: 4096 x 28672 (4 bits, 117 MB in and out) 29.6 -> 28.8 = 4.1 TB/s, 8192 x 8192
+// 20.2 -> 18.9, 4096 x 4096 7.6 -> 6.9; the random rows cost LDS bank conflicts, so that it stays behind the 20 us of the kernel
+// without a permutation.  Two, four or eight loads of the strip in flight per thread instead of one: 0 .. 10 % slower.
+template <int OUT, int C>
+__global__ __launch_bounds__(1024, 6) void repack_native_perm_kernel(const uint32_t* __restrict__ qw, const int32_t* __restrict__ perm,
+                                                                     uint32_t* __restrict__ out, int size_k, int size_n,
+                                                                     int strips_per_xcd) {
+  static_assert(C == 2 || C == 4, "half or whole tiles");
   extern __shared__ __attribute__((aligned(16))) uint32_t strip[];
-  const int nt = (int)(blockIdx.x & 7) * strips_per_xcd + (int)(blockIdx.x >> 3);
-  if (nt * 16 >= size_n) return;
+  typedef uint32_t Row __attribute__((ext_vector_type(C)));
+  const int st = (int)(blockIdx.x & 7) * strips_per_xcd + (int)(blockIdx.x >> 3);
+  if (st * 4 * C >= size_n) return;
   constexpr int LOG_ROWS = OUT == 0 ? 3 : 2;      // codes per word, log2
-  const int rows = size_k >> LOG_ROWS;
-  for (int i = threadIdx.x; i < rows * 4; i += blockDim.x) {
-    const int row = i >> 2, c = i & 3;
-    const v4u w = *reinterpret_cast<const v4u*>(qw + (int64_t)row * size_n + nt * 16 + 4 * c);
+  const int k_tiles = size_k >> 7, pieces = k_tiles * 16;
+  const v4i* order = reinterpret_cast<const v4i*>(perm);
+  v4i idx[8];
+  auto request = [&](int i) {      // the 32 indexes of piece i: rows 32 j + 8 o + e of its tile
 #pragma unroll
-    for (int q = 0; q < 4; ++q) strip[row * 16 + 4 * q + c] = w[q];
+    for (int j = 0; j < 8; ++j) idx[j] = order[(i >> 4) * 32 + (j >> 1) * 8 + ((i >> 2) & 3) * 2 + (j & 1)];
+  };
+  const int chunks = (size_k >> LOG_ROWS) * C;
+  for (int i = threadIdx.x; i < chunks; i += blockDim.x) {
+    const int row = i / C, c = i % C;
+    const v4u w = *reinterpret_cast<const v4u*>(qw + (int64_t)row * size_n + st * 4 * C + 4 * c);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) strip[row * 4 * C + C * q + c] = w[q];
   }
+  if ((int)threadIdx.x < pieces) request(threadIdx.x);
   __syncthreads();
-  const int k_tiles = size_k >> 7;
-  for (int i = threadIdx.x; i < k_tiles * 16; i += blockDim.x) {
+  for (int i = threadIdx.x; i < pieces; i += blockDim.x) {
     const int q = i & 3, o = (i >> 2) & 3, kt = i >> 4;
-    v4u lo[4] = {}, hi[4] = {};
+    v4u lo[C] = {}, hi[C] = {};
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const v4i* p = reinterpret_cast<const v4i*>(perm + kt * 128 + j * 32 + o * 8);
-      const v4i p0 = p[0], p1 = p[1];
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const int src = e < 4 ? p0[e & 3] : p1[e & 3];
-        const v4u w = *reinterpret_cast<const v4u*>(strip + (src >> LOG_ROWS) * 16 + 4 * q);
+        const int src = idx[2 * j + (e >> 2)][e & 3];
+        const Row w = *reinterpret_cast<const Row*>(strip + (src >> LOG_ROWS) * 4 * C + C * q);
         const int shift = (src & ((1 << LOG_ROWS) - 1)) * (32 >> LOG_ROWS);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) put_code<OUT>(lo, hi, c, j, e, w[c], shift);
+        for (int c = 0; c < C; ++c) put_code<OUT>(lo[c], hi[c], j, e, w[c], shift);
       }
-    }
-    const int64_t tile = (int64_t)nt * k_tiles + kt;
+    const int64_t tile = (int64_t)(st * C / 4) * k_tiles + kt;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) store_tile<OUT>(out, tile, 16 * o + 4 * c + q, lo[c], hi[c]);
+    for (int c = 0; c < C; ++c) store_tile<OUT>(out, tile, 16 * o + 4 * (st * C % 4 + c) + q, lo[c], hi[c]);
+    if (i + (int)blockDim.x < pieces) request(i + blockDim.x);
   }
 }
 
@@ -299,9 +310,7 @@ __global__ __launch_bounds__(256) void repack_native_rows_kernel(const uint32_t*
   const int lane = threadIdx.x & 63, o = lane >> 4, r = lane & 15;
   const int nt = blockIdx.x * 4 + (threadIdx.x >> 6), kt = blockIdx.y;
   const uint32_t* src = qw + nt * 16 + r;
-  v4u lo[1][4] = {}, hi[1][4] = {};
-  v4u (&l)[4] = lo[0];
-  v4u (&h)[4] = hi[0];
+  v4u lo = {}, hi = {};
   uint32_t w[4][OUT == 0 ? 1 : 2];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -317,8 +326,8 @@ __global__ __launch_bounds__(256) void repack_native_rows_kernel(const uint32_t*
   for (int j = 0; j < 4; ++j)
 #pragma unroll
     for (int e = 0; e < 8; ++e)
-      put_code<OUT>(l, h, 0, j, e, OUT == 0 ? w[j][0] : w[j][e >> 2], OUT == 0 ? 4 * e : 8 * (e & 3));
-  store_tile<OUT>(out, (int64_t)nt * (size_k >> 7) + kt, lane, l[0], h[0]);
+      put_code<OUT>(lo, hi, j, e, OUT == 0 ? w[j][0] : w[j][e >> 2], OUT == 0 ? 4 * e : 8 * (e & 3));
+  store_tile<OUT>(out, (int64_t)nt * (size_k >> 7) + kt, lane, lo, hi);
 }
 
 // AWQ: input rows are K, a word holds 8 columns of one row.  A workgroup takes 128 rows x 256 columns (whole 128-byte lines;
@@ -343,21 +352,35 @@ __global__ __launch_bounds__(256) void repack_native_awq_kernel(const uint32_t* 
   const int lane = threadIdx.x & 63, o = lane >> 4, r = lane & 15;
   const int shift = (((r & 1) << 2) | ((r & 7) >> 1)) * 4;
   for (int t = threadIdx.x >> 6; 2 * t < words; t += 4) {
-    v4u lo[4] = {}, hi[4] = {};
+    v4u lo = {}, hi = {};
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) put_code<0>(lo, hi, 0, j, e, tile_in[(j * 32 + o * 8 + e) * PITCH + t * 2 + (r >> 3)], shift);
-    store_tile<0>(out, (int64_t)(blockIdx.x * 16 + t) * (size_k >> 7) + kt, lane, lo[0], hi[0]);
+      for (int e = 0; e < 8; ++e) put_code<0>(lo, hi, j, e, tile_in[(j * 32 + o * 8 + e) * PITCH + t * 2 + (r >> 3)], shift);
+    store_tile<0>(out, (int64_t)(blockIdx.x * 16 + t) * (size_k >> 7) + kt, lane, lo, hi);
   }
 }
 
 // Whether the kernels above take a problem: 16-byte pointers, 32-bit indexes, and with act_order a strip that fits LDS.
-constexpr int64_t REPACK_LDS_MAX = 160 * 1024;
 static bool repack_tiles_ok(const void* qweight, const void* perm, const void* out, int64_t size_k, int64_t size_n, int num_bits) {
   if (((uintptr_t)qweight % 16) || ((uintptr_t)out % 16) || ((uintptr_t)perm % 16)) return false;
   if (size_k > (1 << 22) || size_n > (1 << 24)) return false;
-  return !perm || size_k * 2 * num_bits <= REPACK_LDS_MAX;
+  return !perm || size_k * num_bits <= REPACK_LDS_MAX;
+}
+
+template <int OUT, int C>
+static int launch_repack_perm(const uint32_t* qw, const int32_t* perm, uint32_t* out, int64_t size_k, int64_t size_n, hipStream_t s) {
+  const size_t lds = (size_t)size_k * C * (OUT == 0 ? 2 : 4);
+  static size_t reserved[VAQ_MAX_DEVICES];
+  const int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(&repack_native_perm_kernel<OUT, C>), lds, reserved, "w4a16_repack");
+  if (rc != VAQ_OK) return rc;
+  const int per_xcd = (int)((size_n / (4 * C) + 7) / 8);
+  // 12 wavefronts: 8 are up to 12 % slower where a compute unit holds one strip (8 bits 8192 x 8192 39.6 against 34.5 us), 16 up to 6 %
+  // where it holds two (4096 x 28672 29.8 against 28.2); a single whole strip of 4 bits is the exception (14336 x 4096 17.6 -> 17.2)
+  const int threads = OUT == 0 && C == 4 && lds > REPACK_LDS_MAX / 2 ? 1024 : 768;
+  hipLaunchKernelGGL((repack_native_perm_kernel<OUT, C>), dim3(per_xcd * 8), dim3(threads), lds, s, qw, perm, out, (int)size_k, (int)size_n,
+                     per_xcd);
+  return VAQ_OK;
 }
 
 template <int OUT>
@@ -367,15 +390,12 @@ static int launch_repack_tiles(const uint32_t* qw, const int32_t* perm, uint32_t
                        (int)size_k, (int)size_n);
     return VAQ_OK;
   }
-  const size_t lds = (size_t)size_k * (OUT == 0 ? 8 : 16);
-  static size_t reserved[VAQ_MAX_DEVICES];
-  const int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(&repack_native_perm_kernel<OUT>), lds, reserved, "w4a16_repack");
-  if (rc != VAQ_OK) return rc;
-  const int per_xcd = (int)((size_n / 16 + 7) / 8);
-  // one strip per compute unit where two do not fit: then as many wavefronts as it holds
-  const int threads = lds > REPACK_LDS_MAX / 2 ? 1024 : 512;
-  hipLaunchKernelGGL(repack_native_perm_kernel<OUT>, dim3(per_xcd * 8), dim3(threads), lds, s, qw, perm, out, (int)size_k, (int)size_n, per_xcd);
-  return VAQ_OK;
+  // Strips of 16 columns read and write whole 64-byte pieces and look an index up once for four columns.  Strips of 8 take K up to
+  // twice as far (one word per thread beyond: 8 bits 14336 x 4096 137 -> 40 us, 4 bits 24576 x 2048 58 -> 21), and
+  // give every compute unit one where 16 columns leave half of them idle (5120 x 1024 6.0 -> 4.8 us); with as many strips as
+  // compute units they are the slower ones (4096 x 4096 6.9 against 8.0 us).
+  const bool half = size_k * (OUT == 0 ? 8 : 16) > REPACK_LDS_MAX || size_n / 8 <= num_cus_current_device();
+  return half ? launch_repack_perm<OUT, 2>(qw, perm, out, size_k, size_n, s) : launch_repack_perm<OUT, 4>(qw, perm, out, size_k, size_n, s);
 }
 
 }  // namespace vaq
