@@ -46,3 +46,19 @@ def test_long_rows_bit_exact(device, hidden, dtype):
     assert _same(ops.scaled_fp8_quant(x.to(device)), f.ref_dynamic_per_tensor_quant(x))
     scale = torch.tensor([0.01])
     assert _same(ops.scaled_fp8_quant(x.to(device), scale.to(device))[:1], [f.ref_static_quant(x, scale)])
+
+
+@pytest.mark.parametrize("tokens,d", [(1, 8), (3, 24), (517, 1000), (292, 14336), (293, 14336), (2341, 14336)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_silu_chunks_equal_single_elements(device, tokens, d, dtype):
+    """Chunks of 8 against the element-wise kernel of the same arithmetic (an output that is not 8-byte aligned): one chunk, a last
+    workgroup in part, both workgroup sizes beside the line between them, and a thread's second chunk."""
+    import vllm_amd._custom_ops as ops
+    x = torch.randn(tokens, 2 * d, device=device, dtype=dtype, generator=torch.Generator(device=device).manual_seed(d))
+    scale = torch.full((1,), 4 / 448, device=device)
+    buf = torch.zeros(tokens * d + 8, dtype=torch.uint8, device=device)
+    odd = buf[1:1 + tokens * d].view(ops.FP8_DTYPE).view(tokens, d)
+    out = torch.empty(tokens, d, dtype=ops.FP8_DTYPE, device=device)
+    ops.silu_and_mul_quant(odd, x, scale)
+    ops.silu_and_mul_quant(out, x, scale)
+    assert torch.equal(out.view(torch.uint8), odd.view(torch.uint8))
