@@ -62,3 +62,24 @@ def test_silu_chunks_equal_single_elements(device, tokens, d, dtype):
     ops.silu_and_mul_quant(odd, x, scale)
     ops.silu_and_mul_quant(out, x, scale)
     assert torch.equal(out.view(torch.uint8), odd.view(torch.uint8))
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (1, 7), (3, 8), (1, 2047), (5, 411), (333, 3001), (2, 1050633), (1, 33554441)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_per_tensor_runs_equal_rows(device, shape, dtype):
+    """Rows without gaps go as one run of vectors: single elements, remainders behind the last vector, one and several rounds of the
+    grid.  The same rows behind a gap take a workgroup each: codes and scales are the same bits, the first shapes the oracle's too;
+    the largest magnitude is the last element."""
+    import vllm_amd._custom_ops as ops
+    rows, hidden = shape
+    x = torch.randn(rows, hidden, device=device, generator=torch.Generator(device=device).manual_seed(hidden)).to(dtype)
+    x[-1, -1] = -21.5
+    gap = torch.zeros(rows + 1, hidden + 8, dtype=dtype, device=device)[:rows, 8:]
+    gap.copy_(x)
+    scale = torch.full((1,), 0.01, device=device)
+    for given in (scale, None):
+        got, want = (ops.scaled_fp8_quant(v, given) for v in (x, gap))
+        assert torch.equal(got[0].view(torch.uint8), want[0].view(torch.uint8)) and torch.equal(got[1], want[1])
+        if x.numel() < 1 << 20:
+            ref = f.ref_static_quant(x.cpu(), scale.cpu()) if given is not None else f.ref_dynamic_per_tensor_quant(x.cpu())
+            assert _same(got[:1], [ref[0] if isinstance(ref, tuple) else ref])
