@@ -654,3 +654,59 @@ def test_rows_over_workgroups_keep_copies_of_a_stream_on_one_xcd():
                     (98, 5632, 512)):
         assert lib.vaq_w4a16_decode_plan(m, n, k, 1, 0, 2, plan) == _lib.VAQ_OK and plan[5] > 0
         assert -(-n // 16 // int(plan[2])) % 2 == 0, (m, n, k, list(plan))
+
+
+def _workspace_query(m, n, k, tuning=None):
+    import ctypes
+    from vllm_amd import _lib
+    sizes = [ctypes.c_size_t() for _ in range(3)]
+    assert _lib.load().vaq_w4a16_gemm_workspace_tuned(m, n, k, 0, 0, *map(ctypes.byref, sizes),
+                                                      None if tuning is None else ctypes.byref(tuning)) == _lib.VAQ_OK
+    return tuple(s.value for s in sizes)
+
+
+def _library_scratch(kib):
+    """What `vaq_w4a16_gemm_static` passes down: no split of the last round only, partial tiles of at most `kib` KiB."""
+    from vllm_amd import _lib
+    t = _lib.VaqTuning()
+    t.exp[10], t.exp[14] = 1, kib
+    return t
+
+
+@pytest.mark.parametrize("m", [32, 64, 200])
+def test_calls_on_library_owned_scratch_find_their_plans(m):
+    """The calls of `vaq_w4a16_gemm_static` read finished plans like every other call (weighing those of all formats again took
+    three times as long as the query itself).  The best of many short runs of either, so that a busy machine does not decide."""
+    import time
+    scratch = _library_scratch(16384)
+
+    def best(tuning):
+        shortest = float("inf")
+        for _ in range(40):
+            start = time.perf_counter()
+            for _ in range(50):
+                _workspace_query(m, 4096, 4096, tuning)
+            shortest = min(shortest, time.perf_counter() - start)
+        return shortest
+    plain, library = best(None), best(scratch)
+    assert library < 1.35 * plain, f"{library / plain:.2f} times the time of a plain query"
+
+
+def test_finished_plans_keep_what_they_were_made_for_apart():
+    """Queries that differ only in the room for partial tiles, in turn on one thread, against the answers on threads of their
+    own (the table of finished plans is per thread); a forced split is neither kept nor answered from the table."""
+    import threading
+    from vllm_amd import _lib
+    forced = _lib.VaqTuning()
+    forced.prefill_split = 2
+    kinds = [None, _library_scratch(16384), _library_scratch(1), _library_scratch(40000), forced]
+    for m, n, k in ((512, 6144, 24576), (128, 1536, 8192), (4096, 6144, 4096), (40, 2048, 14336), (24, 4096, 4096)):
+        alone = []
+        for tuning in kinds:
+            t = threading.Thread(target=lambda: alone.append(_workspace_query(m, n, k, tuning)))
+            t.start()
+            t.join()
+        for _ in range(3):
+            assert [_workspace_query(m, n, k, tuning) for tuning in kinds] == alone, (m, n, k)
+        if m >= 512:
+            assert alone[0][0] > alone[1][0] >= alone[2][0], (m, n, k)

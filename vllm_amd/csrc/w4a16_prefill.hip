@@ -143,15 +143,20 @@ static TilePlan make_plan_prefill(int M, int N, int K, TileFormat format) {
 }
 
 static TilePlan plan_prefill(int M, int N, int K, bool direct_ok, TileFormat format) {
-  const int forced = tuning().prefill_tile - 1;
+  const VaqTuning& tn = tuning();
+  const int forced = tn.prefill_tile - 1;
   if (!direct_ok || (forced >= 0 && forced < 10)) {
     TilePlan pl;
     pl.id = forced >= 0 ? forced : pick_register_staged(M, N);
     return pl;
   }
+  // The entry point on library-owned scratch sets exp[10] and exp[14] on every call: they are part of the key, so that its calls find
+  // their plans too (six to ten of them a call at 17 .. 256 rows, 0.5 - 1 us each to make).
+  constexpr int KIB_MAX = 1 << 15;
   static thread_local TilePlanTable table;
-  if (tuning_active()) return make_plan_prefill(M, N, K, format);
-  return table.get(M, N, K, num_cus_current_device() * 8 + format, [&] { return make_plan_prefill(M, N, K, format); });
+  if (forced >= 0 || tn.prefill_split > 0 || tn.exp[6] > 1 || tn.exp[14] < 0 || tn.exp[14] >= KIB_MAX) return make_plan_prefill(M, N, K, format);
+  const int key = ((num_cus_current_device() * 8 + format) * 2 + (tn.exp[10] == 1 ? 1 : 0)) * KIB_MAX + tn.exp[14];
+  return table.get(M, N, K, key, [&] { return make_plan_prefill(M, N, K, format); });
 }
 
 // Predicted time of the tile kernel whose weights pass through LDS (negative: not known, register-staged tiles): what the decode
