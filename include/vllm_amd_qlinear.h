@@ -95,6 +95,15 @@ int vaq_w4a16_gemm_workspace(int64_t size_m, int64_t size_n, int64_t size_k, int
                              size_t* c_tmp_bytes, size_t* a_tmp_bytes, size_t* counter_ints);
 
 /*
+ * The same for one weight format (`group_size` and `wtype` as in vaq_w4a16_gemm): what its own kernels need, where the
+ * query above covers every format's -- tens of MB more at hundreds to thousands of rows, and five plans instead of two to
+ * weigh for a new problem.
+ */
+int vaq_w4a16_gemm_workspace_of_format(int64_t size_m, int64_t size_n, int64_t size_k, int group_size, int wtype,
+                                       int has_perm, int device, size_t* c_tmp_bytes, size_t* a_tmp_bytes,
+                                       size_t* counter_ints);
+
+/*
  * W4A16 GEMM  C[M,N] = A[:, perm] . dequant(B) (+ bias), fp32 accumulation, one rounding to the 16-bit dtype.
  * Replaces `gptq_marlin_gemm(...)` (csrc/torch_bindings.cpp:309-315; csrc/quantization/gptq_marlin/gptq_marlin.cu:674-959).
  *   a        [M, K] 16-bit, row stride lda elements (lda % 8 == 0, base 16-byte aligned), unit column stride
@@ -112,7 +121,8 @@ int vaq_w4a16_gemm_workspace(int64_t size_m, int64_t size_n, int64_t size_k, int
  * weights dequantised through LDS or in registers.  `force_path` = 0 auto, 1 decode (M <= 64 at most), 2 prefill (tests /
  * benchmarks).
  * Scratch: `c_tmp` holds at least `c_tmp_bytes` bytes and `counters` at least `counter_ints` zeroed ints; a call whose
- * kernel needs more than it was given returns VAQ_ERR_INVALID_ARG (sizes: vaq_w4a16_gemm_workspace) and launches nothing.
+ * kernel needs more than it was given returns VAQ_ERR_INVALID_ARG (sizes: vaq_w4a16_gemm_workspace, or
+ * vaq_w4a16_gemm_workspace_of_format) and launches nothing.
  * One use of `c_tmp` is optional: at thousands of rows, 256 x 256 tiles that end in a round of workgroups at most half
  * full run the tiles of that round in K parts when `c_tmp` holds their partial tiles, and whole (same result, slower)
  * when it does not -- the workspace query reports the size with that use included.

@@ -46,6 +46,21 @@ def test_w4_layer_equals_the_registered_op(device, shape, group, dtype, bias):
     assert direct is not None, "a plain call went through the dispatcher"
 
 
+def test_w4_scratch_is_that_of_the_layers_own_format(device):
+    """Two formats of one shape in turn, of which one needs scratch for its K split and the other none: neither takes the other's
+    size from the caches of either route, and the second allocates its output only."""
+    plain, grouped = _w4(device, 2048, 512, 128, torch.bfloat16, False), _w4(device, 2048, 512, 32, torch.bfloat16, False)
+    x = torch.randn(40, 2048, device=device).to(torch.bfloat16)
+    for _ in range(2):
+        for layer in (grouped, plain):
+            assert torch.equal(layer(x), _registered(layer, x))
+    for call in (lambda: grouped(x), lambda: _registered(grouped, x)):
+        torch.cuda.reset_peak_memory_stats(device)
+        before = torch.cuda.memory_allocated(device)
+        out = call()
+        assert torch.cuda.max_memory_allocated(device) - before == out.numel() * 2
+
+
 @pytest.mark.parametrize("shape", [(1, 256), (67, 256), (2, 5, 256)])
 @pytest.mark.parametrize("static", [False, True])
 @pytest.mark.parametrize("bias", [False, True])

@@ -710,3 +710,35 @@ def test_finished_plans_keep_what_they_were_made_for_apart():
             assert [_workspace_query(m, n, k, tuning) for tuning in kinds] == alone, (m, n, k)
         if m >= 512:
             assert alone[0][0] > alone[1][0] >= alone[2][0], (m, n, k)
+
+
+def test_scratch_of_one_weight_format():
+    """The query of one format asks for what its own plans need, the one without a format for the largest of them: a 4-bit layer
+    whose plan leaves K whole takes no partial tiles because FP8 weights of the same shape would."""
+    import ctypes
+    from vllm_amd import _lib
+    lib = _lib.load()
+
+    def of_format(m, n, k, group, wtype, perm=0):
+        sizes = [ctypes.c_size_t() for _ in range(3)]
+        rc = lib.vaq_w4a16_gemm_workspace_of_format(m, n, k, group, wtype, perm, 0, *map(ctypes.byref, sizes))
+        return rc, tuple(s.value for s in sizes)
+    formats = [(g, w) for w in (_lib.VAQ_WTYPE_U4B8, _lib.VAQ_WTYPE_U4, _lib.VAQ_WTYPE_U8B128) for g in (-1, 128, 64, 32)]
+    formats += [(128, _lib.VAQ_WTYPE_FE4M3), (-1, _lib.VAQ_WTYPE_FE4M3)]
+    less = 0
+    for n, k in ((4096, 4096), (6144, 4096), (28672, 4096), (4096, 14336), (128256, 4096), (64, 128), (1024, 5120)):
+        for m in (0, 1, 5, 16, 17, 32, 33, 48, 64, 65, 100, 333, 1024, 4096):
+            single = []
+            for g, w in formats:
+                rc, sizes = of_format(m, n, k, g, w)
+                assert rc == _lib.VAQ_OK, (m, n, k, g, w)
+                single.append(sizes)
+            every = _workspace_query(m, n, k)
+            assert tuple(max(s[i] for s in single) for i in range(3)) == every, (m, n, k)
+            less += any(s[0] < every[0] for s in single)
+            assert of_format(m, n, k, 128, _lib.VAQ_WTYPE_U4B8, 1)[1][1] == (2 * m * k if m > 32 else 0)
+    assert less > 20
+    assert of_format(333, 6144, 4096, 128, _lib.VAQ_WTYPE_U4)[1] == (0, 0, 0) and _workspace_query(333, 6144, 4096)[0] > 10 << 20
+    assert of_format(8, 64, 256, 16, _lib.VAQ_WTYPE_U4B8)[0] == _lib.VAQ_ERR_UNSUPPORTED
+    assert of_format(8, 64, 256, 128, 9)[0] == _lib.VAQ_ERR_INVALID_ARG
+    assert of_format(8, 100, 256, 128, _lib.VAQ_WTYPE_U4)[0] == _lib.VAQ_ERR_INVALID_ARG

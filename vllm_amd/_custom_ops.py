@@ -357,17 +357,16 @@ def _gemm_impl(a: torch.Tensor, c_or_none: torch.Tensor | None, b_q_weight: torc
         # graph capture), arrival counters from the caller's `workspace`.  The library checks what it is handed against
         # what the kernel it picks needs and reports a workspace that is too small (gptq_marlin.cu:899-902).
         tune = _tuning.current_ref()
-        key = (size_m, size_n, size_k, has_act_order, dev.index or 0)
+        key = (size_m, size_n, size_k, group_size, wtype, has_act_order, dev.index or 0)
         sizes = _W4_WORKSPACE_SIZES.get(key) if tune is None else None
         if sizes is None:
             n_ctmp, n_atmp, n_cnt = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_size_t()
-            q_args = (size_m, size_n, size_k, int(has_act_order), dev.index or 0, ctypes.byref(n_ctmp),
-                      ctypes.byref(n_atmp), ctypes.byref(n_cnt))
-            _lib.check(lib.vaq_w4a16_gemm_workspace(*q_args) if tune is None
-                       else lib.vaq_w4a16_gemm_workspace_tuned(*q_args, tune))
+            out = (int(has_act_order), dev.index or 0, ctypes.byref(n_ctmp), ctypes.byref(n_atmp), ctypes.byref(n_cnt))
+            _lib.check(lib.vaq_w4a16_gemm_workspace_of_format(size_m, size_n, size_k, group_size, wtype, *out) if tune is None
+                       else lib.vaq_w4a16_gemm_workspace_tuned(size_m, size_n, size_k, *out, tune))
             sizes = (n_ctmp.value, n_atmp.value)
             if tune is None and len(_W4_WORKSPACE_SIZES) < 4096:
-                _W4_WORKSPACE_SIZES[key] = sizes      # (the library's answer depends on the shape and the device only)
+                _W4_WORKSPACE_SIZES[key] = sizes      # (the library's answer depends on shape, format and device only)
         ctmp_bytes, atmp_bytes = sizes
         c_tmp = torch.empty((ctmp_bytes // 4,), dtype=torch.float32, device=dev) if ctmp_bytes else None
         a_tmp = torch.empty((atmp_bytes // 2,), dtype=a.dtype, device=dev) if atmp_bytes else None

@@ -29,6 +29,8 @@ _SIGNATURES = {
     "vaq_w4a16_repack_awq": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int, c_int, c_void_p]),
     "vaq_w4a16_gemm_workspace": (c_int, [c_int64, c_int64, c_int64, c_int, c_int, POINTER(c_size_t), POINTER(c_size_t),
                                          POINTER(c_size_t)]),
+    "vaq_w4a16_gemm_workspace_of_format": (c_int, [c_int64, c_int64, c_int64, c_int, c_int, c_int, c_int, POINTER(c_size_t),
+                                                   POINTER(c_size_t), POINTER(c_size_t)]),
     "vaq_w4a16_gemm": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                c_int64, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int, c_int, c_int,
                                c_int, c_void_p]),

@@ -118,7 +118,7 @@ PyObject* raise_status(int rc) {
   return nullptr;
 }
 
-// Scratch sizes of recent problems: the library's answer depends on the shape and the device only, and planning a
+// Scratch sizes of recent problems: the library's answer depends on shape, format and device only, and planning a
 // problem twice per call costs as much as the checks.  Direct mapped, one cache per thread.
 struct Sizes {
   int64_t m = -1, n = 0, k = 0;
@@ -127,7 +127,7 @@ struct Sizes {
 };
 constexpr int SIZE_SLOTS = 512;
 Sizes& size_slot(Sizes (&cache)[SIZE_SLOTS], int64_t m, int64_t n, int64_t k, int flags) {
-  const uint64_t h = ((uint64_t)m * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)n * 0xc2b2ae3d27d4eb4full) ^ ((uint64_t)k * 0x165667b19e3779f9ull) ^ (uint64_t)flags;
+  const uint64_t h = ((uint64_t)m * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)n * 0xc2b2ae3d27d4eb4full) ^ ((uint64_t)k * 0x165667b19e3779f9ull) ^ ((uint64_t)flags * 0xd6e8feb86659fd93ull);
   return cache[(h >> 40) & (SIZE_SLOTS - 1)];
 }
 
@@ -175,11 +175,11 @@ int w4_gemm(const Call& call, const W4Call& q, int64_t lda, TensorBase& out) {
   const int wtype = q.type == g_fe4m3 ? VAQ_WTYPE_FE4M3 : q.type == g_u8b128 ? VAQ_WTYPE_U8B128 : zp ? VAQ_WTYPE_U4 : VAQ_WTYPE_U4B8;
 
   static thread_local Sizes cache[SIZE_SLOTS];
-  const int flags = call.device * 2 + (act_order ? 1 : 0);
+  const int flags = ((call.device * 2 + (act_order ? 1 : 0)) * 4 + wtype) * 8 + (group_size == -1 ? 0 : (int)group_size / 32);
   Sizes& z = size_slot(cache, m, n, k, flags);
   if (z.m != m || z.n != n || z.k != k || z.flags != flags) {
     size_t counters = 0;
-    const int rc = vaq_w4a16_gemm_workspace(m, n, k, act_order, call.device, &z.c_tmp, &z.extra, &counters);
+    const int rc = vaq_w4a16_gemm_workspace_of_format(m, n, k, (int)group_size, wtype, act_order, call.device, &z.c_tmp, &z.extra, &counters);
     z.m = -1;
     if (rc != VAQ_OK) return 0;
     z.m = m; z.n = n; z.k = k; z.flags = flags;

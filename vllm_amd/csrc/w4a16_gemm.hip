@@ -32,7 +32,72 @@ static int check_shape(int64_t size_m, int64_t size_n, int64_t size_k) {
                 "w4a16_gemm: problem too large");   // (8-bit weights: K*N bytes, still below 2^33; offsets are checked per kernel)
   return VAQ_OK;
 }
+
+// Weight type tag and group size -> 4-bit (0), 8-bit (1) or FP8 (2) weights, groups per 128 rows, channelwise scales or not.
+static int check_format(int64_t size_k, int group_size, int wtype, int* wt, int* sub, bool* channelwise) {
+  VAQ_CHECK_ARG(wtype == VAQ_WTYPE_U4B8 || wtype == VAQ_WTYPE_U4 || wtype == VAQ_WTYPE_U8B128 || wtype == VAQ_WTYPE_FE4M3,
+                "w4a16_gemm: unknown weight type tag %d", wtype);
+  *wt = wtype == VAQ_WTYPE_U8B128 ? 1 : (wtype == VAQ_WTYPE_FE4M3 ? 2 : 0);
+  *channelwise = group_size == -1 || (group_size == size_k && size_k != 128);
+  VAQ_CHECK_SUPPORTED(*channelwise || group_size == 128 || group_size == 64 || group_size == 32,
+                      "w4a16_gemm: group_size = %d is not built (only -1, 32, 64, 128)", group_size);
+  *sub = *channelwise ? 1 : 128 / group_size;
+  return VAQ_OK;
+}
+
+// Scratch of a problem, enough for whichever kernel runs (that also depends on the row stride of A): for one weight format, or with
+// wt < 0 for any of them.
+static int scratch_of(int64_t size_m, int64_t size_n, int64_t size_k, bool has_perm, int wt, int sub, size_t* c_tmp_bytes,
+                      size_t* a_tmp_bytes, size_t* counter_ints) {
+  VAQ_CHECK_ARG(c_tmp_bytes && a_tmp_bytes && counter_ints, "w4a16_gemm_workspace: null output pointer");
+  int rc = check_shape(size_m, size_n, size_k);
+  if (rc != VAQ_OK) return rc;
+  *c_tmp_bytes = 0;
+  *a_tmp_bytes = 0;
+  *counter_ints = 0;
+  const int M = (int)size_m, N = (int)size_n, K = (int)size_k;
+  auto take = [&](size_t t, size_t n) {
+    if (t > *c_tmp_bytes) *c_tmp_bytes = t;
+    if (n > *counter_ints) *counter_ints = n;
+  };
+  size_t t = 0, n = 0;
+  for (int s : {1, 2, 4})
+    for (bool w8 : {false, true}) {
+      const bool plain = s == 1 && !w8;
+      if (size_m > (plain ? DECODE_MAX_M : DECODE_MAX_M_2BLK) || size_m == 0 || (wt >= 0 && (s != sub || w8 != (wt != 0)))) continue;
+      rc = w4a16_decode2_workspace(M, N, K, s, w8, &t, &n);
+      if (rc != VAQ_OK) return rc;
+      take(t, n);
+      if (!plain || size_m > DECODE_MAX_M_2BLK) continue;
+      rc = w4a16_decode_workspace(M, N, K, &t, &n);
+      if (rc != VAQ_OK) return rc;
+      take(t, n);
+    }
+  // from 17 rows on the tile kernel where it is ahead
+  if (size_m > 16)
+    for (TileFormat format : {TILES_PLAIN, TILES_SUB, TILES_8BIT, TILES_FP8}) {
+      if (wt >= 0 && format != tile_format(sub, wt)) continue;
+      rc = w4a16_prefill_workspace(M, N, K, format, &t, &n);
+      if (rc != VAQ_OK) return rc;
+      take(t, n);
+    }
+  if (has_perm && size_m > DECODE_MAX_M_2BLK) *a_tmp_bytes = (size_t)size_m * (size_t)size_k * 2;
+  return VAQ_OK;
+}
 }  // namespace vaq
+
+extern "C" int vaq_w4a16_gemm_workspace_of_format(int64_t size_m, int64_t size_n, int64_t size_k, int group_size, int wtype,
+                                                  int has_perm, int device, size_t* c_tmp_bytes, size_t* a_tmp_bytes,
+                                                  size_t* counter_ints) {
+  using namespace vaq;
+  (void)device;
+  int wt = 0, sub = 1;
+  bool channelwise = false;
+  int rc = check_shape(size_m, size_n, size_k);
+  if (rc == VAQ_OK) rc = check_format(size_k, group_size, wtype, &wt, &sub, &channelwise);
+  if (rc != VAQ_OK) return rc;
+  return scratch_of(size_m, size_n, size_k, has_perm != 0, wt, sub, c_tmp_bytes, a_tmp_bytes, counter_ints);
+}
 
 extern "C" int vaq_w4a16_gemm_workspace(int64_t size_m, int64_t size_n, int64_t size_k, int has_perm, int device,
                                         size_t* c_tmp_bytes, size_t* a_tmp_bytes, size_t* counter_ints) {
@@ -46,50 +111,7 @@ extern "C" int vaq_w4a16_gemm_workspace_tuned(int64_t size_m, int64_t size_n, in
   using namespace vaq;
   (void)device;
   const TuningScope scope(tuning_or_null);
-  VAQ_CHECK_ARG(c_tmp_bytes && a_tmp_bytes && counter_ints, "w4a16_gemm_workspace: null output pointer");
-  int rc = check_shape(size_m, size_n, size_k);
-  if (rc != VAQ_OK) return rc;
-  *c_tmp_bytes = 0;
-  *a_tmp_bytes = 0;
-  *counter_ints = 0;
-  if (size_m == 0) return VAQ_OK;
-  if (size_m <= DECODE_MAX_M) {
-    // Enough for whichever kernel runs: that also depends on the row stride of A, the group size and the weight type,
-    // all unknown here.
-    size_t t = 0, n = 0, t2 = 0, n2 = 0;
-    auto take = [&]() {
-      if (t2 > t) t = t2;
-      if (n2 > n) n = n2;
-    };
-    rc = w4a16_decode2_workspace((int)size_m, (int)size_n, (int)size_k, 1, false, &t2, &n2);
-    if (rc != VAQ_OK) return rc;
-    take();
-    if (size_m <= DECODE_MAX_M_2BLK) {
-      rc = w4a16_decode_workspace((int)size_m, (int)size_n, (int)size_k, &t2, &n2);
-      if (rc != VAQ_OK) return rc;
-      take();
-      for (int sub : {1, 2, 4}) {                              // groups below 128 rows, 8-bit codes
-        for (bool w8 : {false, true}) {
-          if (sub == 1 && !w8) continue;
-          rc = w4a16_decode2_workspace((int)size_m, (int)size_n, (int)size_k, sub, w8, &t2, &n2);
-          if (rc != VAQ_OK) return rc;
-          take();
-        }
-      }
-    }
-    if (size_m > 16) {
-      // those cases take the tile kernel where it is ahead, above 32 rows always or the rows split over workgroups
-      rc = w4a16_prefill_workspace((int)size_m, (int)size_n, (int)size_k, &t2, &n2);
-      if (rc != VAQ_OK) return rc;
-      take();
-      if (has_perm && size_m > DECODE_MAX_M_2BLK) *a_tmp_bytes = (size_t)size_m * (size_t)size_k * 2;
-    }
-    *c_tmp_bytes = t;
-    *counter_ints = n;
-    return VAQ_OK;
-  }
-  if (has_perm) *a_tmp_bytes = (size_t)size_m * (size_t)size_k * 2;
-  return w4a16_prefill_workspace((int)size_m, (int)size_n, (int)size_k, c_tmp_bytes, counter_ints);
+  return scratch_of(size_m, size_n, size_k, has_perm != 0, -1, 0, c_tmp_bytes, a_tmp_bytes, counter_ints);
 }
 
 extern "C" int vaq_w4a16_gemm(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
@@ -112,16 +134,13 @@ extern "C" int vaq_w4a16_gemm_tuned(const void* a, int64_t lda, const int32_t* b
   if (rc != VAQ_OK) return rc;
   VAQ_CHECK_ARG(dtype == VAQ_F16 || dtype == VAQ_BF16, "w4a16_gemm: only supports bfloat16 and float16 (dtype tag %d)",
                 dtype);
-  VAQ_CHECK_ARG(wtype == VAQ_WTYPE_U4B8 || wtype == VAQ_WTYPE_U4 || wtype == VAQ_WTYPE_U8B128 || wtype == VAQ_WTYPE_FE4M3,
-                "w4a16_gemm: unknown weight type tag %d", wtype);
+  int wt = 0, sub = 1;
+  bool channelwise = false;
+  rc = check_format(size_k, group_size, wtype, &wt, &sub, &channelwise);
+  if (rc != VAQ_OK) return rc;
   VAQ_CHECK_ARG((wtype == VAQ_WTYPE_U4) == (zeros != nullptr),
                 "w4a16_gemm: b_q_type must be uint4 when has_zp = True and uint4b8, uint8b128 or float8_e4m3fn when has_zp = False");
-  const int wt = wtype == VAQ_WTYPE_U8B128 ? 1 : (wtype == VAQ_WTYPE_FE4M3 ? 2 : 0);
   const bool w8 = wt != 0;
-  const bool channelwise = group_size == -1 || (group_size == size_k && size_k != 128);
-  VAQ_CHECK_SUPPORTED(channelwise || group_size == 128 || group_size == 64 || group_size == 32,
-                      "w4a16_gemm: group_size = %d is not built (only -1, 32, 64, 128)", group_size);
-  const int sub = channelwise ? 1 : 128 / group_size;
   VAQ_CHECK_SUPPORTED(wt != 2 || (sub == 1 && perm == nullptr),
                       "w4a16_gemm: FP8 weights take channelwise scales or groups of 128 rows, and no act_order");
   VAQ_CHECK_ARG(!w8 || size_k * size_n < (1ll << 32), "w4a16_gemm: problem too large for 8-bit weights");
@@ -153,7 +172,7 @@ extern "C" int vaq_w4a16_gemm_tuned(const void* a, int64_t lda, const int32_t* b
     bool tile_ok = force_path == 0;
     if (tile_ok && size_m <= DECODE_MAX_M_2BLK) {
       size_t t = 0, n = 0;
-      w4a16_prefill_workspace((int)size_m, (int)size_n, (int)size_k, &t, &n);
+      w4a16_prefill_workspace((int)size_m, (int)size_n, (int)size_k, tile_format(sub, wt), &t, &n);
       tile_ok = perm == nullptr && c_tmp_bytes >= (int64_t)t && counter_ints >= (int64_t)n;
     }
     const int kind = w4a16_decode2_choose((int)size_m, (int)size_n, (int)size_k, sub, wt, perm != nullptr, decode, tile_ok || !decode,

@@ -22,7 +22,7 @@ int w4a16_decode2_launch(const void* a, int64_t lda, const int32_t* b, const voi
                          const int32_t* perm, const void* bias, void* c, float* c_tmp, int64_t c_tmp_bytes,
                          int32_t* counters, int64_t counter_ints, int M, int N, int K, int sub, bool channelwise,
                          int wt, int dtype, bool rows, hipStream_t s);      // wt: 0 4-bit codes, 1 8-bit codes, 2 FP8 e4m3 bytes
-int w4a16_prefill_workspace(int M, int N, int K, size_t* c_tmp_bytes, size_t* counter_ints);
+int w4a16_prefill_workspace(int M, int N, int K, TileFormat format, size_t* c_tmp_bytes, size_t* counter_ints);
 int w4a16_prefill_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
                          const void* bias, void* c, float* c_tmp, int64_t c_tmp_bytes, int32_t* counters,
                          int64_t counter_ints, int M, int N, int K, int sub, bool channelwise, int wt, int dtype,

@@ -165,14 +165,10 @@ static TilePlan plan_prefill(int M, int N, int K, bool direct_ok, TileFormat for
 // were strips.
 double w4a16_staged_us(int M, int N, int K, bool plain) { return plan_prefill(M, N, K, true, plain ? TILES_PLAIN_STAGED : TILES_FP8).us; }
 
-int w4a16_prefill_workspace(int M, int N, int K, size_t* c_tmp_bytes, size_t* counter_ints) {
-  // enough for every weight format: it is not known here
-  *c_tmp_bytes = *counter_ints = 0;
-  for (TileFormat format : {TILES_PLAIN, TILES_SUB, TILES_8BIT, TILES_FP8}) {
-    const TilePlan pl = plan_prefill(M, N, K, true, format);
-    if ((size_t)pl.tmp_bytes() > *c_tmp_bytes) *c_tmp_bytes = (size_t)pl.tmp_bytes();
-    if ((size_t)pl.counter_ints() > *counter_ints) *counter_ints = (size_t)pl.counter_ints();
-  }
+int w4a16_prefill_workspace(int M, int N, int K, TileFormat format, size_t* c_tmp_bytes, size_t* counter_ints) {
+  const TilePlan pl = plan_prefill(M, N, K, true, format);
+  *c_tmp_bytes = (size_t)pl.tmp_bytes();
+  *counter_ints = (size_t)pl.counter_ints();
   return VAQ_OK;
 }
 
