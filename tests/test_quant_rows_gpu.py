@@ -83,3 +83,16 @@ def test_per_tensor_runs_equal_rows(device, shape, dtype):
         if x.numel() < 1 << 20:
             ref = f.ref_static_quant(x.cpu(), scale.cpu()) if given is not None else f.ref_dynamic_per_tensor_quant(x.cpu())
             assert _same(got[:1], [ref[0] if isinstance(ref, tuple) else ref])
+
+
+@pytest.mark.parametrize("rows,hidden,gap", [(3, 1061, 0), (300, 2047, 0), (1030, 2049, 0), (1030, 5119, 0), (7, 4097, 1), (5, 16385, 0), (4, 32767, 0),
+                                             (4, 4096, 3), (1030, 2048, 5), (1, 1000, 3), (6, 40000, 0)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_rows_by_single_elements_bit_exact(device, rows, hidden, gap, dtype):
+    """Lengths, row strides and addresses that rule vectors out, on each size of workgroup that takes such rows."""
+    import vllm_amd._custom_ops as ops
+    x = torch.randn(rows, hidden + gap, generator=torch.Generator().manual_seed(hidden)).to(dtype)[:, gap:]
+    x[-1, -1] = 23.0
+    view = torch.zeros(rows, hidden + gap, dtype=dtype, device=device)[:, gap:]
+    view.copy_(x)
+    assert _same(ops.scaled_fp8_quant(view, use_per_token_if_dynamic=True), f.ref_dynamic_per_token_quant(x.contiguous()))

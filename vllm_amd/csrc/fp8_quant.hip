@@ -10,8 +10,9 @@
 // The file is compiled without fast-math, so `/` is the correctly rounded division.
 //
 // HBM-bound: each row is read ONCE -- a workgroup keeps its whole row in registers between the absmax pass and the
-// convert pass whenever the row has at most 512 threads x 4 vectors x 8 elements = 16384 elements and is 16-byte
-// aligned; other rows take a two-pass scalar path.
+// convert pass whenever the row has at most 512 threads x 8 vectors x 8 elements = 32768 elements and its addresses and
+// length allow vectors; other rows are read twice by single elements.  Per tensor, rows without gaps are one run of
+// vectors, whatever their length.
 #include "vaq_common.h"
 
 namespace vaq {
@@ -347,6 +348,12 @@ static int launch_quant(const void* in, int in_dtype, int64_t in_stride, uint8_t
   const std::integral_constant<int, 1> one;
   const std::integral_constant<int, 4> four;
   const std::integral_constant<int, 8> eight;
+  // Rows that go by single elements are better off with many threads and few registers each: 512 rows or fewer of 1000 elements 20 %
+  // ahead of 256 threads (256 x 1061 3.3 against 4.0 us), 802 rows of 32454 60 us with four vectors' registers, 88 with eight.
+  const int64_t align = in_dtype == VAQ_F32 ? 4 : 8;      // elements of 16 bytes
+  const bool strides_ok = rows == 1 || (in_stride % align == 0 && out_stride % 8 == 0);
+  if (hidden % 8 != 0 || hidden > QT * 8 * 8 || (uintptr_t)in % 16 != 0 || (uintptr_t)out % 8 != 0 || !strides_ok)
+    return rows >= 1024 && hidden <= 5120 ? launch(half, four) : launch(full, four);
   if (hidden <= QT / 2 * 8) return launch(half, one);
   if (rows >= 1024 && hidden <= 5120) return launch(half, four);
   if (hidden <= QT * 8) return launch(full, one);
