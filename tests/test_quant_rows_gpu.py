@@ -48,11 +48,11 @@ def test_long_rows_bit_exact(device, hidden, dtype):
     assert _same(ops.scaled_fp8_quant(x.to(device), scale.to(device))[:1], [f.ref_static_quant(x, scale)])
 
 
-@pytest.mark.parametrize("tokens,d", [(1, 8), (3, 24), (517, 1000), (292, 14336), (293, 14336), (2341, 14336)])
+@pytest.mark.parametrize("tokens,d", [(1, 8), (3, 24), (1, 6144), (2, 3080), (2, 6144), (1, 12296), (517, 1000), (292, 14336), (293, 14336), (2341, 14336)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_silu_chunks_equal_single_elements(device, tokens, d, dtype):
     """Chunks of 8 against the element-wise kernel of the same arithmetic (an output that is not 8-byte aligned): one chunk, a last
-    workgroup in part, both workgroup sizes beside the line between them, and a thread's second chunk."""
+    workgroup in part, both workgroup sizes beside the lines between them (768, 1536 and 524288 chunks), and a thread's second chunk."""
     import vllm_amd._custom_ops as ops
     x = torch.randn(tokens, 2 * d, device=device, dtype=dtype, generator=torch.Generator(device=device).manual_seed(d))
     scale = torch.full((1,), 4 / 448, device=device)
@@ -64,7 +64,7 @@ def test_silu_chunks_equal_single_elements(device, tokens, d, dtype):
     assert torch.equal(out.view(torch.uint8), odd.view(torch.uint8))
 
 
-@pytest.mark.parametrize("shape", [(1, 1), (1, 7), (3, 8), (1, 2047), (5, 411), (333, 3001), (2, 1050633), (1, 33554441)])
+@pytest.mark.parametrize("shape", [(1, 1), (1, 7), (3, 8), (1, 2047), (5, 411), (2, 3076), (3, 4096), (3, 4099), (333, 3001), (2, 1050633), (1, 33554441)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_per_tensor_runs_equal_rows(device, shape, dtype):
     """Rows without gaps go as one run of vectors: single elements, remainders behind the last vector, one and several rounds of the

@@ -369,9 +369,11 @@ static int launch_quant_per_tensor(const void* in, int in_dtype, int64_t in_stri
   if (!run) return launch_quant<MODE>(in, in_dtype, in_stride, out, out_stride, scale, nullptr, rows, hidden, s);
   // A given scale: up to eight workgroups of 256 to a compute unit, 512 threads beyond (16 x 14336 1.85 against 1.94 us; 2048 x 4096
   // 6.36 against 6.45); one vector to a thread, two are slower for few rows (250 x 5120 2.4 -> 2.6 us) and for many (4096 x 20480
-  // 40 -> 42).  Maximum: at most one workgroup to a compute unit, two vectors to a thread where they are few.
+  // 40 -> 42).  A launch of up to three workgroups takes 0.12 us less than one of four: 512 threads where that makes three of them
+  // (2 x 4096 1.88 -> 1.74 us).  Maximum: at most one workgroup to a compute unit, two vectors to a thread where they are few.
   const int64_t total = rows * hidden, vecs = total / 8, cus = num_cus_current_device();
-  const int threads = MODE == 2 ? QTA : vecs <= cus * 2048 ? QT / 2 : QT;
+  const bool three = vecs > 3 * (QT / 2) && vecs <= 3 * QT;
+  const int threads = MODE == 2 ? QTA : vecs <= cus * 2048 && !three ? QT / 2 : QT;
   const int64_t share = MODE == 2 ? 2 * QTA : threads, cap = MODE == 2 ? cus : cus * 32 * QT / threads;
   const int64_t blocks = (vecs + share - 1) / share;
   const dim3 grid((unsigned)(blocks < 1 ? 1 : blocks < cap ? blocks : cap)), block(threads);

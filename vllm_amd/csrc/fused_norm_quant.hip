@@ -646,8 +646,10 @@ extern "C" int vaq_silu_and_mul_fp8_quant(uint8_t* out, const void* input, const
   const bool vec = d % 8 == 0 && ((uintptr_t)input % 16) == 0 && ((uintptr_t)out % 8) == 0;
   const int64_t work = vec ? tokens * (d / 8) : tokens * d;
   // Little work on workgroups of 256: twice as many compute units take part (7 tokens of 14336 2.16 -> 2.02 us, 250 of 13824 5.61 ->
-  // 5.46); from eight workgroups of 256 to a compute unit on the two are level or 512 is ahead (2048 of 14336 28.7 against 29.5 us).
-  const int threads = work <= (int64_t)num_cus_current_device() * 2048 ? NQ_T / 2 : NQ_T;
+  // 5.46), but for what three of 512 hold: a launch of up to three workgroups takes 0.12 us less than one of four.  From eight
+  // workgroups of 256 to a compute unit on the two are level or 512 is ahead (2048 of 14336 28.7 against 29.5 us).
+  const bool three = work > 3 * (NQ_T / 2) && work <= 3 * NQ_T;
+  const int threads = work <= (int64_t)num_cus_current_device() * 2048 && !three ? NQ_T / 2 : NQ_T;
   int64_t blocks = (work + threads - 1) / threads;
   const int64_t cap = (int64_t)num_cus_current_device() * 32 * NQ_T / threads;
   if (blocks > cap) blocks = cap;
