@@ -86,11 +86,19 @@ extern "C" int vaq_permute_cols(const void* a, int64_t lda, const int32_t* perm,
   const size_t row_bytes = (size_t)size_k * 2;
   if (row_bytes <= 128 * 1024) {
     // four or two rows to a workgroup only where that leaves two workgroups per compute unit: 4096 columns, 100 / 333 / 1024 rows
-    // 4.0 / 4.2 / 5.0 -> 2.2 / 2.6 / 4.2 us (from one to the other, launch to launch), 4096 rows 12.3 us either way
-    const int64_t few = 2 * (int64_t)num_cus_current_device();
+    // 4.0 / 4.2 / 5.0 -> 2.2 / 2.6 / 4.2 us (from one to the other, launch to launch), 4096 rows 12.3 us either way; and not from 1536
+    // to 4095 columns, where one row is ahead at any number (2048 x 7500 16.1 -> 13.3 us, 3072 x 8192 26.0 -> 21.3, 1536 x 2048 5.9 ->
+    // 4.6; 1024 x 8192 8.3 against 9.0 us, 4096 x 4096 13.1 against 14.9)
+    const int64_t cus = num_cus_current_device(), few = 2 * cus;
     int rows = row_bytes * 4 <= 32 * 1024 ? 4 : (row_bytes * 2 <= 32 * 1024 ? 2 : 1);
-    while (rows > 1 && size_m / rows < few) rows /= 2;
-    const dim3 threads(rows == 1 && size_k > 2048 ? 512 : 256);
+    while (rows > 1 && (size_m / rows < few || (size_k >= 1536 && size_k < 4096))) rows /= 2;
+    // One row: 512 threads for a long one (half the steps of the chain), four such workgroups to a compute unit.  More rows than that
+    // run on 256 threads where all of them are on the device at once then (1280 x 12288 16.9 -> 14.9 us, 1280 x 14336 19.8 -> 18.0,
+    // 1536 x 9088 15.0 -> 13.8), and shorter ones at any number (8192 x 3072 21.6 -> 21.3); else 512 are ahead again (4096 x 14336 54.2
+    // against 48.7).
+    const int64_t held = cus * (row_bytes * 8 < 160 * 1024 ? 8 : (160 * 1024 - 1) / (int64_t)row_bytes);
+    const bool wide = rows == 1 && size_k > 2048 && (size_m <= 4 * cus || (size_m > held && size_k > 4096));
+    const dim3 threads(wide ? 512 : 256);
     const size_t lds = rows * row_bytes;
     const void* kern = rows == 4 ? reinterpret_cast<const void*>(permute_cols_lds_kernel<4>)
                                  : (rows == 2 ? reinterpret_cast<const void*>(permute_cols_lds_kernel<2>)
