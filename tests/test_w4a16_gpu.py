@@ -138,6 +138,26 @@ def test_repack_act_order_half_strips(device, k, n, bits):
         assert np.array_equal(got.cpu().numpy(), nl.native_pack8_bytes(q[perm_np]))
 
 
+@pytest.mark.parametrize("k,n,bits", [(40960, 576, 4), (20608, 512, 4), (20480, 448, 8), (10368, 384, 8), (20480, 832, 8), (10368, 768, 8)])
+def test_repack_act_order_long_narrow_layers(device, k, n, bits):
+    """K beyond the LDS of a whole strip: both sides of the widths from which strips of 8 columns take over, at the largest strip
+    and the smallest.  On the device: output row k of the repacked tensor is row perm[k] of the plain one's source."""
+    import vllm_amd._custom_ops as ops
+    q = torch.randint(0, 1 << bits, (k, n), dtype=torch.int32, device=device, generator=torch.Generator(device=device).manual_seed(k + n))
+    perm = torch.randperm(k, device=device, generator=torch.Generator(device=device).manual_seed(n)).to(torch.int32)
+
+    def pack(codes):
+        per = 32 // bits
+        words = torch.zeros(k // per, n, dtype=torch.int64, device=device)
+        for i in range(per):
+            words |= codes[i::per].long() << (bits * i)
+        return words.to(torch.int32)
+    none = torch.empty(0, dtype=torch.int32, device=device)
+    for layout in ("native",) if bits == 4 else ("native", "native_bytes"):
+        want = ops.gptq_marlin_repack(pack(q[perm.long()]), none, k, n, bits, layout=layout)
+        assert torch.equal(ops.gptq_marlin_repack(pack(q), perm, k, n, bits, layout=layout), want)
+
+
 # ------------------------------------------------------------------------------------------------ permute_cols
 
 @pytest.mark.parametrize("m,k", [(1, 128), (3, 1024), (7, 4096), (130, 14336), (5, 70000)])

@@ -216,7 +216,8 @@ __global__ __launch_bounds__(256) void repack_marlin8_kernel(const uint32_t* __r
 // The three kernels below write every output tile as the 16-byte pieces its lanes own (a wavefront store is contiguous)
 // and read the checkpoint tensor in whole 64-byte pieces or more.  Bound: HBM.  What the one-word-per-thread kernels above
 // lose is the gather: 8 four-byte loads per output word with act_order or AWQ, from lines that other workgroups fetch again.
-// They stay for the MARLIN order, for pointers that are not 16-byte aligned, and for an act_order strip beyond LDS.
+// They stay for the MARLIN order, for pointers that are not 16-byte aligned, and for act_order on long narrow layers (strips beyond
+// LDS, or too few of them).
 
 // OUT 0: 4-bit codes; 1: 8-bit codes as two nibble planes; 2: 8-bit codes as bytes.
 template <int OUT>
@@ -361,11 +362,16 @@ __global__ __launch_bounds__(256) void repack_native_awq_kernel(const uint32_t* 
   }
 }
 
-// Whether the kernels above take a problem: 16-byte pointers, 32-bit indexes, and with act_order a strip that fits LDS.
-static bool repack_tiles_ok(const void* qweight, const void* perm, const void* out, int64_t size_k, int64_t size_n, int num_bits) {
+// Whether the kernels above take a problem: 16-byte pointers, 32-bit indexes, and with act_order a strip that fits LDS.  Where only
+// strips of 8 columns fit, a layer has to be wide enough to give work to many compute units: a strip takes 10 .. 25 us by
+// itself, and up to these widths the kernels of one word per thread are ahead or within a few percent (K = 24064 x 64 columns, 4 bits, 12.0
+// against 5.1 us, 25600 x 512 19.7 against 18.8, x 640 18.9 against 21.5; 8 bits 17920 x 384 21.2 against 20.7, x 448 20.2 against 22.7;
+// bytes 17920 x 768 24.2 against 22.6, x 896 18.0 against 22.3).
+static bool repack_tiles_ok(const void* qweight, const void* perm, const void* out, int64_t size_k, int64_t size_n, int num_bits, int layout) {
   if (((uintptr_t)qweight % 16) || ((uintptr_t)out % 16) || ((uintptr_t)perm % 16)) return false;
   if (size_k > (1 << 22) || size_n > (1 << 24)) return false;
-  return !perm || size_k * num_bits <= REPACK_LDS_MAX;
+  if (!perm || size_k * num_bits * 2 <= REPACK_LDS_MAX) return true;
+  return size_k * num_bits <= REPACK_LDS_MAX && size_n > (num_bits == 4 ? 512 : layout == VAQ_LAYOUT_NATIVE ? 384 : 768);
 }
 
 template <int OUT, int C>
@@ -425,7 +431,7 @@ static int repack_common(const int32_t* qweight, const int32_t* perm, int32_t* o
   const uint32_t* qw = (const uint32_t*)qweight;
   uint32_t* o = (uint32_t*)out;
   const dim3 grid((unsigned)blocks), block(threads);
-  if (layout != VAQ_LAYOUT_MARLIN && repack_tiles_ok(qweight, perm, out, size_k, size_n, num_bits)) {
+  if (layout != VAQ_LAYOUT_MARLIN && repack_tiles_ok(qweight, perm, out, size_k, size_n, num_bits, layout)) {
     int rc = VAQ_OK;
     if (awq)
       hipLaunchKernelGGL(repack_native_awq_kernel, dim3((unsigned)((size_n + 255) / 256), (unsigned)(size_k / 128)), dim3(256), 0, s, qw, o,
