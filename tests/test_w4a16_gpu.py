@@ -138,24 +138,35 @@ def test_repack_act_order_half_strips(device, k, n, bits):
         assert np.array_equal(got.cpu().numpy(), nl.native_pack8_bytes(q[perm_np]))
 
 
-@pytest.mark.parametrize("k,n,bits", [(40960, 576, 4), (20608, 512, 4), (20480, 448, 8), (10368, 384, 8), (20480, 832, 8), (10368, 768, 8)])
-def test_repack_act_order_long_narrow_layers(device, k, n, bits):
-    """K beyond the LDS of a whole strip: both sides of the widths from which strips of 8 columns take over, at the largest strip
-    and the smallest.  On the device: output row k of the repacked tensor is row perm[k] of the plain one's source."""
+def _repack_perm_equals_sorted(device, k, n, bits):
+    """Repacking with a permutation against repacking the tensor whose rows were permuted before they were packed."""
     import vllm_amd._custom_ops as ops
     q = torch.randint(0, 1 << bits, (k, n), dtype=torch.int32, device=device, generator=torch.Generator(device=device).manual_seed(k + n))
     perm = torch.randperm(k, device=device, generator=torch.Generator(device=device).manual_seed(n)).to(torch.int32)
 
     def pack(codes):
-        per = 32 // bits
-        words = torch.zeros(k // per, n, dtype=torch.int64, device=device)
-        for i in range(per):
-            words |= codes[i::per].long() << (bits * i)
+        words = torch.zeros(k * bits // 32, n, dtype=torch.int64, device=device)
+        for i in range(32 // bits):
+            words |= codes[i::32 // bits].long() << (bits * i)
         return words.to(torch.int32)
     none = torch.empty(0, dtype=torch.int32, device=device)
     for layout in ("native",) if bits == 4 else ("native", "native_bytes"):
         want = ops.gptq_marlin_repack(pack(q[perm.long()]), none, k, n, bits, layout=layout)
         assert torch.equal(ops.gptq_marlin_repack(pack(q), perm, k, n, bits, layout=layout), want)
+
+
+@pytest.mark.parametrize("k,n,bits", [(128, 4160, 4), (512, 4160, 4), (640, 4160, 4), (1024, 4160, 4), (1152, 4160, 4), (384, 4160, 8), (512, 4160, 8), (640, 4160, 8),
+                                      (2560, 8256, 8), (4224, 8256, 4), (5248, 4160, 8), (10368, 4160, 4)])
+def test_repack_act_order_threads_of_a_strip(device, k, n, bits):
+    """16-column strips on each size of workgroup: as many threads as 16-byte loads, three workgroups to a compute unit, two, one."""
+    _repack_perm_equals_sorted(device, k, n, bits)
+
+
+@pytest.mark.parametrize("k,n,bits", [(40960, 576, 4), (20608, 512, 4), (20480, 448, 8), (10368, 384, 8), (20480, 832, 8), (10368, 768, 8)])
+def test_repack_act_order_long_narrow_layers(device, k, n, bits):
+    """K beyond the LDS of a whole strip: both sides of the widths from which strips of 8 columns take over, at the largest strip
+    and the smallest."""
+    _repack_perm_equals_sorted(device, k, n, bits)
 
 
 # ------------------------------------------------------------------------------------------------ permute_cols

@@ -382,8 +382,15 @@ static int launch_repack_perm(const uint32_t* qw, const int32_t* perm, uint32_t*
   if (rc != VAQ_OK) return rc;
   const int per_xcd = (int)((size_n / (4 * C) + 7) / 8);
   // 12 wavefronts: 8 are up to 12 % slower where a compute unit holds one strip (8 bits 8192 x 8192 39.6 against 34.5 us), 16 up to 6 %
-  // where it holds two (4096 x 28672 29.8 against 28.2); a single whole strip of 4 bits is the exception (14336 x 4096 17.6 -> 17.2)
-  const int threads = OUT == 0 && C == 4 && lds > REPACK_LDS_MAX / 2 ? 1024 : 768;
+  // where it holds two (4096 x 28672 29.8 against 28.2).  Single whole strips of nibbles take 16 (14336 x 4096 17.6 -> 17.2), of 8 bits
+  // where there are more of them than compute units (8192 x 14336 70.2 -> 68.6, 6144 x 28672 100.5 -> 96.4; 8192 x 4096 18.3 against
+  // 18.7).  A whole strip of few 16-byte loads takes no more threads than loads: more of them share a compute unit (128 x 14336 6.4 ->
+  // 4.7 us in 8 bits, 4.6 -> 3.5 in 4; 512 x 28672 7.7 -> 7.0 in 4 bits, 11.4 -> 10.9 in 8; 384 x 16192 7.8 -> 6.7 in 8).
+  // And three workgroups of 8 wavefronts where they hold all strips at once and two of 12 do not (2560 x 8384 in 8 bits 18.5 -> 16.0).
+  const int64_t loads = size_k / (OUT == 0 ? 8 : 4) * C, strips = size_n / (4 * C), cus = num_cus_current_device();
+  const bool single = lds > REPACK_LDS_MAX / 2 && OUT != 2 && (OUT == 0 || strips > cus);
+  const bool three = lds > REPACK_LDS_MAX / 5 && lds * 3 <= REPACK_LDS_MAX && strips > 2 * cus && strips <= 3 * cus;
+  const int threads = C != 4 ? 768 : loads <= 512 ? (loads <= 256 ? 256 : (int)(loads + 63) / 64 * 64) : three ? 512 : single ? 1024 : 768;
   hipLaunchKernelGGL((repack_native_perm_kernel<OUT, C>), dim3(per_xcd * 8), dim3(threads), lds, s, qw, perm, out, (int)size_k, (int)size_n,
                      per_xcd);
   return VAQ_OK;
