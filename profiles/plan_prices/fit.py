@@ -1,7 +1,7 @@
 """Fits the price formulas of the tile kernels and of the W4A16 decode kernel to the timings of scan.py, and says how good
 the plans are that they choose.
 
-    python profiles/plan_prices/fit.py fp8_tile|w4_tile|w8_tile|w4_decode TIMINGS.csv[.gz] [...] [--fit]
+    python profiles/plan_prices/fit.py fp8_tile|w4_tile|w4sub_tile|w4sub32zp_tile|w8_tile|w8sub_tile|w4_decode TIMINGS.csv[.gz] [...] [--fit]
 
 Without --fit: the constants of the sources, read from them.  The formulas are those of `tile_plan_us` in
 vllm_amd/csrc/tile_plan.h and `decode2_us` in vllm_amd/csrc/w4a16_decode2.hip.
@@ -41,12 +41,15 @@ class Tiles:
         fp8 = kind == "fp8_tile"
         file = "fp8_scaled_mm.hip" if fp8 else "w4a16_prefill.hip"
         prefix = kind.split("_")[0].upper()
+        sub8, prefix = prefix == "W8SUB", "W8" if prefix == "W8SUB" else prefix      # (the table of 8-bit codes, less one slot)
         rows = np.array(source_table(file, f"{prefix}_TILE_SHAPES")).reshape(-1, 10)
+        if sub8:
+            rows[rows[:, 0] == 41, 4] = 1
         self.ids = rows[:, 0].astype(int)
         self.shape = rows[:, 1:5]                        # bm, bn, nw, slots
         self.p_shape = rows[:, 5:]                       # base, step, load, shared, out
         self.p_costs = np.array(source_table(file, f"{prefix}_TILE_COSTS"))
-        self.bytes = 0.5 if kind in ("w4_tile", "lds_tile") else 1.0
+        self.bytes = 0.5 if prefix.startswith(("W4", "LDS")) else 1.0
 
     def pack(self):
         return np.concatenate([self.p_shape.ravel(), self.p_costs])
@@ -55,19 +58,25 @@ class Tiles:
         self.p_shape, self.p_costs = p[:self.p_shape.size].reshape(self.p_shape.shape), p[self.p_shape.size:]
 
     def load(self, files):
-        d = np.concatenate([np.loadtxt(f, delimiter=",", ndmin=2) for f in files])
-        d[:, 3] = np.where(d[:, 3] == 30, 20, d[:, 3]) if self.kind == "w4_tile" else d[:, 3]
-        d = d[np.isin(d[:, 3], self.ids)]
-        # (two forms of the 256 x 256 tile: the faster one, which the planner's last rule is to find)
-        order = np.lexsort((d[:, 6], d[:, 5], d[:, 4], d[:, 3], d[:, 2], d[:, 1], d[:, 0]))
-        d = d[order]
-        first = np.ones(len(d), bool)
-        first[1:] = (d[1:, :6] != d[:-1, :6]).any(1)
-        d = d[first]
+        """Every file is a set of problems of its own (the formats were timed on the same ones)."""
+        parts, problems = [], 0
+        for file in files:
+            d = np.loadtxt(file, delimiter=",", ndmin=2)
+            d[:, 3] = np.where(d[:, 3] == 30, 20, d[:, 3]) if self.kind == "w4_tile" else d[:, 3]
+            d = d[np.isin(d[:, 3], self.ids)]
+            # (two forms of the 256 x 256 tile: the faster one, which the planner's last rule is to find)
+            order = np.lexsort((d[:, 6], d[:, 5], d[:, 4], d[:, 3], d[:, 2], d[:, 1], d[:, 0]))
+            d = d[order]
+            first = np.ones(len(d), bool)
+            first[1:] = (d[1:, :6] != d[:-1, :6]).any(1)
+            d = d[first]
+            key = np.unique(d[:, :3], axis=0, return_inverse=True)[1].ravel() + problems
+            problems = key.max() + 1
+            parts.append((d, key))
+        d, self.key = (np.concatenate(x) for x in zip(*parts))
         self.k, self.n, self.m, ident, self.sk, self.tail, self.us = d.T
         self.which = np.searchsorted(self.ids, ident, sorter=np.argsort(self.ids))
         self.which = np.argsort(self.ids)[self.which]
-        self.key = np.unique(d[:, :3], axis=0, return_inverse=True)[1].ravel()
 
     def price(self, p_shape, p_costs):
         bm, bn, _, slots = self.shape[self.which].T

@@ -1,12 +1,13 @@
 """Times every plan of random problems, for the price formulas that choose among them (fit.py).
 
-    python profiles/plan_prices/scan.py fp8_tile|w4_tile|w8_tile|w4_decode SECONDS SEED OUT.csv
+    python profiles/plan_prices/scan.py fp8_tile|w4_tile|w8_tile|w4g64z_tile|w4g32_tile|w4g32z_tile|w8g64_tile|w8g32_tile|w4_decode SECONDS SEED OUT.csv
 
 Runs on the GPU; the *.csv.gz beside it are what it wrote on an MI355X.  A problem is a layer (K, N) and a number of rows; a plan is forced through the `_tuned` entry points
 (vllm_amd/csrc/vaq_tuning.h).  Weights are cold: a graph of launches walks over copies of the layer (640 MB of them, at most
 400).  One line per plan, with the time of a launch in us:
 
-    fp8_tile, w4_tile, w8_tile (8-bit codes):  k, n, m, tile id, parts of K, 1 if only the tiles of the last round are in parts, us
+    fp8_tile, w4_tile (4-bit codes in groups of 128 rows with zero points), w8_tile (8-bit codes), and both in groups of 64 / 32 rows,
+    z with zero points:  k, n, m, tile id, parts of K, 1 if only the tiles of the last round are in parts, us
     w4_decode:          k, n, m, groups of 128 rows (1, 2, 4), 8-bit codes, kind, gs, wks, wn (0: by the planner), us
                         kind 0 workgroups of all rows, 1 of 16 rows, 2 the tile kernel by its own plan (gs, wks, wn 0; recorded
                         with the shapes up to 20 only, at whose price the decode kernels are weighed)
@@ -32,12 +33,13 @@ class Layer:
     """Operands of one layer: views of one pool of random bytes (finite e4m3 codes) and of one of scales."""
     pool = scales = None
 
-    def __init__(self, fp8: bool, k: int, n: int, most_m: int, bits: int = 4, group: int = 128):
+    def __init__(self, fp8: bool, k: int, n: int, most_m: int, bits: int = 4, group: int = 128, zeros: bool | None = None):
         if Layer.pool is None:
             p = torch.randint(0, 256, (1_500_000_000,), dtype=torch.uint8, device="cuda")
             Layer.pool = torch.where((p & 0x7f) == 0x7f, p ^ 1, p)
             Layer.scales = (torch.rand(150_000_000, device="cuda") * 1e-2 + 1e-3).to(torch.bfloat16)
         self.fp8, self.k, self.n, self.bits, self.group = fp8, k, n, bits, group
+        self.zeros = bits == 4 and group == 128 if zeros is None else zeros      # uint4 with zero points, else uint4b8
         self.bytes = k * n if fp8 else k * n * bits // 8
         self.copies = max(2, min(MOST_COPIES, POOL // self.bytes))
         x = torch.randn(most_m, k, device="cuda", dtype=torch.bfloat16)
@@ -60,9 +62,8 @@ class Layer:
                 _lib.VAQ_BF16, m, self.n, self.k, tmp, tmp_bytes, self.counters.data_ptr(), self.counters.numel(), stream, tune)
         scale_count = self.n * (self.k // self.group)
         at = c * scale_count % max(1, self.scales.numel() - scale_count) // 64 * 64
-        zeros = self.bits == 4 and self.group == 128      # (uint4 with zero points there, uint4b8 in smaller groups)
-        wtype = _lib.VAQ_WTYPE_U8B128 if self.bits == 8 else _lib.VAQ_WTYPE_U4 if zeros else _lib.VAQ_WTYPE_U4B8
-        z = self.pool.data_ptr() + self.pool.numel() - (c + 1) * (scale_count // 2) // 64 * 64 - scale_count if zeros else None
+        wtype = _lib.VAQ_WTYPE_U8B128 if self.bits == 8 else _lib.VAQ_WTYPE_U4 if self.zeros else _lib.VAQ_WTYPE_U4B8
+        z = self.pool.data_ptr() + self.pool.numel() - (c + 1) * (scale_count // 2) // 64 * 64 - scale_count if self.zeros else None
         return lib.vaq_w4a16_gemm_tuned(
             self.a.data_ptr(), self.k, w, self.scales.data_ptr() + 2 * at, z, None, None, self.out.data_ptr(), tmp, tmp_bytes, None,
             self.counters.data_ptr(), self.counters.numel(), m, self.n, self.k, self.group, _lib.VAQ_BF16, wtype, path, stream, tune)
@@ -139,6 +140,12 @@ TILES = {"fp8_tile": {13: (128, 128), 14: (64, 128), 15: (64, 64), 16: (128, 64)
                      48: (256, 256)},
          "w8_tile": {12: (128, 128), 14: (64, 128), 15: (128, 64), 16: (256, 128), 20: (256, 256), 41: (32, 128), 51: (32, 64), 42: (64, 128),
                      52: (64, 64), 43: (96, 128), 44: (128, 128), 46: (128, 256)}}
+FORMATS_OF = {"w4_tile": (4, 128, True), "w8_tile": (8, 128, False)}      # bits, rows of a group, zero points
+for _bits in (4, 8):
+    for _group in (64, 32):
+        for _zeros in ("", "z") if _bits == 4 else ("",):
+            FORMATS_OF[f"w{_bits}g{_group}{_zeros}_tile"] = (_bits, _group, _zeros == "z")
+            TILES[f"w{_bits}g{_group}{_zeros}_tile"] = TILES["w8_tile"]
 
 
 def tile_plans(kind, k, n, m):
@@ -167,7 +174,7 @@ def scan_tiles(lib, kind, rng, until, out):
         rows = [m for m in (log(rng, 9 if fp8 else 17, 8192, 1) for _ in range(3)) if 2.0 * m * n * k < 2e12 and m * n < 6e8]
         if not rows:
             continue
-        layer = Layer(fp8, k, n, max(rows), 8 if kind == "w8_tile" else 4)
+        layer = Layer(fp8, k, n, max(rows), *(() if fp8 else FORMATS_OF[kind]))
         if not layer.fits():
             continue
         for m in rows:
