@@ -62,9 +62,7 @@ class Tiles:
         parts, problems = [], 0
         for file in files:
             d = np.loadtxt(file, delimiter=",", ndmin=2)
-            d[:, 3] = np.where(d[:, 3] == 30, 20, d[:, 3]) if self.kind == "w4_tile" else d[:, 3]
             d = d[np.isin(d[:, 3], self.ids)]
-            # (two forms of the 256 x 256 tile: the faster one, which the planner's last rule is to find)
             order = np.lexsort((d[:, 6], d[:, 5], d[:, 4], d[:, 3], d[:, 2], d[:, 1], d[:, 0]))
             d = d[order]
             first = np.ones(len(d), bool)

@@ -135,7 +135,7 @@ def shape(rng, step_n, most):
 
 
 TILES = {"fp8_tile": {13: (128, 128), 14: (64, 128), 15: (64, 64), 16: (128, 64), 17: (128, 256), 19: (256, 128), 1: (256, 256), 10: (256, 384)},
-         "w4_tile": {12: (128, 128), 14: (64, 128), 15: (128, 64), 16: (256, 128), 13: (128, 256), 20: (256, 256), 30: (256, 256),
+         "w4_tile": {12: (128, 128), 14: (64, 128), 15: (128, 64), 16: (256, 128), 13: (128, 256), 20: (256, 256),
                      41: (32, 128), 51: (32, 64), 42: (64, 128), 52: (64, 64), 43: (96, 128), 44: (128, 128), 46: (128, 256), 66: (128, 256),
                      48: (256, 256)},
          "w8_tile": {12: (128, 128), 14: (64, 128), 15: (128, 64), 16: (256, 128), 20: (256, 256), 41: (32, 128), 51: (32, 64), 42: (64, 128),
@@ -159,7 +159,7 @@ def tile_plans(kind, k, n, m):
         if bm > 64 and bm >= 2 * m:
             continue
         for sk in range(1, 9):
-            if sk == 1 or (steps // sk >= (6 if kind == "fp8_tile" else 3) and tiles * sk <= CUS * 3 and ident != 30):
+            if sk == 1 or (steps // sk >= (6 if kind == "fp8_tile" else 3) and tiles * sk <= CUS * 3):
                 yield ident, sk, 0
         if ident in (1, 20, 48) and tiles > CUS and rest:
             for sk in (2, 3, 4):

@@ -11,8 +11,7 @@ namespace vaq {
 // ----------------------------------------------------------------------------- host side
 
 // tile ids: 0..2 = register-staged kernel (256x256, 128x128, 64x128); 10.. = direct-to-LDS kernel (BM x BN);
-// 30 = 256 x 256 with the weights dequantised in registers (w4a16_prefill3_kernel.h)
-int prefill_launch_reg(const PrefillParams& p, bool bf16, bool zp, hipStream_t s);      // w4a16_prefill3.hip
+// 41.. = strips (w4a16_strip_kernel.h)
 // w4a16_strip*.hip
 int prefill_launch_strip(const PrefillParams& p, int tile, bool bf16, bool zp, hipStream_t s);
 int prefill_launch_strip_sub(const PrefillParams& p, int sub, int tile, bool bf16, bool zp, hipStream_t s);
@@ -23,7 +22,6 @@ static int dispatch_tile(const PrefillParams& p, int tile, hipStream_t s) {
   switch (tile) {
     case 10: return launch_prefill2<BF16, 256, 256, 2, 4, HAS_ZP, 1>(p, s);   // 8 wavefronts, 128 x 64 each
     case 20: return launch_prefill2<BF16, 256, 256, 2, 4, HAS_ZP, 1, false, true>(p, s);   // the same, alternating phases
-    case 30: return prefill_launch_reg(p, BF16, HAS_ZP, s);                                // 4 wavefronts, 256 x 64 each
     case 11: return launch_prefill2<BF16, 256, 256, 2, 2, HAS_ZP, 1>(p, s);   // 4 wavefronts, 128 x 128 each
     case 12: return launch_prefill2<BF16, 128, 128, 2, 4, HAS_ZP, 1>(p, s);   // 8 wavefronts, 64 x 32 each
     case 13: return launch_prefill2<BF16, 128, 256, 2, 4, HAS_ZP, 1>(p, s);   // 8 wavefronts, 64 x 64 each
@@ -120,12 +118,13 @@ static int pick_register_staged(int M, int N) {
   return tiles(256, 256) >= cus ? 0 : (tiles(128, 128) >= cus ? 1 : 2);
 }
 
-// Tile shape and K split for a problem (the shapes 13, 30, 48 and 66 are built for TILES_PLAIN).
+// Tile shape and K split for a problem (the shapes 13, 48 and 66 are built for TILES_PLAIN; 30, another kernel of the shape 20 in
+// recorded timings, stands for 20).
 static TilePlan make_plan_prefill(int M, int N, int K, TileFormat format) {
   const int64_t cus = num_cus_current_device();
   const int G = K / 128;
   const VaqTuning& tn = tuning();
-  const int forced = tn.prefill_tile - 1;
+  const int forced = tn.prefill_tile == 31 ? 20 : tn.prefill_tile - 1;
   const bool plain = format == TILES_PLAIN || format == TILES_PLAIN_STAGED;
   const TilePrices prices = tile_prices(format);
   const double weight_bytes = prices.weight_bytes * N * K;
@@ -136,7 +135,7 @@ static TilePlan make_plan_prefill(int M, int N, int K, TileFormat format) {
     TileShape t = *shape;
     if (t.id == 41 && format == TILES_8BIT_SUB) t.slots = 1;      // (132 .. 147 registers)
     const bool is256 = t.id == 20 || t.id == 48;
-    if (forced >= 0 ? forced != t.id && !(t.id == 20 && (forced == 10 || forced == 11 || forced == 30)) : (t.id == 13 || t.id == 48 || t.id == 66) && !plain) continue;
+    if (forced >= 0 ? forced != t.id && !(t.id == 20 && (forced == 10 || forced == 11)) : (t.id == 13 || t.id == 48 || t.id == 66) && !plain) continue;
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
     const int64_t rest = tiles % cus;
     auto consider = [&](int sk, int64_t tail_first) {
@@ -161,13 +160,7 @@ static TilePlan make_plan_prefill(int M, int N, int K, TileFormat format) {
   }
   if (forced >= 0 && best.id >= 0) {
     best.id = forced;
-    if (forced == 11 || forced == 30) best.nw = 4;
-  } else if (best.id == 20 && best.sk == 1 && plain && K >= 4096 && best.tiles * 5 >= cus * 4) {
-    // Whole 256 x 256 tiles on most of the device and a long K: dequantised in registers (four wavefronts of 256 x 64), 2 % ahead
-    // of the eight wavefronts with alternating phases; on a short K, with fewer tiles or with a split K 1-7 % behind.  (The strip tile
-    // 48 is priced ahead of both wherever this would hold up to M = 8192: 4096 x 28672 at M = 4096 776 -> 771 us.)
-    best.id = 30;
-    best.nw = 4;
+    if (forced == 11) best.nw = 4;
   }
   return best;
 }
@@ -247,8 +240,8 @@ int w4a16_prefill_launch(const void* a, int64_t lda, const int32_t* b, const voi
   p.tail_first = (int)pl.tail_first;
   const bool bf16 = dtype == VAQ_BF16, zp = zeros != nullptr;
   int rc;
-  // the alternating-phase and the register-dequantising variants exist for 4-bit codes in groups of 128 rows / channelwise
-  const int tile_other = (pl.id == 20 || pl.id == 30) ? 10 : pl.id;
+  // the alternating-phase variant exists for 4-bit codes in groups of 128 rows / channelwise
+  const int tile_other = pl.id == 20 ? 10 : pl.id;
   if (pl.id > 40) {
     if (w8) rc = prefill_launch_strip_w8(p, sub, pl.id, bf16, s);
     else if (sub > 1) rc = prefill_launch_strip_sub(p, sub, pl.id, bf16, zp, s);
