@@ -52,8 +52,8 @@ def test_strip_tiles(device, bits, group_size, asym, dtype):
         a, hot = a.to(device), hot.to(device)
         for tile in EVERY_FORMAT + (PLAIN_ONLY if bits == 4 and group_size in (128, -1) else ()):
             what = f"tile {tile} g={group_size} bits={bits} k={k} n={n} m={m}"
-            assert torch.equal(_forced(layer, hot, tile, 1).cpu(), w[rows]), what
             for split in (1, 2, 3):
+                assert torch.equal(_forced(layer, hot, tile, split).cpu(), w[rows]), f"{what} split {split}"
                 out = _forced(layer, a, tile, split)
                 check_gemm_close(out, ref, f"{what} split {split}")
                 assert torch.equal(out, _forced(layer, a, tile, split)), f"{what} split {split}: not deterministic"
@@ -106,6 +106,23 @@ def test_strip_tiles_bias_strided_rows_and_unaligned_output(device):
                 check_gemm_close(buf[4:4 + m * n].view(m, n), ref, f"tile {tile} split {split} k={k} n={n} m={m}")
                 assert bool((buf[:4] == 0).all()) and bool((buf[4 + m * n:] == 0).all()), "stores outside the output"
         assert bool((counters == 0).all())
+
+
+def test_strip_tiles_rows_almost_4_gib_apart(device):
+    """Activations whose last row ends just below the 4 GiB that 32-bit offsets reach; everything between the rows and behind them is
+    NaN, so that no request lands there unseen."""
+    k, n, m, pitch = 1408, 320, 127, 1 << 24
+    assert (m * pitch * 2) < 1 << 32 < ((m + 1) * pitch * 2) + 1
+    base = torch.full(((m + 13) * pitch,), float("nan"), dtype=torch.bfloat16, device=device)
+    a = base[:m * pitch].view(m, pitch)[:, :k]
+    a.copy_(_acts(m, k, seed=4))
+    for bits, group_size in ((4, 128), (8, 64)):
+        case = o.make_w4a16_case(k, n, group_size, asym=bits == 4, seed=n, num_bits=bits)
+        layer = W4A16Layer(case, device)
+        want = [_forced(layer, a.contiguous(), tile, 2) for tile in EVERY_FORMAT]
+        check_gemm_close(want[0], o.gemm_ref(a.cpu(), o.case_w_ref(case)), f"bits={bits}")
+        for tile, ref in zip(EVERY_FORMAT, want):
+            assert torch.equal(_forced(layer, a, tile, 2), ref), f"tile {tile} bits={bits}"
 
 
 def test_strip_tiles_of_last_round_split(device):
