@@ -63,8 +63,8 @@ inline void consider_tile_plan(TilePlan& best, const TileShape& t, const TileCos
 }
 
 // A small table of finished plans, one per thread, replaced on collision: weighing the plans of a problem takes 2 us of host
-// time.  (Calls that force a part of the plan neither read nor fill it; 256 entries: a call asks for up to six plans of its shape, and in
-// 64 those of a model's four shapes already replaced one another.)
+// time.  (Calls that force a part of the plan neither read nor fill it.)  The key's low bits, and those from bit 18 on, move the
+// entry: a call that asks for the plans of several formats or kernels of its problem never has them replace one another.
 template <class Plan>
 struct PlanTable {
   struct Entry {
@@ -74,7 +74,8 @@ struct PlanTable {
   Entry entry[256];
   template <class Make>
   const Plan& get(int m, int n, int k, int key, Make make) {
-    Entry& e = entry[((uint32_t)m * 2654435761u ^ (uint32_t)n * 2246822519u ^ (uint32_t)k * 3266489917u ^ (uint32_t)key * 668265263u) >> 24];
+    const uint32_t at = ((uint32_t)m * 2654435761u ^ (uint32_t)n * 2246822519u ^ (uint32_t)k * 3266489917u) >> 24;
+    Entry& e = entry[(at + (uint32_t)key + 8u * ((uint32_t)key >> 18)) & 255];
     if (e.m != m || e.n != n || e.k != k || e.key != key) {
       e.plan = make();
       e.m = m; e.n = n; e.k = k; e.key = key;

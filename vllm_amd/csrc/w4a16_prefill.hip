@@ -178,7 +178,7 @@ static TilePlan plan_prefill(int M, int N, int K, bool direct_ok, TileFormat for
   constexpr int KIB_MAX = 1 << 15;
   static thread_local TilePlanTable table;
   if (forced >= 0 || tn.prefill_split > 0 || tn.exp[6] > 1 || tn.exp[14] < 0 || tn.exp[14] >= KIB_MAX) return make_plan_prefill(M, N, K, format);
-  const int key = ((num_cus_current_device() * 8 + format) * 2 + (tn.exp[10] == 1 ? 1 : 0)) * KIB_MAX + tn.exp[14];
+  const int key = ((num_cus_current_device() * 2 + (tn.exp[10] == 1 ? 1 : 0)) * KIB_MAX + tn.exp[14]) * 8 + format;
   return table.get(M, N, K, key, [&] { return make_plan_prefill(M, N, K, format); });
 }
 
