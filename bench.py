@@ -733,6 +733,15 @@ def medium_m_section(dev):
     return rows
 
 
+def w4a16_tile_kernel(m, n, k):
+    """The tile kernel that a problem in groups of 128 rows takes, from the library's plan of it."""
+    import ctypes
+    from vllm_amd import _lib
+    plan = (ctypes.c_double * 4)()
+    _lib.check(_lib.load().vaq_w4a16_tile_plan(m, n, k, 1, 0, 0, 0, plan))
+    return "vaq::w4a16_strip_kernel" if plan[0] > 40 else "vaq::w4a16_prefill2_kernel"
+
+
 def roofline_mfma(extra):
     """The compute-bound kernels against the dense MFMA peaks, from the M = 4096 rows of the prefill and FP8 sections
     (HIP-graph timings of this run): per kernel the FLOPs of one launch, its average duration, the fraction of peak and,
@@ -741,7 +750,7 @@ def roofline_mfma(extra):
     out = []
     for r in extra.get("prefill", []):
         if r["M"] == 4096 and r["kind"].endswith("groups"):
-            row = dict(kernel="vaq::w4a16_strip_kernel", K=r["K"], N=r["N"], M=r["M"], flops_per_launch=2.0 * r["M"] * r["N"] * r["K"],
+            row = dict(kernel=w4a16_tile_kernel(r["M"], r["N"], r["K"]), K=r["K"], N=r["N"], M=r["M"], flops_per_launch=2.0 * r["M"] * r["N"] * r["K"],
                        avg_ns=round(r["us"] * 1e3), peak_TFLOPs=BF16_PEAK_TFLOPS, frac=round(r["mfma_frac"], 4))
             v = vendor.get(("vendor_bf16_matmul", r["K"], r["N"]))
             if v:

@@ -9,8 +9,8 @@ Runs on the GPU; the *.csv.gz beside it are what it wrote on an MI355X.  A probl
     fp8_tile, w4_tile (4-bit codes in groups of 128 rows with zero points), w8_tile (8-bit codes), and both in groups of 64 / 32 rows,
     z with zero points:  k, n, m, tile id, parts of K, 1 if only the tiles of the last round are in parts, us
     w4_decode:          k, n, m, groups of 128 rows (1, 2, 4), 8-bit codes, kind, gs, wks, wn (0: by the planner), us
-                        kind 0 workgroups of all rows, 1 of 16 rows, 2 the tile kernel by its own plan (gs, wks, wn 0; recorded
-                        with the shapes up to 20 only, at whose price the decode kernels are weighed)
+                        kind 0 workgroups of all rows, 1 of 16 rows, 2 the tile kernel by the plan of the shapes with weights
+                        through LDS (gs, wks, wn 0), at whose price the decode kernels are weighed
 """
 from __future__ import annotations
 
@@ -222,7 +222,12 @@ def scan_decode(lib, rng, until, out):
         if not layer.fits():
             continue
         for m in rows:
-            us = layer.time(lib, m, path=2) if m > 16 else None
+            us = None
+            if m > 16:      # (the plan whose price the decode kernels are weighed against, not the strips that may take its place)
+                plan = (ctypes.c_double * 4)()
+                lib.vaq_w4a16_tile_plan(m, n, k, 128 // group, int(bits == 8), 0, 1, plan)
+                ident, sk, tail = int(plan[0]), int(plan[1]), plan[2] > 0
+                us = layer.time(lib, m, path=2, prefill_tile=ident + 1, prefill_split=0 if tail else sk, exp={6: sk} if tail else {10: 1})
             if us is not None:
                 print(k, n, m, 128 // group, int(bits == 8), 2, 0, 0, 0, f"{us:.2f}", sep=",", file=out)
             for split, gs, wks, nt in decode_plans(k, n, m, group, bits):

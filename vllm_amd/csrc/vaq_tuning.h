@@ -74,6 +74,13 @@ int vaq_fp8_quant_per_token_tuned(const void* in, int in_dtype, int64_t in_row_s
  */
 int vaq_w4a16_decode_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub, int w8, int kind, double* plan);
 
+/*
+ * The same of the W4A16 tile kernels: plan[0 .. 3] = tile id (41 and above: strips), parts of K, first tile that is split where only
+ * those of the last round are (else 0), predicted us.  `wt` = 0 4-bit, 1 8-bit codes, 2 FP8 weights; `staged` = 1: the cheapest plan
+ * of the shapes with weights through LDS, whose price the decode kernels are weighed against.
+ */
+int vaq_w4a16_tile_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub, int wt, int zero_points, int staged, double* plan);
+
 #pragma GCC visibility pop
 #ifdef __cplusplus
 }

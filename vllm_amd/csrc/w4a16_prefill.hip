@@ -257,3 +257,15 @@ int w4a16_prefill_launch(const void* a, int64_t lda, const int32_t* b, const voi
 }
 
 }  // namespace vaq
+
+extern "C" int vaq_w4a16_tile_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub, int wt, int zero_points, int staged, double* plan) {
+  using namespace vaq;
+  VAQ_CHECK_ARG(size_m > 0 && size_m < (1ll << 31) && size_n > 0 && size_n % 64 == 0 && size_n < (1 << 24) && size_k > 0 &&
+                    size_k % 128 == 0 && size_k < (1 << 24) && (sub == 1 || sub == 2 || sub == 4) && wt >= 0 && wt <= 2 && plan != nullptr,
+                "w4a16_tile_plan: bad arguments");
+  const TileFormat format = staged ? (sub == 1 && wt == 0 ? TILES_PLAIN_STAGED : TILES_FP8) : tile_format(sub, wt, zero_points != 0);
+  const TilePlan pl = plan_prefill((int)size_m, (int)size_n, (int)size_k, true, format);
+  const double out[4] = {(double)pl.id, (double)pl.sk, (double)pl.tail_first, pl.us};
+  for (int i = 0; i < 4; ++i) plan[i] = out[i];
+  return VAQ_OK;
+}
