@@ -85,19 +85,37 @@ static __device__ inline v4u scale_bytes(uint32_t t, uint32_t u, float s, float 
   return r;
 }
 
+// Register t (0..3) of scale_bytes' result: elements 2t and 2t+1.
+template <bool BF16>
+static __device__ inline uint32_t scale_bytes_part(uint32_t tb, uint32_t ub, float s, float neg_zs, int t) {
+  const uint32_t x = (t & 1) ? ub : tb;
+  float l, h;
+  if (t >> 1) {
+    l = cvt_ubyte<1>(x);
+    h = cvt_ubyte<3>(x);
+  } else {
+    l = cvt_ubyte<0>(x);
+    h = cvt_ubyte<2>(x);
+  }
+  return pack2<BF16>(fmaf(l, s, neg_zs), fmaf(h, s, neg_zs));
+}
+
 // Register t (0..3), elements 2t and 2t+1, of the 8 scaled 16-bit weights of one native word (8 4-bit codes of 8 consecutive k).
 // A byte 0 .. 15 read as e4m3 is byte * 2^-9 (0 .. 7 are its subnormals, 8 .. 15 its first binade), so the packed FP8 conversion
-// turns two codes into two floats at once: 19 instructions per word where a conversion per code takes 23.
+// turns two codes into two floats at once: 19 instructions per word where a conversion per code takes 23.  But it needs registers in
+// pairs: BYTES converts code by code, the same bits, for where there are none to spare.
 // nibble positions 0,2,4,6 hold elements 0,4,1,5; nibble positions 1,3,5,7 hold elements 2,6,3,7
-template <bool BF16>
+template <bool BF16, bool BYTES = false>
 static __device__ inline uint32_t dequant_part(uint32_t w, float s, float neg_zs, int t) {
+  if constexpr (BYTES) return scale_bytes_part<BF16>(w & 0x0f0f0f0fu, (w >> 4) & 0x0f0f0f0fu, s, neg_zs, t);
   typedef float v2f __attribute__((ext_vector_type(2)));
   const uint32_t x = (t & 1) ? (w >> 4) & 0x0f0f0f0fu : w & 0x0f0f0f0fu;
   const v2f lo = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(x, 512.0f, false), hi = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(x, 512.0f, true);
   return pack2<BF16>(fmaf(lo[t >> 1], s, neg_zs), fmaf(hi[t >> 1], s, neg_zs));
 }
-template <bool BF16>
+template <bool BF16, bool BYTES = false>
 static __device__ inline v4u dequant_scaled(uint32_t w, float s, float neg_zs) {
+  if constexpr (BYTES) return scale_bytes<BF16>(w & 0x0f0f0f0fu, (w >> 4) & 0x0f0f0f0fu, s, neg_zs);
   v4u r;
 #pragma unroll
   for (int t = 0; t < 4; ++t) r[t] = dequant_part<BF16>(w, s, neg_zs, t);
@@ -132,21 +150,6 @@ static __device__ inline v4u dequant_fp8(uint32_t wa, uint32_t wb, float s) {
 template <bool BF16>
 static __device__ inline uint32_t dequant_fp8_part(uint32_t wa, uint32_t wb, float s, int t) {
   return fp8_pair_scaled<BF16>((t >> 1) ? wb : wa, (t & 1) != 0, s);
-}
-
-// Register t (0..3) of scale_bytes' result: elements 2t and 2t+1.
-template <bool BF16>
-static __device__ inline uint32_t scale_bytes_part(uint32_t tb, uint32_t ub, float s, float neg_zs, int t) {
-  const uint32_t x = (t & 1) ? ub : tb;
-  float l, h;
-  if (t >> 1) {
-    l = cvt_ubyte<1>(x);
-    h = cvt_ubyte<3>(x);
-  } else {
-    l = cvt_ubyte<0>(x);
-    h = cvt_ubyte<2>(x);
-  }
-  return pack2<BF16>(fmaf(l, s, neg_zs), fmaf(h, s, neg_zs));
 }
 
 template <bool BF16>
@@ -531,6 +534,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void w4a16_prefill2_kernel(
   float scur[W_LD][SUBG];
   ZT zcur[W_LD];
   constexpr bool HP = !BF16 && !W8 && SUBG == 1;      // packed fp16 dequantisation (see dequant_pair_h)
+  constexpr bool BYTES = SUBG == 4 && HAS_ZP && BM * BN == 256 * 256;      // (packed conversions spill 11 registers here instead of 5)
   uint32_t s2cur[HP ? W_LD : 1], nzb2cur[HP ? W_LD : 1];
   // the next group's scales and zero-point words as loaded; converted in advance_w, a K step after the request (a
   // conversion next to the load makes the wavefront wait for the memory latency in the middle of the step)
@@ -603,7 +607,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void w4a16_prefill2_kernel(
       if constexpr (F8) dv = dequant_fp8<BF16>(which ? wcur[i].z : wcur[i].x, which ? wcur[i].w : wcur[i].y, sv);      // block 0: words of j = 0, 1
       else if constexpr (W8) dv = dequant_scaled8<BF16>(wsel, which ? wcur_lo[i].y : wcur_lo[i].x, sv, zv);
       else if constexpr (HP) dv = dequant_scaled_h(wsel, s2cur[i], nzb2cur[i]);
-      else dv = dequant_scaled<BF16>(wsel, sv, zv);
+      else dv = dequant_scaled<BF16, BYTES>(wsel, sv, zv);
       *reinterpret_cast<v4u*>(Bb + (row >> 1) * 256 + ((c0 ^ sw) * 16)) = dv;
     }
   };
@@ -703,9 +707,9 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void w4a16_prefill2_kernel(
               if constexpr (SUB == 4) dq[slot][t] = dequant_pair_h(wsel, s2cur[i], nzb2cur[i], t);
               else dq[slot] = dequant_scaled_h(wsel, s2cur[i], nzb2cur[i]);
             } else if constexpr (SUB == 4) {
-              dq[slot][t] = dequant_part<BF16>(wsel, sv, zv, t);
+              dq[slot][t] = dequant_part<BF16, BYTES>(wsel, sv, zv, t);
             } else {
-              dq[slot] = dequant_scaled<BF16>(wsel, sv, zv);
+              dq[slot] = dequant_scaled<BF16, BYTES>(wsel, sv, zv);
             }
             if (t == SUB - 1) {
               const int row = (i * NW + wave) * 16 + r;
