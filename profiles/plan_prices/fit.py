@@ -1,7 +1,7 @@
 """Fits the price formulas of the tile kernels and of the W4A16 decode kernel to the timings of scan.py, and says how good
 the plans are that they choose.
 
-    python profiles/plan_prices/fit.py fp8_tile|w4_tile|w4sub_tile|w4sub32zp_tile|w8_tile|w8sub_tile|w4_decode TIMINGS.csv[.gz] [...] [--fit]
+    python profiles/plan_prices/fit.py fp8_tile|w4_tile|w4sub_tile|w8_tile|w8sub_tile|w4_decode TIMINGS.csv[.gz] [...] [--fit]
 
 Without --fit: the constants of the sources, read from them.  The formulas are those of `tile_plan_us` in
 vllm_amd/csrc/tile_plan.h and `decode2_us` in vllm_amd/csrc/w4a16_decode2.hip.

@@ -1,13 +1,13 @@
 """Times every plan of random problems, for the price formulas that choose among them (fit.py).
 
-    python profiles/plan_prices/scan.py fp8_tile|w4_tile|w8_tile|w4g64z_tile|w4g32_tile|w4g32z_tile|w8g64_tile|w8g32_tile|w4_decode SECONDS SEED OUT.csv
+    python profiles/plan_prices/scan.py fp8_tile|w4_tile|w8_tile|w4g64z_tile|w4g32_tile|w4g32z_tile|w4g32zh_tile|w8g64_tile|w8g32_tile|w4_decode SECONDS SEED OUT.csv
 
 Runs on the GPU; the *.csv.gz beside it are what it wrote on an MI355X.  A problem is a layer (K, N) and a number of rows; a plan is forced through the `_tuned` entry points
 (vllm_amd/csrc/vaq_tuning.h).  Weights are cold: a graph of launches walks over copies of the layer (640 MB of them, at most
 400).  One line per plan, with the time of a launch in us:
 
     fp8_tile, w4_tile (4-bit codes in groups of 128 rows with zero points), w8_tile (8-bit codes), and both in groups of 64 / 32 rows,
-    z with zero points:  k, n, m, tile id, parts of K, 1 if only the tiles of the last round are in parts, us
+    z with zero points, h fp16 instead of bf16:  k, n, m, tile id, parts of K, 1 if only the tiles of the last round are in parts, us
     w4_decode:          k, n, m, groups of 128 rows (1, 2, 4), 8-bit codes, kind, gs, wks, wn (0: by the planner), us
                         kind 0 workgroups of all rows, 1 of 16 rows, 2 the tile kernel by the plan of the shapes with weights
                         through LDS (gs, wks, wn 0), at whose price the decode kernels are weighed
@@ -33,7 +33,8 @@ class Layer:
     """Operands of one layer: views of one pool of random bytes (finite e4m3 codes) and of one of scales."""
     pool = scales = None
 
-    def __init__(self, fp8: bool, k: int, n: int, most_m: int, bits: int = 4, group: int = 128, zeros: bool | None = None):
+    def __init__(self, fp8: bool, k: int, n: int, most_m: int, bits: int = 4, group: int = 128, zeros: bool | None = None,
+                 dtype: torch.dtype = torch.bfloat16):
         if Layer.pool is None:
             p = torch.randint(0, 256, (1_500_000_000,), dtype=torch.uint8, device="cuda")
             Layer.pool = torch.where((p & 0x7f) == 0x7f, p ^ 1, p)
@@ -42,10 +43,11 @@ class Layer:
         self.zeros = bits == 4 and group == 128 if zeros is None else zeros      # uint4 with zero points, else uint4b8
         self.bytes = k * n if fp8 else k * n * bits // 8
         self.copies = max(2, min(MOST_COPIES, POOL // self.bytes))
-        x = torch.randn(most_m, k, device="cuda", dtype=torch.bfloat16)
+        self.tag = _lib.VAQ_F16 if dtype == torch.float16 else _lib.VAQ_BF16
+        x = torch.randn(most_m, k, device="cuda", dtype=dtype)
         self.a = x.to(torch.float8_e4m3fn) if fp8 else x
         self.sa, self.sb = torch.rand(most_m, device="cuda"), torch.rand(n, device="cuda")
-        self.out = torch.empty(most_m, n, device="cuda", dtype=torch.bfloat16)
+        self.out = torch.empty(most_m, n, device="cuda", dtype=dtype)
         self.counters = torch.zeros(1 << 20, dtype=torch.int32, device="cuda")
         self.tmp = torch.empty(1 << 20, device="cuda")
 
@@ -66,7 +68,7 @@ class Layer:
         z = self.pool.data_ptr() + self.pool.numel() - (c + 1) * (scale_count // 2) // 64 * 64 - scale_count if self.zeros else None
         return lib.vaq_w4a16_gemm_tuned(
             self.a.data_ptr(), self.k, w, self.scales.data_ptr() + 2 * at, z, None, None, self.out.data_ptr(), tmp, tmp_bytes, None,
-            self.counters.data_ptr(), self.counters.numel(), m, self.n, self.k, self.group, _lib.VAQ_BF16, wtype, path, stream, tune)
+            self.counters.data_ptr(), self.counters.numel(), m, self.n, self.k, self.group, self.tag, wtype, path, stream, tune)
 
     def scratch(self, lib, m, tune) -> bool:
         t, a, n = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_size_t()
@@ -140,7 +142,9 @@ TILES = {"fp8_tile": {13: (128, 128), 14: (64, 128), 15: (64, 64), 16: (128, 64)
                      48: (256, 256)},
          "w8_tile": {12: (128, 128), 14: (64, 128), 15: (128, 64), 16: (256, 128), 20: (256, 256), 41: (32, 128), 51: (32, 64), 42: (64, 128),
                      52: (64, 64), 43: (96, 128), 44: (128, 128), 46: (128, 256)}}
-FORMATS_OF = {"w4_tile": (4, 128, True), "w8_tile": (8, 128, False)}      # bits, rows of a group, zero points
+FORMATS_OF = {"w4_tile": (4, 128, True), "w8_tile": (8, 128, False),      # bits, rows of a group, zero points, activations
+              "w4g32zh_tile": (4, 32, True, torch.float16)}
+TILES["w4g32zh_tile"] = TILES["w8_tile"]
 for _bits in (4, 8):
     for _group in (64, 32):
         for _zeros in ("", "z") if _bits == 4 else ("",):
@@ -225,7 +229,7 @@ def scan_decode(lib, rng, until, out):
             us = None
             if m > 16:      # (the plan whose price the decode kernels are weighed against, not the strips that may take its place)
                 plan = (ctypes.c_double * 4)()
-                lib.vaq_w4a16_tile_plan(m, n, k, 128 // group, int(bits == 8), 0, 1, plan)
+                lib.vaq_w4a16_tile_plan(m, n, k, 128 // group, int(bits == 8), 1, plan)
                 ident, sk, tail = int(plan[0]), int(plan[1]), plan[2] > 0
                 us = layer.time(lib, m, path=2, prefill_tile=ident + 1, prefill_split=0 if tail else sk, exp={6: sk} if tail else {10: 1})
             if us is not None:

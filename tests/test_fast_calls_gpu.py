@@ -47,18 +47,32 @@ def test_w4_layer_equals_the_registered_op(device, shape, group, dtype, bias):
 
 
 def test_w4_scratch_is_that_of_the_layers_own_format(device):
-    """Two formats of one shape in turn, of which one needs scratch for its K split and the other none: neither takes the other's
-    size from the caches of either route, and the second allocates its output only."""
-    plain, grouped = _w4(device, 2048, 512, 128, torch.bfloat16, False), _w4(device, 2048, 512, 32, torch.bfloat16, False)
-    x = torch.randn(40, 2048, device=device).to(torch.bfloat16)
-    for _ in range(2):
-        for layer in (grouped, plain):
-            assert torch.equal(layer(x), _registered(layer, x))
-    for call in (lambda: grouped(x), lambda: _registered(grouped, x)):
-        torch.cuda.reset_peak_memory_stats(device)
-        before = torch.cuda.memory_allocated(device)
-        out = call()
-        assert torch.cuda.max_memory_allocated(device) - before == out.numel() * 2
+    """Two formats of one shape in turn that need different scratch for their K split: neither takes the other's size from the caches
+    of either route, and a call allocates its output and the scratch of its own format, not that of any."""
+    import ctypes
+    from vllm_amd import _lib
+    lib = _lib.load()
+    layers = {g: _w4(device, 2048, 512, g, torch.bfloat16, False) for g in (128, 32)}
+    smaller = 0
+    for m in (33, 40, 48, 70, 100, 150):
+        x = torch.randn(m, 2048, device=device).to(torch.bfloat16)
+        sizes = [ctypes.c_size_t() for _ in range(3)]
+        _lib.check(lib.vaq_w4a16_gemm_workspace(m, 512, 2048, 0, 0, *map(ctypes.byref, sizes)))
+        every = sizes[0].value
+        for _ in range(2):
+            for layer in layers.values():
+                assert torch.equal(layer(x), _registered(layer, x))
+        for group, layer in layers.items():
+            _lib.check(lib.vaq_w4a16_gemm_workspace_of_format(m, 512, 2048, group, _lib.VAQ_WTYPE_U4B8, 0, 0, *map(ctypes.byref, sizes)))
+            own = sizes[0].value
+            smaller += own < every
+            for call in (lambda: layer(x), lambda: _registered(layer, x)):
+                torch.cuda.reset_peak_memory_stats(device)
+                before = torch.cuda.memory_allocated(device)
+                out = call()
+                assert torch.cuda.max_memory_allocated(device) - before == sum((n + 511) // 512 * 512 for n in (out.numel() * 2, own))
+                del out
+    assert smaller > 3
 
 
 @pytest.mark.parametrize("shape", [(1, 256), (67, 256), (2, 5, 256)])

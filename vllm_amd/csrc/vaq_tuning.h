@@ -79,7 +79,7 @@ int vaq_w4a16_decode_plan(int64_t size_m, int64_t size_n, int64_t size_k, int su
  * those of the last round are (else 0), predicted us.  `wt` = 0 4-bit, 1 8-bit codes, 2 FP8 weights; `staged` = 1: the cheapest plan
  * of the shapes with weights through LDS, whose price the decode kernels are weighed against.
  */
-int vaq_w4a16_tile_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub, int wt, int zero_points, int staged, double* plan);
+int vaq_w4a16_tile_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub, int wt, int staged, double* plan);
 
 #pragma GCC visibility pop
 #ifdef __cplusplus

@@ -47,8 +47,8 @@ static int check_format(int64_t size_k, int group_size, int wtype, int* wt, int*
 
 // Scratch of a problem, enough for whichever kernel runs (that also depends on the row stride of A): for one weight format, or with
 // wt < 0 for any of them.
-static int scratch_of(int64_t size_m, int64_t size_n, int64_t size_k, bool has_perm, int wt, int sub, bool zero_points,
-                      size_t* c_tmp_bytes, size_t* a_tmp_bytes, size_t* counter_ints) {
+static int scratch_of(int64_t size_m, int64_t size_n, int64_t size_k, bool has_perm, int wt, int sub, size_t* c_tmp_bytes,
+                      size_t* a_tmp_bytes, size_t* counter_ints) {
   VAQ_CHECK_ARG(c_tmp_bytes && a_tmp_bytes && counter_ints, "w4a16_gemm_workspace: null output pointer");
   int rc = check_shape(size_m, size_n, size_k);
   if (rc != VAQ_OK) return rc;
@@ -75,8 +75,8 @@ static int scratch_of(int64_t size_m, int64_t size_n, int64_t size_k, bool has_p
     }
   // from 17 rows on the tile kernel where it is ahead
   if (size_m > 16)
-    for (TileFormat format : {TILES_PLAIN, TILES_SUB, TILES_SUB32_ZP, TILES_8BIT, TILES_8BIT_SUB, TILES_FP8}) {
-      if (wt >= 0 && format != tile_format(sub, wt, zero_points)) continue;
+    for (TileFormat format : {TILES_PLAIN, TILES_SUB, TILES_8BIT, TILES_8BIT_SUB, TILES_FP8}) {
+      if (wt >= 0 && format != tile_format(sub, wt)) continue;
       rc = w4a16_prefill_workspace(M, N, K, format, &t, &n);
       if (rc != VAQ_OK) return rc;
       take(t, n);
@@ -96,7 +96,7 @@ extern "C" int vaq_w4a16_gemm_workspace_of_format(int64_t size_m, int64_t size_n
   int rc = check_shape(size_m, size_n, size_k);
   if (rc == VAQ_OK) rc = check_format(size_k, group_size, wtype, &wt, &sub, &channelwise);
   if (rc != VAQ_OK) return rc;
-  return scratch_of(size_m, size_n, size_k, has_perm != 0, wt, sub, wtype == VAQ_WTYPE_U4, c_tmp_bytes, a_tmp_bytes, counter_ints);
+  return scratch_of(size_m, size_n, size_k, has_perm != 0, wt, sub, c_tmp_bytes, a_tmp_bytes, counter_ints);
 }
 
 extern "C" int vaq_w4a16_gemm_workspace(int64_t size_m, int64_t size_n, int64_t size_k, int has_perm, int device,
@@ -111,7 +111,7 @@ extern "C" int vaq_w4a16_gemm_workspace_tuned(int64_t size_m, int64_t size_n, in
   using namespace vaq;
   (void)device;
   const TuningScope scope(tuning_or_null);
-  return scratch_of(size_m, size_n, size_k, has_perm != 0, -1, 0, false, c_tmp_bytes, a_tmp_bytes, counter_ints);
+  return scratch_of(size_m, size_n, size_k, has_perm != 0, -1, 0, c_tmp_bytes, a_tmp_bytes, counter_ints);
 }
 
 extern "C" int vaq_w4a16_gemm(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
@@ -172,7 +172,7 @@ extern "C" int vaq_w4a16_gemm_tuned(const void* a, int64_t lda, const int32_t* b
     bool tile_ok = force_path == 0;
     if (tile_ok && size_m <= DECODE_MAX_M_2BLK) {
       size_t t = 0, n = 0;
-      w4a16_prefill_workspace((int)size_m, (int)size_n, (int)size_k, tile_format(sub, wt, zeros != nullptr), &t, &n);
+      w4a16_prefill_workspace((int)size_m, (int)size_n, (int)size_k, tile_format(sub, wt), &t, &n);
       tile_ok = perm == nullptr && c_tmp_bytes >= (int64_t)t && counter_ints >= (int64_t)n;
     }
     const int kind = w4a16_decode2_choose((int)size_m, (int)size_n, (int)size_k, sub, wt, perm != nullptr, decode, tile_ok || !decode,

@@ -54,31 +54,19 @@ constexpr TileShape W4_TILE_SHAPES[] = {
     {46, 128, 256, 8, 1, 3.64, 0.495, 0.324, 0, 0.0655},      {66, 128, 256, 8, 1, 6.38, 0.566, 0.164, 0, 0.119},
     {48, 256, 256, 8, 1, 8.35, 0.917, 0.387, 0, 0.0423}};
 constexpr TileCosts W4_TILE_COSTS = {0.163, 0.628, 0.63, 0.253, 0.0};
-// Groups of 64 / 32 rows: 1461 such problems (64 rows with zero points, 32 without; 40923 launches).  One workgroup of the shape 42 to a
-// compute unit: its scales of the sub-groups leave no room for a second one in the registers.  In the mean 0.35 % on layers that a fit to the other
-// half had not seen (0.7 %, 1 in 24 problems more than 5 % behind, with the constants above and their two workgroups; now 1 in 55).
+// Groups of 64 / 32 rows: 2744 such problems, 78807 launches (64 rows with zero points, 32 without and with, these in fp16 too).  One workgroup of
+// the shape 42 to a compute unit: its scales of the sub-groups leave no room for a second one in the registers.  In the mean 0.6 % on layers
+// that a fit to the other half had not seen (0.45, 0.3, 0.55 and 1.05 % over the four; with the constants above and their two workgroups
+// 0.7, 0.7, 1.0 and 1.9 %).
 constexpr TileShape W4SUB_TILE_SHAPES[] = {
-    {12, 128, 128, 8, 2, 0.643, 0.603, 0.0848, 0.375, 0.137}, {14, 64, 128, 8, 2, 0, 0.58, 0.022, 0.153, 0.245},
-    {15, 128, 64, 4, 2, 0, 0.56, 0.0135, 0.0977, 0.347},      {16, 256, 128, 8, 1, 2.02, 0.787, 0.185, 0, 0.103},
-    {20, 256, 256, 8, 1, 4.25, 1.32, 0.173, 0, 0.0149},
-    {41, 32, 128, 8, 2, 2.34, 0.207, 0.024, 0.175, 0.142},    {51, 32, 64, 8, 2, 1.45, 0.109, 0.00645, 0.129, 0.581},
-    {42, 64, 128, 8, 1, 2.33, 0.247, 0.0505, 0, 0.0868},      {52, 64, 64, 8, 1, 2.59, 0.145, 0.0213, 0, 0.0736},
-    {43, 96, 128, 8, 1, 2.75, 0.295, 0.0515, 0, 0.222},       {44, 128, 128, 8, 1, 3.07, 0.349, 0.0767, 0, 0.187},
-    {46, 128, 256, 8, 1, 3.71, 0.538, 0.226, 0, 0.0522}};
-constexpr TileCosts W4SUB_TILE_COSTS = {0.146, 0.603, 0.621, 0.25, 0.0};
-// Groups of 32 rows with zero points: four constants more to unpack per word, in the shapes with weights through LDS all in front of a
-// step -- their 256 x 256 tile takes a third longer a step, so that 128 x 256 strips are ahead at thousands of rows, where it is level without zero
-// points.  1770 problems, 51717 launches, two cards 10 % apart; in the mean 0.5 % on layers not seen by the fit (2.8 % with the plain
-// constants: 2047 x 25344 x 11904 1275 us against 1066 with the tiles of before the strips).
-constexpr TileShape W4SUB32ZP_TILE_SHAPES[] = {
-    {12, 128, 128, 8, 2, 0.812, 0.651, 0.0845, 0.408, 0.126}, {14, 64, 128, 8, 2, 0, 0.635, 0.0179, 0.188, 0.283},
-    {15, 128, 64, 4, 2, 0, 0.599, 0.0117, 0.113, 0.383},      {16, 256, 128, 8, 1, 1.92, 0.836, 0.202, 0, 0.114},
-    {20, 256, 256, 8, 1, 3.87, 1.75, 0.291, 0, 0.0175},
-    {41, 32, 128, 8, 2, 2.53, 0.232, 0.0214, 0.204, 0.147},   {51, 32, 64, 8, 2, 1.35, 0.127, 0.00422, 0.143, 0.617},
-    {42, 64, 128, 8, 1, 2.57, 0.261, 0.063, 0, 0.0895},       {52, 64, 64, 8, 1, 2.56, 0.168, 0.0206, 0, 0.0675},
-    {43, 96, 128, 8, 1, 2.61, 0.342, 0.0421, 0, 0.236},       {44, 128, 128, 8, 1, 3.32, 0.386, 0.0619, 0, 0.232},
-    {46, 128, 256, 8, 1, 4.44, 0.61, 0.153, 0, 0.029}};
-constexpr TileCosts W4SUB32ZP_TILE_COSTS = {0.183, 0.531, 0.625, 0.273, 0.0};
+    {12, 128, 128, 8, 2, 0.726, 0.631, 0.0892, 0.392, 0.139}, {14, 64, 128, 8, 2, 0, 0.613, 0.0195, 0.177, 0.269},
+    {15, 128, 64, 4, 2, 0, 0.583, 0.0117, 0.107, 0.358},      {16, 256, 128, 8, 1, 1.95, 0.825, 0.183, 0, 0.11},
+    {20, 256, 256, 8, 1, 4.48, 1.36, 0.12, 0, 0.013},
+    {41, 32, 128, 8, 2, 2.38, 0.236, 0.0194, 0.195, 0.161},   {51, 32, 64, 8, 2, 1.31, 0.124, 0.00437, 0.141, 0.681},
+    {42, 64, 128, 8, 1, 2.47, 0.264, 0.0529, 0, 0.0702},      {52, 64, 64, 8, 1, 2.52, 0.165, 0.0145, 0, 0.067},
+    {43, 96, 128, 8, 1, 2.57, 0.333, 0.0362, 0, 0.257},       {44, 128, 128, 8, 1, 3.05, 0.386, 0.0558, 0, 0.246},
+    {46, 128, 256, 8, 1, 3.85, 0.584, 0.219, 0, 0.0488}};
+constexpr TileCosts W4SUB_TILE_COSTS = {0.131, 0.547, 0.631, 0.274, 0.0};
 // 8-bit codes, whose dequantisation takes longer: fitted to 993 such problems, in the mean 0.7 % over 1216 others (37199 launches, those kept
 // in profiles/plan_prices; 2.4 % with the first constants above).
 // Groups of 64 / 32 rows take them too, but for the slots of the shape 41 (make_plan_prefill): 1755 problems, 49655 launches, 0.5 %.
@@ -105,7 +93,6 @@ struct TilePrices {
 };
 static TilePrices tile_prices(TileFormat format) {
   if (format == TILES_SUB) return {std::begin(W4SUB_TILE_SHAPES), std::end(W4SUB_TILE_SHAPES), W4SUB_TILE_COSTS, 0.5};
-  if (format == TILES_SUB32_ZP) return {std::begin(W4SUB32ZP_TILE_SHAPES), std::end(W4SUB32ZP_TILE_SHAPES), W4SUB32ZP_TILE_COSTS, 0.5};
   if (format == TILES_8BIT || format == TILES_8BIT_SUB) return {std::begin(W8_TILE_SHAPES), std::end(W8_TILE_SHAPES), W8_TILE_COSTS, 1.0};
   if (format == TILES_FP8 || format == TILES_PLAIN_STAGED) return {std::begin(LDS_TILE_SHAPES), std::end(LDS_TILE_SHAPES), LDS_TILE_COSTS, 0.5};
   return {std::begin(W4_TILE_SHAPES), std::end(W4_TILE_SHAPES), W4_TILE_COSTS, 0.5};
@@ -220,7 +207,7 @@ int w4a16_prefill_launch(const void* a, int64_t lda, const int32_t* b, const voi
     set_error("w4a16_gemm(prefill): 8-bit weights with an A of 4 GiB or more are not built");
     return VAQ_ERR_UNSUPPORTED;
   }
-  TilePlan pl = plan_prefill(M, N, K, direct_ok, tile_format(sub, wt, zeros != nullptr));
+  TilePlan pl = plan_prefill(M, N, K, direct_ok, tile_format(sub, wt));
   // A caller that passes no scratch at all gets the unsplit kernel (same result, no K split); scratch that is there but
   // too small is the caller's mistake and is reported, not worked around.
   if (pl.sk > 1 && c_tmp == nullptr && counters == nullptr) pl.sk = 1;
@@ -258,12 +245,12 @@ int w4a16_prefill_launch(const void* a, int64_t lda, const int32_t* b, const voi
 
 }  // namespace vaq
 
-extern "C" int vaq_w4a16_tile_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub, int wt, int zero_points, int staged, double* plan) {
+extern "C" int vaq_w4a16_tile_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub, int wt, int staged, double* plan) {
   using namespace vaq;
   VAQ_CHECK_ARG(size_m > 0 && size_m < (1ll << 31) && size_n > 0 && size_n % 64 == 0 && size_n < (1 << 24) && size_k > 0 &&
                     size_k % 128 == 0 && size_k < (1 << 24) && (sub == 1 || sub == 2 || sub == 4) && wt >= 0 && wt <= 2 && plan != nullptr,
                 "w4a16_tile_plan: bad arguments");
-  const TileFormat format = staged ? (sub == 1 && wt == 0 ? TILES_PLAIN_STAGED : TILES_FP8) : tile_format(sub, wt, zero_points != 0);
+  const TileFormat format = staged ? (sub == 1 && wt == 0 ? TILES_PLAIN_STAGED : TILES_FP8) : tile_format(sub, wt);
   const TilePlan pl = plan_prefill((int)size_m, (int)size_n, (int)size_k, true, format);
   const double out[4] = {(double)pl.id, (double)pl.sk, (double)pl.tail_first, pl.us};
   for (int i = 0; i < 4; ++i) plan[i] = out[i];
