@@ -422,9 +422,12 @@ int w4a16_decode2_choose(int M, int N, int K, int sub, int wt, bool has_perm, bo
     return r.us >= 0 && wgs <= num_cus_current_device() && r.c.wks * r.c.wn >= 8 ? D2_ROWS : D2_WORKGROUP;
   }
   int best = D2_TILE;
-  // (The tile kernel's price is that of 4-bit codes and 2-5 % low at these sizes, 9-13 % with 8-bit codes; the prices of these
-  // workgroups are 3-9 % low.  With these factors the kind chosen is within 0.2 - 0.6 % of the fastest one's time in the mean,
-  // 1.3 % for groups of 64 / 32 rows at 17 .. 32 rows; 6600 problems.  act_order: a launch that permutes the columns first.)
+  // (`tile_us` is the price of the tile shapes with weights through LDS, see w4a16_staged_us, of 4-bit codes: 2-5 % low at these sizes,
+  // 9-13 % with 8-bit codes; the prices of these workgroups are 3-9 % low.  With these factors the kind chosen is, against those shapes,
+  // within 0.2 - 0.6 % of the fastest one's time in the mean, 1.3 % for groups of 64 / 32 rows at 17 .. 32 rows; 6600 problems.  The strips
+  // that run in their place are up to 40 % faster; they take no problem from here because they round the scaled weights to 16 bits.
+  // act_order: a launch that permutes the columns first, at the 4 us that it took before it had few rows spread over the device (2 - 3
+  // now), for the same reason.)
   double us = tile_ok ? tile_us * (!w8 ? 1.04 : M <= 64 ? 1.06 : 1.0) + (has_perm ? 4.0 : 0.0) : -1;
   if (wg_ok) {
     const double t = workgroup_plan(M, N, K, sub, w8).us;
