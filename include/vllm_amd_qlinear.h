@@ -96,7 +96,7 @@ int vaq_w4a16_gemm_workspace(int64_t size_m, int64_t size_n, int64_t size_k, int
 
 /*
  * The same for one weight format (`group_size` and `wtype` as in vaq_w4a16_gemm): what its own kernels need, where the
- * query above covers every format's -- tens of MB more at hundreds to thousands of rows, and five plans instead of one to
+ * query above covers every format's -- tens of MB more at hundreds to thousands of rows, and six plans instead of one to
  * weigh for a new problem.
  */
 int vaq_w4a16_gemm_workspace_of_format(int64_t size_m, int64_t size_n, int64_t size_k, int group_size, int wtype,

@@ -1,7 +1,7 @@
 """Fits the price formulas of the tile kernels and of the W4A16 decode kernel to the timings of scan.py, and says how good
 the plans are that they choose.
 
-    python profiles/plan_prices/fit.py fp8_tile|w4_tile|w4sub_tile|w8_tile|w8sub_tile|w4_decode TIMINGS.csv[.gz] [...] [--fit]
+    python profiles/plan_prices/fit.py fp8_tile|w4_tile|w4sub_tile|w8_tile|w8g64_tile|w8g32_tile|w4_decode TIMINGS.csv[.gz] [...] [--fit]
 
 Without --fit: the constants of the sources, read from them.  The formulas are those of `tile_plan_us` in
 vllm_amd/csrc/tile_plan.h and `decode2_us` in vllm_amd/csrc/w4a16_decode2.hip.
@@ -41,9 +41,9 @@ class Tiles:
         fp8 = kind == "fp8_tile"
         file = "fp8_scaled_mm.hip" if fp8 else "w4a16_prefill.hip"
         prefix = kind.split("_")[0].upper()
-        sub8, prefix = prefix == "W8SUB", "W8" if prefix == "W8SUB" else prefix      # (the table of 8-bit codes, less one slot)
+        g64, prefix = prefix == "W8G64", "W8" if prefix == "W8G64" else prefix      # (the table of 8-bit codes, less one slot)
         rows = np.array(source_table(file, f"{prefix}_TILE_SHAPES")).reshape(-1, 10)
-        if sub8:
+        if g64:
             rows[rows[:, 0] == 41, 4] = 1
         self.ids = rows[:, 0].astype(int)
         self.shape = rows[:, 1:5]                        # bm, bn, nw, slots

@@ -1,6 +1,6 @@
 """Times every plan of random problems, for the price formulas that choose among them (fit.py).
 
-    python profiles/plan_prices/scan.py fp8_tile|w4_tile|w8_tile|w4g64z_tile|w4g32_tile|w4g32z_tile|w4g32zh_tile|w8g64_tile|w8g32_tile|w4_decode SECONDS SEED OUT.csv
+    python profiles/plan_prices/scan.py fp8_tile|w4_tile|w8_tile|w4g64z_tile|w4g32_tile|w4g32z_tile|w4g32zh_tile|w8g64_tile|w8g32_tile|w8g32h_tile|w4_decode SECONDS SEED OUT.csv
 
 Runs on the GPU; the *.csv.gz beside it are what it wrote on an MI355X.  A problem is a layer (K, N) and a number of rows; a plan is forced through the `_tuned` entry points
 (vllm_amd/csrc/vaq_tuning.h).  Weights are cold: a graph of launches walks over copies of the layer (640 MB of them, at most
@@ -143,8 +143,8 @@ TILES = {"fp8_tile": {13: (128, 128), 14: (64, 128), 15: (64, 64), 16: (128, 64)
          "w8_tile": {12: (128, 128), 14: (64, 128), 15: (128, 64), 16: (256, 128), 20: (256, 256), 41: (32, 128), 51: (32, 64), 42: (64, 128),
                      52: (64, 64), 43: (96, 128), 44: (128, 128), 46: (128, 256)}}
 FORMATS_OF = {"w4_tile": (4, 128, True), "w8_tile": (8, 128, False),      # bits, rows of a group, zero points, activations
-              "w4g32zh_tile": (4, 32, True, torch.float16)}
-TILES["w4g32zh_tile"] = TILES["w8_tile"]
+              "w4g32zh_tile": (4, 32, True, torch.float16), "w8g32h_tile": (8, 32, False, torch.float16)}
+TILES["w4g32zh_tile"] = TILES["w8g32h_tile"] = TILES["w8_tile"]
 for _bits in (4, 8):
     for _group in (64, 32):
         for _zeros in ("", "z") if _bits == 4 else ("",):

@@ -75,7 +75,7 @@ static int scratch_of(int64_t size_m, int64_t size_n, int64_t size_k, bool has_p
     }
   // from 17 rows on the tile kernel where it is ahead
   if (size_m > 16)
-    for (TileFormat format : {TILES_PLAIN, TILES_SUB, TILES_8BIT, TILES_8BIT_SUB, TILES_FP8}) {
+    for (TileFormat format : {TILES_PLAIN, TILES_SUB, TILES_8BIT, TILES_8BIT_64, TILES_8BIT_32, TILES_FP8}) {
       if (wt >= 0 && format != tile_format(sub, wt)) continue;
       rc = w4a16_prefill_workspace(M, N, K, format, &t, &n);
       if (rc != VAQ_OK) return rc;

@@ -69,7 +69,7 @@ constexpr TileShape W4SUB_TILE_SHAPES[] = {
 constexpr TileCosts W4SUB_TILE_COSTS = {0.131, 0.547, 0.631, 0.274, 0.0};
 // 8-bit codes, whose dequantisation takes longer: fitted to 993 such problems, in the mean 0.7 % over 1216 others (37199 launches, those kept
 // in profiles/plan_prices; 2.4 % with the first constants above).
-// Groups of 64 / 32 rows take them too, but for the slots of the shape 41 (make_plan_prefill): 1755 problems, 49655 launches, 0.5 %.
+// Groups of 64 rows take them too, but for the slots of the shape 41 (make_plan_prefill): 876 problems, 24724 launches, 0.4 %.
 constexpr TileShape W8_TILE_SHAPES[] = {
     {12, 128, 128, 8, 2, 0.783, 0.635, 0.0684, 0.441, 0.0986}, {14, 64, 128, 8, 2, 0.0101, 0.595, 0.0269, 0.17, 0.261},
     {15, 128, 64, 4, 2, 0.0105, 0.608, 0.0138, 0.106, 0.362},  {16, 256, 128, 8, 1, 1.74, 0.879, 0.156, 0, 0.0659},
@@ -79,6 +79,17 @@ constexpr TileShape W8_TILE_SHAPES[] = {
     {43, 96, 128, 8, 1, 3.07, 0.371, 0.0552, 0, 0.297},        {44, 128, 128, 8, 1, 3.6, 0.421, 0.0724, 0, 0.247},
     {46, 128, 256, 8, 1, 5.19, 0.669, 0.163, 0, 0.0913}};
 constexpr TileCosts W8_TILE_COSTS = {0.176, 0.376, 0.706, 0.291, 0.0};
+// Groups of 32 rows: 1549 such problems, 45867 launches, in bf16 and fp16, whose strips convert code by code here; in the mean 0.6 % on layers
+// that a fit to the other half had not seen (0.45 and 0.8 %; with the constants above 0.55 and 1.55, 1 in 8 fp16 problems more than 5 % behind).
+constexpr TileShape W8G32_TILE_SHAPES[] = {
+    {12, 128, 128, 8, 2, 0.764, 0.714, 0.0825, 0.454, 0.103},  {14, 64, 128, 8, 2, 0.0103, 0.639, 0.0243, 0.232, 0.28},
+    {15, 128, 64, 4, 2, 0.0108, 0.626, 0.0125, 0.155, 0.356},  {16, 256, 128, 8, 1, 2.37, 0.864, 0.185, 0, 0.0685},
+    {20, 256, 256, 8, 1, 4.77, 1.38, 0.191, 0, 0.0156},
+    {41, 32, 128, 8, 1, 2.79, 0.342, 0.0308, 0, 0.108},        {51, 32, 64, 8, 1, 1.09, 0.181, 0.00686, 0, 0.297},
+    {42, 64, 128, 8, 1, 2.97, 0.376, 0.0464, 0, 0.0855},       {52, 64, 64, 8, 1, 2.67, 0.215, 0.0121, 0, 0.0941},
+    {43, 96, 128, 8, 1, 2.53, 0.437, 0.0335, 0, 0.332},        {44, 128, 128, 8, 1, 3.15, 0.51, 0.0439, 0, 0.251},
+    {46, 128, 256, 8, 1, 4.11, 0.838, 0.149, 0, 0.121}};
+constexpr TileCosts W8G32_TILE_COSTS = {0.146, 0.456, 0.643, 0.288, 0.0};
 // The shapes with weights through LDS by themselves, fitted to 815 problems of 4-bit codes: what FP8 weights are built for (but 13),
 // and the price that up to 256 rows are weighed against the decode kernels at (w4a16_staged_us).
 constexpr TileShape LDS_TILE_SHAPES[] = {
@@ -93,7 +104,8 @@ struct TilePrices {
 };
 static TilePrices tile_prices(TileFormat format) {
   if (format == TILES_SUB) return {std::begin(W4SUB_TILE_SHAPES), std::end(W4SUB_TILE_SHAPES), W4SUB_TILE_COSTS, 0.5};
-  if (format == TILES_8BIT || format == TILES_8BIT_SUB) return {std::begin(W8_TILE_SHAPES), std::end(W8_TILE_SHAPES), W8_TILE_COSTS, 1.0};
+  if (format == TILES_8BIT_32) return {std::begin(W8G32_TILE_SHAPES), std::end(W8G32_TILE_SHAPES), W8G32_TILE_COSTS, 1.0};
+  if (format == TILES_8BIT || format == TILES_8BIT_64) return {std::begin(W8_TILE_SHAPES), std::end(W8_TILE_SHAPES), W8_TILE_COSTS, 1.0};
   if (format == TILES_FP8 || format == TILES_PLAIN_STAGED) return {std::begin(LDS_TILE_SHAPES), std::end(LDS_TILE_SHAPES), LDS_TILE_COSTS, 0.5};
   return {std::begin(W4_TILE_SHAPES), std::end(W4_TILE_SHAPES), W4_TILE_COSTS, 0.5};
 }
@@ -120,7 +132,7 @@ static TilePlan make_plan_prefill(int M, int N, int K, TileFormat format) {
   const int64_t most = tn.exp[14] > 0 ? (int64_t)tn.exp[14] * 1024 : (1ll << 32);
   for (const TileShape* shape = prices.begin; shape != prices.end; ++shape) {
     TileShape t = *shape;
-    if (t.id == 41 && format == TILES_8BIT_SUB) t.slots = 1;      // (132 .. 147 registers)
+    if (t.id == 41 && format == TILES_8BIT_64) t.slots = 1;      // (133 registers)
     const bool is256 = t.id == 20 || t.id == 48;
     if (forced >= 0 ? forced != t.id && !(t.id == 20 && (forced == 10 || forced == 11)) : (t.id == 13 || t.id == 48 || t.id == 66) && !plain) continue;
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
