@@ -50,8 +50,10 @@ def test_w4_scratch_is_that_of_the_layers_own_format(device):
     """Two formats of one shape in turn that need different scratch for their K split: neither takes the other's size from the caches
     of either route, and a call allocates its output and the scratch of its own format, not that of any."""
     import ctypes
+    import gc
     from vllm_amd import _lib
     lib = _lib.load()
+    gc.collect()      # a layer and its parameters' loaders refer to each other: one of an earlier test may be freed within a call below
     layers = {g: _w4(device, 2048, 512, g, torch.bfloat16, False) for g in (128, 32)}
     smaller = 0
     for m in (33, 40, 48, 70, 100, 150):
