@@ -742,6 +742,18 @@ def w4a16_tile_kernel(m, n, k):
     return "vaq::w4a16_strip_kernel" if plan[0] > 40 else "vaq::w4a16_prefill2_kernel"
 
 
+def w4a16_decode_kernels(shapes):
+    """The kernels that take the decode GEMMs (m, n, k) in groups of 128 rows, most launches first."""
+    import ctypes
+    from collections import Counter
+    from vllm_amd import _lib
+    plan, names = (ctypes.c_double * 7)(), Counter()
+    for m, n, k in shapes:
+        _lib.check(_lib.load().vaq_w4a16_regs_plan(m, n, k, 1, 0, plan))
+        names["vaq::w4a16_regs_kernel" if plan[6] else "vaq::w4a16_decode2_kernel"] += 1
+    return " + ".join(name for name, _ in names.most_common())
+
+
 def roofline_mfma(extra):
     """The compute-bound kernels against the dense MFMA peaks, from the M = 4096 rows of the prefill and FP8 sections
     (HIP-graph timings of this run): per kernel the FLOPs of one launch, its average duration, the fraction of peak and,
@@ -1032,7 +1044,7 @@ def main():
                                "(14336,4096)} x M in {1,4,16}, group 128, symmetric int4, bf16 act, fp32 acc; one step = "
                                "12 GEMMs in a HIP graph, weights cold (650 MB cycling)",
                    "launches_per_step": launches},
-        "roofline": {"bound": "hbm", "kernel": "vaq::w4a16_decode2_kernel", "achieved": round(value, 2), "peak": HBM_PEAK_GBS,
+        "roofline": {"bound": "hbm", "kernel": w4a16_decode_kernels([(m, n, k) for k, n in LLAMA_SHAPES for m in DECODE_MS]), "achieved": round(value, 2), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(value / HBM_PEAK_GBS, 4),
                      "traffic": int(MEASURED_TRAFFIC_PER_ALGORITHMIC_BYTE * step_bytes / launches),
                      "avg_launch_us": round(sec * 1e6 / launches, 3),

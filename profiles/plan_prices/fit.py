@@ -1,10 +1,10 @@
 """Fits the price formulas of the tile kernels and of the W4A16 decode kernel to the timings of scan.py, and says how good
 the plans are that they choose.
 
-    python profiles/plan_prices/fit.py fp8_tile|w4_tile|w4sub_tile|w8_tile|w8g64_tile|w8g32_tile|w4_decode TIMINGS.csv[.gz] [...] [--fit]
+    python profiles/plan_prices/fit.py fp8_tile|w4_tile|w4sub_tile|w8_tile|w8g64_tile|w8g32_tile|w4_decode|w4_regs TIMINGS.csv[.gz] [...] [--fit]
 
 Without --fit: the constants of the sources, read from them.  The formulas are those of `tile_plan_us` in
-vllm_amd/csrc/tile_plan.h and `decode2_us` in vllm_amd/csrc/w4a16_decode2.hip.
+vllm_amd/csrc/tile_plan.h, `decode2_us` in vllm_amd/csrc/w4a16_decode2.hip and `regs_us` in vllm_amd/csrc/w4a16_regs.hip.
 """
 from __future__ import annotations
 
@@ -292,6 +292,56 @@ class Decode:
         return (self.kind == 2) | (self.by_rule & ~four & ~split & ~((self.kind == 1) & (self.wks * self.wn < 4)))
 
 
+# --------------------------------------------------------------------- W4A16 kernel with activations in registers
+
+class Regs:
+    TABLES = ("W4_4ROWS", "W4", "W4_64", "W4_32", "W8", "W8_64", "W8_32")
+
+    def __init__(self):
+        self.p = np.array([source_table("w4a16_regs.hip", f"REGS_COST_{t}") for t in self.TABLES])      # in the order of RegsCost
+
+    def load(self, files):
+        self.load_rows(np.concatenate([np.loadtxt(f, delimiter=",", ndmin=2) for f in files]))
+
+    def load_rows(self, d):
+        """`other`: the time of what takes each problem without this kernel (nan: not timed)."""
+        key = np.unique(d[:, :7], axis=0, return_inverse=True)[1].ravel()
+        other = np.full(key.max() + 1, np.nan)
+        other[key[d[:, 7] == 0]] = d[d[:, 7] == 0, 11]
+        d, key = d[d[:, 7] > 0], key[d[:, 7] > 0]
+        self.key = np.unique(key, return_inverse=True)[1].ravel()
+        self.other = other[np.unique(key)]
+        self.k, self.n, self.m, self.sub, self.w8, self.zp, self.fp16, self.nw, self.j, self.mb, self.sk = d[:, :11].T.astype(int)
+        self.us = d[:, 11]
+        at = np.where(self.sub == 1, 0, np.where(self.sub == 2, 1, 2))
+        self.table = np.where(self.w8 == 1, 4 + at, np.where((at == 0) & (self.m <= 4), 0, 1 + at))
+
+    def prices(self, p=None):
+        (base, round_, latency, row, tile, tile_mb, kb, mem_mb, last, meet, meet_wave, out, handover, part, part_mb, again, alone, copies,
+         k1024) = (self.p if p is None else p)[self.table].T
+        k, n, m, sub, nw, j, mb, sk = self.k, self.n, self.m, self.sub, self.nw, self.j, self.mb, self.sk
+        planes, mr, rb = 1 + self.w8, np.where((m <= 4) & (mb == 1), 4, 16), -(-m // (16 * mb))
+        registers = 8 * j * planes + 4 * j * mb + 16 * mb + 4 * planes * mb + (4 + sub) * mb + np.where(sub == 4, 65, 45)
+        lds = np.maximum(nw * (mb * mr * 256 + 2 * sub * 256), j * mb * nw * 1024)
+        slots = np.maximum(1, np.minimum(np.clip(512 // registers, 1, 8) * 4 // nw, 160 * 1024 // lds))
+        per_cu = -(-(-(-(n // 16) // j) * rb * sk) // CUS)
+        side, waves = np.minimum(per_cu, slots), np.minimum(per_cu, slots) * nw / 4
+        rounds = np.where(per_cu > slots, per_cu / slots + last * (-(-per_cu // slots) - per_cu / slots), 1.0)
+        tiles = -(-(-(-(k // 128) // sk)) // nw)
+        work = waves * (row * mb * np.where(sub == 4, 2, 1) + j * planes * (tile + tile_mb * mb))
+        work = work * np.where(registers > 256, copies, 1.0) * np.where(waves <= 1, alone, 1.0)
+        moved = kb * side * nw * (mb * mr / 4 + j * planes)
+        each = (latency ** 3 + work ** 3 + moved ** 3) ** (1 / 3) * np.where(k % 1024 == 0, k1024, 1.0)
+        core = rounds * (round_ + tiles * each + j * mb * (meet + meet_wave * side * nw))
+        mem = mem_mb * 0.5e-6 * k * n * planes * (1 + again * (rb - 1))
+        us = base + (core ** 3 + mem ** 3) ** (1 / 3) + out * 2e-6 * m * n
+        return us + (sk > 1) * (handover + sk * (part + part_mb * 4e-6 * rb * 16 * mb * n))
+
+    def allowed(self):
+        units = -(-(self.n // 16) // self.j) * (-(-self.m // (16 * self.mb)))
+        return (self.sk == 1) | ((self.k // 128 // self.sk >= self.nw) & (units < CUS) & (units * self.sk <= 2 * CUS))
+
+
 def show(values, per):
     for i in range(0, len(values), per):
         print("    {" + ", ".join(f"{v:.3g}" for v in values[i:i + per]) + "},")
@@ -299,19 +349,19 @@ def show(values, per):
 
 def main():
     kind, files, refit = sys.argv[1], [a for a in sys.argv[2:] if a != "--fit"], "--fit" in sys.argv
-    t = Decode() if kind == "w4_decode" else Tiles(kind)
+    t = Decode() if kind == "w4_decode" else Regs() if kind == "w4_regs" else Tiles(kind)
     t.load(files)
     size = t.k * t.n
     groups = {"ordinary (K 1024-14336, N <= 28672)": (t.k >= 1024) & (t.k <= 14336) & (t.n >= 1024) & (t.n <= 28672),
               "K > 14336": t.k > 14336, "N > 28672": t.n > 28672, "K < 1024 or N < 1024": (t.k < 1024) | (t.n < 1024),
               "K N < 2^22": size < 2 ** 22, "all": size > 0}
-    if kind != "w4_decode":
+    if kind not in ("w4_decode", "w4_regs"):
         for a, b in ((9, 32), (33, 64), (65, 128), (129, 256), (257, 512), (513, 1024), (1025, 2048), (2049, 8192)):
             groups[f"{a} .. {b} rows"] = (t.m >= a) & (t.m <= b)
     else:
         for sub in (1, 2, 4):
             for w8 in (0, 1):
-                for a, b in ((1, 16), (17, 32), (33, 64), (65, 256)):
+                for a, b in ((1, 4), (5, 16), (17, 32), (33, 64), (65, 256)):
                     groups[f"groups of {128 // sub}, {8 if w8 else 4} bits, {a} .. {b} rows"] = \
                         (t.sub == sub) & (t.w8 == w8) & (t.m >= a) & (t.m <= b)
     if refit and kind == "w4_decode":
@@ -335,6 +385,16 @@ def main():
             for j, name in enumerate(names):
                 t.p[name] = p[22 * j:22 * j + 22]
                 print(name, ", ".join(f"{v:.3g}" for v in t.p[name]))
+    elif refit and kind == "w4_regs":
+        for i, name in enumerate(Regs.TABLES):
+            at = (t.table == i) & t.allowed()
+
+            def prices(p, at=at, i=i):
+                full = t.p.copy()
+                full[i] = p
+                return t.prices(full)[at]
+            t.p[i] = fit(prices, t.p[i], t.us[at], np.unique(t.key[at], return_inverse=True)[1], 0.5)
+            print(name, ", ".join(f"{v:.3g}" for v in t.p[i]))
     elif refit:
         at = t.allowed()
         key = np.unique(t.key[at], return_inverse=True)[1]

@@ -1,6 +1,6 @@
 """Times every plan of random problems, for the price formulas that choose among them (fit.py).
 
-    python profiles/plan_prices/scan.py fp8_tile|w4_tile|w8_tile|w4g64z_tile|w4g32_tile|w4g32z_tile|w4g32zh_tile|w8g64_tile|w8g32_tile|w8g32h_tile|w4_decode SECONDS SEED OUT.csv
+    python profiles/plan_prices/scan.py fp8_tile|w4_tile|w8_tile|w4g64z_tile|w4g32_tile|w4g32z_tile|w4g32zh_tile|w8g64_tile|w8g32_tile|w8g32h_tile|w4_decode|w4_regs SECONDS SEED OUT.csv
 
 Runs on the GPU; the *.csv.gz beside it are what it wrote on an MI355X.  A problem is a layer (K, N) and a number of rows; a plan is forced through the `_tuned` entry points
 (vllm_amd/csrc/vaq_tuning.h).  Weights are cold: a graph of launches walks over copies of the layer (640 MB of them, at most
@@ -11,6 +11,8 @@ Runs on the GPU; the *.csv.gz beside it are what it wrote on an MI355X.  A probl
     w4_decode:          k, n, m, groups of 128 rows (1, 2, 4), 8-bit codes, kind, gs, wks, wn (0: by the planner), us
                         kind 0 workgroups of all rows, 1 of 16 rows, 2 the tile kernel by the plan of the shapes with weights
                         through LDS (gs, wks, wn 0), at whose price the decode kernels are weighed
+    w4_regs:            k, n, m, groups of 128 rows, 8-bit codes, zero points, fp16, wavefronts, n-tiles, m-blocks, parts of K, us: the kernel
+                        with activations in registers; wavefronts 0: what takes the problem without it
 """
 from __future__ import annotations
 
@@ -245,8 +247,52 @@ def scan_decode(lib, rng, until, out):
         out.flush()
 
 
+def regs_plans(rng, k, n, m, sub, w8):
+    """Up to 24 launch shapes and K splits of a problem: those that fill the device most evenly, and some others."""
+    plans = []
+    for mb, nw, j in ((mb, nw, j) for mb in (1, 2, 3) for nw in (4, 8) for j in range(1, 9)):
+        if (mb > 1 and m <= 16 * (mb - 1)) or not ((j <= 4 and not (w8 and sub == 4 and mb * j == 12)) if nw == 8 else 3 <= j <= (6 if w8 else 8)):
+            continue
+        rb = -(-m // (16 * mb))
+        for sk in range(1, 9):
+            units = -(-n // 16 // j) * rb * sk
+            if sk > 1 and (k // 128 // sk < nw or units > 690 or sk * n * rb * mb * 64 > 16 << 20 or n // 16 * rb * mb > max(4096, n // 4)):
+                continue
+            rounds = units / CUS
+            idle = -(-units // CUS) / rounds if rounds < 3 else 1
+            read = k // sk * 32 * mb + j * 16 * k // sk * (1 if w8 else 0.5)
+            plans.append((idle * (1 + 0.15 * rng.random()) * (read * rounds) ** 0.5, nw, j, mb, sk))
+    plans.sort()
+    return [p[1:] for p in plans[:16] + rng.sample(plans[16:], min(8, max(0, len(plans) - 16)))]
+
+
+def scan_regs(lib, rng, until, out):
+    while time.time() < until:
+        k, n = shape(rng, 64, 400_000_000)
+        group, bits = rng.choice(FORMATS + [(128, 4)])
+        zeros, dtype = bits == 4 and rng.random() < 0.5, torch.float16 if rng.random() < 0.33 else torch.bfloat16
+        rows = sorted({log(rng, 1, 200, 1) for _ in range(3)})
+        layer = Layer(False, k, n, max(rows), bits, group, zeros, dtype)
+        if not layer.fits():
+            continue
+        for m in rows:
+            head = (k, n, m, 128 // group, int(bits == 8), int(zeros), int(dtype == torch.float16))
+            us = layer.time(lib, m, exp={8: 1})
+            if us is not None:
+                print(*head, 0, 0, 0, 0, f"{us:.2f}", sep=",", file=out)
+            for nw, j, mb, sk in regs_plans(rng, k, n, m, 128 // group, int(bits == 8)):
+                us = layer.time(lib, m, exp={8: j | mb << 4 | nw << 8 | sk << 12})
+                if us is not None:
+                    print(*head, nw, j, mb, sk, f"{us:.2f}", sep=",", file=out)
+        print("w4_regs", k, n, rows, flush=True)
+        out.flush()
+
+
 if __name__ == "__main__":
     what, seconds, seed, path = sys.argv[1], float(sys.argv[2]), int(sys.argv[3]), sys.argv[4]
     library, numbers, end = _lib.load(), random.Random(seed), time.time() + float(sys.argv[2])
     with open(path, "w") as f:
-        scan_decode(library, numbers, end, f) if what == "w4_decode" else scan_tiles(library, what, numbers, end, f)
+        if what in ("w4_decode", "w4_regs"):
+            (scan_decode if what == "w4_decode" else scan_regs)(library, numbers, end, f)
+        else:
+            scan_tiles(library, what, numbers, end, f)

@@ -44,7 +44,9 @@ typedef struct VaqTuning {
                         /*   per wavefront, 9 = off); [10] = 1 both tile kernels: never split only the tiles of a half-empty last round; */
                         /*   [12] = 1 FP8 tile kernel: every tile starts at the first K step; [13] = 1 FP8 tile kernel: no tile  */
                         /*   row past M; [14] > 0 W4A16 tile kernel: KiB that the partial tiles of a K split may take; [6] > 1 both tile     */
-                        /*   kernels, 256 x 256 tiles: the tiles of the last round in this many parts of K; [8], [9], [11] unused;       */
+                        /*   kernels, 256 x 256 tiles: the tiles of the last round in this many parts of K; [9], [11] unused;            */
+                        /*   [8] W4A16 kernel with activations in registers: 1 never, else its plan, n-tiles | m-blocks << 4 |        */
+                        /*   wavefronts << 8 | parts of K << 12;                                                                     */
                         /*   [7] = 1 LDS-staged decode kernel: n-tiles in launch order, not grouped by XCD             */
 } VaqTuning;
 
@@ -73,6 +75,12 @@ int vaq_fp8_quant_per_token_tuned(const void* in, int in_dtype, int64_t in_row_s
  * rows, `w8` = 8-bit codes, `kind` = 0 workgroups of all rows, 1 the same by the rule instead of the price, 2 of 16 rows.
  */
 int vaq_w4a16_decode_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub, int w8, int kind, double* plan);
+
+/*
+ * The same of the W4A16 kernel with activations in registers: plan[0 .. 6] = n-tiles, m-blocks and wavefronts of a workgroup, parts of K,
+ * predicted us, predicted us of the kernel that takes the problem otherwise, 1 if this one takes it.
+ */
+int vaq_w4a16_regs_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub, int w8, double* plan);
 
 /*
  * The same of the W4A16 tile kernels: plan[0 .. 3] = tile id (41 and above: strips), parts of K, first tile that is split where only

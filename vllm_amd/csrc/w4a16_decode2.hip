@@ -229,6 +229,14 @@ constexpr Decode2Cost D2_COST_SUB_MB2 = {0.772, 0.979, 0.0147, 0.071, 0, 0.218, 
                                          {1.84, 1.84, 1.63}, {0.0643, 0.0643, 0.0498}, {1, 1.08, 1.46}, 0.0313, 0.379, 0.968, 0};
 constexpr Decode2Cost D2_COST_MB34 = {1.97, 1.26, 0.0179, 0.158, 0, 0.0465, 0.224, 0.328, 0.782,
                                       {1.97, 1.97, 0.468}, {0.0886, 0.0886, 0.00497}, {1.72, 1, 1}, 0.107, 0.395, 1.2, 0};
+// 4-bit codes in groups of 128 rows / channelwise by up to 16 rows, whose plan is the rule's: to weigh that against the kernel with activations in
+// registers (up to 4 and 5 .. 16 rows; two m-blocks; 2600 problems of profiles/plan_prices, 5-6 % rms)
+constexpr Decode2Cost D2_COST_4 = {2.27, 0.561, 0.00957, 0.196, 0, 0.000523, 1.17, 0.118, 0.0294,
+                                   {0.0249, 0.0232, 0.834}, {0.0315, 0.0343, 0.028}, {0.93, 1.11, 1.55}, 0.0824, 0.594, 1.15, 0};
+constexpr Decode2Cost D2_COST_16 = {2.34, 0.579, 0.0093, 0.185, 0, 0.00117, 0.907, 0.198, 0.305,
+                                    {0.796, 0.0366, 0.215}, {0.0278, 0.107, 0.105}, {0.372, 1.11, 1.55}, 0.00252, 0.143, 1.36, 0};
+constexpr Decode2Cost D2_COST_MB2 = {2.74, 0.146, 0.0153, 0.13, 0, 0.00417, 0.659, 0.209, 0.283,
+                                     {1.84, 1.84, 0.0436}, {0.0643, 0.0643, 0.0314}, {1.55, 1.08, 1.46}, 0.0769, 0.379, 0.864, 0};
 // the rows split over workgroups (never with a split K)
 constexpr Decode2Cost D2_COST_ROWS_W8 = {1.15, 1.41, 0.013, 0.409, 0.0868, 0.0134, 0, 0, 0,
                                          {0.86, 0.86, 0.411}, {0.0336, 0.0336, 0.0173}, {1.27, 1.51, 2.19}, 0.113, 0.146, 1.2, 2.57};
@@ -240,7 +248,7 @@ constexpr Decode2Cost D2_COST_ROWS = {1.4, 1.16, 0.0093, 0.0946, 0.368, 0.0106, 
 static const Decode2Cost& workgroup_cost(int M, int sub, bool w8) {
   if (w8) return M > 16 ? D2_COST_W8_MB2 : D2_COST_W8;
   if (sub > 1) return M > 16 ? D2_COST_SUB_MB2 : D2_COST_SUB;
-  return D2_COST_MB34;
+  return M > 32 ? D2_COST_MB34 : M > 16 ? D2_COST_MB2 : M > 4 ? D2_COST_16 : D2_COST_4;
 }
 
 static double decode2_us(const Decode2Cost& t, const Decode2Config& c, int M, int N, int K, int sub, bool w8, int MB, int copies) {
@@ -462,6 +470,10 @@ extern "C" int vaq_w4a16_decode_plan(int64_t size_m, int64_t size_n, int64_t siz
 }
 
 namespace vaq {
+
+double w4a16_decode2_us(int M, int N, int K, int sub, bool w8, bool rows) {
+  return (rows ? rows_plan(M, N, K, sub, w8) : workgroup_plan(M, N, K, sub, w8)).us;
+}
 
 int w4a16_decode2_workspace(int M, int N, int K, int sub, bool w8, size_t* c_tmp_bytes, size_t* counter_ints) {
   const Decode2Config c = workgroup_plan(M, N, K, sub, w8).c;

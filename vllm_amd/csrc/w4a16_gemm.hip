@@ -1,4 +1,5 @@
 // C-ABI entry of the W4A16 GEMM: argument validation and the decode / prefill dispatch.
+#include "tile_plan.h"
 #include "w4a16_kernels.h"
 
 #include <mutex>
@@ -45,6 +46,49 @@ static int check_format(int64_t size_k, int group_size, int wtype, int* wt, int*
   return VAQ_OK;
 }
 
+// What takes a problem of up to 256 rows without act_order where the kernel with activations in registers does not, and its predicted time.
+static int other_kind(int M, int N, int K, int sub, int wt, double* us) {
+  const bool w8 = wt != 0, plain = sub == 1 && !w8;
+  int kind = D2_WORKGROUP;
+  if (M > 16) {
+    const int most = !plain ? DECODE_MAX_M_2BLK : N > 8192 ? 48 : DECODE_MAX_M;
+    kind = w4a16_decode2_choose(M, N, K, sub, wt, false, M <= most, true, w4a16_staged_us(M, N, K, plain));
+  }
+  *us = kind == D2_TILE ? w4a16_tile_us(M, N, K, tile_format(sub, wt)) : w4a16_decode2_us(M, N, K, sub, w8, kind == D2_ROWS);
+  return kind;
+}
+
+// Whether the kernel with activations in registers takes a problem: where it is predicted to be ahead of what takes it otherwise by so much that
+// few calls lose.  4-bit codes in groups of 128 rows 15 % up to 4 rows and 13 % up to 32, where the decode kernel's plans by rule are on some
+// layers that much better than priced (14336 x 4096 at M = 4 9.0 us, priced 9.9; this kernel 10.0, priced 8.7), 5 % up to 64 rows and 8 % beyond;
+// in groups of 64 / 32 rows 12 % from 33 rows on, where zero points cost more than priced; all others 5 %.  Over 20254 calls of drawn layers that
+// it took at 5 % where it now asks for 8 and 12, timed both ways afterwards: 0.842 of their time in the mean, 3.9 % more than 3 % slower, 0.5 % more than 10 %.
+static double regs_lead(int M, int sub, int wt) {
+  if (wt != 0) return 0.95;
+  if (sub > 1) return M > 32 ? 0.88 : 0.95;
+  return M <= 4 ? 0.85 : M <= 32 ? 0.87 : M <= 64 ? 0.95 : 0.92;
+}
+bool w4a16_takes_regs(int M, int N, int K, int sub, int wt, double* other) {
+  const TuningScope automatic(nullptr);
+  const double us = w4a16_regs_us(M, N, K, sub, wt);
+  if (us < 0) return false;
+  other_kind(M, N, K, sub, wt, other);
+  return us < *other * regs_lead(M, sub, wt);
+}
+
+// The same for a call, from a table per thread.  A switch that names another kernel or a plan of one keeps it out; exp[8] asks for it.
+static bool regs_chosen(int M, int N, int K, int sub, int wt) {
+  const VaqTuning& tn = tuning();
+  if (M < 1 || M > REGS_MAX_M || N >= (1 << 24) || K >= (1 << 24) || tn.exp[8] == 1) return false;
+  if (tn.exp[8] > 1) return w4a16_regs_us(M, N, K, sub, wt) >= 0;
+  if (tn.decode_impl > 0 || tn.decode2_gs > 0 || tn.decode2_wks > 0 || tn.decode2_wn > 0 || tn.prefill_tile > 0 || tn.prefill_split > 0 ||
+      tn.exp[0] > 0 || tn.exp[1] > 0 || tn.exp[2] > 0 || tn.exp[3] > 0 || tn.exp[5] > 0 || tn.exp[6] > 0)
+    return false;
+  static thread_local PlanTable<int> table;
+  double other;
+  return table.get(M, N, K, (num_cus_current_device() * 8 + sub) * 4 + wt, [&] { return w4a16_takes_regs(M, N, K, sub, wt, &other) ? 1 : 0; }) != 0;
+}
+
 // Scratch of a problem, enough for whichever kernel runs (that also depends on the row stride of A): for one weight format, or with
 // wt < 0 for any of them.
 static int scratch_of(int64_t size_m, int64_t size_n, int64_t size_k, bool has_perm, int wt, int sub, size_t* c_tmp_bytes,
@@ -79,6 +123,12 @@ static int scratch_of(int64_t size_m, int64_t size_n, int64_t size_k, bool has_p
       if (wt >= 0 && format != tile_format(sub, wt)) continue;
       rc = w4a16_prefill_workspace(M, N, K, format, &t, &n);
       if (rc != VAQ_OK) return rc;
+      take(t, n);
+    }
+  for (int s : {1, 2, 4})
+    for (int w : {0, 1}) {
+      if (has_perm || (wt >= 0 && (s != sub || w != wt)) || size_m > REGS_MAX_M || !regs_chosen(M, N, K, s, w)) continue;
+      w4a16_regs_workspace(M, N, K, s, w == 1, &t, &n);
       take(t, n);
     }
   if (has_perm && size_m > DECODE_MAX_M_2BLK) *a_tmp_bytes = (size_t)size_m * (size_t)size_k * 2;
@@ -179,6 +229,15 @@ extern "C" int vaq_w4a16_gemm_tuned(const void* a, int64_t lda, const int32_t* b
                                           w4a16_staged_us((int)size_m, (int)size_n, (int)size_k, !w8 && sub == 1));
     decode = kind != D2_TILE;
     rows = kind == D2_ROWS;
+  }
+  // (a call that brings too little scratch for its parts of K goes where it went without this kernel; so does one whose rows end beyond 2 GiB)
+  if (force_path == 0 && perm == nullptr && size_m <= REGS_MAX_M && size_m * lda * 2 < (1ll << 31) &&
+      regs_chosen((int)size_m, (int)size_n, (int)size_k, sub, wt)) {
+    size_t t = 0, n = 0;
+    w4a16_regs_workspace((int)size_m, (int)size_n, (int)size_k, sub, w8, &t, &n);
+    if ((t == 0 && n == 0) || (c_tmp != nullptr && counters != nullptr && (uintptr_t)c_tmp % 16 == 0 && c_tmp_bytes >= (int64_t)t && counter_ints >= (int64_t)n))
+      return w4a16_regs_launch(a, lda, b, scales, zeros, bias, c, c_tmp, counters, (int)size_m, (int)size_n, (int)size_k, sub, channelwise,
+                               w8, dtype, s);
   }
   if (decode && decode_impl_for(size_m, size_n, lda, sub, w8) == 0)
     return w4a16_decode2_launch(a, lda, b, scales, zeros, perm, bias, c, c_tmp, c_tmp_bytes, counters, counter_ints, (int)size_m,

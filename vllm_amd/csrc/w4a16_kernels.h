@@ -20,11 +20,21 @@ inline TileFormat tile_format(int sub, int wt) {
   if (wt == 1) return sub == 1 ? TILES_8BIT : sub == 2 ? TILES_8BIT_64 : TILES_8BIT_32;
   return wt == 2 ? TILES_FP8 : sub > 1 ? TILES_SUB : TILES_PLAIN;
 }
+double w4a16_decode2_us(int M, int N, int K, int sub, bool w8, bool rows);      // predicted time of the decode kernel's plan
 double w4a16_staged_us(int M, int N, int K, bool plain);
+double w4a16_tile_us(int M, int N, int K, TileFormat format);
 int w4a16_decode2_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
                          const int32_t* perm, const void* bias, void* c, float* c_tmp, int64_t c_tmp_bytes,
                          int32_t* counters, int64_t counter_ints, int M, int N, int K, int sub, bool channelwise,
                          int wt, int dtype, bool rows, hipStream_t s);      // wt: 0 4-bit codes, 1 8-bit codes, 2 FP8 e4m3 bytes
+// The kernel with activations in registers (w4a16_regs.hip), up to REGS_MAX_M rows, no act_order, no FP8 weights: predicted time (negative: it
+// does not take the problem), scratch, launch.
+constexpr int REGS_MAX_M = 256;
+double w4a16_regs_us(int M, int N, int K, int sub, int wt);
+bool w4a16_takes_regs(int M, int N, int K, int sub, int wt, double* other);      // w4a16_gemm.hip; *other: predicted time of what takes it otherwise
+void w4a16_regs_workspace(int M, int N, int K, int sub, bool w8, size_t* c_tmp_bytes, size_t* counter_ints);
+int w4a16_regs_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros, const void* bias, void* c,
+                      float* c_tmp, int32_t* counters, int M, int N, int K, int sub, bool channelwise, bool w8, int dtype, hipStream_t s);
 int w4a16_prefill_workspace(int M, int N, int K, TileFormat format, size_t* c_tmp_bytes, size_t* counter_ints);
 int w4a16_prefill_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
                          const void* bias, void* c, float* c_tmp, int64_t c_tmp_bytes, int32_t* counters,

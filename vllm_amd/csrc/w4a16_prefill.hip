@@ -187,6 +187,8 @@ static TilePlan plan_prefill(int M, int N, int K, bool direct_ok, TileFormat for
 // were strips.
 double w4a16_staged_us(int M, int N, int K, bool plain) { return plan_prefill(M, N, K, true, plain ? TILES_PLAIN_STAGED : TILES_FP8).us; }
 
+double w4a16_tile_us(int M, int N, int K, TileFormat format) { return plan_prefill(M, N, K, true, format).us; }
+
 int w4a16_prefill_workspace(int M, int N, int K, TileFormat format, size_t* c_tmp_bytes, size_t* counter_ints) {
   const TilePlan pl = plan_prefill(M, N, K, true, format);
   *c_tmp_bytes = (size_t)pl.tmp_bytes();

@@ -1,0 +1,353 @@
+// W4A16 GEMM for a few to some dozen rows, weights and activations in registers: C[M,N] = A[M,K] . dequant(B[K,N]) (+bias), the
+// arithmetic of w4a16_decode.hip (codes as exact 16-bit numbers BIAS + code, zero point and group scale in fp32 on the accumulator).
+//
+//  * A wavefront multiplies one k-tile (128 rows of K) of its rows with J neighbouring n-tiles at a time.  What the kernel that stages a
+//    slab of activations once per workgroup (w4a16_decode2_kernel.h) pays from 17 rows on -- one LDS operand read per MFMA (6 us of the
+//    21 us that 4096 x 28672 takes at M = 32), and a hand-over between workgroups where the slab does not fit LDS -- falls by J: the
+//    operands of a k-tile leave LDS once for J tiles, and a wavefront keeps no more of them there than the k-tile to come.
+//  * The NW wavefronts of a workgroup take the k-tiles of its part of K in turn and share nothing until their sums meet in LDS at the end:
+//    no barrier in the K loop.  Activations, scales and zero points come by direct-to-LDS loads into a piece of LDS of the wavefront's own,
+//    weights into a ring of two k-tiles of registers.
+//  * The scales of a k-tile are one row of J * 16 columns: one load for all J tiles, requested with the activations.  (One 8-byte load per
+//    tile, as the other decode kernels do it, cost 3 us on 4096 x 28672 at M = 16: 32-byte pieces of rows 57 KB apart, and the weights
+//    behind them in the queue wait for each: 11.6 us for the weights alone, 14.9 with them.)
+//  * Rows beyond MB * 16 are a second block of rows with workgroups of their own, side by side on the same XCD, so that they find the
+//    weights in its L2.  K may be split over workgroups: partial tiles and one arrival counter per 16 x 16 result, summed in split order.
+//
+// Cold, us, the kernel that took them before and this one: 4096 x 28672 at M = 24 / 32 / 48 20.2 / 21.2 / 29.0 -> 17.1 / 16.9 / 21.8;
+// 14336 x 4096 at M = 48 / 64 21.7 / 25.7 -> 17.2 / 17.7; 4096 x 6144 at M = 48 / 64 10.1 / 11.0 -> 9.2 / 9.6.
+// Not kept: operands straight from memory into registers (pieces of 64 bytes per row: 4096 x 28672 at M = 32 18.5, 14336 x 4096 16.0 us),
+// deeper rings (three and four k-tiles: level or slower), a start of the K loop that differs from workgroup to workgroup (+0.3 us), results
+// gathered in LDS and stored in whole rows of the range instead of 32-byte pieces (level: one more barrier).
+#pragma once
+#include "vaq_common.h"
+
+#include <type_traits>
+
+namespace vaq {
+
+struct RegsParams {
+  const uint16_t* a;
+  const v4u* b;
+  const uint16_t* scales;
+  const uint32_t* zeros;
+  const uint16_t* bias;
+  uint16_t* c;
+  float* c_tmp;
+  int32_t* counters;
+  int M, N, lda;
+  int G, NT;               // k-tiles of 128 rows, n-tiles of 16 columns
+  int SK, RB;              // parts of K, blocks of MB * 16 rows
+  int ranges, per_xcd;     // ranges of J n-tiles; workgroups of an XCD
+  int s_stride, z_stride;  // elements between consecutive rows of scales (N) / zeros (N/8); 0 for channelwise
+  uint32_t k_mask, k_ex;   // 0x000f000f and the exponent pattern, as run-time values (see w4a16_decode.hip)
+  uint32_t b_bytes, s_bytes, z_bytes, a_bytes;      // each below 2 GiB
+};
+
+constexpr size_t regs_lds_bytes(int mb, int mr, int j, int nw, int sub, bool zp) {
+  const size_t run = (size_t)nw * (mb * mr * 256 + 2 * (sub * 256 + (zp ? 256 : 0)));      // activations of a k-tile, scales and zero points of two
+  const size_t sums = (size_t)j * mb * nw * 1024;                                      // partial results
+  return run > sums ? run : sums;
+}
+
+// MR: rows of an m-block that are fetched, 16 or, of a single one, 4 (columns of the MFMAs are independent: those of the other rows read a
+// row that is there, and their results are not stored).  SUBG: quantisation groups per k-tile (1, 2, 4).  W8: 8-bit codes as two nibble planes.  OCC: wavefronts per SIMD that the registers
+// are to allow.
+template <bool BF16, int MB, int MR, int J, bool HAS_ZP, int NW, int SUBG, bool W8, int OCC>
+__global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(const RegsParams p) {
+  using T = F16Traits<BF16>;
+  static_assert(!(W8 && HAS_ZP), "8-bit codes have no zero points");
+  static_assert(MR == 16 || (MR == 4 && MB == 1), "fewer rows of a single m-block only");
+  constexpr int PL = W8 ? 2 : 1;      // planes of codes
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int o = lane >> 4, r16 = lane & 15;
+  // One contiguous range of units per XCD; the K parts and row blocks of one range of n-tiles are neighbours.
+  const int unit = (int)(blockIdx.x & 7u) * p.per_xcd + (int)(blockIdx.x >> 3);
+  const int copies = p.SK * p.RB;
+  if (unit >= p.ranges * copies) return;
+  const int range = unit / copies, rest = unit - range * copies;
+  const int sk = rest / p.RB, rb_i = rest - sk * p.RB;
+  const int nt0 = range * J, row0 = rb_i * MB * 16;
+  const int g_lo = (int)(((int64_t)p.G * sk) / p.SK), g_hi = (int)(((int64_t)p.G * (sk + 1)) / p.SK);
+
+  auto rsrc = [](const void* base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t ra = rsrc(p.a, p.a_bytes), rb = rsrc(p.b, p.b_bytes), rs = rsrc(p.scales, p.s_bytes);
+  const __amdgpu_buffer_rsrc_t rz = rsrc(HAS_ZP ? (const void*)p.zeros : (const void*)p.scales, HAS_ZP ? p.z_bytes : p.s_bytes);
+
+  // This wavefront's piece of LDS: the activations of the next k-tile, MR * MB rows of 256 bytes with chunk c of row r at place
+  // c ^ (r & 15); scales (256 bytes per group row) and zero points (64 per row, one piece) of the k-tile at hand and the next.
+  constexpr int AI = MB * MR / 4, ACT = AI * 1024, SC = SUBG * 256, SIDE = SC + (HAS_ZP ? 256 : 0), OWN = ACT + 2 * SIDE;
+  uint8_t* const mine = lds + (size_t)w * OWN;
+  uint32_t vo_a[AI];      // instruction i fetches rows 4i .. 4i + 3
+#pragma unroll
+  for (int i = 0; i < AI; ++i) {
+    const int r = i * 4 + o;
+    vo_a[i] = (uint32_t)min(row0 + r, p.M - 1) * (uint32_t)p.lda * 2u + (uint32_t)((r16 ^ (r & 15)) * 16);
+  }
+  constexpr uint32_t OUT = 0x80000000u;      // past the end of every buffer: reads as zero
+  struct At {                                // a k-tile: its number, or 0 and OUT for none
+    uint32_t g, out;
+  };
+  auto at = [&](int g) { return At{g < g_hi ? (uint32_t)g : 0u, g < g_hi ? 0u : OUT}; };
+  typedef __attribute__((address_space(3))) void* lds_ptr_t;
+  auto load_act = [&](int s, At t) {      // for slot s of the ring
+#pragma unroll
+    for (int i = 0; i < AI; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(mine + i * 1024), 16, (int)(vo_a[i] | t.out), (int)(t.g * 256u), 0, 0);
+    uint8_t* const side = mine + ACT + s * SIDE;
+#pragma unroll
+    for (int sj = 0; sj < SUBG; ++sj)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(side + sj * 256), 4, (int)((lane < J * 8 ? (uint32_t)lane * 4u : OUT) | t.out),
+                                               (int)(((t.g * SUBG + sj) * (uint32_t)p.s_stride + (uint32_t)nt0 * 16u) * 2u), 0, 0);
+    if constexpr (HAS_ZP) {      // 16 lanes a row
+      const uint32_t vo = o < SUBG && r16 < J * 2 ? (uint32_t)o * (uint32_t)p.z_stride * 4u + (uint32_t)r16 * 4u : OUT;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rz, (lds_ptr_t)(side + SC), 4, (int)(vo | t.out),
+                                               (int)((t.g * SUBG * (uint32_t)p.z_stride + (uint32_t)nt0 * 2u) * 4u), 0, 0);
+    }
+  };
+  v4u wq[2][J][PL];
+  auto load_w = [&](int s, At t, int j) {
+    const uint32_t nt = (uint32_t)min(nt0 + j, p.NT - 1);
+#pragma unroll
+    for (int pl = 0; pl < PL; ++pl)
+      wq[s][j][pl] = __builtin_amdgcn_raw_buffer_load_b128(rb, (int)((uint32_t)lane * 16u | t.out), (int)(((nt * (uint32_t)p.G + t.g) * PL + pl) * 1024u), 2);
+  };
+
+  v4f acc[J][MB];
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) acc[j][mb] = v4f{0.f, 0.f, 0.f, 0.f};
+
+  uint32_t ex;
+  asm volatile("v_mov_b32 %0, %1" : "=v"(ex) : "s"(p.k_ex));
+  const uint32_t msk = p.k_mask;
+
+  // The k-tile in slot s.  Behind it are requested, as soon as there is room: the next one's activations, then tile by tile the weights of
+  // the one after that (the scheduling barriers keep each weight request behind the arithmetic that frees its registers, which is what
+  // saves copying them).
+  auto tile = [&](int s, bool refill_act, At next_act, bool refill_w, At next_w) {
+    v4u act[4][MB];
+    const uint8_t* const side = mine + ACT + s * SIDE;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj)
+        act[jj][mb] = *reinterpret_cast<const v4u*>(mine + mb * 4096 + (r16 & (MR - 1)) * 256 + (((jj * 4 + o) ^ (r16 & (MR - 1))) * 16));
+    if (refill_act) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // this tile's are in registers
+      __builtin_amdgcn_sched_barrier(0);
+      load_act(s ^ 1, next_act);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // row sums S of each group: the same in the four registers.  Plain codes: -(BIAS + 8) S is where the group's MFMA chain starts.
+    constexpr bool CHAIN = SUBG == 1 && !HAS_ZP && !W8;
+    v4f start[MB];
+    float S[SUBG][MB];
+    const v4u ones = {T::ONE2, T::ONE2, T::ONE2, T::ONE2};
+#pragma unroll
+    for (int sj = 0; sj < SUBG; ++sj)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        v4f t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int jj = sj * (4 / SUBG); jj < (sj + 1) * (4 / SUBG); ++jj) t = T::mfma16(ones, act[jj][mb], t);
+        start[mb] = t * -(T::CODE_BIAS + 8.0f);
+        S[sj][mb] = t[0];
+      }
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+#pragma unroll
+      for (int sj = 0; sj < SUBG; ++sj) {
+        const v2u sct = *reinterpret_cast<const v2u*>(side + sj * 256 + j * 32 + o * 8);
+        const uint32_t z4 = HAS_ZP ? *reinterpret_cast<const uint32_t*>(side + SC + sj * 64 + j * 8 + (o >> 1) * 4) >> ((o & 1) * 16) : 0u;
+        v4f P[PL][MB];
+#pragma unroll
+        for (int pl = 0; pl < PL; ++pl) {
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) P[pl][mb] = CHAIN ? start[mb] : v4f{0.f, 0.f, 0.f, 0.f};
+          const uint32_t wj[4] = {wq[s][j][pl].x, wq[s][j][pl].y, wq[s][j][pl].z, wq[s][j][pl].w};
+#pragma unroll
+          for (int jj = sj * (4 / SUBG); jj < (sj + 1) * (4 / SUBG); ++jj) {
+            v4u aop;
+            aop.x = (wj[jj] & msk) | ex;
+            aop.y = ((wj[jj] >> 4) & msk) | ex;
+            aop.z = ((wj[jj] >> 8) & msk) | ex;
+            aop.w = ((wj[jj] >> 12) & msk) | ex;
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) P[pl][mb] = T::mfma16(aop, act[jj][mb], P[pl][mb]);
+          }
+        }
+        float sf[4];
+        if constexpr (BF16) {
+          sf[0] = __uint_as_float(sct.x << 16);
+          sf[1] = __uint_as_float(sct.x & 0xffff0000u);
+          sf[2] = __uint_as_float(sct.y << 16);
+          sf[3] = __uint_as_float(sct.y & 0xffff0000u);
+        } else {
+          sf[0] = T::to_float((uint16_t)(sct.x & 0xffffu));
+          sf[1] = T::to_float((uint16_t)(sct.x >> 16));
+          sf[2] = T::to_float((uint16_t)(sct.y & 0xffffu));
+          sf[3] = T::to_float((uint16_t)(sct.y >> 16));
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float zc = HAS_ZP ? T::CODE_BIAS + (float)((z4 >> (4 * r)) & 0xFu) : T::CODE_BIAS + 8.0f;
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) {
+            if constexpr (CHAIN) {
+              acc[j][mb][r] = fmaf(sf[r], P[0][mb][r], acc[j][mb][r]);
+            } else if constexpr (W8) {      // high plane (bias 8 of its own) times 16, then the low one
+              acc[j][mb][r] = fmaf(16.0f * sf[r], fmaf(-zc, S[sj][mb], P[0][mb][r]), acc[j][mb][r]);
+              acc[j][mb][r] = fmaf(sf[r], fmaf(-T::CODE_BIAS, S[sj][mb], P[PL - 1][mb][r]), acc[j][mb][r]);
+            } else {
+              acc[j][mb][r] = fmaf(sf[r], fmaf(-zc, S[sj][mb], P[0][mb][r]), acc[j][mb][r]);
+            }
+          }
+        }
+      }
+      if (refill_w) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(s, next_w, j);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+
+  // This wavefront's k-tiles: g_lo + w + i * NW.  The order of the requests is W(0) A(0) W(1) | A(1) W(2) | A(2) W(3) | ..., `|` = a tile:
+  // a tile starts when all but the weights requested behind its activations have been answered.
+  auto wait = [&] { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(J * PL) : "memory"); };
+  int g = g_lo + w;
+#pragma unroll
+  for (int j = 0; j < J; ++j) load_w(0, at(g), j);
+  __builtin_amdgcn_sched_barrier(0);
+  load_act(0, at(g));
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < J; ++j) load_w(1, at(g + NW), j);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+  for (; g + NW < g_hi; g += 2 * NW) {
+    wait();
+    tile(0, true, at(g + NW), true, at(g + 2 * NW));
+    wait();
+    tile(1, true, at(g + 2 * NW), true, at(g + 3 * NW));
+  }
+  if (g < g_hi) {
+    wait();
+    tile(0, false, At{0u, OUT}, false, At{0u, OUT});
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (what is requested past the end writes zeros into LDS)
+
+  // ---- the wavefronts' parts of K, on top of the activations ----
+  v4f* const red = reinterpret_cast<v4f*>(lds);                                       // [NW][J * MB][64]
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) red[(w * (J * MB) + j * MB + mb) * 64 + lane] = acc[j][mb];
+  __syncthreads();
+  for (int q = w; q < J * MB; q += NW) {
+    const int j = q / MB, mb = q - j * MB;
+    const int nt = nt0 + j;
+    if (nt >= p.NT || row0 + mb * 16 >= p.M) continue;
+    v4f val = red[q * 64 + lane];
+#pragma unroll
+    for (int s = 1; s < NW; ++s) val += red[(s * (J * MB) + q) * 64 + lane];
+    if (p.SK > 1) {
+      // partial tiles and counters as in w4a16_decode2_kernel.h, step 5
+      constexpr int SC1 = 16;
+      const uint32_t units = (uint32_t)p.NT * (uint32_t)(p.RB * MB), u = (uint32_t)nt * (uint32_t)(p.RB * MB) + (uint32_t)(rb_i * MB + mb);
+      const __amdgpu_buffer_rsrc_t rt = rsrc(p.c_tmp, units * 1024u * (uint32_t)p.SK);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, val), rt, lane * 16, (int)(((uint32_t)sk * units + u) * 1024u), SC1);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // partial tile acknowledged before the counter moves
+      int old = 0;
+      if (lane == 0) old = __hip_atomic_fetch_add(&p.counters[u], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      old = __builtin_amdgcn_readfirstlane(old);
+      if (old != p.SK - 1) continue;
+      val = v4f{0.f, 0.f, 0.f, 0.f};
+      for (int s0 = 0; s0 < p.SK; s0 += 4) {               // four parts in flight, added in split order
+        v4u part[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          part[i] = __builtin_amdgcn_raw_buffer_load_b128(rt, lane * 16, (int)(((uint32_t)min(s0 + i, p.SK - 1) * units + u) * 1024u), SC1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (s0 + i < p.SK) val += __builtin_bit_cast(v4f, part[i]);
+      }
+      if (lane == 0) __hip_atomic_store(&p.counters[u], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const int m = row0 + mb * 16 + r16, n = nt * 16 + o * 4;
+    if (p.bias) {
+      const v2u bb = *reinterpret_cast<const v2u*>(p.bias + n);
+      val[0] += T::to_float((uint16_t)(bb.x & 0xffffu));
+      val[1] += T::to_float((uint16_t)(bb.x >> 16));
+      val[2] += T::to_float((uint16_t)(bb.y & 0xffffu));
+      val[3] += T::to_float((uint16_t)(bb.y >> 16));
+    }
+    v2u outv;
+    outv.x = (uint32_t)T::from_float(val[0]) | ((uint32_t)T::from_float(val[1]) << 16);
+    outv.y = (uint32_t)T::from_float(val[2]) | ((uint32_t)T::from_float(val[3]) << 16);
+    if (m < p.M) *reinterpret_cast<v2u*>(p.c + (int64_t)m * p.N + n) = outv;
+  }
+}
+
+// Registers of a lane, roughly: two k-tiles of weights, sums, operands, a chain per plane, row sums.
+constexpr int regs_estimate(int mb, int j, int sub, bool w8) {
+  const int pl = w8 ? 2 : 1;
+  return 8 * j * pl + 4 * j * mb + 16 * mb + 4 * pl * mb + (4 + sub) * mb + (sub == 4 ? 65 : 45);
+}
+// Launch shapes: eight wavefronts for up to four n-tiles, four for three to eight (of 8-bit codes to six), up to three m-blocks (8-bit codes in
+// groups of 32 rows, three m-blocks of four n-tiles: more registers than eight wavefronts have).
+constexpr bool regs_built(int mb, int j, int nw, int sub, bool w8) {
+  return mb >= 1 && mb <= 3 && (nw == 8 ? j >= 1 && j <= 4 && !(w8 && sub == 4 && mb * j == 12) : nw == 4 && j >= 3 && j <= (w8 ? 6 : 8));
+}
+
+template <bool BF16, bool HAS_ZP, int SUBG, bool W8, int NW, int J, int MB, int MR = 16>
+static int launch_regs(const RegsParams& p, hipStream_t s) {
+  if constexpr (MB == 1 && MR == 16)
+    if (p.M <= 4) return launch_regs<BF16, HAS_ZP, SUBG, W8, NW, J, MB, 4>(p, s);
+  constexpr size_t lds = regs_lds_bytes(MB, MR, J, NW, SUBG, HAS_ZP);
+  static_assert(lds <= 160 * 1024, "LDS");
+  auto kern = w4a16_regs_kernel<BF16, MB, MR, J, HAS_ZP, NW, SUBG, W8, NW == 4 && (regs_estimate(MB, J, SUBG, W8) > 256) ? 1 : 2>;
+  static size_t reserved[VAQ_MAX_DEVICES];
+  if (const int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds, reserved, "w4a16_gemm(regs)"); rc != VAQ_OK) return rc;
+  hipLaunchKernelGGL(kern, dim3(p.per_xcd * 8), dim3(NW * 64), lds, s, p);
+  return VAQ_OK;
+}
+
+template <bool BF16, bool HAS_ZP, int SUBG, bool W8, int NW, int J = 1>
+static int regs_dispatch(const RegsParams& p, int j, int mb, hipStream_t s) {
+  if constexpr (J > 8) {
+    set_error("w4a16_gemm(regs): %d n-tiles and %d m-blocks on %d wavefronts are not built", j, mb, NW);
+    return VAQ_ERR_UNSUPPORTED;
+  } else {
+    if constexpr (regs_built(1, J, NW, SUBG, W8))
+      if (j == J && mb == 1) return launch_regs<BF16, HAS_ZP, SUBG, W8, NW, J, 1>(p, s);
+    if constexpr (regs_built(2, J, NW, SUBG, W8))
+      if (j == J && mb == 2) return launch_regs<BF16, HAS_ZP, SUBG, W8, NW, J, 2>(p, s);
+    if constexpr (regs_built(3, J, NW, SUBG, W8))
+      if (j == J && mb == 3) return launch_regs<BF16, HAS_ZP, SUBG, W8, NW, J, 3>(p, s);
+    return regs_dispatch<BF16, HAS_ZP, SUBG, W8, NW, J + 1>(p, j, mb, s);
+  }
+}
+
+template <int SUBG, bool W8, bool HAS_ZP>
+static int regs_types(const RegsParams& p, int nw, int j, int mb, bool bf16, hipStream_t s) {
+  if (nw == 8) return bf16 ? regs_dispatch<true, HAS_ZP, SUBG, W8, 8>(p, j, mb, s) : regs_dispatch<false, HAS_ZP, SUBG, W8, 8>(p, j, mb, s);
+  return bf16 ? regs_dispatch<true, HAS_ZP, SUBG, W8, 4>(p, j, mb, s) : regs_dispatch<false, HAS_ZP, SUBG, W8, 4>(p, j, mb, s);
+}
+
+// One file each (w4a16_regs_*.hip): 4-bit codes in groups of 128 / 64 / 32 rows, 8-bit codes likewise.
+int regs_launch_w4(const RegsParams& p, int nw, int j, int mb, bool bf16, bool zp, hipStream_t s);
+int regs_launch_w4_sub2(const RegsParams& p, int nw, int j, int mb, bool bf16, bool zp, hipStream_t s);
+int regs_launch_w4_sub4(const RegsParams& p, int nw, int j, int mb, bool bf16, bool zp, hipStream_t s);
+int regs_launch_w8(const RegsParams& p, int nw, int j, int mb, bool bf16, hipStream_t s);
+int regs_launch_w8_sub2(const RegsParams& p, int nw, int j, int mb, bool bf16, hipStream_t s);
+int regs_launch_w8_sub4(const RegsParams& p, int nw, int j, int mb, bool bf16, hipStream_t s);
+
+}  // namespace vaq
