@@ -382,17 +382,17 @@ __global__ __launch_bounds__(256) void fp8_mm_tile2_kernel(const Fp8MMParams p) 
 
 // ----------------------------------------------------------------------------- tile kernel, multi-stage direct-to-LDS
 // The kernel the M > 32 path normally uses.  Differences from fp8_mm_tile2_kernel:
-//  * one MFMA k-slice (64 bytes of K) per stage, NST stages in a ring: the requests for step s+NST-1 go out at the
-//    start of step s, so a tile has NST-2 full steps to arrive before anybody waits for it (with two stages of 128
+//  * one MFMA k-slice (64 bytes of K) per stage, NST stages in a ring: the requests for step s+NST-1 go out in
+//    step s, so a tile has NST-2 full steps to arrive before anybody waits for it (with two stages of 128
 //    bytes the wait at the end of every step saw most of the L2 latency);
 //  * vector-memory operations retire in issue order, so "the tile of step s+1 has landed" is `vmcnt <= requests issued
 //    after it`, a compile-time constant; the workgroup barrier is the bare instruction (a __syncthreads() carries a fence
 //    that drains every outstanding load);
 //  * LDS rows are 64 bytes; four rows form one 256-byte line of 16 chunks (chunk index (row & 3) * 4 + c) and the chunk
-//    index is XOR-ed with (row >> 2) & 3.  The LDS has 64 banks (256 bytes per cycle): 16 lanes reading 16 consecutive
-//    rows at the same k chunk touch 16 different 16-byte bank groups;
+//    index is XOR-ed with (row >> 2) & 3; or (LINE) 128 bytes, two to a line, the chunk index XOR-ed with bits 1, 3, 2 of the row.  The LDS has 64
+//    banks (256 bytes per cycle): 16 lanes reading 16 consecutive rows at the same k chunk touch 16 different 16-byte bank groups;
 //  * two slices of K are requested at a time (KS = 2, or PP = 2 where the ring has no room for whole pairs), for the reason at
-//    load_slices below, and by eight wavefronts even for a 128 x 128 tile: with four a compute unit has fewer requests under
+//    `load` below, and by eight wavefronts even for a 128 x 128 tile: with four a compute unit has fewer requests under
 //    way.  128 x 128 tiles, cold: 4096 x 6144 at M = 333 23.3 -> 19.5 us, 5120 x 13824 at M = 250 29.3 -> 24.3 us (cached);
 //    256 x 128: 4096 x 4096 at M = 2048 40.7 -> 35.8 us; 256 x 256: 4096 x 4096 at M = 4096 59.0 -> 56.1 us (2.45 PFLOP/s),
 //    14336 x 4096 195.5 -> 183.1 us.  Not kept: four slices at a time in two stages, K slices dealt to two groups of
@@ -404,6 +404,7 @@ template <bool BF16_OUT, int BM, int BN, int WAVES_M, int WAVES_N, int NST, int 
 __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(const Fp8MMParams p) {
   // A step is KS k-slices of 64 bytes (KS = 2 for the small tiles, whose steps are otherwise shorter than the barrier
   // and the LDS round trip that every step pays); a stage holds the KS slices of one step, each as [A tile | B tile].
+  constexpr bool PAIR = PP == 2, LINE = KS == 2 || PAIR;        // requests of whole 128-byte lines (see `load`)
   constexpr int NW = WAVES_M * WAVES_N;
   constexpr int TM = BM / WAVES_M, TN = BN / WAVES_N;
   constexpr int WMB = TM / 32, WNB = TN / 32;
@@ -433,18 +434,21 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
 
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.a), 0, (int)((uint32_t)p.M * (uint32_t)p.lda), 0x00020000);
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.b), 0, (int)((uint32_t)p.N * (uint32_t)p.ldb), 0x00020000);
-  // DMA instruction: 16 rows x 64 bytes = four 256-byte lines; lane l lands in slot l: line j = r0/4 + (l >> 4), swizzled
+  // DMA instruction.  One slice: 16 rows x 64 bytes = four 256-byte lines; lane l lands in slot l: line j = r0/4 + (l >> 4), swizzled
   // chunk l & 15 -> c16 = (l & 15) ^ (j & 3), row = 4j + (c16 >> 2), chunk = c16 & 3.  r0 is a multiple of 16, so j & 3 = l >> 4.
+  // Two slices (LINE): 8 rows x 128 bytes; row r0 + (l >> 3), chunk (l & 7) ^ f, f = bits 3, 1, 2 of the row in this order -> with r0 = 8 times the
+  // instruction's number, bits 5 and 4 of l in places 2 and 0, and 2 more for the odd instructions of a wavefront.
   const int c16 = (lane & 15) ^ (lane >> 4);
-  const int lrow = 4 * (lane >> 4) + (c16 >> 2);
-  const uint32_t voff_a = (uint32_t)lrow * (uint32_t)p.lda + (uint32_t)(c16 & 3) * 16u;
-  const uint32_t voff_b = (uint32_t)lrow * (uint32_t)p.ldb + (uint32_t)(c16 & 3) * 16u;
+  const uint32_t lrow = (uint32_t)(LINE ? lane >> 3 : 4 * (lane >> 4) + (c16 >> 2));
+  const uint32_t lbyte = (uint32_t)(LINE ? (lane & 7) ^ ((lane >> 4 & 1) | (lane >> 5) << 2) : c16 & 3) * 16u;
+  const uint32_t row_a = lrow * (uint32_t)p.lda, row_b = lrow * (uint32_t)p.ldb;
+  const uint32_t voff_a = row_a + lbyte, voff_b = row_b + lbyte;
+  const uint32_t voff_a1 = row_a + (lbyte ^ 32u), voff_b1 = row_b + (lbyte ^ 32u);      // (LINE: odd instructions)
 
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   // K may be split over workgroups: this one covers the steps [s_lo, s_hi)
   const int all_steps = p.K / (64 * KS);
   // (in pairs: parts start at even steps, so that the two slices of a request share their cache lines)
-  constexpr bool PAIR = PP == 2;
   const auto part = [&](int i) { return i >= sl.nsplit ? all_steps : (int)(((int64_t)all_steps * i) / sl.nsplit) & (PAIR ? ~1 : ~0); };
   const int s_lo = part(sl.split), s_hi = part(sl.split + 1);
   const int steps = s_hi - s_lo;
@@ -459,37 +463,48 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
   // 5120; with 16 tile rows it costs 3-9 %: the tiles of one column then no longer read their weights together).
   int rot = p.rotate_k == 1 ? (tm * steps) / tiles_m : (p.rotate_k == 2 ? (tn * steps) / tiles_n : 0);
   if (PAIR) rot = steps & 1 ? 0 : rot & ~1;      // a pair never wraps around
-  // Requests for the slices from K byte `koff` on, slice i into slot(i).  The loads of neighbouring slices follow each other
-  // row by row: a row's 64-byte pieces are halves of one 128-byte line, which crosses from the L2 once when both are asked
-  // for together and twice otherwise -- and that port bounds the kernel (operands out of the L2 into LDS without any
-  // arithmetic: 30 bytes per cycle and compute unit one slice at a time, 45 in whole lines).
-  auto load_slices = [&](auto count, uint32_t koff, auto slot) {
+  // Requests for ROWS rows of an operand, from row `first` and K byte `koff` on.  LINE: eight lanes ask for 128 bytes, a whole cache line,
+  // which crosses from the L2 in one piece; else the slices of a step row by row, whose halves of a line cross one after the other.  Weights from
+  // memory, halves -> lines: 128 x 128 tiles: 5120 x 13824 at M = 250 33.6 -> 31.5 us, 4096 x 28672 at M = 100 30.3 -> 27.7; 64 x 128, 128 x 64, 128 x 256:
+  // 2 - 9 %; 64 x 64: 3 - 6 %; 256 x 256: 4096 x 28672 at M = 512 59.1 -> 56.1; from the memory-side cache level.  Pieces of 256 bytes (four slices,
+  // half of the rows at a time): -4 .. +3 % against lines; one operand in lines and the other in halves: in between.
+  auto load = [&](auto rows, const __amdgpu_buffer_rsrc_t& r, uint32_t first, int64_t pitch, uint32_t v0, uint32_t v1, uint32_t koff, uint8_t* at) {
+    constexpr int ROWS = decltype(rows)::value;
+    if constexpr (LINE) {
+      constexpr int LD = ROWS / (8 * NW);
 #pragma unroll
-    for (int i = 0; i < A_LD; ++i) {
-      const int r0 = (wave * A_LD + i) * 16;
+      for (int i = 0; i < LD; ++i) {
+        const int r0 = (wave * LD + i) * 8;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(at + r0 * 128), 16, (int)(i & 1 ? v1 : v0), (int)((first + (uint32_t)r0) * (uint32_t)pitch + koff), 0, 0);
+      }
+    } else {
+      constexpr int LD = ROWS / (16 * NW);
 #pragma unroll
-      for (int c = 0; c < decltype(count)::value; ++c)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(slot(c) + r0 * 64), 16, (int)voff_a,
-                                                 (int)((uint32_t)(m0 + r0) * (uint32_t)p.lda + koff + 64u * c), 0, 0);
+      for (int i = 0; i < LD; ++i) {
+        const int r0 = (wave * LD + i) * 16;
+#pragma unroll
+        for (int c = 0; c < KS; ++c)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(at + (c * ROWS + r0) * 64), 16, (int)v0, (int)((first + (uint32_t)r0) * (uint32_t)pitch + koff + 64u * c), 0, 0);
+      }
     }
-#pragma unroll
-    for (int i = 0; i < B_LD; ++i) {
-      const int r0 = (wave * B_LD + i) * 16;
-#pragma unroll
-      for (int c = 0; c < decltype(count)::value; ++c)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(slot(c) + A_ST + r0 * 64), 16, (int)voff_b,
-                                                 (int)((uint32_t)(n0 + r0) * (uint32_t)p.ldb + koff + 64u * c), 0, 0);
-    }
   };
-  auto k_of = [&](int step) {      // first byte of K of a step, rotation applied
-    const int rel = step - s_lo + rot;
-    return (uint32_t)((s_lo + (rel >= steps ? rel - steps : rel)) * KS) * 64u;
+  auto load_a = [&](uint32_t koff, uint8_t* at) { load(std::integral_constant<int, BM>{}, ra, (uint32_t)m0, p.lda, voff_a, voff_a1, koff, at); };
+  auto load_b = [&](uint32_t koff, uint8_t* at) { load(std::integral_constant<int, BN>{}, rb, (uint32_t)n0, p.ldb, voff_b, voff_b1, koff, at); };
+  // Steps are requested in order: the first byte of K of the next one, rotation applied.  (As few scalar instructions as can be: the matrix
+  // cores wait for them at the start of every step.)
+  constexpr uint32_t K_STEP = PAIR ? 128 : 64 * KS;
+  const uint32_t k_lo = (uint32_t)s_lo * 64u * KS, k_hi = (uint32_t)s_hi * 64u * KS;
+  uint32_t k_at = k_lo + (uint32_t)rot * 64u * KS;
+  auto next_k = [&] {
+    const uint32_t k = k_at;
+    k_at = k + K_STEP >= k_hi ? k_lo : k + K_STEP;
+    return k;
   };
-  auto issue_loads = [&](int step, int stage) {
-    load_slices(std::integral_constant<int, KS>{}, k_of(step), [&](int c) { return lds8 + (size_t)stage * STAGE + c * SLICE; });
-  };
-  auto issue_pair = [&](int step, int stage, int stage2) {      // steps `step` and `step` + 1, one slice each
-    load_slices(std::integral_constant<int, 2>{}, k_of(step), [&](int c) { return lds8 + (size_t)(c ? stage2 : stage) * STAGE; });
+  auto request = [&](int stage) {
+    uint8_t* const at = lds8 + (size_t)stage * STAGE;
+    const uint32_t k = next_k();
+    load_a(k, at);
+    load_b(k, at + KS * A_ST);
   };
 
   v16f acc[WMB][WNB];
@@ -501,40 +516,109 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
   // operand reads: row = lane & 31 of a 32-row block (blocks start at multiples of 32 rows), the lane's 32 bytes are
-  // chunks 2*kh and 2*kh+1 (kh = lane >> 5)
+  // chunks 2*kh and 2*kh+1 (kh = lane >> 5) of the slice.  The 16 lanes that are served together read 16 rows at the same chunk of K: 16
+  // different places of a 256-byte line in either layout.
   const int kh = lane >> 5;
   uint32_t coff[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h)
-    coff[h] = (uint32_t)(((lane & 31) >> 2) * 256 + ((((lane & 3) * 4 + kh * 2 + h) ^ ((lane >> 2) & 3)) * 16));
-  const uint32_t arow = (uint32_t)(wm * TM * 64);
-  const uint32_t brow = (uint32_t)(A_ST + wn * TN * 64);
+    coff[h] = LINE ? (uint32_t)((lane & 31) * 128 + (((kh * 2 + h) ^ ((lane >> 1 & 1) | (lane >> 2 & 1) << 2 | (lane >> 3 & 1) << 1)) * 16))
+                   : (uint32_t)(((lane & 31) >> 2) * 256 + ((((lane & 3) * 4 + kh * 2 + h) ^ ((lane >> 2) & 3)) * 16));
+  // LDS addresses of this wavefront's fragments at the step at hand, slice ks (LINE: half ks of each line)
+  typedef __attribute__((address_space(3))) const v4i* lds_v4i_t;
+  constexpr int SL = LINE ? 2 : 1, ROW_BYTES = LINE ? 128 : 64, PLACE = (BM > BN ? BM : BN) * 128;      // (PLACE: see PP = 2)
+  uint32_t adr_a[SL][2], adr_b[SL][2];
+  {
+    const uint32_t base = (uint32_t)(uintptr_t)(lds_ptr_t)lds8;
+#pragma unroll
+    for (int ks = 0; ks < SL; ++ks)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const uint32_t at = base + (coff[h] ^ (ks ? 64u : 0u));
+        adr_a[ks][h] = at + (uint32_t)(wm * TM * ROW_BYTES + (PAIR ? PLACE : 0));
+        adr_b[ks][h] = at + (uint32_t)(wn * TN * ROW_BYTES + (PAIR ? 0 : KS * A_ST));
+      }
+  }
+  auto fragment = [&](const uint32_t (&adr)[2], int block) {
+    const v4i lo = *reinterpret_cast<lds_v4i_t>((uintptr_t)(adr[0] + block * 32 * ROW_BYTES));
+    const v4i hi = *reinterpret_cast<lds_v4i_t>((uintptr_t)(adr[1] + block * 32 * ROW_BYTES));
+    return v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+  };
+  auto read_a = [&](int ks, v8i (&af)[WMB]) {
+#pragma unroll
+    for (int i = 0; i < WMB; ++i) af[i] = fragment(adr_a[ks], i);
+  };
+  auto read_b = [&](int ks, v8i (&bf)[WNB]) {
+#pragma unroll
+    for (int j = 0; j < WNB; ++j) bf[j] = fragment(adr_b[ks], j);
+  };
+  // (here and now, in the shadow of the reads: the compiler would rather add ahead of the next reads, with everybody waiting)
+  auto move = [&](uint32_t (&adr)[SL][2], int by) {
+#pragma unroll
+    for (int ks = 0; ks < SL; ++ks)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        adr[ks][h] += (uint32_t)by;
+#ifdef __HIP_DEVICE_COMPILE__
+        asm volatile("" : "+v"(adr[ks][h]));
+#endif
+      }
+  };
 
   // (Reading the fragments of step s+1 during the MFMAs of step s -- one more stage of slack, double-buffered weight
   // fragments -- was measured 5% slower than reading them at the start of their own step, and is not done.)
-  auto compute = [&](int stage) {
+  //
+  // A step is a chain -- barrier, addresses, fragment reads, MFMAs -- that every wavefront of the workgroup walks through together, so that what
+  // stands ahead of the reads is paid in full.  The addresses are held, and moved on (`by` bytes) behind the reads; the reads come first, of both slices
+  // where the registers hold them (at most two blocks to a wavefront), the requests behind them; the loops stay rolled.  With whole lines, drawn problems,
+  // weights from the memory-side cache / from memory, against addresses computed ahead of the reads and requests of halves ahead of them: 128 x 128
+  // tiles -4 / -5 % (5120 x 13824 at M = 250 26.0 -> 24.7 us with its quantisation), 64 x 128 -5 / -7, 128 x 64 -6 / -6, 64 x 64 -3 / -3, 128 x 256 -3 / -3, 256 x 128
+  // -10 / -9, 256 x 256 -5 / -5 (14336 x 4096 at M = 4096 183 -> 163 us, 4096 x 28672 at M = 2048 218 -> 200).  Written out for a turn of the ring, with the stages in
+  // the reads' offsets, a long K gains up to 5 % more, but a short one waits for the larger code: 2944 x 8896 at M = 1759 47 -> 51 us, 1152 x 28288 at
+  // M = 492 25.2 -> 27.6.
+  constexpr bool AT_ONCE = KS == 1 || WMB * WNB <= 2;
+  auto compute = [&](int by, auto requests) {
+    if constexpr (AT_ONCE) {
+      v8i af[KS][WMB], bf[KS][WNB];
 #pragma unroll
-   for (int ks = 0; ks < KS; ++ks) {
-    const uint8_t* base = lds8 + (size_t)stage * STAGE + ks * SLICE;
-    v8i af[WMB], bf[WNB];
+      for (int ks = 0; ks < KS; ++ks) {
+        read_b(ks, bf[ks]);
+        read_a(ks, af[ks]);
+      }
+      if constexpr (PP == 0) {      // (256 x 384 has no registers for all of them at once)
+        __builtin_amdgcn_sched_barrier(0);
+        requests();
+        move(adr_a, by);
+        move(adr_b, by);
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
-    for (int j = 0; j < WNB; ++j) {
-      const v4i lo = *reinterpret_cast<const v4i*>(base + brow + j * 2048 + coff[0]);
-      const v4i hi = *reinterpret_cast<const v4i*>(base + brow + j * 2048 + coff[1]);
-      bf[j] = v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int i = 0; i < WMB; ++i)
+#pragma unroll
+          for (int j = 0; j < WNB; ++j) acc[i][j] = mfma_fp8_32(bf[ks][j], af[ks][i], acc[i][j]);   // rows = n, columns = m
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        v8i af[WMB], bf[WNB];
+        read_b(ks, bf);
+        read_a(ks, af);
+        __builtin_amdgcn_sched_barrier(0);
+        if (ks == 0) requests();
+        if (ks == KS - 1) {
+          move(adr_a, by);
+          move(adr_b, by);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < WMB; ++i)
+#pragma unroll
+          for (int j = 0; j < WNB; ++j) acc[i][j] = mfma_fp8_32(bf[j], af[i], acc[i][j]);
+      }
     }
-#pragma unroll
-    for (int i = 0; i < WMB; ++i) {
-      const v4i lo = *reinterpret_cast<const v4i*>(base + arow + i * 2048 + coff[0]);
-      const v4i hi = *reinterpret_cast<const v4i*>(base + arow + i * 2048 + coff[1]);
-      af[i] = v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-    }
-#pragma unroll
-    for (int i = 0; i < WMB; ++i)
-#pragma unroll
-      for (int j = 0; j < WNB; ++j) acc[i][j] = mfma_fp8_32(bf[j], af[i], acc[i][j]);   // rows = n, columns = m
-   }
   };
+  auto nothing = [] {};
   // end of a step: LDS reads of this wavefront done, requests older than the newest `n` landed, then the bare barrier
   auto sync_step = [&](auto n_c) {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(decltype(n_c)::value) : "memory");
@@ -543,115 +627,155 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
   using WAIT_NONE = std::integral_constant<int, 0>;
 
   // Invariant at the start of step s: the tile of step s complete in LDS, the tiles of steps s+1 .. s+NST-2 requested,
-  // stage (s-1) % NST free.  The requests of step s+NST-1 go out first thing in step s.
-  if (PP != 0 && steps >= NST) {      // (a pair's prologue requests NST - 1 slices)
-    // Alternating phases: the two wavefronts that share a SIMD run half a step apart, so that one reads its fragments
-    // (and requests tiles) while the other one issues its MFMAs.  A step is [requests, fragment reads, wait] barrier
-    // [MFMAs] barrier; the late half of the workgroup passes one extra barrier first and skips its last one, so every
-    // wavefront passes the same number.  The tile of step s+1 must have landed at the END OF THE READ PHASE of step s
-    // (the early half reads it two barriers later, the late half three).
-    auto read_frags = [&](int stage, v8i (&af)[KS][WMB], v8i (&bf)[KS][WNB]) {
+  // stage (s-1) % NST free.  The requests of step s+NST-1 go out in step s, behind its first fragment reads.
+  // Alternating phases (PP): the two wavefronts that share a SIMD run half a step apart, so that one reads its fragments
+  // (and requests operands) while the other one issues its MFMAs.  A step is [requests, fragment reads, wait] barrier
+  // [MFMAs] barrier; the late half of the workgroup passes one extra barrier first and skips its last one, so every
+  // wavefront passes the same number.  What the next step reads must have landed at the END OF THE READ PHASE of this one
+  // (the early half reads it two barriers later, the late half three).
+  auto mfmas = [&](v8i (&af)[WMB], v8i (&bf)[WNB]) {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const uint8_t* base = lds8 + (size_t)stage * STAGE + ks * SLICE;
+    for (int i = 0; i < WMB; ++i)
 #pragma unroll
-        for (int j = 0; j < WNB; ++j) {
-          const v4i lo = *reinterpret_cast<const v4i*>(base + brow + j * 2048 + coff[0]);
-          const v4i hi = *reinterpret_cast<const v4i*>(base + brow + j * 2048 + coff[1]);
-          bf[ks][j] = v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-        }
-#pragma unroll
-        for (int i = 0; i < WMB; ++i) {
-          const v4i lo = *reinterpret_cast<const v4i*>(base + arow + i * 2048 + coff[0]);
-          const v4i hi = *reinterpret_cast<const v4i*>(base + arow + i * 2048 + coff[1]);
-          af[ks][i] = v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-        }
+      for (int j = 0; j < WNB; ++j) acc[i][j] = mfma_fp8_32(bf[j], af[i], acc[i][j]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto bare_barrier = [&]() { asm volatile("s_barrier" ::: "memory"); };
+  const bool late = wave >= NW / 2;     // wavefronts w and w + 4 share a SIMD (the other pairing measured 10-25 % slower)
+  if constexpr (PAIR) {
+    // Two steps read the two slices of a pair of them, 128 bytes of every row, the weights of both in the first.  The LDS has five places for
+    // an operand of a pair, which weights and activations take in turn, B(0) A(0) B(1) A(1) ...: those of the pair at hand, of the next, and
+    // the weights of the one after that.  The weights are free after a pair's first step, the activations after its second, and each
+    // is at once replaced by what comes two and a half pairs later, so that a request has three or four steps to be answered.
+    // (Both operands free after the second step: two and four steps, 4 % slower on 4096 x 28672 at M = 4096.)  A step is bound by its chain of
+    // reads and MFMAs and by the power limit: with all operands zero 4096^3 takes 0.7 of the time, without any MFMA half.
+    static_assert(BM == BN && NST == 5, "five places of one size");
+    constexpr int LD = BM / (8 * NW);                          // requests of a wavefront for an operand of a pair
+    const int pairs = (steps + 1) / 2;                         // (the last one may be half a pair: its other slice is fetched and not read)
+    int qb = 0;                                                // place of the pair at hand's weights
+    auto place = [&](int ahead) {                              // that of the operand `ahead` places on
+      const int q = qb + ahead;
+      return lds8 + (q >= 5 ? q - 5 : q) * PLACE;
+    };
+    {
+      const uint32_t k0 = next_k(), k1 = next_k();
+      load_b(k0, place(0));
+      load_a(k0, place(1));
+      if (pairs > 1) {
+        load_b(k1, place(2));
+        load_a(k1, place(3));
+        sync_step(std::integral_constant<int, 2 * LD>{});      // the first pair landed
+      } else {
+        sync_step(WAIT_NONE{});
       }
-    };
-    auto mfmas = [&](v8i (&af)[KS][WMB], v8i (&bf)[KS][WNB]) {
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int i = 0; i < WMB; ++i)
-#pragma unroll
-          for (int j = 0; j < WNB; ++j) acc[i][j] = mfma_fp8_32(bf[ks][j], af[ks][i], acc[i][j]);
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    auto bare_barrier = [&]() { asm volatile("s_barrier" ::: "memory"); };
-    const bool late = wave >= NW / 2;     // wavefronts w and w + 4 share a SIMD (the other pairing measured 10-25 % slower)
-    v8i af[KS][WMB], bf[KS][WNB];
-#pragma unroll
-    for (int s0 = 0; s0 < NST - 1; ++s0) {
-      if (!PAIR) issue_loads(s_lo + s0, s0);
-      else if (!(s0 & 1)) issue_pair(s_lo + s0, s0, s0 + 1);
     }
-    sync_step(std::integral_constant<int, (NST - (PAIR ? 3 : 2)) * LPW>{});      // the first tile (pair) landed
     if (late) bare_barrier();
-    int cur = 0, dst = NST - 1;
-    int step = 0;
-    auto next = [](int stage) { return stage + 1 == NST ? 0 : stage + 1; };
-    if constexpr (PAIR) {
-      // Slices NST - 2 and NST - 1 ahead are requested together in every odd step, into the two stages that are free then;
-      // what has to be in LDS at the end of its read phase is everything but that pair, and after an even step nothing new.
-      static_assert(KS == 1 && (NST & 1), "one stage more than whole pairs");
-      for (; step + NST < steps; step += 2) {
-        read_frags(cur, af, bf);
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        mfmas(af, bf);
-        bare_barrier();
-        cur = next(cur);
-        issue_pair(s_lo + step + NST - 1, dst, next(dst));
-        read_frags(cur, af, bf);
-        sync_step(std::integral_constant<int, (NST - 3) * LPW>{});
-        mfmas(af, bf);
-        bare_barrier();
-        cur = next(cur);
-        dst = next(next(dst));
-      }
-      if (step + NST - 1 < steps) issue_loads(s_lo + step + NST - 1, dst);      // an odd last slice: its stage is free already
-    } else {
-      for (; step + NST - 1 < steps; ++step) {
-        issue_loads(s_lo + step + NST - 1, dst);
-        read_frags(cur, af, bf);
-        sync_step(WAIT_STEADY{});
-        mfmas(af, bf);
-        bare_barrier();
-        cur = next(cur);
-        dst = next(dst);
-      }
+    v8i af[WMB], bf[2][WNB];
+    auto places_on = [](int q) { return q >= 3 ? -3 * PLACE : 2 * PLACE; };      // from place q to the next pair's
+    int pair = 0;
+#pragma unroll 1
+    for (; pair < steps / 2; ++pair) {
+      const bool more = pair + 2 < pairs;
+      const uint32_t k = next_k();
+      read_a(0, af);
+      read_b(0, bf[0]);
+      read_b(1, bf[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) load_b(k, place(4));
+      move(adr_b, places_on(qb));
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      mfmas(af, bf[0]);
+      bare_barrier();
+      read_a(1, af);
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) load_a(k, place(0));
+      move(adr_a, places_on(qb == 4 ? 0 : qb + 1));
+      if (more) sync_step(std::integral_constant<int, 2 * LD>{});      // the next pair landed
+      else sync_step(WAIT_NONE{});
+      mfmas(af, bf[1]);
+      if (!late || 2 * pair + 2 < steps) bare_barrier();
+      qb = qb >= 3 ? qb - 3 : qb + 2;
     }
-    for (; step < steps; ++step) {      // nothing left to request: drain
-      read_frags(cur, af, bf);
-      sync_step(WAIT_NONE{});
-      mfmas(af, bf);
-      if (!(late && step == steps - 1)) bare_barrier();
-      cur = cur + 1 == NST ? 0 : cur + 1;
+    if (steps & 1) {      // half a pair
+      read_a(0, af);
+      read_b(0, bf[0]);
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      mfmas(af, bf[0]);
+      if (!late) bare_barrier();
     }
-  } else if (steps >= NST) {
+  } else if (PP == 1 && steps >= NST) {
+    // (256 x 384: the registers are full, so that stages and requests are computed step by step)
+    auto k_of = [&](int step) {
+      const int rel = step - s_lo + rot;
+      return (uint32_t)(s_lo + (rel >= steps ? rel - steps : rel)) * 64u;
+    };
+    auto issue_loads = [&](int step, int stage) {
+      uint8_t* const at = lds8 + (size_t)stage * STAGE;
+      load_a(k_of(step), at);
+      load_b(k_of(step), at + A_ST);
+    };
 #pragma unroll
     for (int s0 = 0; s0 < NST - 1; ++s0) issue_loads(s_lo + s0, s0);
-    sync_step(WAIT_STEADY{});           // tile 0 landed
+    sync_step(WAIT_STEADY{});           // the first tile landed
+    if (late) bare_barrier();
     int cur = 0, dst = NST - 1;
+    auto next = [](int stage) { return stage + 1 == NST ? 0 : stage + 1; };
+    auto at = [&](int stage) { return lds8 + (size_t)stage * STAGE; };
+    auto fragments = [&](const uint8_t* rows, auto& f) {
+#pragma unroll
+      for (int i = 0; i < (int)(sizeof(f) / sizeof(v8i)); ++i) {
+        const v4i lo = *reinterpret_cast<const v4i*>(rows + i * 2048 + coff[0]), hi = *reinterpret_cast<const v4i*>(rows + i * 2048 + coff[1]);
+        f[i] = v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      }
+    };
     int step = 0;
     for (; step + NST - 1 < steps; ++step) {
       issue_loads(s_lo + step + NST - 1, dst);
-      compute(cur);
+      v8i af[WMB], bf[WNB];
+      fragments(at(cur) + A_ST + wn * TN * 64, bf);
+      fragments(at(cur) + wm * TM * 64, af);
       sync_step(WAIT_STEADY{});
-      cur = cur + 1 == NST ? 0 : cur + 1;
-      dst = dst + 1 == NST ? 0 : dst + 1;
+      mfmas(af, bf);
+      bare_barrier();
+      cur = next(cur);
+      dst = next(dst);
     }
     for (; step < steps; ++step) {      // nothing left to request: drain
-      compute(cur);
+      v8i af[WMB], bf[WNB];
+      fragments(at(cur) + A_ST + wn * TN * 64, bf);
+      fragments(at(cur) + wm * TM * 64, af);
       sync_step(WAIT_NONE{});
-      cur = cur + 1 == NST ? 0 : cur + 1;
+      mfmas(af, bf);
+      if (!(late && step == steps - 1)) bare_barrier();
+      cur = next(cur);
+    }
+  } else if (steps >= NST) {
+#pragma unroll
+    for (int s0 = 0; s0 < NST - 1; ++s0) request(s0);
+    sync_step(WAIT_STEADY{});           // tile 0 landed
+    int cur = 0, dst = NST - 1;
+    int step = 0;
+    auto next = [](int stage) { return stage + 1 == NST ? 0 : stage + 1; };
+#pragma unroll 1
+    for (; step + NST - 1 < steps; ++step) {
+      compute((next(cur) - cur) * STAGE, [&] { request(dst); });
+      sync_step(WAIT_STEADY{});
+      cur = next(cur);
+      dst = next(dst);
+    }
+#pragma unroll 1
+    for (; step < steps; ++step) {      // nothing left to request: drain
+      compute((next(cur) - cur) * STAGE, nothing);
+      sync_step(WAIT_NONE{});
+      cur = next(cur);
     }
   } else {
     // short K: no ring, one tile at a time
     for (int step = 0; step < steps; ++step) {
-      issue_loads(s_lo + step, 0);
+      request(0);
       sync_step(WAIT_NONE{});
-      compute(0);
+      compute(0, nothing);
       sync_step(WAIT_NONE{});
     }
   }
@@ -903,6 +1027,8 @@ static int launch_tile3(const Fp8MMParams& p, hipStream_t s) {
 // time is on average 0.8 % slower than the fastest (99 of 100 less than 15 %), where rules by size were 11 % slower at M = 33 .. 1024 (4096 x 13824 at M = 384 49 -> 33 us,
 // 8192 x 4096 at M = 180 25 -> 19 us, 14336 x 2048 at M = 384 39 -> 27 us).  Constants fitted to the first half's sizes alone lost 4.3 % at
 // N > 28672 and 3.5 % at K or N below 1024 (5120 x 152064 at M = 384 400 -> 326 us, 896 x 4864 at M = 2048 24.2 -> 18.8 us with these).
+// (Timed when every shape still requested halves of lines.  4595 problems timed again with whole lines: 1.0 % with these constants, 0.8 % with new
+// ones, which over layers that stay in the memory-side cache choose worse by as much, up to 20 % where the two best plans change places.)
 constexpr TileShape FP8_TILE_SHAPES[] = {
     {13, 128, 128, 8, 1, 3.48, 0.205, 0.0739, 0, 0}, {14, 64, 128, 4, 1, 3.05, 0.161, 0.118, 0, 0},
     {15, 64, 64, 4, 2, 1.63, 0.103, 0.0209, 0.173, 0}, {16, 128, 64, 4, 1, 2.69, 0.158, 0.0327, 0, 0},
@@ -1014,8 +1140,8 @@ static int dispatch_tile(const Fp8MMParams& p_in, int64_t c_tmp_bytes, int64_t c
     }
     switch (pl.id) {
       case 1: return launch_tile3<BF16_OUT, 256, 256, 2, 4, 5, 1, 2>(p, s);    // alternating phases, slices requested in pairs (see the kernel)
-      case 10: return launch_tile3<BF16_OUT, 256, 384, 2, 4, 4, 1, 1>(p, s);   // 8 wavefronts of 128 x 96, alternating phases
       // two k-slices per step (K % 128 == 0)
+      case 10: return launch_tile3<BF16_OUT, 256, 384, 2, 4, 4, 1, 1>(p, s);   // 8 wavefronts of 128 x 96, alternating phases
       case 13: return launch_tile3<BF16_OUT, 128, 128, 2, 4, 4, 2>(p, s);
       case 14: return launch_tile3<BF16_OUT, 64, 128, 2, 2, 5, 2>(p, s);
       case 15: return launch_tile3<BF16_OUT, 64, 64, 2, 2, 5, 2>(p, s);
