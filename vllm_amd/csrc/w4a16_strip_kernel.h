@@ -81,15 +81,16 @@ __global__ __launch_bounds__(512) void w4a16_strip_kernel(const PrefillParams p)
   }
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   // step h = 2 * round + half; past the end the requests lie past the rows (zeros, no traffic) and keep the wait counts uniform
+  // (One choice a step and one addition a request: rows past M lie past the end by themselves.  A compare, two conjunctions and a select for each
+  // request cost 0.7 % in the mean over 1300 problems of M = 200 .. 4096; 4096 x 6144 at M = 333 24.9 -> 24.6 us, 4096 x 4096 at M = 512 23.2 -> 22.7.)
   auto issue_a = [&](int h, int stage, int from, int to) {
     uint8_t* Ab = lds8 + stage * STAGE + kg * (BM * 128);
     const int g = g_lo + (h >> 1) * KG + kg;
-    const uint32_t kbyte = (uint32_t)(g * 128 + (h & 1) * 64) * 2u;
+    const uint32_t kbyte = g < g_hi ? (uint32_t)(g * 128 + (h & 1) * 64) * 2u : a_bytes;
 #pragma unroll
     for (int i = from; i < to; ++i) {
       const int r0 = (ns * A_LD + i) * 8;
-      const uint32_t so = ((int)(g < g_hi) & (int)(m0 + r0 < p.M)) ? (uint32_t)(m0 + r0) * (uint32_t)p.lda * 2u + kbyte : a_bytes;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(Ab + r0 * 128), 16, (int)voff_a[i], (int)so, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(Ab + r0 * 128), 16, (int)voff_a[i], (int)((uint32_t)(m0 + r0) * (uint32_t)p.lda * 2u + kbyte), 0, 0);
     }
   };
 
