@@ -495,6 +495,24 @@ def test_scaled_mm_whole_line_requests_exact(device, cfg):
         assert torch.equal(out.cpu().float(), a @ w.t()), (cfg, m, n, k)
 
 
+@pytest.mark.parametrize("cfg", [1, 10, 13, 3])
+def test_scaled_mm_trailing_columns_exact(device, cfg):
+    """Both operands are the last columns of their storage, so that the last row ends with it; also with half a pair of slices
+    at the end of K and rows off the tile's edges."""
+    import vllm_amd._custom_ops as ops
+    from vllm_amd import _tuning
+    g = torch.Generator().manual_seed(cfg)
+    for m, n, k, off in ((256, 384, 448, 64), (131, 400, 832, 48), (300, 272, 128, 16), (257, 96, 704, 512)):
+        n = n if cfg != 10 else 384
+        a, w = torch.randint(-2, 3, (m, k), generator=g).float(), torch.randint(-1, 2, (n, k), generator=g).float()
+        wide_a, wide_w = (torch.full((x.shape[0], off + k), 0x7f, dtype=torch.uint8, device=device).view(torch.float8_e4m3fn) for x in (a, w))
+        wide_a[:, off:], wide_w[:, off:] = a.to(torch.float8_e4m3fn).to(device), w.to(torch.float8_e4m3fn).to(device)
+        with _tuning.override(fp8_path=2, fp8_tile_cfg=cfg):
+            out = ops.cutlass_scaled_mm(wide_a[:, off:], wide_w[:, off:].t(), torch.ones(m, 1, device=device), torch.ones(n, 1, device=device),
+                                        torch.float16)
+        assert torch.equal(out.cpu().float(), a @ w.t()), (cfg, m, n, k)
+
+
 @pytest.mark.parametrize("k", range(4096, 24576, 2048))
 def test_scaled_mm_automatic_parts_exact(device, k):
     """Plans of up to eight parts of K as the automatic choice makes them (five and seven among them), ragged rows."""

@@ -1,0 +1,26 @@
+"""How far a kernel's requests may reach: the buffer descriptors over operands whose rows lie further apart than they are long."""
+from __future__ import annotations
+
+import os
+import re
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "vllm_amd", "csrc")
+
+
+@pytest.mark.parametrize("source", ["fp8_scaled_mm.hip", "fp8_stream2_kernel.h", "fp8_quant_mm.hip"])
+def test_descriptors_end_with_the_last_row(source):
+    """Rows times pitch passes the end of a view of trailing columns (its last row ends with the storage), and the FP8 tile kernels request
+    whole cache lines, the last of which may lie past K: a descriptor over such an operand ends (rows - 1) * pitch + K behind its start."""
+    with open(os.path.join(CSRC, source)) as f:
+        text = re.sub(r"//[^\n]*", "", f.read())
+    spans = re.findall(r"make_buffer_rsrc\(([^;]*)\);", text)
+    assert spans or source == "fp8_quant_mm.hip"
+    assert not [s for s in spans if re.search(r"p\.(lda|ldb)", s)]
+    if source != "fp8_stream2_kernel.h":
+        extents = re.findall(r"p\.([ab])_extent = ([^;]*);", text)
+        assert extents
+        for operand, value in extents:
+            rows = "M" if operand == "a" else "N"
+            assert f"(p.{rows} - 1) * p.ld{operand} + p.K" in value, value

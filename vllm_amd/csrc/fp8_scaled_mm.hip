@@ -302,8 +302,8 @@ __global__ __launch_bounds__(256) void fp8_mm_tile2_kernel(const Fp8MMParams p) 
   const int tm = bid % tiles_m, tn = bid / tiles_m;
   const int m0 = tm * BM, n0 = tn * BN;
 
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.a), 0, (int)((uint32_t)p.M * (uint32_t)p.lda), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.b), 0, (int)((uint32_t)p.N * (uint32_t)p.ldb), 0x00020000);
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.a), 0, (int)p.a_extent, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.b), 0, (int)p.b_extent, 0x00020000);
   const int lrow = lane >> 3, lchunk = (lane & 7) ^ lrow;
   const uint32_t voff_a = (uint32_t)lrow * (uint32_t)p.lda + (uint32_t)lchunk * 16u;
   const uint32_t voff_b = (uint32_t)lrow * (uint32_t)p.ldb + (uint32_t)lchunk * 16u;
@@ -432,8 +432,8 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
   const int tm = first_m + tin % gsz, tn = tin / gsz;
   const int m0 = tm * BM, n0 = tn * BN;
 
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.a), 0, (int)((uint32_t)p.M * (uint32_t)p.lda), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.b), 0, (int)((uint32_t)p.N * (uint32_t)p.ldb), 0x00020000);
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.a), 0, (int)p.a_extent, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.b), 0, (int)p.b_extent, 0x00020000);
   // DMA instruction.  One slice: 16 rows x 64 bytes = four 256-byte lines; lane l lands in slot l: line j = r0/4 + (l >> 4), swizzled
   // chunk l & 15 -> c16 = (l & 15) ^ (j & 3), row = 4j + (c16 >> 2), chunk = c16 & 3.  r0 is a multiple of 16, so j & 3 = l >> 4.
   // Two slices (LINE): 8 rows x 128 bytes; row r0 + (l >> 3), chunk (l & 7) ^ f, f = bits 3, 1, 2 of the row in this order -> with r0 = 8 times the
@@ -1091,6 +1091,10 @@ static TilePlan plan_tile3(int M, int N, int K) {
 template <bool BF16_OUT>
 static int dispatch_tile(const Fp8MMParams& p_in, int64_t c_tmp_bytes, int64_t counter_ints, hipStream_t s) {
   Fp8MMParams p = p_in;
+  // Descriptors end with the last row and not a pitch behind its start: an operand may be the trailing columns of its storage, and the
+  // 256 x 256 tile requests 128 bytes where K leaves 64.
+  p.a_extent = (uint32_t)((int64_t)(p.M - 1) * p.lda + p.K);
+  p.b_extent = (uint32_t)((int64_t)(p.N - 1) * p.ldb + p.K);
   const bool direct_ok = tuning().fp8_tile_impl == 0 && p.K % 64 == 0 && (uint64_t)p.M * (uint64_t)p.lda < (1ull << 32) &&
                          (uint64_t)p.N * (uint64_t)p.ldb < (1ull << 32);
   if (direct_ok && tuning().fp8_tile_impl == 0 && tuning().fp8_tile_cfg >= 0) {
