@@ -24,3 +24,15 @@ def test_descriptors_end_with_the_last_row(source):
         for operand, value in extents:
             rows = "M" if operand == "a" else "N"
             assert f"(p.{rows} - 1) * p.ld{operand} + p.K" in value, value
+
+
+@pytest.mark.parametrize("source", ["w4a16_strip_kernel.h", "w4a16_prefill_kernel.h"])
+def test_descriptors_of_the_w4a16_tile_kernels_end_with_the_last_row(source):
+    """The same of their activations.  Their 32-bit offsets wrap for rows past M where the activations end close to 4 GiB: what such
+    a request finds then is at least the call's own."""
+    with open(os.path.join(CSRC, source)) as f:
+        text = re.sub(r"//[^\n]*", "", f.read())
+    spans = [s for s in re.findall(r"make_buffer_rsrc\(([^;]*)\);", text) if "p.a)" in s]
+    assert len(spans) == 1
+    extent = re.search(r"a_bytes = ([^;]*);", text).group(1) if "a_bytes" in spans[0] else spans[0]
+    assert "(uint32_t)(p.M - 1) * (uint32_t)p.lda + (uint32_t)p.K) * 2u" in extent

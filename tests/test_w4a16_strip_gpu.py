@@ -109,12 +109,12 @@ def test_strip_tiles_bias_strided_rows_and_unaligned_output(device):
 
 
 def test_strip_tiles_rows_almost_4_gib_apart(device):
-    """Activations whose last row ends just below the 4 GiB that 32-bit offsets reach; everything between the rows and behind them is
-    NaN, so that no request lands there unseen."""
+    """Activations whose last row ends with its storage, just below the 4 GiB that 32-bit offsets reach; everything between the rows is
+    NaN, so that no result takes anything from there."""
     k, n, m, pitch = 1408, 320, 127, 1 << 24
     assert (m * pitch * 2) < 1 << 32 < ((m + 1) * pitch * 2) + 1
-    base = torch.full(((m + 13) * pitch,), float("nan"), dtype=torch.bfloat16, device=device)
-    a = base[:m * pitch].view(m, pitch)[:, :k]
+    base = torch.full((m, pitch), float("nan"), dtype=torch.bfloat16, device=device)
+    a = base[:, pitch - k:]
     a.copy_(_acts(m, k, seed=4))
     for bits, group_size in ((4, 128), (8, 64)):
         case = o.make_w4a16_case(k, n, group_size, asym=bits == 4, seed=n, num_bits=bits)

@@ -500,7 +500,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void w4a16_prefill2_kernel(
 
   // ---- activation tile: direct-to-LDS loads ----
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(p.a), 0, (int)((uint32_t)p.M * (uint32_t)p.lda * 2u), 0x00020000);
+      const_cast<uint16_t*>(p.a), 0, (int)(((uint32_t)(p.M - 1) * (uint32_t)p.lda + (uint32_t)p.K) * 2u), 0x00020000);      // (no byte past the last row)
   // DMA instruction i of this wavefront fills rows r0 .. r0+7 (r0 = (wave*A_LD + i) * 8): lane l lands in LDS slot
   // r0*8 + l, i.e. row pair j = r0/2 + (l >> 4), swizzled chunk l & 15; it must therefore fetch the element that
   // belongs there: c16 = (l & 15) ^ (j & 15), row = 2j + (c16 >> 3), chunk = c16 & 7.

@@ -36,8 +36,9 @@ constexpr size_t strip_lds_bytes(int nst) {
   return stages > sums ? stages : sums;
 }
 
+// (The smallest strips with zero points of four groups: two workgroups to a compute unit, which 128 registers allow and 130 do not.)
 template <bool BF16, int WMB, int WNB, int NS, bool HAS_ZP, int SUBG, bool W8, int NST, int PD>
-__global__ __launch_bounds__(512) void w4a16_strip_kernel(const PrefillParams p) {
+__global__ __launch_bounds__(512, WMB * WNB == 1 && HAS_ZP && SUBG == 4 ? 4 : 2) void w4a16_strip_kernel(const PrefillParams p) {
   using T = F16Traits<BF16>;
   constexpr int KG = 8 / NS, BM = 32 * WMB, TN = 32 * WNB, BN = TN * NS, NW = 8;
   constexpr int TW = 2 * WNB;                      // native tiles of a strip
@@ -69,29 +70,29 @@ __global__ __launch_bounds__(512) void w4a16_strip_kernel(const PrefillParams p)
   const int t_full = ng / KG, rem = ng % KG;       // rounds in which all K groups take part; wavefronts of the last one
 
   // ---- activations: the rows of this wavefront's own K group are loaded by its NS wavefronts ----
-  const uint32_t a_bytes = (uint32_t)p.M * (uint32_t)p.lda * 2u;
+  // A descriptor of the rows' own bytes and no more: an operand may be the trailing columns of its storage.  The rows are in the lanes' offsets
+  // (up to 4 GiB, checked on the host), those past M at its far end; the scalar offset is the place in K, or all of the extent for a group past the
+  // K part: either requests nothing (zeros, no traffic) and keeps the wait counts uniform.  No sum of the two can wrap.  (Row tests and a select for
+  // every request cost 0.7 % in the mean over 1300 problems of M = 200 .. 4096; rows in the scalar offset, one addition a request, 0.3 % over 3250.)
+  const uint32_t a_bytes = ((uint32_t)(p.M - 1) * (uint32_t)p.lda + (uint32_t)p.K) * 2u;
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a), 0, (int)a_bytes, 0x00020000);
   uint32_t voff_a[A_LD];
 #pragma unroll
   for (int i = 0; i < A_LD; ++i) {
     const int j = (ns * A_LD + i) * 4 + (lane >> 4);
     const int c16 = (lane & 15) ^ (j & 15);
-    const int lrow = 2 * (lane >> 4) + (c16 >> 3);
-    voff_a[i] = ((uint32_t)lrow * (uint32_t)p.lda) * 2u + (uint32_t)(c16 & 7) * 16u;
+    const int row = m0 + (ns * A_LD + i) * 8 + 2 * (lane >> 4) + (c16 >> 3);
+    voff_a[i] = row < p.M ? ((uint32_t)row * (uint32_t)p.lda) * 2u + (uint32_t)(c16 & 7) * 16u : 0xFFFFFF00u;
   }
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
-  // step h = 2 * round + half; past the end the requests lie past the rows (zeros, no traffic) and keep the wait counts uniform
-  // (One choice a step and one addition a request: rows past M lie past the end by themselves.  A compare, two conjunctions and a select for each
-  // request cost 0.7 % in the mean over 1300 problems of M = 200 .. 4096; 4096 x 6144 at M = 333 24.9 -> 24.6 us, 4096 x 4096 at M = 512 23.2 -> 22.7.)
+  // step h = 2 * round + half
   auto issue_a = [&](int h, int stage, int from, int to) {
     uint8_t* Ab = lds8 + stage * STAGE + kg * (BM * 128);
     const int g = g_lo + (h >> 1) * KG + kg;
-    const uint32_t kbyte = g < g_hi ? (uint32_t)(g * 128 + (h & 1) * 64) * 2u : a_bytes;
+    const uint32_t so = g < g_hi ? (uint32_t)g * 256u + (uint32_t)(h & 1) * 128u : a_bytes;
 #pragma unroll
-    for (int i = from; i < to; ++i) {
-      const int r0 = (ns * A_LD + i) * 8;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(Ab + r0 * 128), 16, (int)voff_a[i], (int)((uint32_t)(m0 + r0) * (uint32_t)p.lda * 2u + kbyte), 0, 0);
-    }
+    for (int i = from; i < to; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(Ab + (ns * A_LD + i) * 1024), 16, (int)voff_a[i], (int)so, 0, 0);
   };
 
   // ---- weights ----
