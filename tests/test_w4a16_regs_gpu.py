@@ -76,6 +76,37 @@ def test_special_values_stay_in_their_rows(device):
                 assert torch.equal(got[plain], clean[plain]) and not bool(torch.isfinite(got[special]).any()), f"{shape} {split}"
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bits,group_size,asym", [(4, 128, False), (4, -1, True), (4, 64, True), (4, 32, False), (8, 128, False), (8, 32, False)])
+def test_infinite_and_huge_activations_are_those_of_the_weights(device, bits, group_size, asym, dtype):
+    """inf * w has the sign of w, and is NaN where w = 0; bf16 activations close to the largest number give finite results where the products with
+    the weights are finite (codes with their bias of 128 and more would overflow in fp32).  The other rows keep their bits."""
+    for k, n, m in ((640, 320, 21), (2688, 192, 40), (1152, 64, 4), (1536, 192, 100)):
+        case = o.make_w4a16_case(k, n, group_size, asym=asym, dtype=dtype, seed=k, num_bits=bits)
+        layer, w = W4A16Layer(case, device, dtype), o.case_w_ref(case).double()
+        a = _acts(m, k, dtype, seed=m)
+        clean = a.clone()
+        special, at = ([0, 2] if m < 6 else [0, 3, 5, m - 1]), [(131 * i + 7) % k for i in range(m)]
+        for row, value in zip(special, (float("inf"), 2.0 ** 126 if dtype == torch.bfloat16 else 4096.0, float("-inf"), float("inf"))):
+            a[row, at[row]] = value
+        a, clean = a.to(device), clean.to(device)
+        plain = [i for i in range(m) if i not in special]
+        for shape in _shapes(bits, group_size)[::3]:
+            for split in (1, 2):
+                if split > 1 and k // 128 // split < shape[2]:
+                    continue
+                what = f"{shape} {split} g={group_size} bits={bits} m={m}"
+                with _forced(shape, split):
+                    got, want = layer(a).cpu(), layer(clean).cpu()
+                assert torch.equal(got[plain], want[plain]), what
+                for row in special:
+                    ref = a[row].cpu().double() @ w
+                    if bool(torch.isfinite(a[row]).all()):      # one rounding to 16 bits of the result, fp32 sums of up to k terms beside it
+                        assert bool(((got[row].double() - ref).abs() <= ref.abs() * 2.0 ** -8 + ref.abs().max() * k * 2.0 ** -24).all()), what
+                    else:
+                        assert torch.equal(torch.nan_to_num(got[row].double(), 0.25, 1, -1), torch.nan_to_num(ref, 0.25, 1, -1)), what
+
+
 def test_bias_strided_rows_and_unaligned_output(device):
     """Bias, padded activation rows (NaN between them) and an output that is 8-byte aligned only, through the C ABI; scratch that is too small for the parts
     of K sends the call to another kernel instead of failing."""

@@ -13,6 +13,8 @@
 //    behind them in the queue wait for each: 11.6 us for the weights alone, 14.9 with them.)
 //  * Rows beyond MB * 16 are a second block of rows with workgroups of their own, side by side on the same XCD, so that they find the
 //    weights in its L2.  K may be split over workgroups: partial tiles and one arrival counter per 16 x 16 result, summed in split order.
+//  * Codes with their bias and the correction that takes it out again both overflow where an activation is infinite or close to the largest bf16
+//    number: results that are not finite are computed again with the weights themselves (regs_rounded_tile).
 //
 // Cold, us, the kernel that took them before and this one: 4096 x 28672 at M = 24 / 32 / 48 20.2 / 21.2 / 29.0 -> 17.1 / 16.9 / 21.8;
 // 14336 x 4096 at M = 48 / 64 21.7 / 25.7 -> 17.2 / 17.7; 4096 x 6144 at M = 48 / 64 10.1 / 11.0 -> 9.2 / 9.6.
@@ -48,6 +50,43 @@ constexpr size_t regs_lds_bytes(int mb, int mr, int j, int nw, int sub, bool zp)
   const size_t run = (size_t)nw * (mb * mr * 256 + 2 * (sub * 256 + (zp ? 256 : 0)));      // activations of a k-tile, scales and zero points of two
   const size_t sums = (size_t)j * mb * nw * 1024;                                      // partial results
   return run > sums ? run : sums;
+}
+
+// One 16 x 16 result of the k-tiles [g_lo, g_hi), its weights rounded to 16 bits ahead of the product as the tile kernels do it: what a call
+// gets where codes with their bias give no finite number.  (inf - inf where the weights' own signs would decide; and of bf16
+// activations beyond 2^120 the biased sums overflow, those of the weights do not.)  By one wavefront, without any prefetch.
+template <bool BF16, bool HAS_ZP, int SUBG, bool W8>
+__device__ __attribute__((always_inline)) inline v4f regs_rounded_tile(const __attribute__((address_space(4))) RegsParams& p, int nt, int row, int g_lo,
+                                                                       int g_hi, int lane) {
+  using T = F16Traits<BF16>;
+  constexpr int PL = W8 ? 2 : 1;
+  const int o = lane >> 4, r16 = lane & 15, n = nt * 16 + r16;
+  const v4u* const a = reinterpret_cast<const v4u*>(p.a + (int64_t)min(row + r16, p.M - 1) * p.lda) + o;
+  v4f sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int g = g_lo; g < g_hi; ++g) {
+    const v4u* const word = p.b + (uint32_t)(nt * p.G + g) * (uint32_t)(PL * 64);
+    const v4u w = word[(uint32_t)lane], wl = W8 ? word[(uint32_t)lane + 64] : v4u{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {
+      __builtin_amdgcn_sched_barrier(0);      // (one word after the other: this path is not to set the kernel's register count)
+      const v4u act = a[g * 16 + jj * 4];
+      const uint32_t q = (uint32_t)(g * SUBG + jj * SUBG / 4);      // (offsets below 2 GiB, as in the K loop)
+      const float s = T::to_float((p.scales + q * (uint32_t)p.s_stride)[(uint32_t)n]);
+      const int z = HAS_ZP ? (int)((p.zeros + q * (uint32_t)p.z_stride)[(uint32_t)n / 8] >> ((n & 7) * 4) & 0xFu) : W8 ? 128 : 8;
+      uint32_t aop[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        auto weight = [&](int at) {
+          const uint32_t c = W8 ? (w[jj] >> at & 0xFu) * 16u + (wl[jj] >> at & 0xFu) : w[jj] >> at & 0xFu;
+          return (uint32_t)T::from_float((float)((int)c - z) * s);
+        };
+        aop[i] = weight(4 * i) | weight(4 * i + 16) << 16;
+      }
+      sum = T::mfma16(v4u{aop[0], aop[1], aop[2], aop[3]}, act, sum);
+    }
+  }
+  return sum;
 }
 
 // MR: rows of an m-block that are fetched, 16 or, of a single one, 4 (columns of the MFMAs are independent: those of the other rows read a
@@ -244,29 +283,65 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(const RegsPara
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (what is requested past the end writes zeros into LDS)
 
   // ---- the wavefronts' parts of K, on top of the activations ----
+  const int here = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));      // the lane, not kept over the K loop
   v4f* const red = reinterpret_cast<v4f*>(lds);                                       // [NW][J * MB][64]
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < J; ++j)
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) red[(w * (J * MB) + j * MB + mb) * 64 + lane] = acc[j][mb];
+    for (int mb = 0; mb < MB; ++mb) red[(w * (J * MB) + j * MB + mb) * 64 + here] = acc[j][mb];
   __syncthreads();
   for (int q = w; q < J * MB; q += NW) {
     const int j = q / MB, mb = q - j * MB;
     const int nt = nt0 + j;
     if (nt >= p.NT || row0 + mb * 16 >= p.M) continue;
-    v4f val = red[q * 64 + lane];
+    v4f val = red[q * 64 + here];
 #pragma unroll
-    for (int s = 1; s < NW; ++s) val += red[(s * (J * MB) + q) * 64 + lane];
+    for (int s = 1; s < NW; ++s) val += red[(s * (J * MB) + q) * 64 + here];
+    const auto store = [&](v4f v) {
+      const int m = row0 + mb * 16 + (here & 15), n = nt * 16 + (here >> 4) * 4;
+      if (p.bias) {
+        const v2u bb = *reinterpret_cast<const v2u*>(p.bias + n);
+        v[0] += T::to_float((uint16_t)(bb.x & 0xffffu));
+        v[1] += T::to_float((uint16_t)(bb.x >> 16));
+        v[2] += T::to_float((uint16_t)(bb.y & 0xffffu));
+        v[3] += T::to_float((uint16_t)(bb.y >> 16));
+      }
+      v2u outv;
+      outv.x = (uint32_t)T::from_float(v[0]) | ((uint32_t)T::from_float(v[1]) << 16);
+      outv.y = (uint32_t)T::from_float(v[2]) | ((uint32_t)T::from_float(v[3]) << 16);
+      if (m < p.M) *reinterpret_cast<v2u*>(p.c + (int64_t)m * p.N + n) = outv;
+    };
+    // partial tiles and counters as in w4a16_decode2_kernel.h, step 5
+    constexpr int SC1 = 16;
+    const uint32_t units = (uint32_t)p.NT * (uint32_t)(p.RB * MB), u = (uint32_t)nt * (uint32_t)(p.RB * MB) + (uint32_t)(rb_i * MB + mb);
+    const __amdgpu_buffer_rsrc_t rt = rsrc(p.c_tmp, units * 1024u * (uint32_t)p.SK);
+    const auto give = [&](v4f v) {
+      if (p.SK > 1) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, v), rt, here * 16, (int)(((uint32_t)sk * units + u) * 1024u), SC1);
+      else store(v);
+    };
+    give(val);
+    // A result that is not finite is computed again, behind its store, which waits for nothing then.  (Test and inlined path cost calls that go to this
+    // kernel 0.2 % in the mean over 8750 drawn ones; ahead of the store 0.4 %, in a function that is called 0.6 %.)
+    const float all = fabsf(val[0]) + fabsf(val[1]) + fabsf(val[2]) + fabsf(val[3]);
+    if (__builtin_expect(__ballot(!__builtin_isfinite(all)) != 0, 0)) {
+      // (The arguments are read again, behind a statement that hides where they are: what only this path needs takes no registers in the K loop.
+      // The pointer is the kernel's; in a function that is called it would be null.)
+      auto args = __builtin_amdgcn_kernarg_segment_ptr();
+#ifdef __HIP_DEVICE_COMPILE__
+      asm volatile("" : "+s"(args));
+#endif
+      const v4f again = regs_rounded_tile<BF16, HAS_ZP, SUBG, W8>(*(const __attribute__((address_space(4))) RegsParams*)args, nt, row0 + mb * 16, g_lo, g_hi, here);
+      v4f mended = val;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (!__builtin_isfinite(val[r])) mended[r] = again[r];
+      give(mended);
+    }
     if (p.SK > 1) {
-      // partial tiles and counters as in w4a16_decode2_kernel.h, step 5
-      constexpr int SC1 = 16;
-      const uint32_t units = (uint32_t)p.NT * (uint32_t)(p.RB * MB), u = (uint32_t)nt * (uint32_t)(p.RB * MB) + (uint32_t)(rb_i * MB + mb);
-      const __amdgpu_buffer_rsrc_t rt = rsrc(p.c_tmp, units * 1024u * (uint32_t)p.SK);
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, val), rt, lane * 16, (int)(((uint32_t)sk * units + u) * 1024u), SC1);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // partial tile acknowledged before the counter moves
       int old = 0;
-      if (lane == 0) old = __hip_atomic_fetch_add(&p.counters[u], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (here == 0) old = __hip_atomic_fetch_add(&p.counters[u], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       old = __builtin_amdgcn_readfirstlane(old);
       if (old != p.SK - 1) continue;
       val = v4f{0.f, 0.f, 0.f, 0.f};
@@ -274,25 +349,14 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(const RegsPara
         v4u part[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          part[i] = __builtin_amdgcn_raw_buffer_load_b128(rt, lane * 16, (int)(((uint32_t)min(s0 + i, p.SK - 1) * units + u) * 1024u), SC1);
+          part[i] = __builtin_amdgcn_raw_buffer_load_b128(rt, here * 16, (int)(((uint32_t)min(s0 + i, p.SK - 1) * units + u) * 1024u), SC1);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           if (s0 + i < p.SK) val += __builtin_bit_cast(v4f, part[i]);
       }
-      if (lane == 0) __hip_atomic_store(&p.counters[u], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (here == 0) __hip_atomic_store(&p.counters[u], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      store(val);
     }
-    const int m = row0 + mb * 16 + r16, n = nt * 16 + o * 4;
-    if (p.bias) {
-      const v2u bb = *reinterpret_cast<const v2u*>(p.bias + n);
-      val[0] += T::to_float((uint16_t)(bb.x & 0xffffu));
-      val[1] += T::to_float((uint16_t)(bb.x >> 16));
-      val[2] += T::to_float((uint16_t)(bb.y & 0xffffu));
-      val[3] += T::to_float((uint16_t)(bb.y >> 16));
-    }
-    v2u outv;
-    outv.x = (uint32_t)T::from_float(val[0]) | ((uint32_t)T::from_float(val[1]) << 16);
-    outv.y = (uint32_t)T::from_float(val[2]) | ((uint32_t)T::from_float(val[3]) << 16);
-    if (m < p.M) *reinterpret_cast<v2u*>(p.c + (int64_t)m * p.N + n) = outv;
   }
 }
 
