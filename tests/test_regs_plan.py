@@ -92,3 +92,11 @@ def test_scratch_of_every_plan_fits_the_library_owned_one():
             assert sizes[0].value >= tmp and sizes[2].value >= counters
             split += sk > 1
     assert split > 10
+
+
+@pytest.mark.parametrize("k,m4,m16", [(512, 26.5, 27.2), (1024, 33.4, 34.0), (2048, 38.0, 39.4), (3072, 47.6, 50.3), (4096, 54.9, 59.0), (5120, 153.7, 155.2)])
+def test_vocabulary_layers_are_weighed_against_the_kernel_that_runs(k, m4, m16):
+    """N from 65536 on, 3 .. 16 rows: without this kernel the register-resident one runs (timed us at N = 128256, cold), not the LDS-staged one."""
+    for m, us in ((4, m4), (16, m16)):
+        *_, other, takes = _plan(m, 128256, k, 1, 0)
+        assert abs(other / us - 1) < 0.25 and takes

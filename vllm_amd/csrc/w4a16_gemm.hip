@@ -50,6 +50,12 @@ static int check_format(int64_t size_k, int group_size, int wtype, int* wt, int*
 static int other_kind(int M, int N, int K, int sub, int wt, double* us) {
   const bool w8 = wt != 0, plain = sub == 1 && !w8;
   int kind = D2_WORKGROUP;
+  // 3 .. 16 rows of a vocabulary-sized layer: the register-resident kernel.  A launch, for every 1000 columns its walk, the weights, and those times the
+  // rows, and a hand-over for each started 4096 rows of K beyond the first; 10 % rms over 7.4e4 timings of K 256 .. 20480, N 65536 .. 152064.
+  if (decode_impl_for(M, N, K, sub, w8) == 1) {
+    *us = 3.08 + N * 1e-3 * (0.152 + K / 1024.0 * (0.0654 + 0.0084 * M / 16) + 0.556 * ((K + 4095) / 4096 - 1));
+    return kind;
+  }
   if (M > 16) {
     const int most = !plain ? DECODE_MAX_M_2BLK : N > 8192 ? 48 : DECODE_MAX_M;
     kind = w4a16_decode2_choose(M, N, K, sub, wt, false, M <= most, true, w4a16_staged_us(M, N, K, plain));
@@ -61,10 +67,12 @@ static int other_kind(int M, int N, int K, int sub, int wt, double* us) {
 // Whether the kernel with activations in registers takes a problem: where it is predicted to be ahead of what takes it otherwise by so much that
 // few calls lose.  4-bit codes in groups of 128 rows 15 % up to 4 rows and 13 % up to 32, where the decode kernel's plans by rule are on some
 // layers that much better than priced (14336 x 4096 at M = 4 9.0 us, priced 9.9; this kernel 10.0, priced 8.7), 5 % up to 64 rows and 8 % beyond;
+// vocabulary-sized layers at 3 .. 16 rows, where another kernel is the alternative, 5 % (it takes them all: 0.37 .. 0.96 of the time, 1 of 2000 more than 3 %
+// slower; 4096 x 128256 at M = 4 / 16 54.9 / 59.0 -> 51.9 / 53.4 us, 1024 x 128256 33.4 / 34.0 -> 18.1 / 19.5, 5120 x 65536 80.0 / 81.0 -> 33.2 / 34.7);
 // in groups of 64 / 32 rows 12 % from 33 rows on, where zero points cost more than priced; all others 5 %.  Over 20254 calls of drawn layers that
 // it took at 5 % where it now asks for 8 and 12, timed both ways afterwards: 0.842 of their time in the mean, 3.9 % more than 3 % slower, 0.5 % more than 10 %.
-static double regs_lead(int M, int sub, int wt) {
-  if (wt != 0) return 0.95;
+static double regs_lead(int M, int N, int K, int sub, int wt) {
+  if (wt != 0 || decode_impl_for(M, N, K, sub, false) == 1) return 0.95;
   if (sub > 1) return M > 32 ? 0.88 : 0.95;
   return M <= 4 ? 0.85 : M <= 32 ? 0.87 : M <= 64 ? 0.95 : 0.92;
 }
@@ -73,7 +81,7 @@ bool w4a16_takes_regs(int M, int N, int K, int sub, int wt, double* other) {
   const double us = w4a16_regs_us(M, N, K, sub, wt);
   if (us < 0) return false;
   other_kind(M, N, K, sub, wt, other);
-  return us < *other * regs_lead(M, sub, wt);
+  return us < *other * regs_lead(M, N, K, sub, wt);
 }
 
 // The same for a call, from a table per thread.  A switch that names another kernel or a plan of one keeps it out; exp[8] asks for it.
