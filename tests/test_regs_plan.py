@@ -100,3 +100,10 @@ def test_vocabulary_layers_are_weighed_against_the_kernel_that_runs(k, m4, m16):
     for m, us in ((4, m4), (16, m16)):
         *_, other, takes = _plan(m, 128256, k, 1, 0)
         assert abs(other / us - 1) < 0.25 and takes
+
+
+@pytest.mark.parametrize("k,n,m,takes", [(4096, 4096, 16, 0), (4096, 3072, 16, 0), (2048, 10240, 16, 0), (2048, 4608, 32, 0), (11008, 3584, 1, 0), (13824, 3584, 2, 0),
+                                         (4096, 6144, 4, 1), (4096, 6144, 16, 1), (5120, 5120, 1, 1), (5120, 5120, 16, 1), (4096, 4096, 24, 1), (4096, 28672, 32, 1)])
+def test_layers_where_one_kernel_is_well_ahead(k, n, m, takes):
+    """Timed 4 .. 11 % behind and 5 .. 25 % ahead of the decode kernel."""
+    assert _plan(m, n, k, 1, 0)[-1] == takes

@@ -71,17 +71,32 @@ static int other_kind(int M, int N, int K, int sub, int wt, double* us) {
 // slower; 4096 x 128256 at M = 4 / 16 54.9 / 59.0 -> 51.9 / 53.4 us, 1024 x 128256 33.4 / 34.0 -> 18.1 / 19.5, 5120 x 65536 80.0 / 81.0 -> 33.2 / 34.7);
 // in groups of 64 / 32 rows 12 % from 33 rows on, where zero points cost more than priced; all others 5 %.  Over 20254 calls of drawn layers that
 // it took at 5 % where it now asks for 8 and 12, timed both ways afterwards: 0.842 of their time in the mean, 3.9 % more than 3 % slower, 0.5 % more than 10 %.
-static double regs_lead(int M, int N, int K, int sub, int wt) {
+static double regs_lead(int M, int N, int K, int sub, int wt, int j, int nw) {
   if (wt != 0 || decode_impl_for(M, N, K, sub, false) == 1) return 0.95;
   if (sub > 1) return M > 32 ? 0.88 : 0.95;
-  return M <= 4 ? 0.85 : M <= 32 ? 0.87 : M <= 64 ? 0.95 : 0.92;
+  if (M > 32) return M <= 64 ? 0.95 : 0.92;
+  const double lead = M <= 4 ? 0.85 : 0.87;
+  // Where this kernel loses most of what it loses, by as much as the two prices together are off by: K of whole 1024 rows; one n-tile to a wavefront and K
+  // beyond 8192 at up to 4 rows; two and more n-tiles on a short K.  Off are: this kernel's price, which counts 16 rows to a block, by the rows that a block has;
+  // for workgroups of four; for one n-tile, which leaves 2 KB of weights in flight, by how much of the device waits for them and how long; for three and more
+  // on a short K; the other's by what it fetches for one to four rows.  Fitted to 60520 + 860 timings of either, 6.6 % rms.  Over 33847 random ones
+  // 2.0 -> 1.2 % of the calls lose more than 3 % (ordinary K and N, 75288: 2.5 -> 0.8); 1.4 % (3.2) go back to the decode kernel, 2.6 % ahead on them in the
+  // mean: 4096 x 4096 at M = 16 5.5 -> 5.3 us, 2048 x 10240 6.1 -> 5.6, 11008 x 4096 at M = 1 8.4 -> 7.7, 13824 x 3584 at M = 2 9.6 -> 8.8.  Asked of
+  // every K and plan it would send back as many that gain (K = 1152 .. 1536: +10 %).
+  if (!(K % 1024 == 0 || (M <= 4 && j == 1 && K > 8192) || (K <= 2048 && ((j == 2 && K >= 1024) || (j >= 3 && K > 1536))))) return lead;
+  const double lk = log2(K / 4096.0), full = j == 1 ? fmin(1.0, N / 16.0 / num_cus_current_device()) : 0;
+  const double off = 0.031 + 0.109 * ((M - 1) % 16 + 1) / 16 + (M <= 4 ? 0.044 : 0) - (nw == 4 ? 0.061 : 0) - 0.019 * lk +
+                     full * (0.038 + 0.075 * fmax(0.0, lk)) + (j >= 3 && K <= 2048 && N >= 4096 ? 0.046 : 0);
+  const double by_price = exp(-0.01 - off);
+  return lead < by_price ? lead : by_price;
 }
 bool w4a16_takes_regs(int M, int N, int K, int sub, int wt, double* other) {
   const TuningScope automatic(nullptr);
-  const double us = w4a16_regs_us(M, N, K, sub, wt);
+  int j = 0, nw = 0;
+  const double us = w4a16_regs_us(M, N, K, sub, wt, &j, &nw);
   if (us < 0) return false;
   other_kind(M, N, K, sub, wt, other);
-  return us < *other * regs_lead(M, N, K, sub, wt);
+  return us < *other * regs_lead(M, N, K, sub, wt, j, nw);
 }
 
 // The same for a call, from a table per thread.  A switch that names another kernel or a plan of one keeps it out; exp[8] asks for it.

@@ -91,10 +91,13 @@ static RegsPlan regs_plan(int M, int N, int K, int sub, bool w8) {
   return table.get(M, N, K, (num_cus_current_device() * 8 + sub) * 2 + (w8 ? 1 : 0), [&] { return make_regs_plan(M, N, K, sub, w8); });
 }
 
-double w4a16_regs_us(int M, int N, int K, int sub, int wt) {
+double w4a16_regs_us(int M, int N, int K, int sub, int wt, int* n_tiles, int* wavefronts) {
   // 32-bit offsets with the top bit to spare: it is what a request for nothing sets
   if (M > REGS_MAX_M || wt == 2 || (uint64_t)K * N / (wt == 1 ? 1 : 2) >= (1ull << 31) || (uint64_t)K * N * 2 / 32 >= (1ull << 31)) return -1;
-  return regs_plan(M, N, K, sub, wt == 1).us;
+  const RegsPlan p = regs_plan(M, N, K, sub, wt == 1);
+  if (n_tiles) *n_tiles = p.j;
+  if (wavefronts) *wavefronts = p.nw;
+  return p.us;
 }
 
 void w4a16_regs_workspace(int M, int N, int K, int sub, bool w8, size_t* c_tmp_bytes, size_t* counter_ints) {
