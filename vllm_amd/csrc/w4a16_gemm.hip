@@ -229,6 +229,17 @@ extern "C" int vaq_w4a16_gemm_tuned(const void* a, int64_t lda, const int32_t* b
   VAQ_CHECK_ARG(!bias || ((uintptr_t)bias % 8) == 0, "w4a16_gemm: bias must be 8-byte aligned");
   hipStream_t s = (hipStream_t)stream;
 
+  // The kernel with operands in registers first: a call that it takes looks up none of the other plans.  (One that brings too little scratch for its parts of K
+  // goes on to the others; so does one whose rows end beyond 2 GiB.)
+  if (force_path == 0 && perm == nullptr && size_m <= REGS_MAX_M && size_m * lda * 2 < (1ll << 31) &&
+      regs_chosen((int)size_m, (int)size_n, (int)size_k, sub, wt)) {
+    size_t t = 0, n = 0;
+    w4a16_regs_workspace((int)size_m, (int)size_n, (int)size_k, sub, w8, &t, &n);
+    if ((t == 0 && n == 0) || (c_tmp != nullptr && counters != nullptr && (uintptr_t)c_tmp % 16 == 0 && c_tmp_bytes >= (int64_t)t && counter_ints >= (int64_t)n))
+      return w4a16_regs_launch(a, lda, b, scales, zeros, bias, c, c_tmp, counters, (int)size_m, (int)size_n, (int)size_k, sub, channelwise,
+                               w8, dtype, s);
+  }
+
   // three and four m-blocks exist on the LDS-staged kernel for 4-bit codes in groups of 128 rows / channelwise
   const bool two_blocks_only = sub > 1 || w8 || decode_impl_for(size_m, size_n, lda, sub, w8) != 0;
   // (measured: four m-blocks beat the tile kernel by 1.5-2x on the narrow layers and lose 3 % on a 28672-wide one)
@@ -252,15 +263,6 @@ extern "C" int vaq_w4a16_gemm_tuned(const void* a, int64_t lda, const int32_t* b
                                           w4a16_staged_us((int)size_m, (int)size_n, (int)size_k, !w8 && sub == 1));
     decode = kind != D2_TILE;
     rows = kind == D2_ROWS;
-  }
-  // (a call that brings too little scratch for its parts of K goes where it went without this kernel; so does one whose rows end beyond 2 GiB)
-  if (force_path == 0 && perm == nullptr && size_m <= REGS_MAX_M && size_m * lda * 2 < (1ll << 31) &&
-      regs_chosen((int)size_m, (int)size_n, (int)size_k, sub, wt)) {
-    size_t t = 0, n = 0;
-    w4a16_regs_workspace((int)size_m, (int)size_n, (int)size_k, sub, w8, &t, &n);
-    if ((t == 0 && n == 0) || (c_tmp != nullptr && counters != nullptr && (uintptr_t)c_tmp % 16 == 0 && c_tmp_bytes >= (int64_t)t && counter_ints >= (int64_t)n))
-      return w4a16_regs_launch(a, lda, b, scales, zeros, bias, c, c_tmp, counters, (int)size_m, (int)size_n, (int)size_k, sub, channelwise,
-                               w8, dtype, s);
   }
   if (decode && decode_impl_for(size_m, size_n, lda, sub, w8) == 0)
     return w4a16_decode2_launch(a, lda, b, scales, zeros, perm, bias, c, c_tmp, c_tmp_bytes, counters, counter_ints, (int)size_m,
