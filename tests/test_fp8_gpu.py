@@ -476,16 +476,17 @@ def test_scaled_mm_slices_requested_together_exact(device, cfg):
     assert all(bool((t == 0).all()) for t in ops._FP8_COUNTERS.values()), "arrival counters not restored to zero"
 
 
-@pytest.mark.parametrize("cfg", [1, 13, 14, 16, 17, 19])
-def test_scaled_mm_whole_line_requests_exact(device, cfg):
-    """The shapes that request whole lines of both operands: every number of slices from one to the second turn of the ring, odd ones (the 256 x 256
-    tiles fetch half a pair that they must not read), rows and columns off the tile's edges, rotated starts, operands whose rows
-    lie further apart than K with NaN codes between them.  Small integers: the result must equal the integer GEMM."""
+@pytest.mark.parametrize("cfg,depth", [(1, 5), (13, 4), (14, 5), (15, 5), (16, 5), (17, 3), (19, 3)])
+def test_scaled_mm_whole_line_requests_exact(device, cfg, depth):
+    """The shapes that request whole lines of both operands (a K step of 128 bytes; the 256 x 256 tiles take two steps of 64 for one, and fetch the half behind an
+    odd last one that they must not read): every number of steps from one to past the second turn of the ring, one in parts of K, rows and columns off the tile's
+    edges, operands whose rows lie further apart than K with NaN codes between them.  Small integers: the result must equal the integer GEMM."""
     import vllm_amd._custom_ops as ops
     from vllm_amd import _tuning
     g = torch.Generator().manual_seed(cfg)
-    for steps in (1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 13):
-        m, n, k, split = 1 + 97 * steps % 600, 16 + 112 * steps % 560, 64 * steps, 2 if steps in (8, 13) else 1
+    unit = 64 if cfg == 1 else 128
+    for steps in range(1, 2 * depth + 2):
+        m, n, k, split = 1 + 97 * steps % 600, 16 + 112 * steps % 560, unit * steps, 2 if steps in (2 * depth, 2 * depth + 1) else 1
         a, w = torch.randint(-2, 3, (m, k), generator=g).float(), torch.randint(-1, 2, (n, k), generator=g).float()
         wide_a, wide_w = (torch.full((x.shape[0], k + 64), 0x7f, dtype=torch.uint8, device=device).view(torch.float8_e4m3fn) for x in (a, w))
         wide_a[:, :k], wide_w[:, :k] = a.to(torch.float8_e4m3fn).to(device), w.to(torch.float8_e4m3fn).to(device)

@@ -678,8 +678,9 @@ def test_decode_n_tiles_grouped_by_xcd_same_bits(device, k, n):
     w_ref = o.case_w_ref(case)
     for m in (1, 4, 16, 32, 48):
         a = _acts(m, k, device, seed=m)
-        out = layer(a)
-        with _tuning.override(exp=[0] * 7 + [1]):
+        with _tuning.override(exp=[0] * 8 + [1]):      # (not the kernel with operands in registers, which takes some of these calls)
+            out = layer(a)
+        with _tuning.override(exp=[0] * 7 + [1, 1]):
             plain = layer(a)
         assert torch.equal(out, plain), (k, n, m)
         check_gemm_close(out, o.gemm_ref(a.cpu(), w_ref), f"k={k} n={n} m={m}")

@@ -141,17 +141,3 @@ def test_bias_strided_rows_and_unaligned_output(device):
                     check_gemm_close(buf[4:4 + m * n].view(m, n), ref, f"shape {shape} split {split} k={k} n={n} m={m}")
                     assert bool((buf[:4] == 0).all()) and bool((buf[4 + m * n:] == 0).all()), "stores outside the output"
         assert bool((counters == 0).all())
-
-
-@pytest.mark.parametrize("k,n", [(4096, 6144), (2048, 1984), (14336, 4096)])
-def test_decode_kernel_n_tiles_grouped_by_xcd_without_this_kernel(device, k, n):
-    """The decode kernel's order of n-tiles on the sizes that this kernel takes from it: the same bits with and without the grouping."""
-    from vllm_amd import _tuning
-    layer = W4A16Layer(o.make_w4a16_case(k, n, 128, asym=True, seed=k + n), device)
-    for m in (1, 4, 16, 32, 48):
-        a = _acts(m, k, seed=m).to(device)
-        outs = []
-        for off in (0, 1):
-            with _tuning.override(exp=[0] * 7 + [off, 1]):
-                outs.append(layer(a))
-        assert torch.equal(*outs), (k, n, m)
