@@ -652,7 +652,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
     // reads and MFMAs and by the power limit: with all operands zero 4096^3 takes 0.7 of the time, without any MFMA half.
     static_assert(BM == BN && NST == 5, "five places of one size");
     constexpr int LD = BM / (8 * NW);                          // requests of a wavefront for an operand of a pair
-    const int pairs = (steps + 1) / 2;                         // (the last one may be half a pair: its other slice is fetched and not read)
+    const int pairs = (steps + 1) / 2;                         // (the last one may be half a pair: what follows it is requested, up to the end of the operand, and not read)
     int qb = 0;                                                // place of the pair at hand's weights
     auto place = [&](int ahead) {                              // that of the operand `ahead` places on
       const int q = qb + ahead;
@@ -1144,8 +1144,8 @@ static int dispatch_tile(const Fp8MMParams& p_in, int64_t c_tmp_bytes, int64_t c
     }
     switch (pl.id) {
       case 1: return launch_tile3<BF16_OUT, 256, 256, 2, 4, 5, 1, 2>(p, s);    // alternating phases, slices requested in pairs (see the kernel)
+      case 10: return launch_tile3<BF16_OUT, 256, 384, 2, 4, 4, 1, 1>(p, s);   // 8 wavefronts of 128 x 96, alternating phases, one slice at a time
       // two k-slices per step (K % 128 == 0)
-      case 10: return launch_tile3<BF16_OUT, 256, 384, 2, 4, 4, 1, 1>(p, s);   // 8 wavefronts of 128 x 96, alternating phases
       case 13: return launch_tile3<BF16_OUT, 128, 128, 2, 4, 4, 2>(p, s);
       case 14: return launch_tile3<BF16_OUT, 64, 128, 2, 2, 5, 2>(p, s);
       case 15: return launch_tile3<BF16_OUT, 64, 64, 2, 2, 5, 2>(p, s);
