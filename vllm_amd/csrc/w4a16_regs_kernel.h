@@ -52,19 +52,18 @@ constexpr size_t regs_lds_bytes(int mb, int mr, int j, int nw, int sub, bool zp)
   return run > sums ? run : sums;
 }
 
-// One 16 x 16 result of the k-tiles [g_lo, g_hi), its weights rounded to 16 bits ahead of the product as the tile kernels do it: what a call
-// gets where codes with their bias give no finite number.  (inf - inf where the weights' own signs would decide; and of bf16
+// One 16 x 16 result, all of K, its weights rounded to 16 bits ahead of the product as the tile kernels do it: what a call gets where codes with
+// their bias give no finite number.  (inf - inf where the weights' own signs would decide; and of bf16
 // activations beyond 2^120 the biased sums overflow, those of the weights do not.)  By one wavefront, without any prefetch.
 template <bool BF16, bool HAS_ZP, int SUBG, bool W8>
-__device__ __attribute__((always_inline)) inline v4f regs_rounded_tile(const __attribute__((address_space(4))) RegsParams& p, int nt, int row, int g_lo,
-                                                                       int g_hi, int lane) {
+__device__ __attribute__((always_inline)) inline v4f regs_rounded_tile(const __attribute__((address_space(4))) RegsParams& p, int nt, int row, int lane) {
   using T = F16Traits<BF16>;
   constexpr int PL = W8 ? 2 : 1;
   const int o = lane >> 4, r16 = lane & 15, n = nt * 16 + r16;
   const v4u* const a = reinterpret_cast<const v4u*>(p.a + (int64_t)min(row + r16, p.M - 1) * p.lda) + o;
   v4f sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-  for (int g = g_lo; g < g_hi; ++g) {
+  for (int g = 0; g < p.G; ++g) {
     const v4u* const word = p.b + (uint32_t)(nt * p.G + g) * (uint32_t)(PL * 64);
     const v4u w = word[(uint32_t)lane], wl = W8 ? word[(uint32_t)lane + 64] : v4u{0u, 0u, 0u, 0u};
 #pragma unroll
@@ -87,6 +86,43 @@ __device__ __attribute__((always_inline)) inline v4f regs_rounded_tile(const __a
     }
   }
   return sum;
+}
+
+// The sum of the wavefronts' parts of result q in LDS, and of the parts of K in c_tmp (four in flight, added in split order).
+template <int NW>
+__device__ __attribute__((always_inline)) inline v4f regs_sum(const v4f* red, int results, int q, int lane) {
+  v4f val = red[q * 64 + lane];
+#pragma unroll
+  for (int s = 1; s < NW; ++s) val += red[(s * results + q) * 64 + lane];
+  return val;
+}
+__device__ __attribute__((always_inline)) inline v4f regs_sum_parts(const __amdgpu_buffer_rsrc_t rt, uint32_t units, uint32_t u, int SK, int lane) {
+  v4f val = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < SK; s0 += 4) {
+    v4u part[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      part[i] = __builtin_amdgcn_raw_buffer_load_b128(rt, lane * 16, (int)(((uint32_t)min(s0 + i, SK - 1) * units + u) * 1024u), 16);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (s0 + i < SK) val += __builtin_bit_cast(v4f, part[i]);
+  }
+  return val;
+}
+template <bool BF16, class Params>
+__device__ __attribute__((always_inline)) inline void regs_store(const Params& p, v4f val, int m, int n) {
+  using T = F16Traits<BF16>;
+  if (p.bias) {
+    const v2u bb = *reinterpret_cast<const v2u*>(p.bias + n);
+    val[0] += T::to_float((uint16_t)(bb.x & 0xffffu));
+    val[1] += T::to_float((uint16_t)(bb.x >> 16));
+    val[2] += T::to_float((uint16_t)(bb.y & 0xffffu));
+    val[3] += T::to_float((uint16_t)(bb.y >> 16));
+  }
+  v2u outv;
+  outv.x = (uint32_t)T::from_float(val[0]) | ((uint32_t)T::from_float(val[1]) << 16);
+  outv.y = (uint32_t)T::from_float(val[2]) | ((uint32_t)T::from_float(val[3]) << 16);
+  if (m < p.M) *reinterpret_cast<v2u*>(p.c + (int64_t)m * p.N + n) = outv;
 }
 
 // MR: rows of an m-block that are fetched, 16 or, of a single one, 4 (columns of the MFMAs are independent: those of the other rows read a
@@ -269,6 +305,10 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(const RegsPara
 #pragma unroll
   for (int j = 0; j < J; ++j) load_w(1, at(g + NW), j);
   __builtin_amdgcn_sched_barrier(0);
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("" ::"s"(msk), "s"(p.bias), "s"(p.c), "s"(p.c_tmp), "s"(p.counters), "s"(p.N), "s"(p.NT));      // (arrived before the K loop: with
+  // a scalar load under way its waits for LDS reads are for all of them at once, and loads ahead of the last k-tile were waited for; 0.1 us)
+#endif
 #pragma unroll 1
   for (; g + NW < g_hi; g += 2 * NW) {
     wait();
@@ -291,71 +331,52 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(const RegsPara
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) red[(w * (J * MB) + j * MB + mb) * 64 + here] = acc[j][mb];
   __syncthreads();
-  for (int q = w; q < J * MB; q += NW) {
+  uint32_t odd = 0;      // a bit for each result of this wavefront that is not finite
+  for (int q = w, bit = 1; q < J * MB; q += NW, bit <<= 1) {
     const int j = q / MB, mb = q - j * MB;
     const int nt = nt0 + j;
     if (nt >= p.NT || row0 + mb * 16 >= p.M) continue;
-    v4f val = red[q * 64 + here];
-#pragma unroll
-    for (int s = 1; s < NW; ++s) val += red[(s * (J * MB) + q) * 64 + here];
-    const auto store = [&](v4f v) {
-      const int m = row0 + mb * 16 + (here & 15), n = nt * 16 + (here >> 4) * 4;
-      if (p.bias) {
-        const v2u bb = *reinterpret_cast<const v2u*>(p.bias + n);
-        v[0] += T::to_float((uint16_t)(bb.x & 0xffffu));
-        v[1] += T::to_float((uint16_t)(bb.x >> 16));
-        v[2] += T::to_float((uint16_t)(bb.y & 0xffffu));
-        v[3] += T::to_float((uint16_t)(bb.y >> 16));
-      }
-      v2u outv;
-      outv.x = (uint32_t)T::from_float(v[0]) | ((uint32_t)T::from_float(v[1]) << 16);
-      outv.y = (uint32_t)T::from_float(v[2]) | ((uint32_t)T::from_float(v[3]) << 16);
-      if (m < p.M) *reinterpret_cast<v2u*>(p.c + (int64_t)m * p.N + n) = outv;
-    };
-    // partial tiles and counters as in w4a16_decode2_kernel.h, step 5
-    constexpr int SC1 = 16;
-    const uint32_t units = (uint32_t)p.NT * (uint32_t)(p.RB * MB), u = (uint32_t)nt * (uint32_t)(p.RB * MB) + (uint32_t)(rb_i * MB + mb);
-    const __amdgpu_buffer_rsrc_t rt = rsrc(p.c_tmp, units * 1024u * (uint32_t)p.SK);
-    const auto give = [&](v4f v) {
-      if (p.SK > 1) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, v), rt, here * 16, (int)(((uint32_t)sk * units + u) * 1024u), SC1);
-      else store(v);
-    };
-    give(val);
-    // A result that is not finite is computed again, behind its store, which waits for nothing then.  (Test and inlined path cost calls that go to this
-    // kernel 0.2 % in the mean over 8750 drawn ones; ahead of the store 0.4 %, in a function that is called 0.6 %.)
-    const float all = fabsf(val[0]) + fabsf(val[1]) + fabsf(val[2]) + fabsf(val[3]);
-    if (__builtin_expect(__ballot(!__builtin_isfinite(all)) != 0, 0)) {
-      // (The arguments are read again, behind a statement that hides where they are: what only this path needs takes no registers in the K loop.
-      // The pointer is the kernel's; in a function that is called it would be null.)
-      auto args = __builtin_amdgcn_kernarg_segment_ptr();
-#ifdef __HIP_DEVICE_COMPILE__
-      asm volatile("" : "+s"(args));
-#endif
-      const v4f again = regs_rounded_tile<BF16, HAS_ZP, SUBG, W8>(*(const __attribute__((address_space(4))) RegsParams*)args, nt, row0 + mb * 16, g_lo, g_hi, here);
-      v4f mended = val;
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (!__builtin_isfinite(val[r])) mended[r] = again[r];
-      give(mended);
-    }
+    v4f val = regs_sum<NW>(red, J * MB, q, here);
     if (p.SK > 1) {
+      // partial tiles and counters as in w4a16_decode2_kernel.h, step 5
+      const uint32_t units = (uint32_t)p.NT * (uint32_t)(p.RB * MB), u = (uint32_t)nt * (uint32_t)(p.RB * MB) + (uint32_t)(rb_i * MB + mb);
+      const __amdgpu_buffer_rsrc_t rt = rsrc(p.c_tmp, units * 1024u * (uint32_t)p.SK);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, val), rt, here * 16, (int)(((uint32_t)sk * units + u) * 1024u), 16);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // partial tile acknowledged before the counter moves
       int old = 0;
       if (here == 0) old = __hip_atomic_fetch_add(&p.counters[u], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       old = __builtin_amdgcn_readfirstlane(old);
       if (old != p.SK - 1) continue;
-      val = v4f{0.f, 0.f, 0.f, 0.f};
-      for (int s0 = 0; s0 < p.SK; s0 += 4) {               // four parts in flight, added in split order
-        v4u part[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          part[i] = __builtin_amdgcn_raw_buffer_load_b128(rt, here * 16, (int)(((uint32_t)min(s0 + i, p.SK - 1) * units + u) * 1024u), SC1);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (s0 + i < p.SK) val += __builtin_bit_cast(v4f, part[i]);
-      }
+      val = regs_sum_parts(rt, units, u, p.SK, here);
       if (here == 0) __hip_atomic_store(&p.counters[u], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      store(val);
+    }
+    regs_store<BF16>(p, val, row0 + mb * 16 + (here & 15), nt * 16 + (here >> 4) * 4);
+    const float all = fabsf(val[0]) + fabsf(val[1]) + fabsf(val[2]) + fabsf(val[3]);
+    odd |= __ballot(!__builtin_isfinite(all)) != 0 ? (uint32_t)bit : 0u;
+  }
+  if (__builtin_expect(odd != 0, 0)) {
+    // The results that are not finite once more, behind their stores.  The arguments are read again and everything is made from values that a statement
+    // hides, so that nothing of this is computed, or kept in registers, ahead.  (Tested ahead of each store,
+    // or with the path inside the loop over results, calls that go to this kernel took 1.002 .. 1.006 of their time in the mean; in a function that is called 1.006; so
+    // 0.997.)  The pointer is the kernel's; in a function that is called it
+    // would be null.
+    auto args = __builtin_amdgcn_kernarg_segment_ptr();
+    int q = w, nt_h = nt0, row_h = row0, rb_h = rb_i;
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("" : "+s"(args), "+s"(q), "+s"(nt_h), "+s"(row_h), "+s"(rb_h));
+#endif
+    const auto& pa = *(const __attribute__((address_space(4))) RegsParams*)args;
+#pragma unroll 1
+    for (; odd != 0; q += NW, odd >>= 1) {
+      if (!(odd & 1u)) continue;
+      const int j = q / MB, mb = q - j * MB, nt = nt_h + j, row = row_h + mb * 16;
+      const uint32_t units = (uint32_t)pa.NT * (uint32_t)(pa.RB * MB), u = (uint32_t)nt * (uint32_t)(pa.RB * MB) + (uint32_t)(rb_h * MB + mb);
+      v4f val = pa.SK > 1 ? regs_sum_parts(rsrc(pa.c_tmp, units * 1024u * (uint32_t)pa.SK), units, u, pa.SK, here) : regs_sum<NW>(red, J * MB, q, here);
+      const v4f again = regs_rounded_tile<BF16, HAS_ZP, SUBG, W8>(pa, nt, row, here);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (!__builtin_isfinite(val[r])) val[r] = again[r];
+      regs_store<BF16>(pa, val, row + (here & 15), nt * 16 + (here >> 4) * 4);
     }
   }
 }
