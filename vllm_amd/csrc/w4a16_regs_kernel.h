@@ -54,7 +54,8 @@ constexpr size_t regs_lds_bytes(int mb, int mr, int j, int nw, int sub, bool zp)
 
 // One 16 x 16 result, all of K, its weights rounded to 16 bits ahead of the product as the tile kernels do it: what a call gets where codes with
 // their bias give no finite number.  (inf - inf where the weights' own signs would decide; and of bf16
-// activations beyond 2^120 the biased sums overflow, those of the weights do not.)  By one wavefront, without any prefetch.
+// activations beyond 2^120 the biased sums overflow, those of the weights do not.)  By one wavefront, without any prefetch:
+// 4096 x 28672 at M = 32 takes 144 us with one such row and 18 without.
 template <bool BF16, bool HAS_ZP, int SUBG, bool W8>
 __device__ __attribute__((always_inline)) inline v4f regs_rounded_tile(const __attribute__((address_space(4))) RegsParams& p, int nt, int row, int lane) {
   using T = F16Traits<BF16>;
