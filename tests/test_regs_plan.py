@@ -68,7 +68,8 @@ def test_choices_over_recorded_timings(fit):
     for w8 in (0, 1):
         for sub in (1, 2, 4):
             here = (t.sub[first] == sub) & (t.w8[first] == w8)
-            assert np.exp(np.log(took[here] / best[here]).mean()) < 1.025
+            several = here & (np.bincount(t.key, minlength=n) > 1)      # (of some problems only the plan that the library chooses was timed)
+            assert np.exp(np.log(took[several] / best[several]).mean()) < 1.025
             gain = ratio[here & np.isfinite(ratio)]
             assert len(gain) > 100 and np.exp(np.log(gain).mean()) < 0.9 and (gain > 1.03).mean() < 0.1 and (gain > 1.15).mean() < 0.01
 
