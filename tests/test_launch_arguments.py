@@ -1,0 +1,40 @@
+"""Divisions that the kernels make by multiplication with a number from the host (tile_handover.h, w4a16_regs_kernel.h)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from vllm_amd.build import HIPCC_FLAGS
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 4, 5, 7, 8, 12, 96, 255, 256, 1000, 9504, 65535, 65536, 1 << 20, (1 << 31) - 1, 1 << 31])
+def test_quotients_of_the_tile_order(d):
+    """x / d = umulhi(x, 2^32 / d), plus one where the rest says so, for any 32-bit x."""
+    rng = np.random.default_rng(d)
+    q = rng.integers(0, (1 << 32) // d, 4000, dtype=np.uint64) * d
+    x = np.concatenate([rng.integers(0, 1 << 32, 20000, dtype=np.uint64), q, q + (d - 1), q + (d > 1),
+                        np.array([0, 1, d - 1, d, (1 << 32) - 1], dtype=np.uint64)])
+    x = x[x < (1 << 32)]
+    magic = np.uint64(0xFFFFFFFF if d <= 1 else (1 << 32) // d)
+    got = (x * magic) >> np.uint64(32)
+    got = np.where(x - got * np.uint64(d) >= d, got + np.uint64(1), got)
+    np.testing.assert_array_equal(got, x // np.uint64(d))
+
+
+def test_band_heights_use_the_same_numbers():
+    assert [(1 << 32) // h for h in (4, 3, 2)] == [0x40000000, 0x55555555, 0x80000000]
+
+
+def test_quotients_of_copies():
+    """unit / copies by 2^32 / copies + 1 for up to 2^25 units, and a copy's number / blocks of rows in 12 bits."""
+    x = np.concatenate([np.arange(1 << 16), np.arange((1 << 25) - (1 << 16), 1 << 25)]).astype(np.uint64)
+    for copies in range(2, 129):
+        got = (x * np.uint64((1 << 32) // copies + 1)) >> np.uint64(32)
+        np.testing.assert_array_equal(got, x // np.uint64(copies))
+    rest = np.arange(128)
+    for blocks in range(1, 17):
+        np.testing.assert_array_equal(rest * ((4096 + blocks - 1) // blocks) >> 12, rest // blocks)
+
+
+def test_leading_arguments_are_asked_for_in_registers():
+    assert "-amdgpu-kernarg-preload-count=16" in HIPCC_FLAGS

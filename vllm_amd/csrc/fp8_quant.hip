@@ -169,11 +169,9 @@ __global__ __launch_bounds__(TPB) void fp8_quant_kernel(const T* __restrict__ in
 // registers, the absmax is a butterfly over the lanes -- no LDS, no barrier, four rows per workgroup in flight
 // independently.  Same arithmetic as MODE 0 above (the maximum is order-independent, the division is the IEEE one).
 template <typename T, int NV>
-__global__ __launch_bounds__(QTW) void fp8_quant_row_per_wave_kernel(const T* __restrict__ in, int64_t in_stride,
+__global__ __launch_bounds__(QTW) void fp8_quant_row_per_wave_kernel(const T* __restrict__ in, int64_t in_stride, int hidden, int rows,
                                                                      uint8_t* __restrict__ out, int64_t out_stride,
-                                                                     float* __restrict__ scales,
-                                                                     const float* __restrict__ scale_ub, int hidden,
-                                                                     int64_t rows) {
+                                                                     float* __restrict__ scales, const float* __restrict__ scale_ub) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * (QTW / 64) + (threadIdx.x >> 6);
   if (row >= rows) return;
@@ -296,14 +294,14 @@ static void launch_row_per_wave(const void* in, int64_t in_stride, uint8_t* out,
                                 const float* ub, int64_t rows, int64_t hidden, hipStream_t s) {
   const dim3 grid((unsigned)((rows + QTW / 64 - 1) / (QTW / 64))), block(QTW);
   if (hidden <= 64 * 8 * 2)
-    hipLaunchKernelGGL((fp8_quant_row_per_wave_kernel<T, 2>), grid, block, 0, s, (const T*)in, in_stride, out, out_stride,
-                       scales, ub, (int)hidden, rows);
+    hipLaunchKernelGGL((fp8_quant_row_per_wave_kernel<T, 2>), grid, block, 0, s, (const T*)in, in_stride, (int)hidden, (int)rows, out,
+                       out_stride, scales, ub);
   else if (hidden <= 64 * 8 * 4)
-    hipLaunchKernelGGL((fp8_quant_row_per_wave_kernel<T, 4>), grid, block, 0, s, (const T*)in, in_stride, out, out_stride,
-                       scales, ub, (int)hidden, rows);
+    hipLaunchKernelGGL((fp8_quant_row_per_wave_kernel<T, 4>), grid, block, 0, s, (const T*)in, in_stride, (int)hidden, (int)rows, out,
+                       out_stride, scales, ub);
   else
-    hipLaunchKernelGGL((fp8_quant_row_per_wave_kernel<T, 8>), grid, block, 0, s, (const T*)in, in_stride, out, out_stride,
-                       scales, ub, (int)hidden, rows);
+    hipLaunchKernelGGL((fp8_quant_row_per_wave_kernel<T, 8>), grid, block, 0, s, (const T*)in, in_stride, (int)hidden, (int)rows, out,
+                       out_stride, scales, ub);
 }
 
 template <int MODE, int TPB, int QV>

@@ -24,7 +24,7 @@ static int launch_quant_mm(const Fp8MMParams& p_in, int wk, int gx, hipStream_t 
   auto kern = fp8_mm_stream2_kernel<BF16, KS, 1, NSR, MQ, STATIC>;
   static size_t reserved[VAQ_MAX_DEVICES];
   if (const int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds, reserved, "fp8_quant_scaled_mm"); rc != VAQ_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3(gx), dim3(64, wk), lds, s, p, wk);
+  launch_fp8_stream(kern, dim3(gx), wk, lds, s, p);
   return VAQ_OK;
 }
 

@@ -401,7 +401,12 @@ __global__ __launch_bounds__(256) void fp8_mm_tile2_kernel(const Fp8MMParams p) 
 //    that the tiles resident on one XCD share activation rows and weight columns in its L2.
 // Requires K % 64 == 0 (a partial last step would read the neighbouring row instead of zeros) and M*lda, N*ldb < 2^32.
 template <bool BF16_OUT, int BM, int BN, int WAVES_M, int WAVES_N, int NST, int KS = 1, int PP = 0>
-__global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(const Fp8MMParams p) {
+__global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(VAQ_HEAD_ARGS, const Fp8MMParams p) {
+  // what the first requests need (vaq_common.h; see launch_tile3)
+  const uint8_t* const a = head_ptr<uint8_t>(h0[0], h0[1]);
+  const uint8_t* const b = head_ptr<uint8_t>(h0[2], h0[3]);
+  const uint32_t lda = h0[4], ldb = h0[5], tiles_m = h1[2], tiles_n = h1[1], flags = h2[1];      // (rotate_k from bit 16 on)
+  const int M = (int)h0[6], N = (int)h0[7], K = (int)h1[0];
   // A step is KS k-slices of 64 bytes (KS = 2 for the small tiles, whose steps are otherwise shorter than the barrier
   // and the LDS round trip that every step pays); a stage holds the KS slices of one step, each as [A tile | B tile].
   constexpr bool PAIR = PP == 2, LINE = KS == 2 || PAIR;        // requests of whole 128-byte lines (see `load`)
@@ -420,20 +425,13 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
 
-  const int tiles_m = (p.M + BM - 1) / BM + p.m_tiles_extra, tiles_n = (p.N + BN - 1) / BN;
-  const int total = tiles_m * tiles_n;
-  const TileSlot sl = tile_slot(total, p.SK, p.tail_first);          // one contiguous range of tile positions per XCD
-  const int t = sl.pos;
-  constexpr int GM = 4;                                              // band height in tiles (2 .. 16 measured: 4 is 1-2 % ahead of 8)
-  const int band = t / (GM * tiles_n);
-  const int first_m = band * GM;
-  const int gsz = min(tiles_m - first_m, GM);
-  const int tin = t - band * GM * tiles_n;
-  const int tm = first_m + tin % gsz, tn = tin / gsz;
+  const TileSlot sl = tile_slot(TileGrid{tiles_n, tiles_m, h1[3], h2[0], flags}, p);          // one contiguous range of tile positions per XCD
+  const int tm = sl.tm, tn = sl.tn;
   const int m0 = tm * BM, n0 = tn * BN;
 
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.a), 0, (int)p.a_extent, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.b), 0, (int)p.b_extent, 0x00020000);
+  // (ends as p.a_extent and p.b_extent, formed here from what comes with the launch)
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a), 0, (int)((uint32_t)(M - 1) * lda + (uint32_t)K), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(b), 0, (int)((uint32_t)(N - 1) * ldb + (uint32_t)K), 0x00020000);
   // DMA instruction.  One slice: 16 rows x 64 bytes = four 256-byte lines; lane l lands in slot l: line j = r0/4 + (l >> 4), swizzled
   // chunk l & 15 -> c16 = (l & 15) ^ (j & 3), row = 4j + (c16 >> 2), chunk = c16 & 3.  r0 is a multiple of 16, so j & 3 = l >> 4.
   // Two slices (LINE): 8 rows x 128 bytes; row r0 + (l >> 3), chunk (l & 7) ^ f, f = bits 3, 1, 2 of the row in this order -> with r0 = 8 times the
@@ -441,15 +439,15 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
   const int c16 = (lane & 15) ^ (lane >> 4);
   const uint32_t lrow = (uint32_t)(LINE ? lane >> 3 : 4 * (lane >> 4) + (c16 >> 2));
   const uint32_t lbyte = (uint32_t)(LINE ? (lane & 7) ^ ((lane >> 4 & 1) | (lane >> 5) << 2) : c16 & 3) * 16u;
-  const uint32_t row_a = lrow * (uint32_t)p.lda, row_b = lrow * (uint32_t)p.ldb;
+  const uint32_t row_a = lrow * lda, row_b = lrow * ldb;
   const uint32_t voff_a = row_a + lbyte, voff_b = row_b + lbyte;
   const uint32_t voff_a1 = row_a + (lbyte ^ 32u), voff_b1 = row_b + (lbyte ^ 32u);      // (LINE: odd instructions)
 
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   // K may be split over workgroups: this one covers the steps [s_lo, s_hi)
-  const int all_steps = p.K / (64 * KS);
+  const int all_steps = K / (64 * KS);
   // (in pairs: parts start at even steps, so that the two slices of a request share their cache lines)
-  const auto part = [&](int i) { return i >= sl.nsplit ? all_steps : (int)(((int64_t)all_steps * i) / sl.nsplit) & (PAIR ? ~1 : ~0); };
+  const auto part = [&](int i) { return i >= sl.nsplit ? all_steps : tile_part(p, sl, all_steps, i) & (PAIR ? ~1 : ~0); };
   const int s_lo = part(sl.split), s_hi = part(sl.split + 1);
   const int steps = s_hi - s_lo;
   // Few tile rows (M at most 4 tiles high) on a device that the tiles do not fill: the tiles of one column would read
@@ -461,21 +459,23 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
   // of two all of them ask the same few L2 channels for the same lines at the same time.  Tile column tn starts tn / tiles_n
   // of the way into K instead (4096 x 28672 at M = 72 .. 256, cold: 33.9 .. 45.4 -> 31.1 .. 43.6 us; no change on K = 3584 or
   // 5120; with 16 tile rows it costs 3-9 %: the tiles of one column then no longer read their weights together).
-  int rot = p.rotate_k == 1 ? (tm * steps) / tiles_m : (p.rotate_k == 2 ? (tn * steps) / tiles_n : 0);
+  int rot = 0;
+  if (const uint32_t rotate_k = flags >> 16; rotate_k != 0)
+    rot = (int)div_by((uint32_t)((rotate_k == 1 ? tm : tn) * steps), rotate_k == 1 ? tiles_m : tiles_n, p.rotate_magic);
   if (PAIR) rot = steps & 1 ? 0 : rot & ~1;      // a pair never wraps around
   // Requests for ROWS rows of an operand, from row `first` and K byte `koff` on.  LINE: eight lanes ask for 128 bytes, a whole cache line,
   // which crosses from the L2 in one piece; else the slices of a step row by row, whose halves of a line cross one after the other.  Weights from
   // memory, halves -> lines: 128 x 128 tiles: 5120 x 13824 at M = 250 33.6 -> 31.5 us, 4096 x 28672 at M = 100 30.3 -> 27.7; 64 x 128, 128 x 64, 128 x 256:
   // 2 - 9 %; 64 x 64: 3 - 6 %; 256 x 256: 4096 x 28672 at M = 512 59.1 -> 56.1; from the memory-side cache level.  Pieces of 256 bytes (four slices,
   // half of the rows at a time): -4 .. +3 % against lines; one operand in lines and the other in halves: in between.
-  auto load = [&](auto rows, const __amdgpu_buffer_rsrc_t& r, uint32_t first, int64_t pitch, uint32_t v0, uint32_t v1, uint32_t koff, uint8_t* at) {
+  auto load = [&](auto rows, const __amdgpu_buffer_rsrc_t& r, uint32_t first, uint32_t pitch, uint32_t v0, uint32_t v1, uint32_t koff, uint8_t* at) {
     constexpr int ROWS = decltype(rows)::value;
     if constexpr (LINE) {
       constexpr int LD = ROWS / (8 * NW);
 #pragma unroll
       for (int i = 0; i < LD; ++i) {
         const int r0 = (wave * LD + i) * 8;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(at + r0 * 128), 16, (int)(i & 1 ? v1 : v0), (int)((first + (uint32_t)r0) * (uint32_t)pitch + koff), 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(at + r0 * 128), 16, (int)(i & 1 ? v1 : v0), (int)((first + (uint32_t)r0) * pitch + koff), 0, 0);
       }
     } else {
       constexpr int LD = ROWS / (16 * NW);
@@ -484,12 +484,12 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
         const int r0 = (wave * LD + i) * 16;
 #pragma unroll
         for (int c = 0; c < KS; ++c)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(at + (c * ROWS + r0) * 64), 16, (int)v0, (int)((first + (uint32_t)r0) * (uint32_t)pitch + koff + 64u * c), 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(at + (c * ROWS + r0) * 64), 16, (int)v0, (int)((first + (uint32_t)r0) * pitch + koff + 64u * c), 0, 0);
       }
     }
   };
-  auto load_a = [&](uint32_t koff, uint8_t* at) { load(std::integral_constant<int, BM>{}, ra, (uint32_t)m0, p.lda, voff_a, voff_a1, koff, at); };
-  auto load_b = [&](uint32_t koff, uint8_t* at) { load(std::integral_constant<int, BN>{}, rb, (uint32_t)n0, p.ldb, voff_b, voff_b1, koff, at); };
+  auto load_a = [&](uint32_t koff, uint8_t* at) { load(std::integral_constant<int, BM>{}, ra, (uint32_t)m0, lda, voff_a, voff_a1, koff, at); };
+  auto load_b = [&](uint32_t koff, uint8_t* at) { load(std::integral_constant<int, BN>{}, rb, (uint32_t)n0, ldb, voff_b, voff_b1, koff, at); };
   // Steps are requested in order: the first byte of K of the next one, rotation applied.  (As few scalar instructions as can be: the matrix
   // cores wait for them at the start of every step.)
   constexpr uint32_t K_STEP = PAIR ? 128 : 64 * KS;
@@ -789,7 +789,9 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(co
 // blockDim = (64, WK).  Wavefront w owns K steps [w*KS, (w+1)*KS) of 128 bytes; activations of that slab live in
 // registers for the whole kernel; the workgroup walks a contiguous range of 16-row weight tiles.
 template <bool BF16_OUT, int KS, int MB, bool HALVES = false, bool PF = true>
-__global__ __launch_bounds__(512) void fp8_mm_stream_kernel(const Fp8MMParams p, int WK) {
+__global__ __launch_bounds__(512) void fp8_mm_stream_kernel(VAQ_HEAD_ARGS, const Fp8MMParams rest) {
+  const Fp8MMParams p = stream_params(h0, h1, h2, rest);
+  const int WK = (int)(h1[1] >> 16);
   using T = F16Traits<BF16_OUT>;
   extern __shared__ v4f red[];   // [2][WK][MB][64]
   const int lane = threadIdx.x, w = threadIdx.y;
@@ -1009,14 +1011,20 @@ static int launch_tile2(const Fp8MMParams& p, hipStream_t s) {
 }
 
 template <bool BF16_OUT, int BM, int BN, int WAVES_M, int WAVES_N, int NST, int KS = 1, int PP = 0>
-static int launch_tile3(const Fp8MMParams& p, hipStream_t s) {
+static int launch_tile3(const Fp8MMParams& p_in, hipStream_t s) {
+  Fp8MMParams p = p_in;
   const size_t lds = (size_t)NST * KS * (BM + BN) * 64;
   auto kern = fp8_mm_tile3_kernel<BF16_OUT, BM, BN, WAVES_M, WAVES_N, NST, KS, PP>;
   static size_t reserved[VAQ_MAX_DEVICES];
   if (const int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds, reserved, "fp8_scaled_mm"); rc != VAQ_OK) return rc;
-  const int tiles = ((p.M + BM - 1) / BM + p.m_tiles_extra) * ((p.N + BN - 1) / BN);
+  const int tiles_m = (p.M + BM - 1) / BM + p.m_tiles_extra, tiles_n = (p.N + BN - 1) / BN, tiles = tiles_m * tiles_n;
+  const TileGrid g = tile_grid(tiles_m, tiles_n, p.SK, p.tail_first);
+  p.split_magic = tile_split_magic(tiles, p.SK, p.tail_first);
+  p.rotate_magic = div_magic((uint32_t)(p.rotate_k == 1 ? tiles_m : tiles_n));
   const dim3 grid = p.tail_first > 0 ? dim3(p.tail_first + (tiles - p.tail_first) * p.SK) : dim3(tiles, p.SK);
-  hipLaunchKernelGGL(kern, grid, dim3(WAVES_M * WAVES_N * 64), lds, s, p);
+  hipLaunchKernelGGL(kern, grid, dim3(WAVES_M * WAVES_N * 64), lds, s,
+                     (v8u{ptr_lo(p.a), ptr_hi(p.a), ptr_lo(p.b), ptr_hi(p.b), (uint32_t)p.lda, (uint32_t)p.ldb, (uint32_t)p.M, (uint32_t)p.N}),
+                     (v4u{(uint32_t)p.K, g.n, g.m, g.band_magic}), (v2u{g.per8, g.flags | (uint32_t)p.rotate_k << 16}), p);
   return VAQ_OK;
 }
 
@@ -1186,9 +1194,9 @@ static void launch_stream(const Fp8MMParams& p_in, int wk, int gx, hipStream_t s
   p.b_extent = (uint32_t)((int64_t)(p.N - 1) * p.ldb + p.K);
   const size_t lds = wk > 1 ? (size_t)2 * wk * MB * 64 * sizeof(v4f) : 0;
   if (p.nt_base == 1 && p.nt_rem == 0)
-    hipLaunchKernelGGL((fp8_mm_stream_kernel<BF16_OUT, KS, MB, HALVES, false>), dim3(gx, HALVES ? 2 : 1), dim3(64, wk), lds, s, p, wk);
+    launch_fp8_stream(fp8_mm_stream_kernel<BF16_OUT, KS, MB, HALVES, false>, dim3(gx, HALVES ? 2 : 1), wk, lds, s, p);
   else
-    hipLaunchKernelGGL((fp8_mm_stream_kernel<BF16_OUT, KS, MB, HALVES, true>), dim3(gx, HALVES ? 2 : 1), dim3(64, wk), lds, s, p, wk);
+    launch_fp8_stream(fp8_mm_stream_kernel<BF16_OUT, KS, MB, HALVES, true>, dim3(gx, HALVES ? 2 : 1), wk, lds, s, p);
 }
 
 // The stream kernel addresses its operands with 32-bit offsets from buffer descriptors: both must end below 2 GiB
@@ -1261,7 +1269,7 @@ static bool launch_stream2(const Fp8MMParams& p_in, int wk, int gx, hipStream_t 
   auto kern = fp8_mm_stream2_kernel<BF16_OUT, KS, MB, NSR>;
   static size_t reserved[VAQ_MAX_DEVICES];
   if (reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds, reserved, "fp8_scaled_mm") != VAQ_OK) return false;      // (the kernel above then takes the problem)
-  hipLaunchKernelGGL(kern, dim3(gx), dim3(64, wk), lds, s, p, wk);
+  launch_fp8_stream(kern, dim3(gx), wk, lds, s, p);
   return true;
 }
 

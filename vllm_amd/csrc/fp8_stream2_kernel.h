@@ -1,5 +1,6 @@
 // The FP8 GEMM for few rows whose weights pass through LDS, and the parameters that all FP8 GEMM kernels share.
 #pragma once
+#include "tile_handover.h"
 #include "vaq_common.h"
 
 namespace vaq {
@@ -24,6 +25,8 @@ struct Fp8MMParams {
   int rotate_k = 0;              // multi-stage tile kernel: 1 tile rows, 2 tile columns start their K loop at different places (see the kernel)
   int m_tiles_extra = 0;         // multi-stage tile kernel: tile rows past M (see dispatch_tile: they read the weights with the real ones and store nothing)
   uint32_t a_extent = 0, b_extent = 0;   // bytes up to the end of the last row of a / b (stream kernels: below 2 GiB, tile kernels 4)
+  TileSplitMagic split_magic = {0, 0};      // see tile_handover.h
+  uint32_t rotate_magic = 0;     // of the tile rows (rotate_k = 1) or columns (2)
   int nt_base = 0, nt_rem = 0;   // stream kernel: n-tiles per workgroup = nt_base, one more for the first nt_rem (N/16 split on the host)
 };
 
@@ -75,6 +78,29 @@ static __device__ inline uint32_t wave_maxima(uint32_t (&v)[MQ]) {
   }
 }
 
+// What the first requests of the stream kernels need, as their head (vaq_common.h); the rest is loaded.
+__device__ inline Fp8MMParams stream_params(const v8u& h0, const v4u& h1, const v2u& h2, const Fp8MMParams& rest) {
+  Fp8MMParams p = rest;
+  p.a = head_ptr<uint8_t>(h0[0], h0[1]);
+  p.b = head_ptr<uint8_t>(h0[2], h0[3]);
+  p.sa = head_ptr<float>(h0[4], h0[5]);
+  p.lda = h0[6];
+  p.ldb = h0[7];
+  p.K = (int)h1[0];
+  p.M = (int)(h1[1] & 0xffffu);
+  p.a_extent = h1[2];
+  p.b_extent = h1[3];
+  p.nt_base = (int)h2[0];
+  p.nt_rem = (int)h2[1];
+  return p;
+}
+template <class Kernel>
+inline void launch_fp8_stream(Kernel kern, dim3 grid, int wk, size_t lds, hipStream_t s, const Fp8MMParams& p) {
+  hipLaunchKernelGGL(kern, grid, dim3(64, wk), lds, s,
+                     (v8u{ptr_lo(p.a), ptr_hi(p.a), ptr_lo(p.b), ptr_hi(p.b), ptr_lo(p.sa), ptr_hi(p.sa), (uint32_t)p.lda, (uint32_t)p.ldb}),
+                     (v4u{(uint32_t)p.K, (uint32_t)p.M | (uint32_t)wk << 16, p.a_extent, p.b_extent}), (v2u{(uint32_t)p.nt_base, (uint32_t)p.nt_rem}), p);
+}
+
 // ----------------------------------------------------------------------------- stream kernel, weights through LDS
 // fp8_mm_stream_kernel (fp8_scaled_mm.hip) fetches the weights in the MFMA operand layout: every load instruction takes
 // 64-byte pieces of 16 rows, half a cache line each.  Measured on bare reads of a 4096 x 28672 byte matrix with cold lines, that
@@ -90,7 +116,9 @@ static __device__ inline uint32_t wave_maxima(uint32_t (&v)[MQ]) {
 //    and every wavefront quantises its own K slab, bit for bit as the quantisation kernels do: per token (p.sa null) or with
 //    the one scale at p.sa (STATIC).  A layer is then one launch instead of two.
 template <bool BF16_OUT, int KS, int MB, int NSR, int MQ = 0, bool STATIC = false>
-__global__ __launch_bounds__(512) void fp8_mm_stream2_kernel(const Fp8MMParams p, int WK) {
+__global__ __launch_bounds__(512) void fp8_mm_stream2_kernel(VAQ_HEAD_ARGS, const Fp8MMParams rest) {
+  const Fp8MMParams p = stream_params(h0, h1, h2, rest);
+  const int WK = (int)(h1[1] >> 16);
   using T = F16Traits<BF16_OUT>;
   constexpr int NS = KS / 2;                       // stages per n-tile
   static_assert(KS % 2 == 0 && NS % NSR == 0, "whole stages, ring slots fixed at compile time");

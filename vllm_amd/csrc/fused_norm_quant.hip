@@ -82,6 +82,8 @@ __device__ inline v2u nq_quant8(const float (&y)[8], F&& dv) {
   return o;
 }
 
+// (The kernels' arguments are in the order in which they are needed: the first 14 dwords arrive in registers with the launch.)
+//
 // One token per WAVEFRONT (rows of at most 64 x NV x 8 elements, many tokens): the row sits in the wavefront's
 // registers, both reductions are butterflies over its lanes -- no LDS, no barrier, NQ_W / 64 independent rows per
 // workgroup and every load of a row in flight at once.  DYN: the dynamic per-token quantiser (scale written per token);
@@ -89,12 +91,10 @@ __device__ inline v2u nq_quant8(const float (&y)[8], F&& dv) {
 // below; only the order of the additions inside the sum of squares differs (per lane over its chunks, then the butterfly).
 constexpr int NQ_W = 256;
 template <bool BF16, bool HAS_RES, bool DYN, int NV>
-__global__ __launch_bounds__(NQ_W) void rms_norm_fp8_row_per_wave_kernel(uint8_t* __restrict__ out, float* __restrict__ scales,
-                                                                         const uint16_t* __restrict__ input,
-                                                                         const uint16_t* __restrict__ weight,
-                                                                         const float* __restrict__ scale_ub, float eps,
-                                                                         uint16_t* __restrict__ residual, int hidden,
-                                                                         int64_t in_stride, int64_t tokens) {
+__global__ __launch_bounds__(NQ_W) void rms_norm_fp8_row_per_wave_kernel(const uint16_t* __restrict__ input, uint16_t* __restrict__ residual,
+                                                                         const uint16_t* __restrict__ weight, int64_t in_stride, int tokens,
+                                                                         int hidden, uint8_t* __restrict__ out, float* __restrict__ scales,
+                                                                         const float* __restrict__ scale_ub, float eps) {
   using T = F16Traits<BF16>;
   const int lane = threadIdx.x & 63;
   const int64_t tok = (int64_t)blockIdx.x * (NQ_W / 64) + (threadIdx.x >> 6);
@@ -195,12 +195,10 @@ __global__ __launch_bounds__(NQ_W) void rms_norm_fp8_row_per_wave_kernel(uint8_t
 constexpr bool nq_ahead(bool has_res, int nv) { return !has_res || nv <= 2; }
 
 template <bool BF16, bool HAS_RES, int NV, int TPB>
-__global__ __launch_bounds__(TPB) void rms_norm_per_token_fp8_kernel(uint8_t* __restrict__ out, float* __restrict__ scales,
-                                                                      const uint16_t* __restrict__ input,
-                                                                      const uint16_t* __restrict__ weight,
-                                                                      const float* __restrict__ scale_ub, float eps,
-                                                                      uint16_t* __restrict__ residual, int hidden,
-                                                                      int64_t in_stride) {
+__global__ __launch_bounds__(TPB) void rms_norm_per_token_fp8_kernel(const uint16_t* __restrict__ input, uint16_t* __restrict__ residual,
+                                                                      const uint16_t* __restrict__ weight, uint8_t* __restrict__ out,
+                                                                      int64_t in_stride, int hidden, float eps, float* __restrict__ scales,
+                                                                      const float* __restrict__ scale_ub) {
   using T = F16Traits<BF16>;
   __shared__ float smem[2 * TPB / 64];
   const int64_t tok = blockIdx.x;
@@ -325,12 +323,10 @@ __global__ __launch_bounds__(TPB) void rms_norm_per_token_fp8_kernel(uint8_t* __
 }
 
 template <bool BF16, bool HAS_RES, int NV, int TPB>
-__global__ __launch_bounds__(TPB) void rms_norm_static_fp8_kernel(uint8_t* __restrict__ out,
-                                                                   const uint16_t* __restrict__ input,
-                                                                   const uint16_t* __restrict__ weight,
-                                                                   const float* __restrict__ scale, float eps,
-                                                                   uint16_t* __restrict__ residual, int hidden,
-                                                                   int64_t in_stride) {
+__global__ __launch_bounds__(TPB) void rms_norm_static_fp8_kernel(const uint16_t* __restrict__ input, uint16_t* __restrict__ residual,
+                                                                   const uint16_t* __restrict__ weight, uint8_t* __restrict__ out,
+                                                                   int64_t in_stride, int hidden, float eps,
+                                                                   const float* __restrict__ scale) {
   using T = F16Traits<BF16>;
   __shared__ float smem[TPB / 64];
   const int64_t tok = blockIdx.x;
@@ -571,7 +567,7 @@ extern "C" int vaq_rms_norm_dynamic_per_token_fp8_quant(uint8_t* out, float* sca
     const dim3 wgrid((unsigned)((tokens + NQ_W / 64 - 1) / (NQ_W / 64))), wblock(NQ_W);
     auto launch = [&](auto bf, auto rs, auto nvc) {
       hipLaunchKernelGGL((rms_norm_fp8_row_per_wave_kernel<decltype(bf)::value, decltype(rs)::value, true, decltype(nvc)::value>),
-                         wgrid, wblock, 0, s, out, scales, in, w, scale_ub, epsilon, res, (int)hidden, in_stride, tokens);
+                         wgrid, wblock, 0, s, in, res, w, in_stride, (int)tokens, (int)hidden, out, scales, scale_ub, epsilon);
     };
     nq_dispatch(bf16, res != nullptr, hidden <= 64 * 8 * 2 ? 2 : 4, launch);
     VAQ_CHECK_LAUNCH("rms_norm_dynamic_per_token_quant");
@@ -582,10 +578,10 @@ extern "C" int vaq_rms_norm_dynamic_per_token_fp8_quant(uint8_t* out, float* sca
   auto launch = [&](auto bf, auto rs, auto nvc) {
     if (half_wg)
       hipLaunchKernelGGL((rms_norm_per_token_fp8_kernel<decltype(bf)::value, decltype(rs)::value, 2, NQ_T / 2>), grid,
-                         dim3(NQ_T / 2), 0, s, out, scales, in, w, scale_ub, epsilon, res, (int)hidden, in_stride);
+                         dim3(NQ_T / 2), 0, s, in, res, w, out, in_stride, (int)hidden, epsilon, scales, scale_ub);
     else
       hipLaunchKernelGGL((rms_norm_per_token_fp8_kernel<decltype(bf)::value, decltype(rs)::value, decltype(nvc)::value, NQ_T>),
-                         grid, block, 0, s, out, scales, in, w, scale_ub, epsilon, res, (int)hidden, in_stride);
+                         grid, block, 0, s, in, res, w, out, in_stride, (int)hidden, epsilon, scales, scale_ub);
   };
   nq_dispatch(bf16, res != nullptr, nv, launch);
   VAQ_CHECK_LAUNCH("rms_norm_dynamic_per_token_quant");
@@ -612,8 +608,7 @@ extern "C" int vaq_rms_norm_static_fp8_quant(uint8_t* out, const void* input, in
     const dim3 wgrid((unsigned)((tokens + NQ_W / 64 - 1) / (NQ_W / 64))), wblock(NQ_W);
     auto launch = [&](auto bf, auto rs, auto nvc) {
       hipLaunchKernelGGL((rms_norm_fp8_row_per_wave_kernel<decltype(bf)::value, decltype(rs)::value, false, decltype(nvc)::value>),
-                         wgrid, wblock, 0, s, out, const_cast<float*>(scale), in, w, nullptr, epsilon, res, (int)hidden,
-                         in_stride, tokens);
+                         wgrid, wblock, 0, s, in, res, w, in_stride, (int)tokens, (int)hidden, out, const_cast<float*>(scale), nullptr, epsilon);
     };
     nq_dispatch(dtype == VAQ_BF16, res != nullptr, hidden <= 64 * 8 * 2 ? 2 : 4, launch);
     VAQ_CHECK_LAUNCH("rms_norm_static_fp8_quant");
@@ -624,10 +619,10 @@ extern "C" int vaq_rms_norm_static_fp8_quant(uint8_t* out, const void* input, in
   auto launch = [&](auto bf, auto rs, auto nvc) {
     if (half_wg)
       hipLaunchKernelGGL((rms_norm_static_fp8_kernel<decltype(bf)::value, decltype(rs)::value, 2, NQ_T / 2>), grid, dim3(NQ_T / 2),
-                         0, s, out, in, w, scale, epsilon, res, (int)hidden, in_stride);
+                         0, s, in, res, w, out, in_stride, (int)hidden, epsilon, scale);
     else
       hipLaunchKernelGGL((rms_norm_static_fp8_kernel<decltype(bf)::value, decltype(rs)::value, decltype(nvc)::value, NQ_T>), grid,
-                         block, 0, s, out, in, w, scale, epsilon, res, (int)hidden, in_stride);
+                         block, 0, s, in, res, w, out, in_stride, (int)hidden, epsilon, scale);
   };
   nq_dispatch(dtype == VAQ_BF16, res != nullptr, nv, launch);
   VAQ_CHECK_LAUNCH("rms_norm_static_fp8_quant");

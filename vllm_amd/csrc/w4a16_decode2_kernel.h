@@ -46,13 +46,7 @@ struct Decode2Params {
   int GR;                  // rows of the scale / zero-point tensors (G * SUBG, or 1 for channelwise scales)
   int s_stride, z_stride;  // elements between consecutive rows of scales (N) / zeros (N/8); 0 for channelwise
   uint32_t k_mask, k_ex;   // 0x000f000f and the exponent pattern, passed as run-time values (see and_or)
-  // Set by the launcher (it knows the template arguments): the divisions of the kernel's first instructions, done on
-  // the host.  x / WN = (x * wn_magic) >> 16 for a wavefront index, x / KO = umulhi(x, ko_magic) for a thread index (KO =
-  // k-octets of the staged slab; both exact in those ranges); step_m, step_ko = (threads / KO, threads % KO).
-  uint32_t wn_magic, ko_magic;
-  int step_m, step_ko;
-  int gx8;                 // see the kernel's n-tile order
-  uint32_t b_bytes, s_bytes, z_bytes, a_bytes;   // extents of the buffer descriptors (saturated to 4 GiB - 1)
+  uint32_t z_bytes;        // extent of the zero points (saturated to 4 GiB - 1), set by the launcher
 };
 
 // (x & mask) | ex.  mask and ex reach the kernel as run-time arguments: with literal constants the compiler emits two
@@ -74,17 +68,24 @@ constexpr int DECODE2_MAX_M = 64;           // rows of one workgroup: up to four
 constexpr int DECODE2_MAX_M_ROWS = 256;     // rows when every m-block has workgroups of its own (see MSP)
 
 template <bool BF16, int GS, int MB, bool HAS_ZP, int MR, int SUBG, int WT = 0, int RC = 0, bool MSP = false>
-__global__ __launch_bounds__(D2_WAVES * 64) void w4a16_decode2_kernel(const Decode2Params p) {
+__global__ __launch_bounds__(D2_WAVES * 64) void w4a16_decode2_kernel(VAQ_HEAD_ARGS, const Decode2Params p) {
   using T = F16Traits<BF16>;
+  // what the first requests need (see launch_decode2)
+  const uint16_t* const a = head_ptr<uint16_t>(h0[0], h0[1]);
+  const v4u* const b = head_ptr<v4u>(h0[2], h0[3]);
+  const uint16_t* const scales = head_ptr<uint16_t>(h0[4], h0[5]);
+  const uint32_t lda = h0[6], G = h0[7], n_tiles = h1[0], shape = h1[1], ko_magic = h1[2], steps = h1[3], wn_magic = h2[0], s_stride = h2[1];
+  const int M = (int)(shape & 0x1ffu), WKS = (int)(shape >> 9 & 0x1fu), WN = (int)(shape >> 14 & 0x1fu);
+  const bool priv = (shape >> 19 & 1u) != 0, has_perm = (shape >> 20 & 1u) != 0;
+  const int gx8 = (int)(shape >> 21), NT = (int)n_tiles;
   static_assert(!MSP || (MB == 1 && MR == 16), "rows split over workgroups: one full m-block each");
   // MSP: more than 16 rows handled as independent m-blocks, one per blockIdx.z -- every workgroup is the single-m-block
   // kernel on rows 16z .. 16z+15 (the weights are read once per m-block; the workgroups of one n-tile run side by side
   // and the later ones find the tiles in L2).  Against two m-blocks in one workgroup this halves the staged activations
   // per workgroup: a K of 4096 fits LDS again and needs no split over workgroups.
   const int mz = MSP ? (int)blockIdx.z : 0;
-  const int M_loc = MSP ? min(16, p.M - 16 * mz) : p.M;
-  const uint16_t* const a_loc = MSP ? p.a + (int64_t)mz * 16 * p.lda : p.a;
-  const uint32_t a_bytes_loc = MSP ? p.a_bytes - (uint32_t)mz * 32u * (uint32_t)p.lda : p.a_bytes;
+  const int M_loc = MSP ? min(16, M - 16 * mz) : M;
+  const uint16_t* const a_loc = MSP ? a + (int64_t)mz * 16 * lda : a;
   uint16_t* const c_loc = MSP ? p.c + (int64_t)mz * 16 * p.N : p.c;
   static_assert(SUBG == 1 || SUBG == 2 || SUBG == 4, "quantisation groups per 128-row tile");
   constexpr bool W8 = WT == 1, F8 = WT == 2;           // 8-bit codes as two nibble planes / FP8 e4m3 bytes (see the head comment)
@@ -126,43 +127,62 @@ __global__ __launch_bounds__(D2_WAVES * 64) void w4a16_decode2_kernel(const Deco
   const int lane = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
   const int o = lane >> 4, r16 = lane & 15;
-  const int WKS = p.WKS, WN = p.WN;
-  const int wks = (int)(((uint32_t)w * p.wn_magic) >> 16), wn = w - wks * WN;
+  const int wks = (int)(((uint32_t)w * wn_magic) >> 16), wn = w - wks * WN;
   const int sk = blockIdx.y;
   const int slab_groups = WKS * GS;                 // tiles in this workgroup's K slab
   const int slab_g0 = sk * slab_groups;             // first tile of the slab
   // Workgroups go to the XCDs round robin, and an n-tile's scales, zero points and output are 32-byte pieces of lines that
   // it shares with its neighbours: workgroups of one XCD take neighbouring n-tiles, so that an L2 fetches those lines once
   // instead of once per XCD (gx8 = workgroups along N / 8 where that is a whole number, else 0).
-  const int bx = p.gx8 > 0 ? (int)(blockIdx.x & 7u) * p.gx8 + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+  const int bx = gx8 > 0 ? (int)(blockIdx.x & 7u) * gx8 + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
   const int nt_raw = bx * WN + wn;
-  const bool nt_ok = nt_raw < p.NT;
-  const int nt = nt_ok ? nt_raw : p.NT - 1;
+  const bool nt_ok = nt_raw < NT;
+  const int nt = nt_ok ? nt_raw : NT - 1;
   const int g_first = slab_g0 + wks * GS;           // this wavefront's first group
 
   // ---- 1. activations of the K slab -> LDS, then the first R weight tiles requested ----
   // Loads retire in issue order as far as the wait counter is concerned, so the activation loads go out FIRST: the
   // wait before the barrier then leaves the weight tiles in flight instead of draining them.
-  const __amdgpu_buffer_rsrc_t rb = d2_rsrc32(p.b, p.b_bytes);
-  const __amdgpu_buffer_rsrc_t rs = d2_rsrc32(p.scales, p.s_bytes);
-  const __amdgpu_buffer_rsrc_t rz = d2_rsrc32(HAS_ZP ? (const void*)p.zeros : (const void*)p.scales, p.z_bytes);
+  const int K = (int)(G / (uint32_t)TPG) * 128;
+  const uint32_t a_bytes = ((uint32_t)(M_loc - 1) * lda + (uint32_t)K) * 2u;      // (of the rows here; the launcher holds A below 2 GiB)
+  const __amdgpu_buffer_rsrc_t rb = d2_rsrc(b, (uint64_t)n_tiles * G * 1024u);
+  const __amdgpu_buffer_rsrc_t rs = d2_rsrc(scales, (uint64_t)(s_stride ? G / (uint32_t)TPG * (uint32_t)SUBG : 1u) * n_tiles * 32u);
+  const __amdgpu_buffer_rsrc_t rz = HAS_ZP ? d2_rsrc32(p.zeros, p.z_bytes) : rs;
   // zero points: as an MFMA operand a lane needs the one of column r16, in the output layout those of columns 4o .. 4o+3
   const int vo_b = lane * 16, vo_s = o * 8, vo_z = ((SPRE ? (o >> 1) : (r16 >> 3))) * 4;
   v4u wq[R];
   v2u sc[R][SUBG];
   uint32_t zq[R][SUBG];
-  auto issue_load = [&](int slot, int gi) {
-    const uint32_t g = (uint32_t)min(g_first + gi, p.G - 1);     // clamped: activations past K are zero
-    wq[slot] = __builtin_amdgcn_raw_buffer_load_b128(rb, vo_b, (int)(((uint32_t)nt * (uint32_t)p.G + g) * 1024u), 2);
+  // (the zero points apart: their place is among the arguments that a wavefront has to load, so that they are requested behind the first two tiles)
+  auto issue_zeros = [&](int slot, int gi) {
+    const uint32_t g = (uint32_t)min(g_first + gi, (int)G - 1);
 #pragma unroll
     for (int sj = 0; sj < SUBG; ++sj) {
       const uint32_t row = (g / (uint32_t)TPG) * (uint32_t)SUBG + (uint32_t)sj;
-      sc[slot][sj] = __builtin_amdgcn_raw_buffer_load_b64(rs, vo_s, (int)((row * (uint32_t)p.s_stride + (uint32_t)nt * 16u) * 2u), 0);
       if constexpr (HAS_ZP)
         zq[slot][sj] = __builtin_amdgcn_raw_buffer_load_b32(rz, vo_z, (int)((row * (uint32_t)p.z_stride + (uint32_t)nt * 2u) * 4u), 0);
       else
         zq[slot][sj] = 0u;
     }
+  };
+  auto issue_load = [&](int slot, int gi, bool zeros = true) {
+    const uint32_t g = (uint32_t)min(g_first + gi, (int)G - 1);     // clamped: activations past K are zero
+    wq[slot] = __builtin_amdgcn_raw_buffer_load_b128(rb, vo_b, (int)(((uint32_t)nt * G + g) * 1024u), 2);
+#pragma unroll
+    for (int sj = 0; sj < SUBG; ++sj) {
+      const uint32_t row = (g / (uint32_t)TPG) * (uint32_t)SUBG + (uint32_t)sj;
+      sc[slot][sj] = __builtin_amdgcn_raw_buffer_load_b64(rs, vo_s, (int)((row * s_stride + (uint32_t)nt * 16u) * 2u), 0);
+    }
+    if (zeros) issue_zeros(slot, gi);
+  };
+  auto issue_first = [&](int from) {      // slots from .. R - 1 of the ring
+#pragma unroll
+    for (int s = from; s < (R < 2 ? R : 2); ++s) issue_load(s, s, false);
+    if constexpr (HAS_ZP) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < (R < 2 ? R : 2); ++s) issue_zeros(s, s);
+#pragma unroll
+    for (int s = 2; s < R; ++s) issue_load(s, s);
   };
 
   const int KO = slab_groups / TPG * 16;             // k-octets in the slab
@@ -174,13 +194,13 @@ __global__ __launch_bounds__(D2_WAVES * 64) void w4a16_decode2_kernel(const Deco
     const int tid = w * 64 + lane;
     const int chunks = KO * MR * MB;
     const int k_slab0 = (slab_g0 / TPG) * 128;          // 32-bit arithmetic: the launcher checks that A ends below 2 GiB
-    const int lda32 = (int)p.lda;
+    const int lda32 = (int)lda;
     const int NTHR = WKS * WN * 64;
-    const int step_m = p.step_m, step_ko = p.step_ko;               // NTHR / KO, NTHR % KO
+    const int step_m = (int)(steps >> 16), step_ko = (int)(steps & 0xffffu);              // NTHR / KO, NTHR % KO
     // chunk c = m * KO + ko' (LDS slot c); thread tid handles c = tid, tid + NTHR, ...  The (m, ko') pair is advanced
     // incrementally: one scalar division per kernel instead of one vector division per chunk.
-    int m = (int)__umulhi((uint32_t)tid, p.ko_magic), ko = tid - m * KO;
-    if (p.PRIV != 0) {
+    int m = (int)__umulhi((uint32_t)tid, ko_magic), ko = tid - m * KO;
+    if (priv) {
       // Private fill (one n-tile per workgroup, so no two wavefronts read the same k-octets): every wavefront fetches the
       // k-octets of its own K slice, row by row, and waits for nobody -- the same bytes travel as in the shared fill, but
       // a wavefront starts on its first tile as soon as ITS activations and ITS first weight tile are there instead of
@@ -188,36 +208,36 @@ __global__ __launch_bounds__(D2_WAVES * 64) void w4a16_decode2_kernel(const Deco
       // the next wavefront's slice (or of the next row) and writes there exactly what its owner writes.  The first
       // weight tile is requested before the activations, the others after them: the wait below then leaves R - 1 tiles
       // in flight.
-      const __amdgpu_buffer_rsrc_t ra = d2_rsrc32(a_loc, a_bytes_loc);
+      const __amdgpu_buffer_rsrc_t ra = d2_rsrc32(a_loc, a_bytes);
       typedef __attribute__((address_space(3))) void* lds_ptr_t;
-      issue_load(0, 0);
+      issue_load(0, 0, false);
       const int own = (GS / TPG) * 16;                         // k-octets of this wavefront's slice
       for (int mrow = 0; mrow < MR * MB; ++mrow) {
         for (int q0 = 0; q0 < own; q0 += 64) {
           const int c0 = mrow * KO + wks * own + q0;           // first slot of this instruction (wave-uniform)
           const int sl = c0 + lane;
-          const int m2 = (int)__umulhi((uint32_t)sl, p.ko_magic), ko2 = sl - m2 * KO;
+          const int m2 = (int)__umulhi((uint32_t)sl, ko_magic), ko2 = sl - m2 * KO;
           const int k = k_slab0 + (ko2 ^ (m2 & (MR - 1))) * 8;
-          const bool ok = m2 < MR * MB && m2 < M_loc && k < p.K;
+          const bool ok = m2 < MR * MB && m2 < M_loc && k < K;
           const uint32_t off = ok ? (uint32_t)(m2 * lda32 + k) * 2u : 0x80000000u;
           __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(lds + (size_t)c0 * 16), 16, (int)off, 0, 0, 0);
         }
       }
-#pragma unroll
-      for (int s = 1; s < R; ++s) issue_load(s, s);
-      constexpr int W_LATER = (R - 1) * LPT;      // vector-memory instructions requested after the activations
+      __builtin_amdgcn_sched_barrier(0);      // (the wait below counts on the order of the requests)
+      issue_first(1);
+      constexpr int W_LATER = (R - 1) * LPT + (HAS_ZP ? SUBG : 0);      // vector-memory instructions requested after the activations
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(W_LATER) : "memory");
-    } else if (p.perm == nullptr) {
+    } else if (!has_perm) {
       // Direct-to-LDS loads (no registers, no LDS write instructions): wavefront instruction q fills slots 64q .. 64q+63,
       // lane l fetching the chunk that belongs in slot 64q + l.  Rows past M, k past K and slots past the image get an
       // out-of-range offset of the buffer descriptor (which ends with the last valid element) and arrive as zeros; the
       // image is padded to a multiple of 1 KiB for the last instruction.  The weight tiles are requested after these
       // loads (loads retire in order as far as the wait counter is concerned) and stay in flight across the barrier.
-      const __amdgpu_buffer_rsrc_t ra = d2_rsrc32(a_loc, a_bytes_loc);
+      const __amdgpu_buffer_rsrc_t ra = d2_rsrc32(a_loc, a_bytes);
       typedef __attribute__((address_space(3))) void* lds_ptr_t;
       for (int c0 = w * 64; c0 < chunks; c0 += NTHR) {
         const int k = k_slab0 + (ko ^ (m & (MR - 1))) * 8;
-        const bool ok = m < MR * MB && m < M_loc && k < p.K;
+        const bool ok = m < MR * MB && m < M_loc && k < K;
         const uint32_t off = ok ? (uint32_t)(m * lda32 + k) * 2u : 0x80000000u;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(lds + (size_t)c0 * 16), 16, (int)off, 0, 0, 0);
         m += step_m;
@@ -227,8 +247,8 @@ __global__ __launch_bounds__(D2_WAVES * 64) void w4a16_decode2_kernel(const Deco
           m += 1;
         }
       }
-#pragma unroll
-      for (int s = 0; s < R; ++s) issue_load(s, s);
+      __builtin_amdgcn_sched_barrier(0);
+      issue_first(0);
       constexpr int W_LOADS = R * LPT;      // vector-memory instructions of the weight requests
       static_assert(W_LOADS < 64, "the wait counter holds 6 bits");
       asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(W_LOADS) : "memory");
@@ -245,8 +265,8 @@ __global__ __launch_bounds__(D2_WAVES * 64) void w4a16_decode2_kernel(const Deco
           kk[i] = ko;
           const int64_t k = (int64_t)k_slab0 + (int64_t)(ko ^ (m & (MR - 1))) * 8;
           v[i] = v4u{0u, 0u, 0u, 0u};
-          if (m < MR * MB && m < M_loc && k < p.K) {
-            const uint16_t* row = a_loc + (int64_t)m * p.lda;
+          if (m < MR * MB && m < M_loc && k < K) {
+            const uint16_t* row = a_loc + (int64_t)m * lda;
             const v4i p0 = *reinterpret_cast<const v4i*>(p.perm + k);
             const v4i p1 = *reinterpret_cast<const v4i*>(p.perm + k + 4);
             v[i].x = (uint32_t)row[p0.x] | ((uint32_t)row[p0.y] << 16);
@@ -566,27 +586,22 @@ template <bool BF16, int GS, int MB, bool HAS_ZP, int MR, int SUBG, int WT = 0, 
 static int launch_decode2(const Decode2Params& p_in, hipStream_t s) {
   Decode2Params p = p_in;
   const int WN = p.WN;
-  {
-    const int ko = p.WKS * GS / (WT != 0 ? 2 : 1) * 16, nthr = p.WKS * WN * 64;
-    p.wn_magic = (uint32_t)((65536 + WN - 1) / WN);
-    if (WN != 1 || p.perm != nullptr) p.PRIV = 0;
-    p.ko_magic = (uint32_t)(((1ull << 32) + (uint64_t)ko - 1) / (uint64_t)ko);
-    p.step_m = nthr / ko;
-    p.step_ko = nthr - p.step_m * ko;
-    p.b_bytes = d2_sat32((uint64_t)p.K * p.N / 2 * (WT != 0 ? 2 : 1));
-    p.s_bytes = d2_sat32((uint64_t)p.GR * p.N * 2);
-    p.z_bytes = d2_sat32((uint64_t)p.GR * (p.N / 8) * 4);
-    p.a_bytes = d2_sat32(((uint64_t)(p.M - 1) * (uint64_t)p.lda + (uint64_t)p.K) * 2);
-    if (p.a_bytes >= 0x80000000u) {
-      set_error("w4a16_gemm(decode): activations beyond 2 GiB (M = %d, row stride %lld)", p.M, (long long)p.lda);
-      return VAQ_ERR_UNSUPPORTED;
-    }
+  // The divisions of the kernel's first instructions, done here: x / WN = (x * wn_magic) >> 16 for a wavefront index, x / KO = umulhi(x, ko_magic)
+  // for a thread index (KO = k-octets of the staged slab; both exact in those ranges); steps = threads / KO, threads % KO in 16 bits each.
+  const int ko = p.WKS * GS / (WT != 0 ? 2 : 1) * 16, nthr = p.WKS * WN * 64;
+  const uint32_t wn_magic = (uint32_t)((65536 + WN - 1) / WN), ko_magic = (uint32_t)(((1ull << 32) + (uint64_t)ko - 1) / (uint64_t)ko);
+  const uint32_t steps = (uint32_t)(nthr / ko) << 16 | (uint32_t)(nthr % ko);
+  if (WN != 1 || p.perm != nullptr) p.PRIV = 0;
+  p.z_bytes = d2_sat32((uint64_t)p.GR * (p.N / 8) * 4);
+  if (((uint64_t)(p.M - 1) * (uint64_t)p.lda + (uint64_t)p.K) * 2 >= 0x80000000u) {
+    set_error("w4a16_gemm(decode): activations beyond 2 GiB (M = %d, row stride %lld)", p.M, (long long)p.lda);
+    return VAQ_ERR_UNSUPPORTED;
   }
   const size_t lds = decode2_lds_bytes(p.WKS, GS / (WT != 0 ? 2 : 1), MR, MB);
   if (p.PRIV != 0) {
     // the private fill writes whole 64-slot instructions: the last one (last row, last K slice) must end inside the
     // allocation, whatever the planner chose; otherwise the shared fill, which stays inside the padded image, is taken
-    const int own = GS / (WT != 0 ? 2 : 1) * 16, ko = p.WKS * own;
+    const int own = GS / (WT != 0 ? 2 : 1) * 16;
     const size_t last_c0 = (size_t)(MR * MB - 1) * ko + (size_t)(p.WKS - 1) * own + (size_t)((own - 1) / 64) * 64;
     if ((last_c0 + 64) * 16 > lds) p.PRIV = 0;
   }
@@ -598,8 +613,12 @@ static int launch_decode2(const Decode2Params& p_in, hipStream_t s) {
   // workgroups.  Cold, M = 1 / 4 / 16: 4096 x 6144 5.35 / 5.75 / 6.59 -> 5.16 / 5.55 / 6.32 us, 4096 x 4096 4.44 / 4.55 / 5.42 -> 4.23 /
   // 4.42 / 5.27 us, 14336 x 4096 at M = 1 / 4 8.16 / 9.09 -> 7.78 / 8.76 us; with K parts and their hand-over it costs 4 % (14336 x
   // 4096 at M = 16 / 32), wider layers show nothing either way (4096 x 28672, 4096 x 14336) or lose (8192 x 8192 at M = 1 +9 %).
-  p.gx8 = (gx % 8 == 0 && p.SK == 1 && p.NT * 2 <= num_cus_current_device() * 3 && tuning().exp[7] != 1) ? gx / 8 : 0;
-  hipLaunchKernelGGL(kern, dim3(gx, p.SK, MSP ? (p.M + 15) / 16 : 1), dim3(64, p.WKS * WN), lds, s, p);
+  const int gx8 = (gx % 8 == 0 && p.SK == 1 && p.NT * 2 <= num_cus_current_device() * 3 && tuning().exp[7] != 1) ? gx / 8 : 0;
+  // M (up to 256), K slices and n-tiles per workgroup (16), private fill, act_order, gx8 (below 2^11: gx is up to 1.5 times the compute units)
+  const uint32_t shape = (uint32_t)p.M | (uint32_t)p.WKS << 9 | (uint32_t)WN << 14 | (p.PRIV != 0 ? 1u << 19 : 0) | (p.perm != nullptr ? 1u << 20 : 0) | (uint32_t)gx8 << 21;
+  hipLaunchKernelGGL(kern, dim3(gx, p.SK, MSP ? (p.M + 15) / 16 : 1), dim3(64, p.WKS * WN), lds, s,
+                     (v8u{ptr_lo(p.a), ptr_hi(p.a), ptr_lo(p.b), ptr_hi(p.b), ptr_lo(p.scales), ptr_hi(p.scales), (uint32_t)p.lda, (uint32_t)p.G}),
+                     (v4u{(uint32_t)p.NT, shape, ko_magic, steps}), (v2u{wn_magic, (uint32_t)p.s_stride}), p);
   return VAQ_OK;
 }
 

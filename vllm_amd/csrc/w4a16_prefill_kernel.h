@@ -36,8 +36,32 @@ struct PrefillParams {
   int32_t* counters;   // arrival counters, zero on entry, left zero
   int M, N, K, G, NT, SK;
   int tail_first;      // 0: every tile in SK parts; > 0: only the tiles from this position on (see tile_slot)
+  TileSplitMagic split_magic;      // see tile_handover.h
   int s_stride, z_stride;   // elements between consecutive rows of scales (N) / zeros (N/8); 0 for channelwise scales
 };
+
+// What the first requests of the kernels with direct-to-LDS loads need, as their head (vaq_common.h); the rest is loaded.  Bit 16 of the grid's flags: one
+// row of scales.
+inline KernelHead prefill_head(const PrefillParams& p, const TileGrid& g) {
+  return KernelHead{v8u{ptr_lo(p.a), ptr_hi(p.a), ptr_lo(p.b), ptr_hi(p.b), ptr_lo(p.scales), ptr_hi(p.scales), (uint32_t)p.lda, (uint32_t)p.M},
+                    v4u{(uint32_t)p.NT, (uint32_t)p.G, g.n, g.band_magic}, v2u{g.per8, g.flags | (p.s_stride == 0 ? 1u << 16 : 0u)}};
+}
+__device__ inline PrefillParams prefill_params(const v8u& h0, const v4u& h1, const v2u& h2, const PrefillParams& rest, TileGrid& g) {
+  PrefillParams p = rest;
+  p.a = head_ptr<uint16_t>(h0[0], h0[1]);
+  p.b = head_ptr<v4u>(h0[2], h0[3]);
+  p.scales = head_ptr<uint16_t>(h0[4], h0[5]);
+  p.lda = h0[6];
+  p.M = (int)h0[7];
+  p.NT = (int)h1[0];
+  p.N = p.NT * 16;
+  p.G = (int)h1[1];
+  p.K = p.G * 128;
+  p.s_stride = h2[1] >> 16 & 1u ? 0 : p.N;
+  p.z_stride = h2[1] >> 16 & 1u ? 0 : p.N / 8;
+  g = TileGrid{h1[2], 0, h1[3], h2[0], h2[1]};
+  return p;
+}
 
 constexpr int PF_BK = 64;
 constexpr int PF_PITCH = 72;   // LDS row pitch in 16-bit elements
@@ -460,7 +484,9 @@ static __device__ inline void tile_epilogue(const PrefillParams& p, v16f (&acc)[
 //    output columns of one row: 8 bytes per lane into the epilogue's LDS staging (16-byte global stores from there);
 //  * weight words of group g+1 are requested one K step before they are needed (two register sets, by group parity).
 template <bool BF16, int BM, int BN, int WAVES_M, int WAVES_N, bool HAS_ZP, int SUBG, int WT = 0, bool PP = false>
-__global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void w4a16_prefill2_kernel(const PrefillParams p) {
+__global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void w4a16_prefill2_kernel(VAQ_HEAD_ARGS, const PrefillParams rest) {
+  TileGrid grid;
+  const PrefillParams p = prefill_params(h0, h1, h2, rest, grid);
   using T = F16Traits<BF16>;
   constexpr bool W8 = WT != 0;      // two 1 KiB blocks per tile: nibble planes of 8-bit codes (WT = 1) or FP8 e4m3 bytes (WT = 2)
   constexpr bool F8 = WT == 2;
@@ -485,18 +511,8 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void w4a16_prefill2_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
 
-  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
-  const int total = tiles_m * tiles_n;
-  const TileSlot sl = tile_slot(total, p.SK, p.tail_first);          // one contiguous range of tile positions per XCD
-  const int t = sl.pos;
-  constexpr int GM = 4;                                              // tiles are handed out in bands of 4 tile rows (2 .. 16
-                                                                     // measured: 1-3 % ahead of 8 on the large shapes), so
-  const int band = t / (GM * tiles_n);                               // that the tiles resident on one XCD share
-  const int first_m = band * GM;                                     // activation rows and weight columns in its L2
-  const int gsz = min(tiles_m - first_m, GM);
-  const int tin = t - band * GM * tiles_n;
-  const int tm = first_m + tin % gsz, tn = tin / gsz;
-  const int m0 = tm * BM, n0 = tn * BN, nt0 = n0 / 16;
+  const TileSlot sl = tile_slot(grid.rows((uint32_t)(p.M + BM - 1) / BM), p);      // one contiguous range of tile positions per XCD
+  const int m0 = sl.tm * BM, n0 = sl.tn * BN, nt0 = n0 / 16;
 
   // ---- activation tile: direct-to-LDS loads ----
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
@@ -730,7 +746,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void w4a16_prefill2_kernel(
   using FF = std::false_type;
 
   // K may be split over workgroups: this one covers the groups [g_lo, g_hi)
-  const int g_lo = (int)(((int64_t)p.G * sl.split) / sl.nsplit), g_hi = (int)(((int64_t)p.G * (sl.split + 1)) / sl.nsplit);
+  const int g_lo = tile_part(p, sl, p.G, sl.split), g_hi = tile_part(p, sl, p.G, sl.split + 1);
 
   // ---- prologue: activation tiles of the first two steps, weights of the first step (group g_lo, half 0) ----
   issue_a(2 * g_lo, 0);
@@ -924,14 +940,17 @@ static int launch_prefill(const PrefillParams& p, hipStream_t s) {
 }
 
 template <bool BF16, int BM, int BN, int WAVES_M, int WAVES_N, bool HAS_ZP, int SUBG, int WT = 0, bool PP = false>
-static int launch_prefill2(const PrefillParams& p, hipStream_t s) {
+static int launch_prefill2(const PrefillParams& p_in, hipStream_t s) {
+  PrefillParams p = p_in;
   const size_t lds = (size_t)(3 * BM + 2 * BN) * 128;
   auto kern = w4a16_prefill2_kernel<BF16, BM, BN, WAVES_M, WAVES_N, HAS_ZP, SUBG, WT, PP>;
   static size_t reserved[VAQ_MAX_DEVICES];
   if (const int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds, reserved, "w4a16_gemm(prefill)"); rc != VAQ_OK) return rc;
-  const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN, tiles = tiles_m * tiles_n;
+  const KernelHead h = prefill_head(p, tile_grid(tiles_m, tiles_n, p.SK, p.tail_first));
+  p.split_magic = tile_split_magic(tiles, p.SK, p.tail_first);
   const dim3 grid = p.tail_first > 0 ? dim3(p.tail_first + (tiles - p.tail_first) * p.SK) : dim3(tiles, p.SK);
-  hipLaunchKernelGGL(kern, grid, dim3(WAVES_M * WAVES_N * 64), lds, s, p);
+  hipLaunchKernelGGL(kern, grid, dim3(WAVES_M * WAVES_N * 64), lds, s, h.a, h.b, h.c, p);
   return VAQ_OK;
 }
 

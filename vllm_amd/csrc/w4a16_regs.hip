@@ -129,11 +129,6 @@ int w4a16_regs_launch(const void* a, int64_t lda, const int32_t* b, const void* 
   p.z_stride = channelwise ? 0 : N / 8;
   p.k_mask = 0x000f000fu;
   p.k_ex = dtype == VAQ_BF16 ? 0x43004300u : 0x64006400u;
-  const uint32_t scale_rows = channelwise ? 1 : (uint32_t)p.G * sub;
-  p.b_bytes = (uint32_t)((uint64_t)K * N / (w8 ? 1 : 2));
-  p.s_bytes = scale_rows * (uint32_t)N * 2u;
-  p.z_bytes = scale_rows * (uint32_t)(N / 8) * 4u;
-  p.a_bytes = (uint32_t)(((uint64_t)(M - 1) * (uint64_t)lda + (uint64_t)K) * 2);
   const bool bf16 = dtype == VAQ_BF16, zp = zeros != nullptr;
   int rc;
   if (w8) rc = (sub == 1 ? regs_launch_w8 : sub == 2 ? regs_launch_w8_sub2 : regs_launch_w8_sub4)(p, plan.nw, plan.j, plan.mb, bf16, s);

@@ -43,8 +43,16 @@ struct RegsParams {
   int ranges, per_xcd;     // ranges of J n-tiles; workgroups of an XCD
   int s_stride, z_stride;  // elements between consecutive rows of scales (N) / zeros (N/8); 0 for channelwise
   uint32_t k_mask, k_ex;   // 0x000f000f and the exponent pattern, as run-time values (see w4a16_decode.hip)
-  uint32_t b_bytes, s_bytes, z_bytes, a_bytes;      // each below 2 GiB
 };
+
+// Counts: rows (up to 256), parts of K (8) and blocks of rows (16) in 9, 4 and 5 bits, and above them 2^12 / blocks, rounded up: x / blocks = x * that >> 12
+// for x < 128, a copy's number.  And x / copies = umulhi(x, 2^32 / copies + 1) for the x here, below 2^25.
+inline KernelHead regs_head(const RegsParams& p) {
+  const uint32_t counts = (uint32_t)p.M | (uint32_t)p.SK << 9 | (uint32_t)p.RB << 13 | (uint32_t)((4096 + p.RB - 1) / p.RB) << 18;
+  return KernelHead{v8u{ptr_lo(p.a), ptr_hi(p.a), ptr_lo(p.b), ptr_hi(p.b), ptr_lo(p.scales), ptr_hi(p.scales), (uint32_t)p.lda, (uint32_t)p.G},
+                    v4u{(uint32_t)p.NT, counts, (uint32_t)p.ranges, (uint32_t)p.per_xcd},
+                    v2u{(uint32_t)p.s_stride, (uint32_t)((1ull << 32) / (uint32_t)(p.SK * p.RB) + 1)}};
+}
 
 constexpr size_t regs_lds_bytes(int mb, int mr, int j, int nw, int sub, bool zp) {
   const size_t run = (size_t)nw * (mb * mr * 256 + 2 * (sub * 256 + (zp ? 256 : 0)));      // activations of a k-tile, scales and zero points of two
@@ -130,7 +138,12 @@ __device__ __attribute__((always_inline)) inline void regs_store(const Params& p
 // row that is there, and their results are not stored).  SUBG: quantisation groups per k-tile (1, 2, 4).  W8: 8-bit codes as two nibble planes.  OCC: wavefronts per SIMD that the registers
 // are to allow.
 template <bool BF16, int MB, int MR, int J, bool HAS_ZP, int NW, int SUBG, bool W8, int OCC>
-__global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(const RegsParams p) {
+__global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(VAQ_HEAD_ARGS, const RegsParams p) {
+  // what the first requests need (see regs_head)
+  const uint16_t* const a = head_ptr<uint16_t>(h0[0], h0[1]);
+  const v4u* const b = head_ptr<v4u>(h0[2], h0[3]);
+  const uint16_t* const scales = head_ptr<uint16_t>(h0[4], h0[5]);
+  const uint32_t lda = h0[6], G = h0[7], NT = h1[0], counts = h1[1], ranges = h1[2], per_xcd = h1[3], s_stride = h2[0], copies_magic = h2[1];
   using T = F16Traits<BF16>;
   static_assert(!(W8 && HAS_ZP), "8-bit codes have no zero points");
   static_assert(MR == 16 || (MR == 4 && MB == 1), "fewer rows of a single m-block only");
@@ -139,20 +152,32 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(const RegsPara
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int o = lane >> 4, r16 = lane & 15;
-  // One contiguous range of units per XCD; the K parts and row blocks of one range of n-tiles are neighbours.
-  const int unit = (int)(blockIdx.x & 7u) * p.per_xcd + (int)(blockIdx.x >> 3);
-  const int copies = p.SK * p.RB;
-  if (unit >= p.ranges * copies) return;
-  const int range = unit / copies, rest = unit - range * copies;
-  const int sk = rest / p.RB, rb_i = rest - sk * p.RB;
-  const int nt0 = range * J, row0 = rb_i * MB * 16;
-  const int g_lo = (int)(((int64_t)p.G * sk) / p.SK), g_hi = (int)(((int64_t)p.G * (sk + 1)) / p.SK);
+  const int M = (int)(counts & 0x1ffu), SK = (int)(counts >> 9 & 0xfu), RB = (int)(counts >> 13 & 0x1fu);
+  // One contiguous range of units per XCD; the K parts and row blocks of one range of n-tiles are neighbours.  (No division where K is whole: a 32-bit
+  // one is some 30 instructions, a 64-bit one more than 100.)
+  const uint32_t unit = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3), copies = (uint32_t)(SK * RB);
+  if (unit >= ranges * copies) return;
+  uint32_t range = unit, sk = 0, rb_u = 0, g_lo_u = 0, g_hi_u = G;
+  if (copies > 1) {
+    range = __umulhi(unit, copies_magic);
+    rb_u = unit - range * copies;
+    if (SK > 1) {
+      sk = rb_u * (counts >> 18) >> 12;
+      rb_u -= sk * (uint32_t)RB;
+      g_lo_u = G * sk / (uint32_t)SK;
+      g_hi_u = G * (sk + 1) / (uint32_t)SK;
+    }
+  }
+  const int rb_i = (int)rb_u, g_lo = (int)g_lo_u, g_hi = (int)g_hi_u;
+  const int nt0 = (int)range * J, row0 = rb_i * MB * 16;
 
   auto rsrc = [](const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
   };
-  const __amdgpu_buffer_rsrc_t ra = rsrc(p.a, p.a_bytes), rb = rsrc(p.b, p.b_bytes), rs = rsrc(p.scales, p.s_bytes);
-  const __amdgpu_buffer_rsrc_t rz = rsrc(HAS_ZP ? (const void*)p.zeros : (const void*)p.scales, HAS_ZP ? p.z_bytes : p.s_bytes);
+  // (the extents are those of RegsParams)
+  const __amdgpu_buffer_rsrc_t ra = rsrc(a, ((uint32_t)(M - 1) * lda + G * 128u) * 2u), rb = rsrc(b, NT * G * (uint32_t)(PL * 1024));
+  const uint32_t s_bytes = (s_stride ? G * (uint32_t)SUBG : 1u) * NT * 32u;
+  const __amdgpu_buffer_rsrc_t rs = rsrc(scales, s_bytes), rz = HAS_ZP ? rsrc(p.zeros, s_bytes / 4) : rs;
 
   // This wavefront's piece of LDS: the activations of the next k-tile, MR * MB rows of 256 bytes with chunk c of row r at place
   // c ^ (r & 15); scales (256 bytes per group row) and zero points (64 per row, one piece) of the k-tile at hand and the next.
@@ -162,7 +187,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(const RegsPara
 #pragma unroll
   for (int i = 0; i < AI; ++i) {
     const int r = i * 4 + o;
-    vo_a[i] = (uint32_t)min(row0 + r, p.M - 1) * (uint32_t)p.lda * 2u + (uint32_t)((r16 ^ (r & 15)) * 16);
+    vo_a[i] = (uint32_t)min(row0 + r, M - 1) * lda * 2u + (uint32_t)((r16 ^ (r & 15)) * 16);
   }
   constexpr uint32_t OUT = 0x80000000u;      // past the end of every buffer: reads as zero
   struct At {                                // a k-tile: its number, or 0 and OUT for none
@@ -178,7 +203,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(const RegsPara
 #pragma unroll
     for (int sj = 0; sj < SUBG; ++sj)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(side + sj * 256), 4, (int)((lane < J * 8 ? (uint32_t)lane * 4u : OUT) | t.out),
-                                               (int)(((t.g * SUBG + sj) * (uint32_t)p.s_stride + (uint32_t)nt0 * 16u) * 2u), 0, 0);
+                                               (int)(((t.g * SUBG + sj) * s_stride + (uint32_t)nt0 * 16u) * 2u), 0, 0);
     if constexpr (HAS_ZP) {      // 16 lanes a row
       const uint32_t vo = o < SUBG && r16 < J * 2 ? (uint32_t)o * (uint32_t)p.z_stride * 4u + (uint32_t)r16 * 4u : OUT;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rz, (lds_ptr_t)(side + SC), 4, (int)(vo | t.out),
@@ -187,10 +212,10 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(const RegsPara
   };
   v4u wq[2][J][PL];
   auto load_w = [&](int s, At t, int j) {
-    const uint32_t nt = (uint32_t)min(nt0 + j, p.NT - 1);
+    const uint32_t nt = (uint32_t)min(nt0 + j, (int)NT - 1);
 #pragma unroll
     for (int pl = 0; pl < PL; ++pl)
-      wq[s][j][pl] = __builtin_amdgcn_raw_buffer_load_b128(rb, (int)((uint32_t)lane * 16u | t.out), (int)(((nt * (uint32_t)p.G + t.g) * PL + pl) * 1024u), 2);
+      wq[s][j][pl] = __builtin_amdgcn_raw_buffer_load_b128(rb, (int)((uint32_t)lane * 16u | t.out), (int)(((nt * G + t.g) * PL + pl) * 1024u), 2);
   };
 
   v4f acc[J][MB];
@@ -338,7 +363,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(const RegsPara
     const int nt = nt0 + j;
     if (nt >= p.NT || row0 + mb * 16 >= p.M) continue;
     v4f val = regs_sum<NW>(red, J * MB, q, here);
-    if (p.SK > 1) {
+    if (SK > 1) {
       // partial tiles and counters as in w4a16_decode2_kernel.h, step 5
       const uint32_t units = (uint32_t)p.NT * (uint32_t)(p.RB * MB), u = (uint32_t)nt * (uint32_t)(p.RB * MB) + (uint32_t)(rb_i * MB + mb);
       const __amdgpu_buffer_rsrc_t rt = rsrc(p.c_tmp, units * 1024u * (uint32_t)p.SK);
@@ -366,7 +391,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(const RegsPara
 #ifdef __HIP_DEVICE_COMPILE__
     asm volatile("" : "+s"(args), "+s"(q), "+s"(nt_h), "+s"(row_h), "+s"(rb_h));
 #endif
-    const auto& pa = *(const __attribute__((address_space(4))) RegsParams*)args;
+    const auto& pa = *(const __attribute__((address_space(4))) RegsParams*)((const __attribute__((address_space(4))) char*)args + HEAD_BYTES);
 #pragma unroll 1
     for (; odd != 0; q += NW, odd >>= 1) {
       if (!(odd & 1u)) continue;
@@ -402,7 +427,8 @@ static int launch_regs(const RegsParams& p, hipStream_t s) {
   auto kern = w4a16_regs_kernel<BF16, MB, MR, J, HAS_ZP, NW, SUBG, W8, NW == 4 && (regs_estimate(MB, J, SUBG, W8) > 256) ? 1 : 2>;
   static size_t reserved[VAQ_MAX_DEVICES];
   if (const int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds, reserved, "w4a16_gemm(regs)"); rc != VAQ_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3(p.per_xcd * 8), dim3(NW * 64), lds, s, p);
+  const KernelHead h = regs_head(p);
+  hipLaunchKernelGGL(kern, dim3(p.per_xcd * 8), dim3(NW * 64), lds, s, h.a, h.b, h.c, p);
   return VAQ_OK;
 }
 

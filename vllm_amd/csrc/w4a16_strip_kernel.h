@@ -38,7 +38,9 @@ constexpr size_t strip_lds_bytes(int nst) {
 
 // (The smallest strips with zero points of four groups: two workgroups to a compute unit, which 128 registers allow and 130 do not.)
 template <bool BF16, int WMB, int WNB, int NS, bool HAS_ZP, int SUBG, bool W8, int NST, int PD>
-__global__ __launch_bounds__(512, WMB * WNB == 1 && HAS_ZP && SUBG == 4 ? 4 : 2) void w4a16_strip_kernel(const PrefillParams p) {
+__global__ __launch_bounds__(512, WMB * WNB == 1 && HAS_ZP && SUBG == 4 ? 4 : 2) void w4a16_strip_kernel(VAQ_HEAD_ARGS, const PrefillParams rest) {
+  TileGrid grid;
+  const PrefillParams p = prefill_params(h0, h1, h2, rest, grid);
   using T = F16Traits<BF16>;
   constexpr int KG = 8 / NS, BM = 32 * WMB, TN = 32 * WNB, BN = TN * NS, NW = 8;
   constexpr int TW = 2 * WNB;                      // native tiles of a strip
@@ -55,17 +57,10 @@ __global__ __launch_bounds__(512, WMB * WNB == 1 && HAS_ZP && SUBG == 4 ? 4 : 2)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kg = wave / NS, ns = wave % NS;
 
-  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
-  const TileSlot sl = tile_slot(tiles_m * tiles_n, p.SK, p.tail_first);
-  constexpr int GM = 4;                            // bands of 4 tile rows (see the LDS-staged kernel)
-  const int band = sl.pos / (GM * tiles_n);
-  const int first_m = band * GM;
-  const int gsz = min(tiles_m - first_m, GM);
-  const int tin = sl.pos - band * GM * tiles_n;
-  const int tm = first_m + tin % gsz, tn = tin / gsz;
-  const int m0 = tm * BM, n0 = tn * BN;
+  const TileSlot sl = tile_slot(grid.rows((uint32_t)(p.M + BM - 1) / BM), p);
+  const int m0 = sl.tm * BM, n0 = sl.tn * BN;
   // K may be split over workgroups: this one covers the groups [g_lo, g_hi)
-  const int g_lo = (int)(((int64_t)p.G * sl.split) / sl.nsplit), g_hi = (int)(((int64_t)p.G * (sl.split + 1)) / sl.nsplit);
+  const int g_lo = tile_part(p, sl, p.G, sl.split), g_hi = tile_part(p, sl, p.G, sl.split + 1);
   const int ng = g_hi - g_lo;
   const int t_full = ng / KG, rem = ng % KG;       // rounds in which all K groups take part; wavefronts of the last one
 
@@ -411,15 +406,18 @@ __global__ __launch_bounds__(512, WMB * WNB == 1 && HAS_ZP && SUBG == 4 ? 4 : 2)
 }
 
 template <bool BF16, int WMB, int WNB, int NS, bool HAS_ZP, int SUBG, bool W8, int NST, int PD>
-static int launch_strip(const PrefillParams& p, hipStream_t s) {
+static int launch_strip(const PrefillParams& p_in, hipStream_t s) {
+  PrefillParams p = p_in;
   constexpr size_t lds = strip_lds_bytes<WMB, WNB, NS>(NST);
   static_assert(lds <= 160 * 1024, "LDS");
   auto kern = w4a16_strip_kernel<BF16, WMB, WNB, NS, HAS_ZP, SUBG, W8, NST, PD>;
   static size_t reserved[VAQ_MAX_DEVICES];
   if (const int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds, reserved, "w4a16_gemm(strip)"); rc != VAQ_OK) return rc;
-  const int tiles = ((p.M + 32 * WMB - 1) / (32 * WMB)) * ((p.N + 32 * WNB * NS - 1) / (32 * WNB * NS));
+  const int tiles_m = (p.M + 32 * WMB - 1) / (32 * WMB), tiles_n = (p.N + 32 * WNB * NS - 1) / (32 * WNB * NS), tiles = tiles_m * tiles_n;
+  const KernelHead h = prefill_head(p, tile_grid(tiles_m, tiles_n, p.SK, p.tail_first));
+  p.split_magic = tile_split_magic(tiles, p.SK, p.tail_first);
   const dim3 grid = p.tail_first > 0 ? dim3(p.tail_first + (tiles - p.tail_first) * p.SK) : dim3(tiles, p.SK);
-  hipLaunchKernelGGL(kern, grid, dim3(512), lds, s, p);
+  hipLaunchKernelGGL(kern, grid, dim3(512), lds, s, h.a, h.b, h.c, p);
   return VAQ_OK;
 }
 
