@@ -840,6 +840,7 @@ __global__ __launch_bounds__(512) void fp8_mm_stream_kernel(VAQ_HEAD_ARGS, const
   };
 #pragma unroll
   for (int s = 0; s < KS; ++s) issue(nt0, s, nt0 < nt1);
+  VAQ_ARRIVED4(p.sb, p.bias, p.out, p.sb_per_col);
 
   // Epilogue operands are requested ahead of their use (a load issued after the reduction would stall the reducing
   // wavefront, and through the next barrier the whole workgroup, for a memory round trip per n-tile): the activation

@@ -114,6 +114,12 @@ typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 // head of three vectors a launch that reads 8.4 MB takes 2.95 instead of 3.17 us.  (Vectors because the host's cost of a launch grows with the number
 // of arguments: as 11 scalars they cost 0.3 us a launch.)
 typedef unsigned int v8u __attribute__((ext_vector_type(8)));
+// The rest has to be there ahead of a loop with LDS reads: while a scalar load is under way a wait for one of them is a wait for all.
+#ifdef __HIP_DEVICE_COMPILE__
+#define VAQ_ARRIVED4(a, b, c, d) asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d))
+#else
+#define VAQ_ARRIVED4(a, b, c, d)
+#endif
 #define VAQ_HEAD_ARGS const vaq::v8u h0, const vaq::v4u h1, const vaq::v2u h2
 constexpr int HEAD_BYTES = 56;
 struct KernelHead {
