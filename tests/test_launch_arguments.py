@@ -38,3 +38,24 @@ def test_quotients_of_copies():
 
 def test_leading_arguments_are_asked_for_in_registers():
     assert "-amdgpu-kernarg-preload-count=16" in HIPCC_FLAGS
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k,gs,wks,wn", [(4096, 4, 8, 1), (4096, 4, 8, 2), (4096, 8, 4, 1), (4096, 16, 2, 7), (3584, 7, 4, 1), (3584, 14, 2, 3),
+                                         (2048, 2, 4, 1), (4224, 4, 4, 2), (512, 1, 4, 1), (384, 1, 2, 1)])
+@pytest.mark.parametrize("m", [1, 3, 5, 9, 15, 16, 21])
+def test_activation_fill_of_every_shape(device, k, gs, wks, wn, m):
+    """Workgroups whose wavefronts are a whole number of pieces of a row, of rows, or neither, slabs that end inside K and past it, and rows
+    between the numbers that are staged: a row that is not there leaves the others alone."""
+    import torch
+
+    from oracle import w4a16 as o
+    from tests.helpers import W4A16Layer, check_gemm_close
+    from vllm_amd import _tuning
+    n = 192
+    case = o.make_w4a16_case(k, n, 128, asym=bool(m & 1), seed=k + m + gs)
+    layer = W4A16Layer(case, device)
+    a = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(torch.bfloat16).to(device)
+    with _tuning.override(decode_impl=1, decode2_gs=gs, decode2_wks=wks, decode2_wn=wn):
+        check_gemm_close(layer(a), o.gemm_ref(a.cpu(), o.case_w_ref(case)), f"k={k} plan {gs}, {wks}, {wn} m={m}")
+    assert bool((layer.workspace == 0).all())

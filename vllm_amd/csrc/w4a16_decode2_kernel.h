@@ -200,7 +200,7 @@ __global__ __launch_bounds__(D2_WAVES * 64) void w4a16_decode2_kernel(VAQ_HEAD_A
     // chunk c = m * KO + ko' (LDS slot c); thread tid handles c = tid, tid + NTHR, ...  The (m, ko') pair is advanced
     // incrementally: one scalar division per kernel instead of one vector division per chunk.
     int m = (int)__umulhi((uint32_t)tid, ko_magic), ko = tid - m * KO;
-    if (priv) {
+    if (MR <= 4 && GS <= 8 && priv) {
       // Private fill (one n-tile per workgroup, so no two wavefronts read the same k-octets): every wavefront fetches the
       // k-octets of its own K slice, row by row, and waits for nobody -- the same bytes travel as in the shared fill, but
       // a wavefront starts on its first tile as soon as ITS activations and ITS first weight tile are there instead of
@@ -235,6 +235,24 @@ __global__ __launch_bounds__(D2_WAVES * 64) void w4a16_decode2_kernel(VAQ_HEAD_A
       // loads (loads retire in order as far as the wait counter is concerned) and stay in flight across the barrier.
       const __amdgpu_buffer_rsrc_t ra = d2_rsrc32(a_loc, a_bytes);
       typedef __attribute__((address_space(3))) void* lds_ptr_t;
+      if ((KO & 63) == 0 && (step_m == 0 || step_ko == 0) && slab_g0 + slab_groups <= (int)G) {
+        // Whole pieces of 64 slots of one row, inside K: their place is scalar arithmetic, a lane's is its chunk, and rows past M are left out (nobody
+        // stores what is computed from them).
+        const int Q = KO / 64, NW = WKS * WN;
+        const int rows = min(MR * MB, M_loc), step = step_m > 0 ? step_m : 1;
+        const int m0 = step_m > 0 ? m : 0, q0 = step_m > 0 ? ko / 64 : w;      // (of the wavefront's first lane)
+        const uint32_t s_step = (uint32_t)(step * lda32) * 2u, l_step = (uint32_t)(step * KO) * 16u;
+        for (int q = __builtin_amdgcn_readfirstlane(q0); q < Q; q += NW) {
+          int mr = __builtin_amdgcn_readfirstlane(m0);
+          uint32_t so = (uint32_t)(mr * lda32 + k_slab0 + q * 512) * 2u, at = (uint32_t)(mr * KO + q * 64) * 16u;
+#pragma unroll 1
+          for (; mr < rows; mr += step) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(lds + at), 16, (lane ^ (mr & (MR - 1))) * 16, (int)so, 0, 0);
+            so += s_step;
+            at += l_step;
+          }
+        }
+      } else
       for (int c0 = w * 64; c0 < chunks; c0 += NTHR) {
         const int k = k_slab0 + (ko ^ (m & (MR - 1))) * 8;
         const bool ok = m < MR * MB && m < M_loc && k < K;
