@@ -3,6 +3,8 @@
 #include "tile_handover.h"
 #include "vaq_common.h"
 
+#include <type_traits>
+
 namespace vaq {
 
 struct Fp8MMParams {
@@ -188,7 +190,9 @@ __global__ __launch_bounds__(512) void fp8_mm_stream2_kernel(VAQ_HEAD_ARGS, cons
   };
 #pragma unroll
   for (int st = 0; st < NSR; ++st) issue_stage(nt0, st, st, nt0 < nt1);
-  VAQ_ARRIVED4(p.sb, p.bias, p.out, p.sb_per_col);      // (M = 16 on 4096 x 6144 7.08 -> 6.88 us, M = 7 on 4096 x 4096 5.36 -> 5.07)
+  // (M = 16 on 4096 x 6144 7.08 -> 6.88 us, M = 7 on 4096 x 4096 5.36 -> 5.07, 5.21 with the wait ahead of the loop below.  Quantised here it is there: a given
+  // scale's own load would come behind it, 4096 x 6144 at M = 8 7.02 -> 8.02.)
+  if constexpr (MQ == 0) VAQ_ARRIVED4(p.sb, p.bias, p.out, p.sb_per_col);
 
   const bool reducer_wave = WK > 1 ? w < MB : true;
   float sam_mb[MB];
@@ -289,6 +293,7 @@ __global__ __launch_bounds__(512) void fp8_mm_stream2_kernel(VAQ_HEAD_ARGS, cons
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.sb), 0, p.sb_per_col ? p.N * 4 : 4, 0x00020000);
   const __amdgpu_buffer_rsrc_t rbias =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.bias), 0, p.bias ? p.N * 2 : 0, 0x00020000);
+  if constexpr (MQ > 0) VAQ_ARRIVED4(p.sb, p.bias, p.out, p.sb_per_col);
   int parity = 0;
   for (int nt = nt0; nt < nt1; ++nt) {
     v4f acc[MB];
@@ -329,8 +334,20 @@ __global__ __launch_bounds__(512) void fp8_mm_stream2_kernel(VAQ_HEAD_ARGS, cons
       // the partial tiles are written; the bare barrier leaves the next tile's weight requests in flight (a
       // __syncthreads() would wait for every direct-to-LDS load)
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if (reducer)
-        for (int ww = 0; ww < WK; ++ww) tot += buf[(ww * MB + w) * 64 + lane];
+      // up to eight parts, four or eight reads under way at a time (one by one each waits out the LDS latency, and the others wait for the reducer)
+      auto sum = [&](auto most) {
+        constexpr int N = decltype(most)::value;
+        v4f part[N];
+#pragma unroll
+        for (int ww = 0; ww < N; ++ww) part[ww] = buf[(min(ww, WK - 1) * MB + w) * 64 + lane];
+#pragma unroll
+        for (int ww = 0; ww < N; ++ww)
+          if (ww < WK) tot += part[ww];
+      };
+      if (reducer) {
+        if (WK <= 4) sum(std::integral_constant<int, 4>{});
+        else sum(std::integral_constant<int, 8>{});
+      }
       parity ^= 1;
     } else {
       reducer = true;
