@@ -65,17 +65,21 @@ static int other_kind(int M, int N, int K, int sub, int wt, double* us) {
 }
 
 // Whether the kernel with activations in registers takes a problem: where it is predicted to be ahead of what takes it otherwise by so much that
-// few calls lose.  4-bit codes in groups of 128 rows 15 % up to 4 rows and 13 % up to 32, where the decode kernel's plans by rule are on some
+// few calls lose.  4-bit codes in groups of 128 rows 15 % up to 4 rows and 9 % up to 32, where the decode kernel's plans by rule are on some
 // layers that much better than priced (14336 x 4096 at M = 4 9.0 us, priced 9.9; this kernel 10.0, priced 8.7), 5 % up to 64 rows and 8 % beyond;
 // vocabulary-sized layers at 3 .. 16 rows, where another kernel is the alternative, 5 % (it takes them all: 0.37 .. 0.96 of the time, 1 of 2000 more than 3 %
 // slower; 4096 x 128256 at M = 4 / 16 54.9 / 59.0 -> 51.9 / 53.4 us, 1024 x 128256 33.4 / 34.0 -> 18.1 / 19.5, 5120 x 65536 80.0 / 81.0 -> 33.2 / 34.7);
-// in groups of 64 / 32 rows 12 % from 33 rows on, where zero points cost more than priced; all others 5 %.  Over 20254 calls of drawn layers that
+// in groups of 64 / 32 rows 12 % from 33 rows on, where zero points cost more than priced; 8-bit codes none up to 32 rows (up to 4 rows 17 % behind is
+// still taken); all others 5 %.  The prices are older than the arguments in registers, which gained this kernel more than the others: with 13 % and 5 %
+// in these two places 3 % of 12000 drawn problems of 1 .. 256 rows went elsewhere, for 1.085 of the time in the mean, 8 % of them more than 3 % ahead there.  (Smaller
+// leads for the rest gain less than 0.2 % and lose on a fifth of what they move.)  Over 20254 calls of drawn layers that
 // it took at 5 % where it now asks for 8 and 12, timed both ways afterwards: 0.842 of their time in the mean, 3.9 % more than 3 % slower, 0.5 % more than 10 %.
 static double regs_lead(int M, int N, int K, int sub, int wt, int j, int nw) {
-  if (wt != 0 || decode_impl_for(M, N, K, sub, false) == 1) return 0.95;
+  if (wt == 0 && decode_impl_for(M, N, K, sub, false) == 1) return 0.95;
+  if (wt != 0) return M <= 4 ? 1.17 : M <= 32 ? 1.01 : 0.95;
   if (sub > 1) return M > 32 ? 0.88 : 0.95;
   if (M > 32) return M <= 64 ? 0.95 : 0.92;
-  const double lead = M <= 4 ? 0.85 : 0.87;
+  const double lead = M <= 4 ? 0.85 : 0.91;
   // Where this kernel loses most of what it loses, by as much as the two prices together are off by: K of whole 1024 rows; one n-tile to a wavefront and K
   // beyond 8192 at up to 4 rows; two and more n-tiles on a short K.  Off are: this kernel's price, which counts 16 rows to a block, by the rows that a block has;
   // for workgroups of four; for one n-tile, which leaves 2 KB of weights in flight, by how much of the device waits for them and how long; for three and more
