@@ -399,8 +399,10 @@ __global__ __launch_bounds__(256) void fp8_mm_tile2_kernel(const Fp8MMParams p) 
 //    wavefronts of the same tile (fewer fragment reads, same time), sixteen wavefronts, four-slice stages of 64 x 64 tiles;
 //  * WAVES_M x WAVES_N wavefronts; tiles are handed out in bands of 4 tile rows inside each XCD's contiguous range so
 //    that the tiles resident on one XCD share activation rows and weight columns in its L2.
-// Requires K % 64 == 0 (a partial last step would read the neighbouring row instead of zeros) and M*lda, N*ldb < 2^32.
-template <bool BF16_OUT, int BM, int BN, int WAVES_M, int WAVES_N, int NST, int KS = 1, int PP = 0>
+// Requires M*lda, N*ldb < 2^32, and K % 64 == 0, or a multiple of 16 with TAIL: a step that ends past K would read the neighbouring row instead of
+// zeros, so that every chunk of 16 bytes is tested and those past K are requested behind the operand's end (8 vector instructions a step; all
+// offsets below 2 GiB, see dispatch_tile).
+template <bool BF16_OUT, int BM, int BN, int WAVES_M, int WAVES_N, int NST, int KS = 1, int PP = 0, bool TAIL = false>
 __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(VAQ_HEAD_ARGS, const Fp8MMParams p) {
   // what the first requests need (vaq_common.h; see launch_tile3)
   const uint8_t* const a = head_ptr<uint8_t>(h0[0], h0[1]);
@@ -445,7 +447,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(VA
 
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   // K may be split over workgroups: this one covers the steps [s_lo, s_hi)
-  const int all_steps = K / (64 * KS);
+  const int all_steps = TAIL ? (K + 64 * KS - 1) / (64 * KS) : K / (64 * KS);
   // (in pairs: parts start at even steps, so that the two slices of a request share their cache lines)
   const auto part = [&](int i) { return i >= sl.nsplit ? all_steps : tile_part(p, sl, all_steps, i) & (PAIR ? ~1 : ~0); };
   const int s_lo = part(sl.split), s_hi = part(sl.split + 1);
@@ -488,8 +490,15 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(VA
       }
     }
   };
-  auto load_a = [&](uint32_t koff, uint8_t* at) { load(std::integral_constant<int, BM>{}, ra, (uint32_t)m0, lda, voff_a, voff_a1, koff, at); };
-  auto load_b = [&](uint32_t koff, uint8_t* at) { load(std::integral_constant<int, BN>{}, rb, (uint32_t)n0, ldb, voff_b, voff_b1, koff, at); };
+  // (a chunk past K: an offset past either operand's end)
+  static_assert(!TAIL || LINE, "chunks past K of single slices are not built");
+  auto in_k = [&](uint32_t offset, uint32_t byte) { return !TAIL || byte < (uint32_t)K ? offset : 0x80000000u; };
+  auto load_a = [&](uint32_t koff, uint8_t* at) {
+    load(std::integral_constant<int, BM>{}, ra, (uint32_t)m0, lda, in_k(voff_a, koff + lbyte), in_k(voff_a1, koff + (lbyte ^ 32u)), koff, at);
+  };
+  auto load_b = [&](uint32_t koff, uint8_t* at) {
+    load(std::integral_constant<int, BN>{}, rb, (uint32_t)n0, ldb, in_k(voff_b, koff + lbyte), in_k(voff_b1, koff + (lbyte ^ 32u)), koff, at);
+  };
   // Steps are requested in order: the first byte of K of the next one, rotation applied.  (As few scalar instructions as can be: the matrix
   // cores wait for them at the start of every step.)
   constexpr uint32_t K_STEP = PAIR ? 128 : 64 * KS;
@@ -1011,11 +1020,11 @@ static int launch_tile2(const Fp8MMParams& p, hipStream_t s) {
   return VAQ_OK;
 }
 
-template <bool BF16_OUT, int BM, int BN, int WAVES_M, int WAVES_N, int NST, int KS = 1, int PP = 0>
+template <bool BF16_OUT, int BM, int BN, int WAVES_M, int WAVES_N, int NST, int KS = 1, int PP = 0, bool TAIL = false>
 static int launch_tile3(const Fp8MMParams& p_in, hipStream_t s) {
   Fp8MMParams p = p_in;
   const size_t lds = (size_t)NST * KS * (BM + BN) * 64;
-  auto kern = fp8_mm_tile3_kernel<BF16_OUT, BM, BN, WAVES_M, WAVES_N, NST, KS, PP>;
+  auto kern = fp8_mm_tile3_kernel<BF16_OUT, BM, BN, WAVES_M, WAVES_N, NST, KS, PP, TAIL>;
   static size_t reserved[VAQ_MAX_DEVICES];
   if (const int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds, reserved, "fp8_scaled_mm"); rc != VAQ_OK) return rc;
   const int tiles_m = (p.M + BM - 1) / BM + p.m_tiles_extra, tiles_n = (p.N + BN - 1) / BN, tiles = tiles_m * tiles_n;
@@ -1029,7 +1038,7 @@ static int launch_tile3(const Fp8MMParams& p_in, hipStream_t s) {
   return VAQ_OK;
 }
 
-// The tile shapes of the multi-stage kernel (ids for K % 128 == 0; the two-slice shapes have one with a slice per step, id - 10).
+// The tile shapes of the multi-stage kernel (ids above 10 take two slices of K a step; asked for, id - 10 is the same).
 // Fitted to 2064 problems with M = 9 .. 8192, half of them with K = 1024 .. 14336 and N = 1024 .. 28672, half with K = 256 .. 28672 and
 // N = 256 .. 152064, drawn over the logarithm, every shape and K split of each timed on cold weights (30154 launches,
 // the first half of those in profiles/plan_prices).  Over all 5493 problems there (91351 launches) the plan with the least predicted
@@ -1052,11 +1061,12 @@ constexpr TileCosts FP8_TILE_COSTS = {0.149, 2.14, 0.56, 0.254, 1.0};
 
 static TilePlan make_plan_tile3(int M, int N, int K) {
   const int64_t cus = num_cus_current_device();
-  const int steps = K / 64;
+  const int steps = (K + 63) / 64;
   const VaqTuning& tn = tuning();
   TilePlan best;
   for (const TileShape& t : FP8_TILE_SHAPES) {
     if (tn.fp8_tile_cfg > 0 ? tn.fp8_tile_cfg != t.id && tn.fp8_tile_cfg != t.id - 10 : t.id == 10 && N % 384 != 0) continue;
+    if (K % 64 != 0 && t.id == 10) continue;      // (no registers for the test of chunks past K)
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
     const int64_t rest = tiles % cus;
     auto consider = [&](int sk, int64_t tail_first) {
@@ -1078,8 +1088,6 @@ static TilePlan make_plan_tile3(int M, int N, int K) {
         if (rest * sk <= cus && (tn.exp[6] > 1 ? sk == tn.exp[6] && steps / sk >= 4 : steps / sk >= 16)) consider(sk, tiles - rest);
   }
   if (best.id < 0) return best;      // an unknown shape was forced: the other kernels take the problem
-  if (tn.fp8_tile_cfg > 0) best.id = tn.fp8_tile_cfg;
-  if (best.id > 10 && K % 128 != 0) best.id -= 10;
   // A split K with compute units left for the parts of one more tile row: that row runs past M beside the real ones, as
   // with an unsplit K (see m_tiles_extra in dispatch_tile); its workgroups take no part in the hand-over, but tile
   // positions -- and with them the places in the scratch -- count it.  Cold: 7168 x 2048 at M = 40 / 64 / 192 12.1 / 13.6 /
@@ -1104,10 +1112,19 @@ static int dispatch_tile(const Fp8MMParams& p_in, int64_t c_tmp_bytes, int64_t c
   // 256 x 256 tile requests 128 bytes where K leaves 64.
   p.a_extent = (uint32_t)((int64_t)(p.M - 1) * p.lda + p.K);
   p.b_extent = (uint32_t)((int64_t)(p.N - 1) * p.ldb + p.K);
-  const bool direct_ok = tuning().fp8_tile_impl == 0 && p.K % 64 == 0 && (uint64_t)p.M * (uint64_t)p.lda < (1ull << 32) &&
-                         (uint64_t)p.N * (uint64_t)p.ldb < (1ull << 32);
+  // A step that ends past K: no place of a request, rows past M and N among them, may be beyond 2 GiB, so that it and the offset of a chunk past K do
+  // not wrap.
+  const bool far = ((uint64_t)p.M + 512) * (uint64_t)p.lda >= (1ull << 31) || ((uint64_t)p.N + 512) * (uint64_t)p.ldb >= (1ull << 31);
+  const bool direct_ok = tuning().fp8_tile_impl == 0 && (uint64_t)p.M * (uint64_t)p.lda < (1ull << 32) && (uint64_t)p.N * (uint64_t)p.ldb < (1ull << 32) &&
+                         (p.K % 64 == 0 || !far);
   if (direct_ok && tuning().fp8_tile_impl == 0 && tuning().fp8_tile_cfg >= 0) {
     TilePlan pl = plan_tile3(p.M, p.N, p.K);
+    if (pl.id > 10 && p.K % 128 == 64 && far) {      // (the 256 x 256 tile steps by 64 bytes)
+      pl = TilePlan();
+      pl.id = 1;
+      pl.bm = pl.bn = 256;
+      pl.tiles = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256);
+    }
     // without (enough) scratch from the caller the unsplit kernel still gives the result
     if (pl.sk > 1 && (p.c_tmp == nullptr || p.counters == nullptr || counter_ints < pl.counter_ints() ||
                       c_tmp_bytes < pl.tmp_bytes()))
@@ -1151,23 +1168,29 @@ static int dispatch_tile(const Fp8MMParams& p_in, int64_t c_tmp_bytes, int64_t c
         p.rotate_k = 0;
       }
     }
-    switch (pl.id) {
+    // K in steps of 128 bytes (the 256-wide tiles: of 64) ends inside the last one.  All K that are no multiple of 64 once went through registers and padded LDS:
+    // 80 drawn problems of 33 .. 8192 rows take 0.56 of that time in the mean (126 rows of 8400 x 4096 59.5 -> 22.0 us, 1700 of 5968 x 2368 52.4 -> 50.8); K % 128 = 64
+    // went by slices of 64, half a cache line: 90 problems 0.95 (232 rows of 13632 x 25280 163 -> 136 us, the worst 198 of 1472 x 5632 8.7 -> 9.2).
+    if (p.K % 64 != 0 || (p.K % 128 != 0 && pl.id > 10)) switch (pl.id) {
+        case 1: return launch_tile3<BF16_OUT, 256, 256, 2, 4, 5, 1, 2, true>(p, s);
+        case 13: return launch_tile3<BF16_OUT, 128, 128, 2, 4, 4, 2, 0, true>(p, s);
+        case 14: return launch_tile3<BF16_OUT, 64, 128, 2, 2, 5, 2, 0, true>(p, s);
+        case 15: return launch_tile3<BF16_OUT, 64, 64, 2, 2, 5, 2, 0, true>(p, s);
+        case 16: return launch_tile3<BF16_OUT, 128, 64, 2, 2, 5, 2, 0, true>(p, s);
+        case 17: return launch_tile3<BF16_OUT, 128, 256, 2, 4, 3, 2, 0, true>(p, s);
+        case 19: return launch_tile3<BF16_OUT, 256, 128, 4, 2, 3, 2, 0, true>(p, s);
+        default: break;
+      }
+    else switch (pl.id) {
       case 1: return launch_tile3<BF16_OUT, 256, 256, 2, 4, 5, 1, 2>(p, s);    // alternating phases, slices requested in pairs (see the kernel)
       case 10: return launch_tile3<BF16_OUT, 256, 384, 2, 4, 4, 1, 1>(p, s);   // 8 wavefronts of 128 x 96, alternating phases, one slice at a time
-      // two k-slices per step (K % 128 == 0)
+      // two k-slices per step
       case 13: return launch_tile3<BF16_OUT, 128, 128, 2, 4, 4, 2>(p, s);
       case 14: return launch_tile3<BF16_OUT, 64, 128, 2, 2, 5, 2>(p, s);
       case 15: return launch_tile3<BF16_OUT, 64, 64, 2, 2, 5, 2>(p, s);
       case 16: return launch_tile3<BF16_OUT, 128, 64, 2, 2, 5, 2>(p, s);
       case 17: return launch_tile3<BF16_OUT, 128, 256, 2, 4, 3, 2>(p, s);
       case 19: return launch_tile3<BF16_OUT, 256, 128, 4, 2, 3, 2>(p, s);
-      // one
-      case 3: return launch_tile3<BF16_OUT, 128, 128, 2, 4, 5>(p, s);
-      case 4: return launch_tile3<BF16_OUT, 64, 128, 2, 2, 5>(p, s);
-      case 5: return launch_tile3<BF16_OUT, 64, 64, 2, 2, 5>(p, s);
-      case 6: return launch_tile3<BF16_OUT, 128, 64, 2, 2, 5>(p, s);
-      case 7: return launch_tile3<BF16_OUT, 128, 256, 2, 4, 5>(p, s);
-      case 9: return launch_tile3<BF16_OUT, 256, 128, 4, 2, 5>(p, s);
       default: break;
     }
   }
@@ -1383,7 +1406,7 @@ extern "C" int vaq_fp8_scaled_mm_workspace_tuned(int64_t size_m, int64_t size_n,
     *counter_ints = units;
     return VAQ_OK;
   }
-  if (size_k % 64 != 0 || tuning().fp8_tile_impl != 0 || tuning().fp8_tile_cfg < 0) return VAQ_OK;
+  if (tuning().fp8_tile_impl != 0 || tuning().fp8_tile_cfg < 0) return VAQ_OK;
   const TilePlan pl = plan_tile3((int)size_m, (int)size_n, (int)size_k);
   *c_tmp_bytes = (size_t)pl.tmp_bytes();
   *counter_ints = (size_t)pl.counter_ints();
