@@ -86,8 +86,8 @@ int vaq_w4a16_repack_awq(const int32_t* qweight, int32_t* out, int64_t size_k, i
 
 /*
  * Scratch the caller must hand to vaq_w4a16_gemm for a given problem, in bytes:
- *   *c_tmp_bytes   fp32 split-K partials   (reference: c_tmp, gptq_marlin.cu:752-763)
- *   *a_tmp_bytes   permuted activations    (reference: a_tmp, gptq_marlin.cu:799); 0 when has_perm == 0
+ *   *c_tmp_bytes   fp32 split-K partials   (reference: c_tmp, gptq_marlin.cu:752-763), then permuted activations up to 32 rows
+ *   *a_tmp_bytes   permuted activations    (reference: a_tmp, gptq_marlin.cu:799); 0 when has_perm == 0 or size_m <= 32
  *   *counter_ints  int32 arrival counters that must be ZERO on entry and are left zero
  *                  (reference: `workspace`, marlin_utils.py:237-245, marlin_template.h:225-271)
  */
@@ -119,7 +119,8 @@ int vaq_w4a16_gemm_workspace_of_format(int64_t size_m, int64_t size_n, int64_t s
  * for 4-bit codes in groups of 128 rows or channelwise; workgroups of 16 rows each up to M = 256; from 17 rows on whichever
  * of these and the tile kernels is predicted to be fastest) = MFMA GEMV with in-register dequant; prefill = tile kernels,
  * weights dequantised through LDS or in registers.  `force_path` = 0 auto, 1 decode (M <= 64 at most), 2 prefill (tests /
- * benchmarks).
+ * benchmarks).  act_order: a launch of its own permutes the columns, beyond 32 rows into `a_tmp`, up to 32 where that is predicted to
+ * be ahead into the end of `c_tmp`, and a call that brings less `c_tmp` than the workspace query says gathers inside the decode kernel.
  * Scratch: `c_tmp` holds at least `c_tmp_bytes` bytes and `counters` at least `counter_ints` zeroed ints; a call whose
  * kernel needs more than it was given returns VAQ_ERR_INVALID_ARG (sizes: vaq_w4a16_gemm_workspace, or
  * vaq_w4a16_gemm_workspace_of_format) and launches nothing.

@@ -1,0 +1,94 @@
+"""act_order on the kernels that run on columns permuted ahead of them, and on those that gather: same numbers either way."""
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+from oracle import w4a16 as o
+from tests.helpers import W4A16Layer
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(k, n, g, bits, asym, device):
+    """Scales of one power of two, activations of small integers: every product and every sum in float32 is exact, so each route has to give the
+    same bits."""
+    case = o.make_w4a16_case(k, n, g, asym=asym, act_order=True, seed=k + n, **({"num_bits": 8} if bits == 8 else {}))
+    case["scales"] = torch.full_like(case["scales"], 2.0 ** -8)
+    return W4A16Layer(case, device, torch.float16)
+
+
+def _x(m, k, device, stride=0):
+    wide = torch.full((m, k + stride), float("nan"), dtype=torch.float16, device=device)
+    wide[:, :k] = torch.randint(-2, 3, (m, k), generator=torch.Generator().manual_seed(m * k)).to(torch.float16).to(device)
+    return wide[:, :k]
+
+
+def _sorted_call(layer, x):
+    empty = torch.empty(0, dtype=torch.int32, device=x.device)
+    return layer.ops.gptq_marlin_gemm(x[:, layer.sort_idx.long()].contiguous(), None, layer.w, None, layer.scales, None, layer.zp, empty, empty,
+                                      layer.workspace, layer.wtype, x.shape[0], layer.n, layer.k, is_k_full=True, use_fp32_reduce=True)
+
+
+@pytest.mark.parametrize("k,n,g,bits,asym", [(4096, 4096, 128, 4, False), (2048, 2112, 64, 4, True), (1664, 1152, 32, 4, False), (7040, 1024, 128, 4, True),
+                                             (2560, 2560, 64, 8, False), (4992, 320, 128, 8, False), (1024, 9280, 128, 4, False), (256, 64, 128, 4, False)])
+def test_permuted_ahead_equals_gathered_equals_sorted(device, k, n, g, bits, asym):
+    from vllm_amd import _tuning
+    layer = _layer(k, n, g, bits, asym, device)
+    for m in (1, 2, 4, 5, 8, 16, 17, 31, 32, 33, 48, 64, 65, 128, 200, 256, 257):
+        x = _x(m, k, device, 8 * (m % 2))
+        out = layer(x)
+        with _tuning.override(exp=[0] * 9 + [1]):
+            gathered = layer(x)
+        assert torch.equal(out, gathered) and torch.equal(out, _sorted_call(layer, x)), (m, k, n)
+    assert bool((layer.workspace == 0).all())
+
+
+def _c_call(lib, _lib, layer, x, c_tmp, a_tmp, counters):
+    out = torch.empty((x.shape[0], layer.n), dtype=x.dtype, device=x.device)
+    ptr = lambda t: None if t is None or t.numel() == 0 else ctypes.c_void_p(t.data_ptr())
+    rc = lib.vaq_w4a16_gemm(ptr(x), x.stride(0), ptr(layer.w), ptr(layer.scales), None, ptr(layer.sort_idx), None, ptr(out), ptr(c_tmp),
+                            0 if c_tmp is None else c_tmp.numel() * 4, ptr(a_tmp), ptr(counters), 0 if counters is None else counters.numel(), x.shape[0],
+                            layer.n, layer.k, layer.g, _lib.VAQ_F16, _lib.VAQ_WTYPE_U4B8, 0, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    return rc, out
+
+
+@pytest.mark.parametrize("m", [8, 16, 32])
+def test_callers_without_room_for_permuted_columns(device, m):
+    """Up to 32 rows the gather inside the kernel is left for a caller whose scratch has no room for the columns, down to what that kernel
+    itself needs; what is written behind the scratch would show."""
+    from vllm_amd import _lib
+    lib = _lib.load()
+    layer = _layer(4096, 4096, 128, 4, False, device)
+    x = _x(m, 4096, device)
+    want = layer(x)
+    sizes = [ctypes.c_size_t() for _ in range(3)]
+    _lib.check(lib.vaq_w4a16_gemm_workspace_of_format(m, layer.n, layer.k, layer.g, _lib.VAQ_WTYPE_U4B8, 1, 0, *map(ctypes.byref, sizes)))
+    asked = sizes[0].value // 4
+    assert sizes[0].value >= 2 * m * layer.k and sizes[1].value == 0
+    counters = torch.zeros(max(sizes[2].value, 1), dtype=torch.int32, device=device)
+    for ints in (asked, asked + 1, asked - 1, asked // 2):
+        buf = torch.full((ints + 64,), 7.0, dtype=torch.float32, device=device)
+        rc, out = _c_call(lib, _lib, layer, x, buf[:ints], None, counters)
+        assert rc == (_lib.VAQ_OK if ints >= asked else rc) and (rc != _lib.VAQ_OK or torch.equal(out, want)), ints
+        assert bool((buf[ints:] == 7.0).all()) and bool((counters == 0).all())
+    rc, out = _c_call(lib, _lib, layer, x, None, None, counters)
+    assert rc in (_lib.VAQ_OK, _lib.VAQ_ERR_INVALID_ARG) and (rc != _lib.VAQ_OK or torch.equal(out, want))
+
+
+def test_replayed_graph(device):
+    layer = _layer(4096, 4096, 128, 4, False, device)
+    x = _x(16, 4096, device)
+    layer(x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = layer(x)
+    for seed in range(4):
+        x.copy_(torch.randint(-2, 3, x.shape, generator=torch.Generator().manual_seed(seed)).to(x.dtype))
+        want = layer(x)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), seed

@@ -44,7 +44,8 @@ typedef struct VaqTuning {
                         /*   per wavefront, 9 = off); [10] = 1 both tile kernels: never split only the tiles of a half-empty last round; */
                         /*   [12] = 1 FP8 tile kernel: every tile starts at the first K step; [13] = 1 FP8 tile kernel: no tile  */
                         /*   row past M; [14] > 0 W4A16 tile kernel: KiB that the partial tiles of a K split may take; [6] > 1 both tile     */
-                        /*   kernels, 256 x 256 tiles: the tiles of the last round in this many parts of K; [9], [11] unused;            */
+                        /*   kernels, 256 x 256 tiles: the tiles of the last round in this many parts of K; [9] = 1 act_order: columns */
+                        /*   permuted by a launch of its own for the W4A16 tile kernel only; [11] unused;                             */
                         /*   [8] W4A16 kernel with activations in registers: 1 never, else its plan, n-tiles | m-blocks << 4 |        */
                         /*   wavefronts << 8 | parts of K << 12;                                                                     */
                         /*   [7] = 1 LDS-staged decode kernel: n-tiles in launch order, not grouped by XCD             */

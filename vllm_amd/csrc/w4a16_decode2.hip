@@ -414,12 +414,12 @@ static int dispatch_mr2(const Decode2Params& p, const Decode2Config& c, bool bf1
 }
 
 // Which kernel takes more than 16 rows: workgroups of all rows (`wg_ok`: built for this case), of 16 rows each, or the tile
-// kernel (`tile_ok`, predicted to take `tile_us`).  No act_order and no FP8 weights among the workgroups of 16 rows.
+// kernel (`tile_ok`, predicted to take `tile_us`).  No act_order inside (`has_perm`) and no FP8 weights among the workgroups of 16 rows.
 // 17 .. 32 rows of 4-bit codes in groups of 128 rows / channelwise: 16 rows each where one m-block needs no split of K and one
 // round of workgroups of at least eight wavefronts takes them all; 4096 x 4096 at M = 32 8.5 -> 6.3 us; a 28672-wide layer would
 // need streams of 32 tiles (20.4 -> 21.7 us).  Everything else by predicted time.
 // (development switch exp[2]: 1 never 16 rows each, 2 wherever it is built)
-int w4a16_decode2_choose(int M, int N, int K, int sub, int wt, bool has_perm, bool wg_ok, bool tile_ok, double tile_us) {
+int w4a16_decode2_choose(int M, int N, int K, int sub, int wt, bool act_order, bool has_perm, bool wg_ok, bool tile_ok, double tile_us) {
   const bool w8 = wt != 0, rows_ok = M > 16 && M <= DECODE2_MAX_M_ROWS && wt != 2 && !has_perm && tuning().exp[2] != 1;
   if (!rows_ok && !tile_ok) return D2_WORKGROUP;
   Decode2Plan r;
@@ -434,12 +434,12 @@ int w4a16_decode2_choose(int M, int N, int K, int sub, int wt, bool has_perm, bo
   // 9-13 % with 8-bit codes; the prices of these workgroups are 3-9 % low.  With these factors the kind chosen is, against those shapes,
   // within 0.2 - 0.6 % of the fastest one's time in the mean, 1.3 % for groups of 64 / 32 rows at 17 .. 32 rows; 6600 problems.  The strips
   // that run in their place are up to 40 % faster; they take no problem from here because they round the scaled weights to 16 bits.
-  // act_order: a launch that permutes the columns first, at the 4 us that it took before it had few rows spread over the device (2 - 3
-  // now), for the same reason.)
-  double us = tile_ok ? tile_us * (!w8 ? 1.04 : M <= 64 ? 1.06 : 1.0) + (has_perm ? 4.0 : 0.0) : -1;
+  // act_order: workgroups of all rows, with float32 scales, keep what they were given when the columns were always gathered inside them
+  // and the tile kernel's launch for it was priced at 4 us.)
+  double us = tile_ok ? tile_us * (!w8 ? 1.04 : M <= 64 ? 1.06 : 1.0) : -1;
   if (wg_ok) {
     const double t = workgroup_plan(M, N, K, sub, w8).us;
-    if (us < 0 || t < us) { us = t; best = D2_WORKGROUP; }
+    if (us < 0 || t < us + (act_order ? 4.0 : 0.0)) { us = t; best = D2_WORKGROUP; }
   }
   if (r.us >= 0 && (us < 0 || r.us < us)) best = D2_ROWS;
   return best;
@@ -473,6 +473,15 @@ namespace vaq {
 
 double w4a16_decode2_us(int M, int N, int K, int sub, bool w8, bool rows) {
   return (rows ? rows_plan(M, N, K, sub, w8) : workgroup_plan(M, N, K, sub, w8)).us;
+}
+
+// The same of a call of up to 32 rows with act_order, and what of it is the gather: two dependent loads and, for every 1000 elements that a compute unit's
+// workgroups gather, 0.16 us (1077 timings, 18 % rms, 6 % low).
+double w4a16_decode2_gather_us(int M, int N, int K, int sub, bool w8, double* gather) {
+  const Decode2Plan p = workgroup_plan(M, N, K, sub, w8);
+  const double wgs = (double)((N / 16 + p.c.wn - 1) / p.c.wn) * p.c.sk / num_cus_current_device();
+  *gather = 0.6 + 0.159e-3 * M * 128 * p.c.gs * p.c.wks * fmax(1.0, wgs);
+  return p.us + *gather;
 }
 
 int w4a16_decode2_workspace(int M, int N, int K, int sub, bool w8, size_t* c_tmp_bytes, size_t* counter_ints) {

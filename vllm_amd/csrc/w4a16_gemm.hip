@@ -58,7 +58,7 @@ static int other_kind(int M, int N, int K, int sub, int wt, double* us) {
   }
   if (M > 16) {
     const int most = !plain ? DECODE_MAX_M_2BLK : N > 8192 ? 48 : DECODE_MAX_M;
-    kind = w4a16_decode2_choose(M, N, K, sub, wt, false, M <= most, true, w4a16_staged_us(M, N, K, plain));
+    kind = w4a16_decode2_choose(M, N, K, sub, wt, false, false, M <= most, true, w4a16_staged_us(M, N, K, plain));
   }
   *us = kind == D2_TILE ? w4a16_tile_us(M, N, K, tile_format(sub, wt)) : w4a16_decode2_us(M, N, K, sub, w8, kind == D2_ROWS);
   return kind;
@@ -103,17 +103,41 @@ bool w4a16_takes_regs(int M, int N, int K, int sub, int wt, double* other) {
   return us < *other * regs_lead(M, N, K, sub, wt, j, nw);
 }
 
+// Whether a switch names a kernel or a plan of one.
+static bool plan_named(const VaqTuning& tn) {
+  return tn.decode_impl > 0 || tn.decode2_gs > 0 || tn.decode2_wks > 0 || tn.decode2_wn > 0 || tn.prefill_tile > 0 || tn.prefill_split > 0 ||
+         tn.exp[0] > 0 || tn.exp[1] > 0 || tn.exp[2] > 0 || tn.exp[3] > 0 || tn.exp[5] > 0 || tn.exp[6] > 0;
+}
+
 // The same for a call, from a table per thread.  A switch that names another kernel or a plan of one keeps it out; exp[8] asks for it.
 static bool regs_chosen(int M, int N, int K, int sub, int wt) {
   const VaqTuning& tn = tuning();
   if (M < 1 || M > REGS_MAX_M || N >= (1 << 24) || K >= (1 << 24) || tn.exp[8] == 1) return false;
   if (tn.exp[8] > 1) return w4a16_regs_us(M, N, K, sub, wt) >= 0;
-  if (tn.decode_impl > 0 || tn.decode2_gs > 0 || tn.decode2_wks > 0 || tn.decode2_wn > 0 || tn.prefill_tile > 0 || tn.prefill_split > 0 ||
-      tn.exp[0] > 0 || tn.exp[1] > 0 || tn.exp[2] > 0 || tn.exp[3] > 0 || tn.exp[5] > 0 || tn.exp[6] > 0)
-    return false;
+  if (plan_named(tn)) return false;
   static thread_local PlanTable<int> table;
   double other;
   return table.get(M, N, K, (num_cus_current_device() * 8 + sub) * 4 + wt, [&] { return w4a16_takes_regs(M, N, K, sub, wt, &other) ? 1 : 0; }) != 0;
+}
+
+// Whether act_order's columns are permuted by a launch of their own ahead of the kernels with activations in registers and the decode kernels too,
+// which then run as without act_order (the gather inside the decode kernel is two dependent loads per element, in every workgroup, and the kernel with
+// activations in registers has none).  Beyond 32 rows always: 4096 x 4096 at M = 48 / 64 20.4 / 25.3 -> 9.7 / 10.2 us, 14336 x 4096 50 / 64 -> 21.1 / 21.8.
+// Up to there where the gather is priced above 2 us (the launch takes 2.4 from one to the other) and the call above 8.6, which is what the host needs
+// for a call of two launches (5.5 for one).  Over 1077 calls of drawn act_order layers of 1 .. 32 rows the 773 it takes run in 0.57 of their time in
+// the mean, none slower; of the others 94 would gain more than a tenth replayed from a graph, 28 called.  4096 x 4096 at M = 8 / 16 / 32 12.5 / 20.7 / 23.2 -> 7.1 /
+// 7.7 / 8.2 us, 14336 x 4096 at M = 1 / 16 12.1 / 39.3 -> 10.7 / 14.8, 9088 x 2560 in 8-bit codes at M = 16 31.3 -> 12.4; left as they are 4096 x 28672 at
+// M = 1 13.6 (15.4), 2048 x 2048 at M = 4 5.7 (6.1) and 4096 x 4096 at M = 4 8.6 (6.6, and 8.5 for the host).  3 .. 16 rows of a vocabulary-sized layer, always: 4096 x 128256 at M = 4 61.1 -> 46.4 us.
+static bool permutes_first(int M, int N, int K, int sub, bool w8) {
+  const VaqTuning& tn = tuning();
+  if (M < 1 || N >= (1 << 24) || K >= (1 << 24) || tn.exp[9] == 1 || plan_named(tn)) return false;
+  if (M > DECODE_MAX_M_2BLK || decode_impl_for(M, N, K, sub, w8) == 1) return true;
+  static thread_local PlanTable<int> table;
+  return table.get(M, N, K, num_cus_current_device() * 8 + sub + (w8 ? 1 << 16 : 0), [&] {
+    double gather = 0;
+    const double us = w4a16_decode2_gather_us(M, N, K, sub, w8, &gather);
+    return gather > 2.0 && us > 8.6 ? 1 : 0;
+  }) != 0;
 }
 
 // Scratch of a problem, enough for whichever kernel runs (that also depends on the row stride of A): for one weight format, or with
@@ -152,14 +176,82 @@ static int scratch_of(int64_t size_m, int64_t size_n, int64_t size_k, bool has_p
       if (rc != VAQ_OK) return rc;
       take(t, n);
     }
+  size_t columns = 0;      // act_order: room for the permuted columns, behind the partial tiles up to 32 rows
   for (int s : {1, 2, 4})
     for (int w : {0, 1}) {
-      if (has_perm || (wt >= 0 && (s != sub || w != wt)) || size_m > REGS_MAX_M || !regs_chosen(M, N, K, s, w)) continue;
+      if (size_m == 0 || (wt >= 0 && (s != sub || w != wt)) || (has_perm && !permutes_first(M, N, K, s, w == 1))) continue;
+      if (has_perm && size_m <= DECODE_MAX_M_2BLK) columns = (size_t)size_m * (size_t)size_k * 2;
+      if (size_m > REGS_MAX_M || !regs_chosen(M, N, K, s, w)) continue;
       w4a16_regs_workspace(M, N, K, s, w == 1, &t, &n);
       take(t, n);
     }
+  if (columns) *c_tmp_bytes = ((*c_tmp_bytes + 15) & ~(size_t)15) + columns;
   if (has_perm && size_m > DECODE_MAX_M_2BLK) *a_tmp_bytes = (size_t)size_m * (size_t)size_k * 2;
   return VAQ_OK;
+}
+
+// A checked call on the kernel that takes it.  `act_order` with `perm` null: the columns of A have been permuted.
+static int dispatch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros, const int32_t* perm, bool act_order,
+                    const void* bias, void* c, float* c_tmp, int64_t c_tmp_bytes, void* a_tmp, int32_t* counters, int64_t counter_ints,
+                    int64_t size_m, int64_t size_n, int64_t size_k, int sub, bool channelwise, int wt, int dtype, int force_path, hipStream_t s) {
+  const bool w8 = wt != 0;
+  // The kernel with operands in registers first: a call that it takes looks up none of the other plans.  (One that brings too little scratch for its parts of K
+  // goes on to the others; so does one whose rows end beyond 2 GiB.)
+  if (force_path == 0 && perm == nullptr && size_m <= REGS_MAX_M && size_m * lda * 2 < (1ll << 31) &&
+      regs_chosen((int)size_m, (int)size_n, (int)size_k, sub, wt)) {
+    size_t t = 0, n = 0;
+    w4a16_regs_workspace((int)size_m, (int)size_n, (int)size_k, sub, w8, &t, &n);
+    if ((t == 0 && n == 0) || (c_tmp != nullptr && counters != nullptr && (uintptr_t)c_tmp % 16 == 0 && c_tmp_bytes >= (int64_t)t && counter_ints >= (int64_t)n))
+      return w4a16_regs_launch(a, lda, b, scales, zeros, bias, c, c_tmp, counters, (int)size_m, (int)size_n, (int)size_k, sub, channelwise,
+                               w8, dtype, s);
+  }
+
+  // three and four m-blocks exist on the LDS-staged kernel for 4-bit codes in groups of 128 rows / channelwise
+  const bool two_blocks_only = sub > 1 || w8 || decode_impl_for(size_m, size_n, lda, sub, w8) != 0;
+  // (measured: four m-blocks beat the tile kernel by 1.5-2x on the narrow layers and lose 3 % on a 28672-wide one)
+  const int64_t dec_max = two_blocks_only ? DECODE_MAX_M_2BLK : (size_n > 8192 ? 48 : DECODE_MAX_M);
+  bool decode = size_m <= dec_max, rows = false;
+  VAQ_CHECK_ARG(force_path != 1 || decode, "w4a16_gemm: decode path forced with size_m = %lld > %lld", (long long)size_m,
+                (long long)dec_max);
+  if (force_path == 2) {
+    decode = false;
+  } else if (size_m > 16 && size_m <= 256 && size_n < (1 << 24) && size_k < (1 << 24) &&
+             decode_impl_for(size_m, size_n, lda, sub, w8) == 0) {
+    // 17 .. 256 rows: the decode kernel's workgroups of all rows or of 16 rows each, or the tile kernel (where it is given the
+    // scratch that its plan asks for; up to 32 rows that need not be so, and act_order stays with the decode kernel)
+    bool tile_ok = force_path == 0;
+    if (tile_ok && size_m <= DECODE_MAX_M_2BLK) {
+      size_t t = 0, n = 0;
+      w4a16_prefill_workspace((int)size_m, (int)size_n, (int)size_k, tile_format(sub, wt), &t, &n);
+      tile_ok = !act_order && c_tmp_bytes >= (int64_t)t && counter_ints >= (int64_t)n;
+    }
+    const int kind = w4a16_decode2_choose((int)size_m, (int)size_n, (int)size_k, sub, wt, act_order, perm != nullptr, decode, tile_ok || !decode,
+                                          w4a16_staged_us((int)size_m, (int)size_n, (int)size_k, !w8 && sub == 1));
+    decode = kind != D2_TILE;
+    rows = kind == D2_ROWS;
+  }
+  if (decode && decode_impl_for(size_m, size_n, lda, sub, w8) == 0)
+    return w4a16_decode2_launch(a, lda, b, scales, zeros, perm, bias, c, c_tmp, c_tmp_bytes, counters, counter_ints, (int)size_m,
+                                (int)size_n, (int)size_k, sub, channelwise, wt, dtype, rows, s);
+  if (decode) {
+    VAQ_CHECK_SUPPORTED(sub == 1 && !w8, "w4a16_gemm: group_size = %d / 8-bit weights with an A of 2 GiB or more are not built",
+                        channelwise ? -1 : 128 / sub);
+    return w4a16_decode_launch(a, lda, b, scales, zeros, perm, bias, c, c_tmp, c_tmp_bytes, counters, counter_ints, (int)size_m,
+                               (int)size_n, (int)size_k, channelwise, dtype, s);
+  }
+
+  const void* a_eff = a;
+  int64_t lda_eff = lda;
+  if (perm) {
+    VAQ_CHECK_ARG(a_tmp != nullptr, "w4a16_gemm: act_order on the prefill path needs a_tmp [size_m, size_k]");
+    VAQ_CHECK_ARG(((uintptr_t)a_tmp % 16) == 0, "w4a16_gemm: a_tmp must be 16-byte aligned");
+    const int rc = vaq_permute_cols(a, lda, perm, a_tmp, size_m, size_k, s);
+    if (rc != VAQ_OK) return rc;
+    a_eff = a_tmp;
+    lda_eff = size_k;
+  }
+  return w4a16_prefill_launch(a_eff, lda_eff, b, scales, zeros, bias, c, c_tmp, c_tmp_bytes, counters, counter_ints, (int)size_m,
+                              (int)size_n, (int)size_k, sub, channelwise, wt, dtype, s);
 }
 }  // namespace vaq
 
@@ -233,63 +325,24 @@ extern "C" int vaq_w4a16_gemm_tuned(const void* a, int64_t lda, const int32_t* b
   VAQ_CHECK_ARG(!bias || ((uintptr_t)bias % 8) == 0, "w4a16_gemm: bias must be 8-byte aligned");
   hipStream_t s = (hipStream_t)stream;
 
-  // The kernel with operands in registers first: a call that it takes looks up none of the other plans.  (One that brings too little scratch for its parts of K
-  // goes on to the others; so does one whose rows end beyond 2 GiB.)
-  if (force_path == 0 && perm == nullptr && size_m <= REGS_MAX_M && size_m * lda * 2 < (1ll << 31) &&
-      regs_chosen((int)size_m, (int)size_n, (int)size_k, sub, wt)) {
-    size_t t = 0, n = 0;
-    w4a16_regs_workspace((int)size_m, (int)size_n, (int)size_k, sub, w8, &t, &n);
-    if ((t == 0 && n == 0) || (c_tmp != nullptr && counters != nullptr && (uintptr_t)c_tmp % 16 == 0 && c_tmp_bytes >= (int64_t)t && counter_ints >= (int64_t)n))
-      return w4a16_regs_launch(a, lda, b, scales, zeros, bias, c, c_tmp, counters, (int)size_m, (int)size_n, (int)size_k, sub, channelwise,
-                               w8, dtype, s);
-  }
-
-  // three and four m-blocks exist on the LDS-staged kernel for 4-bit codes in groups of 128 rows / channelwise
-  const bool two_blocks_only = sub > 1 || w8 || decode_impl_for(size_m, size_n, lda, sub, w8) != 0;
-  // (measured: four m-blocks beat the tile kernel by 1.5-2x on the narrow layers and lose 3 % on a 28672-wide one)
-  const int64_t dec_max = two_blocks_only ? DECODE_MAX_M_2BLK : (size_n > 8192 ? 48 : DECODE_MAX_M);
-  bool decode = size_m <= dec_max, rows = false;
-  VAQ_CHECK_ARG(force_path != 1 || decode, "w4a16_gemm: decode path forced with size_m = %lld > %lld", (long long)size_m,
-                (long long)dec_max);
-  if (force_path == 2) {
-    decode = false;
-  } else if (size_m > 16 && size_m <= 256 && size_n < (1 << 24) && size_k < (1 << 24) &&
-             decode_impl_for(size_m, size_n, lda, sub, w8) == 0) {
-    // 17 .. 256 rows: the decode kernel's workgroups of all rows or of 16 rows each, or the tile kernel (where it is given the
-    // scratch that its plan asks for; up to 32 rows that need not be so, and act_order stays with the decode kernel)
-    bool tile_ok = force_path == 0;
-    if (tile_ok && size_m <= DECODE_MAX_M_2BLK) {
-      size_t t = 0, n = 0;
-      w4a16_prefill_workspace((int)size_m, (int)size_n, (int)size_k, tile_format(sub, wt), &t, &n);
-      tile_ok = perm == nullptr && c_tmp_bytes >= (int64_t)t && counter_ints >= (int64_t)n;
+  if (perm && force_path == 0 && size_m * lda * 2 < (1ll << 31) && permutes_first((int)size_m, (int)size_n, (int)size_k, sub, w8)) {
+    // into a_tmp beyond 32 rows, and into the end of c_tmp up to there
+    int64_t left = c_tmp_bytes;
+    void* columns = a_tmp;
+    if (size_m <= DECODE_MAX_M_2BLK) {
+      left = (c_tmp_bytes - size_m * size_k * 2) & ~15ll;
+      columns = c_tmp != nullptr && left >= 0 ? reinterpret_cast<char*>(c_tmp) + left : nullptr;
     }
-    const int kind = w4a16_decode2_choose((int)size_m, (int)size_n, (int)size_k, sub, wt, perm != nullptr, decode, tile_ok || !decode,
-                                          w4a16_staged_us((int)size_m, (int)size_n, (int)size_k, !w8 && sub == 1));
-    decode = kind != D2_TILE;
-    rows = kind == D2_ROWS;
+    if (columns != nullptr && ((uintptr_t)columns % 16) == 0) {
+      rc = vaq_permute_cols(a, lda, perm, columns, size_m, size_k, stream);
+      if (rc != VAQ_OK) return rc;
+      rc = dispatch(columns, size_k, b, scales, zeros, nullptr, true, bias, c, left > 0 ? c_tmp : nullptr, left, a_tmp, counters, counter_ints, size_m, size_n,
+                    size_k, sub, channelwise, wt, dtype, 0, s);
+      if (rc != VAQ_ERR_INVALID_ARG) return rc;      // (given too little scratch for that plan: as without it)
+    }
   }
-  if (decode && decode_impl_for(size_m, size_n, lda, sub, w8) == 0)
-    return w4a16_decode2_launch(a, lda, b, scales, zeros, perm, bias, c, c_tmp, c_tmp_bytes, counters, counter_ints, (int)size_m,
-                                (int)size_n, (int)size_k, sub, channelwise, wt, dtype, rows, s);
-  if (decode) {
-    VAQ_CHECK_SUPPORTED(sub == 1 && !w8, "w4a16_gemm: group_size = %d / 8-bit weights with an A of 2 GiB or more are not built",
-                        group_size);
-    return w4a16_decode_launch(a, lda, b, scales, zeros, perm, bias, c, c_tmp, c_tmp_bytes, counters, counter_ints, (int)size_m,
-                               (int)size_n, (int)size_k, channelwise, dtype, s);
-  }
-
-  const void* a_eff = a;
-  int64_t lda_eff = lda;
-  if (perm) {
-    VAQ_CHECK_ARG(a_tmp != nullptr, "w4a16_gemm: act_order on the prefill path needs a_tmp [size_m, size_k]");
-    VAQ_CHECK_ARG(((uintptr_t)a_tmp % 16) == 0, "w4a16_gemm: a_tmp must be 16-byte aligned");
-    rc = vaq_permute_cols(a, lda, perm, a_tmp, size_m, size_k, stream);
-    if (rc != VAQ_OK) return rc;
-    a_eff = a_tmp;
-    lda_eff = size_k;
-  }
-  return w4a16_prefill_launch(a_eff, lda_eff, b, scales, zeros, bias, c, c_tmp, c_tmp_bytes, counters, counter_ints, (int)size_m,
-                              (int)size_n, (int)size_k, sub, channelwise, wt, dtype, s);
+  return dispatch(a, lda, b, scales, zeros, perm, perm != nullptr, bias, c, c_tmp, c_tmp_bytes, a_tmp, counters, counter_ints, size_m, size_n, size_k,
+                  sub, channelwise, wt, dtype, force_path, s);
 }
 
 // ----------------------------------------------------------------------------- the GEMM on library-owned scratch
@@ -347,6 +400,12 @@ extern "C" int vaq_w4a16_gemm_static(const void* a, int64_t lda, const int32_t* 
   int rc = vaq_w4a16_gemm_workspace_tuned(size_m, size_n, size_k, perm != nullptr, 0, &c_tmp_bytes, &a_tmp_bytes, &counter_ints,
                                           &whole_tiles);
   if (rc != VAQ_OK) return rc;
+  if (perm != nullptr && (counter_ints > STATIC_COUNTER_INTS || ((c_tmp_bytes + 255) & ~(size_t)255) + a_tmp_bytes > STATIC_DATA_BYTES)) {
+    // the routes without the launch that permutes ahead of the decode kernels ask for less
+    whole_tiles.exp[9] = 1;
+    rc = vaq_w4a16_gemm_workspace_tuned(size_m, size_n, size_k, 1, 0, &c_tmp_bytes, &a_tmp_bytes, &counter_ints, &whole_tiles);
+    if (rc != VAQ_OK) return rc;
+  }
   const size_t c_tmp_span = (c_tmp_bytes + 255) & ~(size_t)255;
   VAQ_CHECK_ARG(counter_ints <= STATIC_COUNTER_INTS && c_tmp_span + a_tmp_bytes <= STATIC_DATA_BYTES,
                 "w4a16_gemm_static: M=%lld N=%lld K=%lld needs %zu counters and %zu + %zu bytes of scratch, the "

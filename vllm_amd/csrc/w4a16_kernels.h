@@ -12,7 +12,7 @@ int w4a16_decode_launch(const void* a, int64_t lda, const int32_t* b, const void
 int w4a16_decode2_workspace(int M, int N, int K, int sub, bool w8, size_t* c_tmp_bytes, size_t* counter_ints);
 // Which kernel takes more than 16 rows: the tile kernel, the decode kernel's workgroups of all rows, or of 16 rows each.
 enum { D2_TILE, D2_WORKGROUP, D2_ROWS };
-int w4a16_decode2_choose(int M, int N, int K, int sub, int wt, bool has_perm, bool wg_ok, bool tile_ok, double tile_us);
+int w4a16_decode2_choose(int M, int N, int K, int sub, int wt, bool act_order, bool has_perm, bool wg_ok, bool tile_ok, double tile_us);
 // What the choice of a tile depends on: 4-bit codes in groups of 128 rows / channelwise, in smaller groups, 8-bit codes likewise and in groups
 // of 32, FP8 weights (and plain codes on the shapes with weights through LDS only, to price them).
 enum TileFormat { TILES_PLAIN, TILES_SUB, TILES_8BIT, TILES_8BIT_64, TILES_8BIT_32, TILES_FP8, TILES_PLAIN_STAGED };
@@ -21,6 +21,7 @@ inline TileFormat tile_format(int sub, int wt) {
   return wt == 2 ? TILES_FP8 : sub > 1 ? TILES_SUB : TILES_PLAIN;
 }
 double w4a16_decode2_us(int M, int N, int K, int sub, bool w8, bool rows);      // predicted time of the decode kernel's plan
+double w4a16_decode2_gather_us(int M, int N, int K, int sub, bool w8, double* gather);      // with act_order gathered inside it; `gather`: its share
 double w4a16_staged_us(int M, int N, int K, bool plain);
 double w4a16_tile_us(int M, int N, int K, TileFormat format);
 int w4a16_decode2_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros,
