@@ -64,22 +64,21 @@ static int other_kind(int M, int N, int K, int sub, int wt, double* us) {
   return kind;
 }
 
-// Whether the kernel with activations in registers takes a problem: where it is predicted to be ahead of what takes it otherwise by so much that
-// few calls lose.  4-bit codes in groups of 128 rows 15 % up to 4 rows and 9 % up to 32, where the decode kernel's plans by rule are on some
-// layers that much better than priced (14336 x 4096 at M = 4 9.0 us, priced 9.9; this kernel 10.0, priced 8.7), 5 % up to 64 rows and 8 % beyond;
-// vocabulary-sized layers at 3 .. 16 rows, where another kernel is the alternative, 5 % (it takes them all: 0.37 .. 0.96 of the time, 1 of 2000 more than 3 %
-// slower; 4096 x 128256 at M = 4 / 16 54.9 / 59.0 -> 51.9 / 53.4 us, 1024 x 128256 33.4 / 34.0 -> 18.1 / 19.5, 5120 x 65536 80.0 / 81.0 -> 33.2 / 34.7);
-// in groups of 64 / 32 rows 12 % from 33 rows on, where zero points cost more than priced; 8-bit codes none up to 32 rows (up to 4 rows 17 % behind is
-// still taken); all others 5 %.  The prices are older than the arguments in registers, which gained this kernel more than the others: with 13 % and 5 %
-// in these two places 3 % of 12000 drawn problems of 1 .. 256 rows went elsewhere, for 1.085 of the time in the mean, 8 % of them more than 3 % ahead there.  (Smaller
-// leads for the rest gain less than 0.2 % and lose on a fifth of what they move.)  Over 20254 calls of drawn layers that
-// it took at 5 % where it now asks for 8 and 12, timed both ways afterwards: 0.842 of their time in the mean, 3.9 % more than 3 % slower, 0.5 % more than 10 %.
+// Whether the kernel with activations in registers takes a problem: where its price is below this share of the price of what takes it otherwise.  The
+// prices are older than the arguments in registers and off by as much as the kernels have gained since (this one's 3-5 % low, that of the decode kernel 0-8 % low
+// with 4-bit codes in groups of 128 rows and 3-15 % low with the rest), so the shares are set by the choices, for 1 .. 4, 5 .. 16, 17 .. 32, 33 .. 64 and
+// more rows: over 3575 problems of random layers with both timed now the choice takes 1.009 of the faster one's time in the mean.  The shares before (0.85 up
+// to 4 rows and 0.91 up to 32 for 4-bit codes in groups of 128 rows, 0.95 up to 32 for groups of 64 / 32) took 1.016; of the 300 calls that move 4 % are more
+// than 3 % slower.  Drawn layers: 3712 x 17792 at M = 1 9.8 -> 8.6 us, 9216 x 4416 at M = 4 9.2 -> 8.0, 11520 x 5248 at M = 18 14.0 -> 12.9; 1792 x 11008 at
+// M = 3 4.5 -> 4.9.  From 33 rows on shares nearer to one lose as much as they gain: strips cost less, and zero points in small groups more, than priced (4-bit
+// codes in groups of 32 with zero points at M = 34 13.7 -> 15.7).
 static double regs_lead(int M, int N, int K, int sub, int wt, int j, int nw) {
+  constexpr double SHARE[4][5] = {{0.95, 0.96, 0.97, 0.95, 0.92}, {1.05, 1.0, 1.0, 0.88, 0.88}, {1.05, 1.0, 0.95, 0.88, 0.88}, {1.17, 1.01, 1.01, 0.95, 0.95}};
+  // vocabulary-sized layers at 3 .. 16 rows, where another kernel is the alternative (it takes them all: 0.37 .. 0.96 of the time, 1 of 2000 more than 3 % slower;
+  // 4096 x 128256 at M = 4 / 16 54.9 / 59.0 -> 51.9 / 53.4 us, 1024 x 128256 33.4 / 34.0 -> 18.1 / 19.5, 5120 x 65536 80.0 / 81.0 -> 33.2 / 34.7)
   if (wt == 0 && decode_impl_for(M, N, K, sub, false) == 1) return 0.95;
-  if (wt != 0) return M <= 4 ? 1.17 : M <= 32 ? 1.01 : 0.95;
-  if (sub > 1) return M > 32 ? 0.88 : 0.95;
-  if (M > 32) return M <= 64 ? 0.95 : 0.92;
-  const double lead = M <= 4 ? 0.85 : 0.91;
+  const double lead = SHARE[wt != 0 ? 3 : sub == 1 ? 0 : sub == 2 ? 1 : 2][M <= 4 ? 0 : M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 3 : 4];
+  if (wt != 0 || sub > 1 || M > 32) return lead;
   // Where this kernel loses most of what it loses, by as much as the two prices together are off by: K of whole 1024 rows; one n-tile to a wavefront and K
   // beyond 8192 at up to 4 rows; two and more n-tiles on a short K.  Off are: this kernel's price, which counts 16 rows to a block, by the rows that a block has;
   // for workgroups of four; for one n-tile, which leaves 2 KB of weights in flight, by how much of the device waits for them and how long; for three and more
