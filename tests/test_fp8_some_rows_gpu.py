@@ -1,0 +1,67 @@
+"""The FP8 kernel for some dozen rows, against exact sums: every launch shape, remainders of rows, columns and K, and the calls that go to it."""
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(m, n, k, seed, device, gap=0):
+    """Small integers as e4m3 (every product and sum exact), rows `gap` bytes further apart than K with NaN codes between them."""
+    g = torch.Generator().manual_seed(seed)
+    a, w = torch.randint(-2, 3, (m, k), generator=g).float(), torch.randint(-1, 2, (n, k), generator=g).float()
+    views = []
+    for x in (a, w):
+        wide = torch.full((x.shape[0], k + gap), 0x7f, dtype=torch.uint8, device=device).view(torch.float8_e4m3fn)
+        wide[:, :k] = x.to(torch.float8_e4m3fn).to(device)
+        views.append(wide[:, :k])
+    return views[0], views[1].t(), a @ w.t()
+
+
+def _run(a, b, device, dtype=torch.float16, sa=None, sb=None, bias=None):
+    import vllm_amd._custom_ops as ops
+    m, n = a.shape[0], b.shape[1]
+    return ops.cutlass_scaled_mm(a, b, torch.ones(m, 1, device=device) if sa is None else sa, torch.ones(n, 1, device=device) if sb is None else sb, dtype, bias)
+
+
+@pytest.mark.parametrize("mb", [1, 2, 3, 4])
+@pytest.mark.parametrize("j", [1, 2, 3, 4])
+def test_every_launch_shape_exact(device, mb, j):
+    """From a K of half a step (most wavefronts without one) to several turns of the ring with half a step at the end; one row, ragged last blocks of rows and of
+    n-tiles, several blocks of rows.  (Shapes that do not fit LDS are not built: such a switch changes nothing.)"""
+    from vllm_amd import _tuning
+    for k in (128, 256, 384, 896, 1024, 1152, 2048, 2176, 5248):
+        m, n = 1 + (k * 7 + mb * 37) % 200, 16 * (1 + (k // 128 * 5 + j * 11) % 37)
+        a, b, want = _case(m, n, k, k + mb, device, gap=64 if k % 256 else 0)
+        with _tuning.override(exp=[0] * 11 + [j | mb << 4]):
+            assert torch.equal(_run(a, b, device).cpu().float(), want), (m, n, k)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("per_row,per_col,bias", [(True, True, True), (False, False, False), (True, False, True), (False, True, False)])
+def test_scales_and_bias_as_the_tile_kernel(device, dtype, per_row, per_col, bias):
+    """Exact sums: the scales, the bias and the roundings between them decide every bit, and are those of the tile kernel."""
+    from vllm_amd import _tuning
+    g = torch.Generator().manual_seed(5)
+    m, n, k = 61, 208, 640
+    a, b, _ = _case(m, n, k, 3, device)
+    sa, sb = torch.rand(m if per_row else 1, 1, generator=g).to(device), torch.rand(n if per_col else 1, 1, generator=g).to(device)
+    bb = torch.randn(n, generator=g).to(dtype).to(device) if bias else None
+    with _tuning.override(fp8_path=2):
+        want = _run(a, b, device, dtype, sa, sb, bb)
+    with _tuning.override(exp=[0] * 11 + [3 | 2 << 4]):
+        assert torch.equal(_run(a, b, device, dtype, sa, sb, bb), want)
+
+
+@pytest.mark.parametrize("m,n,k", [(16, 4096, 14336), (17, 1024, 1024), (32, 4096, 4096), (33, 2048, 2048), (64, 1280, 2560), (64, 4096, 4096), (100, 1024, 4096), (128, 2048, 2048),
+                                   (200, 1024, 1024), (256, 1024, 4096)])
+def test_as_chosen_exact(device, m, n, k):
+    from vllm_amd import _lib
+    plan = (ctypes.c_double * 5)()
+    _lib.check(_lib.load().vaq_fp8_regs_plan(m, n, k, plan))
+    assert plan[4] == 1
+    a, b, want = _case(m, n, k, k, device)
+    assert torch.equal(_run(a, b, device).cpu().float(), want)

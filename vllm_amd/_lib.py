@@ -56,6 +56,7 @@ _SIGNATURES = {
                                      c_int64, c_void_p]),
     "vaq_w4a16_decode_plan": (c_int, [c_int64, c_int64, c_int64, c_int, c_int, c_int, POINTER(ctypes.c_double)]),
     "vaq_w4a16_regs_plan": (c_int, [c_int64, c_int64, c_int64, c_int, c_int, POINTER(ctypes.c_double)]),
+    "vaq_fp8_regs_plan": (c_int, [c_int64, c_int64, c_int64, POINTER(ctypes.c_double)]),
     "vaq_w4a16_tile_plan": (c_int, [c_int64, c_int64, c_int64, c_int, c_int, c_int, POINTER(ctypes.c_double)]),
     "vaq_fp8_quant_scaled_mm_takes": (c_int, [c_int64, c_int64, c_int64, c_int]),
     "vaq_fp8_quant_scaled_mm": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p,

@@ -10,12 +10,15 @@
 //    (pitch 144 B), takes what the multi-stage kernel cannot address;
 //  * stream kernels (M <= 32; M <= 64 on narrow layers with K <= 4096): weight-streaming GEMV-like, weights are the A operand
 //    of v_mfma_f32_16x16x128_f8f6f4, activations stay in registers, the wavefronts of a workgroup split K and reduce
-//    through LDS; fp8_mm_stream2_kernel (fp8_stream2_kernel.h) brings the weights in through LDS as whole cache lines.
+//    through LDS; fp8_mm_stream2_kernel (fp8_stream2_kernel.h) brings the weights in through LDS as whole cache lines;
+//  * fp8_mm_regs_kernel (fp8_regs_kernel.h; 5 .. 256 rows, K a multiple of 128, where predicted ahead of the others): both operands as
+//    whole lines through LDS that no other wavefront touches, several n-tiles and m-blocks a wavefront.
 //
 // The per-lane byte -> k assignment inside an MFMA operand is the same function for A and B, so any consistent choice
-// of which 32 bytes a lane supplies yields the exact dot product; both kernels give lane (row, q) the bytes
-// k0 + 32*q .. k0 + 32*q + 31 of its row.
+// of which 32 bytes a lane supplies yields the exact dot product; the tile and stream kernels give lane (row, q) the
+// bytes k0 + 32*q .. k0 + 32*q + 31 of its row.
 #include "vaq_common.h"
+#include "fp8_regs_kernel.h"
 #include "fp8_stream2_kernel.h"
 #include "tile_handover.h"
 #include "tile_plan.h"
@@ -1381,7 +1384,62 @@ static bool dispatch_stream(const Fp8MMParams& p, hipStream_t s) {
   return true;
 }
 
+// Whether the kernel of fp8_regs_kernel.h takes a problem (K a multiple of 128): where its price is 7 % below that of the tile plan, or 3 % below that of the stream
+// kernel with weights through LDS -- its rows' activations, its n-tiles in rounds of one to a compute unit, the weights from memory; fitted to 291 of the
+// timings below, 7 % rms.  (33 .. 64 rows where the other stream kernel was ahead of the tiles: 20 of 20 problems faster here, 0.70 of the time.)  Not up to 4
+// rows, where it is ahead by 2 % of the time where at all.  772 timed problems: takes 0.40 / 0.69 / 0.68 / 0.52 / 0.32 of those of 5 .. 16 / .. 32 / .. 64 / .. 128 / .. 256
+// rows, for 0.94 / 0.85 / 0.77 / 0.80 / 0.86 of the time.  901 calls of other drawn layers: 0.915 of their time, all that stay included; 14 more than 3 % slower, the worst
+// 14208 x 4608 at M = 32 17.4 -> 19.7 us.
+static bool takes_regs(int M, int N, int K, Fp8RegsPlan* plan, double* other) {
+  *plan = fp8_regs_plan(M, N, K);
+  const int steps = K / 128;
+  if (M <= 32 && steps <= (M <= 16 ? 128 : 64)) {      // (stream2_steps_per_wave)
+    const double k = K / 1024.0, act = 0.349 * M / 16 * k * (1 + 0.0311 * k), rounds = ceil(N / 16.0 / num_cus_current_device());
+    const double core = 0.372 * rounds * k + act, mem = 0.137e-6 * K * N;
+    *other = 2.3 + cbrt(core * core * core + mem * mem * mem) + 0.304 * 2e-6 * M * N;
+    return M > 4 && plan->us < 0.97 * *other;
+  }
+  *other = plan_tile3(M, N, K).us;
+  return M > 4 && plan->us < 0.93 * *other;
+}
+
+// The same for a call, from a table per thread.  A switch that names another kernel or a plan of one keeps it out; exp[11]: 1 never, else its plan, n-tiles |
+// m-blocks << 4.
+static bool fp8_regs_chosen(int M, int N, int K, int* mb, int* j) {
+  const VaqTuning& tn = tuning();
+  if (tn.exp[11] > 1) {
+    *mb = tn.exp[11] >> 4;
+    *j = tn.exp[11] & 15;
+    return true;
+  }
+  if (tn.exp[11] == 1 || tn.fp8_path > 0 || tn.fp8_tile_impl != 0 || tn.fp8_tile_cfg != 0 || tn.fp8_split > 0 || tn.fp8_gx > 0 || tn.exp[4] > 0 || tn.exp[6] > 0 ||
+      tn.exp[12] > 0 || tn.exp[13] > 0)
+    return false;
+  static thread_local PlanTable<int> table;
+  const int at = table.get(M, N, K, num_cus_current_device(), [&] {
+    const TuningScope automatic(nullptr);
+    Fp8RegsPlan plan;
+    double other = 0;
+    return takes_regs(M, N, K, &plan, &other) ? plan.j | plan.mb << 4 : 0;
+  });
+  *mb = at >> 4;
+  *j = at & 15;
+  return at != 0;
+}
+
 }  // namespace vaq
+
+extern "C" int vaq_fp8_regs_plan(int64_t size_m, int64_t size_n, int64_t size_k, double* plan) {
+  using namespace vaq;
+  VAQ_CHECK_ARG(size_m > 0 && size_m <= FP8_REGS_MAX_M && size_n > 0 && size_n % 16 == 0 && size_k > 0 && size_k % 128 == 0 && size_n < (1 << 24) &&
+                    size_k < (1 << 24) && plan != nullptr, "fp8_regs_plan: bad arguments");
+  Fp8RegsPlan r;
+  plan[4] = takes_regs((int)size_m, (int)size_n, (int)size_k, &r, &plan[3]) ? 1 : 0;
+  plan[0] = r.j;
+  plan[1] = r.mb;
+  plan[2] = r.us;
+  return VAQ_OK;
+}
 
 extern "C" int vaq_fp8_scaled_mm_workspace(int64_t size_m, int64_t size_n, int64_t size_k, size_t* c_tmp_bytes,
                                            size_t* counter_ints) {
@@ -1473,7 +1531,11 @@ extern "C" int vaq_fp8_scaled_mm_ws_tuned(const uint8_t* a, int64_t lda, const u
   const bool bf16 = out_dtype == VAQ_BF16;
   bool done = false;
   const bool want_stream = tuning().fp8_path != 2 && stream_steps_per_wave(size_m, size_n, size_k) != 0;
-  if (tuning().fp8_path != 2) done = bf16 ? dispatch_stream2<true>(p, s) : dispatch_stream2<false>(p, s);
+  if (size_m <= FP8_REGS_MAX_M && size_k % 128 == 0 && stream_offsets_fit(p)) {
+    int mb = 0, j = 0;
+    if (fp8_regs_chosen(p.M, p.N, p.K, &mb, &j)) done = fp8_regs_launch(p, bf16, mb, j, s);
+  }
+  if (!done && tuning().fp8_path != 2) done = bf16 ? dispatch_stream2<true>(p, s) : dispatch_stream2<false>(p, s);
   if (!done && want_stream) done = bf16 ? dispatch_stream<true>(p, s) : dispatch_stream<false>(p, s);
   if (!done && tuning().fp8_path != 2)
     done = bf16 ? dispatch_stream_split<true>(p, c_tmp_bytes, counter_ints, s)

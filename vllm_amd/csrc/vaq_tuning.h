@@ -45,7 +45,8 @@ typedef struct VaqTuning {
                         /*   [12] = 1 FP8 tile kernel: every tile starts at the first K step; [13] = 1 FP8 tile kernel: no tile  */
                         /*   row past M; [14] > 0 W4A16 tile kernel: KiB that the partial tiles of a K split may take; [6] > 1 both tile     */
                         /*   kernels, 256 x 256 tiles: the tiles of the last round in this many parts of K; [9] = 1 act_order: columns */
-                        /*   permuted by a launch of its own for the W4A16 tile kernel only; [11] unused;                             */
+                        /*   permuted by a launch of its own for the W4A16 tile kernel only; [11] FP8 kernel for some dozen rows: 1 never, else */
+                        /*   its plan, n-tiles | m-blocks << 4;                                                                      */
                         /*   [8] W4A16 kernel with activations in registers: 1 never, else its plan, n-tiles | m-blocks << 4 |        */
                         /*   wavefronts << 8 | parts of K << 12;                                                                     */
                         /*   [7] = 1 LDS-staged decode kernel: n-tiles in launch order, not grouped by XCD             */
@@ -82,6 +83,9 @@ int vaq_w4a16_decode_plan(int64_t size_m, int64_t size_n, int64_t size_k, int su
  * predicted us, predicted us of the kernel that takes the problem otherwise, 1 if this one takes it.
  */
 int vaq_w4a16_regs_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub, int w8, double* plan);
+
+/* The same of the FP8 kernel for some dozen rows (K a multiple of 128): plan[0 .. 4] = n-tiles, m-blocks, predicted us, us of what takes it otherwise, 1 if it takes it. */
+int vaq_fp8_regs_plan(int64_t size_m, int64_t size_n, int64_t size_k, double* plan);
 
 /*
  * The same of the W4A16 tile kernels: plan[0 .. 3] = tile id (41 and above: strips), parts of K, first tile that is split where only
