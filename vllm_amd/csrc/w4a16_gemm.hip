@@ -66,18 +66,19 @@ static int other_kind(int M, int N, int K, int sub, int wt, double* us) {
 
 // Whether the kernel with activations in registers takes a problem: where its price is below this share of the price of what takes it otherwise.  The
 // prices are older than the arguments in registers and off by as much as the kernels have gained since (this one's 3-5 % low, that of the decode kernel 0-8 % low
-// with 4-bit codes in groups of 128 rows and 3-15 % low with the rest), so the shares are set by the choices, for 1 .. 4, 5 .. 16, 17 .. 32, 33 .. 64 and
-// more rows: over 3575 problems of random layers with both timed now the choice takes 1.009 of the faster one's time in the mean.  The shares before (0.85 up
-// to 4 rows and 0.91 up to 32 for 4-bit codes in groups of 128 rows, 0.95 up to 32 for groups of 64 / 32) took 1.016; of the 300 calls that move 4 % are more
-// than 3 % slower.  Drawn layers: 3712 x 17792 at M = 1 9.8 -> 8.6 us, 9216 x 4416 at M = 4 9.2 -> 8.0, 11520 x 5248 at M = 18 14.0 -> 12.9; 1792 x 11008 at
-// M = 3 4.5 -> 4.9.  From 33 rows on shares nearer to one lose as much as they gain: strips cost less, and zero points in small groups more, than priced (4-bit
+// with 4-bit codes in groups of 128 rows and 3-15 % low with the rest), so the shares are set by the choices, for one, 2 .. 4, 5 .. 16, 17 .. 32, 33 .. 64
+// and more rows: over 3575 problems of random layers with both timed now the choice takes 1.010 of the faster one's time in the mean.  The shares before (0.85 up
+// to 4 rows and 0.91 up to 32 for 4-bit codes in groups of 128 rows, 0.95 up to 32 for groups of 64 / 32) took 1.016.  (One row of those: 0.85 still, the decode
+// kernel's instance for it is up to 27 % cheaper than priced; 4096 x 28672 11.9 us there, priced 15.1, and 12.8 here.)  Drawn layers: 9216 x
+// 4416 at M = 4 9.2 -> 8.0 us, 11520 x 5248 at M = 18 14.0 -> 12.9; 1792 x 11008 at M = 3 4.5 -> 4.9.  From 33 rows on shares nearer to one lose as much as they gain: strips cost less, and zero points in small groups more, than priced (4-bit
 // codes in groups of 32 with zero points at M = 34 13.7 -> 15.7).
 static double regs_lead(int M, int N, int K, int sub, int wt, int j, int nw) {
-  constexpr double SHARE[4][5] = {{0.95, 0.96, 0.97, 0.95, 0.92}, {1.05, 1.0, 1.0, 0.88, 0.88}, {1.05, 1.0, 0.95, 0.88, 0.88}, {1.17, 1.01, 1.01, 0.95, 0.95}};
+  constexpr double SHARE[4][6] = {{0.85, 0.95, 0.96, 0.97, 0.95, 0.92}, {1.05, 1.05, 1.0, 1.0, 0.88, 0.88}, {1.05, 1.05, 1.0, 0.95, 0.88, 0.88},
+                                  {1.17, 1.17, 1.01, 1.01, 0.95, 0.95}};
   // vocabulary-sized layers at 3 .. 16 rows, where another kernel is the alternative (it takes them all: 0.37 .. 0.96 of the time, 1 of 2000 more than 3 % slower;
   // 4096 x 128256 at M = 4 / 16 54.9 / 59.0 -> 51.9 / 53.4 us, 1024 x 128256 33.4 / 34.0 -> 18.1 / 19.5, 5120 x 65536 80.0 / 81.0 -> 33.2 / 34.7)
   if (wt == 0 && decode_impl_for(M, N, K, sub, false) == 1) return 0.95;
-  const double lead = SHARE[wt != 0 ? 3 : sub == 1 ? 0 : sub == 2 ? 1 : 2][M <= 4 ? 0 : M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 3 : 4];
+  const double lead = SHARE[wt != 0 ? 3 : sub == 1 ? 0 : sub == 2 ? 1 : 2][M <= 1 ? 0 : M <= 4 ? 1 : M <= 16 ? 2 : M <= 32 ? 3 : M <= 64 ? 4 : 5];
   if (wt != 0 || sub > 1 || M > 32) return lead;
   // Where this kernel loses most of what it loses, by as much as the two prices together are off by: K of whole 1024 rows; one n-tile to a wavefront and K
   // beyond 8192 at up to 4 rows; two and more n-tiles on a short K.  Off are: this kernel's price, which counts 16 rows to a block, by the rows that a block has;
