@@ -30,10 +30,10 @@ def _run(a, b, device, dtype=torch.float16, sa=None, sb=None, bias=None):
 @pytest.mark.parametrize("mb", [1, 2, 3, 4])
 @pytest.mark.parametrize("j", [1, 2, 3, 4])
 def test_every_launch_shape_exact(device, mb, j):
-    """From a K of half a step (most wavefronts without one) to several turns of the ring with half a step at the end; one row, ragged last blocks of rows and of
+    """From a K of one chunk (most wavefronts without a step) to several turns of the ring with any part of a step at the end; one row, ragged last blocks of rows and of
     n-tiles, several blocks of rows.  (Shapes that do not fit LDS are not built: such a switch changes nothing.)"""
     from vllm_amd import _tuning
-    for k in (128, 256, 384, 896, 1024, 1152, 2048, 2176, 5248):
+    for k in (16, 128, 240, 256, 384, 896, 1024, 1040, 1152, 2048, 2176, 3056, 5248):
         m, n = 1 + (k * 7 + mb * 37) % 200, 16 * (1 + (k // 128 * 5 + j * 11) % 37)
         a, b, want = _case(m, n, k, k + mb, device, gap=64 if k % 256 else 0)
         with _tuning.override(exp=[0] * 11 + [j | mb << 4]):
@@ -57,7 +57,7 @@ def test_scales_and_bias_as_the_tile_kernel(device, dtype, per_row, per_col, bia
 
 
 @pytest.mark.parametrize("m,n,k", [(16, 4096, 14336), (17, 1024, 1024), (32, 4096, 4096), (33, 2048, 2048), (64, 1280, 2560), (64, 4096, 4096), (100, 1024, 4096), (128, 2048, 2048),
-                                   (200, 1024, 1024), (256, 1024, 4096)])
+                                   (200, 1024, 1024), (256, 1024, 4096), (33, 4224, 2256), (48, 1024, 1040), (64, 1344, 3904), (100, 1200, 2320)])
 def test_as_chosen_exact(device, m, n, k):
     from vllm_amd import _lib
     plan = (ctypes.c_double * 5)()
@@ -65,3 +65,17 @@ def test_as_chosen_exact(device, m, n, k):
     assert plan[4] == 1
     a, b, want = _case(m, n, k, k, device)
     assert torch.equal(_run(a, b, device).cpu().float(), want)
+
+
+def test_infinite_results_and_nan_codes_stay_in_their_rows_and_columns(device):
+    """A NaN code among the activations or the weights makes its row or column NaN and nothing else; behind K it does nothing (the gap's codes are NaN)."""
+    from vllm_amd import _tuning
+    for k in (512, 720):
+        a, b, want = _case(37, 96, k, 7, device, gap=48)
+        a.view(torch.uint8)[5, k - 1] = 0x7f
+        b.t().view(torch.uint8)[17, 0] = 0xff
+        with _tuning.override(exp=[0] * 11 + [2 | 2 << 4]):
+            out = _run(a, b, device).cpu().float()
+        bad = torch.zeros(37, 96, dtype=torch.bool)
+        bad[5], bad[:, 17] = True, True
+        assert torch.equal(out.isnan(), bad) and torch.equal(out[~bad], want[~bad])

@@ -8,14 +8,16 @@ namespace vaq {
 // In us: `base`, `out` per MB of results; a workgroup `round`, `meet` for each 16 x 16 result and its steps, each the latency, the bytes into the compute unit or the
 // products of all workgroups on it, whichever is longest, more where K is a multiple of 1024 (rows start on the same memory channels); beside that the weights
 // from memory, `again` of them for every further block of rows.  Fitted to the cold times of 772 problems (K 256 .. 28672, N 256 .. 28672, 1 .. 256 rows) with all their
-// plans: 7 % rms, the cheapest plan takes 1.005 of the fastest one's time in the mean.
+// plans: 7 % rms, the cheapest plan takes 1.005 of the fastest one's time in the mean.  Rows that do not start with a cache line, K no multiple of 128: 1.00 of that up to
+// K = 2048, 1.13 to 8192, 1.31 beyond (50 calls; 12080 x 1536 at M = 33 14.3 us, 12032 x 1536 10.5).
 static double plan_us(int mb, int j, double M, double N, double K, int cus) {
   const double rb = ceil(M / (16 * mb)), per_cu = ceil(ceil(N / 16 / j) * rb / cus);
   const double slots = fmin(floor(160.0 * 1024 / fp8_regs_lds_bytes(mb, j)), 4.0), side = fmin(per_cu, slots), rounds = fmax(per_cu / slots, 1.0);
   const double steps = ceil(ceil(K / FP8_REGS_STEP) / FP8_REGS_WAVES), bytes = 0.0119 * 16 * side * (mb + j), work = 0.102 * side * mb * j;
   const double step = cbrt(0.122 + bytes * bytes * bytes + work * work * work) * ((int64_t)K % 1024 == 0 ? 1.077 : 1.0);
   const double core = rounds * (0.272 + steps * step + 0.0906 * mb * j), mem = 0.183e-6 * K * N * (1 + 0.338 * (rb - 1));
-  return 1.66 + cbrt(core * core * core + mem * mem * mem) + 0.258 * 2e-6 * M * N;
+  const double us = 1.66 + cbrt(core * core * core + mem * mem * mem) + 0.258 * 2e-6 * M * N;
+  return (int64_t)K % 128 != 0 ? us * (1 + 0.026 * K / 1024) : us;
 }
 
 Fp8RegsPlan fp8_regs_plan(int M, int N, int K) {
@@ -34,26 +36,28 @@ Fp8RegsPlan fp8_regs_plan(int M, int N, int K) {
   return best;
 }
 
-template <bool BF16_OUT, int MB, int J>
+template <bool BF16_OUT, int MB, int J, bool TAIL>
 static bool launch(const Fp8MMParams& p_in, hipStream_t s) {
-  if constexpr (!fp8_regs_built(MB, J)) {
-    return false;
-  } else {
-    Fp8MMParams p = p_in;
-    const uint32_t NT = (uint32_t)p.N / 16, RB = ((uint32_t)p.M + MB * 16 - 1) / (MB * 16), ranges = (NT + J - 1) / J, per_xcd = (ranges * RB + 7) / 8;
-    p.a_extent = (uint32_t)((int64_t)(p.M - 1) * p.lda + p.K);
-    p.b_extent = (uint32_t)((int64_t)(p.N - 1) * p.ldb + p.K);
-    constexpr size_t lds = fp8_regs_lds_bytes(MB, J);
-    auto kern = fp8_mm_regs_kernel<BF16_OUT, MB, J>;
-    static size_t reserved[VAQ_MAX_DEVICES];
-    if (reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds, reserved, "fp8_scaled_mm") != VAQ_OK) return false;
-    // (unit / RB by multiplication: exact for unit * RB < 2^32)
-    const uint32_t steps = ((uint32_t)p.K + FP8_REGS_STEP - 1) / FP8_REGS_STEP, half = p.K % FP8_REGS_STEP != 0 ? 1u : 0u;
-    hipLaunchKernelGGL(kern, dim3(per_xcd * 8), dim3(FP8_REGS_WAVES * 64), lds, s,
-                       (v8u{ptr_lo(p.a), ptr_hi(p.a), ptr_lo(p.b), ptr_hi(p.b), (uint32_t)p.lda, (uint32_t)p.ldb, p.a_extent, p.b_extent}),
-                       (v4u{steps << 1 | half, (uint32_t)p.M | RB << 16, ranges, per_xcd}), (v2u{NT, (uint32_t)((1ull << 32) / RB + 1)}), p);
-    return true;
-  }
+  Fp8MMParams p = p_in;
+  const uint32_t NT = (uint32_t)p.N / 16, RB = ((uint32_t)p.M + MB * 16 - 1) / (MB * 16), ranges = (NT + J - 1) / J, per_xcd = (ranges * RB + 7) / 8;
+  p.a_extent = (uint32_t)((int64_t)(p.M - 1) * p.lda + p.K);
+  p.b_extent = (uint32_t)((int64_t)(p.N - 1) * p.ldb + p.K);
+  constexpr size_t lds = fp8_regs_lds_bytes(MB, J);
+  auto kern = fp8_mm_regs_kernel<BF16_OUT, MB, J, TAIL>;
+  static size_t reserved[VAQ_MAX_DEVICES];
+  if (reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds, reserved, "fp8_scaled_mm") != VAQ_OK) return false;
+  // (unit / RB by multiplication: exact for unit * RB < 2^32)
+  const uint32_t steps = ((uint32_t)p.K + FP8_REGS_STEP - 1) / FP8_REGS_STEP, rest = (uint32_t)p.K % FP8_REGS_STEP;
+  hipLaunchKernelGGL(kern, dim3(per_xcd * 8), dim3(FP8_REGS_WAVES * 64), lds, s,
+                     (v8u{ptr_lo(p.a), ptr_hi(p.a), ptr_lo(p.b), ptr_hi(p.b), (uint32_t)p.lda, (uint32_t)p.ldb, p.a_extent, p.b_extent}),
+                     (v4u{steps << 8 | rest, (uint32_t)p.M | RB << 16, ranges, per_xcd}), (v2u{NT, (uint32_t)((1ull << 32) / RB + 1)}), p);
+  return true;
+}
+
+template <bool BF16_OUT, int MB, int J>
+static bool launch(const Fp8MMParams& p, hipStream_t s) {
+  if constexpr (!fp8_regs_built(MB, J)) return false;
+  else return p.K % FP8_REGS_STEP != 0 ? launch<BF16_OUT, MB, J, true>(p, s) : launch<BF16_OUT, MB, J, false>(p, s);
 }
 
 template <bool BF16_OUT, int MB>

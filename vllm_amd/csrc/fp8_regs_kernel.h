@@ -25,14 +25,16 @@ constexpr size_t fp8_regs_lds_bytes(int mb, int j) {
   return run > sums ? run : sums;
 }
 
-template <bool BF16_OUT, int MB, int J>
+// TAIL: K ends inside a step.  What a row has behind K is not its own (a NaN in the weights is one whatever it is multiplied with): of the last step each lane asks
+// for the chunks before K, and the rest of both operands arrives as zeros.
+template <bool BF16_OUT, int MB, int J, bool TAIL>
 __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ_HEAD_ARGS, const Fp8MMParams p) {
   using T = F16Traits<BF16_OUT>;
   constexpr int NW = FP8_REGS_WAVES, KT = FP8_REGS_STEP, R = (J * MB + NW - 1) / NW, TB = 16 * KT, LI = TB / 1024;
   const uint8_t* const a = head_ptr<uint8_t>(h0[0], h0[1]);
   const uint8_t* const b = head_ptr<uint8_t>(h0[2], h0[3]);
   const uint32_t lda = h0[4], ldb = h0[5], a_extent = h0[6], b_extent = h0[7];
-  const int all = (int)(h1[0] >> 1), half = (int)(h1[0] & 1u), M = (int)(h1[1] & 0xffffu), NT = (int)h2[0];
+  const int all = (int)(h1[0] >> 8), rest = (int)(h1[0] & 0xffu), M = (int)(h1[1] & 0xffffu), NT = (int)h2[0];
   const uint32_t RB = h1[1] >> 16, ranges = h1[2], per_xcd = h1[3];
   extern __shared__ __attribute__((aligned(16))) uint8_t lds8[];
   const int lane = threadIdx.x & 63;
@@ -66,11 +68,15 @@ __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ
     vo_w[i] = (uint32_t)r * ldb + (uint32_t)((r16 ^ r) * 16);
   }
   // (a step past the last has no extent: its requests fetch nothing and keep the count of requests under way)
+  auto place = [&](uint32_t vo, int r, int g) {
+    if constexpr (TAIL) return g == all - 1 && ((r16 ^ (r & 15)) * 16) >= rest ? 0x80000000u : vo;
+    return vo;
+  };
   auto load_act = [&](int g) {
     const __amdgpu_buffer_rsrc_t ra = rsrc(a, g < steps ? a_extent : 0u);
 #pragma unroll
     for (int i = 0; i < LI * MB; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(mine + i * 1024), 16, (int)vo_a[i], g * KT, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(mine + i * 1024), 16, (int)place(vo_a[i], i * 4 + q, g), g * KT, 0, 0);
   };
   auto load_w = [&](int s, int g) {
     const __amdgpu_buffer_rsrc_t rb = rsrc(b, g < steps ? b_extent : 0u);
@@ -79,7 +85,7 @@ __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ
       const int so = (int)((uint32_t)(min(nt0 + j, NT - 1) * 16) * ldb + (uint32_t)(g * KT));
 #pragma unroll
       for (int i = 0; i < LI; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(mine + (MB + s * J + j) * TB + i * 1024), 16, (int)vo_w[i], so, 0, 2);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(mine + (MB + s * J + j) * TB + i * 1024), 16, (int)place(vo_w[i], i * 4 + q, g), so, 0, 2);
     }
   };
   v4f acc[J][MB];
@@ -94,7 +100,7 @@ __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ
     return v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
   };
   constexpr int U = KT / 128;
-  auto tile = [&](int s, bool refill, bool whole, int next_act, int next_w) {
+  auto tile = [&](int s, bool refill_act, bool refill_w, int next_act, int next_w) {
     v8i act[U][MB], wop[U][J];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -103,21 +109,22 @@ __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ
 #pragma unroll
       for (int j = 0; j < J; ++j) wop[u][j] = operand(mine + (MB + s * J + j) * TB, u);
     }
-    if (refill) {
+    if (refill_act) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // this step's are in registers
       __builtin_amdgcn_sched_barrier(0);
       load_act(next_act);
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if (refill_w) {
       load_w(s, next_w);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (u == 0 || whole)
 #pragma unroll
-        for (int j = 0; j < J; ++j)
+      for (int j = 0; j < J; ++j)
 #pragma unroll
-          for (int mb = 0; mb < MB; ++mb) acc[j][mb] = mfma_fp8_16(wop[u][j], act[u][mb], acc[j][mb]);
+        for (int mb = 0; mb < MB; ++mb) acc[j][mb] = mfma_fp8_16(wop[u][j], act[u][mb], acc[j][mb]);
   };
 
   // W(0) A(0) W(1) | A(1) W(2) | A(2) W(3) | ..., `|` = a step: it starts when all but the weights requested behind its activations have been answered
@@ -127,7 +134,7 @@ __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ
   __builtin_amdgcn_sched_barrier(0);
   load_act(g);
   __builtin_amdgcn_sched_barrier(0);
-  load_w(1, g + 1);
+  if (g + 1 < steps) load_w(1, g + 1);
   __builtin_amdgcn_sched_barrier(0);
   VAQ_ARRIVED4(p.sb, p.bias, p.out, p.sb_per_col);
   // scales and bias of this wavefront's results, ahead of the K loop (behind it they are a round trip to memory on their own)
@@ -149,16 +156,15 @@ __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ
     wait();
     tile(1, true, true, g + 2, g + 3);
   }
-  // the last one or two; only the last of K can be half a step
-  const bool whole = steps < all || half == 0;
+  // the last one or two ask for no weights (requests for nothing behind them cost 3 % of a call)
   if (g + 1 < steps) {
     wait();
-    tile(0, true, true, g + 1, g + 2);
-    wait();
-    tile(1, false, whole, 0, 0);
+    tile(0, true, false, g + 1, 0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    tile(1, false, false, 0, 0);
   } else if (g < steps) {
-    wait();
-    tile(0, false, whole, 0, 0);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R) : "memory");      // (all but the last of the scales, one load at least for each result)
+    tile(0, false, false, 0, 0);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (what is requested past the end writes zeros into LDS)
 

@@ -11,7 +11,7 @@
 //  * stream kernels (M <= 32; M <= 64 on narrow layers with K <= 4096): weight-streaming GEMV-like, weights are the A operand
 //    of v_mfma_f32_16x16x128_f8f6f4, activations stay in registers, the wavefronts of a workgroup split K and reduce
 //    through LDS; fp8_mm_stream2_kernel (fp8_stream2_kernel.h) brings the weights in through LDS as whole cache lines;
-//  * fp8_mm_regs_kernel (fp8_regs_kernel.h; 5 .. 256 rows, K a multiple of 128, where predicted ahead of the others): both operands as
+//  * fp8_mm_regs_kernel (fp8_regs_kernel.h; 5 .. 256 rows, where predicted ahead of the others): both operands as
 //    whole lines through LDS that no other wavefront touches, several n-tiles and m-blocks a wavefront.
 //
 // The per-lane byte -> k assignment inside an MFMA operand is the same function for A and B, so any consistent choice
@@ -1384,7 +1384,7 @@ static bool dispatch_stream(const Fp8MMParams& p, hipStream_t s) {
   return true;
 }
 
-// Whether the kernel of fp8_regs_kernel.h takes a problem (K a multiple of 128): where its price is 7 % below that of the tile plan, or 3 % below that of the stream
+// Whether the kernel of fp8_regs_kernel.h takes a problem: where its price is 7 % below that of the tile plan, or 3 % below that of the stream
 // kernel with weights through LDS -- its rows' activations, its n-tiles in rounds of one to a compute unit, the weights from memory; fitted to 291 of the
 // timings below, 7 % rms.  (33 .. 64 rows where the other stream kernel was ahead of the tiles: 20 of 20 problems faster here, 0.70 of the time.)  Not up to 4
 // rows, where it is ahead by 2 % of the time where at all.  772 timed problems: takes 0.40 / 0.69 / 0.68 / 0.52 / 0.32 of those of 5 .. 16 / .. 32 / .. 64 / .. 128 / .. 256
@@ -1392,7 +1392,7 @@ static bool dispatch_stream(const Fp8MMParams& p, hipStream_t s) {
 // 14208 x 4608 at M = 32 17.4 -> 19.7 us.
 static bool takes_regs(int M, int N, int K, Fp8RegsPlan* plan, double* other) {
   *plan = fp8_regs_plan(M, N, K);
-  const int steps = K / 128;
+  const int steps = (K + 127) / 128;
   if (M <= 32 && steps <= (M <= 16 ? 128 : 64)) {      // (stream2_steps_per_wave)
     const double k = K / 1024.0, act = 0.349 * M / 16 * k * (1 + 0.0311 * k), rounds = ceil(N / 16.0 / num_cus_current_device());
     const double core = 0.372 * rounds * k + act, mem = 0.137e-6 * K * N;
@@ -1431,7 +1431,7 @@ static bool fp8_regs_chosen(int M, int N, int K, int* mb, int* j) {
 
 extern "C" int vaq_fp8_regs_plan(int64_t size_m, int64_t size_n, int64_t size_k, double* plan) {
   using namespace vaq;
-  VAQ_CHECK_ARG(size_m > 0 && size_m <= FP8_REGS_MAX_M && size_n > 0 && size_n % 16 == 0 && size_k > 0 && size_k % 128 == 0 && size_n < (1 << 24) &&
+  VAQ_CHECK_ARG(size_m > 0 && size_m <= FP8_REGS_MAX_M && size_n > 0 && size_n % 16 == 0 && size_k > 0 && size_k % 16 == 0 && size_n < (1 << 24) &&
                     size_k < (1 << 24) && plan != nullptr, "fp8_regs_plan: bad arguments");
   Fp8RegsPlan r;
   plan[4] = takes_regs((int)size_m, (int)size_n, (int)size_k, &r, &plan[3]) ? 1 : 0;
@@ -1531,7 +1531,7 @@ extern "C" int vaq_fp8_scaled_mm_ws_tuned(const uint8_t* a, int64_t lda, const u
   const bool bf16 = out_dtype == VAQ_BF16;
   bool done = false;
   const bool want_stream = tuning().fp8_path != 2 && stream_steps_per_wave(size_m, size_n, size_k) != 0;
-  if (size_m <= FP8_REGS_MAX_M && size_k % 128 == 0 && stream_offsets_fit(p)) {
+  if (size_m <= FP8_REGS_MAX_M && size_n < (1 << 24) && size_k < (1 << 24) && stream_offsets_fit(p)) {
     int mb = 0, j = 0;
     if (fp8_regs_chosen(p.M, p.N, p.K, &mb, &j)) done = fp8_regs_launch(p, bf16, mb, j, s);
   }

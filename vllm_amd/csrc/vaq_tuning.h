@@ -84,7 +84,7 @@ int vaq_w4a16_decode_plan(int64_t size_m, int64_t size_n, int64_t size_k, int su
  */
 int vaq_w4a16_regs_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub, int w8, double* plan);
 
-/* The same of the FP8 kernel for some dozen rows (K a multiple of 128): plan[0 .. 4] = n-tiles, m-blocks, predicted us, us of what takes it otherwise, 1 if it takes it. */
+/* The same of the FP8 kernel for some dozen rows: plan[0 .. 4] = n-tiles, m-blocks, predicted us, us of what takes it otherwise, 1 if it takes it. */
 int vaq_fp8_regs_plan(int64_t size_m, int64_t size_n, int64_t size_k, double* plan);
 
 /*
