@@ -19,8 +19,18 @@ static const VaqTuning g_no_tuning = {};
 
 const VaqTuning& tuning() { return g_tuning ? *g_tuning : g_no_tuning; }
 bool tuning_active() { return g_tuning != nullptr; }
-TuningScope::TuningScope(const VaqTuning* t) : prev_(g_tuning) { g_tuning = t; }
-TuningScope::~TuningScope() { g_tuning = prev_; }
+// Compute units of the device that the entry point under way on this thread runs on, asked for once a call (0: not yet, or outside of one): the
+// rules and plans that a call passes each asked the runtime for the device before.  An eager call of a 2048 x 2048 layer at one row is bound by the host: 6.19 ->
+// 6.01 us, with the reservation of LDS that small launches do not need left out (reserve_dynamic_lds).
+static thread_local int g_depth = 0, g_call_cus = 0;
+TuningScope::TuningScope(const VaqTuning* t) : prev_(g_tuning) {
+  g_tuning = t;
+  ++g_depth;
+}
+TuningScope::~TuningScope() {
+  g_tuning = prev_;
+  if (--g_depth == 0) g_call_cus = 0;
+}
 
 // Immutable per-device cache (the only host-visible state of the library).
 static int g_cus[64];
@@ -37,10 +47,13 @@ static int cus_of(int dev) {
 }
 
 int num_cus_current_device() {
+  if (g_call_cus > 0) return g_call_cus;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 256;
   int c = cus_of(dev);
-  return c > 0 ? c : 256;
+  c = c > 0 ? c : 256;
+  if (g_depth > 0) g_call_cus = c;
+  return c;
 }
 
 }  // namespace vaq

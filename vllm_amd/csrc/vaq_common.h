@@ -62,6 +62,7 @@ class TuningScope {
 // The attribute is idempotent, so two threads racing here at worst set it twice.
 constexpr int VAQ_MAX_DEVICES = 64;
 inline int reserve_dynamic_lds(const void* kern, size_t lds, size_t (&reserved)[VAQ_MAX_DEVICES], const char* what) {
+  if (lds <= 64 * 1024) return VAQ_OK;      // (needs no reservation)
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= VAQ_MAX_DEVICES) {
     set_error("%s: cannot identify the current device", what);
