@@ -1384,12 +1384,14 @@ static bool dispatch_stream(const Fp8MMParams& p, hipStream_t s) {
   return true;
 }
 
-// Whether the kernel of fp8_regs_kernel.h takes a problem: where its price is 7 % below that of the tile plan, or 3 % below that of the stream
-// kernel with weights through LDS -- its rows' activations, its n-tiles in rounds of one to a compute unit, the weights from memory; fitted to 291 of the
-// timings below, 7 % rms.  (33 .. 64 rows where the other stream kernel was ahead of the tiles: 20 of 20 problems faster here, 0.70 of the time.)  Not up to 4
-// rows, where it is ahead by 2 % of the time where at all.  772 timed problems: takes 0.40 / 0.69 / 0.68 / 0.52 / 0.32 of those of 5 .. 16 / .. 32 / .. 64 / .. 128 / .. 256
-// rows, for 0.94 / 0.85 / 0.77 / 0.80 / 0.86 of the time.  901 calls of other drawn layers: 0.915 of their time, all that stay included; 14 more than 3 % slower, the worst
-// 14208 x 4608 at M = 32 17.4 -> 19.7 us.
+// Whether the kernel of fp8_regs_kernel.h takes a problem: where its price is 7 % below that of the tile plan, or not so far above that of the stream kernel with
+// weights through LDS -- its rows' activations, its n-tiles in rounds of one to a compute unit, the weights from memory; fitted to 291 of the timings
+// below, 7 % rms.  Up to 16 rows 3 %; from 17 rows on, which the price counts as 32 whatever their number, 10 % up to N = 12288 and none beyond, where the stream kernel
+// is at memory speed (2944 x 21248 at M = 20 12.4 us, 15.2 here).  At 3 % below throughout 8192 x 8192 at M = 24 stayed there for 22.7 us, 12.9 here.  (33 .. 64 rows
+// where the other stream kernel was ahead of the tiles: 20 of 20 problems faster here, 0.70 of the time.)  Not up to 4 rows, where it is ahead by 2 % of the time
+// where at all.  811 timed problems: takes 0.71 / 0.88 / 0.68 / 0.52 / 0.32 of those of 5 .. 16 / .. 32 / .. 64 / .. 128 / .. 256
+// rows, for 0.95 / 0.84 / 0.77 / 0.80 / 0.86 of the time, 2 % of them more than 3 % slower.  901 calls of other drawn layers 0.915 of their time at the first shares, 600
+// of 5 .. 32 rows another 0.990 from those to these (14208 x 4608 at M = 32 17.4 -> 19.7 us, 2304 x 12800 at M = 16 7.2 -> 7.7).
 static bool takes_regs(int M, int N, int K, Fp8RegsPlan* plan, double* other) {
   *plan = fp8_regs_plan(M, N, K);
   const int steps = (K + 127) / 128;
@@ -1397,7 +1399,7 @@ static bool takes_regs(int M, int N, int K, Fp8RegsPlan* plan, double* other) {
     const double k = K / 1024.0, act = 0.349 * M / 16 * k * (1 + 0.0311 * k), rounds = ceil(N / 16.0 / num_cus_current_device());
     const double core = 0.372 * rounds * k + act, mem = 0.137e-6 * K * N;
     *other = 2.3 + cbrt(core * core * core + mem * mem * mem) + 0.304 * 2e-6 * M * N;
-    return M > 4 && plan->us < 0.97 * *other;
+    return M > 4 && plan->us < (M <= 16 ? 1.03 : N <= 12288 ? 1.1 : 1.0) * *other;
   }
   *other = plan_tile3(M, N, K).us;
   return M > 4 && plan->us < 0.93 * *other;
