@@ -7,7 +7,7 @@ namespace vaq {
 
 // In us: `base`, `out` per MB of results; a workgroup `round`, `meet` for each 16 x 16 result and its steps, each the latency, the bytes into the compute unit or the
 // products of all workgroups on it, whichever is longest, more where K is a multiple of 1024 (rows start on the same memory channels); beside that the weights
-// from memory, `again` of them for every further block of rows.  Fitted to the cold times of 772 problems (K 256 .. 28672, N 256 .. 28672, 1 .. 256 rows) with all their
+// from memory, `again` of them for every further block of rows.  Fitted to the cold times of 772 problems (profiles/plan_prices/fp8_some_rows.csv.gz; 1 .. 256 rows) with all their
 // plans: 7 % rms, the cheapest plan takes 1.005 of the fastest one's time in the mean.  Rows that do not start with a cache line, K no multiple of 128: 1.00 of that up to
 // K = 2048, 1.13 to 8192, 1.31 beyond (50 calls; 12080 x 1536 at M = 33 14.3 us, 12032 x 1536 10.5).
 static double plan_us(int mb, int j, double M, double N, double K, int cus) {
