@@ -67,7 +67,8 @@ __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ
     const int r = i * 4 + q;
     vo_w[i] = (uint32_t)r * ldb + (uint32_t)((r16 ^ r) * 16);
   }
-  // (a step past the last has no extent: its requests fetch nothing and keep the count of requests under way)
+  // A step past the last has no extent and starts at 0, so that every offset is past the end of it (the check is against the extent less the scalar offset, which is
+  // not to pass below zero): its requests fetch nothing and keep the count of requests under way.
   auto place = [&](uint32_t vo, int r, int g) {
     if constexpr (TAIL) return g == all - 1 && ((r16 ^ (r & 15)) * 16) >= rest ? 0x80000000u : vo;
     return vo;
@@ -76,13 +77,13 @@ __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ
     const __amdgpu_buffer_rsrc_t ra = rsrc(a, g < steps ? a_extent : 0u);
 #pragma unroll
     for (int i = 0; i < LI * MB; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(mine + i * 1024), 16, (int)place(vo_a[i], i * 4 + q, g), g * KT, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(mine + i * 1024), 16, (int)place(vo_a[i], i * 4 + q, g), g < steps ? g * KT : 0, 0, 0);
   };
   auto load_w = [&](int s, int g) {
     const __amdgpu_buffer_rsrc_t rb = rsrc(b, g < steps ? b_extent : 0u);
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-      const int so = (int)((uint32_t)(min(nt0 + j, NT - 1) * 16) * ldb + (uint32_t)(g * KT));
+      const int so = g < steps ? (int)((uint32_t)(min(nt0 + j, NT - 1) * 16) * ldb + (uint32_t)(g * KT)) : 0;
 #pragma unroll
       for (int i = 0; i < LI; ++i)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(mine + (MB + s * J + j) * TB + i * 1024), 16, (int)place(vo_w[i], i * 4 + q, g), so, 0, 2);
