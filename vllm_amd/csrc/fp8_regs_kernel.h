@@ -138,6 +138,7 @@ __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ
   if (g + 1 < steps) load_w(1, g + 1);
   __builtin_amdgcn_sched_barrier(0);
   VAQ_ARRIVED4(p.sb, p.bias, p.out, p.sb_per_col);
+  const __amdgpu_buffer_rsrc_t rsa = rsrc(p.sa, p.sa_per_row ? (uint32_t)M * 4u : 4u);
   // scales and bias of this wavefront's results, ahead of the K loop (behind it they are a round trip to memory on their own)
   v4f sb4[R];
   v2u bias4[R];
@@ -145,7 +146,7 @@ __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ
 #pragma unroll
   for (int i = 0; i < R; ++i) {
     const int u = w + i * NW, j = u / MB, mb = u - j * MB, n = min(nt0 + j, NT - 1) * 16 + q * 4, m = min(row0 + mb * 16 + r16, M - 1);
-    sam[i] = p.sa[p.sa_per_row ? m : 0];
+    sam[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsa, p.sa_per_row ? m * 4 : 0, 0, 0));      // (a vector load whatever the scales: counted below)
     if (p.sb_per_col) sb4[i] = *reinterpret_cast<const v4f*>(p.sb + n);
     else sb4[i] = v4f{1.f, 1.f, 1.f, 1.f} * p.sb[0];
     bias4[i] = p.bias ? *reinterpret_cast<const v2u*>(p.bias + n) : v2u{0u, 0u};
