@@ -46,6 +46,30 @@ def test_permuted_ahead_equals_gathered_equals_sorted(device, k, n, g, bits, asy
     assert bool((layer.workspace == 0).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("k,n,g,bits,asym", [(640, 3008, 64, 4, False), (1024, 1024, 128, 4, True), (1152, 2048, 32, 4, True), (512, 4160, 128, 8, False),
+                                             (2048, 1024, 64, 8, False), (4096, 1088, 128, 4, False)])
+def test_infinite_and_huge_activations_beyond_32_rows(device, k, n, g, bits, asym, dtype):
+    """From 33 rows on (4-bit codes in groups of 128 rows: 65) an infinite activation gives infinities of the weights' signs (NaN where the weight is 0), and a bf16 one of 2^122
+    (codes with their bias of 128 and more would overflow, the weights themselves stay below 2^5) finite results, as on the tile kernels: workgroups of 16 rows, which give NaN, take no such call.  The other rows keep their bits."""
+    case = o.make_w4a16_case(k, n, g, asym=asym, act_order=True, dtype=dtype, seed=k + n, num_bits=bits)
+    layer, w = W4A16Layer(case, device, dtype), o.case_w_ref(case).double()
+    for m in (33, 48, 64, 65, 80, 96, 125, 128, 160, 200, 256)[3 if g == 128 and bits == 4 else 0:]:
+        a = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(dtype)
+        clean, special, at = a.clone(), [0, 17, 30, m - 1], [(131 * i + 7) % k for i in range(m)]
+        for row, value in zip(special, (float("inf"), 2.0 ** 122 if dtype == torch.bfloat16 else 4096.0, float("-inf"), float("inf"))):
+            a[row, at[row]] = value
+        got, want = layer(a.to(device)).cpu(), layer(clean.to(device)).cpu()
+        plain = [i for i in range(m) if i not in special]
+        assert torch.equal(got[plain], want[plain]), m
+        for row in special:
+            ref = a[row].double() @ w
+            if bool(torch.isfinite(a[row]).all()):      # one rounding to 16 bits of a weight and one of the result, fp32 sums of up to k terms beside them
+                assert bool(((got[row].double() - ref).abs() <= ref.abs() * 2.0 ** -7 + ref.abs().max() * k * 2.0 ** -24).all()), (m, row)
+            else:
+                assert torch.equal(torch.nan_to_num(got[row].double(), 0.25, 1, -1), torch.nan_to_num(ref, 0.25, 1, -1)), (m, row)
+
+
 def _c_call(lib, _lib, layer, x, c_tmp, a_tmp, counters):
     out = torch.empty((x.shape[0], layer.n), dtype=x.dtype, device=x.device)
     ptr = lambda t: None if t is None or t.numel() == 0 else ctypes.c_void_p(t.data_ptr())

@@ -435,13 +435,14 @@ int w4a16_decode2_choose(int M, int N, int K, int sub, int wt, bool act_order, b
   // within 0.2 - 0.6 % of the fastest one's time in the mean, 1.3 % for groups of 64 / 32 rows at 17 .. 32 rows; 6600 problems.  The strips
   // that run in their place are up to 40 % faster; they take no problem from here because they round the scaled weights to 16 bits.
   // act_order: workgroups of all rows, with float32 scales, keep what they were given when the columns were always gathered inside them
-  // and the tile kernel's launch for it was priced at 4 us.)
+  // and the tile kernel's launch for it was priced at 4 us; workgroups of 16 rows take calls from those only: the tile kernel gives the weights'
+  // infinities where an activation is infinite, and finite results of huge ones, the decode kernel NaN.)
   double us = tile_ok ? tile_us * (!w8 ? 1.04 : M <= 64 ? 1.06 : 1.0) : -1;
   if (wg_ok) {
     const double t = workgroup_plan(M, N, K, sub, w8).us;
     if (us < 0 || t < us + (act_order ? 4.0 : 0.0)) { us = t; best = D2_WORKGROUP; }
   }
-  if (r.us >= 0 && (us < 0 || r.us < us)) best = D2_ROWS;
+  if (r.us >= 0 && (us < 0 || r.us < us) && (!act_order || best == D2_WORKGROUP)) best = D2_ROWS;
   return best;
 }
 
