@@ -56,6 +56,21 @@ def test_scales_and_bias_as_the_tile_kernel(device, dtype, per_row, per_col, bia
         assert torch.equal(_run(a, b, device, dtype, sa, sb, bb), want)
 
 
+@pytest.mark.parametrize("mb,j", [(1, 4), (2, 2), (2, 3), (2, 4), (3, 2), (3, 3), (4, 1), (4, 2), (4, 3)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_one_scale_and_one_step_exact(device, mb, j, bias):
+    """One scale for every row and one for every column, so that all results of a wavefront may share their loads, at K where all wavefronts or the last one with work take
+    a single step: nothing but the wait for the activations stands between the requests and the reads."""
+    from vllm_amd import _tuning
+    for k in (16, 784, 1024, 1280, 1792, 2560, 3328):
+        m, n = 16 * mb - 3, 16 * (3 * j + 1)
+        a, b, want = _case(m, n, k, k + j, device)
+        bb = torch.full((n,), 2.0, dtype=torch.float16, device=device) if bias else None
+        half = torch.full((1, 1), 0.5, device=device)
+        with _tuning.override(exp=[0] * 11 + [j | mb << 4]):
+            assert torch.equal(_run(a, b, device, sa=half, sb=half, bias=bb).cpu().float(), want / 4 + (2 if bias else 0)), (m, n, k)
+
+
 @pytest.mark.parametrize("m,n,k", [(16, 4096, 14336), (17, 1024, 1024), (32, 4096, 4096), (33, 2048, 2048), (64, 1280, 2560), (64, 4096, 4096), (100, 1024, 4096), (128, 2048, 2048),
                                    (200, 1024, 1024), (256, 1024, 4096), (33, 4224, 2256), (48, 1024, 1040), (64, 1344, 3904), (100, 1200, 2320)])
 def test_as_chosen_exact(device, m, n, k):

@@ -36,3 +36,11 @@ def test_descriptors_of_the_w4a16_tile_kernels_end_with_the_last_row(source):
     assert len(spans) == 1
     extent = re.search(r"a_bytes = ([^;]*);", text).group(1) if "a_bytes" in spans[0] else spans[0]
     assert "(uint32_t)(p.M - 1) * (uint32_t)p.lda + (uint32_t)p.K) * 2u" in extent
+
+
+def test_waits_of_the_fp8_kernel_for_some_dozen_rows_leave_only_whole_requests_for_weights_under_way():
+    """What a wait counts on has to be there whatever the compiler makes of it: requests into LDS are, loads of scales that can be one load are not."""
+    with open(os.path.join(CSRC, "fp8_regs_kernel.h")) as f:
+        text = re.sub(r"//[^\n]*", "", f.read())
+    waits = re.findall(r's_waitcnt vmcnt\((%0|\d+)\)"\s*::\s*(?:"n"\(([^"]*)\)\s*:)?', text)
+    assert len(waits) >= 4 and all(counted == "0" or what.strip() == "J * LI" for counted, what in waits), waits

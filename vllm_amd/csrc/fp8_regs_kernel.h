@@ -146,7 +146,7 @@ __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ
 #pragma unroll
   for (int i = 0; i < R; ++i) {
     const int u = w + i * NW, j = u / MB, mb = u - j * MB, n = min(nt0 + j, NT - 1) * 16 + q * 4, m = min(row0 + mb * 16 + r16, M - 1);
-    sam[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsa, p.sa_per_row ? m * 4 : 0, 0, 0));      // (a vector load whatever the scales: counted below)
+    sam[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsa, p.sa_per_row ? m * 4 : 0, 0, 0));
     if (p.sb_per_col) sb4[i] = *reinterpret_cast<const v4f*>(p.sb + n);
     else sb4[i] = v4f{1.f, 1.f, 1.f, 1.f} * p.sb[0];
     bias4[i] = p.bias ? *reinterpret_cast<const v2u*>(p.bias + n) : v2u{0u, 0u};
@@ -165,7 +165,8 @@ __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     tile(1, false, false, 0, 0);
   } else if (g < steps) {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R) : "memory");      // (all but the last of the scales, one load at least for each result)
+    // (all: how many loads the scales and the bias behind the activations have become is the compiler's business)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     tile(0, false, false, 0, 0);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (what is requested past the end writes zeros into LDS)
