@@ -38,9 +38,15 @@ def test_descriptors_of_the_w4a16_tile_kernels_end_with_the_last_row(source):
     assert "(uint32_t)(p.M - 1) * (uint32_t)p.lda + (uint32_t)p.K) * 2u" in extent
 
 
-def test_waits_of_the_fp8_kernel_for_some_dozen_rows_leave_only_whole_requests_for_weights_under_way():
-    """What a wait counts on has to be there whatever the compiler makes of it: requests into LDS are, loads of scales that can be one load are not."""
+def test_waits_of_the_fp8_kernel_for_some_dozen_rows_count_on_loads_that_cannot_be_merged():
+    """What a wait counts on has to be there whatever the compiler makes of it: requests into LDS are, and of the scales the two loads for each of R results whose
+    offsets the compiler cannot see behind the requests for activations."""
     with open(os.path.join(CSRC, "fp8_regs_kernel.h")) as f:
         text = re.sub(r"//[^\n]*", "", f.read())
     waits = re.findall(r's_waitcnt vmcnt\((%0|\d+)\)"\s*::\s*(?:"n"\(([^"]*)\)\s*:)?', text)
-    assert len(waits) >= 4 and all(counted == "0" or what.strip() == "J * LI" for counted, what in waits), waits
+    assert len(waits) >= 4 and all(counted == "0" or what.strip() in ("J * LI", "2 * R") for counted, what in waits), waits
+    loop = text[text.index("load_act(g);"):text.index("vmcnt(%0)\" ::\"n\"(2 * R)")]
+    hidden = re.search(r'asm volatile\("" : ([^;]*)::"memory"\);', loop)
+    assert hidden and all(f'"+v"(at[{i}])' in hidden.group(1) for i in range(3))
+    loads = re.findall(r"raw_buffer_load_b\d+\((\w+), ([^,]*),", loop[hidden.end():])
+    assert loads == [("rsa", "at[0]"), ("rsb", "at[1]"), ("rbias", "at[2]")]
