@@ -50,3 +50,19 @@ def test_waits_of_the_fp8_kernel_for_some_dozen_rows_count_on_loads_that_cannot_
     assert hidden and all(f'"+v"(at[{i}])' in hidden.group(1) for i in range(3))
     loads = re.findall(r"raw_buffer_load_b\d+\((\w+), ([^,]*),", loop[hidden.end():])
     assert loads == [("rsa", "at[0]"), ("rsb", "at[1]"), ("rbias", "at[2]")]
+
+
+@pytest.mark.parametrize("source,requests", [("fp8_scaled_mm.hip", 4), ("fp8_stream2_kernel.h", 1), ("fp8_regs_kernel.h", 2), ("w4a16_prefill_kernel.h", 2), ("w4a16_strip_kernel.h", 1)])
+def test_scalar_offsets_of_requests_into_lds_stay_in_the_operand(source, requests):
+    """A scalar offset past the extent leaves a negative rest to check against: a request's rows are clamped to those that are there where they stand in the
+    scalar offset, and a request for nothing has scalar offset 0 or the extent."""
+    with open(os.path.join(CSRC, source)) as f:
+        text = re.sub(r"//[^\n]*", "", f.read())
+    calls = [c.split("16, ", 1)[1] for c in re.findall(r"raw_ptr_buffer_load_lds\(([^;]*)\);", text)]
+    assert len(calls) == requests
+    by_row = [c for c in calls if re.search(r"lda|ldb|pitch", c)]
+    assert all("min(" in c for c in by_row), by_row
+    named = {"fp8_stream2_kernel.h": ["auto rows_of = [&](int nt) { return (uint32_t)(max(min(nt, nt1 - 1), 0) * 16)", "k_at[st] = (uint32_t)min(kw + st * 256, p.K)"],
+             "fp8_regs_kernel.h": ["const int so = g < steps ? (int)((uint32_t)(min(nt0 + j, NT - 1) * 16)", "g < steps ? g * KT : 0"],
+             "w4a16_strip_kernel.h": ["const uint32_t so = g < g_hi ? (uint32_t)g * 256u + (uint32_t)(h & 1) * 128u : a_bytes;"]}
+    assert all(line in text for line in named.get(source, []))

@@ -67,8 +67,7 @@ __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ
     const int r = i * 4 + q;
     vo_w[i] = (uint32_t)r * ldb + (uint32_t)((r16 ^ r) * 16);
   }
-  // A step past the last has no extent and starts at 0, so that every offset is past the end of it (the check is against the extent less the scalar offset, which is
-  // not to pass below zero): its requests fetch nothing and keep the count of requests under way.
+  // A step past the last has no extent and starts at 0 (vaq_common.h): its requests fetch nothing and keep the count of requests under way.
   auto place = [&](uint32_t vo, int r, int g) {
     if constexpr (TAIL) return g == all - 1 && ((r16 ^ (r & 15)) * 16) >= rest ? 0x80000000u : vo;
     return vo;

@@ -319,13 +319,13 @@ __global__ __launch_bounds__(256) void fp8_mm_tile2_kernel(const Fp8MMParams p) 
     for (int i = 0; i < BM / 32; ++i) {
       const int r0 = wave * (BM / 4) + i * 8;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(Ab + r0 * 128), 16, (int)voff_a,
-                                               (int)((uint32_t)(m0 + r0) * (uint32_t)p.lda + (uint32_t)step * 128u), 0, 0);
+                                               (int)((uint32_t)min(m0 + r0, p.M - 1) * (uint32_t)p.lda + (uint32_t)step * 128u), 0, 0);      // (vaq_common.h)
     }
 #pragma unroll
     for (int i = 0; i < BN / 32; ++i) {
       const int r0 = wave * (BN / 4) + i * 8;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(Bb + r0 * 128), 16, (int)voff_b,
-                                               (int)((uint32_t)(n0 + r0) * (uint32_t)p.ldb + (uint32_t)step * 128u), 0, 0);
+                                               (int)((uint32_t)min(n0 + r0, p.N - 1) * (uint32_t)p.ldb + (uint32_t)step * 128u), 0, 0);
     }
   };
 
@@ -473,14 +473,15 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(VA
   // memory, halves -> lines: 128 x 128 tiles: 5120 x 13824 at M = 250 33.6 -> 31.5 us, 4096 x 28672 at M = 100 30.3 -> 27.7; 64 x 128, 128 x 64, 128 x 256:
   // 2 - 9 %; 64 x 64: 3 - 6 %; 256 x 256: 4096 x 28672 at M = 512 59.1 -> 56.1; from the memory-side cache level.  Pieces of 256 bytes (four slices,
   // half of the rows at a time): -4 .. +3 % against lines; one operand in lines and the other in halves: in between.
-  auto load = [&](auto rows, const __amdgpu_buffer_rsrc_t& r, uint32_t first, uint32_t pitch, uint32_t v0, uint32_t v1, uint32_t koff, uint8_t* at) {
+  // Rows from `last` + 1 on are not there (vaq_common.h): of those that begin at one of them, the first eighth (quarter) of the lanes gets the last row, the others zeros.
+  auto load = [&](auto rows, const __amdgpu_buffer_rsrc_t& r, uint32_t first, uint32_t last, uint32_t pitch, uint32_t v0, uint32_t v1, uint32_t koff, uint8_t* at) {
     constexpr int ROWS = decltype(rows)::value;
     if constexpr (LINE) {
       constexpr int LD = ROWS / (8 * NW);
 #pragma unroll
       for (int i = 0; i < LD; ++i) {
         const int r0 = (wave * LD + i) * 8;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(at + r0 * 128), 16, (int)(i & 1 ? v1 : v0), (int)((first + (uint32_t)r0) * pitch + koff), 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(at + r0 * 128), 16, (int)(i & 1 ? v1 : v0), (int)(min(first + (uint32_t)r0, last) * pitch + koff), 0, 0);
       }
     } else {
       constexpr int LD = ROWS / (16 * NW);
@@ -489,7 +490,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(VA
         const int r0 = (wave * LD + i) * 16;
 #pragma unroll
         for (int c = 0; c < KS; ++c)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(at + (c * ROWS + r0) * 64), 16, (int)v0, (int)((first + (uint32_t)r0) * pitch + koff + 64u * c), 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(at + (c * ROWS + r0) * 64), 16, (int)v0, (int)(min(first + (uint32_t)r0, last) * pitch + koff + 64u * c), 0, 0);
       }
     }
   };
@@ -497,10 +498,10 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void fp8_mm_tile3_kernel(VA
   static_assert(!TAIL || LINE, "chunks past K of single slices are not built");
   auto in_k = [&](uint32_t offset, uint32_t byte) { return !TAIL || byte < (uint32_t)K ? offset : 0x80000000u; };
   auto load_a = [&](uint32_t koff, uint8_t* at) {
-    load(std::integral_constant<int, BM>{}, ra, (uint32_t)m0, lda, in_k(voff_a, koff + lbyte), in_k(voff_a1, koff + (lbyte ^ 32u)), koff, at);
+    load(std::integral_constant<int, BM>{}, ra, (uint32_t)m0, (uint32_t)M - 1u, lda, in_k(voff_a, koff + lbyte), in_k(voff_a1, koff + (lbyte ^ 32u)), koff, at);
   };
   auto load_b = [&](uint32_t koff, uint8_t* at) {
-    load(std::integral_constant<int, BN>{}, rb, (uint32_t)n0, ldb, in_k(voff_b, koff + lbyte), in_k(voff_b1, koff + (lbyte ^ 32u)), koff, at);
+    load(std::integral_constant<int, BN>{}, rb, (uint32_t)n0, (uint32_t)N - 1u, ldb, in_k(voff_b, koff + lbyte), in_k(voff_b1, koff + (lbyte ^ 32u)), koff, at);
   };
   // Steps are requested in order: the first byte of K of the next one, rotation applied.  (As few scalar instructions as can be: the matrix
   // cores wait for them at the start of every step.)
@@ -1157,7 +1158,7 @@ static int dispatch_tile(const Fp8MMParams& p_in, int64_t c_tmp_bytes, int64_t c
       if (p.rotate_k == 0 && pl.sk == 1 && tiles_m <= 2 && pl.tiles * 5 >= cus * 2) p.rotate_k = 2;
       if (tuning().exp[12] == 1) p.rotate_k = 0;      // (development switch: every tile starts at the first K step)
       // A tile row past M.  With at most three tile rows and compute units to spare, one more row of workgroups runs
-      // beside the real ones: its activation rows lie past M (the loads return zeros, nothing is stored), its weight
+      // beside the real ones: its activation rows lie past M (see `load`; nothing is stored), its weight
       // loads are the real tiles' own.  Every weight line is then asked for by two workgroups on two compute units,
       // whichever gets there first, and arrives earlier for the other: what one compute unit has in flight is what bounds
       // a tile's operand stream at these sizes (deeper rings do not help, a second requester does).  Cold, 64 x 64 tiles:

@@ -178,18 +178,22 @@ __global__ __launch_bounds__(512) void fp8_mm_stream2_kernel(VAQ_HEAD_ARGS, cons
     kchunk[i] = (uint32_t)(((lane & 15) ^ row) * 16);
     voffb[i] = (uint32_t)row * (uint32_t)p.ldb + kchunk[i];
   }
-  // `live` = false requests nothing (offsets beyond the extent) but keeps the count of loads in flight the same
-  auto issue_stage = [&](int nt, int st, int slot, bool live) {
+  // `live` = false requests nothing (offsets beyond the extent) but keeps the count of loads in flight the same, and so does a stage past K.  (The scalar offset stays in the
+  // operand: vaq_common.h.)
+  uint32_t k_at[NS];
+#pragma unroll
+  for (int st = 0; st < NS; ++st) k_at[st] = (uint32_t)min(kw + st * 256, p.K);
+  auto rows_of = [&](int nt) { return (uint32_t)(max(min(nt, nt1 - 1), 0) * 16) * (uint32_t)p.ldb; };
+  auto issue_stage = [&](uint32_t rows, int st, int slot, bool live) {
     const int k0 = kw + st * 256;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const uint32_t vo = (live && k0 + (int)kchunk[i] < p.K) ? voffb[i] : OOB;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(ring + slot * 4096 + i * 1024), 16, (int)vo,
-                                               (int)((uint32_t)(nt * 16) * (uint32_t)p.ldb + (uint32_t)k0), 0, 2);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(ring + slot * 4096 + i * 1024), 16, (int)vo, (int)(rows + k_at[st]), 0, 2);
     }
   };
 #pragma unroll
-  for (int st = 0; st < NSR; ++st) issue_stage(nt0, st, st, nt0 < nt1);
+  for (int st = 0; st < NSR; ++st) issue_stage(rows_of(nt0), st, st, nt0 < nt1);
   // (M = 16 on 4096 x 6144 7.08 -> 6.88 us, M = 7 on 4096 x 4096 5.36 -> 5.07, 5.21 with the wait ahead of the loop below.  Quantised here it is there: a given
   // scale's own load would come behind it, 4096 x 6144 at M = 8 7.02 -> 8.02.)
   if constexpr (MQ == 0) VAQ_ARRIVED4(p.sb, p.bias, p.out, p.sb_per_col);
@@ -321,8 +325,8 @@ __global__ __launch_bounds__(512) void fp8_mm_stream2_kernel(VAQ_HEAD_ARGS, cons
       }
       // the slot is free once its operands are in registers: request the stage NSR ahead into it
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      if (st + NSR < NS) issue_stage(nt, st + NSR, slot, true);
-      else issue_stage(nt + 1, st + NSR - NS, slot, nt + 1 < nt1);
+      if (st + NSR < NS) issue_stage(rows_of(nt), st + NSR, slot, true);
+      else issue_stage(rows_of(nt + 1), st + NSR - NS, slot, nt + 1 < nt1);
     }
 
     v4f tot = v4f{0.f, 0.f, 0.f, 0.f};

@@ -533,9 +533,9 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void w4a16_prefill2_kernel(
     uint8_t* Ab = lds8 + (size_t)buf * A_ST;
 #pragma unroll
     for (int i = 0; i < A_LD; ++i) {
-      const int r0 = (wave * A_LD + i) * 8;
+      const int r0 = (wave * A_LD + i) * 8;      // (rows past M count as the last one: vaq_common.h)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(Ab + r0 * 128), 16, (int)voff_a[i],
-                                               (int)(((uint32_t)(m0 + r0) * (uint32_t)p.lda + (uint32_t)step * 64u) * 2u), 0, 0);
+                                               (int)(((uint32_t)min(m0 + r0, p.M - 1) * (uint32_t)p.lda + (uint32_t)step * 64u) * 2u), 0, 0);
     }
   };
 
@@ -631,7 +631,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void w4a16_prefill2_kernel(
     uint8_t* Ab = lds8 + (size_t)buf * A_ST;
     const int r0 = (wave * A_LD + i) * 8;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(Ab + r0 * 128), 16, (int)voff_a[i],
-                                             (int)(((uint32_t)(m0 + r0) * (uint32_t)p.lda + (uint32_t)step * 64u) * 2u), 0, 0);
+                                             (int)(((uint32_t)min(m0 + r0, p.M - 1) * (uint32_t)p.lda + (uint32_t)step * 64u) * 2u), 0, 0);
   };
 
   v16f acc[WMB][WNB];
