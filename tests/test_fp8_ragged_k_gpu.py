@@ -59,8 +59,8 @@ def test_as_chosen_exact(device, m, n, k):
 
 
 def test_operands_beyond_2_gib(device):
-    """Rows so far apart that a place in the operand does not leave room for the offset of a chunk past K: K % 128 = 64 takes the tile that
-    steps by 64, other K the kernel that tests every load."""
+    """Rows so far apart that a place in the operand does not leave room for the offset of a chunk past K: K % 128 = 64 takes the tiles by slices
+    of 64 bytes, other K the kernel that tests every load."""
     for k in (192, 208):
         m, n, pitch = 70, 64, 32 << 20
         g = torch.Generator().manual_seed(k)
@@ -69,3 +69,25 @@ def test_operands_beyond_2_gib(device):
         wide[:, :k] = x.to(torch.float8_e4m3fn).to(device)
         assert torch.equal(_run(wide[:, :k], w.to(torch.float8_e4m3fn).to(device).t(), device), x @ w.t()), k
         del wide
+
+
+@pytest.mark.parametrize("rows_far", ["activations", "weights"])
+def test_every_tile_shape_beyond_2_gib(device, rows_far):
+    """K % 128 = 64 on operands of 2 .. 4 GiB: every shape by slices of 64 bytes (and the 256 x 256 tile), whole and in parts of K, as chosen too."""
+    from vllm_amd import _tuning
+    pitch = 48 << 20
+    k, m, n = 192 + 128 * 4, *((70, 336) if rows_far == "activations" else (300, 80))
+    g = torch.Generator().manual_seed(k + m)
+    x, w = torch.randint(-2, 3, (m, k), generator=g).float(), torch.randint(-1, 2, (n, k), generator=g).float()
+    want = x @ w.t()
+    views = [t.to(torch.float8_e4m3fn).to(device) for t in (x, w)]
+    far = 0 if rows_far == "activations" else 1
+    wide = torch.empty(views[far].shape[0] * pitch, dtype=torch.uint8, device=device).view(torch.float8_e4m3fn).view(-1, pitch)
+    wide[:, k:k + 128] = torch.full((1,), 0x7f, dtype=torch.uint8, device=device).view(torch.float8_e4m3fn)
+    wide[:, :k] = views[far]
+    views[far] = wide[:, :k]
+    assert torch.equal(_run(views[0], views[1].t(), device), want)
+    for cfg in (1, 3, 4, 5, 6, 7, 9, 13, 14, 15, 16, 17, 19):
+        for split in (1, 2):
+            with _tuning.override(fp8_path=2, fp8_tile_cfg=cfg, fp8_split=split):
+                assert torch.equal(_run(views[0], views[1].t(), device), want), (cfg, split)

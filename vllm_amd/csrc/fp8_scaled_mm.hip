@@ -1116,19 +1116,14 @@ static int dispatch_tile(const Fp8MMParams& p_in, int64_t c_tmp_bytes, int64_t c
   // 256 x 256 tile requests 128 bytes where K leaves 64.
   p.a_extent = (uint32_t)((int64_t)(p.M - 1) * p.lda + p.K);
   p.b_extent = (uint32_t)((int64_t)(p.N - 1) * p.ldb + p.K);
-  // A step that ends past K: no place of a request, rows past M and N among them, may be beyond 2 GiB, so that it and the offset of a chunk past K do
-  // not wrap.
-  const bool far = ((uint64_t)p.M + 512) * (uint64_t)p.lda >= (1ull << 31) || ((uint64_t)p.N + 512) * (uint64_t)p.ldb >= (1ull << 31);
+  // A step that ends past K: the offset of a chunk past K, 2 GiB, has to be past the operand's end, and its sum with a place in the operand may not wrap.
+  const bool far = (uint64_t)(p.M - 1) * (uint64_t)p.lda + (uint64_t)p.K >= (1ull << 31) || (uint64_t)(p.N - 1) * (uint64_t)p.ldb + (uint64_t)p.K >= (1ull << 31);
   const bool direct_ok = tuning().fp8_tile_impl == 0 && (uint64_t)p.M * (uint64_t)p.lda < (1ull << 32) && (uint64_t)p.N * (uint64_t)p.ldb < (1ull << 32) &&
                          (p.K % 64 == 0 || !far);
   if (direct_ok && tuning().fp8_tile_impl == 0 && tuning().fp8_tile_cfg >= 0) {
     TilePlan pl = plan_tile3(p.M, p.N, p.K);
-    if (pl.id > 10 && p.K % 128 == 64 && far) {      // (the 256 x 256 tile steps by 64 bytes)
-      pl = TilePlan();
-      pl.id = 1;
-      pl.bm = pl.bn = 256;
-      pl.tiles = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256);
-    }
+    const bool half_step = pl.id > 10 && p.K % 128 != 0;      // K ends inside a step of 128 bytes (the 256-wide tiles step by 64)
+    if (half_step && far) pl.id -= 10;                        // (K % 64 = 0: the same tile by slices of 64 bytes)
     // without (enough) scratch from the caller the unsplit kernel still gives the result
     if (pl.sk > 1 && (p.c_tmp == nullptr || p.counters == nullptr || counter_ints < pl.counter_ints() ||
                       c_tmp_bytes < pl.tmp_bytes()))
@@ -1172,20 +1167,18 @@ static int dispatch_tile(const Fp8MMParams& p_in, int64_t c_tmp_bytes, int64_t c
         p.rotate_k = 0;
       }
     }
-    // K in steps of 128 bytes (the 256-wide tiles: of 64) ends inside the last one.  All K that are no multiple of 64 once went through registers and padded LDS:
-    // 80 drawn problems of 33 .. 8192 rows take 0.56 of that time in the mean (126 rows of 8400 x 4096 59.5 -> 22.0 us, 1700 of 5968 x 2368 52.4 -> 50.8); K % 128 = 64
-    // went by slices of 64, half a cache line: 90 problems 0.95 (232 rows of 13632 x 25280 163 -> 136 us, the worst 198 of 1472 x 5632 8.7 -> 9.2).
-    if (p.K % 64 != 0 || (p.K % 128 != 0 && pl.id > 10)) switch (pl.id) {
-        case 1: return launch_tile3<BF16_OUT, 256, 256, 2, 4, 5, 1, 2, true>(p, s);
-        case 13: return launch_tile3<BF16_OUT, 128, 128, 2, 4, 4, 2, 0, true>(p, s);
-        case 14: return launch_tile3<BF16_OUT, 64, 128, 2, 2, 5, 2, 0, true>(p, s);
-        case 15: return launch_tile3<BF16_OUT, 64, 64, 2, 2, 5, 2, 0, true>(p, s);
-        case 16: return launch_tile3<BF16_OUT, 128, 64, 2, 2, 5, 2, 0, true>(p, s);
-        case 17: return launch_tile3<BF16_OUT, 128, 256, 2, 4, 3, 2, 0, true>(p, s);
-        case 19: return launch_tile3<BF16_OUT, 256, 128, 4, 2, 3, 2, 0, true>(p, s);
-        default: break;
-      }
-    else switch (pl.id) {
+    // All K that are no multiple of 64 once went through registers and padded LDS: 80 drawn problems of 33 .. 8192 rows take 0.56 of that time in the mean (126 rows of
+    // 8400 x 4096 59.5 -> 22.0 us, 1700 of 5968 x 2368 52.4 -> 50.8); K % 128 = 64 went by slices of 64, half a cache line: 90 problems 0.95 (232 rows of 13632 x 25280
+    // 163 -> 136 us, the worst 198 of 1472 x 5632 8.7 -> 9.2), and does so where an operand ends beyond 2 GiB.
+    const bool tail = p.K % 64 != 0 || (half_step && !far);
+    switch (tail ? -pl.id : pl.id) {
+      case -1: return launch_tile3<BF16_OUT, 256, 256, 2, 4, 5, 1, 2, true>(p, s);
+      case -13: return launch_tile3<BF16_OUT, 128, 128, 2, 4, 4, 2, 0, true>(p, s);
+      case -14: return launch_tile3<BF16_OUT, 64, 128, 2, 2, 5, 2, 0, true>(p, s);
+      case -15: return launch_tile3<BF16_OUT, 64, 64, 2, 2, 5, 2, 0, true>(p, s);
+      case -16: return launch_tile3<BF16_OUT, 128, 64, 2, 2, 5, 2, 0, true>(p, s);
+      case -17: return launch_tile3<BF16_OUT, 128, 256, 2, 4, 3, 2, 0, true>(p, s);
+      case -19: return launch_tile3<BF16_OUT, 256, 128, 4, 2, 3, 2, 0, true>(p, s);
       case 1: return launch_tile3<BF16_OUT, 256, 256, 2, 4, 5, 1, 2>(p, s);    // alternating phases, slices requested in pairs (see the kernel)
       case 10: return launch_tile3<BF16_OUT, 256, 384, 2, 4, 4, 1, 1>(p, s);   // 8 wavefronts of 128 x 96, alternating phases, one slice at a time
       // two k-slices per step
@@ -1195,6 +1188,13 @@ static int dispatch_tile(const Fp8MMParams& p_in, int64_t c_tmp_bytes, int64_t c
       case 16: return launch_tile3<BF16_OUT, 128, 64, 2, 2, 5, 2>(p, s);
       case 17: return launch_tile3<BF16_OUT, 128, 256, 2, 4, 3, 2>(p, s);
       case 19: return launch_tile3<BF16_OUT, 256, 128, 4, 2, 3, 2>(p, s);
+      // one
+      case 3: return launch_tile3<BF16_OUT, 128, 128, 2, 4, 5>(p, s);
+      case 4: return launch_tile3<BF16_OUT, 64, 128, 2, 2, 5>(p, s);
+      case 5: return launch_tile3<BF16_OUT, 64, 64, 2, 2, 5>(p, s);
+      case 6: return launch_tile3<BF16_OUT, 128, 64, 2, 2, 5>(p, s);
+      case 7: return launch_tile3<BF16_OUT, 128, 256, 2, 4, 5>(p, s);
+      case 9: return launch_tile3<BF16_OUT, 256, 128, 4, 2, 5>(p, s);
       default: break;
     }
   }
