@@ -123,7 +123,7 @@ int vaq_w4a16_gemm_workspace_of_format(int64_t size_m, int64_t size_n, int64_t s
  * be ahead into the end of `c_tmp`, and a call that brings less `c_tmp` than the workspace query says gathers inside the decode kernel.
  * Scratch: `c_tmp` holds at least `c_tmp_bytes` bytes and `counters` at least `counter_ints` zeroed ints; a call whose
  * kernel needs more than it was given returns VAQ_ERR_INVALID_ARG (sizes: vaq_w4a16_gemm_workspace, or
- * vaq_w4a16_gemm_workspace_of_format) and launches nothing.
+ * vaq_w4a16_gemm_workspace_of_format) and launches nothing (with act_order beyond 32 rows: nothing but the permutation into `a_tmp`).
  * One use of `c_tmp` is optional: at thousands of rows, 256 x 256 tiles that end in a round of workgroups at most half
  * full run the tiles of that round in K parts when `c_tmp` holds their partial tiles, and whole (same result, slower)
  * when it does not -- the workspace query reports the size with that use included.

@@ -79,27 +79,39 @@ def _c_call(lib, _lib, layer, x, c_tmp, a_tmp, counters):
     return rc, out
 
 
-@pytest.mark.parametrize("m", [8, 16, 32])
-def test_callers_without_room_for_permuted_columns(device, m):
-    """Up to 32 rows the gather inside the kernel is left for a caller whose scratch has no room for the columns, down to what that kernel
-    itself needs; what is written behind the scratch would show."""
+@pytest.mark.parametrize("m,k,n", [(8, 4096, 4096), (16, 4096, 4096), (32, 4096, 4096), (8, 14336, 4096), (16, 14336, 4096), (32, 14336, 1024)])
+def test_callers_without_room_for_permuted_columns(device, m, k, n):
+    """Up to 32 rows the gather inside the kernel is left for a caller whose scratch has no room for the columns and what the call needs behind them, down to what
+    that kernel itself needs; below both a call is refused and launches nothing.  What is written behind the scratch would show."""
     from vllm_amd import _lib
     lib = _lib.load()
-    layer = _layer(4096, 4096, 128, 4, False, device)
-    x = _x(m, 4096, device)
+    layer = _layer(k, n, 128, 4, False, device)
+    x = _x(m, k, device)
     want = layer(x)
     sizes = [ctypes.c_size_t() for _ in range(3)]
-    _lib.check(lib.vaq_w4a16_gemm_workspace_of_format(m, layer.n, layer.k, layer.g, _lib.VAQ_WTYPE_U4B8, 1, 0, *map(ctypes.byref, sizes)))
-    asked = sizes[0].value // 4
-    assert sizes[0].value >= 2 * m * layer.k and sizes[1].value == 0
-    counters = torch.zeros(max(sizes[2].value, 1), dtype=torch.int32, device=device)
-    for ints in (asked, asked + 1, asked - 1, asked // 2):
-        buf = torch.full((ints + 64,), 7.0, dtype=torch.float32, device=device)
-        rc, out = _c_call(lib, _lib, layer, x, buf[:ints], None, counters)
-        assert rc == (_lib.VAQ_OK if ints >= asked else rc) and (rc != _lib.VAQ_OK or torch.equal(out, want)), ints
-        assert bool((buf[ints:] == 7.0).all()) and bool((counters == 0).all())
+    _lib.check(lib.vaq_w4a16_gemm_workspace_of_format(m, n, k, layer.g, _lib.VAQ_WTYPE_U4B8, 1, 0, *map(ctypes.byref, sizes)))
+    asked, ints = sizes[0].value // 4, max(sizes[2].value, 1)
+    assert sizes[0].value >= 2 * m * k and sizes[1].value == 0
+    # float32s of scratch: of the kernel that gathers, by its parts of K, and with the columns ahead of them of what runs without act_order
+    plan, regs = (ctypes.c_double * 6)(), (ctypes.c_double * 7)()
+    _lib.check(lib.vaq_w4a16_decode_plan(m, n, k, 1, 0, 0, plan))
+    _lib.check(lib.vaq_w4a16_regs_plan(m, n, k, 1, 0, regs))
+    tile = lambda parts, blocks: int(parts) * (n // 16) * blocks * 256 if parts > 1 else 0
+    columns, gathered = m * k // 2, tile(plan[3], (m + 15) // 16)
+    regs_rows = -(-m // (16 * int(regs[1]))) * int(regs[1])
+    permuted = columns + min(gathered, tile(regs[3], regs_rows) if regs[6] else gathered)
+    need = min(gathered, permuted)
+    assert need < asked
+    counters = torch.zeros(ints, dtype=torch.int32, device=device)
+    given = {asked, asked + 1, asked - 1, asked // 2, columns, columns + 4, columns - 1, permuted, permuted - 1, gathered, need + 1, need - 1, need // 2}
+    for count in sorted(c for c in given if c >= 0):
+        buf = torch.full((count + 64,), 7.0, dtype=torch.float32, device=device)
+        rc, out = _c_call(lib, _lib, layer, x, buf[:count], None, counters)
+        assert rc == (_lib.VAQ_OK if count >= need else _lib.VAQ_ERR_INVALID_ARG), (count, need, asked)
+        assert bool((buf[count if rc == _lib.VAQ_OK else 0:] == 7.0).all()) and bool((counters == 0).all())
+        assert rc != _lib.VAQ_OK or torch.equal(out, want), count
     rc, out = _c_call(lib, _lib, layer, x, None, None, counters)
-    assert rc in (_lib.VAQ_OK, _lib.VAQ_ERR_INVALID_ARG) and (rc != _lib.VAQ_OK or torch.equal(out, want))
+    assert rc == (_lib.VAQ_ERR_INVALID_ARG if need else _lib.VAQ_OK) and (need or torch.equal(out, want))
 
 
 def test_replayed_graph(device):

@@ -140,6 +140,19 @@ static bool permutes_first(int M, int N, int K, int sub, bool w8) {
   }) != 0;
 }
 
+// Whether `bytes` of partial tiles and `ints` counters are enough for a call of up to 32 rows without act_order.
+static bool small_call_fits(int M, int N, int K, int sub, int wt, int64_t bytes, int64_t ints) {
+  size_t t = 0, n = 0;
+  auto fits = [&] { return bytes >= (int64_t)t && ints >= (int64_t)n; };
+  if (regs_chosen(M, N, K, sub, wt)) {
+    w4a16_regs_workspace(M, N, K, sub, wt != 0, &t, &n);
+    if (fits()) return true;
+  }
+  if (decode_impl_for(M, N, K, sub, wt != 0) == 1) w4a16_decode_workspace(M, N, K, &t, &n);
+  else w4a16_decode2_workspace(M, N, K, sub, wt != 0, &t, &n);
+  return fits();
+}
+
 // Scratch of a problem, enough for whichever kernel runs (that also depends on the row stride of A): for one weight format, or with
 // wt < 0 for any of them.
 static int scratch_of(int64_t size_m, int64_t size_n, int64_t size_k, bool has_perm, int wt, int sub, size_t* c_tmp_bytes,
@@ -326,19 +339,20 @@ extern "C" int vaq_w4a16_gemm_tuned(const void* a, int64_t lda, const int32_t* b
   hipStream_t s = (hipStream_t)stream;
 
   if (perm && force_path == 0 && size_m * lda * 2 < (1ll << 31) && permutes_first((int)size_m, (int)size_n, (int)size_k, sub, w8)) {
-    // into a_tmp beyond 32 rows, and into the end of c_tmp up to there
+    // into a_tmp beyond 32 rows, and into the end of c_tmp up to there, where what is left of it is enough for the call without act_order
     int64_t left = c_tmp_bytes;
     void* columns = a_tmp;
     if (size_m <= DECODE_MAX_M_2BLK) {
       left = (c_tmp_bytes - size_m * size_k * 2) & ~15ll;
-      columns = c_tmp != nullptr && left >= 0 ? reinterpret_cast<char*>(c_tmp) + left : nullptr;
+      columns = c_tmp != nullptr && left >= 0 && small_call_fits((int)size_m, (int)size_n, (int)size_k, sub, wt, left, counters != nullptr ? counter_ints : 0)
+                    ? reinterpret_cast<char*>(c_tmp) + left : nullptr;
     }
     if (columns != nullptr && ((uintptr_t)columns % 16) == 0) {
       rc = vaq_permute_cols(a, lda, perm, columns, size_m, size_k, stream);
       if (rc != VAQ_OK) return rc;
       rc = dispatch(columns, size_k, b, scales, zeros, nullptr, true, bias, c, left > 0 ? c_tmp : nullptr, left, a_tmp, counters, counter_ints, size_m, size_n,
                     size_k, sub, channelwise, wt, dtype, 0, s);
-      if (rc != VAQ_ERR_INVALID_ARG) return rc;      // (given too little scratch for that plan: as without it)
+      if (rc != VAQ_ERR_INVALID_ARG) return rc;      // (beyond 32 rows, given too little scratch for that plan: as without it)
     }
   }
   return dispatch(a, lda, b, scales, zeros, perm, perm != nullptr, bias, c, c_tmp, c_tmp_bytes, a_tmp, counters, counter_ints, size_m, size_n, size_k,
