@@ -78,8 +78,13 @@ static double regs_lead(int M, int N, int K, int sub, int wt, int j, int nw) {
   // vocabulary-sized layers at 3 .. 16 rows, where another kernel is the alternative (it takes them all: 0.37 .. 0.96 of the time, 1 of 2000 more than 3 % slower;
   // 4096 x 128256 at M = 4 / 16 54.9 / 59.0 -> 51.9 / 53.4 us, 1024 x 128256 33.4 / 34.0 -> 18.1 / 19.5, 5120 x 65536 80.0 / 81.0 -> 33.2 / 34.7)
   if (wt == 0 && decode_impl_for(M, N, K, sub, false) == 1) return 0.95;
-  const double lead = SHARE[wt != 0 ? 3 : sub == 1 ? 0 : sub == 2 ? 1 : 2][M <= 1 ? 0 : M <= 4 ? 1 : M <= 16 ? 2 : M <= 32 ? 3 : M <= 64 ? 4 : 5];
+  double lead = SHARE[wt != 0 ? 3 : sub == 1 ? 0 : sub == 2 ? 1 : 2][M <= 1 ? 0 : M <= 4 ? 1 : M <= 16 ? 2 : M <= 32 ? 3 : M <= 64 ? 4 : 5];
   if (wt != 0 || sub > 1 || M > 32) return lead;
+  // One n-tile to a wavefront, N from 2048 on, at 2 .. 4 rows: where eight slices of four or of eight k-tiles fill K to nine tenths the decode kernel's plan leaves nobody idle and is up to
+  // 13 % cheaper than priced.  333 problems of K 3200 .. 8192, both timed: at 0.95 the choice takes 1.019 of the faster one's time and 79 calls here are more than 3 % slower
+  // (7040 x 2560 at M = 2 5.7 us, 5.0 there); so 1.004 and 12, the 83 that go back take 0.942 of their time, one 1.05.
+  const int tiles = K / 128;
+  if (M > 1 && M <= 4 && j == 1 && N >= 2048 && ((tiles > 28 && tiles <= 32) || (tiles > 49 && tiles <= 64)) && lead > 0.84) lead = 0.84;
   // Where this kernel loses most of what it loses, by as much as the two prices together are off by: K of whole 1024 rows; one n-tile to a wavefront and K
   // beyond 8192 at up to 4 rows; two and more n-tiles on a short K.  Off are: this kernel's price, which counts 16 rows to a block, by the rows that a block has;
   // for workgroups of four; for one n-tile, which leaves 2 KB of weights in flight, by how much of the device waits for them and how long; for three and more
