@@ -1400,7 +1400,9 @@ static bool takes_regs(int M, int N, int K, Fp8RegsPlan* plan, double* other) {
     const double k = K / 1024.0, act = 0.349 * M / 16 * k * (1 + 0.0311 * k), rounds = ceil(N / 16.0 / num_cus_current_device());
     const double core = 0.372 * rounds * k + act, mem = 0.137e-6 * K * N;
     *other = 2.3 + cbrt(core * core * core + mem * mem * mem) + 0.304 * 2e-6 * M * N;
-    return M > 4 && plan->us < (M <= 16 ? 1.03 : N <= 12288 ? 1.1 : 1.0) * *other;
+    // (17 .. 32 rows of K 1537 .. 3072: 0.98.  378 problems of K 1024 .. 6144, both timed: at 1.1 throughout the choice takes 1.0078 of the faster one's time and 44 calls here are more than 3 %
+    // slower, 27 of them on that K (2976 x 10240 at M = 22 9.6 us, 8.4 there; 2064 x 7104 at M = 30 6.4, 5.8); so 1.0049 and 25.)
+    return M > 4 && plan->us < (M <= 16 ? 1.03 : N > 12288 ? 1.0 : K > 1536 && K <= 3072 ? 0.98 : 1.1) * *other;
   }
   *other = plan_tile3(M, N, K).us;
   return M > 4 && plan->us < 0.93 * *other;
