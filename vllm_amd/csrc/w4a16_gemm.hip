@@ -46,8 +46,9 @@ static int check_format(int64_t size_k, int group_size, int wtype, int* wt, int*
   return VAQ_OK;
 }
 
-// What takes a problem of up to 256 rows without act_order where the kernel with activations in registers does not, and its predicted time.
-static int other_kind(int M, int N, int K, int sub, int wt, double* us) {
+// What takes a problem of up to 256 rows where the kernel with activations in registers does not, and its predicted time; with `act_order` beyond 32 rows, the columns
+// permuted: workgroups of 16 rows take few of those (w4a16_decode2_choose).
+static int other_kind(int M, int N, int K, int sub, int wt, bool act_order, double* us) {
   const bool w8 = wt != 0, plain = sub == 1 && !w8;
   int kind = D2_WORKGROUP;
   // 3 .. 16 rows of a vocabulary-sized layer: the register-resident kernel.  A launch, for every 1000 columns its walk, the weights, and those times the
@@ -58,7 +59,7 @@ static int other_kind(int M, int N, int K, int sub, int wt, double* us) {
   }
   if (M > 16) {
     const int most = !plain ? DECODE_MAX_M_2BLK : N > 8192 ? 48 : DECODE_MAX_M;
-    kind = w4a16_decode2_choose(M, N, K, sub, wt, false, false, M <= most, true, w4a16_staged_us(M, N, K, plain));
+    kind = w4a16_decode2_choose(M, N, K, sub, wt, act_order && M > DECODE_MAX_M_2BLK, false, M <= most, true, w4a16_staged_us(M, N, K, plain));
   }
   *us = kind == D2_TILE ? w4a16_tile_us(M, N, K, tile_format(sub, wt)) : w4a16_decode2_us(M, N, K, sub, w8, kind == D2_ROWS);
   return kind;
@@ -99,12 +100,12 @@ static double regs_lead(int M, int N, int K, int sub, int wt, int j, int nw) {
   const double by_price = exp(-0.01 - off);
   return lead < by_price ? lead : by_price;
 }
-bool w4a16_takes_regs(int M, int N, int K, int sub, int wt, double* other) {
+bool w4a16_takes_regs(int M, int N, int K, int sub, int wt, double* other, bool act_order) {
   const TuningScope automatic(nullptr);
   int j = 0, nw = 0;
   const double us = w4a16_regs_us(M, N, K, sub, wt, &j, &nw);
   if (us < 0) return false;
-  other_kind(M, N, K, sub, wt, other);
+  other_kind(M, N, K, sub, wt, act_order, other);
   return us < *other * regs_lead(M, N, K, sub, wt, j, nw);
 }
 
@@ -115,14 +116,14 @@ static bool plan_named(const VaqTuning& tn) {
 }
 
 // The same for a call, from a table per thread.  A switch that names another kernel or a plan of one keeps it out; exp[8] asks for it.
-static bool regs_chosen(int M, int N, int K, int sub, int wt) {
+static bool regs_chosen(int M, int N, int K, int sub, int wt, bool act_order) {
   const VaqTuning& tn = tuning();
   if (M < 1 || M > REGS_MAX_M || N >= (1 << 24) || K >= (1 << 24) || tn.exp[8] == 1) return false;
   if (tn.exp[8] > 1) return w4a16_regs_us(M, N, K, sub, wt) >= 0;
   if (plan_named(tn)) return false;
   static thread_local PlanTable<int> table;
   double other;
-  return table.get(M, N, K, (num_cus_current_device() * 8 + sub) * 4 + wt, [&] { return w4a16_takes_regs(M, N, K, sub, wt, &other) ? 1 : 0; }) != 0;
+  return table.get(M, N, K, (num_cus_current_device() * 8 + sub) * 8 + wt * 2 + act_order, [&] { return w4a16_takes_regs(M, N, K, sub, wt, &other, act_order) ? 1 : 0; }) != 0;
 }
 
 // Whether act_order's columns are permuted by a launch of their own ahead of the kernels with activations in registers and the decode kernels too,
@@ -145,11 +146,11 @@ static bool permutes_first(int M, int N, int K, int sub, bool w8) {
   }) != 0;
 }
 
-// Whether `bytes` of partial tiles and `ints` counters are enough for a call of up to 32 rows without act_order.
+// Whether `bytes` of partial tiles and `ints` counters are enough for a call of up to 32 rows with act_order whose columns are permuted.
 static bool small_call_fits(int M, int N, int K, int sub, int wt, int64_t bytes, int64_t ints) {
   size_t t = 0, n = 0;
   auto fits = [&] { return bytes >= (int64_t)t && ints >= (int64_t)n; };
-  if (regs_chosen(M, N, K, sub, wt)) {
+  if (regs_chosen(M, N, K, sub, wt, true)) {
     w4a16_regs_workspace(M, N, K, sub, wt != 0, &t, &n);
     if (fits()) return true;
   }
@@ -199,7 +200,7 @@ static int scratch_of(int64_t size_m, int64_t size_n, int64_t size_k, bool has_p
     for (int w : {0, 1}) {
       if (size_m == 0 || (wt >= 0 && (s != sub || w != wt)) || (has_perm && !permutes_first(M, N, K, s, w == 1))) continue;
       if (has_perm && size_m <= DECODE_MAX_M_2BLK) columns = (size_t)size_m * (size_t)size_k * 2;
-      if (size_m > REGS_MAX_M || !regs_chosen(M, N, K, s, w)) continue;
+      if (size_m > REGS_MAX_M || !regs_chosen(M, N, K, s, w, has_perm)) continue;
       w4a16_regs_workspace(M, N, K, s, w == 1, &t, &n);
       take(t, n);
     }
@@ -216,7 +217,7 @@ static int dispatch(const void* a, int64_t lda, const int32_t* b, const void* sc
   // The kernel with operands in registers first: a call that it takes looks up none of the other plans.  (One that brings too little scratch for its parts of K
   // goes on to the others; so does one whose rows end beyond 2 GiB.)
   if (force_path == 0 && perm == nullptr && size_m <= REGS_MAX_M && size_m * lda * 2 < (1ll << 31) &&
-      regs_chosen((int)size_m, (int)size_n, (int)size_k, sub, wt)) {
+      regs_chosen((int)size_m, (int)size_n, (int)size_k, sub, wt, act_order)) {
     size_t t = 0, n = 0;
     w4a16_regs_workspace((int)size_m, (int)size_n, (int)size_k, sub, w8, &t, &n);
     if ((t == 0 && n == 0) || (c_tmp != nullptr && counters != nullptr && (uintptr_t)c_tmp % 16 == 0 && c_tmp_bytes >= (int64_t)t && counter_ints >= (int64_t)n))

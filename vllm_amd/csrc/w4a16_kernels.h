@@ -32,7 +32,7 @@ int w4a16_decode2_launch(const void* a, int64_t lda, const int32_t* b, const voi
 // does not take the problem), scratch, launch.
 constexpr int REGS_MAX_M = 256;
 double w4a16_regs_us(int M, int N, int K, int sub, int wt, int* n_tiles = nullptr, int* wavefronts = nullptr);      // ... of its plan
-bool w4a16_takes_regs(int M, int N, int K, int sub, int wt, double* other);      // w4a16_gemm.hip; *other: predicted time of what takes it otherwise
+bool w4a16_takes_regs(int M, int N, int K, int sub, int wt, double* other, bool act_order = false);      // w4a16_gemm.hip; *other: predicted time of what takes it otherwise
 void w4a16_regs_workspace(int M, int N, int K, int sub, bool w8, size_t* c_tmp_bytes, size_t* counter_ints);
 int w4a16_regs_launch(const void* a, int64_t lda, const int32_t* b, const void* scales, const int32_t* zeros, const void* bias, void* c,
                       float* c_tmp, int32_t* counters, int M, int N, int K, int sub, bool channelwise, bool w8, int dtype, hipStream_t s);
