@@ -1,10 +1,37 @@
 """Divisions that the kernels make by multiplication with a number from the host (tile_handover.h, w4a16_regs_kernel.h)."""
 from __future__ import annotations
 
+import os
+import shutil
+import subprocess
+
 import numpy as np
 import pytest
 
-from vllm_amd.build import HIPCC_FLAGS
+from vllm_amd.build import CSRC, HIPCC_FLAGS
+
+CHECK = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "launch_arguments_check.hip")
+
+
+@pytest.fixture(scope="module")
+def launch_check(tmp_path_factory):
+    """The functions that the kernels find their work by, compiled for the host (native/launch_arguments_check.hip)."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    exe = str(tmp_path_factory.mktemp("launch") / "launch_arguments_check")
+    subprocess.run([hipcc, "--offload-host-only", "-O1", "-std=c++17", "-w", "-I", str(CSRC), CHECK, "-o", exe], check=True)
+    return exe
+
+
+def test_every_workgroup_finds_its_work(launch_check):
+    r = subprocess.run([launch_check], capture_output=True, text=True)
+    assert r.returncode == 0 and "mismatches=0" in r.stdout, r.stdout
+
+
+@pytest.mark.parametrize("mistake", [1, 2, 3, 4])
+def test_and_the_check_can_fail(launch_check, mistake):
+    """A wrong number for bands of tiles, for copies of a range, for blocks of rows, for parts of K."""
+    r = subprocess.run([launch_check, str(mistake)], capture_output=True, text=True)
+    assert r.returncode == 1 and "mismatches=" in r.stdout
 
 
 @pytest.mark.parametrize("d", [1, 2, 3, 4, 5, 7, 8, 12, 96, 255, 256, 1000, 9504, 65535, 65536, 1 << 20, (1 << 31) - 1, 1 << 31])

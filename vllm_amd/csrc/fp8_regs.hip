@@ -46,11 +46,10 @@ static bool launch(const Fp8MMParams& p_in, hipStream_t s) {
   auto kern = fp8_mm_regs_kernel<BF16_OUT, MB, J, TAIL>;
   static size_t reserved[VAQ_MAX_DEVICES];
   if (reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds, reserved, "fp8_scaled_mm") != VAQ_OK) return false;
-  // (unit / RB by multiplication: exact for unit * RB < 2^32)
   const uint32_t steps = ((uint32_t)p.K + FP8_REGS_STEP - 1) / FP8_REGS_STEP, rest = (uint32_t)p.K % FP8_REGS_STEP;
   hipLaunchKernelGGL(kern, dim3(per_xcd * 8), dim3(FP8_REGS_WAVES * 64), lds, s,
                      (v8u{ptr_lo(p.a), ptr_hi(p.a), ptr_lo(p.b), ptr_hi(p.b), (uint32_t)p.lda, (uint32_t)p.ldb, p.a_extent, p.b_extent}),
-                     (v4u{steps << 8 | rest, (uint32_t)p.M | RB << 16, ranges, per_xcd}), (v2u{NT, (uint32_t)((1ull << 32) / RB + 1)}), p);
+                     (v4u{steps << 8 | rest, (uint32_t)p.M | RB << 16, ranges, per_xcd}), (v2u{NT, fp8_regs_magic(RB)}), p);
   return true;
 }
 

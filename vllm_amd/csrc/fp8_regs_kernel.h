@@ -25,6 +25,22 @@ constexpr size_t fp8_regs_lds_bytes(int mb, int j) {
   return run > sums ? run : sums;
 }
 
+// What a workgroup computes: a range of n-tiles and a block of rows; the row blocks of a range are neighbours on one XCD.  unit / RB by multiplication: exact for
+// unit * RB < 2^32.  (Callable on the host for its test.)
+inline uint32_t fp8_regs_magic(uint32_t RB) { return (uint32_t)((1ull << 32) / RB + 1); }
+struct Fp8RegsUnit {
+  uint32_t range, rb;
+};
+__host__ __device__ inline uint32_t fp8_regs_place(uint32_t block, uint32_t per_xcd) { return (block & 7u) * per_xcd + (block >> 3); }
+__host__ __device__ inline Fp8RegsUnit fp8_regs_unit(uint32_t unit, uint32_t RB, uint32_t magic) {
+  Fp8RegsUnit u{unit, 0};
+  if (RB > 1) {
+    u.range = mul_high(unit, magic);
+    u.rb = unit - u.range * RB;
+  }
+  return u;
+}
+
 // TAIL: K ends inside a step.  What a row has behind K is not its own (a NaN in the weights is one whatever it is multiplied with): of the last step each lane asks
 // for the chunks before K, and the rest of both operands arrives as zeros.
 template <bool BF16_OUT, int MB, int J, bool TAIL>
@@ -40,13 +56,10 @@ __global__ __launch_bounds__(FP8_REGS_WAVES * 64, 2) void fp8_mm_regs_kernel(VAQ
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int q = lane >> 4, r16 = lane & 15;
-  const uint32_t unit = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
+  const uint32_t unit = fp8_regs_place(blockIdx.x, per_xcd);
   if (unit >= ranges * RB) return;
-  uint32_t range = unit, rb_u = 0;
-  if (RB > 1) {
-    range = __umulhi(unit, h2[1]);
-    rb_u = unit - range * RB;
-  }
+  const Fp8RegsUnit u = fp8_regs_unit(unit, RB, h2[1]);
+  const uint32_t range = u.range, rb_u = u.rb;
   const int nt0 = (int)range * J, row0 = (int)rb_u * MB * 16;
 
   // steps first .. steps - 1 of K are this wavefront's

@@ -20,10 +20,11 @@ struct TileSlot {
 };
 
 // Integer divisions are emulated in some 30 instructions (64-bit ones in more than 100), and a workgroup that finds its tile by them has gone through
-// 600 instructions, fetched cold, before its first request.  x / d = umulhi(x, div_magic(d)), which is at most one short, for any x.
+// 600 instructions, fetched cold, before its first request.  x / d = mul_high(x, div_magic(d)), which is at most one short, for any x.  (What follows is
+// callable on the host for its test.)
 inline uint32_t div_magic(uint32_t d) { return d <= 1 ? 0xffffffffu : (uint32_t)((1ull << 32) / d); }
-__device__ inline uint32_t div_by(uint32_t x, uint32_t d, uint32_t magic) {
-  const uint32_t q = __umulhi(x, magic);
+__host__ __device__ inline uint32_t div_by(uint32_t x, uint32_t d, uint32_t magic) {
+  const uint32_t q = mul_high(x, magic);
   return x - q * d >= d ? q + 1 : q;
 }
 
@@ -33,7 +34,7 @@ struct TileGrid {
   uint32_t band_magic;       // of a band's tiles
   uint32_t per8;             // tiles per XCD where that is a whole number, else 0
   uint32_t flags;            // K parts (12 bits), tail_first > 0, free bits of the kernel's own from 16 on
-  __device__ TileGrid rows(uint32_t tile_rows) const { return TileGrid{n, tile_rows, band_magic, per8, flags}; }
+  __host__ __device__ TileGrid rows(uint32_t tile_rows) const { return TileGrid{n, tile_rows, band_magic, per8, flags}; }
 };
 constexpr int TILE_BAND = 4;      // tiles are handed out in bands of so many tile rows (2 .. 16 measured: 4 is 1-3 % ahead of 8 on the large shapes)
 inline TileGrid tile_grid(int64_t tiles_m, int64_t tiles_n, int sk, int tail_first) {
@@ -49,15 +50,14 @@ inline TileSplitMagic tile_split_magic(int64_t tiles, int sk, int tail_first) { 
 
 // Where K part i of `steps` steps begins.
 template <class Params>
-__device__ inline int tile_part(const Params& p, const TileSlot& sl, int steps, int i) {
+__host__ __device__ inline int tile_part(const Params& p, const TileSlot& sl, int steps, int i) {
   if (i >= sl.nsplit) return steps;
   return i == 0 ? 0 : (int)div_by((uint32_t)steps * (uint32_t)i, (uint32_t)sl.nsplit, p.split_magic.sk);
 }
 
 template <class Params>
-__device__ inline TileSlot tile_slot_of(const TileGrid& g, const Params& p) {
+__host__ __device__ inline TileSlot tile_slot_of(const TileGrid& g, const Params& p, int b, int block_y) {
   TileSlot r;
-  int b = blockIdx.x;
   if (g.flags >> 12 & 1u) {
     const int tail_first = p.tail_first, sk = p.SK, tiles = (int)(g.m * g.n);
     const int rest = tiles - tail_first;
@@ -81,7 +81,7 @@ __device__ inline TileSlot tile_slot_of(const TileGrid& g, const Params& p) {
   }
   if (g.per8 > 0) b = (b & 7) * (int)g.per8 + (b >> 3);
   r.pos = b;
-  r.split = blockIdx.y;
+  r.split = block_y;
   r.nsplit = (int)(g.flags & 0xfffu);
   r.unit = b;
   r.units = (int)(g.m * g.n);
@@ -89,16 +89,18 @@ __device__ inline TileSlot tile_slot_of(const TileGrid& g, const Params& p) {
 }
 // ... and its tile: the tiles resident on one XCD share activation rows and weight columns in its L2.
 template <class Params>
-__device__ inline TileSlot tile_slot(const TileGrid& g, const Params& p) {
-  TileSlot r = tile_slot_of(g, p);
+__host__ __device__ inline TileSlot tile_slot(const TileGrid& g, const Params& p, int block_x, int block_y) {
+  TileSlot r = tile_slot_of(g, p, block_x, block_y);
   const uint32_t in_band = TILE_BAND * g.n, band = div_by((uint32_t)r.pos, in_band, g.band_magic);
   const uint32_t first_m = band * TILE_BAND, tin = (uint32_t)r.pos - band * in_band;
-  const uint32_t high = min(g.m - first_m, (uint32_t)TILE_BAND);
+  const uint32_t high = g.m - first_m < TILE_BAND ? g.m - first_m : (uint32_t)TILE_BAND;
   const uint32_t tn = div_by(tin, high, high == 4 ? 0x40000000u : high == 3 ? 0x55555555u : high == 2 ? 0x80000000u : 0xffffffffu);
   r.tm = (int)(first_m + tin - tn * high);
   r.tn = (int)tn;
   return r;
 }
+template <class Params>
+__device__ inline TileSlot tile_slot(const TileGrid& g, const Params& p) { return tile_slot(g, p, (int)blockIdx.x, (int)blockIdx.y); }
 
 // Hand-over of partial tiles.  Each wavefront owns WMB x WNB accumulator blocks of its workgroup's tile and one arrival
 // counter per (split tile, wavefront) in the caller's zeroed `counters`.  Every wavefront stores its partial blocks

@@ -128,6 +128,7 @@ struct KernelHead {
   v4u b;
   v2u c;
 };
+__host__ __device__ inline uint32_t mul_high(uint32_t a, uint32_t b) { return (uint32_t)((uint64_t)a * b >> 32); }
 inline uint32_t ptr_lo(const void* p) { return (uint32_t)(uintptr_t)p; }
 inline uint32_t ptr_hi(const void* p) { return (uint32_t)((uintptr_t)p >> 32); }
 template <typename T>

@@ -46,12 +46,35 @@ struct RegsParams {
 };
 
 // Counts: rows (up to 256), parts of K (8) and blocks of rows (16) in 9, 4 and 5 bits, and above them 2^12 / blocks, rounded up: x / blocks = x * that >> 12
-// for x < 128, a copy's number.  And x / copies = umulhi(x, 2^32 / copies + 1) for the x here, below 2^25.
+// for x < 128, a copy's number.  And x / copies = mul_high(x, 2^32 / copies + 1) for the x here, below 2^25.
 inline KernelHead regs_head(const RegsParams& p) {
   const uint32_t counts = (uint32_t)p.M | (uint32_t)p.SK << 9 | (uint32_t)p.RB << 13 | (uint32_t)((4096 + p.RB - 1) / p.RB) << 18;
   return KernelHead{v8u{ptr_lo(p.a), ptr_hi(p.a), ptr_lo(p.b), ptr_hi(p.b), ptr_lo(p.scales), ptr_hi(p.scales), (uint32_t)p.lda, (uint32_t)p.G},
                     v4u{(uint32_t)p.NT, counts, (uint32_t)p.ranges, (uint32_t)p.per_xcd},
                     v2u{(uint32_t)p.s_stride, (uint32_t)((1ull << 32) / (uint32_t)(p.SK * p.RB) + 1)}};
+}
+
+// What a workgroup computes: one contiguous range of units per XCD; the K parts and row blocks of one range of n-tiles are neighbours.  (No division where K is
+// whole: a 32-bit one is some 30 instructions, a 64-bit one more than 100.)  Callable on the host for its test.
+struct RegsUnit {
+  uint32_t range, sk, rb, g_lo, g_hi;      // range of n-tiles, part of K and its k-tiles, block of rows
+};
+__host__ __device__ inline uint32_t regs_place(uint32_t block, uint32_t per_xcd) { return (block & 7u) * per_xcd + (block >> 3); }
+__host__ __device__ inline RegsUnit regs_unit(uint32_t unit, uint32_t counts, uint32_t copies_magic, uint32_t G) {
+  const int SK = (int)(counts >> 9 & 0xfu), RB = (int)(counts >> 13 & 0x1fu);
+  const uint32_t copies = (uint32_t)(SK * RB);
+  RegsUnit u{unit, 0, 0, 0, G};
+  if (copies > 1) {
+    u.range = mul_high(unit, copies_magic);
+    u.rb = unit - u.range * copies;
+    if (SK > 1) {
+      u.sk = u.rb * (counts >> 18) >> 12;
+      u.rb -= u.sk * (uint32_t)RB;
+      u.g_lo = G * u.sk / (uint32_t)SK;
+      u.g_hi = G * (u.sk + 1) / (uint32_t)SK;
+    }
+  }
+  return u;
 }
 
 constexpr size_t regs_lds_bytes(int mb, int mr, int j, int nw, int sub, bool zp) {
@@ -153,22 +176,11 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(VAQ_HEAD_ARGS,
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int o = lane >> 4, r16 = lane & 15;
   const int M = (int)(counts & 0x1ffu), SK = (int)(counts >> 9 & 0xfu), RB = (int)(counts >> 13 & 0x1fu);
-  // One contiguous range of units per XCD; the K parts and row blocks of one range of n-tiles are neighbours.  (No division where K is whole: a 32-bit
-  // one is some 30 instructions, a 64-bit one more than 100.)
-  const uint32_t unit = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3), copies = (uint32_t)(SK * RB);
-  if (unit >= ranges * copies) return;
-  uint32_t range = unit, sk = 0, rb_u = 0, g_lo_u = 0, g_hi_u = G;
-  if (copies > 1) {
-    range = __umulhi(unit, copies_magic);
-    rb_u = unit - range * copies;
-    if (SK > 1) {
-      sk = rb_u * (counts >> 18) >> 12;
-      rb_u -= sk * (uint32_t)RB;
-      g_lo_u = G * sk / (uint32_t)SK;
-      g_hi_u = G * (sk + 1) / (uint32_t)SK;
-    }
-  }
-  const int rb_i = (int)rb_u, g_lo = (int)g_lo_u, g_hi = (int)g_hi_u;
+  const uint32_t unit = regs_place(blockIdx.x, per_xcd);
+  if (unit >= ranges * (uint32_t)(SK * RB)) return;
+  const RegsUnit u = regs_unit(unit, counts, copies_magic, G);
+  const uint32_t range = u.range, sk = u.sk;
+  const int rb_i = (int)u.rb, g_lo = (int)u.g_lo, g_hi = (int)u.g_hi;
   const int nt0 = (int)range * J, row0 = rb_i * MB * 16;
 
   auto rsrc = [](const void* base, uint32_t bytes) {
