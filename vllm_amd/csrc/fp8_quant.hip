@@ -357,7 +357,8 @@ static int launch_quant(const void* in, int in_dtype, int64_t in_stride, uint8_t
   if (rows >= 1024 && hidden <= 5120) return launch(half, four);
   if (hidden <= QT * 8) return launch(full, one);
   if constexpr (MODE == 0) {
-    // Few long rows: four workgroups to a row, each with the row's maximum and a quarter of its codes, the longer part of the arithmetic.  With the GEMM behind
+    // Few long rows: four workgroups to a row, each with the row's maximum and the codes of one in four of a thread's vectors, the longer part of the arithmetic (rows of 8192
+    // have two vectors to a thread, so that two of the workgroups find no codes; above 12288 each has some).  With the GEMM behind
     // it, us: 16 x 8192 10.20 -> 9.97, 16 / 64 x 14336 14.83 / 22.16 -> 14.50 / 21.81, 16 x 16384 18.34 -> 17.79; up to 6144 elements level.  Up to 8 rows a launch by itself takes
     // 0.1 us more and none less.  (Not where the codes go over the rows: another workgroup may still read them.)
     const uint64_t width = in_dtype == VAQ_F32 ? 4 : 2, last = (uint64_t)(rows - 1);

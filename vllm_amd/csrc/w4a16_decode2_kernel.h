@@ -252,17 +252,18 @@ __global__ __launch_bounds__(D2_WAVES * 64) void w4a16_decode2_kernel(VAQ_HEAD_A
             at += l_step;
           }
         }
-      } else
-      for (int c0 = w * 64; c0 < chunks; c0 += NTHR) {
-        const int k = k_slab0 + (ko ^ (m & (MR - 1))) * 8;
-        const bool ok = m < MR * MB && m < M_loc && k < K;
-        const uint32_t off = ok ? (uint32_t)(m * lda32 + k) * 2u : 0x80000000u;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(lds + (size_t)c0 * 16), 16, (int)off, 0, 0, 0);
-        m += step_m;
-        ko += step_ko;
-        if (ko >= KO) {
-          ko -= KO;
-          m += 1;
+      } else {
+        for (int c0 = w * 64; c0 < chunks; c0 += NTHR) {
+          const int k = k_slab0 + (ko ^ (m & (MR - 1))) * 8;
+          const bool ok = m < MR * MB && m < M_loc && k < K;
+          const uint32_t off = ok ? (uint32_t)(m * lda32 + k) * 2u : 0x80000000u;
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(lds + (size_t)c0 * 16), 16, (int)off, 0, 0, 0);
+          m += step_m;
+          ko += step_ko;
+          if (ko >= KO) {
+            ko -= KO;
+            m += 1;
+          }
         }
       }
       __builtin_amdgcn_sched_barrier(0);

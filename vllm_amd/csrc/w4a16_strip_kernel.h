@@ -67,7 +67,7 @@ __global__ __launch_bounds__(512, WMB * WNB == 1 && HAS_ZP && SUBG == 4 ? 4 : 2)
   // ---- activations: the rows of this wavefront's own K group are loaded by its NS wavefronts ----
   // A descriptor of the rows' own bytes and no more: an operand may be the trailing columns of its storage.  The rows are in the lanes' offsets
   // (up to 4 GiB, checked on the host), those past M at its far end; the scalar offset is the place in K, or all of the extent for a group past the
-  // K part: either requests nothing (zeros, no traffic) and keeps the wait counts uniform.  No sum of the two can wrap.  (Row tests and a select for
+  // K part (vaq_common.h): either requests nothing (zeros, no traffic) and keeps the wait counts uniform.  (Row tests and a select for
   // every request cost 0.7 % in the mean over 1300 problems of M = 200 .. 4096; rows in the scalar offset, one addition a request, 0.3 % over 3250.)
   const uint32_t a_bytes = ((uint32_t)(p.M - 1) * (uint32_t)p.lda + (uint32_t)p.K) * 2u;
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a), 0, (int)a_bytes, 0x00020000);
