@@ -8,6 +8,8 @@ Runs on the GPU; the *.csv.gz beside it are what it wrote on an MI355X.  A probl
 
     fp8_tile, w4_tile (4-bit codes in groups of 128 rows with zero points), w8_tile (8-bit codes), and both in groups of 64 / 32 rows,
     z with zero points, h fp16 instead of bf16:  k, n, m, tile id, parts of K, 1 if only the tiles of the last round are in parts, us
+                        (tile id 48, the 256 x 256 tiles of w4a16_tile256_kernel.h, was timed later, on the files' problems of more than 128 rows: its times are
+                        scaled by what the fastest plan of the problem took then and takes in the file)
     w4_decode:          k, n, m, groups of 128 rows (1, 2, 4), 8-bit codes, kind, gs, wks, wn (0: by the planner), us
                         kind 0 workgroups of all rows, 1 of 16 rows, 2 the tile kernel by the plan of the shapes with weights
                         through LDS (gs, wks, wn 0), at whose price the decode kernels are weighed
@@ -144,7 +146,7 @@ TILES = {"fp8_tile": {13: (128, 128), 14: (64, 128), 15: (64, 64), 16: (128, 64)
                      41: (32, 128), 51: (32, 64), 42: (64, 128), 52: (64, 64), 43: (96, 128), 44: (128, 128), 46: (128, 256), 66: (128, 256),
                      48: (256, 256)},
          "w8_tile": {12: (128, 128), 14: (64, 128), 15: (128, 64), 16: (256, 128), 20: (256, 256), 41: (32, 128), 51: (32, 64), 42: (64, 128),
-                     52: (64, 64), 43: (96, 128), 44: (128, 128), 46: (128, 256)}}
+                     52: (64, 64), 43: (96, 128), 44: (128, 128), 46: (128, 256), 48: (256, 256)}}
 FORMATS_OF = {"w4_tile": (4, 128, True), "w8_tile": (8, 128, False),      # bits, rows of a group, zero points, activations
               "w4g32zh_tile": (4, 32, True, torch.float16), "w8g32h_tile": (8, 32, False, torch.float16)}
 TILES["w4g32zh_tile"] = TILES["w8g32h_tile"] = TILES["w8_tile"]

@@ -213,4 +213,54 @@ __device__ inline bool handover_pieces(float* c_tmp, int32_t* counters, v4f (&pa
   return true;
 }
 
+// The same in three steps, for a wavefront whose NP pieces do not all fit its registers a second time: everybody gives its part away (true: the last one), the last one
+// takes CH pieces of the sum at a time and, when it has them all, leaves the counter zero.
+template <int NP, int NW>
+struct HandoverUnit {
+  uint32_t unit, split_stride;
+  __amdgpu_buffer_rsrc_t rt;
+  __device__ HandoverUnit(float* c_tmp, const TileSlot& sl, int wave) {
+    unit = (uint32_t)((sl.unit * NW + wave) * NP) * 1024u;          // bytes
+    split_stride = (uint32_t)sl.units * (uint32_t)(NW * NP) * 1024u;
+    rt = __builtin_amdgcn_make_buffer_rsrc(c_tmp, 0, (int)(split_stride * (uint32_t)sl.nsplit), 0x00020000);
+  }
+};
+template <int NP, int NW, typename Piece>
+__device__ inline bool handover_give(float* c_tmp, int32_t* counters, Piece piece, const TileSlot& sl, int wave, int lane) {
+  constexpr int SC1 = 16;
+  const HandoverUnit<NP, NW> u(c_tmp, sl, wave);
+#pragma unroll
+  for (int c = 0; c < NP; ++c)
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, piece(c)), u.rt, lane * 16, (int)(sl.split * u.split_stride + u.unit + c * 1024), SC1);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // the part is acknowledged before the counter moves
+  int old = 0;
+  if (lane == 0) old = __hip_atomic_fetch_add(counters + (int64_t)sl.unit * NW + wave, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return __builtin_amdgcn_readfirstlane(old) == sl.nsplit - 1;
+}
+template <int CH, int NP, int NW>
+__device__ inline void handover_take(float* c_tmp, v4f (&sum)[CH], int c0, const TileSlot& sl, int wave, int lane) {
+  constexpr int SC1 = 16;
+  const HandoverUnit<NP, NW> u(c_tmp, sl, wave);
+#pragma unroll
+  for (int c = 0; c < CH; ++c) sum[c] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < sl.nsplit; s0 += 2) {
+    const int s1 = s0 + 1 < sl.nsplit ? s0 + 1 : s0;
+    v4u r0[CH], r1[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) r0[c] = __builtin_amdgcn_raw_buffer_load_b128(u.rt, lane * 16, (int)(s0 * u.split_stride + u.unit + (c0 + c) * 1024), SC1);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) r1[c] = __builtin_amdgcn_raw_buffer_load_b128(u.rt, lane * 16, (int)(s1 * u.split_stride + u.unit + (c0 + c) * 1024), SC1);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) sum[c] += __builtin_bit_cast(v4f, r0[c]);
+    if (s0 + 1 < sl.nsplit) {
+#pragma unroll
+      for (int c = 0; c < CH; ++c) sum[c] += __builtin_bit_cast(v4f, r1[c]);
+    }
+  }
+}
+template <int NW>
+__device__ inline void handover_done(int32_t* counters, const TileSlot& sl, int wave, int lane) {
+  if (lane == 0) __hip_atomic_store(counters + (int64_t)sl.unit * NW + wave, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 }  // namespace vaq

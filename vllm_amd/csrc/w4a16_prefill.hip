@@ -11,11 +11,15 @@ namespace vaq {
 // ----------------------------------------------------------------------------- host side
 
 // tile ids: 0..2 = register-staged kernel (256x256, 128x128, 64x128); 10.. = direct-to-LDS kernel (BM x BN);
-// 41.. = strips (w4a16_strip_kernel.h)
+// 41.. = strips (w4a16_strip_kernel.h), 48 = w4a16_tile256_kernel.h
 // w4a16_strip*.hip
 int prefill_launch_strip(const PrefillParams& p, int tile, bool bf16, bool zp, hipStream_t s);
 int prefill_launch_strip_sub(const PrefillParams& p, int sub, int tile, bool bf16, bool zp, hipStream_t s);
 int prefill_launch_strip_w8(const PrefillParams& p, int sub, int tile, bool bf16, hipStream_t s);
+// w4a16_tile256*.hip (id 48)
+int prefill_launch_tile256(const PrefillParams& p, bool bf16, bool zp, hipStream_t s);
+int prefill_launch_tile256_sub(const PrefillParams& p, int sub, bool bf16, bool zp, hipStream_t s);
+int prefill_launch_tile256_w8(const PrefillParams& p, int sub, bool bf16, hipStream_t s);
 
 template <bool BF16, bool HAS_ZP>
 static int dispatch_tile(const PrefillParams& p, int tile, hipStream_t s) {
@@ -44,6 +48,9 @@ static int dispatch_tile(const PrefillParams& p, int tile, hipStream_t s) {
 // than 10 %, as over a half of the layers that a fit to the other half had not seen.  The fastest plan of the shapes
 // 12 .. 20 (weights through LDS) takes this much more than that of the shapes from 41 on (strips): 41 / 29 / 26 / 22 / 17 / 11 / 8 / 3 %
 // at M up to 32 / 64 / 128 / 256 / 512 / 1024 / 2048 / 8192; at M > 512 it is ahead in 10-25 % of the problems, by a few percent.
+// The shape 48 (w4a16_tile256_kernel.h; before it a 256 x 256 shape of the strip kernel, for 4-bit codes in groups of 128 rows alone) came later, in all four tables, timed on
+// their problems of more than 128 rows; its constants, and with them those of a few large shapes of the other tables (of groups of 32 rows in 8 bits of all), are those whose choice loses
+// least.  Over 4581 other problems of M = 200 .. 8192 it is the fastest plan of 47 %, and what it takes there is 0.92 (4 bits in groups of 128 rows) .. 0.88 of what those problems took.
 constexpr TileShape W4_TILE_SHAPES[] = {
     {12, 128, 128, 8, 2, 0.536, 0.606, 0.0793, 0.375, 0.153}, {14, 64, 128, 8, 2, 0, 0.535, 0.0271, 0.177, 0.252},
     {15, 128, 64, 4, 2, 0, 0.553, 0.0166, 0.0944, 0.337},     {16, 256, 128, 8, 1, 1.88, 0.781, 0.176, 0, 0.0912},
@@ -52,7 +59,7 @@ constexpr TileShape W4_TILE_SHAPES[] = {
     {42, 64, 128, 8, 2, 2.44, 0.233, 0.0366, 0.25, 0.116},    {52, 64, 64, 8, 1, 2.68, 0.138, 0.0327, 0, 0.0886},
     {43, 96, 128, 8, 1, 3.1, 0.266, 0.085, 0, 0.169},         {44, 128, 128, 8, 1, 3.63, 0.328, 0.114, 0, 0.126},
     {46, 128, 256, 8, 1, 3.64, 0.495, 0.324, 0, 0.0655},      {66, 128, 256, 8, 1, 6.38, 0.566, 0.164, 0, 0.119},
-    {48, 256, 256, 8, 1, 8.35, 0.917, 0.387, 0, 0.0423}};
+    {48, 256, 256, 4, 1, 5.52, 1.09, 0.156, 0, 0.0428}};
 constexpr TileCosts W4_TILE_COSTS = {0.163, 0.628, 0.63, 0.253, 0.0};
 // Groups of 64 / 32 rows: 2744 such problems, 78807 launches (64 rows with zero points, 32 without and with, these in fp16 too).  One workgroup of
 // the shape 42 to a compute unit: its scales of the sub-groups leave no room for a second one in the registers.  In the mean 0.6 % on layers
@@ -60,35 +67,38 @@ constexpr TileCosts W4_TILE_COSTS = {0.163, 0.628, 0.63, 0.253, 0.0};
 // 0.7, 0.7, 1.0 and 1.9 %).
 constexpr TileShape W4SUB_TILE_SHAPES[] = {
     {12, 128, 128, 8, 2, 0.726, 0.631, 0.0892, 0.392, 0.139}, {14, 64, 128, 8, 2, 0, 0.613, 0.0195, 0.177, 0.269},
-    {15, 128, 64, 4, 2, 0, 0.583, 0.0117, 0.107, 0.358},      {16, 256, 128, 8, 1, 1.95, 0.825, 0.183, 0, 0.11},
-    {20, 256, 256, 8, 1, 4.48, 1.36, 0.12, 0, 0.013},
+    {15, 128, 64, 4, 2, 0, 0.583, 0.0117, 0.107, 0.358},      {16, 256, 128, 8, 1, 1.66, 0.83, 0.166, 0, 0.0983},
+    {20, 256, 256, 8, 1, 4.63, 1.36, 0.123, 0, 0.0118},
     {41, 32, 128, 8, 2, 2.38, 0.236, 0.0194, 0.195, 0.161},   {51, 32, 64, 8, 2, 1.31, 0.124, 0.00437, 0.141, 0.681},
     {42, 64, 128, 8, 1, 2.47, 0.264, 0.0529, 0, 0.0702},      {52, 64, 64, 8, 1, 2.52, 0.165, 0.0145, 0, 0.067},
-    {43, 96, 128, 8, 1, 2.57, 0.333, 0.0362, 0, 0.257},       {44, 128, 128, 8, 1, 3.05, 0.386, 0.0558, 0, 0.246},
-    {46, 128, 256, 8, 1, 3.85, 0.584, 0.219, 0, 0.0488}};
+    {43, 96, 128, 8, 1, 2.31, 0.334, 0.0356, 0, 0.27},       {44, 128, 128, 8, 1, 3.2, 0.381, 0.0552, 0, 0.242},
+    {46, 128, 256, 8, 1, 3.88, 0.573, 0.233, 0, 0.0539},
+    {48, 256, 256, 4, 1, 7.4, 1.2, 0.0749, 0, 0.0156}};
 constexpr TileCosts W4SUB_TILE_COSTS = {0.131, 0.547, 0.631, 0.274, 0.0};
 // 8-bit codes, whose dequantisation takes longer: fitted to 993 such problems, in the mean 0.7 % over 1216 others (37199 launches, those kept
 // in profiles/plan_prices; 2.4 % with the first constants above).
 // Groups of 64 rows take them too, but for the slots of the shape 41 (make_plan_prefill): 876 problems, 24724 launches, 0.4 %.
 constexpr TileShape W8_TILE_SHAPES[] = {
     {12, 128, 128, 8, 2, 0.783, 0.635, 0.0684, 0.441, 0.0986}, {14, 64, 128, 8, 2, 0.0101, 0.595, 0.0269, 0.17, 0.261},
-    {15, 128, 64, 4, 2, 0.0105, 0.608, 0.0138, 0.106, 0.362},  {16, 256, 128, 8, 1, 1.74, 0.879, 0.156, 0, 0.0659},
-    {20, 256, 256, 8, 1, 4.63, 1.25, 0.226, 0, 0.0177},
+    {15, 128, 64, 4, 2, 0.0105, 0.608, 0.0138, 0.106, 0.362},  {16, 256, 128, 8, 1, 1.74, 0.888, 0.131, 0, 0.0597},
+    {20, 256, 256, 8, 1, 4.31, 1.24, 0.285, 0, 0.0287},
     {41, 32, 128, 8, 2, 3.13, 0.244, 0.0253, 0.251, 0.104},    {51, 32, 64, 8, 1, 1.55, 0.164, 0.0131, 0, 0.676},
     {42, 64, 128, 8, 1, 2.76, 0.323, 0.0451, 0, 0.104},        {52, 64, 64, 8, 1, 2.7, 0.187, 0.0172, 0, 0.0905},
-    {43, 96, 128, 8, 1, 3.07, 0.371, 0.0552, 0, 0.297},        {44, 128, 128, 8, 1, 3.6, 0.421, 0.0724, 0, 0.247},
-    {46, 128, 256, 8, 1, 5.19, 0.669, 0.163, 0, 0.0913}};
+    {43, 96, 128, 8, 1, 3.18, 0.358, 0.0528, 0, 0.37},        {44, 128, 128, 8, 1, 3.66, 0.423, 0.0703, 0, 0.185},
+    {46, 128, 256, 8, 1, 4.83, 0.668, 0.166, 0, 0.0828},
+    {48, 256, 256, 4, 1, 8.97, 1.08, 0.161, 0, 0.0389}};
 constexpr TileCosts W8_TILE_COSTS = {0.176, 0.376, 0.706, 0.291, 0.0};
 // Groups of 32 rows: 1549 such problems, 45867 launches, in bf16 and fp16, whose strips convert code by code here; in the mean 0.6 % on layers
 // that a fit to the other half had not seen (0.45 and 0.8 %; with the constants above 0.55 and 1.55, 1 in 8 fp16 problems more than 5 % behind).
 constexpr TileShape W8G32_TILE_SHAPES[] = {
-    {12, 128, 128, 8, 2, 0.764, 0.714, 0.0825, 0.454, 0.103},  {14, 64, 128, 8, 2, 0.0103, 0.639, 0.0243, 0.232, 0.28},
-    {15, 128, 64, 4, 2, 0.0108, 0.626, 0.0125, 0.155, 0.356},  {16, 256, 128, 8, 1, 2.37, 0.864, 0.185, 0, 0.0685},
-    {20, 256, 256, 8, 1, 4.77, 1.38, 0.191, 0, 0.0156},
-    {41, 32, 128, 8, 1, 2.79, 0.342, 0.0308, 0, 0.108},        {51, 32, 64, 8, 1, 1.09, 0.181, 0.00686, 0, 0.297},
-    {42, 64, 128, 8, 1, 2.97, 0.376, 0.0464, 0, 0.0855},       {52, 64, 64, 8, 1, 2.67, 0.215, 0.0121, 0, 0.0941},
-    {43, 96, 128, 8, 1, 2.53, 0.437, 0.0335, 0, 0.332},        {44, 128, 128, 8, 1, 3.15, 0.51, 0.0439, 0, 0.251},
-    {46, 128, 256, 8, 1, 4.11, 0.838, 0.149, 0, 0.121}};
+    {12, 128, 128, 8, 2, 0.506, 0.715, 0.0659, 0.452, 0.102},  {14, 64, 128, 8, 2, 0.00792, 0.631, 0.0184, 0.273, 0.282},
+    {15, 128, 64, 4, 2, 0.014, 0.632, 0.013, 0.177, 0.3},  {16, 256, 128, 8, 1, 2.14, 0.862, 0.189, 0, 0.0627},
+    {20, 256, 256, 8, 1, 4.89, 1.38, 0.191, 0, 0.0155},
+    {41, 32, 128, 8, 1, 3.02, 0.382, 0.0337, 0, 0.0959},        {51, 32, 64, 8, 1, 1.06, 0.194, 0.00849, 0, 0.266},
+    {42, 64, 128, 8, 1, 2.91, 0.406, 0.0459, 0, 0.0971},       {52, 64, 64, 8, 1, 2.21, 0.217, 0.0121, 0, 0.0947},
+    {43, 96, 128, 8, 1, 2.3, 0.435, 0.0374, 0, 0.288},        {44, 128, 128, 8, 1, 2.99, 0.479, 0.0322, 0, 0.411},
+    {46, 128, 256, 8, 1, 4.42, 0.827, 0.133, 0, 0.169},
+    {48, 256, 256, 4, 1, 7.09, 1.34, 0.129, 0, 0.0015}};
 constexpr TileCosts W8G32_TILE_COSTS = {0.146, 0.456, 0.643, 0.288, 0.0};
 // The shapes with weights through LDS by themselves, fitted to 815 problems of 4-bit codes: what FP8 weights are built for (but 13),
 // and the price that up to 256 rows are weighed against the decode kernels at (w4a16_staged_us).
@@ -117,7 +127,7 @@ static int pick_register_staged(int M, int N) {
   return tiles(256, 256) >= cus ? 0 : (tiles(128, 128) >= cus ? 1 : 2);
 }
 
-// Tile shape and K split for a problem (the shapes 13, 48 and 66 are built for TILES_PLAIN; 30, another kernel of the shape 20 in
+// Tile shape and K split for a problem (the shapes 13 and 66 are built for TILES_PLAIN; 30, another kernel of the shape 20 in
 // recorded timings, stands for 20).
 static TilePlan make_plan_prefill(int M, int N, int K, TileFormat format) {
   const int64_t cus = num_cus_current_device();
@@ -134,7 +144,7 @@ static TilePlan make_plan_prefill(int M, int N, int K, TileFormat format) {
     TileShape t = *shape;
     if (t.id == 41 && format == TILES_8BIT_64) t.slots = 1;      // (133 registers)
     const bool is256 = t.id == 20 || t.id == 48;
-    if (forced >= 0 ? forced != t.id && !(t.id == 20 && (forced == 10 || forced == 11)) : (t.id == 13 || t.id == 48 || t.id == 66) && !plain) continue;
+    if (forced >= 0 ? forced != t.id && !(t.id == 20 && (forced == 10 || forced == 11)) : (t.id == 13 || t.id == 66) && !plain) continue;
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
     const int64_t rest = tiles % cus;
     auto consider = [&](int sk, int64_t tail_first) {
@@ -243,7 +253,11 @@ int w4a16_prefill_launch(const void* a, int64_t lda, const int32_t* b, const voi
   int rc;
   // the alternating-phase variant exists for 4-bit codes in groups of 128 rows / channelwise
   const int tile_other = pl.id == 20 ? 10 : pl.id;
-  if (pl.id > 40) {
+  if (pl.id == 48) {
+    if (w8) rc = prefill_launch_tile256_w8(p, sub, bf16, s);
+    else if (sub > 1) rc = prefill_launch_tile256_sub(p, sub, bf16, zp, s);
+    else rc = prefill_launch_tile256(p, bf16, zp, s);
+  } else if (pl.id > 40) {
     if (w8) rc = prefill_launch_strip_w8(p, sub, pl.id, bf16, s);
     else if (sub > 1) rc = prefill_launch_strip_sub(p, sub, pl.id, bf16, zp, s);
     else rc = prefill_launch_strip(p, pl.id, bf16, zp, s);

@@ -434,9 +434,6 @@ static int strip_dispatch(const PrefillParams& p, int tile, hipStream_t s) {
     case 46: return launch_strip<BF16, 4, 1, 8, HAS_ZP, SUBG, W8, 4, WIDE ? 4 : 2>(p, s);      // 128 x 256, eight strips of 32 columns
     case 51: return launch_strip<BF16, 1, 1, 2, HAS_ZP, SUBG, W8, 4, SUBG == 4 ? 2 : 4>(p, s);      //  32 x 64
     case 52: return launch_strip<BF16, 2, 1, 2, HAS_ZP, SUBG, W8, 4, WIDE ? 4 : 2>(p, s);      //  64 x 64
-    case 48:
-      if constexpr (WIDE) return launch_strip<BF16, 8, 1, 8, HAS_ZP, SUBG, W8, 4, 2>(p, s);      // 256 x 256
-      break;
     case 66:
       if constexpr (WIDE) return launch_strip<BF16, 4, 2, 4, HAS_ZP, SUBG, W8, 4, 2>(p, s);      // 128 x 256
       break;
