@@ -10,7 +10,7 @@
 //    the slice before.  No weight passes through LDS, and each is dequantised once per tile.
 //  * Activations: half a group (64 k) of KG groups x BM rows per step, global -> LDS by direct-to-LDS loads, NST stages, the image
 //    of the LDS-staged kernel (128-byte rows, two to a 256-byte line, 16-byte chunks XOR-ed with the line number).
-//  * One workgroup barrier per step (64 k of every group), placed in front of the step's last slice.
+//  * One workgroup barrier per step (64 k of every group), placed in front of the slice in which the next step's fragments are first read.
 //
 // What it is for: the LDS-staged kernel's K step of 64 is a chain -- barrier, fragment reads, MFMAs, weight writes -- of 0.55 us
 // whatever the tile, so that tens to hundreds of rows ran at a fifth of the matrix core's rate and needed K in many parts, with
@@ -47,6 +47,11 @@ __global__ __launch_bounds__(512, WMB * WNB == 1 && HAS_ZP && SUBG == 4 ? 4 : 2)
   constexpr int TPG = W8 ? 2 : 1;
   constexpr int A_LD = 4 * WMB / NS;               // direct-to-LDS instructions per wavefront and step
   constexpr int STAGE = KG * BM * 128;             // bytes
+  // Activation fragments are read two slices ahead, else one.  8-bit codes: a slice's dequantisation is so long that the two wavefronts of a SIMD rarely overlap, and a read of one
+  // slice's length is waited for.  Cold, all groups, of the time with reads one slice ahead: 96 x 128 0.93 .. 0.985 (4096 x 28672 at M = 120, 64-row groups, 70.0 -> 65.4 us), 128 x 128
+  // 0.97 .. 1.0, 128 x 256 0.905 .. 0.957 (4096 x 4096 at M = 333 54.5 -> 50.3), 64 x 128 0.94 .. 0.987, but in groups of 32 level; 32 x 128, 64 x 64 and 32 x 64 0.97 .. 1.04.
+  // 4-bit codes on 96 x 128 0.98 .. 1.04, on 128 x 128 1.01 .. 1.03.
+  constexpr bool DEEP = W8 && WNB == 1 && (WMB >= 3 || (WMB == 2 && NS == 4 && SUBG < 4));
   constexpr int KW = TW * TPG + WNB * SUBG * (HAS_ZP ? 2 : 1);      // vector-memory instructions of one load_w
   constexpr bool HP = !BF16 && SUBG < 4;              // packed fp16 dequantisation (its constants of four sub-groups do not fit the registers)
   static_assert(KG * NS == 8 && (4 * WMB) % NS == 0 && (WMB * WNB * 4) % KG == 0 && !(W8 && HAS_ZP), "strip kernel: shape");
@@ -191,21 +196,21 @@ __global__ __launch_bounds__(512, WMB * WNB == 1 && HAS_ZP && SUBG == 4 ? 4 : 2)
     coff[s4] = (uint32_t)(kg * (BM * 128) + ((lane & 31) >> 1) * 256 + ((((lane & 1) * 8 + chunk) ^ ((lane >> 1) & 15)) * 16));
   }
 
-  v4u af[WMB];       // B operands (activations) of the current slice, refilled in place
+  v4u af[DEEP ? 2 : 1][WMB];      // B operands (activations) of the current slice, with DEEP also of the next, refilled in place
   v4u wf[2][WNB];    // A operands (weights) of the current and of the next slice
 
-  // One k-slice: its MFMAs, with the reads of the next slice's activation fragments and the dequantisation of its weights in
-  // their shadow.
+  // One k-slice: its MFMAs, with the reads of a later slice's activation fragments (slice next_s4 of the step in `next_a`) and the dequantisation of the next
+  // one's weights in their shadow.
   auto slice = [&](auto cbuf_c, const uint8_t* next_a, auto next_s4_c, auto next_j_c, auto requests) {
     constexpr int cbuf = decltype(cbuf_c)::value, nbuf = cbuf ^ 1;
-    constexpr int next_s4 = decltype(next_s4_c)::value, next_j = decltype(next_j_c)::value;
+    constexpr int next_s4 = decltype(next_s4_c)::value, next_j = decltype(next_j_c)::value, next_xy = (cbuf + 1) & 1, ab = DEEP ? cbuf : 0;
 #pragma unroll
     for (int mb = 0; mb < WMB; ++mb) {
 #pragma unroll
-      for (int nb = 0; nb < WNB; ++nb) acc[mb][nb] = T::mfma32(wf[cbuf][nb], af[mb], acc[mb][nb]);      // rows = n, columns = m
-      af[mb] = *reinterpret_cast<const v4u*>(next_a + mb * 4096 + coff[next_s4]);
+      for (int nb = 0; nb < WNB; ++nb) acc[mb][nb] = T::mfma32(wf[cbuf][nb], af[ab][mb], acc[mb][nb]);      // rows = n, columns = m
+      af[ab][mb] = *reinterpret_cast<const v4u*>(next_a + mb * 4096 + coff[next_s4]);
 #pragma unroll
-      for (int x = mb * 4 * WNB / WMB; x < (mb + 1) * 4 * WNB / WMB; ++x) wf[nbuf][x >> 2][x & 3] = dequant_q(x >> 2, next_j, next_s4 & 1, x & 3);
+      for (int x = mb * 4 * WNB / WMB; x < (mb + 1) * 4 * WNB / WMB; ++x) wf[nbuf][x >> 2][x & 3] = dequant_q(x >> 2, next_j, next_xy, x & 3);
       if (mb == 0) requests();
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -248,11 +253,16 @@ __global__ __launch_bounds__(512, WMB * WNB == 1 && HAS_ZP && SUBG == 4 ? 4 : 2)
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 2) * A_LD + (PD - 1) * KW) : "memory");      // step 0 and the first weights
   advance_w(ring[0]);
   quarter(NST - 1, NST - 1, 0);
+  if (DEEP) quarter(NST - 1, NST - 1, 1);
 #pragma unroll
   for (int x = 0; x < 4 * WNB; ++x) wf[0][x >> 2][x & 3] = dequant_q(x >> 2, 0, 0, x & 3);
   asm volatile("s_barrier" ::: "memory");
 #pragma unroll
-  for (int mb = 0; mb < WMB; ++mb) af[mb] = *reinterpret_cast<const v4u*>(lds8 + mb * 4096 + coff[0]);
+  for (int mb = 0; mb < WMB; ++mb) af[0][mb] = *reinterpret_cast<const v4u*>(lds8 + mb * 4096 + coff[0]);
+  if constexpr (DEEP) {
+#pragma unroll
+    for (int mb = 0; mb < WMB; ++mb) af[1][mb] = *reinterpret_cast<const v4u*>(lds8 + mb * 4096 + coff[1]);
+  }
 
   int cur = 0;       // stage of the current step
   auto next_stage = [](int x) { return x + 1 == NST ? 0 : x + 1; };
@@ -272,19 +282,34 @@ __global__ __launch_bounds__(512, WMB * WNB == 1 && HAS_ZP && SUBG == 4 ? 4 : 2)
     const uint8_t* A1 = lds8 + s1 * STAGE;
     const uint8_t* A2 = lds8 + s2 * STAGE;
     const int ha = 2 * r - 1 + NST;
-    slice(C0{}, A0, C1{}, C0{}, [&] { weights(0); weights(1); quarter(ha, sp, 1); });
-    slice(C1{}, A0, C2{}, C1{}, [&] { weights(2); quarter(ha, sp, 2); });
-    slice(C0{}, A0, C3{}, C1{}, [&] { weights(3); quarter(ha, sp, 3); });
-    step_end();
-    slice(C1{}, A1, C0{}, C2{}, [&] { quarter(ha + 1, cur, 0); });
-    slice(C0{}, A1, C1{}, C2{}, [&] { quarter(ha + 1, cur, 1); });
-    slice(C1{}, A1, C2{}, C3{}, [&] { quarter(ha + 1, cur, 2); });
-    slice(C0{}, A1, C3{}, C3{}, [&] { quarter(ha + 1, cur, 3); });
-    step_end();
-    // the operands of the group's last slice are in wf[1] already: the next words become current in front of it
-    advance_w(nxt);
-    __builtin_amdgcn_sched_barrier(0);
-    slice(C1{}, A2, C0{}, C0{}, [&] { quarter(ha + 2, s1, 0); });
+    if constexpr (DEEP) {      // (the barrier stands where the next step's first fragments are read, here ahead of the last two slices)
+      slice(C0{}, A0, C2{}, C0{}, [&] { weights(0); weights(1); quarter(ha, sp, 2); });
+      slice(C1{}, A0, C3{}, C1{}, [&] { weights(2); weights(3); quarter(ha, sp, 3); });
+      step_end();
+      slice(C0{}, A1, C0{}, C1{}, [&] { quarter(ha + 1, cur, 0); });
+      slice(C1{}, A1, C1{}, C2{}, [&] { quarter(ha + 1, cur, 1); });
+      slice(C0{}, A1, C2{}, C2{}, [&] { quarter(ha + 1, cur, 2); });
+      slice(C1{}, A1, C3{}, C3{}, [&] { quarter(ha + 1, cur, 3); });
+      step_end();
+      slice(C0{}, A2, C0{}, C3{}, [&] { quarter(ha + 2, s1, 0); });
+      advance_w(nxt);
+      __builtin_amdgcn_sched_barrier(0);
+      slice(C1{}, A2, C1{}, C0{}, [&] { quarter(ha + 2, s1, 1); });
+    } else {
+      slice(C0{}, A0, C1{}, C0{}, [&] { weights(0); weights(1); quarter(ha, sp, 1); });
+      slice(C1{}, A0, C2{}, C1{}, [&] { weights(2); quarter(ha, sp, 2); });
+      slice(C0{}, A0, C3{}, C1{}, [&] { weights(3); quarter(ha, sp, 3); });
+      step_end();
+      slice(C1{}, A1, C0{}, C2{}, [&] { quarter(ha + 1, cur, 0); });
+      slice(C0{}, A1, C1{}, C2{}, [&] { quarter(ha + 1, cur, 1); });
+      slice(C1{}, A1, C2{}, C3{}, [&] { quarter(ha + 1, cur, 2); });
+      slice(C0{}, A1, C3{}, C3{}, [&] { quarter(ha + 1, cur, 3); });
+      step_end();
+      // the operands of the group's last slice are in wf[1] already: the next words become current in front of it
+      advance_w(nxt);
+      __builtin_amdgcn_sched_barrier(0);
+      slice(C1{}, A2, C0{}, C0{}, [&] { quarter(ha + 2, s1, 0); });
+    }
     cur = s2;
   };
   int r = 0;
@@ -314,21 +339,39 @@ __global__ __launch_bounds__(512, WMB * WNB == 1 && HAS_ZP && SUBG == 4 ? 4 : 2)
   if (rem > 0) {      // the last round, without the wavefronts whose K group lies past the end
     const uint8_t* A0 = lds8 + cur * STAGE;
     const uint8_t* A1 = lds8 + next_stage(cur) * STAGE;
-    if (kg < rem) {
-      slice(C0{}, A0, C1{}, C0{}, nothing);
-      slice(C1{}, A0, C2{}, C1{}, nothing);
-      slice(C0{}, A0, C3{}, C1{}, nothing);
-    }
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (kg < rem) {
-      slice(C1{}, A1, C0{}, C2{}, nothing);
-      slice(C0{}, A1, C1{}, C2{}, nothing);
-      slice(C1{}, A1, C2{}, C3{}, nothing);
-      slice(C0{}, A1, C3{}, C3{}, nothing);
+    auto drained = [] { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    auto last_slice = [&](auto cbuf_c) {
+      constexpr int cbuf = decltype(cbuf_c)::value;
 #pragma unroll
       for (int mb = 0; mb < WMB; ++mb)
 #pragma unroll
-        for (int nb = 0; nb < WNB; ++nb) acc[mb][nb] = T::mfma32(wf[1][nb], af[mb], acc[mb][nb]);
+        for (int nb = 0; nb < WNB; ++nb) acc[mb][nb] = T::mfma32(wf[cbuf][nb], af[DEEP ? cbuf : 0][mb], acc[mb][nb]);
+    };
+    if (kg < rem) {
+      if constexpr (DEEP) {
+        slice(C0{}, A0, C2{}, C0{}, nothing);
+        slice(C1{}, A0, C3{}, C1{}, nothing);
+      } else {
+        slice(C0{}, A0, C1{}, C0{}, nothing);
+        slice(C1{}, A0, C2{}, C1{}, nothing);
+        slice(C0{}, A0, C3{}, C1{}, nothing);
+      }
+    }
+    drained();
+    if (kg < rem) {
+      if constexpr (DEEP) {
+        slice(C0{}, A1, C0{}, C1{}, nothing);
+        slice(C1{}, A1, C1{}, C2{}, nothing);
+        slice(C0{}, A1, C2{}, C2{}, nothing);
+        slice(C1{}, A1, C3{}, C3{}, nothing);
+        slice(C0{}, A1, C3{}, C3{}, nothing);      // (reads a slice again that nobody uses)
+      } else {
+        slice(C1{}, A1, C0{}, C2{}, nothing);
+        slice(C0{}, A1, C1{}, C2{}, nothing);
+        slice(C1{}, A1, C2{}, C3{}, nothing);
+        slice(C0{}, A1, C3{}, C3{}, nothing);
+      }
+      last_slice(C1{});
     }
   }
   // every wavefront is done with the stages and nothing is on its way into them: the partial sums may use the LDS
