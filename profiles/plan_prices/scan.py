@@ -9,7 +9,9 @@ Runs on the GPU; the *.csv.gz beside it are what it wrote on an MI355X.  A probl
     fp8_tile, w4_tile (4-bit codes in groups of 128 rows with zero points), w8_tile (8-bit codes), and both in groups of 64 / 32 rows,
     z with zero points, h fp16 instead of bf16:  k, n, m, tile id, parts of K, 1 if only the tiles of the last round are in parts, us
                         (tile id 48, the 256 x 256 tiles of w4a16_tile256_kernel.h, was timed later, on the files' problems of more than 128 rows: its times are
-                        scaled by what the fastest plan of the problem took then and takes in the file)
+                        scaled by what the fastest plan of the problem took then and takes in the file; the same with the tile ids 42 (not in groups of 32), 43, 44 and
+                        46 of 8-bit codes, whose activation reads changed: twice to four times each where within 1.35 of the fastest plan, geometric mean, the others by the
+                        mean ratio of their id)
     w4_decode:          k, n, m, groups of 128 rows (1, 2, 4), 8-bit codes, kind, gs, wks, wn (0: by the planner), us
                         kind 0 workgroups of all rows, 1 of 16 rows, 2 the tile kernel by the plan of the shapes with weights
                         through LDS (gs, wks, wn 0), at whose price the decode kernels are weighed

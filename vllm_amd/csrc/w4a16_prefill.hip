@@ -75,30 +75,32 @@ constexpr TileShape W4SUB_TILE_SHAPES[] = {
     {46, 128, 256, 8, 1, 3.88, 0.573, 0.233, 0, 0.0539},
     {48, 256, 256, 4, 1, 7.4, 1.2, 0.0749, 0, 0.0156}};
 constexpr TileCosts W4SUB_TILE_COSTS = {0.131, 0.547, 0.631, 0.274, 0.0};
-// 8-bit codes, whose dequantisation takes longer: fitted to 993 such problems, in the mean 0.7 % over 1216 others (37199 launches, those kept
-// in profiles/plan_prices; 2.4 % with the first constants above).
-// Groups of 64 rows take them too, but for the slots of the shape 41 (make_plan_prefill): 876 problems, 24724 launches, 0.4 %.
+// 8-bit codes, whose dequantisation takes longer: 1216 such problems, 37199 launches, in the mean 0.6 % (2.4 % with the first constants above).
+// Groups of 64 rows take them too, but for the slots of the shape 41 (make_plan_prefill): 876 problems, 24724 launches, 0.35 %.
+// The strips that read activation fragments two slices ahead (w4a16_strip_kernel.h: the shapes 42 in groups of 64 rows and more, 43, 44, 46) take 0.94 .. 0.98 of what these problems were
+// timed at first.  All constants of 8-bit codes follow: with those before, 0.9 / 0.65 / 1.07 % in groups of 128 / 64 / 32 rows; 420 drawn calls of M = 33 .. 6500 take 0.997 in the
+// mean of their time with those (25 of them more than 3 % faster, 9 slower).
 constexpr TileShape W8_TILE_SHAPES[] = {
-    {12, 128, 128, 8, 2, 0.783, 0.635, 0.0684, 0.441, 0.0986}, {14, 64, 128, 8, 2, 0.0101, 0.595, 0.0269, 0.17, 0.261},
-    {15, 128, 64, 4, 2, 0.0105, 0.608, 0.0138, 0.106, 0.362},  {16, 256, 128, 8, 1, 1.74, 0.888, 0.131, 0, 0.0597},
-    {20, 256, 256, 8, 1, 4.31, 1.24, 0.285, 0, 0.0287},
-    {41, 32, 128, 8, 2, 3.13, 0.244, 0.0253, 0.251, 0.104},    {51, 32, 64, 8, 1, 1.55, 0.164, 0.0131, 0, 0.676},
-    {42, 64, 128, 8, 1, 2.76, 0.323, 0.0451, 0, 0.104},        {52, 64, 64, 8, 1, 2.7, 0.187, 0.0172, 0, 0.0905},
-    {43, 96, 128, 8, 1, 3.18, 0.358, 0.0528, 0, 0.37},        {44, 128, 128, 8, 1, 3.66, 0.423, 0.0703, 0, 0.185},
-    {46, 128, 256, 8, 1, 4.83, 0.668, 0.166, 0, 0.0828},
-    {48, 256, 256, 4, 1, 8.97, 1.08, 0.161, 0, 0.0389}};
+    {12, 128, 128, 8, 2, 0.789, 0.614, 0.0538, 0.433, 0.0931}, {14, 64, 128, 8, 2, 0.012, 0.602, 0.0299, 0.164, 0.233},
+    {15, 128, 64, 4, 2, 0.00863, 0.61, 0.0136, 0.0904, 0.301},  {16, 256, 128, 8, 1, 1.57, 0.886, 0.136, 0, 0.0688},
+    {20, 256, 256, 8, 1, 4.2, 1.23, 0.29, 0, 0.0258},
+    {41, 32, 128, 8, 2, 4.05, 0.252, 0.0252, 0.241, 0.12},    {51, 32, 64, 8, 1, 2.05, 0.174, 0.013, 0, 0.664},
+    {42, 64, 128, 8, 1, 2.85, 0.306, 0.046, 0, 0.103},        {52, 64, 64, 8, 1, 2.54, 0.194, 0.0205, 0, 0.0657},
+    {43, 96, 128, 8, 1, 3.43, 0.339, 0.0444, 0, 0.39},        {44, 128, 128, 8, 1, 4.19, 0.403, 0.062, 0, 0.157},
+    {46, 128, 256, 8, 1, 4.46, 0.629, 0.162, 0, 0.102},
+    {48, 256, 256, 4, 1, 8.97, 1.07, 0.162, 0, 0.0335}};
 constexpr TileCosts W8_TILE_COSTS = {0.176, 0.376, 0.706, 0.291, 0.0};
-// Groups of 32 rows: 1549 such problems, 45867 launches, in bf16 and fp16, whose strips convert code by code here; in the mean 0.6 % on layers
-// that a fit to the other half had not seen (0.45 and 0.8 %; with the constants above 0.55 and 1.55, 1 in 8 fp16 problems more than 5 % behind).
+// Groups of 32 rows: 1549 such problems, 45867 launches, in bf16 and fp16, whose strips convert code by code here; in the mean 0.67 % (with the constants above
+// 1 in 8 fp16 problems more than 5 % behind).
 constexpr TileShape W8G32_TILE_SHAPES[] = {
-    {12, 128, 128, 8, 2, 0.506, 0.715, 0.0659, 0.452, 0.102},  {14, 64, 128, 8, 2, 0.00792, 0.631, 0.0184, 0.273, 0.282},
-    {15, 128, 64, 4, 2, 0.014, 0.632, 0.013, 0.177, 0.3},  {16, 256, 128, 8, 1, 2.14, 0.862, 0.189, 0, 0.0627},
-    {20, 256, 256, 8, 1, 4.89, 1.38, 0.191, 0, 0.0155},
-    {41, 32, 128, 8, 1, 3.02, 0.382, 0.0337, 0, 0.0959},        {51, 32, 64, 8, 1, 1.06, 0.194, 0.00849, 0, 0.266},
-    {42, 64, 128, 8, 1, 2.91, 0.406, 0.0459, 0, 0.0971},       {52, 64, 64, 8, 1, 2.21, 0.217, 0.0121, 0, 0.0947},
-    {43, 96, 128, 8, 1, 2.3, 0.435, 0.0374, 0, 0.288},        {44, 128, 128, 8, 1, 2.99, 0.479, 0.0322, 0, 0.411},
-    {46, 128, 256, 8, 1, 4.42, 0.827, 0.133, 0, 0.169},
-    {48, 256, 256, 4, 1, 7.09, 1.34, 0.129, 0, 0.0015}};
+    {12, 128, 128, 8, 2, 0.475, 0.714, 0.0654, 0.436, 0.104},  {14, 64, 128, 8, 2, 0.00821, 0.605, 0.0188, 0.298, 0.273},
+    {15, 128, 64, 4, 2, 0.0146, 0.626, 0.0107, 0.207, 0.296},  {16, 256, 128, 8, 1, 2.08, 0.962, 0.141, 0, 0.0507},
+    {20, 256, 256, 8, 1, 4.52, 1.38, 0.228, 0, 0.0128},
+    {41, 32, 128, 8, 1, 2.87, 0.391, 0.0367, 0, 0.0948},        {51, 32, 64, 8, 1, 1.07, 0.196, 0.00868, 0, 0.29},
+    {42, 64, 128, 8, 1, 2.89, 0.381, 0.0473, 0, 0.0972},       {52, 64, 64, 8, 1, 2.41, 0.214, 0.0107, 0, 0.105},
+    {43, 96, 128, 8, 1, 1.95, 0.429, 0.0229, 0, 0.373},        {44, 128, 128, 8, 1, 4.55, 0.455, 0.039, 0, 0.449},
+    {46, 128, 256, 8, 1, 3.74, 0.796, 0.109, 0, 0.164},
+    {48, 256, 256, 4, 1, 7.26, 1.34, 0.129, 0, 0.00143}};
 constexpr TileCosts W8G32_TILE_COSTS = {0.146, 0.456, 0.643, 0.288, 0.0};
 // The shapes with weights through LDS by themselves, fitted to 815 problems of 4-bit codes: what FP8 weights are built for (but 13),
 // and the price that up to 256 rows are weighed against the decode kernels at (w4a16_staged_us).
