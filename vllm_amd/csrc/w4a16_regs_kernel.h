@@ -1,5 +1,5 @@
 // W4A16 GEMM for a few to some dozen rows, weights and activations in registers: C[M,N] = A[M,K] . dequant(B[K,N]) (+bias), the
-// arithmetic of w4a16_decode.hip (codes as exact 16-bit numbers BIAS + code, zero point and group scale in fp32 on the accumulator).
+// arithmetic of w4a16_decode.hip (codes as exact 16-bit numbers BIAS + code, 8-bit ones in bf16 without bias; zero point and group scale in fp32 on the accumulator).
 //
 //  * A wavefront multiplies one k-tile (128 rows of K) of its rows with J neighbouring n-tiles at a time.  What the kernel that stages a
 //    slab of activations once per workgroup (w4a16_decode2_kernel.h) pays from 17 rows on -- one LDS operand read per MFMA (6 us of the
@@ -120,6 +120,26 @@ __device__ __attribute__((always_inline)) inline v4f regs_rounded_tile(const __a
   return sum;
 }
 
+// 8-bit codes of two nibble planes as one operand: 8 codes of consecutive k, in fp16 as 1024 + code (a byte behind the exponent), in bf16, whose 8 bits hold them whole, as they are.
+// As two operands, a plane each with its bias and the high one's products times 16, a code took two products, 14 instructions for 8 codes where these are 8 / 16, and four fused ones
+// for each result and group where there is one now (in groups of 128 rows; two in smaller ones).  Cold, us: 3584 x 4608 at M = 51 / 64 11.5 / 11.8 -> 10.0 / 10.4, 2048 x 23808 at
+// M = 19 in groups of 32 20.2 -> 16.1, 3072 x 16128 at M = 1 12.1 -> 11.5; 300 drawn calls of 1 .. 256 rows 0.963 in the mean, fp16 0.95, bf16 0.97.  Against 64 bits the error
+// is level in bf16 and smaller in fp16 (activations around 3 in groups of 128 rows 2.5e-4 -> 2.1e-4: 1024 + code instead of 16 (1024 + high) + 1024 + low).
+template <bool BF16>
+__device__ inline v4u regs_codes8(uint32_t hi, uint32_t lo) {
+  // bytes 0 .. 3: elements 0,4,1,5 and 2,6,3,7
+  const uint32_t t = ((hi << 4) & 0xf0f0f0f0u) | (lo & 0x0f0f0f0fu), u = (hi & 0xf0f0f0f0u) | ((lo >> 4) & 0x0f0f0f0fu);
+  if constexpr (BF16) {      // (no inline assembly: the compiler keeps clear of a product under way whose unused results share the registers only with its own instructions)
+    auto pair = [](uint32_t lo, uint32_t hi) {
+      typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+      return __builtin_bit_cast(uint32_t, v2bf{(__bf16)(float)(lo & 0xffu), (__bf16)(float)(hi & 0xffu)});
+    };
+    return v4u{pair(t, t >> 16), pair(u, u >> 16), pair(t >> 8, t >> 24), pair(u >> 8, u >> 24)};
+  }
+  return v4u{(t & 0x00ff00ffu) | 0x64006400u, (u & 0x00ff00ffu) | 0x64006400u, __builtin_amdgcn_perm(0x64646464u, t, 0x04030401u),
+             __builtin_amdgcn_perm(0x64646464u, u, 0x04030401u)};
+}
+
 // The sum of the wavefronts' parts of result q in LDS, and of the parts of K in c_tmp (four in flight, added in split order).
 template <int NW>
 __device__ __attribute__((always_inline)) inline v4f regs_sum(const v4f* red, int results, int q, int lane) {
@@ -158,7 +178,7 @@ __device__ __attribute__((always_inline)) inline void regs_store(const Params& p
 }
 
 // MR: rows of an m-block that are fetched, 16 or, of a single one, 4 (columns of the MFMAs are independent: those of the other rows read a
-// row that is there, and their results are not stored).  SUBG: quantisation groups per k-tile (1, 2, 4).  W8: 8-bit codes as two nibble planes.  OCC: wavefronts per SIMD that the registers
+// row that is there, and their results are not stored).  SUBG: quantisation groups per k-tile (1, 2, 4).  W8: 8-bit codes, two nibble planes in memory.  OCC: wavefronts per SIMD that the registers
 // are to allow.
 template <bool BF16, int MB, int MR, int J, bool HAS_ZP, int NW, int SUBG, bool W8, int OCC>
 __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(VAQ_HEAD_ARGS, const RegsParams p) {
@@ -258,7 +278,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(VAQ_HEAD_ARGS,
       __builtin_amdgcn_sched_barrier(0);
     }
     // row sums S of each group: the same in the four registers.  Plain codes: -(BIAS + 8) S is where the group's MFMA chain starts.
-    constexpr bool CHAIN = SUBG == 1 && !HAS_ZP && !W8;
+    constexpr bool CHAIN = SUBG == 1 && !HAS_ZP;
+    constexpr float ZERO = W8 ? (BF16 ? 128.0f : T::CODE_BIAS + 128.0f) : T::CODE_BIAS + 8.0f;      // what the operands have too much (regs_codes8)
     v4f start[MB];
     float S[SUBG][MB];
     const v4u ones = {T::ONE2, T::ONE2, T::ONE2, T::ONE2};
@@ -269,7 +290,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(VAQ_HEAD_ARGS,
         v4f t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int jj = sj * (4 / SUBG); jj < (sj + 1) * (4 / SUBG); ++jj) t = T::mfma16(ones, act[jj][mb], t);
-        start[mb] = t * -(T::CODE_BIAS + 8.0f);
+        start[mb] = t * -ZERO;
         S[sj][mb] = t[0];
       }
 #pragma unroll
@@ -278,22 +299,23 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(VAQ_HEAD_ARGS,
       for (int sj = 0; sj < SUBG; ++sj) {
         const v2u sct = *reinterpret_cast<const v2u*>(side + sj * 256 + j * 32 + o * 8);
         const uint32_t z4 = HAS_ZP ? *reinterpret_cast<const uint32_t*>(side + SC + sj * 64 + j * 8 + (o >> 1) * 4) >> ((o & 1) * 16) : 0u;
-        v4f P[PL][MB];
+        v4f P[MB];
 #pragma unroll
-        for (int pl = 0; pl < PL; ++pl) {
+        for (int mb = 0; mb < MB; ++mb) P[mb] = CHAIN ? start[mb] : v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int mb = 0; mb < MB; ++mb) P[pl][mb] = CHAIN ? start[mb] : v4f{0.f, 0.f, 0.f, 0.f};
-          const uint32_t wj[4] = {wq[s][j][pl].x, wq[s][j][pl].y, wq[s][j][pl].z, wq[s][j][pl].w};
-#pragma unroll
-          for (int jj = sj * (4 / SUBG); jj < (sj + 1) * (4 / SUBG); ++jj) {
-            v4u aop;
-            aop.x = (wj[jj] & msk) | ex;
-            aop.y = ((wj[jj] >> 4) & msk) | ex;
-            aop.z = ((wj[jj] >> 8) & msk) | ex;
-            aop.w = ((wj[jj] >> 12) & msk) | ex;
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb) P[pl][mb] = T::mfma16(aop, act[jj][mb], P[pl][mb]);
+        for (int jj = sj * (4 / SUBG); jj < (sj + 1) * (4 / SUBG); ++jj) {
+          const uint32_t wj = wq[s][j][0][jj];
+          v4u aop;
+          if constexpr (W8) {
+            aop = regs_codes8<BF16>(wj, wq[s][j][PL - 1][jj]);
+          } else {
+            aop.x = (wj & msk) | ex;
+            aop.y = ((wj >> 4) & msk) | ex;
+            aop.z = ((wj >> 8) & msk) | ex;
+            aop.w = ((wj >> 12) & msk) | ex;
           }
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) P[mb] = T::mfma16(aop, act[jj][mb], P[mb]);
         }
         float sf[4];
         if constexpr (BF16) {
@@ -309,17 +331,11 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(VAQ_HEAD_ARGS,
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float zc = HAS_ZP ? T::CODE_BIAS + (float)((z4 >> (4 * r)) & 0xFu) : T::CODE_BIAS + 8.0f;
+          const float zc = HAS_ZP ? T::CODE_BIAS + (float)((z4 >> (4 * r)) & 0xFu) : ZERO;
 #pragma unroll
           for (int mb = 0; mb < MB; ++mb) {
-            if constexpr (CHAIN) {
-              acc[j][mb][r] = fmaf(sf[r], P[0][mb][r], acc[j][mb][r]);
-            } else if constexpr (W8) {      // high plane (bias 8 of its own) times 16, then the low one
-              acc[j][mb][r] = fmaf(16.0f * sf[r], fmaf(-zc, S[sj][mb], P[0][mb][r]), acc[j][mb][r]);
-              acc[j][mb][r] = fmaf(sf[r], fmaf(-T::CODE_BIAS, S[sj][mb], P[PL - 1][mb][r]), acc[j][mb][r]);
-            } else {
-              acc[j][mb][r] = fmaf(sf[r], fmaf(-zc, S[sj][mb], P[0][mb][r]), acc[j][mb][r]);
-            }
+            if constexpr (CHAIN) acc[j][mb][r] = fmaf(sf[r], P[mb][r], acc[j][mb][r]);
+            else acc[j][mb][r] = fmaf(sf[r], fmaf(-zc, S[sj][mb], P[mb][r]), acc[j][mb][r]);
           }
         }
       }
