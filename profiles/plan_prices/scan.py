@@ -16,7 +16,8 @@ Runs on the GPU; the *.csv.gz beside it are what it wrote on an MI355X.  A probl
                         kind 0 workgroups of all rows, 1 of 16 rows, 2 the tile kernel by the plan of the shapes with weights
                         through LDS (gs, wks, wn 0), at whose price the decode kernels are weighed
     w4_regs:            k, n, m, groups of 128 rows, 8-bit codes, zero points, fp16, wavefronts, n-tiles, m-blocks, parts of K, us: the kernel
-                        with activations in registers; wavefronts 0: what takes the problem without it.  (The file's last
+                        with activations in registers (8-bit codes timed again after their planes became one operand, scaled by what the problem takes without this
+                        kernel then and in the file); wavefronts 0: what takes the problem without it.  (The file's last
                         problems, vocabulary layers and ordinary K and N, have the library's plan alone.)
 """
 from __future__ import annotations

@@ -22,7 +22,10 @@ struct RegsPlan {
 // of partial results.
 // Fitted, a set per format (4-bit codes in groups of 128 rows: another for up to 4 rows), to the cold times of 2.2e5 launches: 11400 problems of random layers, half of them with K 1024 .. 14336 and N
 // 1024 .. 28672, half with K 256 .. 28672 and N 256 .. 152064, 1 .. 200 rows, with and without zero points, bf16 and fp16, each with up to 24
-// plans (a part of those in profiles/plan_prices).  The cheapest plan takes 1.012 .. 1.015 of the fastest one's time in the mean.
+// plans (a part of those in profiles/plan_prices).  The cheapest plan takes 1.012 .. 1.015 of the fastest one's time in the mean.  8-bit codes again, after their planes became one
+// operand, to 24326 launches of 1261 problems, which take 0.80 .. 0.97 of the time: cheapest plan 1.011 / 1.012 / 1.013 in groups of 128 / 64 / 32 rows (1.018 / 1.017 / 1.014 with the
+// constants before), choice between this kernel and the others 1.003 / 1.002 / 1.003 of the faster one's time (1.010 / 1.008 / 1.013); 400 drawn calls of 1 .. 256 rows 0.986 by the constants,
+// 5 of them more than 3 % slower, 47 faster (9344 x 2304 at M = 15 8.8 -> 10.1 us: 73 k-tiles on eight wavefronts).
 struct RegsCost {
   double base, round, latency, row, tile, tile_mb, kb, mem_mb, last, meet, meet_wave, out, handover, part, part_mb, again, alone, copies, k1024;
 };
@@ -30,9 +33,9 @@ constexpr RegsCost REGS_COST_W4_4ROWS = {1.81, 0.102, 0.271, 0, 0.0698, 0.0322, 
 constexpr RegsCost REGS_COST_W4 = {1.92, 0.0921, 0.156, 0.0473, 0.0944, 0.0133, 0.0121, 0.162, 0.069, 0.198, 0, 0.134, 0.42, 0.39, 0.893, 0.163, 1.32, 1.18, 1.08};
 constexpr RegsCost REGS_COST_W4_64 = {2.13, 0.00844, 0.197, 0.0341, 0.102, 0.0279, 0.0118, 0.158, 0.121, 0.155, 0.012, 0.0826, 0.463, 0.358, 0.884, 0.173, 1.55, 1.15, 1.09};
 constexpr RegsCost REGS_COST_W4_32 = {2.19, 0, 0.264, 0.00999, 0.127, 0.0499, 0.0136, 0.185, 0.0443, 0.127, 0.0131, 0.142, 0.496, 0.351, 0.912, 0.0388, 1.7, 1.01, 1.08};
-constexpr RegsCost REGS_COST_W8 = {1.97, 0, 0.0427, 0, 0.0788, 0.0246, 0.0125, 0.155, 0, 0.265, 0.00381, 0.0954, 0.43, 0.343, 0.936, 0.165, 1.18, 1.17, 1.09};
-constexpr RegsCost REGS_COST_W8_64 = {2.03, 0, 0.0526, 0, 0.0773, 0.0375, 0.0127, 0.165, 0.0271, 0.281, 0, 0.184, 0.582, 0.311, 0.975, 0.151, 1.31, 1.2, 1.1};
-constexpr RegsCost REGS_COST_W8_32 = {2.09, 0, 0.268, 0, 0.0902, 0.0521, 0.0146, 0.173, 0, 0.127, 0.0286, 0.147, 0.594, 0.314, 1.07, 0.144, 1.6, 0.977, 1.09};
+constexpr RegsCost REGS_COST_W8 = {1.75, 0.00662, 0.0353, 0.00418, 0.0821, 0.021, 0.0113, 0.167, 0.00427, 0.228, 0.00326, 0.101, 0.524, 0.266, 0.925, 0.15, 1.01, 0.879, 1.07};
+constexpr RegsCost REGS_COST_W8_64 = {1.94, 0.00969, 0.157, 0.00336, 0.0761, 0.0347, 0.0117, 0.161, 0.0112, 0.113, 0.00298, 0.186, 0.84, 0.348, 0.784, 0.192, 1.14, 1.05, 0.989};
+constexpr RegsCost REGS_COST_W8_32 = {1.43, 0.00318, 0.38, 0.00372, 0.0848, 0.0367, 0.0136, 0.198, 0.00257, 0.166, 0.0167, 0.0899, 0.925, 0.234, 0.884, 0.128, 1.6, 0.869, 0.94};
 
 static double regs_us(const RegsPlan& p, int M, int N, int K, int sub, bool w8, int cus) {
   const RegsCost& c = w8 ? (sub == 1 ? REGS_COST_W8 : sub == 2 ? REGS_COST_W8_64 : REGS_COST_W8_32)
