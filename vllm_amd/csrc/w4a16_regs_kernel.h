@@ -278,9 +278,9 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(VAQ_HEAD_ARGS,
       __builtin_amdgcn_sched_barrier(0);
     }
     // row sums S of each group: the same in the four registers.  Plain codes: -(BIAS + 8) S is where the group's MFMA chain starts.
-    constexpr bool CHAIN = SUBG == 1 && !HAS_ZP;
+    constexpr bool CHAIN = !HAS_ZP;
     constexpr float ZERO = W8 ? (BF16 ? 128.0f : T::CODE_BIAS + 128.0f) : T::CODE_BIAS + 8.0f;      // what the operands have too much (regs_codes8)
-    v4f start[MB];
+    v4f start[CHAIN ? SUBG : 1][MB];
     float S[SUBG][MB];
     const v4u ones = {T::ONE2, T::ONE2, T::ONE2, T::ONE2};
 #pragma unroll
@@ -290,8 +290,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(VAQ_HEAD_ARGS,
         v4f t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int jj = sj * (4 / SUBG); jj < (sj + 1) * (4 / SUBG); ++jj) t = T::mfma16(ones, act[jj][mb], t);
-        start[mb] = t * -ZERO;
-        S[sj][mb] = t[0];
+        if constexpr (CHAIN) start[sj][mb] = t * -ZERO;
+        else S[sj][mb] = t[0];
       }
 #pragma unroll
     for (int j = 0; j < J; ++j) {
@@ -301,7 +301,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(VAQ_HEAD_ARGS,
         const uint32_t z4 = HAS_ZP ? *reinterpret_cast<const uint32_t*>(side + SC + sj * 64 + j * 8 + (o >> 1) * 4) >> ((o & 1) * 16) : 0u;
         v4f P[MB];
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) P[mb] = CHAIN ? start[mb] : v4f{0.f, 0.f, 0.f, 0.f};
+        for (int mb = 0; mb < MB; ++mb) P[mb] = CHAIN ? start[CHAIN ? sj : 0][mb] : v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int jj = sj * (4 / SUBG); jj < (sj + 1) * (4 / SUBG); ++jj) {
           const uint32_t wj = wq[s][j][0][jj];
@@ -331,7 +331,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(VAQ_HEAD_ARGS,
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float zc = HAS_ZP ? T::CODE_BIAS + (float)((z4 >> (4 * r)) & 0xFu) : ZERO;
+          const float zc = T::CODE_BIAS + (float)((z4 >> (4 * r)) & 0xFu);
 #pragma unroll
           for (int mb = 0; mb < MB; ++mb) {
             if constexpr (CHAIN) acc[j][mb][r] = fmaf(sf[r], P[mb][r], acc[j][mb][r]);
