@@ -740,7 +740,7 @@ def w4a16_tile_kernel(m, n, k):
     from vllm_amd import _lib
     plan = (ctypes.c_double * 4)()
     _lib.check(_lib.load().vaq_w4a16_tile_plan(m, n, k, 1, 0, 0, plan))
-    return "vaq::w4a16_strip_kernel" if plan[0] > 40 else "vaq::w4a16_prefill2_kernel"
+    return "vaq::w4a16_tile256_kernel" if plan[0] == 48 else "vaq::w4a16_strip_kernel" if plan[0] > 40 else "vaq::w4a16_prefill2_kernel"
 
 
 def w4a16_decode_kernels(shapes):

@@ -41,3 +41,16 @@ def test_extra_goes_to_a_side_file(tmp_path):
     p = tmp_path / "x" / "extra.json"
     b.write_extra({"prefill": [dict(K=1)]}, str(p))
     assert json.loads(p.read_text()) == {"prefill": [{"K": 1}]}
+
+
+def test_tile_rows_name_the_kernel_that_runs():
+    """Every tile id that the library's plans hold, by the kernel that it stands for (w4a16_prefill_launch)."""
+    import ctypes
+    from vllm_amd import _lib
+    lib, b, plan, seen = _lib.load(), _bench(), (ctypes.c_double * 4)(), set()
+    for m, n, k in ((4096, 4096, 4096), (4096, 28672, 4096), (300, 6144, 4096), (100, 4096, 4096), (8192, 1024, 256), (2048, 512, 128)):
+        assert lib.vaq_w4a16_tile_plan(m, n, k, 1, 0, 0, plan) == 0
+        kernel = "tile256" if plan[0] == 48 else "strip" if plan[0] > 40 else "prefill2"
+        seen.add(kernel)
+        assert b.w4a16_tile_kernel(m, n, k) == f"vaq::w4a16_{kernel}_kernel", (m, n, k)
+    assert {"tile256", "strip"} <= seen

@@ -88,8 +88,8 @@ int vaq_w4a16_regs_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub,
 int vaq_fp8_regs_plan(int64_t size_m, int64_t size_n, int64_t size_k, double* plan);
 
 /*
- * The same of the W4A16 tile kernels: plan[0 .. 3] = tile id (41 and above: strips), parts of K, first tile that is split where only
- * those of the last round are (else 0), predicted us.  `wt` = 0 4-bit, 1 8-bit codes, 2 FP8 weights; `staged` = 1: the cheapest plan
+ * The same of the W4A16 tile kernels: plan[0 .. 3] = tile id (48: the 256 x 256 kernel of w4a16_tile256_kernel.h, others from 41 on: strips), parts of K,
+ * first tile that is split where only those of the last round are (else 0), predicted us.  `wt` = 0 4-bit, 1 8-bit codes, 2 FP8 weights; `staged` = 1: the cheapest plan
  * of the shapes with weights through LDS, whose price the decode kernels are weighed against.
  */
 int vaq_w4a16_tile_plan(int64_t size_m, int64_t size_n, int64_t size_k, int sub, int wt, int staged, double* plan);
