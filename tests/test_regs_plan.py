@@ -108,3 +108,24 @@ def test_vocabulary_layers_are_weighed_against_the_kernel_that_runs(k, m4, m16):
 def test_layers_where_one_kernel_is_well_ahead(k, n, m, takes):
     """Timed 4 .. 11 % behind and 5 .. 25 % ahead of the decode kernel."""
     assert _plan(m, n, k, 1, 0)[-1] == takes
+
+
+@pytest.mark.parametrize("k,n,m,sub", [(21760, 12096, 157, 1), (14592, 17920, 129, 2), (3456, 5888, 189, 2), (13056, 2880, 69, 2), (11648, 20160, 139, 2)])
+def test_unrounded_weights_stay_where_they_were(k, n, m, sub):
+    """Calls that the kernel with operands in registers took before there were 256 x 256 tiles: these round the weights to 16 bits."""
+    assert _plan(m, n, k, sub, 0)[-1] == 1
+
+
+def test_no_call_is_weighed_against_256_x_256_tiles():
+    """Where those are the cheapest tiles, what this kernel is weighed against costs more than they do."""
+    rng, tile, seen = random.Random(7), (ctypes.c_double * 4)(), 0
+    for _ in range(3000):
+        m, k, n = rng.randint(100, 256), 128 * int(16 * 14 ** rng.random()), 64 * int(64 * 30 ** rng.random())
+        sub, w8 = rng.choice([1, 2, 4]), rng.choice([0, 1])
+        if k * n >= 1 << 30:
+            continue
+        _lib.check(_lib.load().vaq_w4a16_tile_plan(m, n, k, sub, w8, 0, tile))
+        if tile[0] == 48:
+            assert _plan(m, n, k, sub, w8)[5] > tile[3]
+            seen += 1
+    assert seen > 200

@@ -25,6 +25,7 @@ struct TilePlan {
   int64_t tail_first = 0;      // > 0: only the tiles from this position on are split (tile_handover.h)
   int64_t extra_tiles = 0;     // split K: the tiles of a tile row past M that runs beside the real ones (FP8)
   double us = -1;
+  double us_strips = -1;       // W4A16: of the cheapest plan without the 256 x 256 tiles of w4a16_tile256_kernel.h
   // scratch of the K split: partial tiles and arrival counters of the tiles that are split
   int64_t split_tiles() const { return sk > 1 ? tiles + extra_tiles - tail_first : 0; }
   int64_t tmp_bytes() const { return (int64_t)sk * split_tiles() * bm * bn * 4; }
