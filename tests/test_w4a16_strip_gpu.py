@@ -1,4 +1,4 @@
-"""The W4A16 tile kernel with register-resident weight strips (w4a16_strip_kernel.h), every shape of it forced, against the CPU oracle."""
+"""The W4A16 tile kernels with weights dequantised in registers (w4a16_strip_kernel.h, and w4a16_tile256_kernel.h: 48), every shape forced, against the CPU oracle."""
 from __future__ import annotations
 
 import ctypes
@@ -11,8 +11,8 @@ from tests.helpers import W4A16Layer, check_gemm_close
 
 pytestmark = pytest.mark.gpu
 
-EVERY_FORMAT = (41, 42, 43, 44, 46, 51, 52)
-PLAIN_ONLY = (48, 66)      # 4-bit codes in groups of 128 rows / channelwise
+EVERY_FORMAT = (41, 42, 43, 44, 46, 48, 51, 52)
+PLAIN_ONLY = (66,)      # 4-bit codes in groups of 128 rows / channelwise
 
 # (K, N, M): one quantisation group; fewer groups than a workgroup takes side by side, and a remainder of them; one to several turns
 # of the weight ring and each remainder of it; a last strip and a last tile row that are mostly empty
