@@ -23,7 +23,7 @@
 // sums and stores; the K loop's MFMAs alone 13.7 us, with fragment reads and dequantisation 18 us (up to 64 rows the 19 VALU
 // instructions per 8 weights take longer than the MFMAs that hide them); operands that toggle 5 us (power); the rest is the memory
 // traffic beside it (all operands from memory without arithmetic: 13 us).  Not kept: all requests of a step at once behind the
-// barrier (+1 us), more stages (level), a half of the strip's rows per wavefront (256 x 256, +3 %).
+// barrier (+1 us), more stages (level).
 #pragma once
 #include "w4a16_prefill_kernel.h"
 
@@ -220,8 +220,8 @@ __global__ __launch_bounds__(512, WMB * WNB == 1 && HAS_ZP && SUBG == 4 ? 4 : 2)
   using C2 = std::integral_constant<int, 2>;
   using C3 = std::integral_constant<int, 3>;
 
-  // Vector-memory operations retire in issue order.  In front of the last slice of step h the activations of step h + 1 must
-  // have landed; newer than they are those of the NST - 2 steps behind them and the weights requested since.
+  // Vector-memory operations retire in issue order.  At the barrier of step h, ahead of its last slice (with DEEP of its last two), the activations of step h + 1
+  // must have landed; newer than they are those of the NST - 2 steps behind them, the last of whose quarters went out in the slice ahead of it, and the weights requested since.
   constexpr int WAIT = (NST - 2) * A_LD + KW * ((NST - 2) / 2);
   static_assert(NST % 2 == 0 && NST <= 2 * PD, "requests newer than a step's activations: the same for even and odd steps, and in the prologue");
   static_assert(WAIT <= 63 && (NST - 2) * A_LD + (PD - 1) * KW <= 63, "wait counter range");
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(512, WMB * WNB == 1 && HAS_ZP && SUBG == 4 ? 4 : 2)
   // and every wavefront stalls on it with its matrix instructions behind.
   auto quarter = [&](int h, int stage, int q) { issue_a(h, stage, q * A_LD / 4, (q + 1) * A_LD / 4); };
 
-  // ---- prologue: the requests of the first NST steps (of the last a quarter) and PD rounds.  Behind the activations of a step
+  // ---- prologue: the requests of the first NST steps (of the last a quarter, with DEEP two: as many as stand behind a barrier in the loop) and PD rounds.  Behind the activations of a step
   // there must be as many requests as in the loop, where round x's weights go out behind step 2 (x - PD) + NST - 2: the waits in
   // front of the barriers count on it. ----
   auto keep_order = [] { asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); };

@@ -1,7 +1,7 @@
 // W4A16 tile GEMM for many rows: 256 x 256 tiles, weights dequantised in registers, one wavefront to a SIMD.
 //
-// Four wavefronts, each a strip of 64 columns (four native 16-column tiles) for all 256 rows: 64 x 4 blocks of v_mfma_f32_16x16x32 results in all 256
-// accumulation registers, everything else in 160 .. 200 vector registers.
+// Four wavefronts, each a strip of 64 columns (four native 16-column tiles) for all 256 rows: 16 x 4 blocks of v_mfma_f32_16x16x32 results, four registers each, in all 256
+// accumulation registers, everything else in 128 .. 184 vector registers (4-bit codes in groups of 128 rows 128 .. 140).
 //
 //  * Weights: a ring of two quantisation groups (128 rows of K) in registers, requested two groups ahead straight from memory.  A native tile's word is the A
 //    operand (rows = n) of one MFMA as it lies; dequantised with scale and zero point exactly like the other tile kernels do (fma(code, s, -z s) rounded
