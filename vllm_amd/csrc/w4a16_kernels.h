@@ -14,8 +14,8 @@ int w4a16_decode2_workspace(int M, int N, int K, int sub, bool w8, size_t* c_tmp
 enum { D2_TILE, D2_WORKGROUP, D2_ROWS };
 int w4a16_decode2_choose(int M, int N, int K, int sub, int wt, bool act_order, bool has_perm, bool wg_ok, bool tile_ok, double tile_us);
 // What the choice of a tile depends on: 4-bit codes in groups of 128 rows / channelwise, in smaller groups, 8-bit codes likewise and in groups
-// of 32, FP8 weights (and plain codes on the shapes with weights through LDS only, to price them).
-enum TileFormat { TILES_PLAIN, TILES_SUB, TILES_8BIT, TILES_8BIT_64, TILES_8BIT_32, TILES_FP8, TILES_PLAIN_STAGED };
+// of 32, FP8 weights (and two to price calls by: plain codes on the shapes with weights through LDS only, smaller groups on what the kernel with activations in registers is weighed against).
+enum TileFormat { TILES_PLAIN, TILES_SUB, TILES_8BIT, TILES_8BIT_64, TILES_8BIT_32, TILES_FP8, TILES_PLAIN_STAGED, TILES_SUB_WEIGHED };
 inline TileFormat tile_format(int sub, int wt) {
   if (wt == 1) return sub == 1 ? TILES_8BIT : sub == 2 ? TILES_8BIT_64 : TILES_8BIT_32;
   return wt == 2 ? TILES_FP8 : sub > 1 ? TILES_SUB : TILES_PLAIN;

@@ -49,9 +49,8 @@ static int dispatch_tile(const PrefillParams& p, int tile, hipStream_t s) {
 // 12 .. 20 (weights through LDS) takes this much more than that of the shapes from 41 on (strips): 41 / 29 / 26 / 22 / 17 / 11 / 8 / 3 %
 // at M up to 32 / 64 / 128 / 256 / 512 / 1024 / 2048 / 8192; at M > 512 it is ahead in 10-25 % of the problems, by a few percent.
 // The shape 48 (w4a16_tile256_kernel.h; before it a 256 x 256 shape of the strip kernel, for 4-bit codes in groups of 128 rows alone) came later, in all four tables, timed on
-// their problems of more than 128 rows; its constants, and with them those of 8-bit codes, are those whose choice loses
-// least.  (Those of five other large shapes in groups of 64 / 32 rows of 4 bits had followed too, for 0.02 .. 0.06 %; at these prices calls left the kernel with activations in registers, which
-// rounds less.)  Over 4581 other problems of M = 200 .. 8192 it is the fastest plan of 47 %, and what it takes there is 0.92 (4 bits in groups of 128 rows) .. 0.88 of what those problems took.
+// their problems of more than 128 rows; its constants, and with them those of 8-bit codes and of five other large shapes in groups of 64 / 32 rows of 4 bits, are those whose choice loses
+// least.  Over 4581 other problems of M = 200 .. 8192 it is the fastest plan of 47 %, and what it takes there is 0.92 (4 bits in groups of 128 rows) .. 0.88 of what those problems took.
 constexpr TileShape W4_TILE_SHAPES[] = {
     {12, 128, 128, 8, 2, 0.536, 0.606, 0.0793, 0.375, 0.153}, {14, 64, 128, 8, 2, 0, 0.535, 0.0271, 0.177, 0.252},
     {15, 128, 64, 4, 2, 0, 0.553, 0.0166, 0.0944, 0.337},     {16, 256, 128, 8, 1, 1.88, 0.781, 0.176, 0, 0.0912},
@@ -68,13 +67,24 @@ constexpr TileCosts W4_TILE_COSTS = {0.163, 0.628, 0.63, 0.253, 0.0};
 // 0.7, 0.7, 1.0 and 1.9 %).
 constexpr TileShape W4SUB_TILE_SHAPES[] = {
     {12, 128, 128, 8, 2, 0.726, 0.631, 0.0892, 0.392, 0.139}, {14, 64, 128, 8, 2, 0, 0.613, 0.0195, 0.177, 0.269},
+    {15, 128, 64, 4, 2, 0, 0.583, 0.0117, 0.107, 0.358},      {16, 256, 128, 8, 1, 1.66, 0.83, 0.166, 0, 0.0983},
+    {20, 256, 256, 8, 1, 4.63, 1.36, 0.123, 0, 0.0118},
+    {41, 32, 128, 8, 2, 2.38, 0.236, 0.0194, 0.195, 0.161},   {51, 32, 64, 8, 2, 1.31, 0.124, 0.00437, 0.141, 0.681},
+    {42, 64, 128, 8, 1, 2.47, 0.264, 0.0529, 0, 0.0702},      {52, 64, 64, 8, 1, 2.52, 0.165, 0.0145, 0, 0.067},
+    {43, 96, 128, 8, 1, 2.31, 0.334, 0.0356, 0, 0.27},       {44, 128, 128, 8, 1, 3.2, 0.381, 0.0552, 0, 0.242},
+    {46, 128, 256, 8, 1, 3.88, 0.573, 0.233, 0, 0.0539},
+    {48, 256, 256, 4, 1, 7.4, 1.2, 0.0749, 0, 0.0156}};
+constexpr TileCosts W4SUB_TILE_COSTS = {0.131, 0.547, 0.631, 0.274, 0.0};
+// What the kernel with activations in registers is weighed against (w4a16_tile_us): the strips ahead of that shape, at the prices that its shares (w4a16_gemm.hip) were set at.  Five large shapes
+// followed the shape 48, for 0.02 .. 0.06 % of what the choice among tiles loses; at those 14 of 29310 drawn problems of 17 .. 256 rows would leave that kernel, which rounds less.
+constexpr TileShape W4SUB_WEIGHED_SHAPES[] = {
+    {12, 128, 128, 8, 2, 0.726, 0.631, 0.0892, 0.392, 0.139}, {14, 64, 128, 8, 2, 0, 0.613, 0.0195, 0.177, 0.269},
     {15, 128, 64, 4, 2, 0, 0.583, 0.0117, 0.107, 0.358},      {16, 256, 128, 8, 1, 1.95, 0.825, 0.183, 0, 0.11},
     {20, 256, 256, 8, 1, 4.48, 1.36, 0.12, 0, 0.013},
     {41, 32, 128, 8, 2, 2.38, 0.236, 0.0194, 0.195, 0.161},   {51, 32, 64, 8, 2, 1.31, 0.124, 0.00437, 0.141, 0.681},
     {42, 64, 128, 8, 1, 2.47, 0.264, 0.0529, 0, 0.0702},      {52, 64, 64, 8, 1, 2.52, 0.165, 0.0145, 0, 0.067},
     {43, 96, 128, 8, 1, 2.57, 0.333, 0.0362, 0, 0.257},       {44, 128, 128, 8, 1, 3.05, 0.386, 0.0558, 0, 0.246},
-    {46, 128, 256, 8, 1, 3.85, 0.584, 0.219, 0, 0.0488},      {48, 256, 256, 4, 1, 7.4, 1.2, 0.0749, 0, 0.0156}};
-constexpr TileCosts W4SUB_TILE_COSTS = {0.131, 0.547, 0.631, 0.274, 0.0};
+    {46, 128, 256, 8, 1, 3.85, 0.584, 0.219, 0, 0.0488}};
 // 8-bit codes, whose dequantisation takes longer: 1216 such problems, 37199 launches, in the mean 0.6 % (2.4 % with the first constants above).
 // Groups of 64 rows take them too, but for the slots of the shape 41 (make_plan_prefill): 876 problems, 24724 launches, 0.35 %.
 // The strips that read activation fragments two slices ahead (w4a16_strip_kernel.h: the shapes 42 in groups of 64 rows and more, 43, 44, 46) take 0.94 .. 0.98 of what these problems were
@@ -109,7 +119,7 @@ constexpr TileShape LDS_TILE_SHAPES[] = {
     {15, 128, 64, 4, 2, 0, 0.456, 0.025, 0.176, 0.392},     {16, 256, 128, 8, 1, 2.57, 0.764, 0.194, 0, 0.122},
     {13, 128, 256, 8, 1, 2.93, 0.869, 0.186, 0, 0.061},     {20, 256, 256, 8, 1, 6.10, 1.200, 0.422, 0, 0.024}};
 constexpr TileCosts LDS_TILE_COSTS = {0.277, 1.42, 0.796, 0.162, 0.0};
-static_assert(W4_TILE_SHAPES[std::size(W4_TILE_SHAPES) - 1].id == 48 && W4SUB_TILE_SHAPES[std::size(W4SUB_TILE_SHAPES) - 1].id == 48 &&
+static_assert(W4_TILE_SHAPES[std::size(W4_TILE_SHAPES) - 1].id == 48 && std::size(W4SUB_WEIGHED_SHAPES) == std::size(W4SUB_TILE_SHAPES) - 1 &&
                   W8_TILE_SHAPES[std::size(W8_TILE_SHAPES) - 1].id == 48 && W8G32_TILE_SHAPES[std::size(W8G32_TILE_SHAPES) - 1].id == 48,
               "what the kernel with activations in registers is weighed against is known ahead of the last shape");
 struct TilePrices {
@@ -118,6 +128,7 @@ struct TilePrices {
   double weight_bytes;      // per element, as the fit counted them
 };
 static TilePrices tile_prices(TileFormat format) {
+  if (format == TILES_SUB_WEIGHED) return {std::begin(W4SUB_WEIGHED_SHAPES), std::end(W4SUB_WEIGHED_SHAPES), W4SUB_TILE_COSTS, 0.5};
   if (format == TILES_SUB) return {std::begin(W4SUB_TILE_SHAPES), std::end(W4SUB_TILE_SHAPES), W4SUB_TILE_COSTS, 0.5};
   if (format == TILES_8BIT_32) return {std::begin(W8G32_TILE_SHAPES), std::end(W8G32_TILE_SHAPES), W8G32_TILE_COSTS, 1.0};
   if (format == TILES_8BIT || format == TILES_8BIT_64) return {std::begin(W8_TILE_SHAPES), std::end(W8_TILE_SHAPES), W8_TILE_COSTS, 1.0};
@@ -208,7 +219,7 @@ double w4a16_staged_us(int M, int N, int K, bool plain) { return plan_prefill(M,
 // above, no call loses those bits to the 256 x 256 tiles, which came last and are cheaper than the strips from 130 rows on where K N is large (6 of 6677 problems of
 // 17 .. 256 rows of 4-bit codes in groups of 128, 28 and 2 in groups of 64 and 32 had gone, at the prices of two steps; 21760 x 12096 at M = 157 is priced 105.8 there, 111.5 in such
 // tiles and 117.7 in strips).
-double w4a16_tile_us(int M, int N, int K, TileFormat format) { return plan_prefill(M, N, K, true, format).us_strips; }
+double w4a16_tile_us(int M, int N, int K, TileFormat format) { return plan_prefill(M, N, K, true, format == TILES_SUB ? TILES_SUB_WEIGHED : format).us_strips; }
 
 int w4a16_prefill_workspace(int M, int N, int K, TileFormat format, size_t* c_tmp_bytes, size_t* counter_ints) {
   const TilePlan pl = plan_prefill(M, N, K, true, format);
