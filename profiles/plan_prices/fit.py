@@ -49,6 +49,7 @@ class Tiles:
         self.shape = rows[:, 1:5]                        # bm, bn, nw, slots
         self.p_shape = rows[:, 5:]                       # base, step, load, shared, out
         self.p_costs = np.array(source_table(file, f"{prefix}_TILE_COSTS"))
+        self.few_rows = 512 if prefix in ("W4", "W8") else 0
         self.bytes = 0.5 if prefix.startswith(("W4", "LDS")) else 1.0
 
     def pack(self):
@@ -79,6 +80,8 @@ class Tiles:
     def price(self, p_shape, p_costs):
         bm, bn, _, slots = self.shape[self.which].T
         base, step, load, shared, out = p_shape[self.which].T
+        few = np.where((self.ids[self.which] == 48) & (self.m <= self.few_rows), 1.03, 1.0)      # (TILE256_FEW_ROWS_PRICE)
+        base, step, load = base * few, step * few, load * few
         weight_mb, handover, part_cost, handover_mb, sum_mb = p_costs[:5]
         tiles = np.ceil(self.m / bm) * np.ceil(self.n / bn)
         steps = self.k // 64

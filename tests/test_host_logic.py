@@ -784,3 +784,13 @@ def test_w4a16_tile_plans_of_every_format(kind, files, group, wtype, most, most_
         assert m <= 64 or int(plan[0]) != int(t.ids[t.which[i]]) or sizes[0].value == want
     # (a plan that was not timed, because its shape is far too large for the problem, may be the cheapest; and equal prices)
     assert agree > 0.97 * total, (agree, total)
+
+
+@pytest.mark.parametrize("k,n,m,group", [(9856, 23488, 313, 128), (1280, 24384, 365, 64)])
+def test_256_x_256_tiles_of_few_rows_are_not_taken_for_their_price(k, n, m, group):
+    """8-bit codes: timed 7 and 10 % behind the shapes that the library chooses."""
+    import ctypes
+    from vllm_amd import _lib
+    plan = (ctypes.c_double * 4)()
+    _lib.check(_lib.load().vaq_w4a16_tile_plan(m, n, k, 128 // group, 1, 0, plan))
+    assert plan[0] != 48

@@ -143,6 +143,12 @@ static int pick_register_staged(int M, int N) {
   return tiles(256, 256) >= cus ? 0 : (tiles(128, 128) >= cus ? 1 : 2);
 }
 
+// One or two tiles one below the other, up to 512 rows, the shape 48 takes 4 .. 10 % longer beside the others than its constants say, which are fitted to thousands of rows too.  Of the recorded
+// problems of 129 .. 256 rows the chosen plan takes 1.0072 -> 1.0066 of the fastest one's time (4 bits, groups of 128), 1.0077 -> 1.0065 (8 bits) and 1.0037 -> 1.0031 (groups of 64); from 257 to
+// 512 1.0071, 1.0084 -> 1.0083 and 1.0050 -> 1.0048.  90 drawn calls whose plan moves by it take 0.957 of the time, 63 more than 3 % faster, 3 slower (4 % at most); 8 bits, 9856 x 23488 at
+// M = 313 227 -> 203 us, 1280 x 24384 at M = 365 in groups of 64 38.7 -> 36.2.  Not in smaller groups, whose recorded choice it makes no better (fp16 up to 15 % slower).
+constexpr double TILE256_FEW_ROWS_PRICE = 1.03;
+
 // Tile shape and K split for a problem (the shapes 13 and 66 are built for TILES_PLAIN; 30, another kernel of the shape 20 in
 // recorded timings, stands for 20).
 static TilePlan make_plan_prefill(int M, int N, int K, TileFormat format) {
@@ -159,6 +165,11 @@ static TilePlan make_plan_prefill(int M, int N, int K, TileFormat format) {
   for (const TileShape* shape = prices.begin; shape != prices.end; ++shape) {
     TileShape t = *shape;
     if (t.id == 41 && format == TILES_8BIT_64) t.slots = 1;      // (133 registers)
+    if (t.id == 48 && M <= 512 && (format == TILES_PLAIN || format == TILES_8BIT || format == TILES_8BIT_64)) {
+      t.base *= TILE256_FEW_ROWS_PRICE;
+      t.step *= TILE256_FEW_ROWS_PRICE;
+      t.load *= TILE256_FEW_ROWS_PRICE;
+    }
     const bool is256 = t.id == 20 || t.id == 48;
     if (t.id == 48) best.us_strips = best.us;      // (the last row of a table)
     if (forced >= 0 ? forced != t.id && !(t.id == 20 && (forced == 10 || forced == 11)) : (t.id == 13 || t.id == 66) && !plain) continue;
