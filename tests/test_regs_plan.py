@@ -110,6 +110,12 @@ def test_layers_where_one_kernel_is_well_ahead(k, n, m, takes):
     assert _plan(m, n, k, 1, 0)[-1] == takes
 
 
+@pytest.mark.parametrize("k,n,m,sub,single", [(9344, 2304, 15, 1, False), (8192, 2304, 15, 1, True), (4736, 2304, 15, 1, True)])
+def test_long_streams_of_one_n_tile_of_8_bit_codes(k, n, m, sub, single):
+    """73 k-tiles on eight wavefronts, ten turns: 10.05 us with one n-tile and K whole, 8.8 with two and K in three parts, at prices 6 % apart."""
+    assert (_plan(m, n, k, sub, 1)[0] == 1) == single
+
+
 @pytest.mark.parametrize("k,n,m,sub", [(21760, 12096, 157, 1), (14592, 17920, 129, 2), (3456, 5888, 189, 2), (13056, 2880, 69, 2), (11648, 20160, 139, 2)])
 def test_unrounded_weights_stay_where_they_were(k, n, m, sub):
     """Calls that the kernel with operands in registers took before there were 256 x 256 tiles: these round the weights to 16 bits."""

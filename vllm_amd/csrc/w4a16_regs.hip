@@ -25,7 +25,7 @@ struct RegsPlan {
 // plans (a part of those in profiles/plan_prices).  The cheapest plan takes 1.012 .. 1.015 of the fastest one's time in the mean.  8-bit codes again, after their planes became one
 // operand, to 24326 launches of 1261 problems, which take 0.80 .. 0.97 of the time: cheapest plan 1.011 / 1.012 / 1.013 in groups of 128 / 64 / 32 rows (1.018 / 1.017 / 1.014 with the
 // constants before), choice between this kernel and the others 1.003 / 1.002 / 1.003 of the faster one's time (1.010 / 1.008 / 1.013); 400 drawn calls of 1 .. 256 rows 0.986 by the constants,
-// 5 of them more than 3 % slower, 47 faster (9344 x 2304 at M = 15 8.8 -> 10.1 us: 73 k-tiles on eight wavefronts).
+// 5 of them more than 3 % slower, 47 faster.
 struct RegsCost {
   double base, round, latency, row, tile, tile_mb, kb, mem_mb, last, meet, meet_wave, out, handover, part, part_mb, again, alone, copies, k1024;
 };
@@ -62,11 +62,19 @@ static double regs_us(const RegsPlan& p, int M, int N, int K, int sub, bool w8, 
   return us;
 }
 
+// 8-bit codes, one n-tile to a wavefront, K in nine turns and more, no second workgroup on any compute unit: 4 KB of weights in flight for each wavefront do not cover the latency of that many
+// turns, which takes 1.12 .. 1.18 of the price where other plans take 1.0 .. 1.05.  K is weighed in parts, or more n-tiles, as if that were 8 % more.  Of drawn calls of 1 .. 256 rows 0.8 %
+// move by it; 115 of those, both plans timed, take 0.950 of the time, 74 more than 3 % less, 11 more (8 % at most).  Not in groups of 32 rows beyond 4 rows, whose arithmetic
+// takes longer than that (32 such calls 1.001, 8 more than 3 % slower, 6 faster), and not from seven turns on.  9344 x 2304 at M = 15 10.05 -> 8.8 us (one n-tile, K whole -> two, three parts).
+constexpr int LONG_STREAM_TURNS = 9;
+constexpr double LONG_STREAM_PRICE = 1.08;
+
 // exp[8]: 1 never this kernel, else a plan: n-tiles | m-blocks << 4 | wavefronts << 8 | parts of K << 12
 static RegsPlan make_regs_plan(int M, int N, int K, int sub, bool w8) {
   const int G = K / 128, NT = N / 16, cus = num_cus_current_device();
   const int forced = tuning().exp[8];
   RegsPlan best;
+  double best_us = -1;
   for (int nw : {4, 8})
     for (int mb = 1; mb <= 3; ++mb)
       for (int j = 1; j <= 8; ++j) {
@@ -82,7 +90,11 @@ static RegsPlan make_regs_plan(int M, int N, int K, int sub, bool w8) {
           if (sk > 1 && forced <= 1 && (units >= cus || units * sk > 2 * cus)) break;
           if (sk > 1 && (G / sk < nw || p.tmp_bytes(N) > VAQ_STATIC_SCRATCH_DATA_BYTES || p.counter_ints(N) > (size_t)(NT > 1024 ? NT * 4 : 4096))) break;
           p.us = regs_us(p, M, N, K, sub, w8, cus);
-          if (best.us < 0 || p.us < best.us) best = p;
+          const double us = p.us * (w8 && (sub < 4 || M <= 4) && j == 1 && units * sk <= cus && ((G + sk - 1) / sk + nw - 1) / nw >= LONG_STREAM_TURNS ? LONG_STREAM_PRICE : 1.0);
+          if (best.us < 0 || us < best_us) {
+            best = p;
+            best_us = us;
+          }
         }
       }
   return best;
