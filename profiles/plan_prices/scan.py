@@ -2,7 +2,8 @@
 
     python profiles/plan_prices/scan.py fp8_tile|w4_tile|w8_tile|w4g64z_tile|w4g32_tile|w4g32z_tile|w4g32zh_tile|w8g64_tile|w8g32_tile|w8g32h_tile|w4_decode|w4_regs SECONDS SEED OUT.csv
 
-Runs on the GPU; the *.csv.gz beside it are what it wrote on an MI355X.  A problem is a layer (K, N) and a number of rows; a plan is forced through the `_tuned` entry points
+Runs on the GPU; the *.csv.gz beside it are what it wrote on an MI355X, but for the rows of kernels that changed or came after a file was written: those are what it wrote then, scaled to
+the file as said below by a step that is not kept here, so that their ratios to a problem's other rows count and not their us.  A problem is a layer (K, N) and a number of rows; a plan is forced through the `_tuned` entry points
 (vllm_amd/csrc/vaq_tuning.h).  Weights are cold: a graph of launches walks over copies of the layer (640 MB of them, at most
 400).  One line per plan, with the time of a launch in us:
 
