@@ -445,7 +445,9 @@ __global__ __launch_bounds__(NW * 64, OCC) void w4a16_regs_kernel(VAQ_HEAD_ARGS,
   }
 }
 
-// Registers of a lane, roughly: two k-tiles of weights, sums, operands, a chain per plane, row sums.
+// Registers of a lane as the prices count them (they are fitted on it): two k-tiles of weights, sums, operands, a chain per plane, row sums.  8-bit codes have one chain now and, like groups of 64 / 32 rows
+// of 4-bit codes, starts of their own: against the compiled instances this is up to 39 too many for 8-bit codes, 21 too few to 38 too many for 4-bit ones; counted as compiled, with another fit or without,
+// the plans are no better.  Above 256 sums lie in accumulation registers too; which instances those are it says rightly but for one (bf16 in groups of 32 rows, three m-blocks of six n-tiles: 249).
 constexpr int regs_estimate(int mb, int j, int sub, bool w8) {
   const int pl = w8 ? 2 : 1;
   return 8 * j * pl + 4 * j * mb + 16 * mb + 4 * pl * mb + (4 + sub) * mb + (sub == 4 ? 65 : 45);
