@@ -587,7 +587,7 @@ def operand_toggle_section(dev):
         a = torch.randn(mm, k, device=dev, generator=gen).to(torch.bfloat16)
 
         def whole_tiles():
-            with _tuning.override(prefill_tile=21, prefill_split=1):
+            with _tuning.override(prefill_tile=49, prefill_split=1):      # (id 48: w4a16_tile256_kernel)
                 layer(a)
         t = time_graph(lambda: [whole_tiles() for _ in range(2)], iters=8, warmup=3, inner=2)
         rows.append(dict(kind="w4a16_whole_tiles", workgroups=(mm // 256) * (n // 256), K=k, N=n, M=mm, us=t * 1e6))
