@@ -10,7 +10,7 @@
 //    rows, two to a 256-byte line, 16-byte chunks XOR-ed with the line number).  A fragment is read once and multiplied with four tiles.
 //  * One barrier a step, where the first fragment of the next step is read.
 //  * One instruction stream holds everything that goes on between two MFMAs: a wavefront alone on its SIMD issues two vector instructions beside a 16-cycle MFMA
-//    at no cost (measured 16.2 / 16.6 / 17.3 / 21.7 / 26.8 cycles an MFMA with 0 .. 4 of them), so the dequantisation of the next word is cut into sixteen steps of
+//    at no cost (measured 16.3 / 16.6 / 16.7 / 21.7 / 25.2 cycles an MFMA with 0 .. 4 of them), so the dequantisation of the next word is cut into sixteen steps of
 //    at most two, one behind each MFMA, and a scheduling barrier behind each keeps them there.
 //
 // Why this shape.  At this size the device runs at its power limit (the loop with operands that do not toggle is 1.2 .. 1.3 times faster), so what counts is what an MFMA
